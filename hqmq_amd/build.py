@@ -28,7 +28,7 @@ BENCH_OUT = HERE / "libhqmq_bench.so"
 
 COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-EXACT = {"joint.hip", "quantize.hip", "med3x.hip", "dequant.hip"}
+EXACT = {"joint.hip", "quantize.hip", "quantize_grid.hip", "med3x.hip", "dequant.hip"}
 
 
 def hipcc() -> str:

@@ -3,7 +3,8 @@
 
 using namespace hqmq;
 
-extern "C" int hqmq_append_kv(const hqmq_append_args *k, const hqmq_append_args *v, void *stream) {
+extern "C" int hqmq_append_kv_grid(const hqmq_append_args *k, const hqmq_append_args *v, const void *k_grid, const void *v_grid,
+                                   void *stream) {
     if (!k || !v) return HQMQ_ERR_NULL;
     hipStream_t st = (hipStream_t)stream;
     const hqmq_append_args *a[2] = {k, v};
@@ -35,11 +36,16 @@ extern "C" int hqmq_append_kv(const hqmq_append_args *k, const hqmq_append_args 
     if (rc) return rc;
     // short appends: the quantize launch compacts as well; longer ones get the compaction kernels
     bool compacted[2];
-    rc = quantize_two(&q[0], &q[1], with_q[0], with_q[1], compacted, st);
+    const void *const grids[2] = {k_grid, v_grid};
+    rc = quantize_two(&q[0], &q[1], grids, with_q[0], with_q[1], compacted, st);
     if (rc) return rc;
     CompactCall rest[2];
     int n_rest = 0;
     for (int i = 0; i < 2; i++)
         if (with_q[i] && !compacted[i]) rest[n_rest++] = *with_q[i];
     return n_rest ? compact_calls(rest, n_rest, st) : HQMQ_OK;
+}
+
+extern "C" int hqmq_append_kv(const hqmq_append_args *k, const hqmq_append_args *v, void *stream) {
+    return hqmq_append_kv_grid(k, v, nullptr, nullptr, stream);
 }

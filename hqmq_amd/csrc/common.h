@@ -30,7 +30,7 @@ struct F16 {
     // The empty asm keeps the fp32 value opaque: without it the compiler folds a preceding fused
     // multiply-add into v_fma_mixlo_f16, which rounds once to fp16 instead of fp32-then-fp16.
     static __device__ __forceinline__ float rnd(float f) {
-        asm volatile("" : "+v"(f));
+        asm("" : "+v"(f));
         return __half2float(__float2half_rn(f));
     }
     static __device__ __forceinline__ float eps() { return 4.8828125e-4f; }  // 2^-11
@@ -67,6 +67,52 @@ __device__ __forceinline__ float norm4(float a, float b, float c, float d) {
     s = s + c * c;
     s = s + d * d;
     return sqrtf(s);
+}
+
+// RNE_D(norm4(...)), through v_sqrt_f32 (1 unit in the last place) and one correction step g + (s - g^2) / (2 g) where
+// s is far from the ends of the fp32 range.  Equal to the correctly rounded square root for every mantissa of two
+// binades of s (checked exhaustively on the GPU, all three types); half the instructions.
+template <class D>
+__device__ __forceinline__ float chunk_norm_d(float a, float b, float c, float d) {
+    float s = a * a;
+    s = s + b * b;
+    s = s + c * c;
+    s = s + d * d;
+    const bool fast = (s > 1.2e-29f || s == 0.f) && s < 1.2e30f;         // 2^-96, 2^100
+    if (__builtin_amdgcn_ballot_w64(!fast) != 0ull) return D::rnd(sqrtf(s));
+    const float g = __builtin_amdgcn_sqrtf(s), half_inv = 0.5f * __builtin_amdgcn_rsqf(s);
+    return D::rnd(s == 0.f ? 0.f : fmaf(fmaf(-g, g, s), half_inv, g));
+}
+
+// RNE_D(x / d) for 16-bit D with y = v_rcp_f32(d): the quotient of two numbers of D lies so far from every midpoint
+// between numbers of D (or on it exactly) that a quotient good to a unit in fp32's last place rounds to the same number
+// of D as the correctly rounded one.  bf16: x * y; fp16 (11-bit mantissas) needs one correction.  Checked exhaustively
+// on the GPU over all pairs of mantissas, quotients 2^-30 .. 2^8.  d: ordinary, see quick_divisor.
+template <class D>
+__device__ __forceinline__ float quick_div(float x, float d, float y) {
+    const float q = x * y;
+    return D::rnd(D::code == HQMQ_F16 ? fmaf(fmaf(-d, q, x), y, q) : q);
+}
+template <class D>
+__device__ __forceinline__ bool quick_divisor(float d) {
+    return D::code == HQMQ_F16 ? d > 6.0e-5f && d < 65536.f : d > 1e-30f && d < 1e30f;
+}
+// v[0 .. 3] = RNE_D(v / d)
+template <class D>
+__device__ __forceinline__ void div4_d(float (&v)[4], float d) {
+    if (D::code != HQMQ_F32 && __builtin_amdgcn_ballot_w64(!quick_divisor<D>(d)) == 0ull) {
+        const float y = __builtin_amdgcn_rcpf(d);
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = quick_div<D>(v[j], d, y);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = D::rnd(v[j] / d);
+    }
+}
+template <class D>
+__device__ __forceinline__ float div_d(float x, float d) {
+    if (D::code != HQMQ_F32 && __builtin_amdgcn_ballot_w64(!quick_divisor<D>(d)) == 0ull) return quick_div<D>(x, d, __builtin_amdgcn_rcpf(d));
+    return D::rnd(x / d);
 }
 
 inline int layout_bits(int S, int radius_bits, int *idx_bits, int *main_bits, int *aux_bits) {
@@ -146,8 +192,10 @@ __device__ __forceinline__ void degrade_to_plain(const CompactCall &a, size_t pr
 int med3x_calls(const Med3xCall *c, int count, hipStream_t st);                                            // med3x.hip
 int compact_calls(const CompactCall *c, int count, hipStream_t st);                                        // med3x.hip
 int check_compact(const CompactCall &c);                                                                   // med3x.hip
-// ck / cv (may be NULL): the compaction that follows; compacted[i] tells whether the quantize launch did it
-int quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v, const CompactCall *ck, const CompactCall *cv,
-                 bool compacted[2], hipStream_t st);                                                           // quantize.hip
+// grids: the cell lists of the two codebooks or NULL; ck / cv (may be NULL): the compaction that follows; compacted[i] tells
+// whether the quantize launch did it
+int quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v, const void *const grids[2], const CompactCall *ck,
+                 const CompactCall *cv, bool compacted[2], hipStream_t st);                                    // quantize.hip
+int64_t search_grid_blocks(int S, int dtype);      // uint4 per head of the cell lists, 0: none for this size                  quantize_grid.hip
 
 }  // namespace hqmq

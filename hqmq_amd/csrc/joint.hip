@@ -27,36 +27,36 @@ __device__ __forceinline__ void quat_mul_d(const float a[4], const float b[4], f
     o[3] = A(S(A(M(a[0], b[3]), M(a[1], b[2])), M(a[2], b[1])), M(a[3], b[0]));
 }
 
-// One block per head.
+// One block per head, a thread per codeword (24 S of them in rounds of 1024).
+constexpr int kJointThreads = 1024;
 template <class D>
-__global__ void build_joint_kernel(const float *__restrict__ raw, int S, typename D::storage *__restrict__ joint,
+__global__ __launch_bounds__(kJointThreads) void build_joint_kernel(const float *__restrict__ raw, int S, typename D::storage *__restrict__ joint,
                                    float *__restrict__ slack) {
     const int h = blockIdx.x;
-    __shared__ float red[256];
+    __shared__ float red[kJointThreads];
     float worst = 0.f;
-    for (int s = threadIdx.x; s < S; s += blockDim.x) {
+    for (int k = threadIdx.x; k < 24 * S; k += kJointThreads) {
+        const int p = k / S, s = k - p * S;
         const float *r = raw + ((size_t)h * S + s) * 4;
         float nrm = norm4(r[0], r[1], r[2], r[3]);
         if (!is_nan(nrm) && nrm < 1e-8f) nrm = 1e-8f;
         float q[4];
         for (int j = 0; j < 4; j++) q[j] = D::rnd(r[j] / nrm);
-        for (int p = 0; p < 24; p++) {
-            float pv[4], o[4];
-            cell24_vertex(p, pv);
-            quat_mul_d<D>(pv, q, o);
-            // exact product of the same operands, in double
-            double a0 = pv[0], a1 = pv[1], a2 = pv[2], a3 = pv[3];
-            double b0 = q[0], b1 = q[1], b2 = q[2], b3 = q[3];
-            double e0 = a0 * b0 - a1 * b1 - a2 * b2 - a3 * b3;
-            double e1 = a0 * b1 + a1 * b0 + a2 * b3 - a3 * b2;
-            double e2 = a0 * b2 - a1 * b3 + a2 * b0 + a3 * b1;
-            double e3 = a0 * b3 + a1 * b2 - a2 * b1 + a3 * b0;
-            double d0 = o[0] - e0, d1 = o[1] - e1, d2 = o[2] - e2, d3 = o[3] - e3;
-            float err = (float)sqrt(d0 * d0 + d1 * d1 + d2 * d2 + d3 * d3);
-            if (err > worst || is_nan(err)) worst = err;
-            typename D::storage *dst = joint + (((size_t)h * 24 + p) * S + s) * 4;
-            for (int j = 0; j < 4; j++) D::store(dst + j, o[j]);
-        }
+        float pv[4], o[4];
+        cell24_vertex(p, pv);
+        quat_mul_d<D>(pv, q, o);
+        // exact product of the same operands, in double
+        double a0 = pv[0], a1 = pv[1], a2 = pv[2], a3 = pv[3];
+        double b0 = q[0], b1 = q[1], b2 = q[2], b3 = q[3];
+        double e0 = a0 * b0 - a1 * b1 - a2 * b2 - a3 * b3;
+        double e1 = a0 * b1 + a1 * b0 + a2 * b3 - a3 * b2;
+        double e2 = a0 * b2 - a1 * b3 + a2 * b0 + a3 * b1;
+        double e3 = a0 * b3 + a1 * b2 - a2 * b1 + a3 * b0;
+        double d0 = o[0] - e0, d1 = o[1] - e1, d2 = o[2] - e2, d3 = o[3] - e3;
+        float err = (float)sqrt(d0 * d0 + d1 * d1 + d2 * d2 + d3 * d3);
+        if (err > worst || is_nan(err)) worst = err;
+        typename D::storage *dst = joint + ((size_t)h * 24 * S + k) * 4;
+        for (int j = 0; j < 4; j++) D::store(dst + j, o[j]);
     }
     red[threadIdx.x] = worst;
     __syncthreads();
@@ -79,7 +79,7 @@ extern "C" int hqmq_build_joint(const float *raw, int H, int S, int dtype, void 
     if (!raw || !joint) return HQMQ_ERR_NULL;
     if (H < 1 || S < 1 || S > 2730) return HQMQ_ERR_SHAPE;
     hipStream_t st = (hipStream_t)stream;
-    dim3 grid(H), block(256);
+    dim3 grid(H), block(kJointThreads);
     switch (dtype) {
         case HQMQ_F32: hipLaunchKernelGGL(build_joint_kernel<F32>, grid, block, 0, st, raw, S, (float *)joint, slack); break;
         case HQMQ_F16: hipLaunchKernelGGL(build_joint_kernel<F16>, grid, block, 0, st, raw, S, (uint16_t *)joint, slack); break;

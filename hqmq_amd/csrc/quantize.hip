@@ -20,7 +20,7 @@
 // overflow, or whose direction is not finite, score all 24*S rows instead.
 //
 // Compiled with -ffp-contract=off; fused multiply-adds are written explicitly.
-#include "common.h"
+#include "quantize_common.h"
 #include <type_traits>
 
 namespace hqmq {
@@ -28,65 +28,8 @@ namespace hqmq {
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 
-constexpr int kQThreads = 256;
 constexpr int kSCap = 32;  // candidate secondaries kept per lane
 constexpr int kKCap = 24;  // candidate codewords kept per lane
-
-// Maximum over groups of `n` neighbouring lanes (n a power of two up to 64), every lane of a group receiving it:
-// lane permutations inside the vector unit (quad, half-row and row mirrors, then the 16- and 32-lane row swaps).
-// The operands are ordinary numbers or -inf (no NaN), as unsigned bit patterns of non-negative floats order like the
-// values, the same routine serves both.
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, false);
-}
-template <class T, class MAX>
-__device__ __forceinline__ T group_max(T x, int n, MAX mx) {
-    auto step = [&](uint32_t other) { x = mx(x, __builtin_bit_cast(T, other)); };
-    if (n >= 2) step(dpp_u32<0xB1>(__builtin_bit_cast(uint32_t, x)));       // quad_perm [1,0,3,2]
-    if (n >= 4) step(dpp_u32<0x4E>(__builtin_bit_cast(uint32_t, x)));       // quad_perm [2,3,0,1]
-    if (n >= 8) step(dpp_u32<0x141>(__builtin_bit_cast(uint32_t, x)));      // row_half_mirror
-    if (n >= 16) step(dpp_u32<0x140>(__builtin_bit_cast(uint32_t, x)));     // row_mirror
-    if (n >= 32) {
-        const uint32_t b = __builtin_bit_cast(uint32_t, x);
-        const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-        x = mx(__builtin_bit_cast(T, (uint32_t)r[0]), __builtin_bit_cast(T, (uint32_t)r[1]));
-    }
-    if (n >= 64) {
-        const uint32_t b = __builtin_bit_cast(uint32_t, x);
-        const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-        x = mx(__builtin_bit_cast(T, (uint32_t)r[0]), __builtin_bit_cast(T, (uint32_t)r[1]));
-    }
-    return x;
-}
-
-struct QParams {
-    const void *x;
-    int64_t xsb, xsh, xst;
-    int B, H, T, n;
-    const void *joint;
-    const float *slack;
-    int S, qmax;
-    int32_t *idx_out, *rq_out;
-    void *rmax_out, *dense_out;
-    const void *thr;
-    uint8_t *mask_out;
-    uint8_t *main_plane, *aux_plane, *flag_plane;
-    void *scale_plane;
-    int64_t t_cap;
-    int t_off;
-    const int32_t *pos;
-    int idx_bits, main_bits, aux_bits;
-    int tokens_per_block;
-    int32_t *stats;
-    uint32_t *scale_max;
-    // sideband compaction in the same launch (compact != 0): see the end of quantize_body
-    int compact;
-    void *sideband;
-    int64_t sb_cap;
-    int32_t *sb_tile_off, *sb_count, *overflow;
-    uint16_t *sb_coord;
-};
 
 __device__ __forceinline__ void rotate_conj(const float u[4], float qw, float qx, float qy, float qz, float v[4]) {
     // v = u * conj(q)
@@ -148,80 +91,22 @@ __device__ __forceinline__ float exact2_of(const float v[4], int p) {
     return (t0 + t1) + (t2 + t3);
 }
 
-template <class D>
-__device__ __forceinline__ float ref_score(const float u[4], const typename D::storage *row) {
-    float j0 = D::load(row), j1 = D::load(row + 1), j2 = D::load(row + 2), j3 = D::load(row + 3);
-    float acc = u[0] * j0;
-    acc = fmaf(u[1], j1, acc);
-    acc = fmaf(u[2], j2, acc);
-    acc = fmaf(u[3], j3, acc);
-    return D::rnd(acc);
-}
-
-// argmax over all K rows with torch's rule: first maximum, NaN counts as maximum.
-template <class D>
-__device__ int brute_argmax(const float u[4], const typename D::storage *jh, int K) {
-    int best = 0;
-    float bs = 0.f;
-    for (int k = 0; k < K; k++) {
-        float s = ref_score<D>(u, jh + (size_t)k * 4);
-        if (is_nan(s)) return k;
-        if (k == 0 || s > bs) { bs = s; best = k; }
-    }
-    return best;
-}
-
-// Little-endian bit stream of `w`-bit fields (field i = vals[base + i] >> shift, masked)
-// -> output byte `byte` of the row.
-template <int W>
-__device__ __forceinline__ uint8_t gather_byte_w(const uint32_t *vals, int count, int w, int shift, int byte) {
-    const int ww = W ? W : w;       // W != 0: the width is a constant and the divisions below fold into shifts
-    uint32_t out = 0;
-    uint32_t fmask = (ww >= 32) ? 0xffffffffu : ((1u << ww) - 1u);
-#pragma unroll
-    for (int bit = 0; bit < 8; bit++) {
-        int pos = byte * 8 + bit;
-        int i = pos / ww, o = pos - i * ww;
-        if (i < count) out |= ((((vals[i] >> shift) & fmask) >> o) & 1u) << bit;
-    }
-    return (uint8_t)out;
-}
-__device__ __forceinline__ uint8_t gather_byte(const uint32_t *vals, int count, int w, int shift, int byte) {
-    switch (w) {        // the widths the layout rule produces (main 8 / 12, aux 1..3, flags 1)
-        case 1: return gather_byte_w<1>(vals, count, w, shift, byte);
-        case 2: return gather_byte_w<2>(vals, count, w, shift, byte);
-        case 3: return gather_byte_w<3>(vals, count, w, shift, byte);
-        case 8: return gather_byte_w<8>(vals, count, w, shift, byte);
-        case 12: return gather_byte_w<12>(vals, count, w, shift, byte);
-        default: return gather_byte_w<0>(vals, count, w, shift, byte);
-    }
-}
-
-// SPLIT (single-token appends, 16-bit dtypes, n a power of two): the block's 256 / n token slots all hold the one new
-// token of (b, h) and share its secondaries between them: slot w scores s = w, w + slots, ...  A decode-step append is
-// one wavefront's serial instruction stream otherwise; this divides the search part of it by the number of slots.
-// The slots' candidates are merged exactly: the filter threshold comes from the maximum over all slots, the winner
-// is the highest exact score with the lowest index, as in the unsplit search.
-template <class D, int ALGO, bool SPLIT = false>
+template <class D, int ALGO, bool ROWS>
 __device__ __forceinline__ void quantize_body(const QParams &a) {
     using ST = typename D::storage;
-    static_assert(!SPLIT || (ALGO == 0 && D::code != HQMQ_F32), "the split search is the MFMA search");
     extern __shared__ float sec[];  // [S][4] secondaries, then [S][4] fp16 columns of their rotation matrices
     uint2 *rot = reinterpret_cast<uint2 *>(sec + 4 * a.S);
-    __shared__ float radius_sh[kQThreads];
     __shared__ uint32_t code_sh[kQThreads];
-    __shared__ uint32_t mask_sh[kQThreads];
+    __shared__ uint32_t aux_sh[kQThreads];
     __shared__ uint16_t slist[kSCap][kQThreads];
     __shared__ uint16_t klist[kKCap][kQThreads];
 
     const int tid = threadIdx.x;
     const int bh = blockIdx.y, b = bh / a.H, h = bh - b * a.H;
     const int n = a.n, S = a.S, K = 24 * S;
-    const int tok_local = tid / n, c = tid - tok_local * n;       // SPLIT: tok_local is the slot
-    const int t = SPLIT ? (int)blockIdx.x : blockIdx.x * a.tokens_per_block + tok_local;
+    const int tok_local = tid / n, c = tid - tok_local * n;
+    const int t = blockIdx.x * a.tokens_per_block + tok_local;
     const bool active = tok_local < a.tokens_per_block && t < a.T;
-    const bool writer = !SPLIT || tok_local == 0;                 // one slot stores the results
-    const int slots = SPLIT ? kQThreads / n : 1, s_first = SPLIT ? tok_local : 0;
     const ST *jh = (const ST *)a.joint + (size_t)h * K * 4;
 
     for (int i = tid; i < S * 4; i += kQThreads) sec[i] = D::load(jh + i);  // rows k = s are q_s itself
@@ -241,16 +126,13 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
         }
     }
 
-    float xv[4] = {0.f, 0.f, 0.f, 0.f};
-    if (active) {
-        const ST *xp = (const ST *)a.x + b * a.xsb + h * a.xsh + (int64_t)t * a.xst + c * 4;
-        for (int j = 0; j < 4; j++) xv[j] = D::load(xp + j);
-    }
-    const float nrm = D::rnd(norm4(xv[0], xv[1], xv[2], xv[3]));
+    RawChunk<D> raw = {};
+    if (active) raw.load((const ST *)a.x + b * a.xsb + h * a.xsh + (int64_t)t * a.xst + c * 4, a.vec_in);
+    const float xv[4] = {raw.get(0), raw.get(1), raw.get(2), raw.get(3)};
+    const float nrm = chunk_norm_d<D>(xv[0], xv[1], xv[2], xv[3]);
     const float r = clamp_min_d<D>(nrm, 1e-8f);
-    float u[4];
-    for (int j = 0; j < 4; j++) u[j] = D::rnd(xv[j] / r);
-    radius_sh[tid] = r;
+    float u[4] = {xv[0], xv[1], xv[2], xv[3]};
+    div4_d<D>(u, r);
     __syncthreads();
 
     // ---- codeword search ----
@@ -282,21 +164,20 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
             // become a bit mask (a compare and an add-with-carry each) and go into the list of the re-score below.  A
             // threshold that has moved above the maximum before the block leaves everything listed before below the
             // final threshold: the list starts over.
-            const int iters = (S + slots - 1) / slots;          // of the slot with the most secondaries (wave-uniform)
-            uint2 a_next = acol[4 * min(s_first, S - 1)];
+            uint2 a_next = acol[0];
             float thr = -INFINITY;
             auto scan_block = [&](int i0, auto tail) -> uint32_t {
                 float b2v[32];
 #pragma unroll
                 for (int i = 0; i < 32; i++) {
-                    const int sn = s_first + (i0 + i + 1) * slots;
+                    const int sn = i0 + i + 1;
                     const half4 am = __builtin_bit_cast(half4, a_next);
                     // the next column is on its way during this one; inside a whole block it exists, so its address is
                     // the block's base plus a constant
                     a_next = (decltype(tail)::value || i == 31) ? acol[4 * min(sn, S - 1)] : acol[4 * sn];
                     const float4v vv = __builtin_amdgcn_mfma_f32_4x4x4f16(am, ub, float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                     float b2 = best2_mfma(vv[0], vv[1], vv[2], vv[3]);
-                    if (decltype(tail)::value && sn - slots >= S) b2 = -INFINITY;      // behind the slot's last secondary
+                    if (decltype(tail)::value && sn > S) b2 = -INFINITY;      // behind the last secondary
                     b2v[i] = b2;
                     // the running maximum takes two scores at a time (all ordinary numbers or -inf here)
                     if (i & 1) asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m2) : "v"(m2), "v"(b2v[i - 1]), "v"(b2));
@@ -306,22 +187,17 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
 #pragma unroll
                 for (int i = 31; i >= 0; i--)       // word = 2 word + (score >= thr): iteration i ends up in bit i
                     asm("v_cmp_ge_f32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(word) : "v"(b2v[i]), "v"(thr) : "vcc");
-                if (decltype(tail)::value) {        // a slot whose secondaries end inside the block: only those count
-                    const int left = S - s_first - i0 * slots;
-                    const int valid = left <= 0 ? 0 : min((left + slots - 1) / slots, 32);
-                    word &= valid >= 32 ? ~0u : (1u << valid) - 1u;
-                }
+                if (decltype(tail)::value) word &= (1u << (S - i0)) - 1u;       // fewer than 32 are left
                 return word;
             };
-            for (int i0 = 0; i0 < iters; i0 += 32) {
+            for (int i0 = 0; i0 < S; i0 += 32) {
                 const float m_before = m2;
-                const bool whole = (slots - 1) + (i0 + 31) * slots < S;     // every slot has all 32 secondaries of this block
-                uint32_t bits = whole ? scan_block(i0, std::false_type{}) : scan_block(i0, std::true_type{});
+                uint32_t bits = i0 + 32 <= S ? scan_block(i0, std::false_type{}) : scan_block(i0, std::true_type{});
                 if (m_before < thr) cnt = 0;
                 while (bits) {
                     const int i = __builtin_ctz(bits);
                     bits &= bits - 1u;
-                    if (cnt < kSCap) slist[cnt][tid] = (uint16_t)(s_first + (i0 + i) * slots);
+                    if (cnt < kSCap) slist[cnt][tid] = (uint16_t)(i0 + i);
                     cnt++;
                 }
             }
@@ -338,13 +214,6 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
                 }
                 m2 = fmaxf(m2, b2);
             }
-        }
-        if (SPLIT) {        // the maximum over all slots of this chunk (every slot holds the same direction)
-            float *m2_sh = reinterpret_cast<float *>(code_sh);
-            m2_sh[tid] = m2;
-            __syncthreads();
-            for (int w = 0; w < slots; w++) m2 = fmaxf(m2, m2_sh[w * n + c]);
-            __syncthreads();
         }
         float bs = -INFINITY;
         int bk = 0x7fffffff;
@@ -401,248 +270,34 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
             }
         }
         if (brute) idx = brute_argmax<D>(u, jh, K);
-        if (SPLIT) {
-            // merge the slots: a slot that fell back to the exhaustive search holds the answer; otherwise the highest
-            // exact score wins, the lowest index among equals; no candidate anywhere (all-zero direction) -> index 0
-            float *bs_sh = reinterpret_cast<float *>(code_sh);
-            int *bk_sh = reinterpret_cast<int *>(mask_sh);
-            bs_sh[tid] = bs;
-            bk_sh[tid] = brute ? (idx | (int)0x80000000) : (search ? bk : 0x7fffffff);
-            __syncthreads();
-            float ms = -INFINITY;
-            int mk = 0x7fffffff;
-            bool exact = false;
-            for (int w = 0; w < slots; w++) {
-                const int kw = bk_sh[w * n + c];
-                const float sw = bs_sh[w * n + c];
-                if (kw < 0) {
-                    if (!exact) { exact = true; mk = kw & 0x7fffffff; }
-                } else if (!exact && kw != 0x7fffffff && (sw > ms || (sw == ms && kw < mk))) {
-                    ms = sw;
-                    mk = kw;
-                }
-            }
-            idx = mk == 0x7fffffff ? 0 : mk;
-            __syncthreads();
-        }
         if (a.stats && active) {
-            if (brute && writer) atomicAdd(a.stats, 1);      // once per chunk, also when its slots split the search
+            if (brute) atomicAdd(a.stats, 1);
             if (search && !brute) atomicAdd(a.stats + 1, cnt);
         }
     }
 
-    // ---- per-token scale and radius code ----
-    float rm = -INFINITY;
-    bool rm_nan = false;
-    if ((n & (n - 1)) == 0 && n <= 64) {
-        // the n lanes of a token sit side by side inside one wavefront
-        const int lane = tid & 63;
-        const uint64_t tok_lanes = n == 64 ? ~0ull : ((1ull << n) - 1ull) << (lane / n * n);
-        rm_nan = (__builtin_amdgcn_ballot_w64(is_nan(r)) & tok_lanes) != 0ull;
-        rm = group_max(is_nan(r) ? -INFINITY : r, n, [](float p, float q) { return q > p ? q : p; });
-    } else {
-        const int base = tok_local * n;
-        for (int i = 0; i < n; i++) {
-            float o = (base + i < kQThreads) ? radius_sh[base + i] : 0.f;
-            if (is_nan(o)) rm_nan = true;
-            else if (o > rm) rm = o;
-        }
-    }
-    rm = clamp_min_d<D>(rm_nan ? NAN : rm, 1e-8f);
-    const float qmaxf = (float)a.qmax;
-    const float scale = D::rnd(rm / qmaxf);
-    float qf = rintf(D::rnd(r / scale));
-    if (!is_nan(qf)) qf = fminf(fmaxf(qf, 0.f), qmaxf);
-    const int rq = is_nan(qf) ? 0 : (int)qf;
-
-    bool flagged = false;
-    if (a.thr) flagged = nrm > D::load((const ST *)a.thr + h);
-
-    if (active && writer) {
-        const size_t o = (((size_t)b * a.H + h) * a.T + t) * n + c;
-        if (a.idx_out) a.idx_out[o] = idx;
-        if (a.rq_out) a.rq_out[o] = rq;
-        if (a.mask_out) a.mask_out[o] = flagged ? 1 : 0;
-        if (a.rmax_out && c == 0) D::store((ST *)a.rmax_out + o / n, rm);
-        if (a.dense_out) {
-            ST *dst = (ST *)a.dense_out + o * 4;
-            if (flagged) {
-                const ST *xp = (const ST *)a.x + b * a.xsb + h * a.xsh + (int64_t)t * a.xst + c * 4;
-                for (int j = 0; j < 4; j++) dst[j] = xp[j];
-            } else {
-                const float rqs = D::rnd(qf * scale);
-                const ST *row = jh + (size_t)idx * 4;
-                for (int j = 0; j < 4; j++) D::store(dst + j, D::rnd(rqs * D::load(row + j)));
-            }
-        }
-    }
-
-    // ---- packed rows ----
-    if (a.main_plane || a.flag_plane || a.scale_plane) {
-        const int64_t row = (a.pos ? a.pos[b] : 0) + a.t_off + t;
-        const bool row_ok = active && writer && row >= 0 && row < a.t_cap;  // a bad pos[] must not write outside the plane
-        // Sideband compaction in the same launch, for appends whose new rows of a (b, h) all sit in this block
-        // (T <= tokens_per_block; n a power of two, so the lanes of a token share a wavefront).  Entries, tile
-        // offsets and counters come out as the in-order compaction kernel leaves them: flagged chunks in
-        // (row, chunk) order behind the entries already there, the offset of a tile = the count before its
-        // first row.  The entry slots are worked out before the rows are packed: a flagged chunk that finds the
-        // sideband full is packed as a plain chunk (its radius code, no flag) instead of decoding to zero.
-        bool keep = flagged;            // stays an outlier in the packed planes
-        bool entry = false;             // this lane writes a sideband entry
-        int ent_slot = 0, tile_first = 0, ent_total = 0;
-        if (a.compact) {
-            __syncthreads();            // radius_sh is free from here on
-            const bool f = row_ok && flagged;
-            const uint64_t m = __builtin_amdgcn_ballot_w64(f);
-            const int lane = tid & 63;
-            const uint64_t tok_bits = n == 64 ? ~0ull : ((1ull << n) - 1ull) << ((lane / n) * n);
-            const int before_c = __popcll(m & tok_bits & ((1ull << lane) - 1ull));
-            int *cnt_sh = reinterpret_cast<int *>(radius_sh);           // free since the scales were taken
-            if (c == 0 && tok_local < a.tokens_per_block) cnt_sh[tok_local] = __popcll(m & tok_bits);
-            const int base = a.sb_count[(size_t)b * a.H + h];           // read by every thread before the barrier,
-            __syncthreads();                                            // rewritten by one thread at the end
-            int mine = base, total = base;
-            for (int i = 0; i < a.T; i++) {
-                const int ci = cnt_sh[i];
-                if (i < tok_local) mine += ci;
-                total += ci;
-            }
-            tile_first = mine;
-            ent_total = total;
-            ent_slot = mine + before_c;
-            entry = f && ent_slot < a.sb_cap;
-            if (f && !entry) {
-                keep = false;
-                *a.overflow = 1;
-            }
-        }
-        // a flagged chunk is read from the sideband; its packed code keeps idx with radius code 0, which decodes to zero
-        code_sh[tid] = (uint32_t)idx | ((uint32_t)(keep ? 0 : rq) << a.idx_bits);
-        mask_sh[tid] = keep ? 1u : 0u;
-        __syncthreads();
-        // one-bit planes (flags, a one-bit aux field) of tokens whose lanes sit side by side in a wavefront come
-        // straight from a ballot: the token's n bits are n / 8 whole bytes of it
-        const bool side_by_side = (n & (n - 1)) == 0 && n >= 8 && n <= 64;
-        const int lane_base = (tid & 63) / n * n;
-        const uint64_t aux_bits1 = __builtin_amdgcn_ballot_w64(((code_sh[tid] >> a.main_bits) & 1u) != 0u);
-        const uint64_t flag_bits1 = __builtin_amdgcn_ballot_w64(keep);
-        if (row_ok) {
-            const size_t prow = ((size_t)b * a.H + h) * a.t_cap + row;
-            const uint32_t *codes = code_sh + tok_local * n;
-            if (a.main_plane) {
-                const int rb = (n * a.main_bits + 7) >> 3;
-                uint8_t *dst = a.main_plane + prow * rb;
-                if (a.main_bits == 16) {
-                    reinterpret_cast<uint16_t *>(dst)[c] = (uint16_t)codes[c];   // one code per lane
-                } else if (a.main_bits == 12 && !(n & 1)) {
-                    if (!(c & 1)) {                                             // two codes = three bytes
-                        const uint32_t two = (codes[c] & 0xfffu) | ((codes[c + 1] & 0xfffu) << 12);
-                        uint8_t *d = dst + (c >> 1) * 3;
-                        d[0] = (uint8_t)two;
-                        d[1] = (uint8_t)(two >> 8);
-                        d[2] = (uint8_t)(two >> 16);
-                    }
-                } else {
-                    for (int byte = c; byte < rb; byte += n) dst[byte] = gather_byte(codes, n, a.main_bits, 0, byte);
-                }
-            }
-            if (a.aux_plane && a.aux_bits) {
-                const int rb = (n * a.aux_bits + 7) >> 3;
-                uint8_t *dst = a.aux_plane + prow * rb;
-                if (a.aux_bits == 1 && side_by_side) {
-                    if (c < rb) dst[c] = (uint8_t)(aux_bits1 >> (lane_base + 8 * c));
-                } else {
-                    for (int byte = c; byte < rb; byte += n) dst[byte] = gather_byte(codes, n, a.aux_bits, a.main_bits, byte);
-                }
-            }
-            if (a.flag_plane) {
-                const int rb = (n + 7) >> 3;
-                uint8_t *dst = a.flag_plane + prow * rb;
-                if (side_by_side) {
-                    if (c < rb) dst[c] = (uint8_t)(flag_bits1 >> (lane_base + 8 * c));
-                } else {
-                    for (int byte = c; byte < rb; byte += n) dst[byte] = gather_byte(mask_sh + tok_local * n, n, 1, 0, byte);
-                }
-            }
-            if (a.scale_plane && c == 0) D::store((ST *)a.scale_plane + prow, rm);
-        }
-        if (a.scale_max && a.scale_plane) {
-            // the largest finite scale written so far, for the attention kernels' range guard: the wavefront's maximum,
-            // and an atomic only when it raises the value (after the first blocks it hardly ever does)
-            uint32_t mine = (row_ok && c == 0 && rm < INFINITY) ? __float_as_uint(rm) : 0u;     // scales are positive: bits order like values
-            mine = group_max(mine, 64, [](uint32_t p, uint32_t q) { return max(p, q); });
-            if ((tid & 63) == 0 && mine > __hip_atomic_load(a.scale_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                atomicMax(a.scale_max, mine);
-        }
-        if (a.compact) {
-            const size_t bhs = (size_t)b * a.H + h;
-            if (row_ok) {
-                const int64_t tiles = (a.t_cap + kTile - 1) / kTile;
-                if (c == 0 && (row & (kTile - 1)) == 0) a.sb_tile_off[bhs * tiles + (row >> 4)] = tile_first;
-                if (entry) {
-                    const ST *xp = (const ST *)a.x + b * a.xsb + h * a.xsh + (int64_t)t * a.xst + c * 4;
-                    ST *dst = (ST *)a.sideband + (bhs * a.sb_cap + ent_slot) * 4;
-                    for (int j = 0; j < 4; j++) dst[j] = xp[j];
-                    if (a.sb_coord) a.sb_coord[bhs * a.sb_cap + ent_slot] = (uint16_t)(((row & (kTile - 1)) << 8) | c);
-                }
-            }
-            if (tid == 0) a.sb_count[bhs] = ent_total;
-        }
-    }
+    ChunkSink<D, kQThreads, ROWS, kUnpacked | kPlanes | kCompact, 0> sink(a, b, h, tok_local, c, code_sh, aux_sh);
+    sink.put(blockIdx.x * a.tokens_per_block, active, raw, nrm, r, idx, jh + (size_t)idx * 4);
+    sink.done();
 }
 
-template <class D, int ALGO>
+template <class D, int ALGO, bool ROWS>
 __global__ __launch_bounds__(kQThreads) void quantize_kernel(QParams a) {
-    quantize_body<D, ALGO>(a);
-}
-
-// The K and the V rows of one append in one launch (same shapes): blockIdx.z picks the tensor.  A single-token
-// append is latency-bound (32 lanes per block for a few microseconds), so the two run side by side for free.
-struct QPair {
-    QParams p[2];       // K, V
-};
-// (indexed in the kernel-argument segment: one set of scalar registers, not a select per field of two structs)
-template <class D, bool SPLIT>
-__global__ __launch_bounds__(kQThreads) void quantize_pair_kernel(QPair kv) {
-    quantize_body<D, 0, SPLIT>(kv.p[blockIdx.z]);
-}
-template <class D>
-__global__ __launch_bounds__(kQThreads) void quantize_split_kernel(QParams a) {
-    quantize_body<D, 0, true>(a);
-}
-
-// one new token per sequence, 16-bit dtype, the lanes of a token inside a wavefront: the split search
-template <class D>
-static bool use_split(const QParams &p, int algo) {
-    return sizeof(typename D::storage) == 2 && algo == 0 && p.T == 1 && p.n >= 4 && p.n <= 64 && !(p.n & (p.n - 1));
+    quantize_body<D, ALGO, ROWS>(a);
 }
 
 template <class D>
 static int launch_quantize(const QParams &p, int algo, hipStream_t st) {
     dim3 grid((p.T + p.tokens_per_block - 1) / p.tokens_per_block, p.B * p.H), block(kQThreads);
     size_t shmem = (size_t)p.S * 4 * sizeof(float) + (size_t)p.S * 4 * sizeof(uint2);
-    if constexpr (sizeof(typename D::storage) == 2) {
-        if (use_split<D>(p, algo)) {
-            hipLaunchKernelGGL(quantize_split_kernel<D>, grid, block, shmem, st, p);
-            return hip_status(hipGetLastError());
-        }
+    const bool rows = !(p.n & (p.n - 1)) && p.n <= 64;
+    if (algo == 1) {
+        if (rows) hipLaunchKernelGGL((quantize_kernel<D, 1, true>), grid, block, shmem, st, p);
+        else hipLaunchKernelGGL((quantize_kernel<D, 1, false>), grid, block, shmem, st, p);
+    } else {
+        if (rows) hipLaunchKernelGGL((quantize_kernel<D, 0, true>), grid, block, shmem, st, p);
+        else hipLaunchKernelGGL((quantize_kernel<D, 0, false>), grid, block, shmem, st, p);
     }
-    if (algo == 1) hipLaunchKernelGGL((quantize_kernel<D, 1>), grid, block, shmem, st, p);
-    else hipLaunchKernelGGL((quantize_kernel<D, 0>), grid, block, shmem, st, p);
-    return hip_status(hipGetLastError());
-}
-
-template <class D>
-static int launch_quantize_pair(const QParams &k, const QParams &v, hipStream_t st) {
-    dim3 grid((k.T + k.tokens_per_block - 1) / k.tokens_per_block, k.B * k.H, 2), block(kQThreads);
-    size_t shmem = (size_t)k.S * 4 * sizeof(float) + (size_t)k.S * 4 * sizeof(uint2);
-    if constexpr (sizeof(typename D::storage) == 2) {
-        if (use_split<D>(k, 0) && use_split<D>(v, 0)) {
-            hipLaunchKernelGGL((quantize_pair_kernel<D, true>), grid, block, shmem, st, QPair{{k, v}});
-            return hip_status(hipGetLastError());
-        }
-    }
-    hipLaunchKernelGGL((quantize_pair_kernel<D, false>), grid, block, shmem, st, QPair{{k, v}});
     return hip_status(hipGetLastError());
 }
 
@@ -655,7 +310,7 @@ extern "C" int hqmq_layout_bits(int S, int radius_bits, int *idx_bits, int *main
 }
 
 // Checks one call's arguments and fills the kernel parameters; *empty is set for T == 0 (nothing to launch).
-static int fill_qparams(const hqmq_quantize_args *a, QParams *out, bool *empty) {
+static int fill_qparams(const hqmq_quantize_args *a, const void *grid, QParams *out, bool *empty) {
     *empty = false;
     if (!a || !a->x || !a->joint) return HQMQ_ERR_NULL;
     if (a->algo == 0 && !a->slack) return HQMQ_ERR_NULL;
@@ -693,6 +348,15 @@ static int fill_qparams(const hqmq_quantize_args *a, QParams *out, bool *empty) 
     p.scale_max = a->scale_max_bits;
     p.compact = 0;
     p.sideband = nullptr; p.sb_cap = 0; p.sb_tile_off = p.sb_count = p.overflow = nullptr; p.sb_coord = nullptr;
+    const int elt = a->dtype == HQMQ_F32 ? 4 : 2;
+    p.vec_in = !(((uintptr_t)a->x | (uintptr_t)(a->x_stride_b * elt) | (uintptr_t)(a->x_stride_h * elt) | (uintptr_t)(a->x_stride_t * elt)) & (4 * elt - 1));
+    p.vec_out = !((uintptr_t)a->dense_out & (4 * elt - 1));
+    p.vec_rows = !(((uintptr_t)a->main_plane | (uintptr_t)a->aux_plane | (uintptr_t)a->flag_plane) & 3);
+    if (grid && ((uintptr_t)grid & 15)) return HQMQ_ERR_ALIGN;
+    const int64_t cells = search_grid_blocks(a->secondary_size, a->dtype);
+    p.grid = cells && !((uintptr_t)a->joint & (4 * elt - 1)) ? (const uint4 *)grid : nullptr;      // (rows of the table are read as vectors)
+    p.grid_stride = cells;
+    p.iters = 1;
     return HQMQ_OK;
 }
 
@@ -714,36 +378,36 @@ static int launch_one_tensor(const QParams &p, int dtype, int algo, hipStream_t 
     }
 }
 
-extern "C" int hqmq_quantize(const hqmq_quantize_args *a, void *stream) {
+extern "C" int hqmq_quantize_grid(const hqmq_quantize_args *a, const void *grid, void *stream) {
     QParams p;
     bool empty;
-    const int rc = fill_qparams(a, &p, &empty);
+    const int rc = fill_qparams(a, grid, &p, &empty);
     if (rc || empty) return rc;
+    if (p.grid && a->algo == 0) return launch_quantize_grid(QPair{{p, p}}, 1, a->dtype, (hipStream_t)stream);
     return launch_one_tensor(p, a->dtype, a->algo, (hipStream_t)stream);
 }
 
-int hqmq::quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v, const CompactCall *ck, const CompactCall *cv,
-                       bool compacted[2], hipStream_t st) {
-    QParams pk, pv;
-    bool ek, ev;
-    int rc = fill_qparams(k, &pk, &ek);
-    if (rc) return rc;
-    rc = fill_qparams(v, &pv, &ev);
-    if (rc) return rc;
-    compacted[0] = !ek && take_compaction(pk, ck);
-    compacted[1] = !ev && take_compaction(pv, cv);
-    const bool same = !ek && !ev && k->dtype == v->dtype && k->B == v->B && k->H == v->H && k->T == v->T &&
-                      k->n_chunks == v->n_chunks && k->secondary_size == v->secondary_size && k->algo == 0 && v->algo == 0;
-    if (same) {
-        switch (k->dtype) {
-            case HQMQ_F32: return launch_quantize_pair<F32>(pk, pv, st);
-            case HQMQ_F16: return launch_quantize_pair<F16>(pk, pv, st);
-            default: return launch_quantize_pair<BF16>(pk, pv, st);
-        }
+extern "C" int hqmq_quantize(const hqmq_quantize_args *a, void *stream) { return hqmq_quantize_grid(a, nullptr, stream); }
+
+int hqmq::quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v, const void *const grids[2], const CompactCall *ck,
+                       const CompactCall *cv, bool compacted[2], hipStream_t st) {
+    QParams p[2];
+    bool empty[2];
+    const hqmq_quantize_args *a[2] = {k, v};
+    const CompactCall *cc[2] = {ck, cv};
+    for (int i = 0; i < 2; i++) {
+        const int rc = fill_qparams(a[i], grids[i], &p[i], &empty[i]);
+        if (rc) return rc;
+        compacted[i] = !empty[i] && take_compaction(p[i], cc[i]);
     }
-    if (!ek) {
-        rc = launch_one_tensor(pk, k->dtype, k->algo, st);
+    const bool by_cells[2] = {p[0].grid && k->algo == 0, p[1].grid && v->algo == 0};
+    if (!empty[0] && !empty[1] && by_cells[0] && by_cells[1] && k->dtype == v->dtype && k->B == v->B && k->H == v->H && k->T == v->T &&
+        k->n_chunks == v->n_chunks && k->secondary_size == v->secondary_size)
+        return launch_quantize_grid(QPair{{p[0], p[1]}}, 2, k->dtype, st);
+    for (int i = 0; i < 2; i++) {
+        if (empty[i]) continue;
+        const int rc = by_cells[i] ? launch_quantize_grid(QPair{{p[i], p[i]}}, 1, a[i]->dtype, st) : launch_one_tensor(p[i], a[i]->dtype, a[i]->algo, st);
         if (rc) return rc;
     }
-    return ev ? HQMQ_OK : launch_one_tensor(pv, v->dtype, v->algo, st);
+    return HQMQ_OK;
 }

@@ -20,7 +20,9 @@ def _dt(t: torch.Tensor) -> int:
 
 
 def build_joint(raw_hs4: torch.Tensor, dtype: torch.dtype):
-    """(H, S, 4) fp32 raw secondaries on the GPU -> (joint (H, 24S, 4) in dtype, slack (H,) fp32)."""
+    """(H, S, 4) fp32 raw secondaries on the GPU -> (joint (H, 24S, 4) in dtype, slack (H,) fp32).
+    The table's cell lists for the quantize kernels (see include/hqmq_amd.h) are built along and travel as an attribute
+    of `slack`; a slack tensor without it quantizes through the scan over the secondaries, with the same results."""
     L.require_gpu(raw_hs4, "raw")
     raw = raw_hs4.detach().to(torch.float32).contiguous()
     H, S, _ = raw.shape
@@ -29,7 +31,16 @@ def build_joint(raw_hs4: torch.Tensor, dtype: torch.dtype):
     with torch.cuda.device(raw.device):
         L.check(L.lib().hqmq_build_joint(L.ptr(raw), C.c_int(H), C.c_int(S), C.c_int(L.DT_CODE[dtype]), L.ptr(joint),
                                          L.ptr(slack), L.stream_ptr(raw.device)), "hqmq_build_joint")
+        nbytes = int(L.lib().hqmq_search_grid_bytes(C.c_int(H), C.c_int(S), C.c_int(L.DT_CODE[dtype])))
+        if nbytes:
+            slack.hqmq_grid = grid = torch.empty(nbytes, dtype=torch.uint8, device=raw.device)
+            L.check(L.lib().hqmq_build_search_grid(L.ptr(joint), C.c_int(H), C.c_int(S), C.c_int(L.DT_CODE[dtype]),
+                                                   L.ptr(grid), L.i64(nbytes), L.stream_ptr(raw.device)), "hqmq_build_search_grid")
     return joint, slack
+
+
+def _grid(slack: Optional[torch.Tensor]):
+    return L.ptr(getattr(slack, "hqmq_grid", None))
 
 
 def _strided_x(x: torch.Tensor):
@@ -99,7 +110,7 @@ def quantize(x: torch.Tensor, joint: torch.Tensor, slack: Optional[torch.Tensor]
     a.stats = L.ptr(stats)
     if T > 0:
         with torch.cuda.device(dev):
-            L.check(L.lib().hqmq_quantize(C.byref(a), L.stream_ptr(dev)), "hqmq_quantize")
+            L.check(L.lib().hqmq_quantize_grid(C.byref(a), _grid(slack), L.stream_ptr(dev)), "hqmq_quantize_grid")
     if "mask8" in out:
         out["mask"] = out.pop("mask8").bool()
     return out
@@ -241,7 +252,8 @@ def append_kv(k: torch.Tensor, v: torch.Tensor, k_cache, v_cache, k_joint, k_sla
         args.append(a)
         counts.append(cnt)
     with torch.cuda.device(dev):
-        L.check(L.lib().hqmq_append_kv(C.byref(args[0]), C.byref(args[1]), L.stream_ptr(dev)), "hqmq_append_kv")
+        L.check(L.lib().hqmq_append_kv_grid(C.byref(args[0]), C.byref(args[1]), _grid(k_slack), _grid(v_slack), L.stream_ptr(dev)),
+                "hqmq_append_kv_grid")
     return counts[0], counts[1]
 
 

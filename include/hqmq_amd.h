@@ -104,6 +104,18 @@ typedef struct hqmq_quantize_args {
 } hqmq_quantize_args;
 int hqmq_quantize(const hqmq_quantize_args *a, void *stream);
 
+/* Cell lists of a codebook: for every box of a grid over the directions next to one Hurwitz unit, the codewords that
+ * can win the reference's rounded comparison there (see csrc/quantize_grid.hip).  Worked out once per codebook, they
+ * replace the quantize kernel's scan over the secondaries; the codes are the same, bit for bit.
+ *   hqmq_search_grid_bytes    size for H heads of S secondaries; 0 where the lists do not exist (S > 341)
+ *   joint                     as hqmq_build_joint left it
+ *   grid                      (out) hqmq_search_grid_bytes bytes, 16-byte aligned */
+int64_t hqmq_search_grid_bytes(int H, int S, int dtype);
+int hqmq_build_search_grid(const void *joint, int H, int S, int dtype, void *grid, int64_t grid_bytes, void *stream);
+/* hqmq_quantize with the codebook's cell lists (NULL: without); algo and every other argument as there.  stats[1] counts
+ * the chunks that were searched through the lists. */
+int hqmq_quantize_grid(const hqmq_quantize_args *a, const void *grid, void *stream);
+
 /* Med3x statistics: per-head median of the chunk norms of one call and the
  * threshold RNE_D(median * mult).  Replaces the torch.quantile half of
  * OutlierAwareHQMQQuantizer._qdq (src/quantizers/outlier_aware.py:60-69).
@@ -163,6 +175,8 @@ typedef struct hqmq_append_args {
     uint16_t *sb_coord;                                /* may be NULL */
 } hqmq_append_args;
 int hqmq_append_kv(const hqmq_append_args *k, const hqmq_append_args *v, void *stream);
+/* The same with the cell lists of the two codebooks (hqmq_build_search_grid; NULL: without). */
+int hqmq_append_kv_grid(const hqmq_append_args *k, const hqmq_append_args *v, const void *k_grid, const void *v_grid, void *stream);
 
 /* Dense decode of unpacked codes: out = joint[h, idx] * ((rq * rs) / qmax) in D.
  * Replaces hqmq_decode_triton (src/quantizers/hqmq_kernel.py:102-132) with the
