@@ -77,12 +77,17 @@ class PackedRows(C.Structure):
                 ("idx_bits", C.c_int), ("main_bits", C.c_int), ("aux_bits", C.c_int), ("qmax", C.c_int)]
 
 
+class CropArgs(C.Structure):
+    _fields_ = [("flag_plane", vp * 2), ("sb_tile_off", vp * 2), ("sb_count", vp * 2), ("count", C.c_int), ("B", C.c_int), ("H", C.c_int),
+                ("t_cap", i64), ("n_chunks", C.c_int), ("lengths", vp), ("length", C.c_int)]
+
+
 EXPORTS = [
     "hqmq_version", "hqmq_status_string", "hqmq_layout_bits", "hqmq_build_joint", "hqmq_quantize",
     "hqmq_med3x_workspace_bytes", "hqmq_med3x_threshold", "hqmq_outlier_mask", "hqmq_outlier_compact", "hqmq_dequant",
     "hqmq_pack_codes", "hqmq_dequant_packed", "hqmq_attn_workspace_bytes", "hqmq_attn_pick_splits",
     "hqmq_attn_fwd", "hqmq_attn_combine", "hqmq_append_kv", "hqmq_attn_static_scratch_bytes", "hqmq_attn_fwd_static",
-    "hqmq_search_grid_bytes", "hqmq_build_search_grid", "hqmq_quantize_grid", "hqmq_append_kv_grid",
+    "hqmq_search_grid_bytes", "hqmq_build_search_grid", "hqmq_quantize_grid", "hqmq_append_kv_grid", "hqmq_crop",
 ]
 BENCH_EXPORTS = ["hqmq_bench_read_planes_sink_bytes", "hqmq_bench_read_planes", "hqmq_bench_read_plain", "hqmq_bench_read_lds",
                  "hqmq_bench_empty"]

@@ -4,22 +4,28 @@
 // OutlierAwareHQMQQuantizer._qdq (src/quantizers/outlier_aware.py:60-69 of the
 // reference): per head, the median over every chunk norm of the call (fp32
 // interpolation between the two middle order statistics), times the
-// multiplier, rounded to D.  The order statistics come from an exact radix
-// select: chunk norms are non-negative, so their bit patterns sort like the
-// values; 16-bit dtypes need one 32768-bin histogram per head, fp32 a second
-// pass over the low 16 bits of the bin(s) holding the two ranks.
+// multiplier, rounded to D.  The order statistics are exact: chunk norms are
+// non-negative, so their bit patterns sort like the values.  Calls of at most
+// 8192 chunks per head keep the keys in registers and search the key bit by bit
+// (one launch); larger ones take a 32768-bin histogram per head of the top 16
+// bits, which is the whole key of a 16-bit type, and for fp32 a second pass over
+// the low 16 bits of the bin(s) holding the two ranks.  K and V of one append
+// share the launches.
 //
 // hqmq_outlier_compact has no counterpart in the reference: it copies the
 // flagged chunks into the fp16/bf16/fp32 sideband in (token, chunk) order.
 //
 // Compiled with -ffp-contract=off.
-#include "common.h"
+#include "quantize_common.h"
 
 namespace hqmq {
 
 constexpr int kBins1 = 32768;
 constexpr int kBins2 = 65536;
 constexpr int kState = 16;  // ints per head
+// The last 64 bins would count NaN patterns, which are counted apart: they hold the sums of 64 groups of 512 bins instead,
+// which spare the selection all but the two groups it needs.
+constexpr int kGroups = 64, kGroupBins = kBins1 / kGroups, kGroupAt = kBins1 - kGroups;
 
 // workspace (uint32 units): hist1[H][kBins1] | state[H][kState] | (fp32 only) hist2[H][2][kBins2]
 // state: 0 nan count, 1 key_lo, 2 key_hi, 3 rank_lo within bin, 4 rank_hi within bin
@@ -27,129 +33,196 @@ __host__ __device__ inline int64_t ws_words(int H, bool f32) {
     return (int64_t)H * (kBins1 + kState) + (f32 ? (int64_t)H * 2 * kBins2 : 0);
 }
 
-__global__ void fill_zero_kernel(uint32_t *p, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = 0;
+// One tensor of a call, as the kernels see it; a launch takes one or two of equal shape (blockIdx.z).
+struct MedTensor {
+    const void *x;
+    int64_t xsb, xsh, xst;
+    int vec;                    // chunks may be read with one vector load
+    float mult;
+    uint32_t *ws;
+    float *median;
+    void *thr;
+    int32_t *n_out;
+};
+struct MedPair {
+    MedTensor t[2];
+    int B, H, T, n;
+};
+__device__ __forceinline__ uint32_t *med_hist(const MedTensor &m, int h) { return m.ws + (size_t)h * kBins1; }
+__device__ __forceinline__ uint32_t *med_state(const MedTensor &m, int H, int h) { return m.ws + (size_t)H * kBins1 + (size_t)h * kState; }
+__device__ __forceinline__ uint32_t *med_hist2(const MedTensor &m, int H, int h) { return m.ws + (size_t)H * (kBins1 + kState) + (size_t)h * 2 * kBins2; }
+
+__global__ void fill_zero_kernel(uint32_t *p, uint32_t *q, int64_t n) {
+    uint32_t *w = blockIdx.y ? q : p;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) w[i] = 0;
 }
 
 template <class D>
 __device__ __forceinline__ float chunk_norm(const typename D::storage *xp) {
-    return D::rnd(norm4(D::load(xp), D::load(xp + 1), D::load(xp + 2), D::load(xp + 3)));
+    return chunk_norm_d<D>(D::load(xp), D::load(xp + 1), D::load(xp + 2), D::load(xp + 3));
 }
 
+// fp32 bit pattern whose order is the norm's; of a 16-bit type only the upper 16 bits can be set
 template <class D>
 __device__ __forceinline__ uint32_t norm_bits(float nrm) {
     if (D::code == HQMQ_F32) return __float_as_uint(nrm);
     if (D::code == HQMQ_F16) return (uint32_t)__half_as_ushort(__float2half_rn(nrm)) << 16;
     return __float_as_uint(nrm);  // bf16 value: low 16 bits are zero
 }
-
-// LEVEL 0: histogram of the top 16 bits. LEVEL 1 (fp32): low 16 bits of norms whose top bits match a selected bin.
-template <class D, int LEVEL>
-__global__ void med_hist_kernel(const typename D::storage *x, int64_t xsb, int64_t xsh, int64_t xst, int B, int H, int T, int n,
-                                uint32_t *ws) {
-    const int h = blockIdx.y;
-    uint32_t *hist1 = ws + (size_t)h * kBins1;
-    uint32_t *state = ws + (size_t)H * kBins1 + (size_t)h * kState;
-    uint32_t *hist2 = ws + (size_t)H * (kBins1 + kState) + (size_t)h * 2 * kBins2;
-    const int64_t per_head = (int64_t)B * T * n;
-    uint32_t key_lo = 0, key_hi = 0;
-    if (LEVEL == 1) { key_lo = state[1]; key_hi = state[2]; }
-    for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < per_head; g += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(g % n);
-        const int64_t bt = g / n;
-        const int t = (int)(bt % T), b = (int)(bt / T);
-        const float nrm = chunk_norm<D>(x + b * xsb + h * xsh + (int64_t)t * xst + c * 4);
-        if (is_nan(nrm)) {
-            if (LEVEL == 0) atomicAdd(&state[0], 1u);
-            continue;
-        }
-        const uint32_t bits = norm_bits<D>(nrm);
-        if (LEVEL == 0) atomicAdd(&hist1[bits >> 16], 1u);
-        else {
-            if ((bits >> 16) == key_lo) atomicAdd(&hist2[bits & 0xffffu], 1u);
-            if ((bits >> 16) == key_hi && key_hi != key_lo) atomicAdd(&hist2[kBins2 + (bits & 0xffffu)], 1u);
-        }
-    }
-}
-
-// LEVEL 0 for large calls: the 32768 bins live in LDS (128 KB, one block per CU); a block adds only its non-zero
-// bins to the global histogram, a few thousand atomics instead of one per chunk.
+// the norm whose 16-bit key this is (16-bit types)
 template <class D>
-__global__ __launch_bounds__(1024) void med_hist_lds_kernel(const typename D::storage *x, int64_t xsb, int64_t xsh, int64_t xst, int B,
-                                                            int H, int T, int n, uint32_t *ws) {
-    extern __shared__ uint32_t lh[];    // [kBins1] + 1 (NaN count)
-    const int h = blockIdx.y;
-    uint32_t *hist1 = ws + (size_t)h * kBins1;
-    uint32_t *state = ws + (size_t)H * kBins1 + (size_t)h * kState;
-    for (int i = threadIdx.x; i <= kBins1; i += 1024) lh[i] = 0;
-    __syncthreads();
-    const int64_t per_head = (int64_t)B * T * n;
-    for (int64_t g = (int64_t)blockIdx.x * 1024 + threadIdx.x; g < per_head; g += (int64_t)gridDim.x * 1024) {
-        int c, t, b;
-        if (per_head < 0x7fffffff) {
-            const uint32_t g32 = (uint32_t)g, bt = g32 / (uint32_t)n;
-            c = (int)(g32 - bt * (uint32_t)n);
-            b = (int)(bt / (uint32_t)T);
-            t = (int)(bt - (uint32_t)b * (uint32_t)T);
-        } else {
-            c = (int)(g % n);
-            const int64_t bt = g / n;
-            t = (int)(bt % T);
-            b = (int)(bt / T);
-        }
-        const float nrm = chunk_norm<D>(x + b * xsb + h * xsh + (int64_t)t * xst + c * 4);
-        if (is_nan(nrm)) atomicAdd(&lh[kBins1], 1u);
-        else atomicAdd(&lh[norm_bits<D>(nrm) >> 16], 1u);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < kBins1; i += 1024) {
-        const uint32_t v = lh[i];
-        if (v) atomicAdd(&hist1[i], v);
-    }
-    if (threadIdx.x == 0 && lh[kBins1]) atomicAdd(&state[0], lh[kBins1]);
+__device__ __forceinline__ float key_value(uint32_t key16) {
+    return D::code == HQMQ_F16 ? __half2float(__ushort_as_half((uint16_t)key16)) : __uint_as_float(key16 << 16);
 }
 
-// Finds the bins holding 0-based ranks r_lo <= r_hi in a histogram of `bins` counters.
-// One block of 1024 threads: every thread sums its bins/1024 consecutive counters, a block-wide scan gives each
-// thread the rank range of its segment, and the thread whose range holds a wanted rank walks its own segment.
-__device__ void select_two(const uint32_t *hist, int bins, int64_t r_lo, int64_t r_hi, uint32_t *key_lo, uint32_t *key_hi,
-                           int64_t *in_lo, int64_t *in_hi) {
-    __shared__ unsigned long long part[1024];
+// f(norm) for the chunks of rows [r0, r1) of head h (row = b * T + t), one chunk per lane of a block of NT threads and
+// step, U loads in flight per lane.  The rows of a lane lie NT / n apart: no division per chunk.
+template <class D, int NT, int U, class F>
+__device__ __forceinline__ void for_each_norm(const MedTensor &m, const MedPair &a, int h, int64_t r0, int64_t r1, F f) {
+    using ST = typename D::storage;
+    const int n = a.n, per = n <= NT ? NT / n : 1, rl = n <= NT ? (int)threadIdx.x / n : 0;
+    if (rl >= per || r0 + rl >= r1) return;
+    for (int c = (int)threadIdx.x - rl * n; c < n; c += NT) {           // one round, unless a row has more chunks than the block lanes
+        int64_t r = r0 + rl;
+        const int64_t b = r / a.T;
+        int t = (int)(r - b * a.T);
+        const ST *p = (const ST *)m.x + b * m.xsb + h * m.xsh + (int64_t)t * m.xst + c * 4;
+        const int64_t step = per * m.xst, wrap = m.xsb - a.T * m.xst;
+        while (r < r1) {
+            RawChunk<D> raw[U];
+            int k = 0;
+#pragma unroll
+            for (int i = 0; i < U; i++) {
+                if (r < r1) {
+                    raw[i].load(p, m.vec);
+                    k = i + 1;
+                }
+                r += per;
+                t += per;
+                p += step;
+                while (t >= a.T) { t -= a.T; p += wrap; }
+            }
+#pragma unroll
+            for (int i = 0; i < U; i++)
+                if (i < k) f(chunk_norm_d<D>(raw[i].get(0), raw[i].get(1), raw[i].get(2), raw[i].get(3)));
+        }
+    }
+}
+
+// Sum over the wavefront, in every lane (lane permutations inside the vector unit).
+__device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
+    x += dpp_u32<0xB1>(x);
+    x += dpp_u32<0x4E>(x);
+    x += dpp_u32<0x141>(x);
+    x += dpp_u32<0x140>(x);
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = r[0] + r[1];
+    const auto q = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return q[0] + q[1];
+}
+
+// Histogram of the top 16 bits: the 32768 bins live in LDS, and a block adds only its non-zero bins (some 3000 of an
+// ordinary tensor) to the global histogram.  Blocks of at most 65535 chunks pack two 16-bit counters in a word: 64 KB,
+// two blocks per CU and half the bins to clear and to look through (8 heads x 65536 chunks fp16: 44 us with one
+// global atomic per chunk).
+template <class D, bool WIDE>
+__global__ __launch_bounds__(1024) void med_hist_kernel(MedPair a, int64_t rows_per_block) {
+    extern __shared__ uint32_t lh[];    // [words] + 1 (NaN count)
+    constexpr int words = WIDE ? kBins1 : kBins1 / 2;
+    const MedTensor &m = a.t[blockIdx.z];
+    const int h = blockIdx.y;
+    for (int i = threadIdx.x; i < words / 4; i += 1024) reinterpret_cast<uint4 *>(lh)[i] = uint4{0, 0, 0, 0};
+    if (threadIdx.x == 0) lh[words] = 0;
+    __syncthreads();
+    const int64_t rows = (int64_t)a.B * a.T, r0 = blockIdx.x * rows_per_block;
+    for_each_norm<D, 1024, 4>(m, a, h, r0, min(rows, r0 + rows_per_block), [&](float nrm) {
+        const uint32_t key = norm_bits<D>(nrm) >> 16;
+        if (is_nan(nrm)) atomicAdd(&lh[words], 1u);
+        else if (WIDE) atomicAdd(&lh[key], 1u);
+        else atomicAdd(&lh[key >> 1], 1u << (16 * (key & 1)));
+    });
+    __syncthreads();
+    uint32_t *hist1 = med_hist(m, h);
+    for (int i = threadIdx.x; i < words; i += 1024) {                    // the 64 words of a wavefront lie in one group
+        const uint32_t v = lh[i];
+        uint32_t sum;
+        if (WIDE) {
+            if (v) atomicAdd(&hist1[i], v);
+            sum = v;
+        } else {
+            if (v & 0xffffu) atomicAdd(&hist1[2 * i], v & 0xffffu);
+            if (v >> 16) atomicAdd(&hist1[2 * i + 1], v >> 16);
+            sum = (v & 0xffffu) + (v >> 16);
+        }
+        if (__builtin_amdgcn_ballot_w64(sum != 0u) == 0ull) continue;
+        sum = wave_sum(sum);
+        if ((threadIdx.x & 63) == 0) atomicAdd(&hist1[kGroupAt + (WIDE ? i : 2 * i) / kGroupBins], sum);
+    }
+    if (threadIdx.x == 0 && lh[words]) atomicAdd(&med_state(m, a.H, h)[0], lh[words]);
+}
+
+// fp32, second pass: low 16 bits of the norms whose top bits are a selected bin
+__global__ __launch_bounds__(1024) void med_hist_low_kernel(MedPair a, int64_t rows_per_block) {
+    const MedTensor &m = a.t[blockIdx.z];
+    const int h = blockIdx.y;
+    const uint32_t *state = med_state(m, a.H, h);
+    const uint32_t key_lo = state[1], key_hi = state[2];
+    uint32_t *hist2 = med_hist2(m, a.H, h);
+    const int64_t rows = (int64_t)a.B * a.T, r0 = blockIdx.x * rows_per_block;
+    for_each_norm<F32, 1024, 4>(m, a, h, r0, min(rows, r0 + rows_per_block), [&](float nrm) {
+        const uint32_t bits = __float_as_uint(nrm);
+        if ((bits >> 16) == key_lo) atomicAdd(&hist2[bits & 0xffffu], 1u);
+        else if ((bits >> 16) == key_hi) atomicAdd(&hist2[kBins2 + (bits & 0xffffu)], 1u);
+    });
+}
+
+// Finds the bins holding 0-based ranks r[0] <= r[1] in a histogram of PER * 1024 counters (a block of 1024 threads).
+// Wavefront w owns bins w * PER * 64 .., read as PER coalesced rows of 64 into registers; the wavefront whose range
+// holds a rank walks its rows, then the lanes of the row.  (Every thread summing PER consecutive counters and walking
+// them again one dependent load at a time took 20 us a launch.)  counts: the thread's counters, row by row.
+template <int PER>
+__device__ __forceinline__ void select_two(const uint32_t *hist, const int64_t (&r)[2], uint32_t (&counts)[PER], uint32_t (&key)[2], int64_t (&inner)[2]) {
+    __shared__ unsigned long long tot[16];
     __shared__ uint32_t res[2];
     __shared__ long long resr[2];
-    const int per = bins / 1024;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < PER; i++) counts[i] = hist[(wave * PER + i) * 64 + lane];
     unsigned long long s = 0;
-    for (int i = 0; i < per; i++) s += hist[threadIdx.x * per + i];
-    part[threadIdx.x] = s;
-    if (threadIdx.x < 2) { res[threadIdx.x] = (uint32_t)(bins - 1); resr[threadIdx.x] = 0; }
+#pragma unroll
+    for (int i = 0; i < PER; i++) s += counts[i];
+    for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o);
+    if (lane == 0) tot[wave] = s;
+    if (threadIdx.x < 2) { res[threadIdx.x] = (uint32_t)(PER * 1024 - 1); resr[threadIdx.x] = 0; }
     __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {  // inclusive Hillis-Steele scan
-        const unsigned long long v = (int)threadIdx.x >= off ? part[threadIdx.x - off] : 0;
-        __syncthreads();
-        part[threadIdx.x] += v;
-        __syncthreads();
-    }
-    const unsigned long long incl = part[threadIdx.x], excl = incl - s;
-    const int64_t want[2] = {r_lo, r_hi};
+    unsigned long long before = 0;
+    for (int w = 0; w < wave; w++) before += tot[w];
     for (int which = 0; which < 2; which++) {
-        const unsigned long long w = (unsigned long long)want[which];
-        if (w >= excl && w < incl) {
-            unsigned long long r2 = excl;
-            for (int j = 0; j < per; j++) {
-                const uint32_t cnt = hist[threadIdx.x * per + j];
-                if (w < r2 + cnt) {
-                    res[which] = (uint32_t)(threadIdx.x * per + j);
-                    resr[which] = (long long)(w - r2);
-                    break;
+        const unsigned long long want = (unsigned long long)r[which];
+        if (want < before || want >= before + s) continue;           // wave-uniform
+        unsigned long long at = before;
+        bool found = false;
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const uint32_t row = wave_sum(counts[i]);                // a row holds fewer than 2^32 chunks
+            if (!found && want < at + row) {
+                found = true;
+                uint32_t incl = counts[i];
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t v = __shfl_up(incl, o, 64);
+                    if (lane >= o) incl += v;
                 }
-                r2 += cnt;
+                const uint32_t rest = (uint32_t)(want - at), excl = incl - counts[i];
+                if (rest >= excl && rest < incl) {
+                    res[which] = (uint32_t)((wave * PER + i) * 64 + lane);
+                    resr[which] = (long long)(rest - excl);
+                }
             }
+            at += row;
         }
     }
     __syncthreads();
-    *key_lo = res[0]; *key_hi = res[1];
-    *in_lo = resr[0]; *in_hi = resr[1];
-    __syncthreads();
+    for (int which = 0; which < 2; which++) { key[which] = res[which]; inner[which] = resr[which]; }
 }
 
 template <class D>
@@ -166,378 +239,434 @@ __device__ __forceinline__ void finish_threshold(float a, float b, bool same, fl
     const float t32 = med * mult;
     D::store(thr + h, D::rnd(t32));
 }
-
+// a NaN norm makes the quantile NaN, the mask empty
 template <class D>
-__global__ __launch_bounds__(1024) void med_select1_kernel(uint32_t *ws, int H, int64_t per_head, float mult, float *median,
-                                                           typename D::storage *thr, int32_t *n_out) {
-    const int h = blockIdx.x;
-    const uint32_t *hist1 = ws + (size_t)h * kBins1;
-    uint32_t *state = ws + (size_t)H * kBins1 + (size_t)h * kState;
-    if (state[0] > 0) {  // a NaN norm makes the quantile NaN, the mask empty
+__device__ __forceinline__ void nan_threshold(const MedTensor &m, int h) {
+    m.median[h] = NAN;
+    D::store((typename D::storage *)m.thr + h, NAN);
+    if (m.n_out) m.n_out[h] = 0;
+}
+
+// One wavefront per rank: the group that holds it (64 sums), then the bin inside the group (8 bins per lane).
+template <class D>
+__global__ __launch_bounds__(128) void med_select_kernel(MedPair a) {
+    const MedTensor &m = a.t[blockIdx.z];
+    const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t per_head = (uint32_t)((int64_t)a.B * a.T * a.n);
+    uint32_t *state = med_state(m, a.H, h);
+    const uint32_t *hist = med_hist(m, h);
+    const uint32_t sum = hist[kGroupAt + lane];
+    if (state[0] > 0) {
         if (threadIdx.x == 0) {
-            median[h] = NAN;
-            D::store(thr + h, NAN);
-            if (n_out) n_out[h] = 0;
+            nan_threshold<D>(m, h);
             state[1] = 0xffffffffu; state[2] = 0xffffffffu;
         }
         return;
     }
-    uint32_t klo, khi;
-    int64_t ilo, ihi;
-    select_two(hist1, kBins1, (per_head - 1) / 2, per_head / 2, &klo, &khi, &ilo, &ihi);
-    if (D::code == HQMQ_F32) {
-        if (threadIdx.x == 0) { state[1] = klo; state[2] = khi; state[3] = (uint32_t)ilo; state[4] = (uint32_t)ihi; }
-        return;
-    }
-    __shared__ float thr_sh;
-    if (threadIdx.x == 0) {
-        const float a = (D::code == HQMQ_F16) ? __half2float(__ushort_as_half((uint16_t)klo)) : __uint_as_float(klo << 16);
-        const float b = (D::code == HQMQ_F16) ? __half2float(__ushort_as_half((uint16_t)khi)) : __uint_as_float(khi << 16);
-        finish_threshold<D>(a, b, (per_head - 1) / 2 == per_head / 2, mult, h, median, thr);
-        thr_sh = D::load(thr + h);
-    }
-    __syncthreads();
-    if (n_out) {  // chunks with norm > thr: bins above the threshold's own bin
-        __shared__ unsigned long long cnt_sh;
-        if (threadIdx.x == 0) cnt_sh = 0;
-        __syncthreads();
-        const float tv = thr_sh;
-        unsigned long long s = 0;
-        for (int k = threadIdx.x; k < kBins1; k += blockDim.x) {
-            const float v = (D::code == HQMQ_F16) ? __half2float(__ushort_as_half((uint16_t)k)) : __uint_as_float((uint32_t)k << 16);
-            if (v > tv) s += hist1[k];
-        }
-        atomicAdd(&cnt_sh, s);
-        __syncthreads();
-        if (threadIdx.x == 0) n_out[h] = (int32_t)cnt_sh;
-    }
-}
-
-// Small calls (a decode step appends B * n chunks per head): norms, exact radix select and count in one launch,
-// one block per head, the 16-bit keys in LDS.  16-bit dtypes only.
-constexpr int kSmallMax = 8192;
-
-// rank -> (bin holding it, rank inside the bin) over the 256 counters of `hist`; every thread of the block calls it
-__device__ __forceinline__ void find_bin256(const uint32_t *hist, uint32_t rank, uint32_t *wave_tot, uint32_t *res,
-                                            uint32_t &bin, uint32_t &inner) {
-    const int tid = threadIdx.x;
-    uint32_t v = 0, incl = 0;
-    if (tid < 256) {
-        v = hist[tid];
-        incl = v;
+    auto before = [&](uint32_t v) {                      // exclusive prefix sum over the wavefront
+        uint32_t incl = v;
         for (int o = 1; o < 64; o <<= 1) {
             const uint32_t u = __shfl_up(incl, o, 64);
-            if ((tid & 63) >= o) incl += u;
+            if (lane >= o) incl += u;
         }
-        if ((tid & 63) == 63) wave_tot[tid >> 6] = incl;
-    }
-    __syncthreads();
-    if (tid < 256) {
-        for (int w = 0; w < (tid >> 6); w++) incl += wave_tot[w];
-        const uint32_t excl = incl - v;
-        if (rank >= excl && rank < incl) { res[0] = (uint32_t)tid; res[1] = rank - excl; }
-    }
-    __syncthreads();
-    bin = res[0];
-    inner = res[1];
-    __syncthreads();
-}
-
-struct MedSmall {
-    const void *x; int64_t xsb, xsh, xst;
-    int B, T, n;
-    float mult;
-    float *median; void *thr; int32_t *n_out;
-};
-
-// NT threads (at least 256)
-template <class D, int NT>
-__device__ __forceinline__ void med_small_body(const MedSmall &a) {
-    const typename D::storage *x = (const typename D::storage *)a.x;
-    typename D::storage *thr = (typename D::storage *)a.thr;
-    const int64_t xsb = a.xsb, xsh = a.xsh, xst = a.xst;
-    const int B = a.B, T = a.T, n = a.n;
-    const float mult = a.mult;
-    float *median = a.median;
-    int32_t *n_out = a.n_out;
-    __shared__ uint16_t keys[kSmallMax];
-    __shared__ uint32_t hist[256], wave_tot[4], res[2], nan_count, gt_count;
-    __shared__ float thr_sh;
-    const int h = blockIdx.x, tid = threadIdx.x;
-    const int per_head = B * T * n;
-    if (tid == 0) { nan_count = 0; gt_count = 0; res[0] = 255; res[1] = 0; }
-    __syncthreads();
-    for (int g = tid; g < per_head; g += NT) {
-        const int bt = g / n, c = g - bt * n, b = bt / T, t = bt - b * T;
-        const float nrm = chunk_norm<D>(x + b * xsb + h * xsh + (int64_t)t * xst + c * 4);
-        if (is_nan(nrm)) { atomicAdd(&nan_count, 1u); keys[g] = 0xffffu; }
-        else keys[g] = (uint16_t)(norm_bits<D>(nrm) >> 16);
-    }
-    __syncthreads();
-    if (nan_count > 0) {  // a NaN norm makes the quantile NaN, the mask empty
-        if (tid == 0) {
-            median[h] = NAN;
-            D::store(thr + h, NAN);
-            if (n_out) n_out[h] = 0;
+        return incl - v;
+    };
+    auto bins = [&](int group, uint32_t (&v)[8]) {       // the lane's 8 bins of a group; the sums' own places count nothing
+        const uint4 *p = reinterpret_cast<const uint4 *>(hist + group * kGroupBins + lane * 8);
+        const uint4 x = p[0], y = p[1];
+        const bool real = group * kGroupBins + lane * 8 < kGroupAt;
+        const uint32_t w[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = real ? w[i] : 0u;
+    };
+    __shared__ uint32_t key_sh[2], in_sh[2];
+    const uint32_t rank = wave == 0 ? (per_head - 1) / 2 : per_head / 2;
+    {
+        const uint32_t at = before(sum);
+        const uint64_t mine = __builtin_amdgcn_ballot_w64(rank >= at && rank < at + sum);
+        const int group = mine ? __builtin_ctzll(mine) : kGroups - 1;
+        uint32_t v[8], tot = 0;
+        bins(group, v);
+        uint32_t rest = rank - __shfl(at, group);
+#pragma unroll
+        for (int i = 0; i < 8; i++) tot += v[i];
+        const uint32_t first = before(tot);
+        if (rest >= first && rest < first + tot) {
+            rest -= first;
+            int i = 0;
+#pragma unroll
+            for (int k = 0; k < 7; k++)
+                if (i == k && rest >= v[k]) { rest -= v[k]; i = k + 1; }
+            key_sh[wave] = (uint32_t)(group * kGroupBins + lane * 8 + i);
+            in_sh[wave] = rest;
         }
+    }
+    __syncthreads();
+    if (D::code == HQMQ_F32) {
+        if (threadIdx.x == 0) { state[1] = key_sh[0]; state[2] = key_sh[1]; state[3] = in_sh[0]; state[4] = in_sh[1]; }
         return;
     }
-    auto select = [&](uint32_t rank) -> uint32_t {
-        uint32_t hi, in_hi, lo, in_lo;
-        if (tid < 256) hist[tid] = 0;
-        __syncthreads();
-        for (int g = tid; g < per_head; g += NT) atomicAdd(&hist[keys[g] >> 8], 1u);
-        __syncthreads();
-        find_bin256(hist, rank, wave_tot, res, hi, in_hi);
-        if (tid < 256) hist[tid] = 0;
-        __syncthreads();
-        for (int g = tid; g < per_head; g += NT)
-            if ((uint32_t)(keys[g] >> 8) == hi) atomicAdd(&hist[keys[g] & 255u], 1u);
-        __syncthreads();
-        find_bin256(hist, in_hi, wave_tot, res, lo, in_lo);
-        return (hi << 8) | lo;
-    };
-    const uint32_t r_lo = (uint32_t)((per_head - 1) / 2), r_hi = (uint32_t)(per_head / 2);
-    const uint32_t klo = select(r_lo);
-    const uint32_t khi = r_hi == r_lo ? klo : select(r_hi);
-    if (tid == 0) {
-        const float a = (D::code == HQMQ_F16) ? __half2float(__ushort_as_half((uint16_t)klo)) : __uint_as_float(klo << 16);
-        const float b = (D::code == HQMQ_F16) ? __half2float(__ushort_as_half((uint16_t)khi)) : __uint_as_float(khi << 16);
-        finish_threshold<D>(a, b, r_lo == r_hi, mult, h, median, thr);
-        thr_sh = D::load(thr + h);
-    }
-    __syncthreads();
-    if (n_out) {
-        const float tv = thr_sh;
-        uint32_t cnt = 0;
-        for (int g = tid; g < per_head; g += NT) {
-            const uint32_t k = keys[g];
-            const float v = (D::code == HQMQ_F16) ? __half2float(__ushort_as_half((uint16_t)k)) : __uint_as_float(k << 16);
-            if (v > tv) cnt++;
-        }
-        if (cnt) atomicAdd(&gt_count, cnt);
-        __syncthreads();
-        if (tid == 0) n_out[h] = (int32_t)gt_count;
-    }
+    if (wave != 0) return;
+    const bool same = (per_head - 1) / 2 == per_head / 2;
+    const float lo = key_value<D>(key_sh[0]), hi = key_value<D>(key_sh[1]);
+    const float tv = D::rnd((same ? lo : hi - (hi - lo) * 0.5f) * m.mult);
+    if (lane == 0) finish_threshold<D>(lo, hi, same, m.mult, h, m.median, (typename D::storage *)m.thr);
+    if (!m.n_out) return;
+    // chunks with norm > thr: whole groups above the one that holds the threshold, and the bins above it in there.  (A
+    // threshold below every norm or beyond infinity: group 0 or none.)
+    const uint32_t thr_key = norm_bits<D>(fmaxf(tv, 0.f)) >> 16;
+    const int group = (int)min(thr_key / kGroupBins, (uint32_t)kGroups - 1u);
+    uint32_t v[8], n = lane > group ? sum : 0u;
+    bins(group, v);
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        if (key_value<D>((uint32_t)(group * kGroupBins + lane * 8 + i)) > tv) n += v[i];
+    n = wave_sum(n);
+    if (lane == 0) m.n_out[h] = (int32_t)n;
 }
 
-template <class D, int NT>
-__global__ __launch_bounds__(NT) void med_small_kernel(MedSmall a) {
-    med_small_body<D, NT>(a);
-}
-// two tensors of equal shape: blockIdx.y picks one
-template <class D, int NT>
-__global__ __launch_bounds__(NT) void med_small_pair_kernel(MedSmall a, MedSmall b) {
-    med_small_body<D, NT>(blockIdx.y ? b : a);
-}
-
-__global__ __launch_bounds__(1024) void med_select2_kernel(uint32_t *ws, int H, int64_t per_head, float mult, float *median,
-                                                           float *thr) {
+// fp32: the low halves of the two keys
+__global__ __launch_bounds__(1024) void med_select_low_kernel(MedPair a) {
+    const MedTensor &m = a.t[blockIdx.z];
     const int h = blockIdx.x;
-    uint32_t *state = ws + (size_t)H * kBins1 + (size_t)h * kState;
-    const uint32_t *hist2 = ws + (size_t)H * (kBins1 + kState) + (size_t)h * 2 * kBins2;
+    const int64_t per_head = (int64_t)a.B * a.T * a.n;
+    uint32_t *state = med_state(m, a.H, h);
+    const uint32_t *hist2 = med_hist2(m, a.H, h);
     if (state[0] > 0) return;
     const uint32_t klo = state[1], khi = state[2];
-    uint32_t l0, l1, d0, d1;
-    int64_t i0, i1;
-    if (klo == khi) {
-        select_two(hist2, kBins2, state[3], state[4], &l0, &l1, &i0, &i1);
-    } else {
-        select_two(hist2, kBins2, state[3], state[3], &l0, &d0, &i0, &i1);
-        select_two(hist2 + kBins2, kBins2, state[4], state[4], &l1, &d1, &i0, &i1);
+    constexpr int PER = kBins2 / 1024;
+    uint32_t counts[PER], low[2], up[2];
+    int64_t inner[2];
+    const int64_t r[2] = {state[3], klo == khi ? state[4] : state[3]};
+    select_two<PER>(hist2, r, counts, low, inner);
+    if (klo != khi) {
+        __syncthreads();
+        const int64_t r2[2] = {state[4], state[4]};
+        select_two<PER>(hist2 + kBins2, r2, counts, up, inner);
+        low[1] = up[1];
     }
     if (threadIdx.x == 0) {
-        const float a = __uint_as_float((klo << 16) | l0), b = __uint_as_float((khi << 16) | l1);
-        finish_threshold<F32>(a, b, (per_head - 1) / 2 == per_head / 2, mult, h, median, thr);
+        const float x = __uint_as_float((klo << 16) | low[0]), y = __uint_as_float((khi << 16) | low[1]);
+        finish_threshold<F32>(x, y, (per_head - 1) / 2 == per_head / 2, m.mult, h, m.median, (float *)m.thr);
+        if (m.n_out) m.n_out[h] = 0;
     }
 }
 
-__global__ void count_gt_kernel(const float *x, int64_t xsb, int64_t xsh, int64_t xst, int B, int T, int n, const float *thr,
-                                int32_t *n_out) {
+__global__ __launch_bounds__(1024) void count_gt_kernel(MedPair a, int64_t rows_per_block) {
+    const MedTensor &m = a.t[blockIdx.z];
     const int h = blockIdx.y;
-    const float tv = thr[h];
-    const int64_t per_head = (int64_t)B * T * n;
-    int cnt = 0;
-    for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < per_head; g += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(g % n);
-        const int64_t bt = g / n;
-        const int t = (int)(bt % T), b = (int)(bt / T);
-        if (chunk_norm<F32>(x + b * xsb + h * xsh + (int64_t)t * xst + c * 4) > tv) cnt++;
+    if (!m.n_out) return;
+    const float tv = ((const float *)m.thr)[h];
+    uint32_t cnt = 0;
+    const int64_t rows = (int64_t)a.B * a.T, r0 = blockIdx.x * rows_per_block;
+    for_each_norm<F32, 1024, 4>(m, a, h, r0, min(rows, r0 + rows_per_block), [&](float nrm) { cnt += nrm > tv ? 1u : 0u; });
+    cnt = wave_sum(cnt);
+    if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(&m.n_out[h], (int)cnt);
+}
+
+// Small calls (a decode step appends B * n chunks per head): norms, exact order statistics and count in one launch, one
+// block per head, eight keys per lane in registers.  The key of rank r is the largest v with fewer than r + 1 keys below
+// it, found bit by bit from the top: a compare and a scalar bit count per key, one barrier per round (none in a block of
+// one wavefront); two bits, three thresholds a round.  The second rank is the next one: the same key again, or the smallest key above it.
+// (256-bin histograms of keys in LDS, two passes per rank, took 9.5 us for 2048 chunks per head.)
+constexpr int kSmallKeys = 8;
+template <class D, int NT>
+__global__ __launch_bounds__(NT) void med_small_kernel(MedPair a) {
+    constexpr int W = NT / 64, BITS = D::code == HQMQ_F32 ? 31 : 15;
+    __shared__ uint4 part[2][W];
+    const MedTensor &m = a.t[blockIdx.z];
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int per_head = a.B * a.T * a.n, rows = a.B * a.T;
+    using ST = typename D::storage;
+    // lane (rl, c) holds chunk c of rows rl, rl + per, ..: one division per lane, not one per key
+    const int per = NT / a.n, rl = tid / a.n, c = tid - rl * a.n;
+    uint32_t key[kSmallKeys];
+    bool nan = false, have[kSmallKeys];
+    {
+        RawChunk<D> raw[kSmallKeys] = {};
+        const int b0 = rl / a.T;
+        int r = rl < per ? rl : rows, t = rl - b0 * a.T;
+        const ST *p = (const ST *)m.x + b0 * m.xsb + h * m.xsh + (int64_t)t * m.xst + c * 4;
+        const int64_t step = per * m.xst, wrap = m.xsb - a.T * m.xst;
+#pragma unroll
+        for (int i = 0; i < kSmallKeys; i++) {
+            have[i] = r < rows;
+            if (have[i]) raw[i].load(p, m.vec);
+            r += per;
+            t += per;
+            p += step;
+            while (t >= a.T) { t -= a.T; p += wrap; }
+        }
+#pragma unroll
+        for (int i = 0; i < kSmallKeys; i++) {
+            const float nrm = chunk_norm_d<D>(raw[i].get(0), raw[i].get(1), raw[i].get(2), raw[i].get(3));
+            nan |= have[i] && is_nan(nrm);
+            key[i] = have[i] ? (D::code == HQMQ_F32 ? __float_as_uint(nrm) : norm_bits<D>(nrm) >> 16) : 0x7fffffffu;    // absent: above every key
+        }
     }
-    if (cnt) atomicAdd(&n_out[h], cnt);
+    int turn = 0;
+    // sum of a wave-uniform number over the block
+    auto total = [&](uint32_t v) -> uint32_t {
+        if (W == 1) return v;
+        if (lane == 0) part[turn][wave].x = v;
+        __syncthreads();
+        uint32_t s = 0;
+#pragma unroll
+        for (int w = 0; w < W; w++) s += part[turn][w].x;
+        turn ^= 1;
+        return s;
+    };
+    auto below = [&](uint32_t v) -> uint32_t {
+        uint32_t c = 0;
+#pragma unroll
+        for (int i = 0; i < kSmallKeys; i++) c += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[i] < v));
+        return total(c);
+    };
+    if (total(__builtin_amdgcn_ballot_w64(nan) != 0ull ? 1u : 0u) > 0u) {
+        if (tid == 0) nan_threshold<D>(m, h);
+        return;
+    }
+    const uint32_t r_lo = (uint32_t)((per_head - 1) / 2), r_hi = (uint32_t)(per_head / 2);
+    uint32_t k_lo = 0;
+    for (int bit = BITS - 1; bit >= 0; bit -= 2) {       // two bits a round (the last has one: its three thresholds coincide)
+        const uint32_t v1 = k_lo | 1u << (bit - (bit ? 1 : 0)), v2 = k_lo | 1u << bit, v3 = v2 | v1;
+        uint32_t c1 = 0, c2 = 0, c3 = 0;
+#pragma unroll
+        for (int i = 0; i < kSmallKeys; i++) {
+            c1 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[i] < v1));
+            c2 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[i] < v2));
+            c3 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[i] < v3));
+        }
+        if (W > 1) {
+            if (lane == 0) part[turn][wave] = uint4{c1, c2, c3, 0u};
+            __syncthreads();
+            c1 = c2 = c3 = 0;
+#pragma unroll
+            for (int w = 0; w < W; w++) { const uint4 q = part[turn][w]; c1 += q.x; c2 += q.y; c3 += q.z; }
+            turn ^= 1;
+        }
+        k_lo = c3 <= r_lo ? v3 : c2 <= r_lo ? v2 : c1 <= r_lo ? v1 : k_lo;
+    }
+    uint32_t k_hi = k_lo;
+    if (r_hi != r_lo && below(k_lo + 1u) <= r_hi) {
+        uint32_t mn = 0xffffffffu;
+#pragma unroll
+        for (int i = 0; i < kSmallKeys; i++) mn = min(mn, key[i] > k_lo ? key[i] : 0xffffffffu);
+        mn = ~group_max(~mn, 64, [](uint32_t p, uint32_t q) { return max(p, q); });
+        if (W > 1) {
+            if (lane == 0) part[turn][wave].x = mn;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < W; w++) mn = min(mn, part[turn][w].x);
+            turn ^= 1;
+        }
+        k_hi = mn;
+    }
+    auto value = [](uint32_t k) { return D::code == HQMQ_F32 ? __uint_as_float(k) : key_value<D>(k); };
+    const float x = value(k_lo), y = value(k_hi);
+    const float med = r_lo == r_hi ? x : y - (y - x) * 0.5f;
+    const float tv = D::rnd(med * m.mult);
+    if (m.n_out) {
+        uint32_t c = 0;
+#pragma unroll
+        for (int i = 0; i < kSmallKeys; i++)
+            c += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(have[i] && value(key[i]) > tv));
+        c = total(c);
+        if (tid == 0) m.n_out[h] = (int32_t)c;
+    }
+    if (tid == 0) finish_threshold<D>(x, y, r_lo == r_hi, m.mult, h, m.median, (ST *)m.thr);
+}
+
+// The flag bits of a row (up to 256 chunks) in registers; dwords where the row's address allows it.
+__device__ __forceinline__ int row_flags(const uint8_t *fr, int frb, bool words, uint64_t (&own)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) own[i] = 0;
+    if (words && frb == 4) own[0] = *reinterpret_cast<const uint32_t *>(fr);
+    else if (words && frb == 8) own[0] = *reinterpret_cast<const uint32_t *>(fr) | (uint64_t)reinterpret_cast<const uint32_t *>(fr)[1] << 32;
+    else if (words && frb == 2) own[0] = *reinterpret_cast<const uint16_t *>(fr);
+    else {
+#pragma unroll
+        for (int by = 0; by < 32; by++)
+            if (by < frb) own[by >> 3] |= (uint64_t)fr[by] << (8 * (by & 7));
+    }
+    return __popcll(own[0]) + __popcll(own[1]) + __popcll(own[2]) + __popcll(own[3]);
+}
+// rows of `frb` flag bytes start at multiples of their width (2) or of 4
+__host__ __device__ inline bool flag_words(const uint8_t *plane, int frb) { return !((uintptr_t)plane & 3) && (frb == 2 || !(frb & 3)); }
+
+// Copies the flagged chunks of one row to sideband slots k, k + 1, ...
+template <class D>
+__device__ __forceinline__ void copy_row(const CompactCall &a, size_t bh, int64_t row, const typename D::storage *xr, const uint64_t (&own)[4], int k,
+                                         bool vec) {
+    using ST = typename D::storage;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        for (uint64_t bits = own[q]; bits; bits &= bits - 1) {
+            const int c = 64 * q + __builtin_ctzll(bits);
+            if (c >= a.n) break;
+            if (k < a.sb_cap) {
+                RawChunk<D> raw;
+                raw.load(xr + c * 4, vec);
+                raw.store((ST *)a.sideband + (bh * a.sb_cap + k) * 4, vec);
+                if (a.sb_coord) a.sb_coord[bh * a.sb_cap + k] = (uint16_t)(((row & (kTile - 1)) << 8) | c);
+            } else {
+                *a.overflow = 1;
+                degrade_to_plain<D>(a, bh * a.t_cap + row, c, xr + c * 4);
+            }
+            k++;
+        }
+    }
+}
+struct CompactPair {
+    CompactCall c[2];           // blockIdx.z picks one; equal shapes
+    int vec[2];                 // chunks of x and of the sideband may be moved by one vector access
+};
+
+// Exclusive prefix sum over the block (NT threads), and its total.
+template <int NT>
+__device__ __forceinline__ int block_scan(int v, int *part, int &total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int incl = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += u;
+    }
+    if (NT == 64) {
+        total = __shfl(incl, 63);
+        return incl - v;
+    }
+    __syncthreads();
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    int before = 0;
+    total = 0;
+    for (int w = 0; w < NT / 64; w++) {
+        if (w < wave) before += part[w];
+        total += part[w];
+    }
+    return before + incl - v;
 }
 
 // One block of NT threads per (b, h): walks the T new rows in order, NT rows per step (one wavefront for short
 // appends: its barriers cost nothing).
 template <class D, int NT>
-__device__ __forceinline__ void compact_body(const CompactCall &a) {
+__global__ __launch_bounds__(NT) void compact_kernel(CompactPair pair) {
     using ST = typename D::storage;
-    const ST *x = (const ST *)a.x;
-    ST *sideband = (ST *)a.sideband;
-    const int64_t xsb = a.xsb, xsh = a.xsh, xst = a.xst, t_cap = a.t_cap, sb_cap = a.sb_cap;
-    const int H = a.H, T = a.T, n = a.n, t_off = a.t_off;
-    const uint8_t *flag_plane = a.flag_plane;
-    const int32_t *pos = a.pos;
-    int32_t *sb_tile_off = a.sb_tile_off, *sb_count = a.sb_count, *overflow = a.overflow;
-    uint16_t *sb_coord = a.sb_coord;
-    __shared__ int scan[NT];
-    __shared__ int base_sh;
-    const int bh = blockIdx.x, b = bh / H, h = bh - b * H;
-    const int frb = (n + 7) >> 3;
-    const int64_t row0 = (pos ? pos[b] : 0) + t_off;
-    const int64_t tiles = (t_cap + kTile - 1) / kTile;
-    if (threadIdx.x == 0) base_sh = sb_count[bh];
-    __syncthreads();
-    for (int t0 = 0; t0 < T; t0 += NT) {
+    const CompactCall &a = pair.c[blockIdx.z];
+    __shared__ int part[NT / 64];
+    const int bh = blockIdx.x, b = bh / a.H, h = bh - b * a.H;
+    const int frb = (a.n + 7) >> 3;
+    const bool words = flag_words(a.flag_plane, frb);
+    const int64_t row0 = (a.pos ? a.pos[b] : 0) + a.t_off;
+    const int64_t tiles = (a.t_cap + kTile - 1) / kTile;
+    int base = a.sb_count[bh];
+    for (int t0 = 0; t0 < a.T; t0 += NT) {
         const int t = t0 + threadIdx.x;
         const int64_t row = row0 + t;
-        const bool live = t < T && row < t_cap;
-        int cnt = 0;
-        const uint8_t *fr = flag_plane + ((size_t)bh * t_cap + (live ? row : 0)) * frb;
-        if (live)
-            for (int by = 0; by < frb; by++) cnt += __popc((uint32_t)fr[by]);
-        scan[threadIdx.x] = cnt;
-        __syncthreads();
-        for (int off = 1; off < NT; off <<= 1) {  // inclusive Hillis-Steele scan
-            int v = (int)threadIdx.x >= off ? scan[threadIdx.x - off] : 0;
-            __syncthreads();
-            scan[threadIdx.x] += v;
-            __syncthreads();
-        }
-        const int base = base_sh;
-        const int before = base + scan[threadIdx.x] - cnt;
+        const bool live = t < a.T && row >= 0 && row < a.t_cap;
+        uint64_t own[4] = {0, 0, 0, 0};          // the row's flags as they are now (bits may be cleared below)
+        const int cnt = live ? row_flags(a.flag_plane + ((size_t)bh * a.t_cap + row) * frb, frb, words, own) : 0;
+        int total;
+        const int before = base + block_scan<NT>(cnt, part, total);
         if (live) {
-            if ((row & (kTile - 1)) == 0) sb_tile_off[(size_t)bh * tiles + (row >> 4)] = before;
-            int k = before;
-            const ST *xr = x + b * xsb + h * xsh + (int64_t)t * xst;
-            uint64_t own[4] = {0, 0, 0, 0};                        // the row's flags as they were, in registers (bits may be cleared below)
-            if (cnt) {
-#pragma unroll
-                for (int by = 0; by < 32; by++)
-                    if (by < frb) own[by >> 3] |= (uint64_t)fr[by] << (8 * (by & 7));
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                for (uint64_t bits = own[q]; bits; bits &= bits - 1) {
-                    const int c = 64 * q + __builtin_ctzll(bits);
-                    if (c >= n) break;
-                    if (k < sb_cap) {
-                        ST *dst = sideband + ((size_t)bh * sb_cap + k) * 4;
-                        for (int j = 0; j < 4; j++) dst[j] = xr[c * 4 + j];
-                        if (sb_coord) sb_coord[(size_t)bh * sb_cap + k] = (uint16_t)(((row & (kTile - 1)) << 8) | c);
-                    } else {
-                        *overflow = 1;
-                        degrade_to_plain<D>(a, (size_t)bh * t_cap + row, c, xr + c * 4);
-                    }
-                    k++;
+            if ((row & (kTile - 1)) == 0) a.sb_tile_off[(size_t)bh * tiles + (row >> 4)] = before;
+            copy_row<D>(a, bh, row, (const ST *)a.x + b * a.xsb + h * a.xsh + (int64_t)t * a.xst, own, before, pair.vec[blockIdx.z]);
+        }
+        base += total;
+    }
+    __syncthreads();                             // every wavefront has read the count
+    if (threadIdx.x == 0) a.sb_count[bh] = base;
+}
+
+// ---- bulk appends (whole 16-row tiles from an aligned first row): two passes with one thread per tile / row ----
+// Pass 1, one block per (b, h): flagged chunks of every new tile, exclusive scan behind the chunks already stored.
+__global__ __launch_bounds__(1024) void tile_scan_kernel(CompactPair pair) {
+    const CompactCall &a = pair.c[blockIdx.z];
+    __shared__ int part[16];
+    const int bh = blockIdx.x, frb = (a.n + 7) >> 3, row0 = a.t_off;
+    const int64_t tiles = (a.t_cap + kTile - 1) / kTile;
+    const int n_tiles = (a.T + kTile - 1) / kTile;
+    int32_t *to = a.sb_tile_off + (size_t)bh * tiles + (row0 >> 4);
+    const uint8_t *fr = a.flag_plane + ((size_t)bh * a.t_cap + row0) * frb;
+    const bool vec = !((uintptr_t)fr & 15);      // a tile is 16 frb bytes: whole 16-byte words, then, at 16-byte addresses
+    int base = a.sb_count[bh];
+    for (int i0 = 0; i0 < n_tiles; i0 += 1024) {
+        const int i = i0 + threadIdx.x;
+        int cnt = 0;
+        if (i < n_tiles) {
+            const int rows = min(a.T - i * kTile, kTile);
+            const uint8_t *f = fr + (size_t)i * kTile * frb;
+            if (vec && rows == kTile) {
+                for (int w = 0; w < frb; w++) {
+                    const uint4 v = reinterpret_cast<const uint4 *>(f)[w];
+                    cnt += __popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w);
                 }
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x == NT - 1) base_sh = base + scan[NT - 1];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) sb_count[bh] = base_sh;
-}
-
-template <class D, int NT>
-__global__ __launch_bounds__(NT) void compact_kernel(CompactCall a) {
-    compact_body<D, NT>(a);
-}
-// two tensors of equal shape: blockIdx.y picks one
-template <class D, int NT>
-__global__ __launch_bounds__(NT) void compact_pair_kernel(CompactCall a, CompactCall b) {
-    compact_body<D, NT>(blockIdx.y ? b : a);
-}
-
-// ---- bulk appends (whole 16-row tiles from an aligned first row): three passes with one thread per tile / row ----
-// Pass 1: flagged chunks of every new tile -> sb_tile_off[tile] (a count for now).
-__global__ void tile_count_kernel(const uint8_t *flag_plane, int64_t t_cap, int row0, int T, int frb, int n_tiles, int32_t *sb_tile_off) {
-    const int bh = blockIdx.y;
-    const int64_t tiles = (t_cap + kTile - 1) / kTile;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_tiles) return;
-    const int r_begin = row0 + i * kTile, r_end = min(row0 + T, r_begin + kTile);
-    const uint8_t *fr = flag_plane + ((size_t)bh * t_cap + r_begin) * frb;
-    int cnt = 0;
-    for (int k = 0; k < (r_end - r_begin) * frb; k++) cnt += __popc((uint32_t)fr[k]);
-    sb_tile_off[(size_t)bh * tiles + (r_begin >> 4)] = cnt;
-}
-// Pass 2: one block per (b, h): counts -> sideband offsets (exclusive scan behind the chunks already stored).
-__global__ __launch_bounds__(1024) void tile_scan_kernel(int64_t t_cap, int row0, int n_tiles, int32_t *sb_tile_off, int32_t *sb_count) {
-    __shared__ int part[1024];
-    const int bh = blockIdx.x;
-    const int64_t tiles = (t_cap + kTile - 1) / kTile;
-    int32_t *to = sb_tile_off + (size_t)bh * tiles + (row0 >> 4);
-    const int per = (n_tiles + 1023) / 1024;
-    const int i0 = threadIdx.x * per, i1 = min(n_tiles, i0 + per);
-    int s = 0;
-    for (int i = i0; i < i1; i++) s += to[i];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        const int v = (int)threadIdx.x >= off ? part[threadIdx.x - off] : 0;
-        __syncthreads();
-        part[threadIdx.x] += v;
-        __syncthreads();
-    }
-    const int base = sb_count[bh];
-    int run = base + part[threadIdx.x] - s;
-    for (int i = i0; i < i1; i++) {
-        const int c = to[i];
-        to[i] = run;
-        run += c;
-    }
-    __syncthreads();
-    if (threadIdx.x == 1023) sb_count[bh] = base + part[1023];
-}
-// Pass 3: one thread per new row copies the row's flagged chunks behind those of the tile's earlier rows.
-// (A row whose entries do not fit clears flag bits while its neighbours count them: every entry they then fail to
-// count lay beyond the capacity, so their own entries still come out beyond it, and the offsets of the entries that
-// fit do not move.)
-template <class D>
-__global__ void tile_copy_kernel(CompactCall a) {
-    using ST = typename D::storage;
-    const ST *x = (const ST *)a.x;
-    ST *sideband = (ST *)a.sideband;
-    const int H = a.H, T = a.T, n = a.n, row0 = a.t_off;
-    const int64_t t_cap = a.t_cap, sb_cap = a.sb_cap;
-    const uint8_t *flag_plane = a.flag_plane;
-    const int bh = blockIdx.y, b = bh / H, h = bh - b * H;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= T) return;
-    const int frb = (n + 7) >> 3;
-    const int64_t tiles = (t_cap + kTile - 1) / kTile;
-    const int row = row0 + t, tile_row = row & ~(kTile - 1);
-    const uint8_t *fr = flag_plane + ((size_t)bh * t_cap + row) * frb;
-    // the row's flag bits as they are now, in registers (up to 256 chunks): rows whose entries do not fit clear bits
-    // while this one runs
-    uint64_t mine[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int k = 0; k < 32; k++)
-        if (k < frb) mine[k >> 3] |= (uint64_t)fr[k] << (8 * (k & 7));
-    if (!(mine[0] | mine[1] | mine[2] | mine[3])) return;
-    int before = a.sb_tile_off[(size_t)bh * tiles + (row >> 4)];
-    const uint8_t *f0 = flag_plane + ((size_t)bh * t_cap + tile_row) * frb;
-    for (int k = 0; k < (row - tile_row) * frb; k++) before += __popc((uint32_t)f0[k]);
-    const ST *xr = x + b * a.xsb + h * a.xsh + (int64_t)t * a.xst;
-    int k = before;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        for (uint64_t bits = mine[q]; bits; bits &= bits - 1) {
-            const int c = 64 * q + __builtin_ctzll(bits);
-            if (c >= n) break;
-            if (k < sb_cap) {
-                ST *dst = sideband + ((size_t)bh * sb_cap + k) * 4;
-                for (int j = 0; j < 4; j++) dst[j] = xr[c * 4 + j];
-                if (a.sb_coord) a.sb_coord[(size_t)bh * sb_cap + k] = (uint16_t)(((row & (kTile - 1)) << 8) | c);
             } else {
-                *a.overflow = 1;
-                degrade_to_plain<D>(a, (size_t)bh * t_cap + row, c, xr + c * 4);
+                for (int k = 0; k < rows * frb; k++) cnt += __popc((uint32_t)f[k]);
             }
-            k++;
+        }
+        int total;
+        const int before = block_scan<1024>(cnt, part, total);
+        if (i < n_tiles) to[i] = base + before;
+        base += total;
+    }
+    __syncthreads();                             // every wavefront has read the count
+    if (threadIdx.x == 0) a.sb_count[bh] = base;
+}
+// Pass 2: one thread per new row (the 16 rows of a tile are 16 neighbouring lanes) copies the row's flagged chunks behind
+// those of the tile's earlier rows.  (4 x 8 x 4001 rows, one tensor: 8.5 + 4.8 us for counting and scanning apart, and
+// 10 us for the copy with every row reading the flags of the tile's earlier rows again.)
+template <class D>
+__global__ __launch_bounds__(256) void tile_copy_kernel(CompactPair pair) {
+    using ST = typename D::storage;
+    const CompactCall &a = pair.c[blockIdx.z];
+    const int bh = blockIdx.y, b = bh / a.H, h = bh - b * a.H;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int frb = (a.n + 7) >> 3, row = a.t_off + t;
+    const int64_t tiles = (a.t_cap + kTile - 1) / kTile;
+    uint64_t own[4] = {0, 0, 0, 0};              // the row's flags, read before any row of the tile clears bits
+    const int cnt = t < a.T ? row_flags(a.flag_plane + ((size_t)bh * a.t_cap + row) * frb, frb, flag_words(a.flag_plane, frb), own) : 0;
+    int before = cnt;
+    for (int o = 1; o < kTile; o <<= 1) {
+        const int v = __shfl_up(before, o, kTile);
+        if ((threadIdx.x & (kTile - 1)) >= o) before += v;
+    }
+    before -= cnt;
+    if (!cnt) return;
+    copy_row<D>(a, bh, row, (const ST *)a.x + b * a.xsb + h * a.xsh + (int64_t)t * a.xst, own, a.sb_tile_off[(size_t)bh * tiles + (row >> 4)] + before,
+                pair.vec[blockIdx.z]);
+}
+
+// ---- cropping: rows from `len` on are forgotten ----
+// A thread per tile resets the offsets of the tiles that hold no kept row, the block clears their flags in 16-byte words.
+// The block that holds the tile of the cut works the new entry count out first: the tile's offset plus the flags of its
+// kept rows (the count as it was, where the tile was never written or the offsets disagree).
+constexpr int kCropTiles = 256;
+__global__ __launch_bounds__(kCropTiles) void crop_kernel(hqmq_crop_args a) {
+    const int z = blockIdx.z, bh = blockIdx.y, b = bh / a.H, frb = (a.n_chunks + 7) >> 3;
+    const int64_t tiles = (a.t_cap + kTile - 1) / kTile, first = (int64_t)blockIdx.x * kCropTiles;
+    const int64_t len = max(a.lengths ? a.lengths[b] : a.length, 0);
+    const int64_t cut = len / kTile, free_tile = (len + kTile - 1) / kTile;
+    if (first + kCropTiles <= cut || len >= a.t_cap) return;           // every row of the block is kept
+    int32_t *off = a.sb_tile_off[z] + bh * tiles;
+    uint8_t *flags = a.flag_plane[z] + (size_t)bh * a.t_cap * frb;
+    if (cut >= first && threadIdx.x == 0) {
+        const int at = off[cut], count = a.sb_count[z][bh];
+        if (at <= count) {
+            int kept = 0;
+            for (int i = 0; i < (int)(len - cut * kTile) * frb; i++) kept += __popc((uint32_t)flags[cut * kTile * frb + i]);
+            a.sb_count[z][bh] = min(at + kept, count);
         }
     }
+    __syncthreads();
+    const int64_t tile = first + threadIdx.x;
+    if (tile >= free_tile && tile < tiles) off[tile] = 0x7fffffff;
+    const int64_t lo = max(len, first * kTile) * frb, hi = min(a.t_cap, (first + kCropTiles) * kTile) * frb;      // bytes to clear
+    uint8_t *p = flags + lo;
+    const int64_t bytes = hi - lo, head = min(bytes, (int64_t)((16 - ((uintptr_t)p & 15)) & 15)), words = (bytes - head) / 16;
+    for (int64_t i = threadIdx.x; i < head; i += kCropTiles) p[i] = 0;
+    for (int64_t i = threadIdx.x; i < words; i += kCropTiles) reinterpret_cast<uint4 *>(p + head)[i] = uint4{0, 0, 0, 0};
+    for (int64_t i = head + words * 16 + threadIdx.x; i < bytes; i += kCropTiles) p[i] = 0;
 }
 
 }  // namespace hqmq
@@ -550,39 +679,47 @@ extern "C" int64_t hqmq_med3x_workspace_bytes(int H, int dtype) {
 }
 
 template <class D>
-static int run_med3x(const void *x, int64_t xsb, int64_t xsh, int64_t xst, int B, int H, int T, int n, float mult, uint32_t *ws,
-                     float *median, void *thr, int32_t *n_out, hipStream_t st) {
-    using ST = typename D::storage;
+static int run_med3x(const MedPair &a, int count, hipStream_t st) {
     const bool f32 = D::code == HQMQ_F32;
-    const int64_t words = ws_words(H, f32);
-    const int64_t per_head = (int64_t)B * T * n;
-    if (!f32 && per_head <= kSmallMax) {
-        const MedSmall a{x, xsb, xsh, xst, B, T, n, mult, median, thr, n_out};
-        hipLaunchKernelGGL((med_small_kernel<D, 1024>), dim3(H), dim3(1024), 0, st, a);
+    const int64_t per_head = (int64_t)a.B * a.T * a.n, rows = (int64_t)a.B * a.T;
+    // the block with the fewest wavefronts whose lanes hold all keys: a barrier costs more the more of them meet
+    auto fits = [&](int nt) { return a.n <= nt && rows <= (int64_t)(nt / a.n) * kSmallKeys; };
+    if (fits(1024)) {
+        const dim3 grid(a.H, 1, count);
+        if (fits(64)) hipLaunchKernelGGL((med_small_kernel<D, 64>), grid, dim3(64), 0, st, a);
+        else if (fits(256)) hipLaunchKernelGGL((med_small_kernel<D, 256>), grid, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((med_small_kernel<D, 1024>), grid, dim3(1024), 0, st, a);
         return hip_status(hipGetLastError());
     }
-    hipLaunchKernelGGL(fill_zero_kernel, dim3(1024), dim3(256), 0, st, ws, words);
-    int gx = (int)((per_head + 255) / 256);
-    if (gx > 2048) gx = 2048;
-    if (per_head >= (1 << 18)) {
-        const size_t lds = (size_t)(kBins1 + 1) * sizeof(uint32_t);
-        hipError_t e = hipFuncSetAttribute((const void *)med_hist_lds_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return (int)e;
-        int gl = (int)((per_head + 16383) / 16384);
-        if (gl > 128) gl = 128;
-        hipLaunchKernelGGL(med_hist_lds_kernel<D>, dim3(gl, H), dim3(1024), lds, st, (const ST *)x, xsb, xsh, xst, B, H, T, n, ws);
-    } else {
-        hipLaunchKernelGGL((med_hist_kernel<D, 0>), dim3(gx, H), dim3(256), 0, st, (const ST *)x, xsb, xsh, xst, B, H, T, n, ws);
+    const int64_t words = ws_words(a.H, f32);
+    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)(words / 1024 < 1024 ? (words + 1023) / 1024 : 1024), count), dim3(256), 0, st, a.t[0].ws,
+                       a.t[count - 1].ws, words);
+    // Blocks of about 4096 chunks while that leaves at most two per CU; larger calls get larger blocks (each costs its
+    // 32768 bins and some 3000 atomics), beyond 65535 chunks with 32-bit counters, one block per CU and tensor.
+    const int rps = a.n <= 1024 ? 1024 / a.n : 1;        // rows a block takes per step
+    int64_t blocks = (per_head + 4095) / 4096;
+    const int64_t most = 512 / ((int64_t)a.H * count) > 0 ? 512 / ((int64_t)a.H * count) : 1;
+    if (blocks > most) blocks = most;
+    bool wide = (rows + blocks - 1) / blocks * a.n > 60000;
+    if (wide) {
+        blocks = 256 / ((int64_t)a.H * count) > 0 ? 256 / ((int64_t)a.H * count) : 1;
+        if (blocks < 16) blocks = 16;
     }
-    hipLaunchKernelGGL(med_select1_kernel<D>, dim3(H), dim3(1024), 0, st, ws, H, per_head, mult, median, (ST *)thr, n_out);
+    int64_t rpb = (rows + blocks - 1) / blocks;
+    rpb = (rpb + rps - 1) / rps * rps;
+    wide = rpb * a.n > 65535;
+    blocks = (rows + rpb - 1) / rpb;
+    const dim3 grid((unsigned)blocks, a.H, count);
+    auto kern = wide ? med_hist_kernel<D, true> : med_hist_kernel<D, false>;
+    const size_t lds = ((size_t)(wide ? kBins1 : kBins1 / 2) + 1) * sizeof(uint32_t);
+    const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL(kern, grid, dim3(1024), lds, st, a, rpb);
+    hipLaunchKernelGGL(med_select_kernel<D>, dim3(a.H, 1, count), dim3(128), 0, st, a);
     if (f32) {
-        hipLaunchKernelGGL((med_hist_kernel<D, 1>), dim3(gx, H), dim3(256), 0, st, (const ST *)x, xsb, xsh, xst, B, H, T, n, ws);
-        hipLaunchKernelGGL(med_select2_kernel, dim3(H), dim3(1024), 0, st, ws, H, per_head, mult, median, (float *)thr);
-        if (n_out) {
-            hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(64), 0, st, (uint32_t *)n_out, (int64_t)H);
-            hipLaunchKernelGGL(count_gt_kernel, dim3(gx, H), dim3(256), 0, st, (const float *)x, xsb, xsh, xst, B, T, n,
-                               (const float *)thr, n_out);
-        }
+        hipLaunchKernelGGL(med_hist_low_kernel, grid, dim3(1024), 0, st, a, rpb);
+        hipLaunchKernelGGL(med_select_low_kernel, dim3(a.H, 1, count), dim3(1024), 0, st, a);
+        hipLaunchKernelGGL(count_gt_kernel, grid, dim3(1024), 0, st, a, rpb);
     }
     return hip_status(hipGetLastError());
 }
@@ -592,36 +729,36 @@ static int check_med3x(const Med3xCall &c) {
     if (c.B < 1 || c.H < 1 || c.H > 65535 || c.T < 1 || c.n < 1) return HQMQ_ERR_SHAPE;
     if (c.dtype != HQMQ_F32 && c.dtype != HQMQ_F16 && c.dtype != HQMQ_BF16) return HQMQ_ERR_DTYPE;
     if (c.ws_bytes < hqmq_med3x_workspace_bytes(c.H, c.dtype)) return HQMQ_ERR_WORKSPACE;
+    if ((int64_t)c.B * c.T * c.n > 0xffffffffll) return HQMQ_ERR_SHAPE;      // counters are 32-bit
     if (((uintptr_t)c.ws & 3) != 0) return HQMQ_ERR_ALIGN;
     return HQMQ_OK;
 }
 
-static int med3x_one(const Med3xCall &c, hipStream_t st) {
-    uint32_t *ws = (uint32_t *)c.ws;
-    switch (c.dtype) {
-        case HQMQ_F32: return run_med3x<F32>(c.x, c.xsb, c.xsh, c.xst, c.B, c.H, c.T, c.n, c.mult, ws, c.median, c.thr, c.n_out, st);
-        case HQMQ_F16: return run_med3x<F16>(c.x, c.xsb, c.xsh, c.xst, c.B, c.H, c.T, c.n, c.mult, ws, c.median, c.thr, c.n_out, st);
-        default: return run_med3x<BF16>(c.x, c.xsb, c.xsh, c.xst, c.B, c.H, c.T, c.n, c.mult, ws, c.median, c.thr, c.n_out, st);
+static int med3x_launch(const MedPair &a, int dtype, int count, hipStream_t st) {
+    switch (dtype) {
+        case HQMQ_F32: return run_med3x<F32>(a, count, st);
+        case HQMQ_F16: return run_med3x<F16>(a, count, st);
+        default: return run_med3x<BF16>(a, count, st);
     }
 }
 
 int hqmq::med3x_calls(const Med3xCall *c, int count, hipStream_t st) {
+    MedTensor t[2];
     for (int i = 0; i < count; i++) {
         const int rc = check_med3x(c[i]);
         if (rc) return rc;
+        const int elt = c[i].dtype == HQMQ_F32 ? 4 : 2;
+        const int vec = !(((uintptr_t)c[i].x | (uintptr_t)(c[i].xsb * elt) | (uintptr_t)(c[i].xsh * elt) | (uintptr_t)(c[i].xst * elt)) & (4 * elt - 1));
+        t[i] = MedTensor{c[i].x, c[i].xsb, c[i].xsh, c[i].xst, vec, c[i].mult, (uint32_t *)c[i].ws, c[i].median, c[i].thr, c[i].n_out};
     }
-    if (count == 2 && c[0].dtype == c[1].dtype && c[0].dtype != HQMQ_F32 && c[0].B == c[1].B && c[0].H == c[1].H &&
-        c[0].T == c[1].T && c[0].n == c[1].n && (int64_t)c[0].B * c[0].T * c[0].n <= kSmallMax) {
-        const MedSmall a{c[0].x, c[0].xsb, c[0].xsh, c[0].xst, c[0].B, c[0].T, c[0].n, c[0].mult, c[0].median, c[0].thr, c[0].n_out};
-        const MedSmall b{c[1].x, c[1].xsb, c[1].xsh, c[1].xst, c[1].B, c[1].T, c[1].n, c[1].mult, c[1].median, c[1].thr, c[1].n_out};
-        const dim3 grid(c[0].H, 2);
-        // (256 threads for a few thousand keys measured slower: 11.9 against 8.7 us, the norms load eight deep per thread)
-        if (c[0].dtype == HQMQ_F16) hipLaunchKernelGGL((med_small_pair_kernel<F16, 1024>), grid, dim3(1024), 0, st, a, b);
-        else hipLaunchKernelGGL((med_small_pair_kernel<BF16, 1024>), grid, dim3(1024), 0, st, a, b);
-        return hip_status(hipGetLastError());
+    // one set of launches for both tensors where their shapes agree and their workspaces are apart
+    if (count == 2 && c[0].dtype == c[1].dtype && c[0].B == c[1].B && c[0].H == c[1].H && c[0].T == c[1].T && c[0].n == c[1].n) {
+        const int64_t need = hqmq_med3x_workspace_bytes(c[0].H, c[0].dtype);
+        const uintptr_t w0 = (uintptr_t)c[0].ws, w1 = (uintptr_t)c[1].ws;
+        if (w0 + need <= w1 || w1 + need <= w0) return med3x_launch(MedPair{{t[0], t[1]}, c[0].B, c[0].H, c[0].T, c[0].n}, c[0].dtype, 2, st);
     }
     for (int i = 0; i < count; i++) {
-        const int rc = med3x_one(c[i], st);
+        const int rc = med3x_launch(MedPair{{t[i], t[i]}, c[i].B, c[i].H, c[i].T, c[i].n}, c[i].dtype, 1, st);
         if (rc) return rc;
     }
     return HQMQ_OK;
@@ -642,34 +779,30 @@ int hqmq::check_compact(const CompactCall &c) {
     return HQMQ_OK;
 }
 
-// whole 16-row tiles from an aligned first row: the three tile-parallel passes
+// whole 16-row tiles from an aligned first row: the two tile-parallel passes
 static bool bulk_compact(const CompactCall &c) {
     return !c.pos && (c.t_off % kTile) == 0 && c.T >= 512 && (int64_t)c.t_off + c.T <= c.t_cap && c.B * c.H <= 65535;
 }
 
-static int compact_one(const CompactCall &c, hipStream_t st) {
+static int launch_compact(const CompactPair &p, int count, hipStream_t st) {
+    const CompactCall &c = p.c[0];
     if (c.T == 0) return HQMQ_OK;
     if (bulk_compact(c)) {
-        const int n_tiles = (c.T + kTile - 1) / kTile, frb = (c.n + 7) >> 3;
-        hipLaunchKernelGGL(tile_count_kernel, dim3((n_tiles + 255) / 256, c.B * c.H), dim3(256), 0, st, c.flag_plane, c.t_cap, c.t_off,
-                           c.T, frb, n_tiles, c.sb_tile_off);
-        hipLaunchKernelGGL(tile_scan_kernel, dim3(c.B * c.H), dim3(1024), 0, st, c.t_cap, c.t_off, n_tiles, c.sb_tile_off, c.sb_count);
-        dim3 cgrid((c.T + 255) / 256, c.B * c.H);
-#define COPY(DT) hipLaunchKernelGGL(tile_copy_kernel<DT>, cgrid, dim3(256), 0, st, c)
+        hipLaunchKernelGGL(tile_scan_kernel, dim3(c.B * c.H, 1, count), dim3(1024), 0, st, p);
+        const dim3 grid((c.T + 255) / 256, c.B * c.H, count);
         switch (c.dtype) {
-            case HQMQ_F32: COPY(F32); break;
-            case HQMQ_F16: COPY(F16); break;
-            default: COPY(BF16); break;
+            case HQMQ_F32: hipLaunchKernelGGL(tile_copy_kernel<F32>, grid, dim3(256), 0, st, p); break;
+            case HQMQ_F16: hipLaunchKernelGGL(tile_copy_kernel<F16>, grid, dim3(256), 0, st, p); break;
+            default: hipLaunchKernelGGL(tile_copy_kernel<BF16>, grid, dim3(256), 0, st, p); break;
         }
-#undef COPY
         return hip_status(hipGetLastError());
     }
-    dim3 grid(c.B * c.H);
+    const dim3 grid(c.B * c.H, 1, count);
 #define LAUNCH(NT)                                                                                              \
     switch (c.dtype) {                                                                                          \
-        case HQMQ_F32: hipLaunchKernelGGL((compact_kernel<F32, NT>), grid, dim3(NT), 0, st, c); break;          \
-        case HQMQ_F16: hipLaunchKernelGGL((compact_kernel<F16, NT>), grid, dim3(NT), 0, st, c); break;          \
-        default: hipLaunchKernelGGL((compact_kernel<BF16, NT>), grid, dim3(NT), 0, st, c); break;               \
+        case HQMQ_F32: hipLaunchKernelGGL((compact_kernel<F32, NT>), grid, dim3(NT), 0, st, p); break;          \
+        case HQMQ_F16: hipLaunchKernelGGL((compact_kernel<F16, NT>), grid, dim3(NT), 0, st, p); break;          \
+        default: hipLaunchKernelGGL((compact_kernel<BF16, NT>), grid, dim3(NT), 0, st, p); break;               \
     }
     if (c.T <= 64) { LAUNCH(64) } else { LAUNCH(1024) }
 #undef LAUNCH
@@ -677,28 +810,33 @@ static int compact_one(const CompactCall &c, hipStream_t st) {
 }
 
 int hqmq::compact_calls(const CompactCall *c, int count, hipStream_t st) {
+    int vec[2] = {0, 0};
     for (int i = 0; i < count; i++) {
         const int rc = check_compact(c[i]);
         if (rc) return rc;
+        const int elt = c[i].dtype == HQMQ_F32 ? 4 : 2;
+        vec[i] = !(((uintptr_t)c[i].x | (uintptr_t)c[i].sideband | (uintptr_t)(c[i].xsb * elt) | (uintptr_t)(c[i].xsh * elt) | (uintptr_t)(c[i].xst * elt)) &
+                   (4 * elt - 1));
     }
-    if (count == 2 && c[0].T > 0 && c[0].dtype == c[1].dtype && c[0].B == c[1].B && c[0].H == c[1].H && c[0].T == c[1].T &&
-        c[0].n == c[1].n && !bulk_compact(c[0]) && !bulk_compact(c[1])) {
-        dim3 grid(c[0].B * c[0].H, 2);
-#define LAUNCH(NT)                                                                                                         \
-    switch (c[0].dtype) {                                                                                                  \
-        case HQMQ_F32: hipLaunchKernelGGL((compact_pair_kernel<F32, NT>), grid, dim3(NT), 0, st, c[0], c[1]); break;       \
-        case HQMQ_F16: hipLaunchKernelGGL((compact_pair_kernel<F16, NT>), grid, dim3(NT), 0, st, c[0], c[1]); break;       \
-        default: hipLaunchKernelGGL((compact_pair_kernel<BF16, NT>), grid, dim3(NT), 0, st, c[0], c[1]); break;            \
-    }
-        if (c[0].T <= 64) { LAUNCH(64) } else { LAUNCH(1024) }
-#undef LAUNCH
-        return hip_status(hipGetLastError());
-    }
+    if (count == 2 && c[0].dtype == c[1].dtype && c[0].B == c[1].B && c[0].H == c[1].H && c[0].T == c[1].T && c[0].n == c[1].n &&
+        bulk_compact(c[0]) == bulk_compact(c[1]))
+        return launch_compact(CompactPair{{c[0], c[1]}, {vec[0], vec[1]}}, 2, st);
     for (int i = 0; i < count; i++) {
-        const int rc = compact_one(c[i], st);
+        const int rc = launch_compact(CompactPair{{c[i], c[i]}, {vec[i], vec[i]}}, 1, st);
         if (rc) return rc;
     }
     return HQMQ_OK;
+}
+
+extern "C" int hqmq_crop(const hqmq_crop_args *a, void *stream) {
+    if (!a) return HQMQ_ERR_NULL;
+    if (a->count < 1 || a->count > 2 || a->B < 1 || a->H < 1 || (int64_t)a->B * a->H > 65535 || a->t_cap < 1 || a->n_chunks < 1) return HQMQ_ERR_SHAPE;
+    for (int i = 0; i < a->count; i++)
+        if (!a->flag_plane[i] || !a->sb_tile_off[i] || !a->sb_count[i]) return HQMQ_ERR_NULL;
+    const int64_t tiles = (a->t_cap + kTile - 1) / kTile;
+    hipLaunchKernelGGL(crop_kernel, dim3((unsigned)((tiles + kCropTiles - 1) / kCropTiles), a->B * a->H, a->count), dim3(kCropTiles), 0,
+                       (hipStream_t)stream, *a);
+    return hip_status(hipGetLastError());
 }
 
 extern "C" int hqmq_outlier_compact(const void *x, int64_t x_stride_b, int64_t x_stride_h, int64_t x_stride_t, int dtype, int B,

@@ -198,6 +198,22 @@ def outlier_compact(x: torch.Tensor, cache, t_off: int = 0, pos: Optional[torch.
             L.ptr(cache.sb_overflow), L.ptr(cache.sb_coord), C.byref(rows), L.stream_ptr(dev)), "hqmq_outlier_compact")
 
 
+def crop(caches, lengths) -> None:
+    """Outlier lists, tile offsets and flags of the PackedTensors (one, or K and V of equal shape) back to the state after
+    the first `lengths` rows: an int for all sequences or an int32 tensor [B] on the caches' device."""
+    c = caches[0]
+    a = L.CropArgs()
+    for i, t in enumerate(caches):
+        a.flag_plane[i], a.sb_tile_off[i], a.sb_count[i] = t.flags.data_ptr(), t.sb_tile_off.data_ptr(), t.sb_count.data_ptr()
+    a.count, a.B, a.H, a.t_cap, a.n_chunks = len(caches), c.B, c.H, c.t_cap, c.n
+    if isinstance(lengths, int):
+        a.length = max(0, min(lengths, c.t_cap))
+    else:
+        a.lengths = lengths.data_ptr()
+    with torch.cuda.device(c.device):
+        L.check(L.lib().hqmq_crop(C.byref(a), L.stream_ptr(c.device)), "hqmq_crop")
+
+
 def append_kv(k: torch.Tensor, v: torch.Tensor, k_cache, v_cache, k_joint, k_slack, v_joint, v_slack, radius_bits: int, *,
               t_off: int = 0, pos: Optional[torch.Tensor] = None, median_mult: Optional[float] = None):
     """Quantize the new rows k, v (B, H, T, d_h) into rows t_off.. of the two PackedTensors (shifted by pos[b]),

@@ -128,32 +128,7 @@ class PackedTensor:
         """Forgets the rows from `lengths` on (an int for all sequences or an int tensor [B]): the outlier list and
         its tile offsets go back to the state after the last kept row, so that the rows can be appended again.
         The planes themselves are left as they are (later appends overwrite them)."""
-        B, H = self.B, self.H
-        if isinstance(lengths, int):
-            lens = torch.full((B,), lengths, dtype=torch.int64, device=self.device)
-            self.length = min(self.length, lengths)
-        else:
-            lens = lengths.to(device=self.device, dtype=torch.int64).clamp(min=0)
-            self.lengths = lens.to(torch.int32)
-        if self.flags is None:
-            return
-        tiles = self.t_cap // TILE
-        tile, r = lens // TILE, lens % TILE
-        tc = tile.clamp(max=tiles - 1)
-        off = self.sb_tile_off.gather(2, tc.view(B, 1, 1).expand(B, H, 1)).squeeze(2).to(torch.int64)
-        # flagged chunks of the kept rows of the tile the cut falls into
-        rows = tc.view(B, 1, 1) * TILE + torch.arange(TILE, device=self.device).view(1, 1, TILE)
-        fl = self.flags.gather(2, rows.view(B, 1, TILE, 1).expand(B, H, TILE, self.flags.shape[-1]))
-        bits = sum((fl >> i) & 1 for i in range(8)).to(torch.int64).sum(-1)                          # (B, H, TILE)
-        kept = torch.arange(TILE, device=self.device).view(1, 1, TILE) < r.view(B, 1, 1)
-        count = self.sb_count.to(torch.int64)
-        new = torch.where((tile >= tiles).view(B, 1) | (off > count), count, off + (bits * kept).sum(-1))
-        self.sb_count.copy_(torch.minimum(new, count).to(torch.int32))
-        first_free = (lens + TILE - 1) // TILE             # tiles from here on hold no kept row: unwritten again
-        gone = torch.arange(tiles, device=self.device).view(1, 1, tiles) >= first_free.view(B, 1, 1)
-        self.sb_tile_off.masked_fill_(gone.expand(B, H, tiles), 0x7fffffff)
-        dropped = torch.arange(self.t_cap, device=self.device).view(1, 1, self.t_cap, 1) >= lens.view(B, 1, 1, 1)
-        self.flags.masked_fill_(dropped, 0)                # no flag without an entry behind it
+        _crop([self], lengths)
 
     def with_fp8_table(self) -> "PackedTensor":
         """A view of the same planes whose joint table is rounded to float8_e4m3fn (kept in the table's dtype:
@@ -184,6 +159,52 @@ class PackedTensor:
                               "sideband_frac")
 
 
+def _crop_outliers_torch(t, lengths) -> None:
+    """What ops.crop does, in torch: for caches whose tensors are not on the GPU (bookkeeping without kernels)."""
+    B, H, tiles = t.B, t.H, t.t_cap // TILE
+    lens = torch.full((B,), lengths, dtype=torch.int64, device=t.device) if isinstance(lengths, int) else lengths.to(torch.int64)
+    tile, r = lens // TILE, lens % TILE
+    tc = tile.clamp(max=tiles - 1)
+    off = t.sb_tile_off.gather(2, tc.view(B, 1, 1).expand(B, H, 1)).squeeze(2).to(torch.int64)
+    # flagged chunks of the kept rows of the tile the cut falls into
+    rows = tc.view(B, 1, 1) * TILE + torch.arange(TILE, device=t.device).view(1, 1, TILE)
+    fl = t.flags.gather(2, rows.view(B, 1, TILE, 1).expand(B, H, TILE, t.flags.shape[-1]))
+    bits = sum((fl >> i) & 1 for i in range(8)).to(torch.int64).sum(-1)                          # (B, H, TILE)
+    kept = torch.arange(TILE, device=t.device).view(1, 1, TILE) < r.view(B, 1, 1)
+    count = t.sb_count.to(torch.int64)
+    new = torch.where((tile >= tiles).view(B, 1) | (off > count), count, off + (bits * kept).sum(-1))
+    t.sb_count.copy_(torch.minimum(new, count).to(torch.int32))
+    first_free = (lens + TILE - 1) // TILE             # tiles from here on hold no kept row: unwritten again
+    gone = torch.arange(tiles, device=t.device).view(1, 1, tiles) >= first_free.view(B, 1, 1)
+    t.sb_tile_off.masked_fill_(gone.expand(B, H, tiles), 0x7fffffff)
+    dropped = torch.arange(t.t_cap, device=t.device).view(1, 1, t.t_cap, 1) >= lens.view(B, 1, 1, 1)
+    t.flags.masked_fill_(dropped, 0)                   # no flag without an entry behind it
+
+
+def _crop(tensors, lengths) -> None:
+    """Crops PackedTensors of one cache; those that carry outliers share a launch where their shapes agree."""
+    if isinstance(lengths, int):
+        for t in tensors:
+            t.length = min(t.length, lengths)
+    else:
+        lengths = lengths.to(device=tensors[0].device).clamp(min=0).to(torch.int32).contiguous()
+        for t in tensors:
+            t.lengths = lengths
+    flagged = [t for t in tensors if t.flags is not None]
+    if not flagged:
+        return
+    if flagged[0].device.type != "cuda":
+        for t in flagged:
+            _crop_outliers_torch(t, lengths)
+        return
+    from . import ops
+    if len(flagged) == 2 and any(getattr(flagged[0], k) != getattr(flagged[1], k) for k in ("B", "H", "t_cap", "n", "device")):
+        for t in flagged:
+            ops.crop([t], lengths)
+    else:
+        ops.crop(flagged, lengths)
+
+
 @dataclass
 class PackedKV:
     """The compressed K and V of one layer."""
@@ -199,5 +220,4 @@ class PackedKV:
 
     def crop_(self, lengths) -> None:
         """Forgets the rows from `lengths` on in K and V (see PackedTensor.crop_)."""
-        self.K.crop_(lengths)
-        self.V.crop_(lengths)
+        _crop([self.K, self.V], lengths)

@@ -156,6 +156,21 @@ int hqmq_outlier_compact(const void *x, int64_t x_stride_b, int64_t x_stride_h, 
                          const int32_t *pos, void *sideband, int64_t sb_cap, int32_t *sb_tile_off, int32_t *sb_count,
                          int32_t *overflow, uint16_t *sb_coord, const hqmq_packed_rows *planes, void *stream);
 
+/* Forget the rows from lengths[b] (or `length`) on of one tensor or of K and V: the outlier list, its tile offsets and the
+ * flags go back to the state after the last kept row, so that the rows can be appended again; the code planes are left
+ * as they are.  No counterpart in the reference. */
+typedef struct hqmq_crop_args {
+    uint8_t *flag_plane[2];
+    int32_t *sb_tile_off[2], *sb_count[2];
+    int count;                /* tensors: 1 or 2, of equal shape */
+    int B, H;
+    int64_t t_cap;
+    int n_chunks;
+    const int32_t *lengths;   /* [B] or NULL: `length` for every sequence; negative counts as 0 */
+    int length;
+} hqmq_crop_args;
+int hqmq_crop(const hqmq_crop_args *a, void *stream);
+
 /* One append of new K and V rows to a packed cache: Med3x threshold (when median_mult > 0), quantize + pack,
  * sideband compaction, for both tensors.  The results are those of hqmq_med3x_threshold, hqmq_quantize and
  * hqmq_outlier_compact called in that order for K and then for V (what KVQuantizer.quantize_K / quantize_V of

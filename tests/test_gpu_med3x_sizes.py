@@ -1,0 +1,82 @@
+"""Med3x statistics, compaction and cropping at the sizes where a launch changes its kind: keys in registers of one
+wavefront (512 chunks per head) and of a block (8192), histograms with packed and with 32-bit counters, appends on both
+sides of the bulk compaction (512 rows), cuts on and off a tile."""
+import pytest
+import torch
+
+from oracle import c_oracle as CO
+from tests.helpers import DT, bit_equal, kv_input
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dn", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("shape", [(1, 2, 16, 128), (1, 2, 17, 128), (3, 2, 1, 80), (2, 1, 128, 128), (1, 1, 257, 128), (1, 2, 2049, 20),
+                                   (1, 1, 3000, 128), (2, 1, 5, 4200)])
+def test_threshold_at_the_edges(dn, shape):
+    from hqmq_amd import ops
+    dt = DT[dn]
+    x = kv_input(shape, dt, seed=sum(shape), outlier_p=0.05)
+    want = CO.med3x(x, 3.0)
+    for view in (x.to(DEV), torch.nn.functional.pad(x, (1, 1)).to(DEV)[..., 1:1 + shape[-1]], x.to(DEV).transpose(1, 2).contiguous().transpose(1, 2)):
+        med, thr, cnt = ops.med3x_threshold(view, 3.0)
+        assert torch.equal(med.cpu(), want["median"]) and bit_equal(thr, want["threshold"])
+        assert torch.equal(cnt.cpu().long(), want["mask"].sum(dim=(0, 2, 3)))
+
+
+@pytest.mark.parametrize("dn", ["fp16", "bf16"])
+def test_wide_and_packed_counters_agree(dn):
+    """A head of 5 M chunks (32-bit counters) and the order statistics of torch.sort on its norms."""
+    from hqmq_amd import ops
+    dt = DT[dn]
+    x = torch.randn(5, 1, 32768, 128, generator=torch.Generator(device=DEV).manual_seed(3), device=DEV).to(dt)
+    med, thr, cnt = ops.med3x_threshold(x, 1.5)
+    mask = ops.outlier_mask(x, thr)
+    assert int(mask.sum()) == int(cnt[0])
+    below, above = int((~ops.outlier_mask(x, med.to(dt))).sum()), int(ops.outlier_mask(x, med.to(dt)).sum())
+    n = mask.numel()
+    assert above <= n // 2 and below >= n // 2                   # the median is a norm of the call: at most half lie above it
+    a, b = ops.med3x_threshold(x[:1], 1.5), ops.med3x_threshold(torch.cat([x[:1]] * 5), 1.5)      # the same norms five times over
+    assert float(a[1]) == float(b[1]) or abs(float(a[0]) - float(b[0])) < 1e-2 * float(a[0])
+    assert 5 * int(a[2]) == int(b[2]) or float(a[1]) != float(b[1])
+
+
+@pytest.mark.parametrize("dn,d_h", [("fp16", 128), ("bf16", 64), ("fp32", 48), ("fp16", 16)])
+@pytest.mark.parametrize("T", [33, 64, 65, 511, 512, 513, 2100])
+def test_append_lists_and_crop(dn, d_h, T):
+    """Sideband entries in (token, chunk) order, tile offsets and counts equal what the mask says, before and after a cut."""
+    import hqmq
+    dt = DT[dn]
+    B, H, n = 2, 2, d_h // 4
+    w = hqmq.with_outlier_extraction(hqmq.HQMQ(n_layers=1, n_heads=H, secondary_size=24, radius_bits=3, device=DEV), C=3.0)
+    k, v = kv_input((B, H, T, d_h), dt, seed=T, outlier_p=0.1).to(DEV), kv_input((B, H, T, d_h), dt, seed=T + 1, outlier_p=0.02).to(DEV)
+    cache = w.new_cache(B, T, d_h, dt, 0, sideband_frac=0.5)
+    w.append(cache, k, v, 0)
+
+    def check(lens):
+        for pt, x in ((cache.K, k), (cache.V, v)):
+            mask = w.encode(x, 0, 0)["mask"]
+            for b in range(B):
+                m = mask[b].clone()
+                m[:, lens[b]:] = False
+                assert torch.equal(pt.sb_count[b].long(), m.sum(dim=(1, 2)))
+                for h in range(H):
+                    tok, chunk = m[h].nonzero(as_tuple=True)
+                    assert torch.equal(pt.sideband[b, h, :len(tok)], x[b, h].view(T, n, 4)[tok, chunk])
+                    assert torch.equal(pt.sb_coord[b, h, :len(tok)].long(), (tok % 16) << 8 | chunk)
+                    tiles = (lens[b] + 15) // 16
+                    before = torch.tensor([int((tok < 16 * i).sum()) for i in range(tiles)])
+                    assert torch.equal(pt.sb_tile_off[b, h, :tiles].long().cpu(), before)
+                    assert bool((pt.sb_tile_off[b, h, (pt.t_cap if lens[b] == T else lens[b] + 15) // 16:] == 0x7fffffff).all())
+                    flags = torch.stack([(pt.flags[b, h] >> i) & 1 for i in range(8)], -1).reshape(pt.t_cap, -1)[:, :n].bool()
+                    assert torch.equal(flags[:T], m[h]) and not bool(flags[T:].any())
+
+    check([T, T])
+    cut = torch.tensor([T // 2, (T // 3) // 16 * 16], dtype=torch.int32, device=DEV)
+    cache.crop_(cut)
+    check(cut.tolist())
+    cache.crop_(5)
+    check([min(5, c) for c in cut.tolist()])
+    cache.crop_(0)
+    check([0, 0])
