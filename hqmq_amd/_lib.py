@@ -109,6 +109,11 @@ def lib():
         for name in ("hqmq_med3x_workspace_bytes", "hqmq_attn_workspace_bytes", "hqmq_attn_static_scratch_bytes",
                      "hqmq_search_grid_bytes"):
             getattr(L, name).restype = i64
+        # the calls of a decode loop take addresses as plain integers
+        for name, n in (("hqmq_attn_fwd", 2), ("hqmq_attn_fwd_static", 2), ("hqmq_quantize_grid", 3), ("hqmq_append_kv_grid", 5), ("hqmq_crop", 2),
+                        ("hqmq_quantize", 2), ("hqmq_append_kv", 3)):
+            getattr(L, name).argtypes = [vp] * n
+        L.hqmq_med3x_threshold.argtypes = [vp, i64, i64, i64, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, vp, i64, vp, vp, vp, vp]
         _lib = L
     return _lib
 
@@ -142,6 +147,27 @@ def ptr(t):
 
 def stream_ptr(device=None):
     return vp(torch.cuda.current_stream(device).cuda_stream)
+
+
+def addr(t) -> int:
+    """The address as an integer, for calls with declared argument types and for structure fields; 0 for None."""
+    return t.data_ptr() if t is not None else 0
+
+
+# the current stream of a device as an integer, without a Stream object
+raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_getCurrentRawStream") else (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
+def call(fn, what: str, index: int, *args) -> None:
+    """fn(*args, stream) on device `index` and its current stream; raises on a bad status."""
+    if torch.cuda.current_device() == index:
+        status = fn(*args, raw_stream(index))
+    else:
+        with torch.cuda.device(index):
+            status = fn(*args, raw_stream(index))
+    if status != 0:
+        check(status, what)
 
 
 def require_gpu(t: torch.Tensor, name: str) -> None:

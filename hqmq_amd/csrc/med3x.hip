@@ -87,7 +87,8 @@ __device__ __forceinline__ void for_each_norm(const MedTensor &m, const MedPair 
         const int64_t b = r / a.T;
         int t = (int)(r - b * a.T);
         const ST *p = (const ST *)m.x + b * m.xsb + h * m.xsh + (int64_t)t * m.xst + c * 4;
-        const int64_t step = per * m.xst, wrap = m.xsb - a.T * m.xst;
+        const int dq = per / a.T, dt = per - dq * a.T;               // `per` rows on: dq sequences and dt tokens
+        const int64_t step = dq * m.xsb + dt * m.xst, wrap = m.xsb - a.T * m.xst;
         while (r < r1) {
             RawChunk<D> raw[U];
             int k = 0;
@@ -98,9 +99,9 @@ __device__ __forceinline__ void for_each_norm(const MedTensor &m, const MedPair 
                     k = i + 1;
                 }
                 r += per;
-                t += per;
+                t += dt;
                 p += step;
-                while (t >= a.T) { t -= a.T; p += wrap; }
+                if (t >= a.T) { t -= a.T; p += wrap; }
             }
 #pragma unroll
             for (int i = 0; i < U; i++)
@@ -365,103 +366,101 @@ __global__ __launch_bounds__(1024) void count_gt_kernel(MedPair a, int64_t rows_
 }
 
 // Small calls (a decode step appends B * n chunks per head): norms, exact order statistics and count in one launch, one
-// block per head, eight keys per lane in registers.  The key of rank r is the largest v with fewer than r + 1 keys below
+// block per head, up to eight keys per lane in registers.  The key of rank r is the largest v with fewer than r + 1 keys below
 // it, found bit by bit from the top: a compare and a scalar bit count per key, one barrier per round (none in a block of
 // one wavefront); two bits, three thresholds a round.  The second rank is the next one: the same key again, or the smallest key above it.
 // (256-bin histograms of keys in LDS, two passes per rank, took 9.5 us for 2048 chunks per head.)
-constexpr int kSmallKeys = 8;
-template <class D, int NT>
+template <class D, int NT, int KEYS>
 __global__ __launch_bounds__(NT) void med_small_kernel(MedPair a) {
     constexpr int W = NT / 64, BITS = D::code == HQMQ_F32 ? 31 : 15;
-    __shared__ uint4 part[2][W];
+    __shared__ uint4 sums[W > 1 ? BITS / 2 + 4 : 1];
     const MedTensor &m = a.t[blockIdx.z];
-    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int per_head = a.B * a.T * a.n, rows = a.B * a.T;
     using ST = typename D::storage;
+    if (W > 1) {
+        if (tid < BITS / 2 + 4) sums[tid] = uint4{0, 0, 0, 0};
+        __syncthreads();
+    }
     // lane (rl, c) holds chunk c of rows rl, rl + per, ..: one division per lane, not one per key
     const int per = NT / a.n, rl = tid / a.n, c = tid - rl * a.n;
-    uint32_t key[kSmallKeys];
-    bool nan = false, have[kSmallKeys];
+    uint32_t key[KEYS];
+    bool nan = false, have[KEYS];
     {
-        RawChunk<D> raw[kSmallKeys] = {};
+        RawChunk<D> raw[KEYS] = {};
         const int b0 = rl / a.T;
         int r = rl < per ? rl : rows, t = rl - b0 * a.T;
         const ST *p = (const ST *)m.x + b0 * m.xsb + h * m.xsh + (int64_t)t * m.xst + c * 4;
-        const int64_t step = per * m.xst, wrap = m.xsb - a.T * m.xst;
+        const int dq = per / a.T, dt = per - dq * a.T;               // `per` rows on: dq sequences and dt tokens
+        const int64_t step = dq * m.xsb + dt * m.xst, wrap = m.xsb - a.T * m.xst;
 #pragma unroll
-        for (int i = 0; i < kSmallKeys; i++) {
+        for (int i = 0; i < KEYS; i++) {
             have[i] = r < rows;
             if (have[i]) raw[i].load(p, m.vec);
             r += per;
-            t += per;
+            t += dt;
             p += step;
-            while (t >= a.T) { t -= a.T; p += wrap; }
+            if (t >= a.T) { t -= a.T; p += wrap; }
         }
 #pragma unroll
-        for (int i = 0; i < kSmallKeys; i++) {
+        for (int i = 0; i < KEYS; i++) {
             const float nrm = chunk_norm_d<D>(raw[i].get(0), raw[i].get(1), raw[i].get(2), raw[i].get(3));
             nan |= have[i] && is_nan(nrm);
             key[i] = have[i] ? (D::code == HQMQ_F32 ? __float_as_uint(nrm) : norm_bits<D>(nrm) >> 16) : 0x7fffffffu;    // absent: above every key
         }
     }
-    int turn = 0;
-    // sum of a wave-uniform number over the block
-    auto total = [&](uint32_t v) -> uint32_t {
-        if (W == 1) return v;
-        if (lane == 0) part[turn][wave].x = v;
+    // Sums over the block of up to three wave-uniform numbers: one LDS atomic each per wavefront into the round's own
+    // counters, one broadcast read back (sixteen wavefronts reading sixteen partial sums each took 1.7 us a round).
+    int round = 0;
+    auto total3 = [&](uint32_t &x, uint32_t &y, uint32_t &z) {
+        if (W == 1) return;
+        if (lane == 0) {
+            atomicAdd(&sums[round].x, x);
+            atomicAdd(&sums[round].y, y);
+            atomicAdd(&sums[round].z, z);
+        }
         __syncthreads();
-        uint32_t s = 0;
-#pragma unroll
-        for (int w = 0; w < W; w++) s += part[turn][w].x;
-        turn ^= 1;
-        return s;
+        const uint4 s = sums[round++];
+        x = s.x; y = s.y; z = s.z;
     };
-    auto below = [&](uint32_t v) -> uint32_t {
-        uint32_t c = 0;
-#pragma unroll
-        for (int i = 0; i < kSmallKeys; i++) c += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[i] < v));
-        return total(c);
-    };
-    if (total(__builtin_amdgcn_ballot_w64(nan) != 0ull ? 1u : 0u) > 0u) {
-        if (tid == 0) nan_threshold<D>(m, h);
-        return;
-    }
     const uint32_t r_lo = (uint32_t)((per_head - 1) / 2), r_hi = (uint32_t)(per_head / 2);
-    uint32_t k_lo = 0;
+    uint32_t k_lo = 0, any_nan = __builtin_amdgcn_ballot_w64(nan) != 0ull ? 1u : 0u;
+#pragma unroll 1
     for (int bit = BITS - 1; bit >= 0; bit -= 2) {       // two bits a round (the last has one: its three thresholds coincide)
         const uint32_t v1 = k_lo | 1u << (bit - (bit ? 1 : 0)), v2 = k_lo | 1u << bit, v3 = v2 | v1;
         uint32_t c1 = 0, c2 = 0, c3 = 0;
 #pragma unroll
-        for (int i = 0; i < kSmallKeys; i++) {
+        for (int i = 0; i < KEYS; i++) {
             c1 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[i] < v1));
             c2 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[i] < v2));
             c3 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[i] < v3));
         }
-        if (W > 1) {
-            if (lane == 0) part[turn][wave] = uint4{c1, c2, c3, 0u};
-            __syncthreads();
-            c1 = c2 = c3 = 0;
-#pragma unroll
-            for (int w = 0; w < W; w++) { const uint4 q = part[turn][w]; c1 += q.x; c2 += q.y; c3 += q.z; }
-            turn ^= 1;
-        }
+        total3(c1, c2, c3);
         k_lo = c3 <= r_lo ? v3 : c2 <= r_lo ? v2 : c1 <= r_lo ? v1 : k_lo;
     }
-    uint32_t k_hi = k_lo;
-    if (r_hi != r_lo && below(k_lo + 1u) <= r_hi) {
-        uint32_t mn = 0xffffffffu;
+    // how many keys are at most k_lo, and the smallest one above it (complemented: a sum's place serves a maximum as well)
+    uint32_t upto = 0, above = 0;
 #pragma unroll
-        for (int i = 0; i < kSmallKeys; i++) mn = min(mn, key[i] > k_lo ? key[i] : 0xffffffffu);
-        mn = ~group_max(~mn, 64, [](uint32_t p, uint32_t q) { return max(p, q); });
-        if (W > 1) {
-            if (lane == 0) part[turn][wave].x = mn;
-            __syncthreads();
-#pragma unroll
-            for (int w = 0; w < W; w++) mn = min(mn, part[turn][w].x);
-            turn ^= 1;
-        }
-        k_hi = mn;
+    for (int i = 0; i < KEYS; i++) {
+        upto += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[i] <= k_lo));
+        above = max(above, key[i] > k_lo ? ~key[i] : 0u);
     }
+    above = group_max(above, 64, [](uint32_t p, uint32_t q) { return max(p, q); });
+    if (W > 1) {
+        if (lane == 0) {
+            atomicAdd(&sums[round].x, upto);
+            atomicMax(&sums[round].y, above);
+            atomicAdd(&sums[round].z, any_nan);
+        }
+        __syncthreads();
+        upto = sums[round].x; above = sums[round].y; any_nan = sums[round].z;
+        round++;
+    }
+    if (any_nan) {
+        if (tid == 0) nan_threshold<D>(m, h);
+        return;
+    }
+    const uint32_t k_hi = upto > r_hi ? k_lo : ~above;
     auto value = [](uint32_t k) { return D::code == HQMQ_F32 ? __uint_as_float(k) : key_value<D>(k); };
     const float x = value(k_lo), y = value(k_hi);
     const float med = r_lo == r_hi ? x : y - (y - x) * 0.5f;
@@ -469,9 +468,10 @@ __global__ __launch_bounds__(NT) void med_small_kernel(MedPair a) {
     if (m.n_out) {
         uint32_t c = 0;
 #pragma unroll
-        for (int i = 0; i < kSmallKeys; i++)
+        for (int i = 0; i < KEYS; i++)
             c += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(have[i] && value(key[i]) > tv));
-        c = total(c);
+        uint32_t y = 0, z = 0;
+        total3(c, y, z);
         if (tid == 0) m.n_out[h] = (int32_t)c;
     }
     if (tid == 0) finish_threshold<D>(x, y, r_lo == r_hi, m.mult, h, m.median, (ST *)m.thr);
@@ -682,13 +682,15 @@ template <class D>
 static int run_med3x(const MedPair &a, int count, hipStream_t st) {
     const bool f32 = D::code == HQMQ_F32;
     const int64_t per_head = (int64_t)a.B * a.T * a.n, rows = (int64_t)a.B * a.T;
-    // the block with the fewest wavefronts whose lanes hold all keys: a barrier costs more the more of them meet
-    auto fits = [&](int nt) { return a.n <= nt && rows <= (int64_t)(nt / a.n) * kSmallKeys; };
-    if (fits(1024)) {
+    // Few keys per lane before few lanes: such a call lasts about as long as its code takes to arrive (every launch starts
+    // with cold instruction caches), and the code is written out once per key.
+    auto fits = [&](int nt, int keys) { return a.n <= nt && rows <= (int64_t)(nt / a.n) * keys; };
+    if (fits(1024, 8)) {
         const dim3 grid(a.H, 1, count);
-        if (fits(64)) hipLaunchKernelGGL((med_small_kernel<D, 64>), grid, dim3(64), 0, st, a);
-        else if (fits(256)) hipLaunchKernelGGL((med_small_kernel<D, 256>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((med_small_kernel<D, 1024>), grid, dim3(1024), 0, st, a);
+        if (fits(64, 1)) hipLaunchKernelGGL((med_small_kernel<D, 64, 1>), grid, dim3(64), 0, st, a);
+        else if (fits(256, 2)) hipLaunchKernelGGL((med_small_kernel<D, 256, 2>), grid, dim3(256), 0, st, a);
+        else if (fits(1024, 2)) hipLaunchKernelGGL((med_small_kernel<D, 1024, 2>), grid, dim3(1024), 0, st, a);
+        else hipLaunchKernelGGL((med_small_kernel<D, 1024, 8>), grid, dim3(1024), 0, st, a);
         return hip_status(hipGetLastError());
     }
     const int64_t words = ws_words(a.H, f32);

@@ -39,8 +39,25 @@ def build_joint(raw_hs4: torch.Tensor, dtype: torch.dtype):
     return joint, slack
 
 
-def _grid(slack: Optional[torch.Tensor]):
-    return L.ptr(getattr(slack, "hqmq_grid", None))
+def _book(joint: torch.Tensor, slack: Optional[torch.Tensor], radius_bits: int, n: int):
+    """A QuantizeArgs with everything a codebook fixes, kept with `slack` from call to call, and the address of the cell
+    lists."""
+    book = getattr(slack, "hqmq_book", None)
+    if book is not None and book[0] is joint and book[1] == joint.data_ptr() and book[2] == (radius_bits, n):
+        return book[3], book[4]
+    a = L.QuantizeArgs()
+    a.dtype, a.H, a.n_chunks = _dt(joint), joint.shape[0], n
+    a.joint, a.slack = L.addr(joint), L.addr(slack)
+    a.secondary_size, a.radius_bits = joint.shape[1] // 24, radius_bits
+    grid = L.addr(getattr(slack, "hqmq_grid", None))
+    if slack is not None:
+        slack.hqmq_book = (joint, joint.data_ptr(), (radius_bits, n), a, grid)
+    return a, grid
+
+
+def _check_joint(x: torch.Tensor, joint: torch.Tensor) -> None:
+    if joint.dtype != x.dtype or joint.shape[0] != x.shape[1] or not joint.is_contiguous():
+        raise ValueError("joint must be a contiguous (H, 24S, 4) table in the dtype of x")
 
 
 def _strided_x(x: torch.Tensor):
@@ -67,56 +84,45 @@ def quantize(x: torch.Tensor, joint: torch.Tensor, slack: Optional[torch.Tensor]
     if d_h % 4 != 0:
         raise ValueError(f"d_head={d_h} not divisible by 4")
     n = d_h // 4
-    S = joint.shape[1] // 24
-    if joint.dtype != x.dtype or joint.shape[0] != H or not joint.is_contiguous():
-        raise ValueError("joint must be a contiguous (H, 24S, 4) table in the dtype of x")
+    _check_joint(x, joint)
     dev = x.device
-    a = L.QuantizeArgs()
-    a.x = L.ptr(x)
-    a.x_stride_b, a.x_stride_h, a.x_stride_t = x.stride(0), x.stride(1), x.stride(2)
-    a.dtype = _dt(x)
-    a.B, a.H, a.T, a.n_chunks = B, H, T, n
-    a.joint = L.ptr(joint)
-    a.slack = L.ptr(slack)
-    a.secondary_size, a.radius_bits, a.algo = S, radius_bits, algo
+    tmpl, grid = _book(joint, slack, radius_bits, n)
+    a = L.QuantizeArgs.from_buffer_copy(tmpl)
+    a.x = x.data_ptr()
+    a.x_stride_b, a.x_stride_h, a.x_stride_t, _ = x.stride()
+    a.B, a.T, a.algo = B, T, algo
     out = {}
-    keep = [x, joint, slack]
     if want_codes:
-        out["idx"] = torch.empty(B, H, T, n, dtype=torch.int32, device=dev)
-        out["rq"] = torch.empty(B, H, T, n, dtype=torch.int32, device=dev)
-        out["r_max"] = torch.empty(B, H, T, dtype=x.dtype, device=dev)
-        a.idx_out, a.rq_out, a.rmax_out = L.ptr(out["idx"]), L.ptr(out["rq"]), L.ptr(out["r_max"])
+        out["idx"], out["rq"] = x.new_empty((B, H, T, n), dtype=torch.int32), x.new_empty((B, H, T, n), dtype=torch.int32)
+        out["r_max"] = x.new_empty((B, H, T))
+        a.idx_out, a.rq_out, a.rmax_out = out["idx"].data_ptr(), out["rq"].data_ptr(), out["r_max"].data_ptr()
     if want_dense:
-        out["out"] = torch.empty(B, H, T, d_h, dtype=x.dtype, device=dev)
-        a.dense_out = L.ptr(out["out"])
+        out["out"] = x.new_empty((B, H, T, d_h))
+        a.dense_out = out["out"].data_ptr()
     if thr is not None:
         thr = thr.to(x.dtype).contiguous()
-        keep.append(thr)
-        a.thr = L.ptr(thr)
+        a.thr = thr.data_ptr()
         if want_mask:
-            out["mask8"] = torch.empty(B, H, T, n, dtype=torch.uint8, device=dev)
-            a.mask_out = L.ptr(out["mask8"])
+            out["mask"] = x.new_empty((B, H, T, n), dtype=torch.bool)        # one byte per chunk, 0 or 1
+            a.mask_out = out["mask"].data_ptr()
     if cache is not None:
-        a.main_plane, a.aux_plane = L.ptr(cache.main), L.ptr(cache.aux)
-        a.scale_plane = L.ptr(cache.scale)
-        a.flag_plane = L.ptr(cache.flags) if thr is not None else None
+        a.main_plane, a.aux_plane = L.addr(cache.main), L.addr(cache.aux)
+        a.scale_plane = L.addr(cache.scale)
+        a.flag_plane = L.addr(cache.flags) if thr is not None else 0
         a.t_cap, a.t_off = cache.t_cap, t_off
         a.main_bits, a.aux_bits = cache.main_bits, cache.aux_bits
-        a.scale_max_bits = L.ptr(cache.scale_max)
+        a.scale_max_bits = L.addr(cache.scale_max)
         if pos is not None:
             pos = pos.to(device=dev, dtype=torch.int32).contiguous()
-            keep.append(pos)
-            a.pos = L.ptr(pos)
-    a.stats = L.ptr(stats)
+            a.pos = pos.data_ptr()
+    a.stats = L.addr(stats)
     if T > 0:
-        with torch.cuda.device(dev):
-            L.check(L.lib().hqmq_quantize_grid(C.byref(a), _grid(slack), L.stream_ptr(dev)), "hqmq_quantize_grid")
-    if "mask8" in out:
-        out["mask"] = out.pop("mask8").bool()
+        L.call(L.lib().hqmq_quantize_grid, "hqmq_quantize_grid", dev.index, C.addressof(a), grid)
     return out
 
 
 _WS = {}
+_WS_MOST = 256
 
 # torch.quantile refuses more than 2^24 elements along the reduced dimension ("quantile() input tensor is too large"),
 # which bounds the chunks per head of one Med-C call of the reference (src/quantizers/outlier_aware.py:68).  The
@@ -135,10 +141,12 @@ def check_quantile_limit(chunks_per_head: int, strict: bool) -> bool:
 
 def _workspace(nbytes: int, device, tag: str) -> torch.Tensor:
     """A cached scratch buffer of at least nbytes (grown on demand, reused across calls on the same stream; any content)."""
-    dev = torch.device(device)
-    key = (tag, dev, torch.cuda.current_stream(dev).cuda_stream)     # calls on different streams may overlap
+    index = device.index
+    key = (tag, index, L.raw_stream(index))                          # calls on different streams may overlap
     buf = _WS.get(key)
     if buf is None or buf.numel() < nbytes:
+        if len(_WS) >= _WS_MOST:                                     # streams that are gone: their buffers go back to torch
+            _WS.clear()
         buf = torch.empty(max(nbytes, 1 << 16), dtype=torch.uint8, device=device)
         _WS[key] = buf
     return buf
@@ -153,17 +161,58 @@ def med3x_threshold(x: torch.Tensor, mult: float = 3.0, want_count: bool = True,
     n = d_h // 4
     check_quantile_limit(B * T * n, strict_quantile_limit)
     dev = x.device
-    nbytes = int(L.lib().hqmq_med3x_workspace_bytes(C.c_int(H), C.c_int(_dt(x))))
-    ws = _workspace(nbytes, dev, "med3x")
+    ws = _med_workspace(x, "med3x")
     med = torch.empty(H, dtype=torch.float32, device=dev)
     thr = torch.empty(H, dtype=x.dtype, device=dev)
     cnt = torch.empty(H, dtype=torch.int32, device=dev) if want_count else None     # written for every head
-    with torch.cuda.device(dev):
-        L.check(L.lib().hqmq_med3x_threshold(
-            L.ptr(x), L.i64(x.stride(0)), L.i64(x.stride(1)), L.i64(x.stride(2)), C.c_int(_dt(x)), C.c_int(B), C.c_int(H),
-            C.c_int(T), C.c_int(n), C.c_float(mult), L.ptr(ws), L.i64(ws.numel()), L.ptr(med), L.ptr(thr), L.ptr(cnt),
-            L.stream_ptr(dev)), "hqmq_med3x_threshold")
+    _median(x, mult, ws, med.data_ptr(), thr.data_ptr(), L.addr(cnt))
     return med, thr, cnt
+
+
+def _med_workspace(x: torch.Tensor, tag: str) -> torch.Tensor:
+    H, f32 = x.shape[1], x.dtype == torch.float32
+    key = (H, f32)
+    nbytes = _MED_BYTES.get(key)
+    if nbytes is None:
+        nbytes = _MED_BYTES[key] = int(L.lib().hqmq_med3x_workspace_bytes(C.c_int(H), C.c_int(_dt(x))))
+    return _workspace(nbytes + 12 * H + 16, x.device, tag)        # behind it: room for a median and a threshold nobody asked for
+
+
+_MED_BYTES = {}
+
+
+def _median(x: torch.Tensor, mult: float, ws: torch.Tensor, med: int, thr: int, cnt: int) -> None:
+    B, H, T, d_h = x.shape
+    sb, sh, st, _ = x.stride()
+    L.call(L.lib().hqmq_med3x_threshold, "hqmq_med3x_threshold", x.device.index, x.data_ptr(), sb, sh, st, _dt(x), B, H, T, d_h // 4, mult,
+           ws.data_ptr(), ws.numel(), med, thr, cnt)
+
+
+def fake_quant(x: torch.Tensor, joint: torch.Tensor, slack: torch.Tensor, radius_bits: int, median_mult: Optional[float] = None):
+    """The fake-quant tensor of x (B, H, T, d_h), with Med-C extraction when median_mult is given: what med3x_threshold
+    and quantize(want_dense=True) give, without tensors for the statistics in between.  Returns (out, flagged chunks
+    per head or None)."""
+    L.require_gpu(x, "x")
+    x = _strided_x(x)
+    B, H, T, d_h = x.shape
+    _check_joint(x, joint)
+    tmpl, grid = _book(joint, slack, radius_bits, d_h // 4)
+    a = L.QuantizeArgs.from_buffer_copy(tmpl)
+    a.x = x.data_ptr()
+    a.x_stride_b, a.x_stride_h, a.x_stride_t, _ = x.stride()
+    a.B, a.T = B, T
+    out = x.new_empty((B, H, T, d_h))
+    a.dense_out = out.data_ptr()
+    cnt = None
+    if median_mult is not None:
+        ws = _med_workspace(x, "med3x")
+        cnt = torch.empty(H, dtype=torch.int32, device=x.device)
+        spare = ws.data_ptr() + (ws.numel() - 12 * H & -16)
+        a.thr = spare + 4 * H
+        _median(x, median_mult, ws, spare, spare + 4 * H, cnt.data_ptr())
+    if T > 0:
+        L.call(L.lib().hqmq_quantize_grid, "hqmq_quantize_grid", x.device.index, C.addressof(a), grid)
+    return out, cnt
 
 
 def outlier_mask(x: torch.Tensor, thr: torch.Tensor) -> torch.Tensor:
@@ -210,8 +259,7 @@ def crop(caches, lengths) -> None:
         a.length = max(0, min(lengths, c.t_cap))
     else:
         a.lengths = lengths.data_ptr()
-    with torch.cuda.device(c.device):
-        L.check(L.lib().hqmq_crop(C.byref(a), L.stream_ptr(c.device)), "hqmq_crop")
+    L.call(L.lib().hqmq_crop, "hqmq_crop", c.device.index, C.addressof(a))
 
 
 def append_kv(k: torch.Tensor, v: torch.Tensor, k_cache, v_cache, k_joint, k_slack, v_joint, v_slack, radius_bits: int, *,
@@ -227,50 +275,54 @@ def append_kv(k: torch.Tensor, v: torch.Tensor, k_cache, v_cache, k_joint, k_sla
     dev = k.device
     if pos is not None:
         pos = pos.to(device=dev, dtype=torch.int32).contiguous()
-    keep = [pos]
-    args, counts = [], []
-    for tag, x, cache, joint, slack in (("k", k, k_cache, k_joint, k_slack), ("v", v, v_cache, v_joint, v_slack)):
-        x = _strided_x(x)
-        B, H, T, d_h = x.shape
+    ak, grid_k, k, cnt_k = _append_args(k, k_cache, k_joint, k_slack, radius_bits, t_off, pos, median_mult, "med3x_k")
+    av, grid_v, v, cnt_v = _append_args(v, v_cache, v_joint, v_slack, radius_bits, t_off, pos, median_mult, "med3x_v")
+    L.call(L.lib().hqmq_append_kv_grid, "hqmq_append_kv_grid", dev.index, C.addressof(ak), C.addressof(av), grid_k, grid_v)
+    return cnt_k, cnt_v
+
+
+def _append_args(x, cache, joint, slack, radius_bits, t_off, pos, median_mult, tag):
+    """The arguments of one tensor's append.  What the cache and its codebook fix is filled in once and copied; the copy is
+    this call's own (several threads may append to one cache on streams of their own)."""
+    x = _strided_x(x)
+    B, H, T, d_h = x.shape
+    med = median_mult is not None and T > 0
+    tmpl = cache._append_template
+    if tmpl is None or tmpl[0] is not joint or tmpl[1] is not slack or tmpl[2] != (joint.data_ptr(), radius_bits, d_h, med):
         if d_h % 4 != 0:
             raise ValueError(f"d_head={d_h} not divisible by 4")
-        if joint.dtype != x.dtype or joint.shape[0] != H or not joint.is_contiguous():
-            raise ValueError("joint must be a contiguous (H, 24S, 4) table in the dtype of x")
+        _check_joint(x, joint)
+        book, grid = _book(joint, slack, radius_bits, d_h // 4)
         a = L.AppendArgs()
+        C.memmove(C.addressof(a), C.addressof(book), C.sizeof(book))       # q is the first member
         q = a.q
-        q.x = L.ptr(x)
-        q.x_stride_b, q.x_stride_h, q.x_stride_t = x.stride(0), x.stride(1), x.stride(2)
-        q.dtype = _dt(x)
-        q.B, q.H, q.T, q.n_chunks = B, H, T, d_h // 4
-        q.joint, q.slack = L.ptr(joint), L.ptr(slack)
-        q.secondary_size, q.radius_bits, q.algo = joint.shape[1] // 24, radius_bits, 0
-        q.main_plane, q.aux_plane, q.scale_plane = L.ptr(cache.main), L.ptr(cache.aux), L.ptr(cache.scale)
-        q.t_cap, q.t_off = cache.t_cap, t_off
-        q.main_bits, q.aux_bits = cache.main_bits, cache.aux_bits
-        q.scale_max_bits = L.ptr(cache.scale_max)
-        q.pos = L.ptr(pos)
-        keep += [x, joint, slack]
-        cnt = None
-        if median_mult is not None and T > 0:
-            nbytes = int(L.lib().hqmq_med3x_workspace_bytes(C.c_int(H), C.c_int(_dt(x))))
-            ws = _workspace(nbytes, dev, "med3x_" + tag)
-            med = torch.empty(H, dtype=torch.float32, device=dev)
-            thr = torch.empty(H, dtype=x.dtype, device=dev)
-            cnt = torch.empty(H, dtype=torch.int32, device=dev)      # every path of the library writes all H counts
-            keep += [ws, med, thr]
-            q.flag_plane = L.ptr(cache.flags)
-            a.median_mult = median_mult
-            a.med_workspace, a.med_workspace_bytes = L.ptr(ws), ws.numel()
-            a.median, a.thr, a.n_out = L.ptr(med), L.ptr(thr), L.ptr(cnt)
-            a.sideband, a.sb_cap = L.ptr(cache.sideband), cache.sb_cap
-            a.sb_tile_off, a.sb_count = L.ptr(cache.sb_tile_off), L.ptr(cache.sb_count)
-            a.overflow, a.sb_coord = L.ptr(cache.sb_overflow), L.ptr(cache.sb_coord)
-        args.append(a)
-        counts.append(cnt)
-    with torch.cuda.device(dev):
-        L.check(L.lib().hqmq_append_kv_grid(C.byref(args[0]), C.byref(args[1]), _grid(k_slack), _grid(v_slack), L.stream_ptr(dev)),
-                "hqmq_append_kv_grid")
-    return counts[0], counts[1]
+        q.main_plane, q.aux_plane, q.scale_plane = L.addr(cache.main), L.addr(cache.aux), L.addr(cache.scale)
+        q.t_cap, q.main_bits, q.aux_bits = cache.t_cap, cache.main_bits, cache.aux_bits
+        q.scale_max_bits = L.addr(cache.scale_max)
+        if med:
+            q.flag_plane = L.addr(cache.flags)
+            a.sideband, a.sb_cap = L.addr(cache.sideband), cache.sb_cap
+            a.sb_tile_off, a.sb_count = L.addr(cache.sb_tile_off), L.addr(cache.sb_count)
+            a.overflow, a.sb_coord = L.addr(cache.sb_overflow), L.addr(cache.sb_coord)
+        tmpl = cache._append_template = (joint, slack, (joint.data_ptr(), radius_bits, d_h, med), a, grid)
+    elif joint.dtype != x.dtype or joint.shape[0] != H:
+        _check_joint(x, joint)
+    a = L.AppendArgs.from_buffer_copy(tmpl[3])
+    q = a.q
+    q.x = x.data_ptr()
+    q.x_stride_b, q.x_stride_h, q.x_stride_t, _ = x.stride()
+    q.B, q.T, q.t_off = B, T, t_off
+    if pos is not None:
+        q.pos = pos.data_ptr()
+    cnt = None
+    if med:
+        ws = _med_workspace(x, tag)
+        cnt = torch.empty(H, dtype=torch.int32, device=x.device)           # every path of the library writes all H counts
+        base, n = ws.data_ptr(), ws.numel()
+        spare = base + (n - 12 * H & -16)
+        a.median_mult, a.med_workspace, a.med_workspace_bytes = median_mult, base, n
+        a.median, a.thr, a.n_out = spare, spare + 4 * H, cnt.data_ptr()
+    return a, tmpl[4], x, cnt
 
 
 def _i32(t: torch.Tensor) -> torch.Tensor:
@@ -325,8 +377,17 @@ def dequant_packed(cache, T: Optional[int] = None, mode: int = 0) -> torch.Tenso
 
 
 def pick_splits(B: int, H_q: int, H_kv: int, T_q: int, T_kv: int, ragged: bool = False) -> int:
-    return int(L.lib().hqmq_attn_pick_splits(C.c_int(B), C.c_int(H_q), C.c_int(H_kv), C.c_int(T_q), C.c_int(T_kv),
-                                             C.c_int(1 if ragged else 0)))
+    key = (B, H_q, H_kv, T_q, (T_kv + 63) // 64, ragged)               # the library's choice changes at multiples of 64 tokens only
+    n = _SPLITS.get(key)
+    if n is None:
+        if len(_SPLITS) >= 4096:
+            _SPLITS.clear()
+        n = _SPLITS[key] = int(L.lib().hqmq_attn_pick_splits(C.c_int(B), C.c_int(H_q), C.c_int(H_kv), C.c_int(T_q), C.c_int(T_kv),
+                                                             C.c_int(1 if ragged else 0)))
+    return n
+
+
+_SPLITS = {}
 
 
 def longest_first(kv_lens: torch.Tensor) -> torch.Tensor:
@@ -351,62 +412,64 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
     skip_combine: leave the split partials unmerged and return (O, partials, n_splits): the partials are in `workspace`
     if given, else in a buffer of their own (never the cached scratch that the next call on the stream overwrites);
     attn_combine(partials, O, n_splits) merges them."""
-    L.require_gpu(Q, "Q")
-    if Q.stride(-1) != 1:
+    if not Q.is_cuda:
+        L.require_gpu(Q, "Q")
+    shape, stride = Q.shape, Q.stride()
+    if stride[-1] != 1:
         Q = Q.contiguous()
-    B, Hq, Tq, d_h = Q.shape
-    if d_h != Kc.d_head or d_h != Vc.d_head:
-        raise AssertionError(f"d_h={d_h} != n_chunks*4={Kc.d_head}")
-    if Hq % Kc.H:
-        raise AssertionError(f"H_q={Hq} must be divisible by H_kv={Kc.H}")
-    if Q.dtype != Kc.dtype:
-        raise L.HqmqError(f"Q dtype {Q.dtype} differs from the cache dtype {Kc.dtype}")
+        stride = Q.stride()
+    ks, vs = Kc.c_struct(), Vc.c_struct()
+    plan = Kc._attn_plans.get((shape, stride))
+    if plan is None or plan[0] is not ks or plan[1] is not vs or plan[2] is not Q.dtype:
+        plan = _attn_plan(Q, Kc, Vc, ks, vs)
+    _, _, _, tmpl, o_stride, rows, floats = plan
     dev = Q.device
-    O = out if out is not None else torch.empty_like(Q)
-    if softmax_scale is None:
-        softmax_scale = d_h ** -0.5
-    if n_splits <= 0:
-        n_splits = pick_splits(B, Hq, Kc.H, Tq, max(T_kv, 1), kv_lens is not None)
-    a = L.AttnArgs()
-    a.Q, a.O = L.ptr(Q), L.ptr(O)
-    a.q_sb, a.q_sh, a.q_st = Q.stride(0), Q.stride(1), Q.stride(2)
-    a.o_sb, a.o_sh, a.o_st = O.stride(0), O.stride(1), O.stride(2)
-    a.K, a.V = Kc.c_struct(), Vc.c_struct()
-    a.dtype = L.DT_CODE[Q.dtype]
-    a.B, a.H_q, a.H_kv, a.T_q, a.T_kv, a.n_chunks = B, Hq, Kc.H, Tq, T_kv, Kc.n
-    a.t_cap = Kc.t_cap
-    a.idx_bits, a.main_bits, a.aux_bits, a.qmax = Kc.idx_bits, Kc.main_bits, Kc.aux_bits, Kc.qmax
-    keep = None
+    index = dev.index
+    O = torch.empty_like(Q) if out is None else out
+    a = L.AttnArgs.from_buffer_copy(tmpl)          # this call's own: several threads may attend over one cache
+    a.Q, a.O = Q.data_ptr(), O.data_ptr()
+    strides = O.stride()
+    if strides != o_stride:
+        a.o_sb, a.o_sh, a.o_st = strides[0], strides[1], strides[2]
+    a.T_kv = T_kv
+    if softmax_scale is not None:
+        a.softmax_scale = softmax_scale
     if kv_lens is not None:
-        keep = kv_lens.to(device=dev, dtype=torch.int32).contiguous()
-        a.kv_len = L.ptr(keep)
-    keep_start = None
+        if kv_lens.dtype is not torch.int32 or kv_lens.device != dev or not kv_lens.is_contiguous():
+            kv_lens = kv_lens.to(device=dev, dtype=torch.int32).contiguous()
+        a.kv_len = kv_lens.data_ptr()
     if kv_starts is not None:
-        keep_start = kv_starts.to(device=dev, dtype=torch.int32).contiguous()
-        if keep_start.numel() != B:
-            raise L.HqmqError(f"kv_starts must hold one entry per sequence ({B})")
-        a.kv_start = L.ptr(keep_start)
-    keep_order = None
+        kv_starts = kv_starts.to(device=dev, dtype=torch.int32).contiguous()
+        if kv_starts.numel() != shape[0]:
+            raise L.HqmqError(f"kv_starts must hold one entry per sequence ({shape[0]})")
+        a.kv_start = kv_starts.data_ptr()
     if batch_order is not None:
-        keep_order = batch_order.to(device=dev, dtype=torch.int32).contiguous()
-        if keep_order.numel() != B:
-            raise L.HqmqError(f"batch_order must be a permutation of the {B} sequences")
-        a.batch_order = L.ptr(keep_order)
-    a.causal, a.causal_offset, a.softmax_scale = int(causal), causal_offset, softmax_scale
+        if batch_order.dtype is not torch.int32 or batch_order.device != dev or not batch_order.is_contiguous():
+            batch_order = batch_order.to(device=dev, dtype=torch.int32).contiguous()
+        if batch_order.numel() != shape[0]:
+            raise L.HqmqError(f"batch_order must be a permutation of the {shape[0]} sequences")
+        a.batch_order = batch_order.data_ptr()
+    if causal:
+        a.causal, a.causal_offset = 1, causal_offset
+    if n_splits <= 0:
+        n_splits = pick_splits(shape[0], shape[1], Kc.H, shape[2], max(T_kv, 1), kv_lens is not None)
     a.n_splits = n_splits
-    a.skip_combine = int(skip_combine)
-    a.force_generic = int(force_generic)
-    a.fp8_table_storage = int(fp8_table_storage)
-    a.wide_range = int(bool(getattr(Vc, "wide_range", False)))      # V scales outside [2^-8, 2^15): the generic kernel guards the range
+    if skip_combine:
+        a.skip_combine = 1
+    if force_generic:
+        a.force_generic = int(force_generic)
+    if fp8_table_storage:
+        a.fp8_table_storage = 1
+    if Vc.wide_range:                              # V scales outside [2^-8, 2^15): the generic kernel guards the range
+        a.wide_range = 1
     if kernel_events is not None:
-        a.start_event, a.stop_event = C.c_void_p(kernel_events[0]), C.c_void_p(kernel_events[1])
-    ws = None
+        a.start_event, a.stop_event = kernel_events
     if static_scratch:
-        with torch.cuda.device(dev):
-            L.check(L.lib().hqmq_attn_fwd_static(C.byref(a), L.stream_ptr(dev)), "hqmq_attn_fwd_static")
+        L.call(L.lib().hqmq_attn_fwd_static, "hqmq_attn_fwd_static", index, C.addressof(a))
         return O
+    ws = None
     if n_splits > 1:
-        nbytes = int(L.lib().hqmq_attn_workspace_bytes(C.c_int(B), C.c_int(Hq), C.c_int(Tq), C.c_int(d_h), C.c_int(n_splits)))
+        nbytes = rows * floats * n_splits * 4
         if workspace is not None:
             if workspace.device != dev or workspace.numel() * workspace.element_size() < nbytes:
                 raise L.HqmqError(f"workspace must hold {nbytes} bytes on {dev}")
@@ -415,12 +478,40 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
             ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         else:
             ws = _workspace(nbytes, dev, "attn")
-        a.workspace, a.workspace_bytes = L.ptr(ws), ws.numel() * ws.element_size()
-    with torch.cuda.device(dev):
-        L.check(L.lib().hqmq_attn_fwd(C.byref(a), L.stream_ptr(dev)), "hqmq_attn_fwd")
+        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel() * ws.element_size()
+    L.call(L.lib().hqmq_attn_fwd, "hqmq_attn_fwd", index, C.addressof(a))
     if skip_combine:
         return O, ws, n_splits
     return O
+
+
+def _attn_plan(Q: torch.Tensor, Kc, Vc, ks, vs):
+    """What a shape of Q and a pair of packed tensors fix of an attention call, kept with the K cache: the argument block,
+    the strides of an output like Q, the partial rows and floats per row and split."""
+    B, Hq, Tq, d_h = Q.shape
+    if d_h != Kc.d_head or d_h != Vc.d_head:
+        raise AssertionError(f"d_h={d_h} != n_chunks*4={Kc.d_head}")
+    if Hq % Kc.H:
+        raise AssertionError(f"H_q={Hq} must be divisible by H_kv={Kc.H}")
+    if Q.dtype != Kc.dtype:
+        raise L.HqmqError(f"Q dtype {Q.dtype} differs from the cache dtype {Kc.dtype}")
+    a = L.AttnArgs()
+    a.q_sb, a.q_sh, a.q_st = Q.stride(0), Q.stride(1), Q.stride(2)
+    o_stride = torch.empty_like(Q).stride()
+    a.o_sb, a.o_sh, a.o_st = o_stride[0], o_stride[1], o_stride[2]
+    a.K, a.V = ks, vs
+    a.dtype = L.DT_CODE[Q.dtype]
+    a.B, a.H_q, a.H_kv, a.T_q, a.n_chunks = B, Hq, Kc.H, Tq, Kc.n
+    a.t_cap = Kc.t_cap
+    a.idx_bits, a.main_bits, a.aux_bits, a.qmax = Kc.idx_bits, Kc.main_bits, Kc.aux_bits, Kc.qmax
+    a.softmax_scale = d_h ** -0.5
+    per_split = int(L.lib().hqmq_attn_workspace_bytes(C.c_int(B), C.c_int(Hq), C.c_int(Tq), C.c_int(d_h), C.c_int(2))) // 8
+    rows = B * Hq * Tq
+    plan = (ks, vs, Q.dtype, a, o_stride, rows, per_split // rows)
+    if len(Kc._attn_plans) >= 64:                  # shapes that no longer come
+        Kc._attn_plans.clear()
+    Kc._attn_plans[(Q.shape, Q.stride())] = plan
+    return plan
 
 
 def attn_combine(partials: Optional[torch.Tensor], O: torch.Tensor, n_splits: int) -> torch.Tensor:

@@ -22,14 +22,37 @@ def _round_up(x: int, m: int) -> int:
     return (x + m - 1) // m * m
 
 
+class RangeWatch:
+    """The largest finite scales the quantize kernels have written, as fp32 bits, one slot per tensor that shares the watch,
+    and their way to the host: a copy into pinned memory behind the append that may have changed them, waited for only when
+    the value is looked at."""
+
+    def __init__(self, device, slots: int = 1):
+        self.device_values = torch.zeros(slots, dtype=torch.int32, device=device)
+        self.host = self.event = None
+
+    def fetch(self) -> None:
+        if self.host is None:
+            self.host = torch.empty(self.device_values.numel(), dtype=torch.int32, pin_memory=True)
+            self.event = torch.cuda.Event()
+        self.host.copy_(self.device_values, non_blocking=True)
+        self.event.record()
+
+    def read(self, slot: int, wait: bool) -> float:
+        if wait:
+            self.event.synchronize()
+        return float(self.host.view(torch.float32)[slot])
+
+
 class PackedTensor:
     """Packed codes of a (B, H, T, d_h) tensor; rows [0, length) are valid."""
 
     def __init__(self, B: int, H: int, t_cap: int, d_head: int, secondary_size: int, radius_bits: int,
                  dtype: torch.dtype, device, joint: Optional[torch.Tensor] = None, outliers: bool = False,
-                 sideband_frac: float = 0.125, layout: Optional[tuple] = None):
+                 sideband_frac: float = 0.125, layout: Optional[tuple] = None, watch: Optional[tuple] = None):
         if d_head % 4:
             raise ValueError(f"d_head={d_head} not divisible by 4")
+        self._attn_plans = {}
         self.B, self.H, self.d_head, self.n = B, H, d_head, d_head // 4
         self.d_head_orig = d_head            # smaller for zero-padded heads (PaddedHQMQ): what Q and O carry
         self.t_cap = _round_up(max(t_cap, 1), T_ALIGN)
@@ -46,12 +69,13 @@ class PackedTensor:
         self.joint = joint
         # the largest finite scale written so far as fp32 bits (the quantize kernel keeps it up to date): the attention
         # kernels' range guard for bf16 / fp32 caches; fp16 scales cannot leave the range
-        self.scale_max = None if dtype == torch.float16 else torch.zeros(1, dtype=torch.int32, device=self.device)
+        # (watch: a RangeWatch and this tensor's slot in it, for tensors that are appended together)
+        self._watch, self._slot = (None, 0) if dtype == torch.float16 else watch or (RangeWatch(self.device), 0)
+        self.scale_max = self._watch_view = None if self._watch is None else self._watch.device_values[self._slot:self._slot + 1]
         # host-side copy of "scale_max lies outside [2^-8, 2^15)": such a cache takes the layout-generic attention kernel, which
-        # guards the fp16 range (refresh_range reads the device value; the quantizer calls it after bulk appends and
-        # every RANGE_CHECK_EVERY small ones)
-        self.wide_range = False
-        self._huge = False
+        # guards the fp16 range (refresh_range reads the device value; due after bulk appends and every
+        # RANGE_CHECK_EVERY small ones, done when the flag is next looked at)
+        self._wide = self._huge = self._range_due = False
         self._appends_since_range_check = 0
         self.length = 0                      # rows written when all sequences advance together
         self.lengths: Optional[torch.Tensor] = None  # per-sequence rows (int32, device) for ragged batches
@@ -88,7 +112,39 @@ class PackedTensor:
             total += int(self.sb_count.sum().item()) * 4 * self.scale.element_size()
         return int(total)
 
+    # arguments of the library's calls that are kept while the attributes they are made of stay what they are
+    _STRUCT_FIELDS = frozenset(("main", "aux", "flags", "scale", "sideband", "sb_tile_off", "sb_coord", "sb_count", "sb_overflow", "sb_cap", "joint",
+                                "scale_max", "B", "H", "n", "d_head", "t_cap", "dtype", "qmax", "idx_bits", "main_bits", "aux_bits"))
+
+    def __setattr__(self, name, value):
+        object.__setattr__(self, name, value)
+        if name in self._STRUCT_FIELDS:
+            d = self.__dict__
+            d["_struct"] = d["_append_template"] = None
+            d["_attn_plans"] = {}
+
+    @property
+    def wide_range(self) -> bool:
+        """V scales of a bf16 / fp32 cache outside [2^-8, 2^15).  Waits for the last bulk append if the value behind it has
+        not been looked at yet (under stream capture, which begins with everything done, it is read as it stands)."""
+        if self._range_due:
+            self._take_range(self._watch.read(self._slot, wait=not torch.cuda.is_current_stream_capturing()))
+        return self._wide
+
+    @wide_range.setter
+    def wide_range(self, value: bool) -> None:
+        self._wide, self._range_due = bool(value), False
+
     def c_struct(self) -> L.Packed:
+        """The tensors as the library takes them; the same object until one of them is replaced."""
+        s = self._struct
+        if s is not None and s.main_plane == self.main.data_ptr():
+            return s
+        s = self._make_struct()
+        object.__setattr__(self, "_struct", s)
+        return s
+
+    def _make_struct(self) -> L.Packed:
         s = L.Packed()
         s.main_plane, s.aux_plane, s.flag_plane = L.ptr(self.main), L.ptr(self.aux), L.ptr(self.flags)
         s.scale_plane = L.ptr(self.scale)
@@ -109,20 +165,33 @@ class PackedTensor:
         normal range.  The largest scale only grows: a cache of tiny values leaves the flag again when larger ones
         arrive; a cache beyond 2^15 keeps it."""
         if self.scale_max is not None and not self._huge:
-            v = float(self.scale_max.view(torch.float32).item())
-            self._huge = v >= 32768.0
-            self.wide_range = self._huge or 0.0 < v < 2.0 ** -8
+            self._take_range(float(self.scale_max.view(torch.float32).item()))
         self._appends_since_range_check = 0
-        return self.wide_range
+        return self._wide
 
-    def note_append(self, rows: int) -> None:
-        """Called by the quantizer after an append of `rows` rows per sequence: bulk appends (a prefill) and every
-        RANGE_CHECK_EVERY-th small one refresh the range flag; never while the stream is being captured."""
+    def _take_range(self, v: float) -> None:
+        self._huge = self._huge or v >= 32768.0
+        self._wide = self._huge or 0.0 < v < 2.0 ** -8
+        self._range_due = False
+
+    def note_append(self, rows: int, fetch: bool = True) -> bool:
+        """Called by the quantizer after an append of `rows` rows per sequence: after bulk appends (a prefill) and every
+        RANGE_CHECK_EVERY-th small one the range is due to be read again, never while the stream is being captured.  The
+        value sets out for the host at once (fetch=False: the caller fetches the shared watch) and is waited for when the
+        flag is next used.  Returns whether it is due."""
         if self.scale_max is None or self._huge:
-            return
+            return False
         self._appends_since_range_check += 1
-        if (rows >= 64 or self._appends_since_range_check >= self.RANGE_CHECK_EVERY) and not torch.cuda.is_current_stream_capturing():
+        if (rows < 64 and self._appends_since_range_check < self.RANGE_CHECK_EVERY) or torch.cuda.is_current_stream_capturing():
+            return False
+        if self.scale_max is not self._watch_view:         # somebody else's tensor
             self.refresh_range()
+            return False
+        self._appends_since_range_check = 0
+        self._range_due = True
+        if fetch:
+            self._watch.fetch()
+        return True
 
     def crop_(self, lengths) -> None:
         """Forgets the rows from `lengths` on (an int for all sequences or an int tensor [B]): the outlier list and

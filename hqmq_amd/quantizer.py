@@ -23,7 +23,7 @@ import torch.nn as nn
 from . import _lib as L
 from . import ops
 from .codebook import _make_24cell_codebook
-from .packed import PackedKV, PackedTensor
+from .packed import PackedKV, PackedTensor, RangeWatch
 
 
 class KVQuantizer(ABC):
@@ -102,7 +102,8 @@ class HQMQQuantizer(KVQuantizer):
                 "with 1..8 bits, evaluation mode")
 
     def _joint_and_slack(self, layer_idx: int, kv: int, ref: torch.Tensor):
-        L.require_gpu(ref, "tensor")
+        if not ref.is_cuda:
+            L.require_gpu(ref, "tensor")
         raw = self.secondary_raw
         if raw.device != ref.device:
             raise L.HqmqError(f"quantizer parameters are on {raw.device}, the tensor is on {ref.device}")
@@ -125,7 +126,7 @@ class HQMQQuantizer(KVQuantizer):
             raise ValueError(f"d_head={x.shape[-1]} not divisible by 4")
         self._check_supported()
         joint, slack = self._joint_and_slack(layer_idx, kv, x)
-        return ops.quantize(x, joint, slack, self.radius_bits, want_codes=False, want_dense=True)["out"]
+        return ops.fake_quant(x, joint, slack, self.radius_bits)[0]
 
     def quantize_K(self, k, layer_idx):
         return self._qdq(k, layer_idx, kv=0)
@@ -175,9 +176,10 @@ class HQMQQuantizer(KVQuantizer):
         self._check_supported()
         dev = self.secondary_raw.device
         ref = torch.empty(0, dtype=dtype, device=dev)
+        watch = RangeWatch(dev, 2) if dtype != torch.float16 else None
         mk = lambda kv: PackedTensor(batch, self.n_heads, max_tokens, d_head, self.secondary_size, self.radius_bits,
                                      dtype, dev, joint=self._joint_and_slack(layer_idx, kv, ref)[0], outliers=outliers,
-                                     sideband_frac=sideband_frac)
+                                     sideband_frac=sideband_frac, watch=watch and (watch, kv))
         return PackedKV(mk(0), mk(1))
 
     def _append_one(self, cache: PackedTensor, x: torch.Tensor, layer_idx: int, kv: int, pos, median_mult=None):
@@ -211,23 +213,26 @@ class HQMQQuantizer(KVQuantizer):
         if k.shape[2] != v.shape[2]:
             raise ValueError("k and v must bring the same number of new tokens")
         T = k.shape[2]
-        for pt in (cache.K, cache.V):
+        K, V = cache.K, cache.V
+        for pt in (K, V):
             if pos is None and pt.length + T > pt.t_cap:
                 raise L.HqmqError(f"cache capacity {pt.t_cap} exceeded by append of {T} rows at {pt.length}")
-            if median_mult is not None and not pt.has_outliers:
+            if median_mult is not None and pt.flags is None:
                 raise L.HqmqError("this cache was allocated without an outlier sideband")
-        if pos is None and cache.K.length != cache.V.length:      # never the case for caches filled through append()
-            return (self._append_one(cache.K, k, layer_idx, 0, pos, median_mult),
-                    self._append_one(cache.V, v, layer_idx, 1, pos, median_mult))
+        if pos is None and K.length != V.length:      # never the case for caches filled through append()
+            return (self._append_one(K, k, layer_idx, 0, pos, median_mult),
+                    self._append_one(V, v, layer_idx, 1, pos, median_mult))
         kj, ks = self._joint_and_slack(layer_idx, 0, k)
         vj, vs = self._joint_and_slack(layer_idx, 1, v)
-        t_off = 0 if pos is not None else cache.K.length
-        counts = ops.append_kv(k, v, cache.K, cache.V, kj, ks, vj, vs, self.radius_bits, t_off=t_off, pos=pos,
-                               median_mult=median_mult)
+        t_off = 0 if pos is not None else K.length
+        counts = ops.append_kv(k, v, K, V, kj, ks, vj, vs, self.radius_bits, t_off=t_off, pos=pos, median_mult=median_mult)
         if pos is None:
-            cache.K.length = cache.V.length = t_off + T
-        cache.K.note_append(T)
-        cache.V.note_append(T)
+            K.length = V.length = t_off + T
+        if K.scale_max is not None:
+            shared = K._watch is V._watch
+            due_k, due_v = K.note_append(T, fetch=not shared), V.note_append(T, fetch=not shared)
+            if shared and (due_k or due_v):
+                K._watch.fetch()
         return counts
 
 
@@ -245,8 +250,17 @@ class _OutlierStats:
             self._fold()
 
     def _fold(self):
-        for count, total in self._pending:
-            rate = float(count.sum().item()) / max(total, 1)
+        if not self._pending:
+            return
+        by_shape = {}                               # one device read per device and head count, not one per call
+        for i, (count, _) in enumerate(self._pending):
+            by_shape.setdefault((count.device, count.shape), []).append(i)
+        sums = [0] * len(self._pending)
+        for index in by_shape.values():
+            for i, n in zip(index, torch.stack([self._pending[i][0] for i in index]).sum(dim=1).tolist()):
+                sums[i] = n
+        for n, (_, total) in zip(sums, self._pending):
+            rate = float(n) / max(total, 1)
             self._observed_outlier_rate = (self._observed_outlier_rate * self._n_observations + rate) / (self._n_observations + 1)
             self._n_observations += 1
         self._pending = []
@@ -288,9 +302,11 @@ class OutlierAwareHQMQQuantizer(KVQuantizer, _OutlierStats):
             raise ValueError(f"d_head={x.shape[-1]} not divisible by 4")
         self.inner._check_supported()
         joint, slack = self.inner._joint_and_slack(layer_idx, kv, x)
-        _, thr, count = ops.med3x_threshold(x, self.median_mult, strict_quantile_limit=self.strict_quantile_limit)
+        if self.strict_quantile_limit:
+            ops.check_quantile_limit(x.shape[0] * x.shape[2] * (x.shape[3] // 4), strict=True)
+        out, count = ops.fake_quant(x, joint, slack, self.inner.radius_bits, self.median_mult)
         self._note(count, x.numel() // 4)
-        return ops.quantize(x, joint, slack, self.inner.radius_bits, want_codes=False, want_dense=True, thr=thr)["out"]
+        return out
 
     def quantize_K(self, k, layer_idx):
         return self._qdq(k, layer_idx, kv=0)
