@@ -85,7 +85,7 @@ class CropArgs(C.Structure):
 EXPORTS = [
     "hqmq_version", "hqmq_status_string", "hqmq_layout_bits", "hqmq_build_joint", "hqmq_quantize",
     "hqmq_med3x_workspace_bytes", "hqmq_med3x_threshold", "hqmq_outlier_mask", "hqmq_outlier_compact", "hqmq_dequant",
-    "hqmq_pack_codes", "hqmq_dequant_packed", "hqmq_attn_workspace_bytes", "hqmq_attn_pick_splits",
+    "hqmq_pack_codes", "hqmq_dequant_packed", "hqmq_attn_workspace_bytes", "hqmq_attn_pick_splits", "hqmq_attn_splits",
     "hqmq_attn_fwd", "hqmq_attn_combine", "hqmq_append_kv", "hqmq_attn_static_scratch_bytes", "hqmq_attn_fwd_static",
     "hqmq_search_grid_bytes", "hqmq_build_search_grid", "hqmq_quantize_grid", "hqmq_append_kv_grid", "hqmq_crop",
 ]
@@ -110,7 +110,7 @@ def lib():
                      "hqmq_search_grid_bytes"):
             getattr(L, name).restype = i64
         # the calls of a decode loop take addresses as plain integers
-        for name, n in (("hqmq_attn_fwd", 2), ("hqmq_attn_fwd_static", 2), ("hqmq_quantize_grid", 3), ("hqmq_append_kv_grid", 5), ("hqmq_crop", 2),
+        for name, n in (("hqmq_attn_fwd", 2), ("hqmq_attn_fwd_static", 2), ("hqmq_attn_splits", 1), ("hqmq_quantize_grid", 3), ("hqmq_append_kv_grid", 5), ("hqmq_crop", 2),
                         ("hqmq_quantize", 2), ("hqmq_append_kv", 3)):
             getattr(L, name).argtypes = [vp] * n
         L.hqmq_med3x_threshold.argtypes = [vp, i64, i64, i64, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, vp, i64, vp, vp, vp, vp]

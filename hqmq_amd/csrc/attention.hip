@@ -514,6 +514,12 @@ extern "C" int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv
     return (int)s;
 }
 
+extern "C" int hqmq_attn_splits(const hqmq_attn_args *a) {
+    if (!a || a->B < 1 || a->H_kv < 1 || a->H_q < 1 || a->T_q < 1 || a->T_kv < 1) return 1;
+    const int splits = attn_prefill_splits(a, 0);
+    return splits > 0 ? splits : hqmq_attn_pick_splits(a->B, a->H_q, a->H_kv, a->T_q, a->T_kv, a->kv_len != nullptr);
+}
+
 extern "C" int hqmq_attn_combine(const void *workspace, void *O, int dtype, int B, int H_q, int T_q, int d_h, int n_splits,
                                  int64_t o_sb, int64_t o_sh, int64_t o_st, void *stream) {
     if (!workspace || !O) return HQMQ_ERR_NULL;
@@ -618,7 +624,12 @@ static int attn_fwd_impl(const hqmq_attn_args *a, void *stream) {
     tm.stop = (hipEvent_t)a->stop_event;
     int rc = HQMQ_OK;
     bool handled = false;
-    if (p.scale_vec && a->force_generic != 1 && a->softmax_scale > 0.f) {
+    if (p.scale_vec && attn_prefill_splits(a, n_splits) > 0) {
+        rc = launch_attn_prefill(p, a->main_bits, st, tm);
+        if (rc) return rc;
+        handled = true;
+    }
+    if (!handled && p.scale_vec && a->force_generic != 1 && a->softmax_scale > 0.f) {
         rc = launch_attn_fast(p, a->main_bits, flags, grid, ((size_t)a->K.K + a->V.K) * 8, st, tm, &handled);
         if (rc) return rc;
     }

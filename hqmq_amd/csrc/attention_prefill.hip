@@ -1,0 +1,554 @@
+// Attention with many query columns per KV head (chunked and whole prefill) over plain 16-bit caches, d_h 64 / 128.
+//
+// The decode kernels give a wavefront 16 or 32 columns and let it decode every KV tile for itself; with hundreds of
+// columns the same tile is decoded again and again.  Here a block of eight wavefronts decodes each tile of 64 tokens once
+// into LDS (K and V as fp16 codeword * radius code, [token][d]) and all its columns use it:
+//   * a wavefront owns 32 columns (a column is a query token and a query head of the group), 256 per block with KVG = 1;
+//     with KVG = 2 four wavefronts take the first half of every tile and four the second half for the same 128 columns, and the
+//     halves merge through LDS at the end: twice the blocks, for launches that would leave compute units idle otherwise;
+//   * S^T = K . Q^T and O^T += V^T . P^T on v_mfma_f32_32x32x16_f16.  The accumulators of S^T (lane = column + 32 * half,
+//     rows 8 i + 4 half + j) are the B operand of the second product if the 16 tokens of a step are numbered
+//     {4 half + j, 8 + 4 half + j}: P never leaves the registers, and V^T comes from LDS in that order by two transposing
+//     reads (ds_read_b64_tr_b16) per 32 x 16 operand;
+//   * LDS rows are stored with their 16-byte parts permuted by the token, so that the writes (16 tokens at the same part),
+//     the K reads (16 tokens) and the transposing V reads (4 tokens by 64 bytes) all meet 64 different banks;
+//   * K in LDS is codeword * radius code; the token's scale is applied to the score in fp32.  V is codeword * (radius code *
+//     scale / qmax), where the decode kernels put the scale into P: the same number of fp16 roundings, one less per score;
+//   * one basic block per 32 tokens, written out one matrix instruction at a time: the scores of the next 32 tokens run with
+//     the exponentials of these, their products with V with the decoding of a later tile.  A matrix instruction takes 32
+//     cycles of its own pipe, a vector instruction about 4.3 of the shared issue slot (8.3 for an exponential), so that the
+//     two kinds have to be interleaved, and every vector instruction saved counts;
+//   * two tile buffers, one barrier per tile (two with KVG = 1).  The codes of a tile are requested two tiles ahead into
+//     registers that nothing copies (a copy would wait for them).
+// Measured, B = 1, 32 / 8 heads of 128, s96_r4, 1024 queries on 32768 tokens (541 GFLOP, 0.43 ms at the rate of a large matrix
+// product): 0.69 ms against 0.96 with the decode kernels' two-column-group variants; 4096 on 4096 tokens causal, s24_r3:
+// 0.19 against 0.41; four sequences of 300 on 300: 0.022 against 0.048.  What bounds it: a compute unit spends 36 % of the
+// time in the matrix pipe, 50 % issuing vector instructions (a quarter of them decode) and 46 % in LDS, at 2.0 to 2.1 GHz.
+#include "attention_mfma.h"
+#include <algorithm>
+
+namespace hqmq {
+
+typedef float float16v __attribute__((ext_vector_type(16)));
+typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
+typedef short short4v __attribute__((ext_vector_type(4)));
+
+constexpr uint32_t kPfV = 16384, kPfBuf = 32768, kPfScale = 2 * kPfBuf, kPfTab = kPfScale + 2048;   // LDS: K | V, twice; scales; tables
+
+// permutation of a row's 16-byte parts
+template <int DH>
+__device__ __forceinline__ uint32_t pf_part(uint32_t t, uint32_t q) {
+    if (DH == 128) return q ^ ((t & 3u) << 2 | ((t >> 2) & 3u));
+    return q ^ (((t >> 1) & 1u) << 2 | ((t >> 2) & 3u));
+}
+
+#define PF_INLINE __attribute__((always_inline))
+
+template <int DH, int MB, bool AUX, int DT, int KVG>
+__global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int gx, int rows) {
+    constexpr int n = DH / 4, ROWB = DH * 2, CW = 8 / KVG, KS = DH / 16, DB = DH / 32;
+    constexpr int TILE = 8192 / DH, NSUB = TILE / 32 / KVG;              // tokens per tile; units of 32 of them per wavefront
+    constexpr int TOK = DH == 128 ? 16 : 32;                             // tokens a wavefront decodes: 8 chunks per lane
+    extern __shared__ uint2 lds_tab[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, col = lane & 31;
+    const int G = p.G, nz = p.B * p.Hkv;
+    // block numbers: (sequence, KV head) fastest, then splits, then `rows` rows; row r takes the column blocks r, 2 rows - 1 - r,
+    // 2 rows + r, ... counted from the last (the longest of a causal launch), so that all rows get about the same work
+    const int r0 = (int)blockIdx.x / nz, bz = (int)blockIdx.x - r0 * nz;
+    const int row0 = r0 / p.n_splits, sp = r0 % p.n_splits;
+    const int slot = bz / p.Hkv, hkv = bz - slot * p.Hkv;
+    const int b = p.batch_order ? min(max(uniform_word(p.batch_order, slot), 0), p.B - 1) : slot;
+    const size_t plane_row0 = (size_t)(b * p.Hkv + hkv) * p.t_cap;
+    const int cw = wave % CW, kvg = wave / CW;
+
+    // ---- codeword tables as fp16: K, then V; every load is on its way before the first one is stored ----
+    auto tables = [&]() PF_INLINE {
+        constexpr int U = 5;
+        const uint2 *kj = (const uint2 *)p.Kc.joint + hkv * (p.Kc.jsh / 4), *vj = (const uint2 *)p.Vc.joint + hkv * (p.Vc.jsh / 4);
+        const int kk = p.Kc.K, all = kk + p.Vc.K;
+        const uint32_t vt = kPfTab + ((kk * 8 + 127) & ~127);
+        for (int k0 = tid; k0 < all; k0 += 512 * U) {
+            uint2 w[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int k = min(k0 + 512 * u, all - 1);
+                w[u] = k < kk ? kj[k] : vj[k - kk];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int k = k0 + 512 * u;
+                if (k < all)
+                    *(uint2v __attribute__((address_space(3))) *)(uintptr_t)(k < kk ? kPfTab + 8u * k : vt + 8u * (k - kk)) = __builtin_bit_cast(uint2v, chunk_to_half<DT>(w[u]));
+            }
+        }
+    };
+    for (int it = 0; it * rows < gx; it++) {
+    const int pos = (it & 1) ? (it + 1) * rows - 1 - row0 : it * rows + row0;
+    if (pos >= gx) continue;
+    const int cb = gx - 1 - pos;
+    // ---- this wavefront's columns and the block's KV range ----
+    int kv_end = p.kv_len ? uniform_word(p.kv_len, b) : p.Tkv;
+    kv_end = min(max(kv_end, 0), p.Tkv);
+    const int cols = p.Tq * G, cidx = (cb * CW + cw) * 32 + col;
+    const bool col_ok = cidx < cols;
+    const int tq = col_ok ? cidx / G : 0, hq = hkv * G + (col_ok ? cidx - tq * G : 0);
+    auto limit = [&](int q) PF_INLINE { return p.causal ? (int)max((int64_t)0, min((int64_t)kv_end, (int64_t)q + p.causal_offset + 1)) : kv_end; };
+    const int col_lim = col_ok ? limit(tq) : 0;
+    // columns are ordered by query token: the last real column of a range sees most, the first least
+    const int first_c = (cb * CW + cw) * 32;
+    const int wave_min = first_c + 31 < cols ? limit(first_c / G) : 0;
+    const int blk_lim = limit((min((cb + 1) * CW * 32, cols) - 1) / G);
+    const int col_start = p.kv_start ? min(max(uniform_word(p.kv_start, b), 0), blk_lim) : 0;
+    const int blk_lo = col_start / TILE * TILE;
+    int per_split = (blk_lim - blk_lo + p.n_splits - 1) / p.n_splits;
+    per_split = (per_split + TILE - 1) / TILE * TILE;
+    const int b_begin = min(blk_lo + sp * per_split, blk_lim), b_end = min(blk_lim, b_begin + per_split);
+    const bool work = b_begin < b_end;
+
+    // ---- decoding: wavefronts 0..3 take K, 4..7 take V; lane = token + TOK * (group of 8 chunks) ----
+    const bool dec_v = wave >= 4;
+    const int d_tok = (wave & 3) * TOK + lane % TOK, d_grp = lane / TOK;
+    const PackedDev &dc = dec_v ? p.Vc : p.Kc;
+    constexpr int NW = MB / 4;
+    constexpr uint32_t mrb = n * MB / 8;
+    const uint32_t ab = AUX ? p.aux_bits : 0, arb = n * ab / 8;
+    const uint8_t *d_main = dc.main_plane + plane_row0 * mrb;
+    const uint32_t *d_aux = AUX ? (const uint32_t *)(dc.aux_plane + plane_row0 * arb) : nullptr;
+    const uint16_t *d_scale = (const uint16_t *)dc.scale_plane + b * dc.ssb + hkv * dc.ssh;
+    const uint32_t idx_mask = (1u << p.idx_bits) - 1u;
+    const int idx_bits = p.idx_bits;
+    const uint32_t tab = kPfTab + (dec_v ? (uint32_t)((p.Kc.K * 8 + 127) & ~127) : 0u);
+    struct Codes { uint32_t w[NW], aux, aux2, sh, scale; };
+    auto request = [&](int t0, Codes &c) PF_INLINE {
+        const uint32_t row = (uint32_t)min(t0 + d_tok, b_end - 1);        // rows past the range were perhaps never written
+        const uint8_t *m = d_main + (row * mrb + (uint32_t)d_grp * MB);
+        if (MB == 16) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(m);
+            c.w[0] = v.x; c.w[1] = v.y; c.w[2] = v.z; c.w[NW - 1] = v.w;
+        } else {
+#pragma unroll
+            for (int i = 0; i < NW; i++) c.w[i] = reinterpret_cast<const uint32_t *>(m)[i];
+        }
+        if (AUX) {                                                        // the dwords of the plane that hold the lane's bytes
+            const uint32_t o = row * arb + (uint32_t)d_grp * ab;
+            c.aux = d_aux[o >> 2];
+            c.aux2 = d_aux[(o + ab - 1) >> 2];
+            c.sh = o;
+        }
+        c.scale = d_scale[row];
+    };
+    // decoding goes in eight pieces, so that it can be spread between the matrix instructions: codewords requested (0, 1),
+    // radii unpacked (2, 3), products stored (4 .. 7); in registers between them:
+    half4 wg[8];
+    half2v wr[4];
+    float w_scale = 0.f;
+    uint32_t w_at = (dec_v ? kPfV : 0u) + (uint32_t)d_tok * ROWB + (pf_part<DH>((uint32_t)d_tok, (uint32_t)(d_grp * 4)) << 4);
+    uint32_t ws_at = kPfScale + 4u * (uint32_t)d_tok;
+    const bool w_lane = !dec_v && d_grp == 0;
+    auto piece = [&](int j, Codes &c) PF_INLINE {
+        if (j == 0) {
+#pragma unroll
+            for (int i = 0; i < NW; i++) asm volatile("" : "+v"(c.w[i]));     // nothing of this moves up
+        }
+        if (j < 2) {
+            const uint32_t aux = AUX ? __builtin_amdgcn_alignbyte(c.aux2, c.aux, c.sh) : 0u;
+#pragma unroll
+            for (int i = 4 * j; i < 4 * j + 4; i++) {
+                if constexpr (MB == 16 && !AUX) {
+                    wg[i] = __builtin_bit_cast(half4, *(lds_u2_ptr)(uintptr_t)(((i & 1 ? c.w[i / 2] >> 16 : c.w[i / 2]) & idx_mask) * 8u + tab));
+                } else {
+                    uint32_t code = code_at<MB, NW>(c.w, i);
+                    if (AUX) code |= ((aux >> (i * ab)) & ((1u << ab) - 1u)) << MB;
+                    wg[i] = __builtin_bit_cast(half4, *(lds_u2_ptr)(uintptr_t)((code & idx_mask) * 8u + tab));
+                    wr[i >> 1][i & 1] = (_Float16)(uint16_t)(code >> idx_bits);
+                }
+            }
+        } else if (j < 4) {
+            if constexpr (MB == 16 && !AUX) {
+                uint32_t rq2 = (0xffffu >> idx_bits) * 0x00010001u, magic = 0x64006400u;
+                asm("" : "+s"(rq2));
+                asm("" : "+v"(magic));
+#pragma unroll
+                for (int i = 2 * j - 4; i < 2 * j - 2; i++) {
+                    const uint32_t t = ((c.w[i] >> idx_bits) & rq2) | magic;             // 0x6400 | rq = the fp16 number 1024 + rq
+                    wr[i] = __builtin_bit_cast(half2v, t) - half2v{(_Float16)1024.0f, (_Float16)1024.0f};
+                }
+            }
+            // K keeps its radius codes (the token's scale is applied to the score, in fp32); V takes radius * scale, rounded once
+            if (j == 3) {
+                w_scale = DT == HQMQ_F16 ? __half2float(__ushort_as_half((uint16_t)c.scale)) : __uint_as_float(c.scale << 16);
+                const float f = dec_v ? w_scale * p.inv_qmax : 1.f;
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int x = 0; x < 2; x++) wr[i][x] = (_Float16)__builtin_fmaf((float)wr[i][x], f, 0.f);
+            }
+        } else {
+            const int i = j - 4;
+            *(uint4v __attribute__((address_space(3))) *)(uintptr_t)(w_at ^ ((uint32_t)i << 4)) =
+                __builtin_bit_cast(uint4v, cat8(wg[2 * i] * wr[i][0], wg[2 * i + 1] * wr[i][1]));
+            if (j == 7) {
+                if (w_lane) *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = w_scale * p.c_log2;
+                w_at ^= kPfBuf;
+                ws_at ^= 512u;
+            }
+        }
+    };
+    // K runs one tile ahead of V: while tile i is multiplied, K of tile i + 2 and V of tile i + 1 are decoded
+    // (in even steps from cc[0], in odd ones from cc[1], then the codes of the tile two further on are requested)
+    Codes cc[2];
+    if (work) {
+        request(b_begin, cc[1]);
+        request(b_begin + TILE, cc[0]);
+    }
+    int d_t = b_begin + (dec_v ? 3 : 4) * TILE;                           // the tile requested next
+
+    // ---- query columns: the B operand of S^T, lane (col, half) holds d = 16 kk + 8 half .. + 7 ----
+    half8 qf[KS];
+    {
+        const uint16_t *qp = (const uint16_t *)p.Q + b * p.qsb + hq * p.qsh + (int64_t)tq * p.qst + 8 * half;
+#pragma unroll
+        for (int kk = 0; kk < KS; kk++) {
+            const uint2 lo = *reinterpret_cast<const uint2 *>(qp + 16 * kk), hi = *reinterpret_cast<const uint2 *>(qp + 16 * kk + 4);
+            const half4 z = half4{0, 0, 0, 0};
+            qf[kk] = cat8(col_ok ? chunk_to_half<DT>(lo) : z, col_ok ? chunk_to_half<DT>(hi) : z);
+        }
+    }
+    if (it == 0) tables();
+    __syncthreads();
+    if (work) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) piece(j, cc[1]);
+        request(b_begin + 2 * TILE, cc[1]);
+        if (!dec_v) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) piece(j, cc[0]);
+            cc[0] = cc[1];
+            request(b_begin + 3 * TILE, cc[1]);
+        }
+    }
+    __syncthreads();
+
+    // ---- LDS addresses of the operands (tile buffer 0) ----
+    uint32_t ka[KS], va[2][DB];
+    const uint32_t wo = (uint32_t)kvg * (32u * NSUB * ROWB);              // this wavefront's share of a tile
+#pragma unroll
+    for (int kk = 0; kk < KS; kk++) ka[kk] = wo + (uint32_t)col * ROWB + (pf_part<DH>((uint32_t)col, (uint32_t)(2 * kk + half)) << 4);
+#pragma unroll
+    for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+        for (int db = 0; db < DB; db++) {
+            // lane i of a group of 16 reads token row i / 4, d part i % 4; afterwards it holds d = i of the four rows
+            const uint32_t i = lane & 15, t = (uint32_t)(8 * hf + 4 * half) + (i >> 2);
+            const uint32_t q = (uint32_t)(4 * db + 2 * ((lane >> 4) & 1)) + ((i & 3) >> 1);
+            va[hf][db] = wo + kPfV + t * ROWB + (pf_part<DH>(t, q) << 4) + (i & 1) * 8u;
+        }
+    const uint32_t sa = kPfScale + 16u * (uint32_t)half + 128u * NSUB * (uint32_t)kvg;
+
+    // exponents are in base 2: s becomes score * scale - (running maximum); seen is -inf until a column has met a token, then 0
+    float neg_m = 0.f, seen = -INFINITY, l_run = 0.f;
+    float16v acc[DB], s;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[db][e] = 0.f;
+
+    // sub-unit u of the tile in buffer buf, u == NSUB: the first one of the next tile
+    constexpr int AHEAD = 4;
+    auto k_load = [&](uint32_t buf, int u, int kk) PF_INLINE {
+        const uint32_t at = ((u == NSUB ? buf ^ 1u : buf) * kPfBuf + (uint32_t)(u % NSUB) * (32u * ROWB)) / 16;
+        return __builtin_bit_cast(half8, ((lds_u4_ptr)(uintptr_t)ka[kk])[at]);
+    };
+    auto v_load = [&](uint32_t buf, int u, int i) PF_INLINE {             // operand i: tokens 16 (i / DB) .. + 15, d block i % DB
+        typedef short4v __attribute__((address_space(3))) *lds_s4;
+        const uint32_t at = (buf * kPfBuf + (uint32_t)u * (32u * ROWB) + 16u * ROWB * (uint32_t)(i / DB)) / 8;
+        const half4 v0 = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(uintptr_t)va[0][i % DB] + at));
+        const half4 v1 = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(uintptr_t)va[1][i % DB] + at));
+        return cat8(v0, v1);
+    };
+    auto s_load = [&](uint32_t buf, int u, int i) PF_INLINE {             // K scales of tokens 8 i + 4 half .. + 3
+        const uint32_t at = ((u == NSUB ? buf ^ 1u : buf) * 512u + 128u * (uint32_t)(u % NSUB) + 32u * i) / 16;
+        return __builtin_bit_cast(float4v, ((lds_u4_ptr)(uintptr_t)sa)[at]);
+    };
+    // scores of a unit (first token tw): times their K scale, relative to the running maximum, which moves if it has to
+    auto maxima = [&](int tw, const float4v (&ks)[4]) PF_INLINE {
+        const bool edge = !(tw + 32 <= wave_min && tw + 32 <= b_end && tw >= col_start);
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; e++) s[e] = __builtin_fmaf(s[e], ks[e >> 2][e & 3], neg_m);
+        if (edge) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const int t = tw + 8 * (e >> 2) + 4 * half + (e & 3);
+                if (!(t < col_lim && t < b_end && t >= col_start)) s[e] = -INFINITY;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e++) tmax = fmaxf(tmax, s[e]);
+        {
+            const uint32_t x = __float_as_uint(tmax);
+            const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+            tmax = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+        }
+        if (__builtin_amdgcn_ballot_w64(tmax > seen) != 0) {
+            const float d = tmax > seen ? tmax : 0.f;
+            const float alpha = seen == 0.f ? __builtin_amdgcn_exp2f(-d) : 0.f;
+            l_run *= alpha;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[db][e] *= alpha;
+#pragma unroll
+            for (int e = 0; e < 16; e++) s[e] -= d;
+            neg_m -= d;
+            seen = tmax > seen ? 0.f : seen;
+        }
+    };
+    // One unit of 32 tokens.  In program order, one matrix instruction at a time with vector work behind it:
+    //   S^T of the next unit, with the exponentials of this one; O^T += V^T . P^T of this one, with the decoding.
+    half8 kf[AHEAD];                                                      // operands of the next unit's first products
+    auto unit = [&](int tw, uint32_t buf, int u) PF_INLINE {
+        constexpr int NV = 2 * DB, PER = 8 / KS;               // pairs of exponentials per matrix instruction
+        const bool dec = u == NSUB - 1;
+        half8 vf[AHEAD];
+        float4v ks[4];
+        float16v sn;
+        float pe[2 * PER];
+        uint32_t pp[8];
+#pragma unroll
+        for (int e = 0; e < 16; e++) sn[e] = 0.f;
+        auto finish = [&](int k) PF_INLINE {                              // the exponentials of step k: summed, packed
+#pragma unroll
+            for (int x = 0; x < PER; x++) {
+                const int i = k * PER + x;
+                l_run += pe[2 * x] + pe[2 * x + 1];
+                pp[i] = __builtin_bit_cast(uint32_t, half2v{(_Float16)pe[2 * x], (_Float16)pe[2 * x + 1]});
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < KS; k++) {
+            __builtin_amdgcn_sched_barrier(0);
+            sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[k % AHEAD], qf[k], sn, 0, 0, 0);
+            if (k + AHEAD < KS) kf[k % AHEAD] = k_load(buf, u + 1, k + AHEAD);
+            else vf[k + AHEAD - KS] = v_load(buf, u, k + AHEAD - KS);
+            if (k > 0) finish(k - 1);
+#pragma unroll
+            for (int x = 0; x < 2 * PER; x++) pe[x] = __builtin_amdgcn_exp2f(s[2 * PER * k + x]);
+        }
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            if (i == 0) finish(KS - 1);
+            if (i > 0) __builtin_amdgcn_sched_barrier(0);
+            const int st = i / DB, db = i % DB;
+            acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i % AHEAD], __builtin_bit_cast(half8, uint4v{pp[4 * st], pp[4 * st + 1], pp[4 * st + 2], pp[4 * st + 3]}), acc[db], 0, 0, 0);
+            if (i + AHEAD < NV) vf[i % AHEAD] = v_load(buf, u, i + AHEAD);
+            if (dec) {
+#pragma unroll
+                for (int j = i * 8 / NV; j < (i + 1) * 8 / NV; j++) piece(j, cc[buf]);
+                if (i * 8 / NV <= 3 && (i + 1) * 8 / NV > 3) {
+                    request(d_t, cc[buf]);
+                    d_t += TILE;
+                }
+            }
+            if (i == NV / 2) {
+#pragma unroll
+                for (int x = 0; x < 4; x++) ks[x] = s_load(buf, u + 1, x);
+            }
+        }
+        s = sn;
+        if (dec) __syncthreads();
+        const bool over = u + 1 == NSUB;                                  // the next unit is the first one of the next tile
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) kf[i] = k_load(over ? buf ^ 1u : buf, over ? 1 : u + 2, i);
+        maxima(over ? tw + 32 + TILE - 32 * NSUB : tw + 32, ks);
+    };
+    auto tile = [&](int t0, uint32_t buf) PF_INLINE {
+#pragma unroll
+        for (int u = 0; u < NSUB; u++) {
+            if (NSUB > 1 && u == NSUB - 1) __syncthreads();               // K of this tile is read no more: its buffer is next
+            unit(t0 + 32 * (NSUB * kvg + u), buf, u);
+        }
+    };
+    if (work) {
+        float4v ks[4];
+#pragma unroll
+        for (int x = 0; x < 4; x++) ks[x] = s_load(0u, 0, x);
+#pragma unroll
+        for (int e = 0; e < 16; e++) s[e] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < KS; kk++) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k_load(0u, 0, kk), qf[kk], s, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) kf[i] = k_load(0u, 1, i);
+        maxima(b_begin + 32 * NSUB * kvg, ks);
+    }
+    // (a wavefront whose columns end before the block's goes on with masked scores: it has to decode anyway)
+    for (int t0 = b_begin; t0 < b_end;) {
+        tile(t0, 0u);
+        t0 += TILE;
+        if (t0 >= b_end) break;
+        tile(t0, 1u);
+        t0 += TILE;
+    }
+
+    // ---- epilogue: lane (col, half) holds d = 32 db + 8 i + 4 half + j of its column ----
+    {
+        const uint32_t x = __float_as_uint(l_run);
+        const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        l_run = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    float m_run = seen == 0.f ? -neg_m : -INFINITY;
+    if (KVG == 2) {
+        // the wavefronts of tokens 32..63 hand their part over: [wave][element][lane], then m and l
+        float *red = reinterpret_cast<float *>(lds_tab) + cw * (DB * 16 * 64);
+        float *ml = reinterpret_cast<float *>((unsigned char *)lds_tab + kPfScale) + cw * 128;
+        if (kvg == 1) {
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) red[(db * 16 + e) * 64 + lane] = acc[db][e];
+            ml[lane] = m_run;
+            ml[64 + lane] = l_run;
+        }
+        __syncthreads();
+        if (kvg == 0) {
+        const float m1 = ml[lane], l1 = ml[64 + lane], m = fmaxf(m_run, m1);
+        const float f0 = m > -INFINITY ? __builtin_amdgcn_exp2f(m_run - m) : 0.f, f1 = m > -INFINITY ? __builtin_amdgcn_exp2f(m1 - m) : 0.f;
+        l_run = fmaf(l1, f1, l_run * f0);
+        m_run = m;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[db][e] = fmaf(red[(db * 16 + e) * 64 + lane], f1, acc[db][e] * f0);
+        }
+    }
+    if (!col_ok || (KVG == 2 && kvg == 1)) {
+    } else if (p.n_splits == 1) {
+        const float f = l_run > 0.f ? 1.f / l_run : 0.f;
+        uint16_t *o = (uint16_t *)p.O + b * p.osb + hq * p.osh + (int64_t)tq * p.ost + 4 * half;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint16_t h[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float v = acc[db][4 * i + j] * f;
+                    h[j] = DT == HQMQ_F16 ? __half_as_ushort(__float2half_rn(v)) : f32_to_bf16_bits(v);
+                }
+                *reinterpret_cast<uint2 *>(o + 32 * db + 8 * i) = uint2{(uint32_t)h[0] | (uint32_t)h[1] << 16, (uint32_t)h[2] | (uint32_t)h[3] << 16};
+            }
+    } else {
+        float *wp = p.ws + ((((size_t)b * p.Hq + hq) * p.Tq + tq) * p.n_splits + sp) * (size_t)(DH + kPartialHead);
+        if (half == 0) { wp[0] = m_run; wp[1] = l_run; }
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float4v v;
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = acc[db][4 * i + j];
+                *reinterpret_cast<float4v *>(wp + kPartialHead + 32 * db + 8 * i + 4 * half) = v;
+            }
+    }
+    __syncthreads();
+    }
+}
+
+// Launch plan, from measured times in us: a tile takes a block of 128 columns 1.37, one of 256 columns 2.7 (all compute units
+// busy); starting (tables, first tiles) and finishing take a block 12; a compute unit holds one block; partials are written
+// and merged at 2 TB/s.
+struct PfPlan {
+    bool wide;
+    int splits;
+    double us;
+};
+static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int causal, int64_t off, int fixed_splits) {
+    const double last = causal ? std::max(1.0, std::min((double)Tkv, (double)off + Tq)) : std::max(Tkv, 1);      // tokens the last query sees
+    const double mean = causal ? std::min(1.0, std::max(0.5, ((double)off + 0.5 * Tq) / last)) : 1.0;            // all, relative to it
+    const int tiles = (int)((last * d_h + 8191) / 8192);
+    PfPlan best{false, 1, 1e30};
+    static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+    for (int i = 0; i < (fixed_splits > 0 ? 1 : (int)(sizeof(kSplits) / sizeof(int))); i++) {
+        const int s = fixed_splits > 0 ? fixed_splits : kSplits[i];
+        if (i > 0 && s > tiles / 2) break;
+        for (int wide = 0; wide < 2; wide++) {
+            const double rounds = (double)(((cols + (wide ? 255 : 127)) / (wide ? 256 : 128) * nz * s + 255) / 256);
+            // the longest block or a compute unit's share of all of them, whichever is more; partials: written and read at 3 TB/s
+            const double us = std::max(1.0, mean * rounds) * ((tiles + s - 1) / s) * (wide ? 2.7 : 1.37) + 12.0 * rounds +
+                              (s > 1 ? 5.0 + (double)(cols * nz) * s * (d_h + 4) * 8 / 2e6 : 0.0);
+            if (us < best.us) best = PfPlan{wide != 0, s, us};
+        }
+    }
+    return best;
+}
+// Whether these kernels can take the call at all.
+static bool attn_prefill_takes(const hqmq_attn_args *a) {
+    if ((a->dtype != HQMQ_F16 && a->dtype != HQMQ_BF16) || a->wide_range || a->K.flag_plane || (a->n_chunks != 16 && a->n_chunks != 32) ||
+        a->fp8_table_storage || (a->force_generic && a->force_generic != 3) || a->softmax_scale <= 0.f)
+        return false;
+    if (a->main_bits != 16 && (a->main_bits != 12 || a->aux_bits < 1)) return false;
+    if (a->idx_bits < 6 || a->aux_bits > 4) return false;                          // the 16-bit decode needs radius codes below 1024
+    if (a->t_cap % 64 || a->t_cap >= (1 << 25)) return false;                      // rows are addressed by 32-bit offsets
+    if (kPfTab + ((size_t)a->K.K + a->V.K) * 8 + 128 > 160 * 1024) return false;
+    if (a->aux_bits && (((uintptr_t)a->K.aux_plane | (uintptr_t)a->V.aux_plane) & 3)) return false;
+    if ((((uintptr_t)a->O) | (uintptr_t)(a->o_sb * 2) | (uintptr_t)(a->o_sh * 2) | (uintptr_t)(a->o_st * 2)) & 7) return false;
+    return true;
+}
+// The same for the kernels of attention_fast.hip: blocks of 16 columns (0.47 us a tile) or, where that leaves a block per
+// compute unit, of 32 (0.6 us), which start and finish in 6 us.
+static double fast_us(int64_t cols, int64_t nz, int Tkv, int d_h, int splits) {
+    const int64_t cg = (cols + 15) / 16, pairs = (cg + 1) / 2 * nz * splits;
+    const bool two = cg > 1 && pairs >= 256;
+    const double tiles = ((double)Tkv * d_h + 8191) / 8192;
+    return 3.0 + (double)(((two ? pairs : cg * nz * splits) + 255) / 256) * (6.0 + tiles / splits * (two ? 0.6 : 0.47)) +
+           (splits > 1 ? 3.0 + (double)(cols * nz) * splits * (d_h + 4) * 8 / 2e6 : 0.0);
+}
+// The number of splits of a call that leaves it open, 0 if it is better off with the other kernels (by a clear margin: the
+// estimates are good to some 15 %); splits > 0: the same decision for a given number.
+int attn_prefill_splits(const hqmq_attn_args *a, int splits) {
+    const int64_t cols = (int64_t)a->T_q * (a->H_q / a->H_kv), nz = (int64_t)a->B * a->H_kv;
+    if (cols < 64 || !attn_prefill_takes(a)) return 0;
+    const PfPlan plan = pf_plan(cols, nz, a->T_q, a->T_kv, 4 * a->n_chunks, a->causal, a->causal_offset, splits);
+    const int other = splits > 0 ? splits : hqmq_attn_pick_splits(a->B, a->H_q, a->H_kv, a->T_q, a->T_kv, a->kv_len != nullptr);
+    return a->force_generic == 3 || plan.us < 0.85 * fast_us(cols, nz, a->T_kv, 4 * a->n_chunks, other) ? plan.splits : 0;
+}
+
+template <int DH, int MB, bool AUX, int DT>
+static int launch_pf(const AttnParams &p, hipStream_t st, const LaunchTiming &tm) {
+    const int64_t cols = (int64_t)p.Tq * p.G, nz = (int64_t)p.B * p.Hkv * p.n_splits;
+    const bool wide = pf_plan(cols, (int64_t)p.B * p.Hkv, p.Tq, p.Tkv, DH, p.causal, p.causal_offset, p.n_splits).wide;
+    const int64_t gx = (cols + (wide ? 255 : 127)) / (wide ? 256 : 128);
+    // Column blocks per block, one after the other (the tables stay in LDS): as few rounds of 256 blocks as possible.  Ragged
+    // batches leave the choice of the next block to the hardware.
+    int64_t rows = gx;
+    if (!p.kv_len && !p.kv_start) {
+        int64_t best = (gx * nz + 255) / 256;
+        for (int64_t per = 2; per <= gx && per <= 64; per++) {
+            const int64_t r = (gx + per - 1) / per, rounds = (r * nz + 255) / 256 * per;
+            if (rounds <= best) { best = rounds; rows = r; }
+        }
+    }
+    if (rows * nz > 0x7fffffff) return HQMQ_ERR_SHAPE;
+    const size_t shmem = kPfTab + (size_t)((p.Kc.K * 8 + 127) & ~127) + (size_t)p.Vc.K * 8;
+    auto kern = wide ? attn_prefill_kernel<DH, MB, AUX, DT, 1> : attn_prefill_kernel<DH, MB, AUX, DT, 2>;
+    const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+    if (e != hipSuccess) return (int)e;
+    const dim3 grid((unsigned)(rows * nz));
+    if (tm.start || tm.stop) hipExtLaunchKernelGGL(kern, grid, dim3(512), shmem, st, tm.start, tm.stop, 0, p, (int)gx, (int)rows);
+    else hipLaunchKernelGGL(kern, grid, dim3(512), shmem, st, p, (int)gx, (int)rows);
+    return hip_status(hipGetLastError());
+}
+
+template <int DH, int DT>
+static int launch_pf_layout(const AttnParams &p, int mb, hipStream_t st, const LaunchTiming &tm) {
+    if (mb == 16 && p.aux_bits == 0) return launch_pf<DH, 16, false, DT>(p, st, tm);
+    return mb == 16 ? launch_pf<DH, 16, true, DT>(p, st, tm) : launch_pf<DH, 12, true, DT>(p, st, tm);
+}
+
+int launch_attn_prefill(const AttnParams &p, int mb, hipStream_t st, const LaunchTiming &tm) {
+    if (p.n == 32) return p.dtype == HQMQ_F16 ? launch_pf_layout<128, HQMQ_F16>(p, mb, st, tm) : launch_pf_layout<128, HQMQ_BF16>(p, mb, st, tm);
+    return p.dtype == HQMQ_F16 ? launch_pf_layout<64, HQMQ_F16>(p, mb, st, tm) : launch_pf_layout<64, HQMQ_BF16>(p, mb, st, tm);
+}
+
+}  // namespace hqmq

@@ -451,9 +451,10 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
         a.batch_order = batch_order.data_ptr()
     if causal:
         a.causal, a.causal_offset = 1, causal_offset
+    many = False
     if n_splits <= 0:
         n_splits = pick_splits(shape[0], shape[1], Kc.H, shape[2], max(T_kv, 1), kv_lens is not None)
-    a.n_splits = n_splits
+        many = shape[2] > 1 and not static_scratch
     if skip_combine:
         a.skip_combine = 1
     if force_generic:
@@ -464,6 +465,9 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
         a.wide_range = 1
     if kernel_events is not None:
         a.start_event, a.stop_event = kernel_events
+    if many:
+        n_splits = L.lib().hqmq_attn_splits(C.addressof(a))
+    a.n_splits = n_splits
     if static_scratch:
         L.call(L.lib().hqmq_attn_fwd_static, "hqmq_attn_fwd_static", index, C.addressof(a))
         return O

@@ -262,7 +262,8 @@ typedef struct hqmq_attn_args {
     int skip_combine;         /* 1: leave the split partials in the workspace (merge later with hqmq_attn_combine) */
     int force_generic;        /* 1: use the layout-generic kernel even where a specialised one exists (testing);
                                  2: keep the specialised kernels that hold their tiles in registers where the kernel that
-                                 lands its loads in LDS would run (plain 16+0 caches at d_h 128; identical results) */
+                                 lands its loads in LDS would run (plain 16+0 caches at d_h 128; identical results);
+                                 3: take the chunked-prefill kernel wherever it can run, not only where it is faster */
     const int32_t *kv_start;  /* [B] or NULL: first visible token of every sequence (left-padded batches) */
     const int32_t *batch_order; /* [B] or NULL: a permutation of 0..B-1, the order in which the sequences' blocks are
                                    started (pass the sequences sorted by length, longest first, for ragged batches) */
@@ -284,6 +285,9 @@ typedef struct hqmq_attn_args {
 int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, int n_splits);
 /* The n_splits hqmq_attn_fwd would choose; ragged = 1 when kv_len is passed (more, smaller blocks). */
 int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv, int ragged);
+/* The n_splits that suits these arguments best (a->n_splits is not looked at), for callers that size the workspace by it:
+   chunked prefill over plain caches wants other counts than hqmq_attn_pick_splits names from the shapes alone. */
+int hqmq_attn_splits(const hqmq_attn_args *a);
 int hqmq_attn_fwd(const hqmq_attn_args *a, void *stream);
 /* Merge of the split-KV partials (m, l, acc) left in the workspace; hqmq_attn_fwd runs it unless skip_combine. */
 int hqmq_attn_combine(const void *workspace, void *O, int dtype, int B, int H_q, int T_q, int d_h, int n_splits,

@@ -690,3 +690,39 @@ def test_lds_landing_kernel_equals_register_tile_kernel(dn, T, B, Tq, causal, ns
     refs = masked_two_refs(cache, Q, T, mask)
     assert_attention_close(O, *refs, base=2e-3, what="LDS landing")
     assert_attention_close(Og, *refs, base=2e-3, what="generic")
+
+
+@pytest.mark.parametrize("dn,S,b_r,d_h,Hq,Hkv,B,Tq,T,ns,lens,starts", [
+    ("fp16", 96, 4, 128, 4, 1, 1, 32, 32, 0, None, None),           # one block of 128 columns, half a tile
+    ("fp16", 96, 4, 128, 4, 1, 1, 33, 65, 1, None, None),           # one column block and a bit, one token past a tile
+    ("bf16", 96, 4, 128, 6, 2, 2, 257, 129, 2, None, None),         # columns that split a query token's group over wavefronts
+    ("fp16", 24, 3, 128, 8, 8, 1, 255, 300, 3, None, None),         # 12 + 1 bits, G = 1
+    ("bf16", 192, 6, 128, 8, 2, 2, 64, 641, 0, [641, 3], [70, 0]),  # 16 + 3 bits, limits on both sides
+    ("fp16", 192, 4, 64, 8, 1, 3, 97, 190, 2, [190, 0, 64], None),  # 16 + 1 bits, an empty sequence
+    ("bf16", 24, 3, 64, 16, 8, 1, 130, 130, 1, None, [129]),        # 12 + 1 bits at d_h 64
+    ("fp16", 96, 4, 64, 32, 8, 8, 520, 520, 1, None, None),         # blocks of 256 columns (512 of them and more)
+    ("bf16", 192, 4, 128, 32, 8, 4, 1030, 1100, 1, [1100, 1, 64, 1037], None)])
+def test_prefill_tiles_shared_by_a_block(dn, S, b_r, d_h, Hq, Hkv, B, Tq, T, ns, lens, starts):
+    """Many query columns per KV head (chunked and whole prefill): tiles decoded once per block into LDS (force_generic=3 takes
+    that kernel at every size)."""
+    import hqmq
+    dt = DT[dn]
+    g = torch.Generator().manual_seed(T + 3 * Tq)
+    k, v = torch.randn(B, Hkv, T, d_h, generator=g).to(dt).to(DEV), torch.randn(B, Hkv, T, d_h, generator=g).to(dt).to(DEV)
+    q = hqmq.HQMQ(n_layers=1, n_heads=Hkv, secondary_size=S, radius_bits=b_r, device=DEV)
+    cache = q.new_cache(B, T, d_h, dt, 0)
+    q.append(cache, k, v, 0)
+    Q = torch.randn(B, Hq, Tq, d_h, generator=g).to(dt).to(DEV)
+    as_t = lambda a: None if a is None else torch.tensor(a, dtype=torch.int32, device=DEV)
+    kk, qq = torch.arange(T, device=DEV).view(1, 1, 1, T), torch.arange(Tq, device=DEV).view(1, 1, Tq, 1)
+    for causal in (True, False):
+        off = T - Tq
+        O = hqmq.fused_attention_packed(Q, cache, causal=causal, causal_offset=off if causal else 0, n_splits=ns, kv_lens=as_t(lens),
+                                        kv_starts=as_t(starts), T_kv=T, force_generic=3)
+        mask = (kk <= qq + off) if causal else torch.ones(1, 1, Tq, T, dtype=torch.bool, device=DEV)
+        mask = mask.expand(B, 1, Tq, T)
+        if lens is not None:
+            mask = mask & (kk < as_t(lens).view(B, 1, 1, 1))
+        if starts is not None:
+            mask = mask & (kk >= as_t(starts).view(B, 1, 1, 1))
+        assert_attention_close(O, *masked_two_refs(cache, Q, T, mask), base=2e-3, what=f"causal={causal}")
