@@ -82,12 +82,24 @@ class CropArgs(C.Structure):
                 ("t_cap", i64), ("n_chunks", C.c_int), ("lengths", vp), ("length", C.c_int)]
 
 
+class PackSide(C.Structure):
+    _fields_ = [("idx", vp), ("idx_sb", i64), ("idx_sh", i64), ("idx_st", i64), ("rq", vp), ("rq_sb", i64), ("rq_sh", i64), ("rq_st", i64),
+                ("scale_in", vp), ("scale_sb", i64), ("scale_sh", i64), ("scale_st", i64), ("T", C.c_int),
+                ("main_plane", vp), ("aux_plane", vp), ("scale_plane", vp), ("scale_max_bits", vp)]
+
+
+class PackArgs(C.Structure):
+    _fields_ = [("side", PackSide * 2), ("dtype", C.c_int), ("B", C.c_int), ("H", C.c_int), ("n_chunks", C.c_int), ("idx_bits", C.c_int),
+                ("main_bits", C.c_int), ("aux_bits", C.c_int), ("t_cap", i64)]
+
+
 EXPORTS = [
     "hqmq_version", "hqmq_status_string", "hqmq_layout_bits", "hqmq_build_joint", "hqmq_quantize",
     "hqmq_med3x_workspace_bytes", "hqmq_med3x_threshold", "hqmq_outlier_mask", "hqmq_outlier_compact", "hqmq_dequant",
     "hqmq_pack_codes", "hqmq_dequant_packed", "hqmq_attn_workspace_bytes", "hqmq_attn_pick_splits", "hqmq_attn_splits",
     "hqmq_attn_fwd", "hqmq_attn_combine", "hqmq_append_kv", "hqmq_attn_static_scratch_bytes", "hqmq_attn_fwd_static",
     "hqmq_search_grid_bytes", "hqmq_build_search_grid", "hqmq_quantize_grid", "hqmq_append_kv_grid", "hqmq_crop",
+    "hqmq_pack_kv",
 ]
 BENCH_EXPORTS = ["hqmq_bench_read_planes_sink_bytes", "hqmq_bench_read_planes", "hqmq_bench_read_plain", "hqmq_bench_read_lds",
                  "hqmq_bench_empty"]
@@ -111,8 +123,9 @@ def lib():
             getattr(L, name).restype = i64
         # the calls of a decode loop take addresses as plain integers
         for name, n in (("hqmq_attn_fwd", 2), ("hqmq_attn_fwd_static", 2), ("hqmq_attn_splits", 1), ("hqmq_quantize_grid", 3), ("hqmq_append_kv_grid", 5), ("hqmq_crop", 2),
-                        ("hqmq_quantize", 2), ("hqmq_append_kv", 3)):
+                        ("hqmq_quantize", 2), ("hqmq_append_kv", 3), ("hqmq_pack_kv", 2)):
             getattr(L, name).argtypes = [vp] * n
+        L.hqmq_dequant.argtypes = [vp, i64, i64, i64, vp, i64, i64, i64, vp, i64, i64, i64, vp, i64] + [C.c_int] * 7 + [vp, vp]
         L.hqmq_med3x_threshold.argtypes = [vp, i64, i64, i64, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, vp, i64, vp, vp, vp, vp]
         _lib = L
     return _lib

@@ -20,44 +20,13 @@ import torch.nn.functional as F
 
 from . import _lib as L
 from . import ops
-from .packed import PackedKV, PackedTensor
+from .packed import PackedKV
 
 
 def decode_dequant(idx: torch.Tensor, radius_q: torch.Tensor, radius_scale: torch.Tensor, joint: torch.Tensor,
                    r_qmax: int) -> torch.Tensor:
     """(B, H, T, n) codes -> dense (B, H, T, 4n) in joint.dtype."""
     return ops.dequant(idx, radius_q, radius_scale, joint, r_qmax)
-
-
-def _bits_for(r_qmax: int) -> int:
-    b = max(1, int(r_qmax).bit_length())
-    if b > 8:
-        raise L.HqmqError(f"r_qmax={r_qmax} needs more than 8 radius bits")
-    return b
-
-
-def _pack_unpacked(idx, rq, rs, joint, r_qmax: int) -> PackedTensor:
-    """The reference's unpacked representation -> a PackedTensor (codes packed on the GPU)."""
-    B, H, T, n = idx.shape
-    K = joint.shape[1]
-    if joint.stride(-1) != 1 or joint.stride(1) != 4:
-        joint = joint.contiguous()
-    # a table of K rows is addressed like one of ceil(K/24) secondaries; the radius field holds r_qmax
-    S_eff = max(1, -(-K // 24))
-    rb = _bits_for(r_qmax)
-    ib, mb, ab = L.layout_bits(S_eff, rb)
-    if mb == 12 and (n // 4) % 2:      # a lane's share of a 12-bit row must be whole bytes: use 16-bit codes
-        mb, ab = 16, max(0, ib + rb - 16)
-    pt = PackedTensor(B, H, T, 4 * n, S_eff, rb, joint.dtype, idx.device, joint=joint, layout=(ib, mb, ab))
-    pt.qmax = int(r_qmax)
-    ops.pack_codes(idx, rq, pt)
-    pt.scale[:, :, :T] = rs            # into the padded plane: rows up to the capacity stay readable
-    if pt.scale_max is not None:       # the range guard of bf16 / fp32 caches: the largest finite scale, as fp32 bits
-        pt.scale_max = torch.nan_to_num(rs.detach().float().abs(), nan=0.0, posinf=0.0).amax().reshape(1).view(torch.int32)
-        if pt.dtype == torch.bfloat16 and not torch.cuda.is_current_stream_capturing():
-            pt.refresh_range()         # one device read: bf16 scales of 2^15 and more take the guarded kernel
-    pt.length = T
-    return pt
 
 
 def _through_fp8(joint: torch.Tensor) -> torch.Tensor:
@@ -100,10 +69,8 @@ def fused_attention(
     if use_fp8_codebook:
         joint_K, joint_V = _through_fp8(joint_K), _through_fp8(joint_V)
     Qc = Q if Q.dtype == dt else Q.to(dt)
-    Kc = _pack_unpacked(K_idx, K_radius_q, K_radius_scale, joint_K, r_qmax)
-    Vc = _pack_unpacked(V_idx, V_radius_q, V_radius_scale, joint_V.to(dt), r_qmax)
-    O = ops.attn_fwd(Qc, Kc, Vc, T_kv, kv_lens=kv_lens, causal=causal, causal_offset=causal_offset,
-                     softmax_scale=softmax_scale, n_splits=n_splits)
+    O = ops.fused_unpacked(Qc, (K_idx, K_radius_q, K_radius_scale, joint_K), (V_idx, V_radius_q, V_radius_scale, joint_V.to(dt)), int(r_qmax),
+                           kv_lens=kv_lens, causal=causal, causal_offset=causal_offset, softmax_scale=softmax_scale, n_splits=n_splits)
     return O if O.dtype == Q.dtype else O.to(Q.dtype)
 
 

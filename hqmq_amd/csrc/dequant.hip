@@ -3,9 +3,11 @@
 //                        (src/quantizers/hqmq_attention.py:39-65 of the reference);
 //                        replaces hqmq_decode_triton (src/quantizers/hqmq_kernel.py:102-132)
 //   hqmq_pack_codes      unpacked int32 codes -> packed main/aux rows
+//   hqmq_pack_kv         unpacked int32 codes and scales of K and V -> all planes, in one launch
 //   hqmq_dequant_packed  packed cache (+ outlier sideband) -> dense
 // Compiled with -ffp-contract=off: every product rounds to D on its own.
 #include "common.h"
+#include <algorithm>
 
 namespace hqmq {
 
@@ -22,26 +24,150 @@ __device__ __forceinline__ uint32_t read_bits(const uint8_t *row, int row_bytes,
     return nbits >= 32 ? v : (v & ((1u << nbits) - 1u));
 }
 
-template <class D>
-__global__ void dequant_kernel(const int32_t *idx, int64_t isb, int64_t ish, int64_t ist, const int32_t *rq, int64_t rsb_,
+// PER chunks per thread (2: 16-bit types, even rows, aligned operands: 8-byte loads of the codes, 16-byte stores of the
+// values); a row of the grid is one (b, h).  Bound by memory: 16 bytes in, 8 out and a gathered codeword per chunk of a
+// 16-bit type.  fp16, B = 1, 8 heads, 4096 tokens of 128: 6.7 us against 13.9 with a chunk per thread and 64-bit index
+// divisions.
+template <class D, int PER>
+__global__ __launch_bounds__(256) void dequant_kernel(const int32_t *idx, int64_t isb, int64_t ish, int64_t ist, const int32_t *rq, int64_t rsb_,
                                int64_t rsh_, int64_t rst_, const typename D::storage *rs, int64_t ssb, int64_t ssh,
-                               int64_t sst, const typename D::storage *joint, int64_t jsh, int K, int B, int H, int T, int n,
+                               int64_t sst, const typename D::storage *joint, int64_t jsh, int K, int BH, int H, int T, int n,
                                int qmax, typename D::storage *out) {
-    const int64_t total = (int64_t)B * H * T * n;
-    for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(g % n);
-        const int64_t row = g / n;
-        const int t = (int)(row % T);
-        const int h = (int)((row / T) % H);
-        const int b = (int)(row / ((int64_t)T * H));
-        int k = idx[b * isb + h * ish + t * ist + c];
-        k = k < 0 ? 0 : (k >= K ? K - 1 : k);
-        const float q = D::rnd((float)rq[b * rsb_ + h * rsh_ + t * rst_ + c]);
-        const float s = D::load(rs + b * ssb + h * ssh + t * sst);
-        const float r = D::rnd(D::rnd(q * s) / (float)qmax);
-        const typename D::storage *cw = joint + h * jsh + (int64_t)k * 4;
-        for (int j = 0; j < 4; j++) D::store(out + g * 4 + j, D::rnd(D::load(cw + j) * r));
+    using ST = typename D::storage;
+    const uint32_t per_row = (uint32_t)n / PER;
+    for (int bh = blockIdx.y; bh < BH; bh += gridDim.y) {
+        const int b = bh / H, h = bh - b * H;
+        const int32_t *ib = idx + b * isb + h * ish, *rb = rq + b * rsb_ + h * rsh_;
+        const ST *sb = rs + b * ssb + h * ssh, *jb = joint + h * jsh;
+        ST *ob = out + (int64_t)bh * T * n * 4;
+        for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < (int64_t)T * per_row; g += (int64_t)gridDim.x * 256) {
+            const uint32_t t = g <= 0xffffffffll ? (uint32_t)g / per_row : (uint32_t)(g / per_row);
+            const int c = (int)(g - (int64_t)t * per_row) * PER;
+            int k[PER], q[PER];
+            if constexpr (PER == 2) {
+                const int2 kv = *reinterpret_cast<const int2 *>(ib + t * ist + c), qv = *reinterpret_cast<const int2 *>(rb + t * rst_ + c);
+                k[0] = kv.x; k[1] = kv.y; q[0] = qv.x; q[1] = qv.y;
+            } else {
+                k[0] = ib[t * ist + c];
+                q[0] = rb[t * rst_ + c];
+            }
+            const float s = D::load(sb + t * sst);
+            ST v[4 * PER];
+#pragma unroll
+            for (int i = 0; i < PER; i++) {
+                const int ki = k[i] < 0 ? 0 : (k[i] >= K ? K - 1 : k[i]);
+                const float r = D::rnd(D::rnd(D::rnd((float)q[i]) * s) / (float)qmax);
+                const ST *cw = jb + (int64_t)ki * 4;
+                if constexpr (PER == 2) {
+                    const uint2 w = *reinterpret_cast<const uint2 *>(cw);
+                    const ST e[4] = {(ST)w.x, (ST)(w.x >> 16), (ST)w.y, (ST)(w.y >> 16)};
+#pragma unroll
+                    for (int j = 0; j < 4; j++) D::store(v + 4 * i + j, D::rnd(D::load(e + j) * r));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) D::store(v + 4 * i + j, D::rnd(D::load(cw + j) * r));
+                }
+            }
+            ST *dst = ob + ((int64_t)t * n + c) * 4;
+            if constexpr (PER == 2) {
+                uint4 w;
+                w.x = (uint32_t)v[0] | (uint32_t)v[1] << 16; w.y = (uint32_t)v[2] | (uint32_t)v[3] << 16;
+                w.z = (uint32_t)v[4] | (uint32_t)v[5] << 16; w.w = (uint32_t)v[6] | (uint32_t)v[7] << 16;
+                *reinterpret_cast<uint4 *>(dst) = w;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) dst[j] = v[j];
+            }
+        }
     }
+}
+
+// The unpacked codes of K and V -> the planes that attention reads, one launch: a thread packs eight chunks of a row (of
+// the last group of a row perhaps four), rows T .. t_cap - 1 are written as zeros, so that the planes need no clearing, and
+// the largest finite scale goes to *scale_max.  Bound by reading the 8 bytes of a chunk: 2048 tokens of 8 heads of 128,
+// 16.8 MB: 5.1 us for both tensors; packed a byte per thread they took 15 us each, and 8 launches for clearing and copying.
+struct PackSide {
+    const int32_t *idx, *rq;
+    int64_t isb, ish, ist, rsb, rsh, rst;
+    const void *scale_in;
+    int64_t ssb, ssh, sst;
+    uint8_t *main_plane, *aux_plane;
+    void *scale_plane;
+    uint32_t *scale_max;
+    int T, vec;             // vec: the rows of idx and rq can be read 16 bytes at a time
+};
+struct PackPair { PackSide s[2]; };
+
+template <class D, int MB>
+__global__ __launch_bounds__(256) void pack_kv_kernel(PackPair pair, int BH, int H, int n, int idx_bits, int ab, int t_cap) {
+    using ST = typename D::storage;
+    const PackSide &p = pair.s[blockIdx.z];
+    const int groups = (n + 7) >> 3, mrb = n * MB / 8, arb = (n * ab + 7) >> 3;
+    const uint32_t g = blockIdx.x * 256u + threadIdx.x, t = g / (uint32_t)groups, grp = g - t * (uint32_t)groups;
+    const uint32_t idx_mask = (1u << idx_bits) - 1u;
+    uint32_t most = 0;
+    if (t < (uint32_t)t_cap)
+        for (int bh = blockIdx.y; bh < BH; bh += gridDim.y) {
+            const int b = bh / H, h = bh - b * H;
+            const int left = n - (int)grp * 8;                           // chunks in this group: 8, or 4 at the end of a row
+            uint32_t code[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) code[i] = 0;
+            ST scale = 0;
+            if ((int)t < p.T) {
+                const int32_t *ip = p.idx + b * p.isb + h * p.ish + t * p.ist + grp * 8;
+                const int32_t *rp = p.rq + b * p.rsb + h * p.rsh + t * p.rst + grp * 8;
+                if (p.vec && left >= 8) {
+                    const int4 i0 = reinterpret_cast<const int4 *>(ip)[0], i1 = reinterpret_cast<const int4 *>(ip)[1];
+                    const int4 r0 = reinterpret_cast<const int4 *>(rp)[0], r1 = reinterpret_cast<const int4 *>(rp)[1];
+                    const int32_t ii[8] = {i0.x, i0.y, i0.z, i0.w, i1.x, i1.y, i1.z, i1.w}, rr[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+                    for (int i = 0; i < 8; i++) code[i] = ((uint32_t)ii[i] & idx_mask) | ((uint32_t)rr[i] << idx_bits);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; i++)
+                        if (i < left) code[i] = ((uint32_t)ip[i] & idx_mask) | ((uint32_t)rp[i] << idx_bits);
+                }
+                if (grp == 0) scale = ((const ST *)p.scale_in)[b * p.ssb + h * p.ssh + t * p.sst];
+            }
+            uint32_t w[MB / 4];
+#pragma unroll
+            for (int i = 0; i < MB / 4; i++) w[i] = 0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const uint32_t m = code[i] & ((1u << MB) - 1u);
+                w[i * MB >> 5] |= m << (i * MB & 31);
+                if ((i * MB & 31) + MB > 32) w[(i * MB >> 5) + 1] |= m >> (32 - (i * MB & 31));
+            }
+            const size_t row = (size_t)bh * t_cap + t;
+            uint8_t *mp = p.main_plane + row * mrb + grp * MB;
+            if ((n & 7) == 0) {
+                if constexpr (MB == 16) *reinterpret_cast<uint4 *>(mp) = uint4{w[0], w[1], w[2], w[3]};
+                else if constexpr (MB == 12) {
+                    for (int i = 0; i < 3; i++) reinterpret_cast<uint32_t *>(mp)[i] = w[i];
+                } else *reinterpret_cast<uint2 *>(mp) = uint2{w[0], w[1]};
+            } else {
+#pragma unroll
+                for (int i = 0; i < MB; i++)
+                    if (left >= 8 || i < MB / 2) mp[i] = (uint8_t)(w[i >> 2] >> (8 * (i & 3)));
+            }
+            if (ab) {
+                uint64_t a = 0;
+#pragma unroll
+                for (int i = 0; i < 8; i++) a |= (uint64_t)((code[i] >> MB) & ((1u << ab) - 1u)) << (i * ab);
+                uint8_t *ap = p.aux_plane + row * arb + grp * ab;
+                const int bytes = left >= 8 ? ab : (4 * ab + 7) >> 3;
+                for (int i = 0; i < bytes; i++) ap[i] = (uint8_t)(a >> (8 * i));
+            }
+            if (grp == 0) {
+                ((ST *)p.scale_plane)[row] = scale;
+                const float f = fabsf(D::load(&scale));
+                if (f < __builtin_inff()) most = max(most, __float_as_uint(f));
+            }
+        }
+    if (D::code == HQMQ_F16 || !p.scale_max) return;
+    for (int o = 32; o; o >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, o));
+    if ((threadIdx.x & 63) == 0 && most > __hip_atomic_load(p.scale_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p.scale_max, most);
 }
 
 // one thread per output byte of the main plane, then of the aux plane
@@ -151,20 +277,57 @@ extern "C" int hqmq_dequant(const int32_t *idx, int64_t idx_sb, int64_t idx_sh, 
     if (!idx || !rq || !rs || !joint || !out) return HQMQ_ERR_NULL;
     if (B < 1 || H < 1 || T < 0 || n_chunks < 1 || K < 1 || qmax < 1) return HQMQ_ERR_SHAPE;
     if (T == 0) return HQMQ_OK;
-    const int64_t total = (int64_t)B * H * T * n_chunks;
-    dim3 grid(grid_for(total, 256)), block(256);
+    if ((int64_t)B * H > 0x7fffffff) return HQMQ_ERR_SHAPE;
+    // two chunks per thread where every row can be read and written that way
+    const bool pairs = dtype != HQMQ_F32 && (n_chunks & 1) == 0 && !((idx_sb | idx_sh | idx_st | rq_sb | rq_sh | rq_st) & 1) && !(joint_sh & 3) &&
+                       !(((uintptr_t)idx | (uintptr_t)rq | (uintptr_t)joint) & 7) && !((uintptr_t)out & 15);
+    const int64_t per_bh = ((int64_t)T * (n_chunks / (pairs ? 2 : 1)) + 255) / 256;
+    const dim3 grid((unsigned)std::min<int64_t>(per_bh, 1 << 20), (unsigned)std::min<int64_t>((int64_t)B * H, 65535)), block(256);
     hipStream_t st = (hipStream_t)stream;
-#define LAUNCH(DT, ST)                                                                                                   \
-    hipLaunchKernelGGL(dequant_kernel<DT>, grid, block, 0, st, idx, idx_sb, idx_sh, idx_st, rq, rq_sb, rq_sh, rq_st,      \
-                       (const ST *)rs, rs_sb, rs_sh, rs_st, (const ST *)joint, joint_sh, K, B, H, T, n_chunks, qmax, (ST *)out)
+#define LAUNCH(DT, ST, PER)                                                                                              \
+    hipLaunchKernelGGL((dequant_kernel<DT, PER>), grid, block, 0, st, idx, idx_sb, idx_sh, idx_st, rq, rq_sb, rq_sh, rq_st, \
+                       (const ST *)rs, rs_sb, rs_sh, rs_st, (const ST *)joint, joint_sh, K, B * H, H, T, n_chunks, qmax, (ST *)out)
     switch (dtype) {
-        case HQMQ_F32: LAUNCH(F32, float); break;
-        case HQMQ_F16: LAUNCH(F16, uint16_t); break;
-        case HQMQ_BF16: LAUNCH(BF16, uint16_t); break;
+        case HQMQ_F32: LAUNCH(F32, float, 1); break;
+        case HQMQ_F16: if (pairs) LAUNCH(F16, uint16_t, 2); else LAUNCH(F16, uint16_t, 1); break;
+        case HQMQ_BF16: if (pairs) LAUNCH(BF16, uint16_t, 2); else LAUNCH(BF16, uint16_t, 1); break;
         default: return HQMQ_ERR_DTYPE;
     }
 #undef LAUNCH
     return hip_status(hipGetLastError());
+}
+
+template <class D>
+static int launch_pack(const PackPair &p, const hqmq_pack_args *a, int mb, hipStream_t st) {
+    const int64_t items = (int64_t)a->t_cap * ((a->n_chunks + 7) / 8);
+    const dim3 grid((unsigned)((items + 255) / 256), (unsigned)std::min<int64_t>((int64_t)a->B * a->H, 65535), 2), block(256);
+    auto kern = mb == 16 ? pack_kv_kernel<D, 16> : mb == 12 ? pack_kv_kernel<D, 12> : pack_kv_kernel<D, 8>;
+    hipLaunchKernelGGL(kern, grid, block, 0, st, p, a->B * a->H, a->H, a->n_chunks, a->idx_bits, a->aux_bits, (int)a->t_cap);
+    return hip_status(hipGetLastError());
+}
+
+extern "C" int hqmq_pack_kv(const hqmq_pack_args *a, void *stream) {
+    if (!a) return HQMQ_ERR_NULL;
+    if (a->B < 1 || a->H < 1 || a->n_chunks < 4 || (a->n_chunks & 3) || a->t_cap < 1 || (int64_t)a->B * a->H > 0x7fffffff) return HQMQ_ERR_SHAPE;
+    if (a->t_cap * ((a->n_chunks + 7) / 8) > 0x7fffffff) return HQMQ_ERR_SHAPE;
+    if (a->idx_bits < 1 || a->idx_bits > 16 || a->aux_bits < 0 || a->aux_bits > 8) return HQMQ_ERR_LAYOUT;
+    if (a->main_bits != 8 && a->main_bits != 12 && a->main_bits != 16) return HQMQ_ERR_LAYOUT;
+    PackPair p;
+    for (int i = 0; i < 2; i++) {
+        const hqmq_pack_side &k = a->side[i];
+        if (k.T < 0 || k.T > a->t_cap) return HQMQ_ERR_SHAPE;
+        if ((k.T && (!k.idx || !k.rq || !k.scale_in)) || !k.main_plane || !k.scale_plane || (a->aux_bits && !k.aux_plane)) return HQMQ_ERR_NULL;
+        if ((uintptr_t)k.main_plane & 15) return HQMQ_ERR_ALIGN;
+        const int vec = !((k.idx_sb | k.idx_sh | k.idx_st | k.rq_sb | k.rq_sh | k.rq_st) & 3) && !(((uintptr_t)k.idx | (uintptr_t)k.rq) & 15);
+        p.s[i] = PackSide{k.idx, k.rq, k.idx_sb, k.idx_sh, k.idx_st, k.rq_sb, k.rq_sh, k.rq_st, k.scale_in, k.scale_sb, k.scale_sh, k.scale_st,
+                          k.main_plane, k.aux_plane, k.scale_plane, k.scale_max_bits, k.T, vec};
+    }
+    switch (a->dtype) {
+        case HQMQ_F32: return launch_pack<F32>(p, a, a->main_bits, (hipStream_t)stream);
+        case HQMQ_F16: return launch_pack<F16>(p, a, a->main_bits, (hipStream_t)stream);
+        case HQMQ_BF16: return launch_pack<BF16>(p, a, a->main_bits, (hipStream_t)stream);
+        default: return HQMQ_ERR_DTYPE;
+    }
 }
 
 extern "C" int hqmq_pack_codes(const int32_t *idx, int64_t idx_sb, int64_t idx_sh, int64_t idx_st, const int32_t *rq,

@@ -339,13 +339,9 @@ def dequant(idx, radius_q, radius_scale, joint, r_qmax: int) -> torch.Tensor:
     if joint.stride(-1) != 1 or joint.stride(1) != 4:
         joint = joint.contiguous()
     out = torch.empty(B, H, T, 4 * n, dtype=joint.dtype, device=idx.device)
-    with torch.cuda.device(idx.device):
-        L.check(L.lib().hqmq_dequant(
-            L.ptr(idx), L.i64(idx.stride(0)), L.i64(idx.stride(1)), L.i64(idx.stride(2)),
-            L.ptr(rq), L.i64(rq.stride(0)), L.i64(rq.stride(1)), L.i64(rq.stride(2)),
-            L.ptr(rs), L.i64(rs.stride(0)), L.i64(rs.stride(1)), L.i64(rs.stride(2)),
-            L.ptr(joint), L.i64(joint.stride(0)), C.c_int(joint.shape[1]), C.c_int(_dt(joint)), C.c_int(B), C.c_int(H),
-            C.c_int(T), C.c_int(n), C.c_int(r_qmax), L.ptr(out), L.stream_ptr(idx.device)), "hqmq_dequant")
+    si, sr, ss = idx.stride(), rq.stride(), rs.stride()
+    L.call(L.lib().hqmq_dequant, "hqmq_dequant", idx.device.index, idx.data_ptr(), si[0], si[1], si[2], rq.data_ptr(), sr[0], sr[1], sr[2],
+           rs.data_ptr(), ss[0], ss[1], ss[2], joint.data_ptr(), joint.stride(0), joint.shape[1], _dt(joint), B, H, T, n, r_qmax, out.data_ptr())
     return out
 
 
@@ -487,6 +483,114 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
     if skip_combine:
         return O, ws, n_splits
     return O
+
+
+_FUSED = {}
+
+
+def fused_unpacked(Q: torch.Tensor, k: tuple, v: tuple, r_qmax: int, *, kv_lens: Optional[torch.Tensor] = None, causal: bool = True,
+                   causal_offset: int = 0, softmax_scale: Optional[float] = None, n_splits: int = 0) -> torch.Tensor:
+    """Attention of Q over unpacked codes: k and v are (idx, radius_q, radius_scale, joint).  One launch packs both tensors into
+    planes of this call, then the packed attention runs over them."""
+    dt = Q.dtype
+    sides = []
+    for idx, rq, rs, joint in (k, v):
+        idx, rq = _i32(idx), _i32(rq)
+        if rq.shape != idx.shape:
+            raise L.HqmqError(f"radius codes {tuple(rq.shape)} and indices {tuple(idx.shape)} differ in shape")
+        if rs.dtype is not dt:
+            rs = rs.to(dt)
+        if rs.shape != idx.shape[:3]:
+            rs = rs.expand(idx.shape[:3])
+        if joint.stride(-1) != 1 or joint.stride(1) != 4:
+            joint = joint.contiguous()
+        sides.append((idx, rq, rs, joint))
+    (idx, _, _, joint), (idx_v, _, _, joint_v) = sides
+    if idx_v.shape[0] != idx.shape[0] or idx_v.shape[1] != idx.shape[1] or idx_v.shape[3] != idx.shape[3] or Q.shape[0] != idx.shape[0]:
+        raise L.HqmqError("K and V codes must have equal batch, head and chunk counts, Q the same batch")
+    if Q.stride(-1) != 1:
+        Q = Q.contiguous()
+    dev = idx.device
+    key = (Q.shape, Q.stride(), idx.shape, idx_v.shape[2], joint.shape[1], joint_v.shape[1], r_qmax, dt)
+    plan = _FUSED.get(key)
+    if plan is None:
+        if len(_FUSED) >= 256:                     # shapes that no longer come
+            _FUSED.clear()
+        plan = _FUSED[key] = _fused_plan(Q, idx, idx_v.shape[2], joint.shape[1], joint_v.shape[1], r_qmax)
+    pack_tmpl, attn_tmpl, offsets, nbytes, o_stride, per_split = plan
+    buf = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    base = buf.data_ptr()
+    most = None if dt is torch.float16 else torch.zeros(2, dtype=torch.int32, device=dev)
+    pack, a = L.PackArgs.from_buffer_copy(pack_tmpl), L.AttnArgs.from_buffer_copy(attn_tmpl)
+    for i, (t, (ix, rq, rs, jt)) in enumerate(zip((a.K, a.V), sides)):
+        p = pack.side[i]
+        p.idx, p.rq, p.scale_in = ix.data_ptr(), rq.data_ptr(), rs.data_ptr()
+        p.idx_sb, p.idx_sh, p.idx_st, _ = ix.stride()
+        p.rq_sb, p.rq_sh, p.rq_st, _ = rq.stride()
+        p.scale_sb, p.scale_sh, p.scale_st = rs.stride()
+        p.main_plane = t.main_plane = base + offsets[i]
+        p.scale_plane = t.scale_plane = base + offsets[2 + i]
+        if pack.aux_bits:
+            p.aux_plane = t.aux_plane = base + offsets[4 + i]
+        t.joint, t.joint_sh = jt.data_ptr(), jt.stride(0)
+        if most is not None:
+            p.scale_max_bits = t.scale_max_bits = most.data_ptr() + 4 * i
+    L.call(L.lib().hqmq_pack_kv, "hqmq_pack_kv", dev.index, C.addressof(pack))
+    if dt is torch.bfloat16 and not torch.cuda.is_current_stream_capturing():
+        # one device read: V scales outside [2^-8, 2^15) take the kernel that guards the fp16 range
+        top = float(most.cpu().view(torch.float32)[1])
+        a.wide_range = 1 if top >= 32768.0 or 0.0 < top < 2.0 ** -8 else 0
+    O = torch.empty_like(Q)
+    a.Q, a.O = Q.data_ptr(), O.data_ptr()
+    if softmax_scale is not None:
+        a.softmax_scale = softmax_scale
+    if kv_lens is not None:
+        kv_lens = kv_lens.to(device=dev, dtype=torch.int32).contiguous()
+        a.kv_len = kv_lens.data_ptr()
+    if causal:
+        a.causal, a.causal_offset = 1, causal_offset
+    a.n_splits = n_splits if n_splits > 0 else L.lib().hqmq_attn_splits(C.addressof(a))
+    if a.n_splits > 1:
+        ws = _workspace(per_split * a.n_splits, dev, "attn")
+        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel() * ws.element_size()
+    L.call(L.lib().hqmq_attn_fwd, "hqmq_attn_fwd", dev.index, C.addressof(a))
+    return O
+
+
+def _fused_plan(Q: torch.Tensor, idx: torch.Tensor, T_v: int, K: int, K_v: int, r_qmax: int):
+    """What the shapes fix of a fused_unpacked call: both argument blocks, where the planes lie in its buffer, the bytes of the
+    buffer, the output's strides, the workspace bytes per split."""
+    B, H, T, n = idx.shape
+    Hq, Tq = Q.shape[1], Q.shape[2]
+    radius_bits = max(1, int(r_qmax).bit_length())
+    if radius_bits > 8:
+        raise L.HqmqError(f"r_qmax={r_qmax} needs more than 8 radius bits")
+    # a table of K rows is addressed like one of ceil(K/24) secondaries; the radius field holds r_qmax
+    ib, mb, ab = L.layout_bits(max(1, -(-max(K, K_v) // 24)), radius_bits)
+    if mb == 12 and (n // 4) % 2:      # a lane's share of a 12-bit row must be whole bytes: use 16-bit codes
+        mb, ab = 16, max(0, ib + radius_bits - 16)
+    cap = (max(T, T_v, 1) + 63) // 64 * 64         # whole attention super-tiles
+    sizes = [cap * B * H * ((n * mb + 7) // 8)] * 2 + [cap * B * H * Q.element_size()] * 2 + [cap * B * H * ((n * ab + 7) // 8)] * 2
+    offsets, at = [], 0
+    for size in sizes:
+        offsets.append(at)
+        at += (size + 255) // 256 * 256
+    pack, a = L.PackArgs(), L.AttnArgs()
+    for p, t in zip(pack.side, (T, T_v)):
+        p.T = t
+    code = L.DT_CODE[Q.dtype]
+    pack.dtype, pack.B, pack.H, pack.n_chunks, pack.t_cap = code, B, H, n, cap
+    pack.idx_bits, pack.main_bits, pack.aux_bits = ib, mb, ab
+    a.q_sb, a.q_sh, a.q_st = Q.stride(0), Q.stride(1), Q.stride(2)
+    o_stride = torch.empty_like(Q).stride()
+    a.o_sb, a.o_sh, a.o_st = o_stride[0], o_stride[1], o_stride[2]
+    for t, rows in ((a.K, K), (a.V, K_v)):
+        t.scale_sb, t.scale_sh, t.scale_st, t.K = H * cap, cap, 1, rows
+    a.dtype, a.B, a.H_q, a.H_kv, a.T_q, a.T_kv, a.n_chunks, a.t_cap = code, B, Hq, H, Tq, T, n, cap
+    a.idx_bits, a.main_bits, a.aux_bits, a.qmax = ib, mb, ab, int(r_qmax)
+    a.softmax_scale = Q.shape[3] ** -0.5
+    per_split = int(L.lib().hqmq_attn_workspace_bytes(C.c_int(B), C.c_int(Hq), C.c_int(Tq), C.c_int(Q.shape[3]), C.c_int(2))) // 2
+    return pack, a, offsets, max(at, 256), o_stride, per_split
 
 
 def _attn_plan(Q: torch.Tensor, Kc, Vc, ks, vs):

@@ -210,6 +210,25 @@ int hqmq_pack_codes(const int32_t *idx, int64_t idx_sb, int64_t idx_sh, int64_t 
                     int B, int H, int T, int n_chunks, int idx_bits, int main_bits, int aux_bits,
                     uint8_t *main_plane, uint8_t *aux_plane, int64_t t_cap, void *stream);
 
+/* The same for K and V in one launch, scales included: rows [T, t_cap) of every plane are written as zeros (the planes need
+ * no clearing), and the largest finite scale is raised in *scale_max_bits as hqmq_quantize does.  idx and rq rows are
+ * contiguous; scale_in and the planes hold numbers of `dtype`; main_bits 8, 12 or 16, main planes 16-byte aligned,
+ * scale planes [B][H][t_cap].  No counterpart in the reference. */
+typedef struct hqmq_pack_side {
+    const int32_t *idx; int64_t idx_sb, idx_sh, idx_st;
+    const int32_t *rq; int64_t rq_sb, rq_sh, rq_st;
+    const void *scale_in; int64_t scale_sb, scale_sh, scale_st;
+    int T;
+    uint8_t *main_plane, *aux_plane; void *scale_plane;
+    uint32_t *scale_max_bits; /* may be NULL; not written for fp16 */
+} hqmq_pack_side;
+typedef struct hqmq_pack_args {
+    hqmq_pack_side side[2];
+    int dtype, B, H, n_chunks, idx_bits, main_bits, aux_bits;
+    int64_t t_cap;
+} hqmq_pack_args;
+int hqmq_pack_kv(const hqmq_pack_args *a, void *stream);
+
 /* One packed tensor (K or V) as the attention and dense-decode kernels read it. */
 typedef struct hqmq_packed {
     const uint8_t *main_plane, *aux_plane, *flag_plane; /* aux/flag may be NULL */

@@ -726,3 +726,28 @@ def test_prefill_tiles_shared_by_a_block(dn, S, b_r, d_h, Hq, Hkv, B, Tq, T, ns,
         if starts is not None:
             mask = mask & (kk >= as_t(starts).view(B, 1, 1, 1))
         assert_attention_close(O, *masked_two_refs(cache, Q, T, mask), base=2e-3, what=f"causal={causal}")
+
+
+@pytest.mark.parametrize("d_h,T,S,b_r,dn,odd", [
+    (16, 1, 24, 3, "fp16", False), (16, 65, 24, 3, "fp32", True), (80, 63, 96, 4, "fp16", False), (80, 130, 24, 3, "bf16", True),
+    (64, 64, 192, 6, "bf16", False), (128, 129, 96, 4, "fp16", True), (128, 33, 192, 6, "fp16", False), (256, 40, 24, 3, "bf16", False)])
+def test_unpacked_codes_at_odd_sizes(d_h, T, S, b_r, dn, odd):
+    """The packer of the unpacked entry point (groups of eight chunks, of four at the end of a row, every code width) and the dense
+    decode (one or two chunks per thread); odd: rows of codes that cannot be read as vectors."""
+    import hqmq
+    from hqmq_amd import ops
+    B, Hq, H, n, qmax, dt = 2, 6, 3, d_h // 4, (1 << b_r) - 1, DT[dn]
+    g = torch.Generator().manual_seed(d_h + T)
+    joint = torch.stack([CO.joint_table(TO.secondary_raw(1, H, S, 42)[0, :, kv], dt) for kv in (0, 1)])
+    codes = []
+    for kv in (0, 1):
+        wide = torch.randint(0, 24 * S, (B, H, T, n + 1), generator=g, dtype=torch.int32), torch.randint(0, qmax + 1, (B, H, T, n + 1), generator=g, dtype=torch.int32)
+        rs = (torch.rand(B, H, T, generator=g) + 0.5).to(dt)
+        codes.append(tuple(w[..., 1:] if odd else w[..., 1:].contiguous() for w in wide) + (rs, joint[kv]))
+    dev = [tuple(c.to(DEV) if not odd or c.dim() != 4 else torch.nn.functional.pad(c, (1, 0)).to(DEV)[..., 1:] for c in t) for t in codes]
+    Q = torch.randn(B, Hq, 5, d_h, generator=g).to(dt)
+    dense = [CO.dequant(*(x.contiguous() for x in t), qmax) for t in codes]
+    for t, want in zip(dev, dense):
+        assert bit_equal(ops.dequant(*t, qmax), want)
+    O = hqmq.fused_attention(Q.to(DEV), *dev[0], *dev[1], r_qmax=qmax, causal=False)
+    assert_close(O, CO.attention_dense(Q, dense[0], dense[1], causal=False), dt, 1e-3 if dn == "fp32" else 2e-3)
