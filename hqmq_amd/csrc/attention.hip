@@ -625,7 +625,7 @@ static int attn_fwd_impl(const hqmq_attn_args *a, void *stream) {
     int rc = HQMQ_OK;
     bool handled = false;
     if (p.scale_vec && attn_prefill_splits(a, n_splits) > 0) {
-        rc = launch_attn_prefill(p, a->main_bits, st, tm);
+        rc = launch_attn_prefill(p, a->main_bits, flags, st, tm);
         if (rc) return rc;
         handled = true;
     }

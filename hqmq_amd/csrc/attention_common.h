@@ -235,9 +235,9 @@ inline void launch_timed(Kern kern, dim3 grid, dim3 block, size_t shmem, hipStre
     else hipLaunchKernelGGL(kern, grid, block, shmem, st, p);
 }
 
-// Implemented in attention_prefill.hip: many query columns per KV head over plain 16-bit caches.
+// Implemented in attention_prefill.hip: many query columns per KV head over plain 16-bit and fp16 outlier caches.
 int attn_prefill_splits(const hqmq_attn_args *a, int splits);
-int launch_attn_prefill(const AttnParams &p, int main_bits, hipStream_t st, const LaunchTiming &tm);
+int launch_attn_prefill(const AttnParams &p, int main_bits, bool flags, hipStream_t st, const LaunchTiming &tm);
 int launch_attn_fast(const AttnParams &p, int main_bits, bool flags, dim3 grid, size_t table_bytes, hipStream_t st,
                      const LaunchTiming &tm, bool *handled);
 

@@ -1,4 +1,5 @@
-// Attention with many query columns per KV head (chunked and whole prefill) over plain 16-bit caches, d_h 64 / 128.
+// Attention with many query columns per KV head (chunked and whole prefill) over plain 16-bit caches and fp16 caches with verbatim
+// outliers, d_h 64 / 128.
 //
 // The decode kernels give a wavefront 16 or 32 columns and let it decode every KV tile for itself; with hundreds of
 // columns the same tile is decoded again and again.  Here a block of eight wavefronts decodes each tile of 64 tokens once
@@ -14,6 +15,10 @@
 //     the K reads (16 tokens) and the transposing V reads (4 tokens by 64 bytes) all meet 64 different banks;
 //   * K in LDS is codeword * radius code; the token's scale is applied to the score in fp32.  V is codeword * (radius code *
 //     scale / qmax), where the decode kernels put the scale into P: the same number of fp16 roundings, one less per score;
+//   * fp16 outlier caches (FL): K and V in LDS are the values themselves, multiplied out in fp32 and rounded once, and the wavefront
+//     that decoded a tile then writes the tile's verbatim chunks over the zeros that flagged chunks decode to.  They stay exact, and
+//     no sparse product is left (the decode kernels spend a third of their time on it).  bf16 caches keep the decode kernels: a
+//     verbatim bf16 chunk need not fit fp16;
 //   * one basic block per 32 tokens, written out one matrix instruction at a time: the scores of the next 32 tokens run with
 //     the exponentials of these, their products with V with the decoding of a later tile.  A matrix instruction takes 32
 //     cycles of its own pipe, a vector instruction about 4.3 of the shared issue slot (8.3 for an exponential), so that the
@@ -22,7 +27,8 @@
 //     registers that nothing copies (a copy would wait for them).
 // Measured, B = 1, 32 / 8 heads of 128, s96_r4, 1024 queries on 32768 tokens (541 GFLOP, 0.43 ms at the rate of a large matrix
 // product): 0.69 ms against 0.96 with the decode kernels' two-column-group variants; 4096 on 4096 tokens causal, s24_r3:
-// 0.19 against 0.41; four sequences of 300 on 300: 0.022 against 0.048.  What bounds it: a compute unit spends 36 % of the
+// 0.19 against 0.41; four sequences of 300 on 300: 0.022 against 0.048.  With 2 % of the K and V chunks verbatim: 1024 queries on
+// 32768 tokens 0.70 ms against 2.87, 300 on 8000 (28 / 4 heads, s192_r6) 0.10 against 0.32.  What bounds it: a compute unit spends 36 % of the
 // time in the matrix pipe, 50 % issuing vector instructions (a quarter of them decode) and 46 % in LDS, at 2.0 to 2.1 GHz.
 #include "attention_mfma.h"
 #include <algorithm>
@@ -44,7 +50,7 @@ __device__ __forceinline__ uint32_t pf_part(uint32_t t, uint32_t q) {
 
 #define PF_INLINE __attribute__((always_inline))
 
-template <int DH, int MB, bool AUX, int DT, int KVG>
+template <int DH, int MB, bool AUX, int DT, int KVG, bool FL>
 __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int gx, int rows) {
     constexpr int n = DH / 4, ROWB = DH * 2, CW = 8 / KVG, KS = DH / 16, DB = DH / 32;
     constexpr int TILE = 8192 / DH, NSUB = TILE / 32 / KVG;              // tokens per tile; units of 32 of them per wavefront
@@ -119,6 +125,42 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     const uint32_t idx_mask = (1u << p.idx_bits) - 1u;
     const int idx_bits = p.idx_bits;
     const uint32_t tab = kPfTab + (dec_v ? (uint32_t)((p.Kc.K * 8 + 127) & ~127) : 0u);
+    // Outlier caches (FL): a wavefront decodes whole 16-token tiles of the sideband (one at d_h 128, two at 64), so it also writes
+    // their verbatim chunks, over the zeros that flagged chunks decode to.  Lane e takes entry e of the contiguous range that the tile
+    // offsets name; the offsets (scalar loads) travel
+    // a tile ahead of the entries, the entries from the start of a tile's products to the end of its decoding.
+    constexpr int SBT = TOK / 16;
+    const int bh = b * p.Hkv + hkv, sb_tiles = (int)(p.t_cap >> 4);
+    const int32_t *sb_off = FL ? dc.sb_tile_off + (size_t)bh * sb_tiles : nullptr;
+    const uint2 *sb_val = FL ? (const uint2 *)dc.sideband + (size_t)bh * dc.sb_cap : nullptr;
+    const uint16_t *sb_xy = FL ? dc.sb_coord + (size_t)bh * dc.sb_cap : nullptr;
+    const int sb_count = FL ? min(max(uniform_word(dc.sb_count, bh), 0), (int)dc.sb_cap) : 0;
+    int rg[SBT + 1];                                                      // of the tile whose entries are requested next
+    auto offsets = [&](int t0) PF_INLINE {
+        const int first = (t0 >> 4) + (wave & 3) * SBT;
+#pragma unroll
+        for (int i = 0; i <= SBT; i++) {
+            const int o = uniform_word(sb_off, min(first + i, sb_tiles - 1));
+            rg[i] = first + i < sb_tiles ? o : 0x7fffffff;              // tiles never written hold that, too: up to the count
+        }
+    };
+    struct { uint2 val; uint32_t xy; int t0, from, mid, to; } ent;
+    auto entries = [&](int t0) PF_INLINE {
+        ent.t0 = t0;
+        ent.from = min(max(rg[0], 0), sb_count);
+        ent.to = max(ent.from, min(rg[SBT], sb_count));
+        ent.mid = rg[SBT - 1];
+        const int e = min(ent.from + lane, (int)dc.sb_cap - 1);
+        ent.val = sb_val[e];
+        ent.xy = sb_xy[e];
+        offsets(t0 + TILE);
+    };
+    // entry e into LDS; those of rows past the range are dropped (their scores are masked, but 0 * inf is not 0)
+    auto patch = [&](int e, uint2 val, uint32_t xy, uint32_t at) PF_INLINE {
+        const uint32_t t = (uint32_t)(wave & 3) * TOK + ((xy >> 8) & 15u) + (SBT > 1 && e >= ent.mid ? 16u : 0u), ch = xy & (uint32_t)(n - 1);
+        if (e < ent.to && ent.t0 + (int)t < b_end)
+            *(uint2v __attribute__((address_space(3))) *)(uintptr_t)(at + t * ROWB + (pf_part<DH>(t, ch >> 1) << 4) + (ch & 1u) * 8u) = __builtin_bit_cast(uint2v, val);
+    };
     struct Codes { uint32_t w[NW], aux, aux2, sh, scale; };
     auto request = [&](int t0, Codes &c) PF_INLINE {
         const uint32_t row = (uint32_t)min(t0 + d_tok, b_end - 1);        // rows past the range were perhaps never written
@@ -178,6 +220,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
             // K keeps its radius codes (the token's scale is applied to the score, in fp32); V takes radius * scale, rounded once
             if (j == 3) {
                 w_scale = DT == HQMQ_F16 ? __half2float(__ushort_as_half((uint16_t)c.scale)) : __uint_as_float(c.scale << 16);
+                if (FL) return;
                 const float f = dec_v ? w_scale * p.inv_qmax : 1.f;
 #pragma unroll
                 for (int i = 0; i < 4; i++)
@@ -186,10 +229,26 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
             }
         } else {
             const int i = j - 4;
-            *(uint4v __attribute__((address_space(3))) *)(uintptr_t)(w_at ^ ((uint32_t)i << 4)) =
+            if (FL) {                                                     // the value itself, rounded once, as the verbatim chunks are
+                const float f = w_scale * p.inv_qmax;
+                half8 v;
+#pragma unroll
+                for (int x = 0; x < 2; x++) {
+                    const float r = (float)wr[i][x] * f;
+#pragma unroll
+                    for (int y = 0; y < 4; y++) v[4 * x + y] = (_Float16)__builtin_fmaf((float)wg[2 * i + x][y], r, 0.f);
+                }
+                *(uint4v __attribute__((address_space(3))) *)(uintptr_t)(w_at ^ ((uint32_t)i << 4)) = __builtin_bit_cast(uint4v, v);
+            } else *(uint4v __attribute__((address_space(3))) *)(uintptr_t)(w_at ^ ((uint32_t)i << 4)) =
                 __builtin_bit_cast(uint4v, cat8(wg[2 * i] * wr[i][0], wg[2 * i + 1] * wr[i][1]));
+            if (FL && j == 7) {
+                asm volatile("" ::: "memory");                            // the wavefront's LDS writes keep their order
+                const uint32_t at = (w_at & kPfBuf) | (dec_v ? kPfV : 0u);
+                patch(ent.from + lane, ent.val, ent.xy, at);
+                for (int e = ent.from + 64 + lane; e < ent.to; e += 64) patch(e, sb_val[e], sb_xy[e], at);
+            }
             if (j == 7) {
-                if (w_lane) *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = w_scale * p.c_log2;
+                if (!FL && w_lane) *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = w_scale * p.c_log2;
                 w_at ^= kPfBuf;
                 ws_at ^= 512u;
             }
@@ -199,6 +258,10 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     // (in even steps from cc[0], in odd ones from cc[1], then the codes of the tile two further on are requested)
     Codes cc[2];
     if (work) {
+        if (FL) {
+            offsets(b_begin);
+            entries(b_begin);
+        }
         request(b_begin, cc[1]);
         request(b_begin + TILE, cc[0]);
     }
@@ -222,6 +285,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         for (int j = 0; j < 8; j++) piece(j, cc[1]);
         request(b_begin + 2 * TILE, cc[1]);
         if (!dec_v) {
+            if (FL) entries(b_begin + TILE);
 #pragma unroll
             for (int j = 0; j < 8; j++) piece(j, cc[0]);
             cc[0] = cc[1];
@@ -276,7 +340,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         const bool edge = !(tw + 32 <= wave_min && tw + 32 <= b_end && tw >= col_start);
         float tmax = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < 16; e++) s[e] = __builtin_fmaf(s[e], ks[e >> 2][e & 3], neg_m);
+        for (int e = 0; e < 16; e++) s[e] = __builtin_fmaf(s[e], FL ? p.c_plain : ks[e >> 2][e & 3], neg_m);
         if (edge) {
 #pragma unroll
             for (int e = 0; e < 16; e++) {
@@ -316,6 +380,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         float16v sn;
         float pe[2 * PER];
         uint32_t pp[8];
+        if (FL && u == 0) entries(d_t - 2 * TILE);                        // of the tile decoded next
 #pragma unroll
         for (int e = 0; e < 16; e++) sn[e] = 0.f;
         auto finish = [&](int k) PF_INLINE {                              // the exponentials of step k: summed, packed
@@ -351,7 +416,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
                     d_t += TILE;
                 }
             }
-            if (i == NV / 2) {
+            if (!FL && i == NV / 2) {
 #pragma unroll
                 for (int x = 0; x < 4; x++) ks[x] = s_load(buf, u + 1, x);
             }
@@ -373,7 +438,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     if (work) {
         float4v ks[4];
 #pragma unroll
-        for (int x = 0; x < 4; x++) ks[x] = s_load(0u, 0, x);
+        for (int x = 0; x < 4 && !FL; x++) ks[x] = s_load(0u, 0, x);
 #pragma unroll
         for (int e = 0; e < 16; e++) s[e] = 0.f;
 #pragma unroll
@@ -484,24 +549,31 @@ static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int ca
 }
 // Whether these kernels can take the call at all.
 static bool attn_prefill_takes(const hqmq_attn_args *a) {
-    if ((a->dtype != HQMQ_F16 && a->dtype != HQMQ_BF16) || a->wide_range || a->K.flag_plane || (a->n_chunks != 16 && a->n_chunks != 32) ||
+    if ((a->dtype != HQMQ_F16 && a->dtype != HQMQ_BF16) || a->wide_range || (a->n_chunks != 16 && a->n_chunks != 32) ||
         a->fp8_table_storage || (a->force_generic && a->force_generic != 3) || a->softmax_scale <= 0.f)
         return false;
     if (a->main_bits != 16 && (a->main_bits != 12 || a->aux_bits < 1)) return false;
     if (a->idx_bits < 6 || a->aux_bits > 4) return false;                          // the 16-bit decode needs radius codes below 1024
     if (a->t_cap % 64 || a->t_cap >= (1 << 25)) return false;                      // rows are addressed by 32-bit offsets
     if (kPfTab + ((size_t)a->K.K + a->V.K) * 8 + 128 > 160 * 1024) return false;
+    if (a->K.flag_plane || a->V.flag_plane) {
+        if (a->dtype != HQMQ_F16) return false;                                   // verbatim bf16 chunks need not fit fp16
+        const hqmq_packed *kv[2] = {&a->K, &a->V};
+        for (const hqmq_packed *t : kv)
+            if (!t->flag_plane || !t->sideband || !t->sb_coord || !t->sb_count || !t->sb_tile_off || t->sb_cap < 1 || t->sb_cap >= (1 << 28) || ((uintptr_t)t->sideband & 7))
+                return false;
+    }
     if (a->aux_bits && (((uintptr_t)a->K.aux_plane | (uintptr_t)a->V.aux_plane) & 3)) return false;
     if ((((uintptr_t)a->O) | (uintptr_t)(a->o_sb * 2) | (uintptr_t)(a->o_sh * 2) | (uintptr_t)(a->o_st * 2)) & 7) return false;
     return true;
 }
 // The same for the kernels of attention_fast.hip: blocks of 16 columns (0.47 us a tile) or, where that leaves a block per
-// compute unit, of 32 (0.6 us), which start and finish in 6 us.
-static double fast_us(int64_t cols, int64_t nz, int Tkv, int d_h, int splits) {
+// compute unit, of 32 (0.6 us), over outlier caches always of 16 (0.7 us), which start and finish in 6 us.
+static double fast_us(int64_t cols, int64_t nz, int Tkv, int d_h, int splits, bool flags) {
     const int64_t cg = (cols + 15) / 16, pairs = (cg + 1) / 2 * nz * splits;
-    const bool two = cg > 1 && pairs >= 256;
+    const bool two = !flags && cg > 1 && pairs >= 256;
     const double tiles = ((double)Tkv * d_h + 8191) / 8192;
-    return 3.0 + (double)(((two ? pairs : cg * nz * splits) + 255) / 256) * (6.0 + tiles / splits * (two ? 0.6 : 0.47)) +
+    return 3.0 + (double)(((two ? pairs : cg * nz * splits) + 255) / 256) * (6.0 + tiles / splits * (two ? 0.6 : flags ? 0.7 : 0.47)) +
            (splits > 1 ? 3.0 + (double)(cols * nz) * splits * (d_h + 4) * 8 / 2e6 : 0.0);
 }
 // The number of splits of a call that leaves it open, 0 if it is better off with the other kernels (by a clear margin: the
@@ -511,10 +583,14 @@ int attn_prefill_splits(const hqmq_attn_args *a, int splits) {
     if (cols < 64 || !attn_prefill_takes(a)) return 0;
     const PfPlan plan = pf_plan(cols, nz, a->T_q, a->T_kv, 4 * a->n_chunks, a->causal, a->causal_offset, splits);
     const int other = splits > 0 ? splits : hqmq_attn_pick_splits(a->B, a->H_q, a->H_kv, a->T_q, a->T_kv, a->kv_len != nullptr);
-    return a->force_generic == 3 || plan.us < 0.85 * fast_us(cols, nz, a->T_kv, 4 * a->n_chunks, other) ? plan.splits : 0;
+    // Outlier caches of three radius bits: most radius codes are 1, 2 or 4, with which the decode kernels' codeword * radius code is
+    // exact, and a value rounded once is up to 16 % further from 64-bit results (s24_r3, lognormal channels; s96 and s192 are 5 %
+    // nearer on average): they keep those kernels.
+    if (a->K.flag_plane && a->qmax < 15 && a->force_generic != 3) return 0;
+    return a->force_generic == 3 || plan.us < 0.85 * fast_us(cols, nz, a->T_kv, 4 * a->n_chunks, other, a->K.flag_plane != nullptr) ? plan.splits : 0;
 }
 
-template <int DH, int MB, bool AUX, int DT>
+template <int DH, int MB, bool AUX, int DT, bool FL>
 static int launch_pf(const AttnParams &p, hipStream_t st, const LaunchTiming &tm) {
     const int64_t cols = (int64_t)p.Tq * p.G, nz = (int64_t)p.B * p.Hkv * p.n_splits;
     const bool wide = pf_plan(cols, (int64_t)p.B * p.Hkv, p.Tq, p.Tkv, DH, p.causal, p.causal_offset, p.n_splits).wide;
@@ -531,7 +607,7 @@ static int launch_pf(const AttnParams &p, hipStream_t st, const LaunchTiming &tm
     }
     if (rows * nz > 0x7fffffff) return HQMQ_ERR_SHAPE;
     const size_t shmem = kPfTab + (size_t)((p.Kc.K * 8 + 127) & ~127) + (size_t)p.Vc.K * 8;
-    auto kern = wide ? attn_prefill_kernel<DH, MB, AUX, DT, 1> : attn_prefill_kernel<DH, MB, AUX, DT, 2>;
+    auto kern = wide ? attn_prefill_kernel<DH, MB, AUX, DT, 1, FL> : attn_prefill_kernel<DH, MB, AUX, DT, 2, FL>;
     const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     if (e != hipSuccess) return (int)e;
     const dim3 grid((unsigned)(rows * nz));
@@ -540,15 +616,19 @@ static int launch_pf(const AttnParams &p, hipStream_t st, const LaunchTiming &tm
     return hip_status(hipGetLastError());
 }
 
-template <int DH, int DT>
+template <int DH, int DT, bool FL>
 static int launch_pf_layout(const AttnParams &p, int mb, hipStream_t st, const LaunchTiming &tm) {
-    if (mb == 16 && p.aux_bits == 0) return launch_pf<DH, 16, false, DT>(p, st, tm);
-    return mb == 16 ? launch_pf<DH, 16, true, DT>(p, st, tm) : launch_pf<DH, 12, true, DT>(p, st, tm);
+    if (mb == 16 && p.aux_bits == 0) return launch_pf<DH, 16, false, DT, FL>(p, st, tm);
+    return mb == 16 ? launch_pf<DH, 16, true, DT, FL>(p, st, tm) : launch_pf<DH, 12, true, DT, FL>(p, st, tm);
+}
+template <int DH>
+static int launch_pf_type(const AttnParams &p, int mb, bool flags, hipStream_t st, const LaunchTiming &tm) {
+    if (flags) return launch_pf_layout<DH, HQMQ_F16, true>(p, mb, st, tm);
+    return p.dtype == HQMQ_F16 ? launch_pf_layout<DH, HQMQ_F16, false>(p, mb, st, tm) : launch_pf_layout<DH, HQMQ_BF16, false>(p, mb, st, tm);
 }
 
-int launch_attn_prefill(const AttnParams &p, int mb, hipStream_t st, const LaunchTiming &tm) {
-    if (p.n == 32) return p.dtype == HQMQ_F16 ? launch_pf_layout<128, HQMQ_F16>(p, mb, st, tm) : launch_pf_layout<128, HQMQ_BF16>(p, mb, st, tm);
-    return p.dtype == HQMQ_F16 ? launch_pf_layout<64, HQMQ_F16>(p, mb, st, tm) : launch_pf_layout<64, HQMQ_BF16>(p, mb, st, tm);
+int launch_attn_prefill(const AttnParams &p, int mb, bool flags, hipStream_t st, const LaunchTiming &tm) {
+    return p.n == 32 ? launch_pf_type<128>(p, mb, flags, st, tm) : launch_pf_type<64>(p, mb, flags, st, tm);
 }
 
 }  // namespace hqmq

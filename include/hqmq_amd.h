@@ -305,7 +305,7 @@ int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, int n_splits
 /* The n_splits hqmq_attn_fwd would choose; ragged = 1 when kv_len is passed (more, smaller blocks). */
 int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv, int ragged);
 /* The n_splits that suits these arguments best (a->n_splits is not looked at), for callers that size the workspace by it:
-   chunked prefill over plain caches wants other counts than hqmq_attn_pick_splits names from the shapes alone. */
+   chunked prefill wants other counts than hqmq_attn_pick_splits names from the shapes alone. */
 int hqmq_attn_splits(const hqmq_attn_args *a);
 int hqmq_attn_fwd(const hqmq_attn_args *a, void *stream);
 /* Merge of the split-KV partials (m, l, acc) left in the workspace; hqmq_attn_fwd runs it unless skip_combine. */

@@ -728,6 +728,55 @@ def test_prefill_tiles_shared_by_a_block(dn, S, b_r, d_h, Hq, Hkv, B, Tq, T, ns,
         assert_attention_close(O, *masked_two_refs(cache, Q, T, mask), base=2e-3, what=f"causal={causal}")
 
 
+@pytest.mark.parametrize("S,b_r,d_h,Hq,Hkv,B,Tq,T,ns,lens,starts,share", [
+    (96, 4, 128, 4, 1, 1, 32, 32, 0, None, None, 0.05),             # half a tile
+    (96, 4, 128, 4, 1, 1, 33, 65, 1, None, None, 0.3),              # more than 64 entries in a 16-token tile
+    (24, 3, 128, 8, 8, 1, 255, 300, 3, None, None, 0.05),           # 12 + 1 bits, cache ends inside a tile of the sideband
+    (192, 6, 128, 8, 2, 2, 64, 641, 0, [641, 3], [70, 0], 0.02),    # 16 + 3 bits, limits on both sides
+    (192, 4, 64, 8, 1, 3, 97, 190, 2, [190, 0, 64], None, 0.3),     # 16 + 1 bits at d_h 64, an empty sequence
+    (24, 3, 64, 16, 8, 1, 130, 130, 1, None, [129], 0.05),
+    (96, 4, 64, 32, 8, 8, 520, 520, 1, None, None, 0.01),           # blocks of 256 columns
+    (192, 4, 128, 32, 8, 4, 1030, 1100, 1, [1100, 1, 64, 1037], None, 0.02)])
+def test_prefill_tiles_with_verbatim_chunks(S, b_r, d_h, Hq, Hkv, B, Tq, T, ns, lens, starts, share):
+    """The same kernel over fp16 outlier caches (verbatim chunks written over the decoded tile): against dense attention, and no
+    verbatim chunk behind a sequence's end reaches the output, infinite ones included."""
+    import hqmq
+    dt = torch.float16
+    g = torch.Generator().manual_seed(T + 3 * Tq)
+    kv = []
+    for _ in range(2):
+        x = torch.randn(B, Hkv, T, d_h // 4, 4, generator=g)
+        x = torch.where(torch.rand(B, Hkv, T, d_h // 4, 1, generator=g) < share, x * 40.0, x).reshape(B, Hkv, T, d_h)
+        kv.append(x.to(dt))
+    w = hqmq.with_outlier_extraction(hqmq.HQMQ(n_layers=1, n_heads=Hkv, secondary_size=S, radius_bits=b_r, device=DEV), C=3.0)
+    cache = w.new_cache(B, T, d_h, dt, 0, sideband_frac=0.5)
+    w.append(cache, kv[0].to(DEV), kv[1].to(DEV), 0)
+    cache.K.check_overflow()
+    Q = (torch.randn(B, Hq, Tq, d_h, generator=g) * 0.3).to(dt).to(DEV)
+    as_t = lambda a: None if a is None else torch.tensor(a, dtype=torch.int32, device=DEV)
+    kk, qq = torch.arange(T, device=DEV).view(1, 1, 1, T), torch.arange(Tq, device=DEV).view(1, 1, Tq, 1)
+    for causal in (True, False):
+        off = T - Tq
+        O = hqmq.fused_attention_packed(Q, cache, causal=causal, causal_offset=off if causal else 0, n_splits=ns, kv_lens=as_t(lens),
+                                        kv_starts=as_t(starts), T_kv=T, force_generic=3)
+        mask = (kk <= qq + off) if causal else torch.ones(1, 1, Tq, T, dtype=torch.bool, device=DEV)
+        mask = mask.expand(B, 1, Tq, T)
+        if lens is not None:
+            mask = mask & (kk < as_t(lens).view(B, 1, 1, 1))
+        if starts is not None:
+            mask = mask & (kk >= as_t(starts).view(B, 1, 1, 1))
+        assert_attention_close(O, *masked_two_refs(cache, Q, T, mask), base=2e-3, what=f"causal={causal}")
+    if lens is None:
+        return
+    for b, n in enumerate(lens):
+        for h in range(Hkv):
+            tile = (n + 15) // 16
+            if tile < cache.V.sb_tile_off.shape[2]:
+                cache.V.sideband[b, h, int(cache.V.sb_tile_off[b, h, tile]):] = float("inf")
+    again = hqmq.fused_attention_packed(Q, cache, causal=False, n_splits=ns, kv_lens=as_t(lens), kv_starts=as_t(starts), T_kv=T, force_generic=3)
+    assert torch.equal(again, O)
+
+
 @pytest.mark.parametrize("d_h,T,S,b_r,dn,odd", [
     (16, 1, 24, 3, "fp16", False), (16, 65, 24, 3, "fp32", True), (80, 63, 96, 4, "fp16", False), (80, 130, 24, 3, "bf16", True),
     (64, 64, 192, 6, "bf16", False), (128, 129, 96, 4, "fp16", True), (128, 33, 192, 6, "fp16", False), (256, 40, 24, 3, "bf16", False)])
