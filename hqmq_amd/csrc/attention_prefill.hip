@@ -13,8 +13,9 @@
 //     reads (ds_read_b64_tr_b16) per 32 x 16 operand;
 //   * LDS rows are stored with their 16-byte parts permuted by the token, so that the writes (16 tokens at the same part),
 //     the K reads (16 tokens) and the transposing V reads (4 tokens by 64 bytes) all meet 64 different banks;
-//   * K in LDS is codeword * radius code; the token's scale is applied to the score in fp32.  V is codeword * (radius code *
-//     scale / qmax), where the decode kernels put the scale into P: the same number of fp16 roundings, one less per score;
+//   * K and V in LDS are codeword * radius code; K's scale of the token is applied to the score and V's to P, in fp32, as the decode
+//     kernels do (V times radius * scale / qmax in LDS saves 16 multiplications per 32 tokens, but rounds once more: 4 to 8 % further
+//     from 64-bit results at fp16);
 //   * fp16 outlier caches (FL): K and V in LDS are the values themselves, multiplied out in fp32 and rounded once, and the wavefront
 //     that decoded a tile then writes the tile's verbatim chunks over the zeros that flagged chunks decode to.  They stay exact, and
 //     no sparse product is left (the decode kernels spend a third of their time on it).  bf16 caches keep the decode kernels: a
@@ -39,7 +40,7 @@ typedef float float16v __attribute__((ext_vector_type(16)));
 typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kPfV = 16384, kPfBuf = 32768, kPfScale = 2 * kPfBuf, kPfTab = kPfScale + 2048;   // LDS: K | V, twice; scales; tables
+constexpr uint32_t kPfV = 16384, kPfBuf = 32768, kPfScale = 2 * kPfBuf, kPfScaleV = 1024, kPfTab = kPfScale + 2048;   // LDS: K | V, twice; scales; tables
 
 // permutation of a row's 16-byte parts
 template <int DH>
@@ -186,8 +187,8 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     half2v wr[4];
     float w_scale = 0.f;
     uint32_t w_at = (dec_v ? kPfV : 0u) + (uint32_t)d_tok * ROWB + (pf_part<DH>((uint32_t)d_tok, (uint32_t)(d_grp * 4)) << 4);
-    uint32_t ws_at = kPfScale + 4u * (uint32_t)d_tok;
-    const bool w_lane = !dec_v && d_grp == 0;
+    uint32_t ws_at = kPfScale + (dec_v ? kPfScaleV : 0u) + 4u * (uint32_t)d_tok;
+    const bool w_lane = d_grp == 0;
     auto piece = [&](int j, Codes &c) PF_INLINE {
         if (j == 0) {
 #pragma unroll
@@ -217,15 +218,9 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
                     wr[i] = __builtin_bit_cast(half2v, t) - half2v{(_Float16)1024.0f, (_Float16)1024.0f};
                 }
             }
-            // K keeps its radius codes (the token's scale is applied to the score, in fp32); V takes radius * scale, rounded once
+            // K and V keep their radius codes; the token's scales are applied to the score and to P, in fp32
             if (j == 3) {
                 w_scale = DT == HQMQ_F16 ? __half2float(__ushort_as_half((uint16_t)c.scale)) : __uint_as_float(c.scale << 16);
-                if (FL) return;
-                const float f = dec_v ? w_scale * p.inv_qmax : 1.f;
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-#pragma unroll
-                    for (int x = 0; x < 2; x++) wr[i][x] = (_Float16)__builtin_fmaf((float)wr[i][x], f, 0.f);
             }
         } else {
             const int i = j - 4;
@@ -248,7 +243,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
                 for (int e = ent.from + 64 + lane; e < ent.to; e += 64) patch(e, sb_val[e], sb_xy[e], at);
             }
             if (j == 7) {
-                if (!FL && w_lane) *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = w_scale * p.c_log2;
+                if (!FL && w_lane) *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = dec_v ? w_scale : w_scale * p.c_log2;
                 w_at ^= kPfBuf;
                 ws_at ^= 512u;
             }
@@ -335,6 +330,10 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         const uint32_t at = ((u == NSUB ? buf ^ 1u : buf) * 512u + 128u * (uint32_t)(u % NSUB) + 32u * i) / 16;
         return __builtin_bit_cast(float4v, ((lds_u4_ptr)(uintptr_t)sa)[at]);
     };
+    auto vs_load = [&](uint32_t buf, int u, int i) PF_INLINE {            // V scales of the same tokens
+        const uint32_t at = (kPfScaleV + buf * 512u + 128u * (uint32_t)u + 32u * i) / 16;
+        return __builtin_bit_cast(float4v, ((lds_u4_ptr)(uintptr_t)sa)[at]);
+    };
     // scores of a unit (first token tw): times their K scale, relative to the running maximum, which moves if it has to
     auto maxima = [&](int tw, const float4v (&ks)[4]) PF_INLINE {
         const bool edge = !(tw + 32 <= wave_min && tw + 32 <= b_end && tw >= col_start);
@@ -376,19 +375,21 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         constexpr int NV = 2 * DB, PER = 8 / KS;               // pairs of exponentials per matrix instruction
         const bool dec = u == NSUB - 1;
         half8 vf[AHEAD];
-        float4v ks[4];
+        float4v ks[4], vs[4];
         float16v sn;
         float pe[2 * PER];
         uint32_t pp[8];
         if (FL && u == 0) entries(d_t - 2 * TILE);                        // of the tile decoded next
 #pragma unroll
         for (int e = 0; e < 16; e++) sn[e] = 0.f;
-        auto finish = [&](int k) PF_INLINE {                              // the exponentials of step k: summed, packed
+        if (!FL) vs[0] = vs_load(buf, u, 0);
+        auto finish = [&](int k) PF_INLINE {                              // the exponentials of step k: summed, times V's scale, packed
 #pragma unroll
             for (int x = 0; x < PER; x++) {
                 const int i = k * PER + x;
                 l_run += pe[2 * x] + pe[2 * x + 1];
-                pp[i] = __builtin_bit_cast(uint32_t, half2v{(_Float16)pe[2 * x], (_Float16)pe[2 * x + 1]});
+                const float v0 = FL ? 1.f : vs[i >> 1][2 * i & 3], v1 = FL ? 1.f : vs[i >> 1][(2 * i & 3) + 1];
+                pp[i] = __builtin_bit_cast(uint32_t, half2v{(_Float16)(FL ? pe[2 * x] : pe[2 * x] * v0), (_Float16)(FL ? pe[2 * x + 1] : pe[2 * x + 1] * v1)});
             }
         };
 #pragma unroll
@@ -398,6 +399,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
             if (k + AHEAD < KS) kf[k % AHEAD] = k_load(buf, u + 1, k + AHEAD);
             else vf[k + AHEAD - KS] = v_load(buf, u, k + AHEAD - KS);
             if (k > 0) finish(k - 1);
+            if (!FL && (2 * PER * (k + 1)) % 4 == 0 && k + 1 < KS) vs[PER * (k + 1) / 2] = vs_load(buf, u, PER * (k + 1) / 2);
 #pragma unroll
             for (int x = 0; x < 2 * PER; x++) pe[x] = __builtin_amdgcn_exp2f(s[2 * PER * k + x]);
         }
@@ -489,7 +491,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     }
     if (!col_ok || (KVG == 2 && kvg == 1)) {
     } else if (p.n_splits == 1) {
-        const float f = l_run > 0.f ? 1.f / l_run : 0.f;
+        const float f = l_run > 0.f ? (FL ? 1.f : p.inv_qmax) / l_run : 0.f;
         uint16_t *o = (uint16_t *)p.O + b * p.osb + hq * p.osh + (int64_t)tq * p.ost + 4 * half;
 #pragma unroll
         for (int db = 0; db < DB; db++)
@@ -512,7 +514,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
             for (int i = 0; i < 4; i++) {
                 float4v v;
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = acc[db][4 * i + j];
+                for (int j = 0; j < 4; j++) v[j] = FL ? acc[db][4 * i + j] : acc[db][4 * i + j] * p.inv_qmax;
                 *reinterpret_cast<float4v *>(wp + kPartialHead + 32 * db + 8 * i + 4 * half) = v;
             }
     }
