@@ -27,7 +27,7 @@
 //   * two tile buffers, one barrier per tile (two with KVG = 1).  The codes of a tile are requested two tiles ahead into
 //     registers that nothing copies (a copy would wait for them).
 // Measured, B = 1, 32 / 8 heads of 128, s96_r4, 1024 queries on 32768 tokens (541 GFLOP, 0.43 ms at the rate of a large matrix
-// product): 0.69 ms against 0.96 with the decode kernels' two-column-group variants; 4096 on 4096 tokens causal, s24_r3:
+// product): 0.68 ms against 0.96 with the decode kernels' two-column-group variants; 4096 on 4096 tokens causal, s24_r3:
 // 0.19 against 0.41; four sequences of 300 on 300: 0.022 against 0.048.  With 2 % of the K and V chunks verbatim: 1024 queries on
 // 32768 tokens 0.70 ms against 2.87, 300 on 8000 (28 / 4 heads, s192_r6) 0.10 against 0.32.  What bounds it: a compute unit spends 36 % of the
 // time in the matrix pipe, 50 % issuing vector instructions (a quarter of them decode) and 46 % in LDS, at 2.0 to 2.1 GHz.
