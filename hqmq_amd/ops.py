@@ -123,6 +123,7 @@ def quantize(x: torch.Tensor, joint: torch.Tensor, slack: Optional[torch.Tensor]
 
 _WS = {}
 _WS_MOST = 256
+_WS_CAPTURED = {}          # buffers that a captured graph writes to at every replay: kept when a larger one takes their place
 
 # torch.quantile refuses more than 2^24 elements along the reduced dimension ("quantile() input tensor is too large"),
 # which bounds the chunks per head of one Med-C call of the reference (src/quantizers/outlier_aware.py:68).  The
@@ -149,6 +150,8 @@ def _workspace(nbytes: int, device, tag: str) -> torch.Tensor:
             _WS.clear()
         buf = torch.empty(max(nbytes, 1 << 16), dtype=torch.uint8, device=device)
         _WS[key] = buf
+    if torch.cuda.is_current_stream_capturing():
+        _WS_CAPTURED[buf.data_ptr()] = buf
     return buf
 
 

@@ -77,3 +77,34 @@ def test_graph_replays_equal_eager_steps(med3x, dn, S, b_r):
                 x, y = getattr(a, name), getattr(b, name)
                 if x is not None:
                     assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), f"replay {i}: {name}"
+
+
+def test_graph_keeps_its_workspace_when_a_larger_one_takes_its_place():
+    """The split partials' buffer of a captured call stays allocated when a later call on the stream needs a larger one and the
+    memory is handed out again."""
+    import hqmq
+    from hqmq_amd import ops
+    q = hqmq.HQMQ(n_layers=1, n_heads=2, secondary_size=96, radius_bits=4, device=DEV)
+    cache = q.new_cache(1, 4096, 128, torch.float16, 0)
+    q.append(cache, kv_input((1, 2, 4096, 128), torch.float16, 1).to(DEV), kv_input((1, 2, 4096, 128), torch.float16, 2).to(DEV), 0)
+    Q = torch.randn(1, 8, 1, 128, generator=torch.Generator().manual_seed(3)).half().to(DEV)
+    out = torch.empty_like(Q)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        side.wait_stream(torch.cuda.default_stream())
+        want = hqmq.fused_attention_packed(Q, cache, n_splits=8).clone()              # the buffer is there before the capture
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            hqmq.fused_attention_packed(Q, cache, n_splits=8, out=out)
+        key = ("attn", Q.device.index, side.cuda_stream)
+        small = ops._WS[key].numel()
+        many = torch.randn(1, 8, 64, 128, generator=torch.Generator().manual_seed(4)).half().to(DEV)
+        hqmq.fused_attention_packed(many, cache, n_splits=16)
+        assert ops._WS[key].numel() > small
+        other = torch.full((small,), 7, dtype=torch.uint8, device=DEV)                # would be the old buffer, were it free
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            side.synchronize()
+            assert torch.equal(out, want) and bool((other == 7).all())
