@@ -291,7 +291,7 @@ def _append_args(x, cache, joint, slack, radius_bits, t_off, pos, median_mult, t
     B, H, T, d_h = x.shape
     med = median_mult is not None and T > 0
     tmpl = cache._append_template
-    if tmpl is None or tmpl[0] is not joint or tmpl[1] is not slack or tmpl[2] != (joint.data_ptr(), radius_bits, d_h, med):
+    if tmpl is None or tmpl[0] is not joint or tmpl[1] is not slack or tmpl[2] != (joint.data_ptr(), cache.main.data_ptr(), radius_bits, d_h, med):
         if d_h % 4 != 0:
             raise ValueError(f"d_head={d_h} not divisible by 4")
         _check_joint(x, joint)
@@ -307,7 +307,7 @@ def _append_args(x, cache, joint, slack, radius_bits, t_off, pos, median_mult, t
             a.sideband, a.sb_cap = L.addr(cache.sideband), cache.sb_cap
             a.sb_tile_off, a.sb_count = L.addr(cache.sb_tile_off), L.addr(cache.sb_count)
             a.overflow, a.sb_coord = L.addr(cache.sb_overflow), L.addr(cache.sb_coord)
-        tmpl = cache._append_template = (joint, slack, (joint.data_ptr(), radius_bits, d_h, med), a, grid)
+        tmpl = cache._append_template = (joint, slack, (joint.data_ptr(), cache.main.data_ptr(), radius_bits, d_h, med), a, grid)
     elif joint.dtype != x.dtype or joint.shape[0] != H:
         _check_joint(x, joint)
     a = L.AppendArgs.from_buffer_copy(tmpl[3])

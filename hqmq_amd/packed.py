@@ -33,7 +33,7 @@ class RangeWatch:
 
     def fetch(self) -> None:
         if self.host is None:
-            self.host = torch.empty(self.device_values.numel(), dtype=torch.int32, pin_memory=True)
+            self.host = torch.zeros(self.device_values.numel(), dtype=torch.int32, pin_memory=True)      # 0: nothing written yet
             self.event = torch.cuda.Event()
         self.host.copy_(self.device_values, non_blocking=True)
         self.event.record()
@@ -128,7 +128,10 @@ class PackedTensor:
         """V scales of a bf16 / fp32 cache outside [2^-8, 2^15).  Waits for the last bulk append if the value behind it has
         not been looked at yet (under stream capture, which begins with everything done, it is read as it stands)."""
         if self._range_due:
-            self._take_range(self._watch.read(self._slot, wait=not torch.cuda.is_current_stream_capturing()))
+            capturing = torch.cuda.is_current_stream_capturing()
+            value = self._watch.read(self._slot, wait=not capturing)
+            self._take_range(value)
+            self._range_due = capturing                # looked at without waiting: due again afterwards
         return self._wide
 
     @wide_range.setter
