@@ -440,7 +440,7 @@ __device__ __forceinline__ void grid_body(const QParams &a) {
             }
             const uint32_t next = e.w >> 16;
             if (__builtin_amdgcn_ballot_w64(next != 0u) == 0ull) break;
-            if (next == 0xffffu) brute = active && ordinary;
+            if (next == 0xffffu) brute |= active && ordinary;           // (a direction that is not ordinary keeps its own reason)
             e = lists[kCells + (next == 0xffffu ? 0u : next)];
         }
         const uint32_t at = D::code == HQMQ_F32 ? best_at : (uint32_t)key & 0xffffu;

@@ -44,3 +44,37 @@ def test_cell_lists_pick_what_the_scan_picks(S, crowded, dn):
                 assert bit_equal(a["out"], other["out"]) and bit_equal(a["r_max"], other["r_max"]), (T, d_h)
     want = CO.quantize(x, CO.joint_table(raw, dt), 4)
     assert torch.equal(a["idx"].cpu(), want["idx"]) and torch.equal(a["rq"].cpu(), want["rq"]) and bit_equal(a["out"], want["out"])
+
+
+@pytest.mark.parametrize("dn", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("S", [192, 341])
+def test_unordinary_chunks_in_boxes_without_a_list(S, dn):
+    """Directions that do not have length 1 (norm below the clamp, 16-bit subnormal, infinite, NaN) score all rows, also where
+    their box carries no list: codebooks crowded round the units leave the boxes at the cell's centre without one."""
+    import hqmq
+    from hqmq_amd import ops
+    dt = DT[dn]
+    if S == 192:
+        raw = hqmq.HQMQ(n_layers=1, n_heads=2, secondary_size=S, init="hurwitz_perturbed", device="cpu").secondary_raw.detach()[0, :, 0]
+    else:
+        raw = _raw(S, True, torch.Generator().manual_seed(S))
+    J, slack = ops.build_joint(raw.to(DEV), dt)
+    units = hqmq.HQMQ(n_layers=1, n_heads=2, device="cpu")._primary.float()
+    x = torch.randn(1, 2, 96, 128, generator=torch.Generator().manual_seed(S + 1))
+    gains = (1e-9, 3e-9, 4e-9, 6e-8, 1.2e-7, 1e-30, float("inf"), float("nan"))
+    for i, gain in enumerate(gains):
+        rows = x[:, :, 8 * i:8 * i + 6]
+        rows[..., :96] = (units * gain).nan_to_num(nan=float("nan") if gain != gain else 0.0, posinf=float("inf"), neginf=float("-inf")).reshape(-1)
+        rows[..., 96:] = (torch.tensor([[1.2, 0.6, 0, 0]] * 8) * (gain if gain < 1 else 1e-7)).reshape(-1)      # subnormal ratios: between two units
+    x = x.to(dt)
+    want = CO.quantize(x, CO.joint_table(raw, dt), 4)
+    assert not (want["idx"] == 24 * S - 1).all()
+    for t in (96, 8, 1):                    # a block's copy of the table, a block of four wavefronts, one wavefront
+        for t0 in range(0, 96, t if t > 1 else 8):
+            part = x[:, :, t0:t0 + t].to(DEV)
+            got = ops.quantize(part, J, slack, 4, want_dense=True)
+            scan = ops.quantize(part, J, slack, 4, want_dense=True, algo=1)
+            ref = {k: want[k][:, :, t0:t0 + t] for k in ("idx", "rq", "r_max", "out")}
+            assert torch.equal(scan["idx"].cpu(), ref["idx"]), (t, t0)
+            assert torch.equal(got["idx"].cpu(), ref["idx"]) and torch.equal(got["rq"].cpu(), ref["rq"]), (t, t0)
+            assert bit_equal(got["out"], ref["out"]) and bit_equal(got["r_max"], ref["r_max"]), (t, t0)
