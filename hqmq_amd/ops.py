@@ -261,6 +261,8 @@ def crop(caches, lengths) -> None:
     if isinstance(lengths, int):
         a.length = max(0, min(lengths, c.t_cap))
     else:
+        if lengths.numel() != c.B or lengths.dtype is not torch.int32 or lengths.device != c.flags.device or not lengths.is_contiguous():
+            raise L.HqmqError(f"lengths must be {c.B} contiguous int32 on the caches' device")       # the kernel reads all B of them
         a.lengths = lengths.data_ptr()
     L.call(L.lib().hqmq_crop, "hqmq_crop", c.device.index, C.addressof(a))
 

@@ -197,7 +197,7 @@ class PackedTensor:
         return True
 
     def crop_(self, lengths) -> None:
-        """Forgets the rows from `lengths` on (an int for all sequences or an int tensor [B]): the outlier list and
+        """Forgets the rows from `lengths` on (an int for all sequences or an int tensor of B entries): the outlier list and
         its tile offsets go back to the state after the last kept row, so that the rows can be appended again.
         The planes themselves are left as they are (later appends overwrite them)."""
         _crop([self], lengths)
@@ -259,7 +259,10 @@ def _crop(tensors, lengths) -> None:
         for t in tensors:
             t.length = min(t.length, lengths)
     else:
-        lengths = lengths.to(device=tensors[0].device).clamp(min=0).to(torch.int32).contiguous()
+        for t in tensors:
+            if lengths.numel() != t.B:
+                raise L.HqmqError(f"crop_ needs one length per sequence ({t.B}), got {tuple(lengths.shape)}")
+        lengths = lengths.reshape(-1).to(device=tensors[0].device).clamp(min=0).to(torch.int32).contiguous()
         for t in tensors:
             t.lengths = lengths
     flagged = [t for t in tensors if t.flags is not None]

@@ -249,6 +249,22 @@ def test_crop_bookkeeping_on_cpu():
     assert pt.length == 20 and np.array_equal(pt.sb_count.numpy(), cnt3) and np.array_equal(pt.sb_tile_off.numpy(), off3)
 
 
+@pytest.mark.parametrize("outliers", [False, True])
+def test_crop_refuses_lengths_that_do_not_match_the_batch(outliers):
+    """One length per sequence: the GPU kernel reads B of them from the tensor's address.  Nothing changes in a refused call."""
+    from hqmq_amd.packed import PackedKV, PackedTensor
+    make = lambda: PackedTensor(3, 2, 150, 64, 96, 4, torch.float16, "cpu", outliers=outliers)
+    cache = PackedKV(make(), make())
+    cache.K.length = cache.V.length = 150
+    for bad in (torch.tensor([5]), torch.tensor(5), torch.tensor([5, 6]), torch.tensor([5, 6, 7, 8]), torch.zeros(0, dtype=torch.int64)):
+        for obj in (cache, cache.K):
+            with pytest.raises(RuntimeError, match="one length per sequence"):
+                obj.crop_(bad)
+    assert cache.K.lengths is None and cache.length == 150
+    cache.crop_(torch.tensor([[5], [6], [7]]))
+    assert cache.K.lengths.tolist() == cache.V.lengths.tolist() == [5, 6, 7]
+
+
 def test_quantile_limit_check():
     """The reference's Med-C median is torch.quantile, which refuses more than 2^24 elements per row
     (src/quantizers/outlier_aware.py:68 of the reference); the check that mirrors it on request."""
