@@ -264,7 +264,7 @@ def crop(caches, lengths) -> None:
         if lengths.numel() != c.B or lengths.dtype is not torch.int32 or lengths.device != c.flags.device or not lengths.is_contiguous():
             raise L.HqmqError(f"lengths must be {c.B} contiguous int32 on the caches' device")       # the kernel reads all B of them
         a.lengths = lengths.data_ptr()
-    L.call(L.lib().hqmq_crop, "hqmq_crop", c.device.index, C.addressof(a))
+    L.call(L.lib().hqmq_crop, "hqmq_crop", c.flags.device.index, C.addressof(a))
 
 
 def append_kv(k: torch.Tensor, v: torch.Tensor, k_cache, v_cache, k_joint, k_slack, v_joint, v_slack, radius_bits: int, *,

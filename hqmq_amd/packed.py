@@ -262,22 +262,20 @@ def _crop(tensors, lengths) -> None:
         for t in tensors:
             if lengths.numel() != t.B:
                 raise L.HqmqError(f"crop_ needs one length per sequence ({t.B}), got {tuple(lengths.shape)}")
-        lengths = lengths.reshape(-1).to(device=tensors[0].device).clamp(min=0).to(torch.int32).contiguous()
+        lengths = lengths.reshape(-1).to(device=tensors[0].main.device).clamp(min=0).to(torch.int32).contiguous()
         for t in tensors:
-            t.lengths = lengths
+            t.lengths = lengths.to(t.main.device)
     flagged = [t for t in tensors if t.flags is not None]
     if not flagged:
         return
-    if flagged[0].device.type != "cuda":
+    if not flagged[0].flags.is_cuda:
         for t in flagged:
             _crop_outliers_torch(t, lengths)
         return
     from . import ops
-    if len(flagged) == 2 and any(getattr(flagged[0], k) != getattr(flagged[1], k) for k in ("B", "H", "t_cap", "n", "device")):
-        for t in flagged:
-            ops.crop([t], lengths)
-    else:
-        ops.crop(flagged, lengths)
+    shared = len({(t.B, t.H, t.t_cap, t.n, t.flags.device) for t in flagged}) == 1
+    for group in [flagged] if shared else [[t] for t in flagged]:
+        ops.crop(group, lengths if isinstance(lengths, int) else group[0].lengths)
 
 
 @dataclass

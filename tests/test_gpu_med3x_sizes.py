@@ -80,3 +80,18 @@ def test_append_lists_and_crop(dn, d_h, T):
     check([min(5, c) for c in cut.tolist()])
     cache.crop_(0)
     check([0, 0])
+
+
+def test_crop_of_a_cache_made_for_cuda_without_an_index():
+    """device="cuda" names no GPU index: the call goes to the device the planes are on.  Lengths on the host are accepted, K and V
+    of different capacity are cropped one after the other."""
+    from hqmq_amd.packed import PackedKV, PackedTensor
+    K, V = (PackedTensor(2, 1, cap, 64, 24, 3, torch.float16, "cuda", outliers=True) for cap in (128, 192))
+    for t in (K, V):
+        t.flags.fill_(1)                # two flagged chunks in every row
+        t.sb_tile_off.copy_(32 * torch.arange(t.t_cap // 16, dtype=torch.int32).expand(2, 1, -1))
+        t.sb_count.fill_(2 * t.t_cap)
+    PackedKV(K, V).crop_(torch.tensor([40, 128]))
+    assert K.sb_count.flatten().tolist() == [2 * 40, 2 * 128] and V.sb_count.flatten().tolist() == [2 * 40, 2 * 128]
+    K.crop_(16)
+    assert K.sb_count.flatten().tolist() == [2 * 16, 2 * 16] and not bool(K.flags[:, :, 16:].any())
