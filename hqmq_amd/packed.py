@@ -7,6 +7,7 @@ Plane layout: include/hqmq_amd.h.
 """
 from __future__ import annotations
 
+import threading
 from dataclasses import dataclass
 from typing import Optional
 
@@ -24,24 +25,53 @@ def _round_up(x: int, m: int) -> int:
 
 class RangeWatch:
     """The largest finite scales the quantize kernels have written, as fp32 bits, one slot per tensor that shares the watch,
-    and their way to the host: a copy into pinned memory behind the append that may have changed them, waited for only when
-    the value is looked at."""
+    and their way to the host: a copy into pinned memory behind every append that may have changed them, waited for only when
+    the value is looked at.  Every copy has a buffer and an event of its own, recorded on the stream of the append, so that
+    appends on several streams or threads, and on another device than the current one, are all waited for."""
+
+    _SPARE_MOST, _PENDING_MOST = 4, 64      # buffers kept for the next copies; copies nobody has looked at
 
     def __init__(self, device, slots: int = 1):
         self.device_values = torch.zeros(slots, dtype=torch.int32, device=device)
-        self.host = self.event = None
+        self.issued = 0                     # copies sent so far
+        self._most = [0.0] * slots          # largest values seen on the host; 0: nothing written yet
+        self._pending, self._spare = {}, []          # by number: (buffer, event)
+        self._lock = threading.Lock()
 
     def fetch(self) -> None:
-        if self.host is None:
-            self.host = torch.zeros(self.device_values.numel(), dtype=torch.int32, pin_memory=True)      # 0: nothing written yet
-            self.event = torch.cuda.Event()
-        self.host.copy_(self.device_values, non_blocking=True)
-        self.event.record()
+        """Sends the values to the host behind the work of the current stream of their device."""
+        with self._lock:
+            host, event = self._spare.pop() if self._spare else (None, None)
+        if host is None:
+            host = torch.zeros(self.device_values.numel(), dtype=torch.int32, pin_memory=self.device_values.is_cuda)
+            event = torch.cuda.Event()
+        host.copy_(self.device_values, non_blocking=True)            # on that stream, whichever device is current
+        event.record(torch.cuda.current_stream(self.device_values.device))
+        with self._lock:
+            self.issued += 1
+            self._pending[self.issued] = host, event
+            oldest = next(iter(self._pending)) if len(self._pending) > self._PENDING_MOST else None
+        if oldest is not None:
+            self._take(oldest, wait=True)
 
-    def read(self, slot: int, wait: bool) -> float:
+    def read(self, slot: int, wait: bool):
+        """The largest value of a slot over all copies sent so far, waiting for them or as they stand, and their number."""
+        with self._lock:
+            issued, pending = self.issued, tuple(self._pending)
+        for number in pending:
+            self._take(number, wait)
+        return self._most[slot], issued
+
+    def _take(self, number: int, wait: bool) -> None:
+        entry = self._pending.get(number)
+        if entry is None:                                            # another thread has looked at it
+            return
         if wait:
-            self.event.synchronize()
-        return float(self.host.view(torch.float32)[slot])
+            entry[1].synchronize()
+        with self._lock:
+            self._most = [max(m, v) for m, v in zip(self._most, entry[0].view(torch.float32).tolist())]
+            if wait and self._pending.pop(number, None) is not None and len(self._spare) < self._SPARE_MOST:
+                self._spare.append(entry)
 
 
 class PackedTensor:
@@ -75,7 +105,8 @@ class PackedTensor:
         # host-side copy of "scale_max lies outside [2^-8, 2^15)": such a cache takes the layout-generic attention kernel, which
         # guards the fp16 range (refresh_range reads the device value; due after bulk appends and every
         # RANGE_CHECK_EVERY small ones, done when the flag is next looked at)
-        self._wide = self._huge = self._range_due = False
+        self._wide = self._huge = False
+        self._range_seen = 0                 # copies of the watch that the flag takes account of
         self._appends_since_range_check = 0
         self.length = 0                      # rows written when all sequences advance together
         self.lengths: Optional[torch.Tensor] = None  # per-sequence rows (int32, device) for ragged batches
@@ -125,18 +156,22 @@ class PackedTensor:
 
     @property
     def wide_range(self) -> bool:
-        """V scales of a bf16 / fp32 cache outside [2^-8, 2^15).  Waits for the last bulk append if the value behind it has
-        not been looked at yet (under stream capture, which begins with everything done, it is read as it stands)."""
-        if self._range_due:
+        """V scales of a bf16 / fp32 cache outside [2^-8, 2^15).  Waits for the bulk appends whose values have not been
+        looked at yet (under stream capture, which begins with everything done, it is read as it stands)."""
+        watch = self._watch
+        if watch is not None and self._range_seen != watch.issued:
             capturing = torch.cuda.is_current_stream_capturing()
-            value = self._watch.read(self._slot, wait=not capturing)
+            value, issued = watch.read(self._slot, wait=not capturing)
             self._take_range(value)
-            self._range_due = capturing                # looked at without waiting: due again afterwards
+            if not capturing:                          # looked at without waiting: due again afterwards
+                self._range_seen = issued
         return self._wide
 
     @wide_range.setter
     def wide_range(self, value: bool) -> None:
-        self._wide, self._range_due = bool(value), False
+        self._wide = bool(value)
+        if self._watch is not None:
+            self._range_seen = self._watch.issued
 
     def c_struct(self) -> L.Packed:
         """The tensors as the library takes them; the same object until one of them is replaced."""
@@ -168,14 +203,16 @@ class PackedTensor:
         normal range.  The largest scale only grows: a cache of tiny values leaves the flag again when larger ones
         arrive; a cache beyond 2^15 keeps it."""
         if self.scale_max is not None and not self._huge:
-            self._take_range(float(self.scale_max.view(torch.float32).item()))
+            v = float(self.scale_max.view(torch.float32).item())
+            if self.scale_max is self._watch_view:          # and what appends on other streams have sent
+                v = max(v, self._watch.read(self._slot, wait=True)[0])
+            self._take_range(v)
         self._appends_since_range_check = 0
         return self._wide
 
     def _take_range(self, v: float) -> None:
         self._huge = self._huge or v >= 32768.0
         self._wide = self._huge or 0.0 < v < 2.0 ** -8
-        self._range_due = False
 
     def note_append(self, rows: int, fetch: bool = True) -> bool:
         """Called by the quantizer after an append of `rows` rows per sequence: after bulk appends (a prefill) and every
@@ -191,7 +228,6 @@ class PackedTensor:
             self.refresh_range()
             return False
         self._appends_since_range_check = 0
-        self._range_due = True
         if fetch:
             self._watch.fetch()
         return True

@@ -265,6 +265,44 @@ def test_crop_refuses_lengths_that_do_not_match_the_batch(outliers):
     assert cache.K.lengths.tolist() == cache.V.lengths.tolist() == [5, 6, 7]
 
 
+def test_range_watch_waits_for_every_stream_that_sent_a_value(monkeypatch):
+    """Every copy of the largest scales has an event of its own, recorded on the current stream of the values' device (not of the
+    current device), and a look at the value waits for all of them; under stream capture it waits for none and stays due."""
+    from hqmq_amd import packed
+    log, streams, capturing = [], ["first", "second"], [False]
+
+    class Event:
+        def record(self, stream):
+            self.stream = stream
+
+        def synchronize(self):              # the copy arrives
+            log.append(self.stream)
+            for host, event in list(watch._pending.values()):
+                if event is self:
+                    host.copy_(torch.tensor(arriving[self.stream], dtype=torch.float32).view(torch.int32))
+
+    monkeypatch.setattr(packed.torch.cuda, "Event", Event)
+    monkeypatch.setattr(packed.torch.cuda, "current_stream", lambda device=None: (str(device), streams[0]))
+    monkeypatch.setattr(packed.torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    arriving = {("cpu", "first"): [1.0, 40000.0], ("cpu", "second"): [2.0, 3.0]}
+    watch = packed.RangeWatch(torch.device("cpu"), 2)
+    K, V = (packed.PackedTensor(1, 1, 64, 64, 24, 3, torch.bfloat16, "cpu", watch=(watch, i)) for i in (0, 1))
+    for _ in range(2):
+        assert K.note_append(100, fetch=False) and V.note_append(100, fetch=False)
+        watch.fetch()
+        streams.reverse()
+    capturing[0] = True
+    assert not V.wide_range and log == []
+    capturing[0] = False
+    assert V.wide_range and sorted(log) == sorted(arriving)      # 40000 came on the first stream, the second one's event is later
+    assert not K.wide_range and len(log) == 2
+    V.wide_range = False
+    assert not V.wide_range
+    for _ in range(200):
+        watch.fetch()
+    assert len(watch._pending) <= 64 and len(watch._spare) <= 4 and V.wide_range
+
+
 def test_quantile_limit_check():
     """The reference's Med-C median is torch.quantile, which refuses more than 2^24 elements per row
     (src/quantizers/outlier_aware.py:68 of the reference); the check that mirrors it on request."""

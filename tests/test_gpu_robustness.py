@@ -234,3 +234,27 @@ def test_outlier_kernels_with_huge_k_and_ordinary_v_stay_on_the_fast_path():
         O = hqmq.fused_attention_packed(Q, cache, force_generic=generic)
         assert torch.isfinite(O.float()).all()
         assert_attention_close(O, *refs, base=2e-3 * max(1.0, float(refs[0].abs().max())), what=f"generic={generic}")
+
+
+def test_range_of_appends_on_two_streams():
+    """A bulk append whose V scales leave [2^-8, 2^15) is still running on one stream when an ordinary one on another stream is
+    done: the first look at the range waits for both."""
+    import hqmq
+    dt = torch.bfloat16
+    q = hqmq.HQMQ(n_layers=1, n_heads=2, secondary_size=96, radius_bits=4, device=DEV)
+    cache = q.new_cache(1, 512, 128, dt, 0)
+    x = kv_input((1, 2, 128, 128), dt, 5).to(DEV)
+    big = (x.float() * 1e6).to(dt)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(20_000_000)               # some 10 ms
+        q.append(cache, x, big, 0)
+    with torch.cuda.stream(second):
+        q.append(cache, x, x, 0)
+        second.synchronize()
+        assert cache.V.wide_range and not cache.K.wide_range
+    torch.cuda.synchronize()
+    assert cache.length == 256
+    Q = torch.randn(1, 8, 1, 128, generator=torch.Generator().manual_seed(6)).to(dt).to(DEV)
+    assert torch.isfinite(hqmq.fused_attention_packed(Q, cache).float()).all()
