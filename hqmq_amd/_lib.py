@@ -153,6 +153,18 @@ def check(status: int, what: str) -> None:
         raise HqmqError(f"{what} failed: status {status} ({msg})")
 
 
+class Kept:
+    """Argument blocks worked out from an object's tensors and kept with it.  They hold addresses: a copy or a pickle of the
+    object starts without them (None)."""
+    __slots__ = ("value",)
+
+    def __init__(self, value=None):
+        self.value = value
+
+    def __reduce__(self):
+        return Kept, ()
+
+
 def ptr(t):
     """Device (or host) address of a tensor, NULL for None."""
     return vp(t.data_ptr()) if t is not None else vp(0)

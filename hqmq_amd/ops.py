@@ -42,7 +42,7 @@ def build_joint(raw_hs4: torch.Tensor, dtype: torch.dtype):
 def _book(joint: torch.Tensor, slack: Optional[torch.Tensor], radius_bits: int, n: int):
     """A QuantizeArgs with everything a codebook fixes, kept with `slack` from call to call, and the address of the cell
     lists."""
-    book = getattr(slack, "hqmq_book", None)
+    book = getattr(getattr(slack, "hqmq_book", None), "value", None)
     if book is not None and book[0] is joint and book[1] == joint.data_ptr() and book[2] == (radius_bits, n):
         return book[3], book[4]
     a = L.QuantizeArgs()
@@ -51,7 +51,7 @@ def _book(joint: torch.Tensor, slack: Optional[torch.Tensor], radius_bits: int, 
     a.secondary_size, a.radius_bits = joint.shape[1] // 24, radius_bits
     grid = L.addr(getattr(slack, "hqmq_grid", None))
     if slack is not None:
-        slack.hqmq_book = (joint, joint.data_ptr(), (radius_bits, n), a, grid)
+        slack.hqmq_book = L.Kept((joint, joint.data_ptr(), (radius_bits, n), a, grid))
     return a, grid
 
 

@@ -38,6 +38,14 @@ class RangeWatch:
         self._pending, self._spare = {}, []          # by number: (buffer, event)
         self._lock = threading.Lock()
 
+    def __getstate__(self):
+        """Copies and pickles take the values along, waited for; buffers, events and the lock are this object's own."""
+        self.read(0, wait=not (self.device_values.is_cuda and torch.cuda.is_current_stream_capturing()))
+        return {"device_values": self.device_values, "issued": self.issued, "_most": list(self._most)}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state, _pending={}, _spare=[], _lock=threading.Lock())
+
     def fetch(self) -> None:
         """Sends the values to the host behind the work of the current stream of their device."""
         with self._lock:
@@ -153,6 +161,21 @@ class PackedTensor:
             d = self.__dict__
             d["_struct"] = d["_append_template"] = None
             d["_attn_plans"] = {}
+
+    def __getstate__(self):
+        """What a copy or a pickle takes along: the tensors and the state, no argument blocks (they hold addresses)."""
+        state = dict(self.__dict__)
+        for name in ("_struct", "_append_template", "_attn_plans", "_fp8_view"):
+            state.pop(name, None)
+        if state.pop("_watch_view") is self.scale_max:          # a part of the watch's tensor, there as here
+            del state["scale_max"]
+        return state
+
+    def __setstate__(self, state):
+        d = self.__dict__
+        d.update(state, _struct=None, _append_template=None, _attn_plans={})
+        d["_watch_view"] = None if self._watch is None else self._watch.device_values[self._slot:self._slot + 1]
+        d.setdefault("scale_max", d["_watch_view"])
 
     @property
     def wide_range(self) -> bool:

@@ -43,6 +43,13 @@ class KVQuantizer(ABC):
         return type(self).__name__
 
 
+class _Codebooks(dict):
+    """Tables by (layer, K or V, type).  They belong to one parameter: a deep copy or a pickle of the quantizer builds its own."""
+
+    def __reduce__(self):
+        return _Codebooks, ()
+
+
 class HQMQQuantizer(KVQuantizer):
     """Hurwitz quaternion multiplicative quantizer (direction = q_p * q_s, per-token max radius scale)."""
 
@@ -71,7 +78,7 @@ class HQMQQuantizer(KVQuantizer):
         else:
             raise ValueError(init)
         self.secondary_raw = nn.Parameter(raw.to(device=device, dtype=torch.float32))
-        self._joint_cache: dict = {}
+        self._joint_cache = _Codebooks()
 
     # ---- hooks the reference's calibration glue looks for ----
     def trainable_parameters(self):

@@ -303,6 +303,47 @@ def test_range_watch_waits_for_every_stream_that_sent_a_value(monkeypatch):
     assert len(watch._pending) <= 64 and len(watch._spare) <= 4 and V.wide_range
 
 
+@pytest.mark.parametrize("how", ["deepcopy", "pickle"])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_used_caches_and_quantizers_can_be_copied(dt, how):
+    """The argument blocks a used object keeps hold addresses: a copy goes without them and works out its own.  The K and V of a
+    copy share one range watch, and its slots are their scale_max, as in the original."""
+    import copy
+    import pickle
+    import hqmq
+    from hqmq_amd import _lib as L
+    from hqmq_amd.packed import PackedKV, PackedTensor, RangeWatch
+    twin = copy.deepcopy if how == "deepcopy" else lambda x: pickle.loads(pickle.dumps(x))
+    watch = None if dt == torch.float16 else RangeWatch(torch.device("cpu"), 2)
+    joint = torch.randn(2, 24 * 24, 4).to(dt)
+    mk = lambda i: PackedTensor(1, 2, 100, 64, 24, 3, dt, "cpu", joint=joint, outliers=True, watch=watch and (watch, i))
+    cache = PackedKV(mk(0), mk(1))
+    cache.K.main.random_(0, 256)
+    cache.K.length = 100
+    old = cache.K.c_struct()
+    cache.K._append_template = (joint, L.AppendArgs())
+    cache.K._attn_plans["shape"] = (old, L.AttnArgs())
+    other = twin(cache)
+    assert torch.equal(other.K.main, cache.K.main) and other.length == 100
+    assert other.K.c_struct().main_plane == other.K.main.data_ptr() != old.main_plane
+    assert other.K._append_template is None and not other.K._attn_plans
+    assert cache.K.c_struct() is old and cache.K._append_template is not None
+    if watch is not None:
+        assert other.K._watch is other.V._watch is not watch
+        other.V.scale_max.fill_(7)
+        assert other.K._watch.device_values.tolist() == [0, 7] and watch.device_values.tolist() == [0, 0]
+        assert other.V.c_struct().scale_max_bits == other.V.scale_max.data_ptr() and other.V.scale_max is other.V._watch_view
+    view = cache.K.with_fp8_table()
+    assert view.main is cache.K.main and view.c_struct().joint == view.joint.data_ptr() != joint.data_ptr()
+    q = hqmq.with_outlier_extraction(hqmq.HQMQ(n_layers=1, n_heads=2, device="cpu"))
+    slack = torch.zeros(2)
+    slack.hqmq_grid, slack.hqmq_book = torch.zeros(4), L.Kept((joint, L.QuantizeArgs()))
+    q.inner._joint_cache[0, 0, dt] = ((), joint, slack)
+    assert not twin(q).inner._joint_cache and q.inner._joint_cache
+    assert torch.equal(twin(q).inner.secondary_raw, q.inner.secondary_raw)
+    assert twin(slack).hqmq_book.value is None and torch.equal(twin(slack).hqmq_grid, slack.hqmq_grid)
+
+
 def test_quantile_limit_check():
     """The reference's Med-C median is torch.quantile, which refuses more than 2^24 elements per row
     (src/quantizers/outlier_aware.py:68 of the reference); the check that mirrors it on request."""

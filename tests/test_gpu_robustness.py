@@ -258,3 +258,35 @@ def test_range_of_appends_on_two_streams():
     assert cache.length == 256
     Q = torch.randn(1, 8, 1, 128, generator=torch.Generator().manual_seed(6)).to(dt).to(DEV)
     assert torch.isfinite(hqmq.fused_attention_packed(Q, cache).float()).all()
+
+
+@pytest.mark.parametrize("how", ["deepcopy", "pickle"])
+@pytest.mark.parametrize("dn,med3x", [("fp16", False), ("bf16", True)])
+def test_a_copy_of_a_used_cache_goes_on_by_itself(dn, med3x, how):
+    """One prompt's cache copied for several continuations, with its quantizer: the copy gives the original's results, appends of
+    either leave the other as it is, and the bf16 range flag comes along."""
+    import copy
+    import pickle
+    import hqmq
+    from tests.helpers import DT
+    twin = copy.deepcopy if how == "deepcopy" else lambda x: pickle.loads(pickle.dumps(x))
+    dt = DT[dn]
+    q = hqmq.HQMQ(n_layers=1, n_heads=2, secondary_size=96, radius_bits=4, device=DEV)
+    w = hqmq.with_outlier_extraction(q, C=3.0) if med3x else q
+    cache = w.new_cache(1, 400, 128, dt, 0)
+    k, v = kv_input((1, 2, 302, 128), dt, 11, outlier_p=0.02).to(DEV), kv_input((1, 2, 302, 128), dt, 12).to(DEV)
+    Q = (0.01 * torch.randn(1, 8, 1, 128, generator=torch.Generator().manual_seed(13))).to(dt).to(DEV)      # every token counts
+    w.append(cache, k[:, :, :300], v[:, :, :300], 0)
+    base = hqmq.fused_attention_packed(Q, cache)
+    hqmq.fused_attention_packed(Q, cache, use_fp8_codebook=True)
+    other, w2 = twin(cache), twin(w)
+    assert torch.equal(hqmq.fused_attention_packed(Q, other), base) and other.length == 300
+    w2.append(other, k[:, :, 300:301], v[:, :, 300:301], 0)
+    longer = hqmq.fused_attention_packed(Q, other)
+    assert torch.equal(hqmq.fused_attention_packed(Q, cache), base) and not torch.equal(longer, base)
+    w.append(cache, k[:, :, 300:301], v[:, :, 300:301], 0)
+    assert torch.equal(hqmq.fused_attention_packed(Q, cache), longer)
+    if dn == "bf16":
+        big = (v.float() * 1e7).to(dt)
+        w2.append(other, k[:, :, :64], big[:, :, :64], 0)
+        assert twin(other).V.wide_range and other.V.wide_range and not cache.V.wide_range
