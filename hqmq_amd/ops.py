@@ -123,7 +123,6 @@ def quantize(x: torch.Tensor, joint: torch.Tensor, slack: Optional[torch.Tensor]
 
 _WS = {}
 _WS_MOST = 256
-_WS_CAPTURED = {}          # buffers that a captured graph writes to at every replay: kept when a larger one takes their place
 
 # torch.quantile refuses more than 2^24 elements along the reduced dimension ("quantile() input tensor is too large"),
 # which bounds the chunks per head of one Med-C call of the reference (src/quantizers/outlier_aware.py:68).  The
@@ -141,7 +140,11 @@ def check_quantile_limit(chunks_per_head: int, strict: bool) -> bool:
 
 
 def _workspace(nbytes: int, device, tag: str) -> torch.Tensor:
-    """A cached scratch buffer of at least nbytes (grown on demand, reused across calls on the same stream; any content)."""
+    """A cached scratch buffer of at least nbytes (grown on demand, reused across calls on the same stream; any content).
+    Under stream capture a buffer of the call's own: torch takes it from the graph's memory, which later calls of the capture
+    use again in stream order, no call outside it does, and the graph gives back when it goes."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
     index = device.index
     key = (tag, index, L.raw_stream(index))                          # calls on different streams may overlap
     buf = _WS.get(key)
@@ -150,8 +153,6 @@ def _workspace(nbytes: int, device, tag: str) -> torch.Tensor:
             _WS.clear()
         buf = torch.empty(max(nbytes, 1 << 16), dtype=torch.uint8, device=device)
         _WS[key] = buf
-    if torch.cuda.is_current_stream_capturing():
-        _WS_CAPTURED[buf.data_ptr()] = buf
     return buf
 
 
@@ -280,15 +281,16 @@ def append_kv(k: torch.Tensor, v: torch.Tensor, k_cache, v_cache, k_joint, k_sla
     dev = k.device
     if pos is not None:
         pos = pos.to(device=dev, dtype=torch.int32).contiguous()
-    ak, grid_k, k, cnt_k = _append_args(k, k_cache, k_joint, k_slack, radius_bits, t_off, pos, median_mult, "med3x_k")
-    av, grid_v, v, cnt_v = _append_args(v, v_cache, v_joint, v_slack, radius_bits, t_off, pos, median_mult, "med3x_v")
+    ak, grid_k, k, cnt_k, ws_k = _append_args(k, k_cache, k_joint, k_slack, radius_bits, t_off, pos, median_mult, "med3x_k")
+    av, grid_v, v, cnt_v, ws_v = _append_args(v, v_cache, v_joint, v_slack, radius_bits, t_off, pos, median_mult, "med3x_v")
     L.call(L.lib().hqmq_append_kv_grid, "hqmq_append_kv_grid", dev.index, C.addressof(ak), C.addressof(av), grid_k, grid_v)
     return cnt_k, cnt_v
 
 
 def _append_args(x, cache, joint, slack, radius_bits, t_off, pos, median_mult, tag):
-    """The arguments of one tensor's append.  What the cache and its codebook fix is filled in once and copied; the copy is
-    this call's own (several threads may append to one cache on streams of their own)."""
+    """The arguments of one tensor's append, and the tensors whose addresses they hold (the caller keeps them until the launch).
+    What the cache and its codebook fix is filled in once and copied; the copy is this call's own (several threads may append to
+    one cache on streams of their own)."""
     x = _strided_x(x)
     B, H, T, d_h = x.shape
     med = median_mult is not None and T > 0
@@ -319,7 +321,7 @@ def _append_args(x, cache, joint, slack, radius_bits, t_off, pos, median_mult, t
     q.B, q.T, q.t_off = B, T, t_off
     if pos is not None:
         q.pos = pos.data_ptr()
-    cnt = None
+    cnt = ws = None
     if med:
         ws = _med_workspace(x, tag)
         cnt = torch.empty(H, dtype=torch.int32, device=x.device)           # every path of the library writes all H counts
@@ -327,7 +329,7 @@ def _append_args(x, cache, joint, slack, radius_bits, t_off, pos, median_mult, t
         spare = base + (n - 12 * H & -16)
         a.median_mult, a.med_workspace, a.med_workspace_bytes = median_mult, base, n
         a.median, a.thr, a.n_out = spare, spare + 4 * H, cnt.data_ptr()
-    return a, tmpl[4], x, cnt
+    return a, tmpl[4], x, cnt, ws
 
 
 def _i32(t: torch.Tensor) -> torch.Tensor:

@@ -108,3 +108,39 @@ def test_graph_keeps_its_workspace_when_a_larger_one_takes_its_place():
             graph.replay()
             side.synchronize()
             assert torch.equal(out, want) and bool((other == 7).all())
+
+
+def test_graphs_give_their_workspaces_back():
+    """Captured calls take their scratch memory from the graph: eager calls on the stream of the capture and on the one of the
+    replay do not share it, several captured calls use it one after the other, and it is free again when the graph is gone."""
+    import gc
+    import hqmq
+    from hqmq_amd import ops
+    w = hqmq.with_outlier_extraction(hqmq.HQMQ(n_layers=1, n_heads=2, secondary_size=96, radius_bits=4, device=DEV), C=3.0)
+    cache = w.new_cache(1, 4096, 128, torch.float16, 0)
+    w.append(cache, kv_input((1, 2, 4096, 128), torch.float16, 1).to(DEV), kv_input((1, 2, 4096, 128), torch.float16, 2).to(DEV), 0)
+    Q = torch.randn(1, 8, 64, 128, generator=torch.Generator().manual_seed(3)).half().to(DEV)
+    queries, outs = (Q, -Q), [torch.empty_like(Q) for _ in range(2)]
+    want = [hqmq.fused_attention_packed(x, cache, n_splits=16) for x in queries]
+    med = ops.med3x_threshold(Q, 3.0)[0]
+    side = torch.cuda.Stream()                  # no eager call has left a buffer for this stream
+    torch.cuda.synchronize()
+    kept = {key: buf.data_ptr() for key, buf in ops._WS.items()}
+    before = torch.cuda.memory_allocated()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        for x, out in zip(queries, outs):
+            hqmq.fused_attention_packed(x, cache, n_splits=16, out=out)
+        m = ops.med3x_threshold(Q, 3.0)[0]
+    assert kept == {key: buf.data_ptr() for key, buf in ops._WS.items()}
+    for _ in range(3):
+        for out in outs:
+            out.zero_()
+        m.zero_()
+        graph.replay()
+        assert torch.equal(hqmq.fused_attention_packed(Q, cache, n_splits=16), want[0])
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], want[0]) and torch.equal(outs[1], want[1]) and torch.equal(m, med)
+    del graph, m
+    gc.collect()
+    assert torch.cuda.memory_allocated() <= before
