@@ -98,7 +98,7 @@ EXPORTS = [
     "hqmq_med3x_workspace_bytes", "hqmq_med3x_threshold", "hqmq_outlier_mask", "hqmq_outlier_compact", "hqmq_dequant",
     "hqmq_pack_codes", "hqmq_dequant_packed", "hqmq_attn_workspace_bytes", "hqmq_attn_pick_splits", "hqmq_attn_splits",
     "hqmq_attn_fwd", "hqmq_attn_combine", "hqmq_append_kv", "hqmq_attn_static_scratch_bytes", "hqmq_attn_fwd_static",
-    "hqmq_search_grid_bytes", "hqmq_build_search_grid", "hqmq_quantize_grid", "hqmq_append_kv_grid", "hqmq_crop",
+    "hqmq_search_grid_bytes", "hqmq_search_grid_kept_bytes", "hqmq_build_search_grid", "hqmq_quantize_grid", "hqmq_append_kv_grid", "hqmq_crop",
     "hqmq_pack_kv",
 ]
 BENCH_EXPORTS = ["hqmq_bench_read_planes_sink_bytes", "hqmq_bench_read_planes", "hqmq_bench_read_plain", "hqmq_bench_read_lds",
@@ -119,7 +119,7 @@ def lib():
         L.hqmq_status_string.restype = C.c_char_p
         L.hqmq_status_string.argtypes = [C.c_int]
         for name in ("hqmq_med3x_workspace_bytes", "hqmq_attn_workspace_bytes", "hqmq_attn_static_scratch_bytes",
-                     "hqmq_search_grid_bytes"):
+                     "hqmq_search_grid_bytes", "hqmq_search_grid_kept_bytes"):
             getattr(L, name).restype = i64
         # the calls of a decode loop take addresses as plain integers
         for name, n in (("hqmq_attn_fwd", 2), ("hqmq_attn_fwd_static", 2), ("hqmq_attn_splits", 1), ("hqmq_quantize_grid", 3), ("hqmq_append_kv_grid", 5), ("hqmq_crop", 2),

@@ -22,8 +22,9 @@
 //
 // Lists, per head, in blocks of 16 bytes: seven 16-bit entries p' << 2 | s' << 7 (s' = S - 1 - s; p' = 31: no entry) and
 // the number of the block that goes on (0: none, 0xffff: no list, score all rows).  The first kCells blocks are the
-// boxes', the others a pool that the build hands out; block 0 of the pool holds no entry.  Behind the lists of all
-// heads: the pools' counters, then the centres and radii of the codewords, which only the build reads.
+// boxes', the others a pool that the build hands out; block 0 of the pool holds no entry.  That is 185 KB per head (fp16,
+// fp32) or 371 KB (bf16) at every S.  Behind the lists of all heads lies what only the build reads and a caller may drop
+// afterwards (hqmq_search_grid_kept_bytes): the pools' counters, the centres and radii of the codewords.
 //
 // What it costs: per wavefront of 64 chunks about 330 vector-ALU instructions (180 for norm, division, nearest unit and
 // box, 11 per list entry, 60 - 80 for scale, radius code and packing) where the scan over 96 secondaries takes 1,885.
@@ -522,6 +523,10 @@ extern "C" int64_t hqmq_search_grid_bytes(int H, int S, int dtype) {
     if (H < 1 || (dtype != HQMQ_F32 && dtype != HQMQ_F16 && dtype != HQMQ_BF16)) return 0;
     const int64_t blocks = search_grid_blocks(S, dtype);
     return blocks ? (blocks * H + (H + 3) / 4) * 16 + (int64_t)H * 24 * S * 20 : 0;
+}
+
+extern "C" int64_t hqmq_search_grid_kept_bytes(int H, int S, int dtype) {
+    return hqmq_search_grid_bytes(H, S, dtype) > 0 ? search_grid_blocks(S, dtype) * H * 16 : 0;
 }
 
 extern "C" int hqmq_build_search_grid(const void *joint, int H, int S, int dtype, void *grid, int64_t grid_bytes, void *stream) {

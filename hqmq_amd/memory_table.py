@@ -10,6 +10,7 @@ comes from the packed layout itself: whole bits per code (main + aux planes), th
 Runs on the CPU: it only asks the library for the layout's bit widths.
 """
 import argparse
+import ctypes as C
 import json
 import math
 
@@ -51,6 +52,14 @@ def packed_kv_bytes(n_layers, n_kv_heads, d_head, seq_len, secondary_size, radiu
     return 2 * batch * n_layers * n_kv_heads * seq_len * row_bytes(d_head, secondary_size, radius_bits, med3x)
 
 
+def codebook_bytes(n_layers, n_kv_heads, secondary_size, dtype=L.F16):
+    """Bytes a model's codebooks hold on the GPU beside the caches, K and V of every layer: (joint tables, cell lists of the
+    quantize kernels).  They do not grow with the context."""
+    heads = 2 * n_layers * n_kv_heads
+    lists = L.lib().hqmq_search_grid_kept_bytes(C.c_int(1), C.c_int(secondary_size), C.c_int(dtype))
+    return heads * 24 * secondary_size * 4 * (4 if dtype == L.F32 else 2), heads * int(lists)
+
+
 def table(batch=1, med3x=None):
     rows = []
     for name, arch in MODELS.items():
@@ -82,6 +91,13 @@ def main():
     for r in rows:
         print(f"{r['model']:<12s} {r['seq_len']:>8d} {r['fp16_MB']:>10.1f} " +
               " ".join(f"{r[k + '_MB']:>9.1f} ({r[k + '_ratio']:.2f}x)" for k in keys))
+    print("\ncodebooks beside that, joint tables + cell lists in MB (fp16 / bf16 caches):")
+    for name, arch in MODELS.items():
+        cells = []
+        for S in sorted({S for S, _ in CONFIGS}):
+            (joint, lists), (_, lists_bf16) = (codebook_bytes(arch["n_layers"], arch["n_kv_heads"], S, d) for d in (L.F16, L.BF16))
+            cells.append(f"s{S}: {joint / 1e6:.1f} + {lists / 1e6:.0f} / {lists_bf16 / 1e6:.0f}")
+        print(f"{name:<12s} " + ", ".join(cells))
     print("\npacked bytes per (token, head, tensor) at d_head 128: " +
           ", ".join(f"s{S}_r{b}: {row_bytes(128, S, b, a.med3x):g}" for S, b in CONFIGS))
 

@@ -31,11 +31,13 @@ def build_joint(raw_hs4: torch.Tensor, dtype: torch.dtype):
     with torch.cuda.device(raw.device):
         L.check(L.lib().hqmq_build_joint(L.ptr(raw), C.c_int(H), C.c_int(S), C.c_int(L.DT_CODE[dtype]), L.ptr(joint),
                                          L.ptr(slack), L.stream_ptr(raw.device)), "hqmq_build_joint")
-        nbytes = int(L.lib().hqmq_search_grid_bytes(C.c_int(H), C.c_int(S), C.c_int(L.DT_CODE[dtype])))
+        nbytes, kept = (int(f(C.c_int(H), C.c_int(S), C.c_int(L.DT_CODE[dtype])))
+                        for f in (L.lib().hqmq_search_grid_bytes, L.lib().hqmq_search_grid_kept_bytes))
         if nbytes:
-            slack.hqmq_grid = grid = torch.empty(nbytes, dtype=torch.uint8, device=raw.device)
+            grid = torch.empty(nbytes, dtype=torch.uint8, device=raw.device)
             L.check(L.lib().hqmq_build_search_grid(L.ptr(joint), C.c_int(H), C.c_int(S), C.c_int(L.DT_CODE[dtype]),
                                                    L.ptr(grid), L.i64(nbytes), L.stream_ptr(raw.device)), "hqmq_build_search_grid")
+            slack.hqmq_grid = grid[:kept].clone()            # behind it: scratch memory of the build
     return joint, slack
 
 

@@ -108,9 +108,12 @@ int hqmq_quantize(const hqmq_quantize_args *a, void *stream);
  * can win the reference's rounded comparison there (see csrc/quantize_grid.hip).  Worked out once per codebook, they
  * replace the quantize kernel's scan over the secondaries; the codes are the same, bit for bit.
  *   hqmq_search_grid_bytes    size for H heads of S secondaries; 0 where the lists do not exist (S > 341)
+ *   hqmq_search_grid_kept_bytes  the part from the start that the quantize kernels read; the rest is scratch memory of the
+ *                             build, and the lists may be copied to a buffer of this size afterwards
  *   joint                     as hqmq_build_joint left it
  *   grid                      (out) hqmq_search_grid_bytes bytes, 16-byte aligned */
 int64_t hqmq_search_grid_bytes(int H, int S, int dtype);
+int64_t hqmq_search_grid_kept_bytes(int H, int S, int dtype);
 int hqmq_build_search_grid(const void *joint, int H, int S, int dtype, void *grid, int64_t grid_bytes, void *stream);
 /* hqmq_quantize with the codebook's cell lists (NULL: without); algo and every other argument as there.  stats[1] counts
  * the chunks that were searched through the lists. */

@@ -210,6 +210,17 @@ def test_memory_table_uses_packed_layout():
         assert r[k + "_analytic_MB"] <= r[k + "_MB"] <= 1.08 * r[k + "_analytic_MB"]
 
 
+def test_cell_lists_are_counted_without_the_scratch_memory_of_their_build():
+    from hqmq_amd import _lib as L, memory_table as MT
+    lib = L.lib()
+    for code in (L.F32, L.F16, L.BF16):
+        for S in (1, 24, 341):
+            kept, full = (f(C.c_int(8), C.c_int(S), C.c_int(code)) for f in (lib.hqmq_search_grid_kept_bytes, lib.hqmq_search_grid_bytes))
+            assert 0 < kept < full and full - kept == 32 + 8 * 24 * S * 20 and kept % (8 * 16) == 0
+            assert MT.codebook_bytes(32, 8, S, code) == (512 * 24 * S * 4 * (4 if code == L.F32 else 2), 64 * kept)
+    assert lib.hqmq_search_grid_kept_bytes(C.c_int(8), C.c_int(342), C.c_int(L.F16)) == 0
+
+
 def test_crop_bookkeeping_on_cpu():
     """PackedTensor.crop_ is plain torch: after a crop, the entry count and the tile offsets equal what appending
     only the kept rows would have left, and no flag stays behind in a dropped row."""

@@ -22,12 +22,15 @@ def _raw(S, crowded, g):
 @pytest.mark.parametrize("dn", ["fp32", "fp16", "bf16"])
 @pytest.mark.parametrize("S,crowded", [(1, False), (24, True), (96, False), (341, False), (341, True), (342, False)])
 def test_cell_lists_pick_what_the_scan_picks(S, crowded, dn):
-    from hqmq_amd import ops
+    from hqmq_amd import _lib, ops
     dt = DT[dn]
     g = torch.Generator().manual_seed(S)
     raw = _raw(S, crowded, g)
     J, slack = ops.build_joint(raw.to(DEV), dt)
     assert hasattr(slack, "hqmq_grid") == (S <= 341)
+    if S <= 341:                            # the lists alone are kept (2 heads): no memory of the build behind them
+        kept = _lib.lib().hqmq_search_grid_kept_bytes(2, S, _lib.DT_CODE[dt])
+        assert slack.hqmq_grid.numel() == slack.hqmq_grid.untyped_storage().nbytes() == kept
     for T, d_h in ((1, 128), (2, 128), (3, 80), (8, 128), (9, 128), (33, 128), (70, 64), (5, 1024), (300, 160)):
         x = torch.randn(1, 2, T, d_h, generator=g)
         x[:, :, T // 2, :4] = J[0, 0].float().cpu()          # a codeword, a zero chunk, a chunk on a unit, one between two units
