@@ -91,9 +91,17 @@ __device__ __forceinline__ float exact2_of(const float v[4], int p) {
     return (t0 + t1) + (t2 + t3);
 }
 
-template <class D, int ALGO, bool ROWS>
+// SPLIT (single-token appends, 16-bit dtypes, n a power of two): the block's 256 / n token slots all hold the one new
+// token of (b, h) and share its secondaries between them: slot w scores s = w, w + slots, ...  A decode-step append is
+// one wavefront's serial instruction stream otherwise; this divides the search part of it by the number of slots.
+// The slots' candidates are merged exactly: the filter threshold comes from the maximum over all slots, the winner
+// is the highest exact score with the lowest index, as in the unsplit search.
+// K and V of one token, 8 heads, in one launch instead of two unsplit ones: S = 384 51 -> 13 us (fp16), 1651 -> 18 us (bf16, where
+// the list of an unsplit lane overflows and all rows are scored), S = 1024 110 -> 20 us.
+template <class D, int ALGO, bool ROWS, bool SPLIT>
 __device__ __forceinline__ void quantize_body(const QParams &a) {
     using ST = typename D::storage;
+    static_assert(!SPLIT || (ALGO == 0 && ROWS && D::code != HQMQ_F32), "the split search is the MFMA search");
     extern __shared__ float sec[];  // [S][4] secondaries, then [S][4] fp16 columns of their rotation matrices
     uint2 *rot = reinterpret_cast<uint2 *>(sec + 4 * a.S);
     __shared__ uint32_t code_sh[kQThreads];
@@ -104,9 +112,11 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
     const int tid = threadIdx.x;
     const int bh = blockIdx.y, b = bh / a.H, h = bh - b * a.H;
     const int n = a.n, S = a.S, K = 24 * S;
-    const int tok_local = tid / n, c = tid - tok_local * n;
-    const int t = blockIdx.x * a.tokens_per_block + tok_local;
+    const int tok_local = tid / n, c = tid - tok_local * n;       // SPLIT: tok_local is the slot
+    const int t = SPLIT ? 0 : blockIdx.x * a.tokens_per_block + tok_local;
     const bool active = tok_local < a.tokens_per_block && t < a.T;
+    const bool writer = !SPLIT || tok_local == 0;                 // one slot stores the results
+    const int slots = SPLIT ? kQThreads / n : 1, s_first = SPLIT ? tok_local : 0;
     const ST *jh = (const ST *)a.joint + (size_t)h * K * 4;
 
     for (int i = tid; i < S * 4; i += kQThreads) sec[i] = D::load(jh + i);  // rows k = s are q_s itself
@@ -164,20 +174,21 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
             // become a bit mask (a compare and an add-with-carry each) and go into the list of the re-score below.  A
             // threshold that has moved above the maximum before the block leaves everything listed before below the
             // final threshold: the list starts over.
-            uint2 a_next = acol[0];
+            const int iters = (S + slots - 1) / slots;          // of the slot with the most secondaries (wave-uniform)
+            uint2 a_next = acol[4 * min(s_first, S - 1)];
             float thr = -INFINITY;
             auto scan_block = [&](int i0, auto tail) -> uint32_t {
                 float b2v[32];
 #pragma unroll
                 for (int i = 0; i < 32; i++) {
-                    const int sn = i0 + i + 1;
+                    const int sn = s_first + (i0 + i + 1) * slots;
                     const half4 am = __builtin_bit_cast(half4, a_next);
                     // the next column is on its way during this one; inside a whole block it exists, so its address is
                     // the block's base plus a constant
                     a_next = (decltype(tail)::value || i == 31) ? acol[4 * min(sn, S - 1)] : acol[4 * sn];
                     const float4v vv = __builtin_amdgcn_mfma_f32_4x4x4f16(am, ub, float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                     float b2 = best2_mfma(vv[0], vv[1], vv[2], vv[3]);
-                    if (decltype(tail)::value && sn > S) b2 = -INFINITY;      // behind the last secondary
+                    if (decltype(tail)::value && sn - slots >= S) b2 = -INFINITY;      // behind the slot's last secondary
                     b2v[i] = b2;
                     // the running maximum takes two scores at a time (all ordinary numbers or -inf here)
                     if (i & 1) asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m2) : "v"(m2), "v"(b2v[i - 1]), "v"(b2));
@@ -187,17 +198,22 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
 #pragma unroll
                 for (int i = 31; i >= 0; i--)       // word = 2 word + (score >= thr): iteration i ends up in bit i
                     asm("v_cmp_ge_f32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(word) : "v"(b2v[i]), "v"(thr) : "vcc");
-                if (decltype(tail)::value) word &= (1u << (S - i0)) - 1u;       // fewer than 32 are left
+                if (decltype(tail)::value) {        // a slot whose secondaries end inside the block: only those count
+                    const int left = S - s_first - i0 * slots;
+                    const int valid = left <= 0 ? 0 : min((left + slots - 1) / slots, 32);
+                    word &= valid >= 32 ? ~0u : (1u << valid) - 1u;
+                }
                 return word;
             };
-            for (int i0 = 0; i0 < S; i0 += 32) {
+            for (int i0 = 0; i0 < iters; i0 += 32) {
                 const float m_before = m2;
-                uint32_t bits = i0 + 32 <= S ? scan_block(i0, std::false_type{}) : scan_block(i0, std::true_type{});
+                const bool whole = (slots - 1) + (i0 + 31) * slots < S;     // every slot has all 32 secondaries of this block
+                uint32_t bits = whole ? scan_block(i0, std::false_type{}) : scan_block(i0, std::true_type{});
                 if (m_before < thr) cnt = 0;
                 while (bits) {
                     const int i = __builtin_ctz(bits);
                     bits &= bits - 1u;
-                    if (cnt < kSCap) slist[cnt][tid] = (uint16_t)(i0 + i);
+                    if (cnt < kSCap) slist[cnt][tid] = (uint16_t)(s_first + (i0 + i) * slots);
                     cnt++;
                 }
             }
@@ -214,6 +230,13 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
                 }
                 m2 = fmaxf(m2, b2);
             }
+        }
+        if (SPLIT) {        // the maximum over all slots of this chunk (every slot holds the same direction)
+            float *m2_sh = reinterpret_cast<float *>(code_sh);
+            m2_sh[tid] = m2;
+            __syncthreads();
+            for (int w = 0; w < slots; w++) m2 = fmaxf(m2, m2_sh[w * n + c]);
+            __syncthreads();
         }
         float bs = -INFINITY;
         int bk = 0x7fffffff;
@@ -270,33 +293,68 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
             }
         }
         if (brute) idx = brute_argmax<D>(u, jh, K);
+        if (SPLIT) {
+            // merge the slots: a slot that fell back to the exhaustive search holds the answer; otherwise the highest
+            // exact score wins, the lowest index among equals; no candidate anywhere (all-zero direction) -> index 0
+            float *bs_sh = reinterpret_cast<float *>(code_sh);
+            int *bk_sh = reinterpret_cast<int *>(aux_sh);
+            bs_sh[tid] = bs;
+            bk_sh[tid] = brute ? (idx | (int)0x80000000) : (search ? bk : 0x7fffffff);
+            __syncthreads();
+            float ms = -INFINITY;
+            int mk = 0x7fffffff;
+            bool exact = false;
+            for (int w = 0; w < slots; w++) {
+                const int kw = bk_sh[w * n + c];
+                const float sw = bs_sh[w * n + c];
+                if (kw < 0) {
+                    if (!exact) { exact = true; mk = kw & 0x7fffffff; }
+                } else if (!exact && kw != 0x7fffffff && (sw > ms || (sw == ms && kw < mk))) {
+                    ms = sw;
+                    mk = kw;
+                }
+            }
+            idx = mk == 0x7fffffff ? 0 : mk;
+            __syncthreads();
+        }
         if (a.stats && active) {
-            if (brute) atomicAdd(a.stats, 1);
+            if (brute && writer) atomicAdd(a.stats, 1);      // once per chunk, also when its slots split the search
             if (search && !brute) atomicAdd(a.stats + 1, cnt);
         }
     }
 
     ChunkSink<D, kQThreads, ROWS, kUnpacked | kPlanes | kCompact, 0> sink(a, b, h, tok_local, c, code_sh, aux_sh);
-    sink.put(blockIdx.x * a.tokens_per_block, active, raw, nrm, r, idx, jh + (size_t)idx * 4);
+    sink.put(blockIdx.x * a.tokens_per_block, active && writer, raw, nrm, r, idx, jh + (size_t)idx * 4);
     sink.done();
 }
 
-template <class D, int ALGO, bool ROWS>
-__global__ __launch_bounds__(kQThreads) void quantize_kernel(QParams a) {
-    quantize_body<D, ALGO, ROWS>(a);
+// One tensor, or the K and the V rows of one append in one launch (same shapes): blockIdx.z picks the tensor.  A single-token
+// append is latency-bound (32 lanes per block for a few microseconds), so the two run side by side for free.
+// (indexed in the kernel-argument segment: one set of scalar registers, not a select per field of two structs)
+template <class D, int ALGO, bool ROWS, bool SPLIT>
+__global__ __launch_bounds__(kQThreads) void quantize_kernel(QPair kv) {
+    quantize_body<D, ALGO, ROWS, SPLIT>(kv.p[blockIdx.z]);
 }
 
 template <class D>
-static int launch_quantize(const QParams &p, int algo, hipStream_t st) {
-    dim3 grid((p.T + p.tokens_per_block - 1) / p.tokens_per_block, p.B * p.H), block(kQThreads);
+static int launch_quantize(const QPair &kv, int count, int algo, hipStream_t st) {
+    const QParams &p = kv.p[0];
+    dim3 grid((p.T + p.tokens_per_block - 1) / p.tokens_per_block, p.B * p.H, count), block(kQThreads);
     size_t shmem = (size_t)p.S * 4 * sizeof(float) + (size_t)p.S * 4 * sizeof(uint2);
     const bool rows = !(p.n & (p.n - 1)) && p.n <= 64;
+    if constexpr (sizeof(typename D::storage) == 2) {
+        // one new token per sequence, the lanes of a token inside a wavefront: the split search
+        if (algo == 0 && p.T == 1 && rows && p.n >= 4) {
+            hipLaunchKernelGGL((quantize_kernel<D, 0, true, true>), grid, block, shmem, st, kv);
+            return hip_status(hipGetLastError());
+        }
+    }
     if (algo == 1) {
-        if (rows) hipLaunchKernelGGL((quantize_kernel<D, 1, true>), grid, block, shmem, st, p);
-        else hipLaunchKernelGGL((quantize_kernel<D, 1, false>), grid, block, shmem, st, p);
+        if (rows) hipLaunchKernelGGL((quantize_kernel<D, 1, true, false>), grid, block, shmem, st, kv);
+        else hipLaunchKernelGGL((quantize_kernel<D, 1, false, false>), grid, block, shmem, st, kv);
     } else {
-        if (rows) hipLaunchKernelGGL((quantize_kernel<D, 0, true>), grid, block, shmem, st, p);
-        else hipLaunchKernelGGL((quantize_kernel<D, 0, false>), grid, block, shmem, st, p);
+        if (rows) hipLaunchKernelGGL((quantize_kernel<D, 0, true, false>), grid, block, shmem, st, kv);
+        else hipLaunchKernelGGL((quantize_kernel<D, 0, false, false>), grid, block, shmem, st, kv);
     }
     return hip_status(hipGetLastError());
 }
@@ -370,11 +428,12 @@ static bool take_compaction(QParams &p, const CompactCall *c) {
     return true;
 }
 
-static int launch_one_tensor(const QParams &p, int dtype, int algo, hipStream_t st) {
+// one tensor (count = 1) or K and V of equal shape
+static int launch_scan(const QPair &kv, int count, int dtype, int algo, hipStream_t st) {
     switch (dtype) {
-        case HQMQ_F32: return launch_quantize<F32>(p, algo, st);
-        case HQMQ_F16: return launch_quantize<F16>(p, algo, st);
-        default: return launch_quantize<BF16>(p, algo, st);
+        case HQMQ_F32: return launch_quantize<F32>(kv, count, algo, st);
+        case HQMQ_F16: return launch_quantize<F16>(kv, count, algo, st);
+        default: return launch_quantize<BF16>(kv, count, algo, st);
     }
 }
 
@@ -384,7 +443,7 @@ extern "C" int hqmq_quantize_grid(const hqmq_quantize_args *a, const void *grid,
     const int rc = fill_qparams(a, grid, &p, &empty);
     if (rc || empty) return rc;
     if (p.grid && a->algo == 0) return launch_quantize_grid(QPair{{p, p}}, 1, a->dtype, (hipStream_t)stream);
-    return launch_one_tensor(p, a->dtype, a->algo, (hipStream_t)stream);
+    return launch_scan(QPair{{p, p}}, 1, a->dtype, a->algo, (hipStream_t)stream);
 }
 
 extern "C" int hqmq_quantize(const hqmq_quantize_args *a, void *stream) { return hqmq_quantize_grid(a, nullptr, stream); }
@@ -401,12 +460,14 @@ int hqmq::quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v,
         compacted[i] = !empty[i] && take_compaction(p[i], cc[i]);
     }
     const bool by_cells[2] = {p[0].grid && k->algo == 0, p[1].grid && v->algo == 0};
-    if (!empty[0] && !empty[1] && by_cells[0] && by_cells[1] && k->dtype == v->dtype && k->B == v->B && k->H == v->H && k->T == v->T &&
-        k->n_chunks == v->n_chunks && k->secondary_size == v->secondary_size)
-        return launch_quantize_grid(QPair{{p[0], p[1]}}, 2, k->dtype, st);
+    const bool same = !empty[0] && !empty[1] && k->dtype == v->dtype && k->B == v->B && k->H == v->H && k->T == v->T && k->n_chunks == v->n_chunks &&
+                      k->secondary_size == v->secondary_size && k->algo == 0 && v->algo == 0;
+    if (same && by_cells[0] && by_cells[1]) return launch_quantize_grid(QPair{{p[0], p[1]}}, 2, k->dtype, st);
+    if (same && !by_cells[0] && !by_cells[1]) return launch_scan(QPair{{p[0], p[1]}}, 2, k->dtype, 0, st);
     for (int i = 0; i < 2; i++) {
         if (empty[i]) continue;
-        const int rc = by_cells[i] ? launch_quantize_grid(QPair{{p[i], p[i]}}, 1, a[i]->dtype, st) : launch_one_tensor(p[i], a[i]->dtype, a[i]->algo, st);
+        const QPair one{{p[i], p[i]}};
+        const int rc = by_cells[i] ? launch_quantize_grid(one, 1, a[i]->dtype, st) : launch_scan(one, 1, a[i]->dtype, a[i]->algo, st);
         if (rc) return rc;
     }
     return HQMQ_OK;

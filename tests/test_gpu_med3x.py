@@ -162,18 +162,18 @@ def test_decode_appends_keep_sideband_consistent():
     assert w._n_observations == 2 * steps
 
 
-@pytest.mark.parametrize("dn,d_h,med,ragged", [("bf16", 128, True, True), ("fp16", 64, True, False), ("fp16", 128, False, True),
-                                               ("fp32", 32, True, False)])
-def test_shared_launches_equal_single_tensor_calls(dn, d_h, med, ragged):
-    """append() sends K and V through every stage together (one launch per stage when the shapes allow it, one
-    after the other for fp32 and for bulk appends); every plane, the sideband and the counters equal those of the
+@pytest.mark.parametrize("dn,d_h,med,ragged,S", [("bf16", 128, True, True, 24), ("fp16", 64, True, False, 24), ("fp16", 128, False, True, 24),
+                                                 ("fp32", 32, True, False, 24), ("fp16", 128, True, True, 350), ("bf16", 64, True, False, 400)])
+def test_shared_launches_equal_single_tensor_calls(dn, d_h, med, ragged, S):
+    """append() sends K and V through every stage together (one launch per stage when the shapes allow it), with cell lists
+    and, beyond 341 secondaries, without; every plane, the sideband and the counters equal those of the
     single-tensor calls, for a bulk append followed by short ones."""
     import hqmq
     dt = DT[dn]
     B, H, T0 = 3, 2, 640
     steps = [T0, 1, 0, 1, 5, 1, 16, 3]        # an empty append changes nothing
     total = sum(steps) + 8
-    inner = hqmq.HQMQ(n_layers=1, n_heads=H, secondary_size=24, radius_bits=3, device=DEV)
+    inner = hqmq.HQMQ(n_layers=1, n_heads=H, secondary_size=S, radius_bits=3, device=DEV)
     w = hqmq.with_outlier_extraction(inner) if med else inner
     mult = w.median_mult if med else None
     make = lambda: w.new_cache(B, total, d_h, dt, 0, sideband_frac=0.5) if med else w.new_cache(B, total, d_h, dt, 0)

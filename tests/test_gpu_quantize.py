@@ -91,20 +91,34 @@ def test_adversarial_ties(dn):
 @pytest.mark.parametrize("dn", ["fp16", "bf16"])
 @pytest.mark.parametrize("d_h", [16, 64, 128, 256])
 def test_single_token_calls_match_oracle(S, b_r, dn, d_h):
-    """Calls with one token per sequence (the decode-step append) search with the secondaries split over the
-    block's token slots; indices, radius codes and scales equal the oracle's, edge cases and ties included."""
+    """Calls with one token per sequence (the decode-step append), through the cell lists: indices, radius codes and scales
+    equal the oracle's, edge cases and ties included."""
+    _check_single_tokens(S, b_r, dn, d_h, lists=True)
+
+
+@pytest.mark.parametrize("S,b_r", [(1, 3), (24, 3), (192, 6), (384, 4), (1000, 4)])
+@pytest.mark.parametrize("dn,d_h", [("fp16", 16), ("fp16", 64), ("fp16", 256), ("bf16", 128), ("fp32", 128), ("fp16", 80)])
+def test_single_token_scans_match_oracle(S, b_r, dn, d_h):
+    """The same without lists (S > 341, callers that pass none): 16-bit calls search with the secondaries split over the block's
+    token slots, fewer secondaries than slots and partial blocks of 32 among them; fp32 and d_h 80 take the unsplit scan."""
+    _check_single_tokens(S, b_r, dn, d_h, lists=False)
+
+
+def _check_single_tokens(S, b_r, dn, d_h, lists):
     ops, dt = _ops(), DT[dn]
     H, N = 2, 160
     raw = TO.secondary_raw(1, H, S, 9)[0, :, 0]
     Jc = CO.joint_table(raw, dt)
     J, slack = ops.build_joint(raw.to(DEV), dt)
+    if not lists:
+        slack = slack.clone()                               # the lists are an attribute of the original
     x = kv_input((N, H, 1, d_h), dt, seed=21, outlier_p=0.02)
     e = edge_cases(x.transpose(0, 2).contiguous())          # the helper plants along the token axis
     x = e.transpose(0, 2).contiguous()
     Jf = Jc[0].float()                                      # exact codewords, negatives and midpoints: ties
     ties = torch.cat([Jf[:40], -Jf[40:80], Jf[:40] + Jf.roll(1, 0)[:40], Jf[:40] + Jf.roll(S, 0)[:40]], 0).to(dt)
     flat = ties.reshape(-1)
-    n_tok = flat.numel() // d_h
+    n_tok = min(flat.numel() // d_h, N)
     x[:n_tok, 0, 0] = flat[:n_tok * d_h].reshape(n_tok, d_h)
     want = CO.quantize(x, Jc, b_r)
     got = ops.quantize(x.to(DEV), J, slack, b_r, want_dense=True)
@@ -114,9 +128,11 @@ def test_single_token_calls_match_oracle(S, b_r, dn, d_h):
     assert bit_equal(got["out"], want["out"])
 
 
-@pytest.mark.parametrize("S,b_r,dn,d_h", [(24, 3, "bf16", 128), (96, 4, "fp16", 128), (192, 6, "fp16", 64), (96, 4, "bf16", 32)])
+@pytest.mark.parametrize("S,b_r,dn,d_h", [(24, 3, "bf16", 128), (96, 4, "fp16", 128), (192, 6, "fp16", 64), (96, 4, "bf16", 32),
+                                           (384, 4, "fp16", 128), (384, 3, "bf16", 64), (350, 4, "fp32", 32)])
 def test_token_by_token_appends_equal_one_bulk_append(S, b_r, dn, d_h):
-    """The split search of single-token appends and the bulk search leave the same planes."""
+    """The short form of single-token appends and the bulk search leave the same planes: through the cell lists, and with
+    scans for codebooks without lists (K and V share each launch)."""
     import hqmq
     dt = DT[dn]
     B, H, T = 3, 2, 37
