@@ -16,10 +16,12 @@
 //   * K and V in LDS are codeword * radius code; K's scale of the token is applied to the score and V's to P, in fp32, as the decode
 //     kernels do (V times radius * scale / qmax in LDS saves 16 multiplications per 32 tokens, but rounds once more: 4 to 8 % further
 //     from 64-bit results at fp16);
-//   * fp16 outlier caches (FL): K and V in LDS are the values themselves, multiplied out in fp32 and rounded once, and the wavefront
-//     that decoded a tile then writes the tile's verbatim chunks over the zeros that flagged chunks decode to.  They stay exact, and
-//     no sparse product is left (the decode kernels spend a third of their time on it).  bf16 caches keep the decode kernels: a
-//     verbatim bf16 chunk need not fit fp16;
+//   * fp16 outlier caches (FL): the wavefront that decoded a tile writes the tile's verbatim chunks over the zeros that flagged
+//     chunks decode to, and marks K's in a flag word per token.  K is codeword * radius code elsewhere, as above: the operand of
+//     a score step is split by the flags into codes and verbatim values (a mask per chunk), which are multiplied one after
+//     the other; the two sums meet when the token's scale is applied, so that K has the decode kernels' precision at every magnitude.
+//     V is held as values, multiplied out in fp32 and rounded once, in which the verbatim chunks have their place, and P is not
+//     multiplied with scales, one rounding less.  bf16 caches keep the decode kernels: a verbatim bf16 chunk need not fit fp16;
 //   * one basic block per 32 tokens, written out one matrix instruction at a time: the scores of the next 32 tokens run with
 //     the exponentials of these, their products with V with the decoding of a later tile.  A matrix instruction takes 32
 //     cycles of its own pipe, a vector instruction about 4.3 of the shared issue slot (8.3 for an exponential), so that the
@@ -29,8 +31,13 @@
 // Measured, B = 1, 32 / 8 heads of 128, s96_r4, 1024 queries on 32768 tokens (541 GFLOP, 0.43 ms at the rate of a large matrix
 // product): 0.68 ms against 0.96 with the decode kernels' two-column-group variants; 4096 on 4096 tokens causal, s24_r3:
 // 0.19 against 0.41; four sequences of 300 on 300: 0.022 against 0.048.  With 2 % of the K and V chunks verbatim: 1024 queries on
-// 32768 tokens 0.70 ms against 2.87, 300 on 8000 (28 / 4 heads, s192_r6) 0.10 against 0.32.  What bounds it: a compute unit spends 36 % of the
-// time in the matrix pipe, 50 % issuing vector instructions (a quarter of them decode) and 46 % in LDS, at 2.0 to 2.1 GHz.
+// 32768 tokens 0.93 ms against 2.88, 300 on 8000 (28 / 4 heads, s192_r6) 0.122 against 0.318.  (K held as values like V, without the
+// second product: 0.70 and 0.101, but up to 1.55 times as far from 64-bit results at K of 3e-5 and 1.34 times at K of order one;
+// values only in tokens with verbatim chunks, in units of a power of two: 0.80 and 0.107, still up to 1.11.)  Error against 64-bit
+// results relative to the decode kernels', 162 calls: K from 3e-5 to 30 at V of order one 0.92 on average, 0.99 at most; V of 1e-4
+// 0.77 and 1.00, V of 3e-5, where outputs are fp16 subnormals, 0.81 and 1.08.
+// What bounds it (plain caches): a compute unit spends 36 % of the time in the matrix pipe, 50 % issuing vector instructions (a
+// quarter of them decode) and 46 % in LDS, at 2.0 to 2.1 GHz.
 #include "attention_mfma.h"
 #include <algorithm>
 
@@ -40,7 +47,8 @@ typedef float float16v __attribute__((ext_vector_type(16)));
 typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kPfV = 16384, kPfBuf = 32768, kPfScale = 2 * kPfBuf, kPfScaleV = 1024, kPfTab = kPfScale + 2048;   // LDS: K | V, twice; scales; tables
+constexpr uint32_t kPfV = 16384, kPfBuf = 32768, kPfScale = 2 * kPfBuf, kPfScaleV = 1024, kPfFlag = kPfScale + 2048;   // LDS: K | V, twice; scales; flags (FL); tables
+constexpr uint32_t pf_tab(bool fl) { return kPfFlag + (fl ? 1024u : 0u); }
 
 // permutation of a row's 16-byte parts
 template <int DH>
@@ -56,6 +64,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     constexpr int n = DH / 4, ROWB = DH * 2, CW = 8 / KVG, KS = DH / 16, DB = DH / 32;
     constexpr int TILE = 8192 / DH, NSUB = TILE / 32 / KVG;              // tokens per tile; units of 32 of them per wavefront
     constexpr int TOK = DH == 128 ? 16 : 32;                             // tokens a wavefront decodes: 8 chunks per lane
+    constexpr uint32_t kPfTab = pf_tab(FL);
     extern __shared__ uint2 lds_tab[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5, col = lane & 31;
@@ -136,6 +145,14 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     const uint2 *sb_val = FL ? (const uint2 *)dc.sideband + (size_t)bh * dc.sb_cap : nullptr;
     const uint16_t *sb_xy = FL ? dc.sb_coord + (size_t)bh * dc.sb_cap : nullptr;
     const int sb_count = FL ? min(max(uniform_word(dc.sb_count, bh), 0), (int)dc.sb_cap) : 0;
+    // LEAN: no registers are left over, and a spilled one that is read back in the loop waits for every request in flight
+    constexpr bool LEAN = FL && AUX;
+    auto lane_id = [&]() PF_INLINE {
+        if (!LEAN) return lane;
+        int id = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+        asm volatile("" : "+v"(id));
+        return id;
+    };
     int rg[SBT + 1];                                                      // of the tile whose entries are requested next
     auto offsets = [&](int t0) PF_INLINE {
         const int first = (t0 >> 4) + (wave & 3) * SBT;
@@ -151,16 +168,19 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         ent.from = min(max(rg[0], 0), sb_count);
         ent.to = max(ent.from, min(rg[SBT], sb_count));
         ent.mid = rg[SBT - 1];
-        const int e = min(ent.from + lane, (int)dc.sb_cap - 1);
+        const int e = min(ent.from + lane_id(), (int)dc.sb_cap - 1);
         ent.val = sb_val[e];
         ent.xy = sb_xy[e];
         offsets(t0 + TILE);
     };
-    // entry e into LDS; those of rows past the range are dropped (their scores are masked, but 0 * inf is not 0)
-    auto patch = [&](int e, uint2 val, uint32_t xy, uint32_t at) PF_INLINE {
+    // Entry e into LDS; those of rows past the range are dropped (their scores are masked, but 0 * inf is not 0).  K's are marked in
+    // their token's flag word.
+    auto patch = [&](int e, uint2 val, uint32_t xy, uint32_t buf) PF_INLINE {
         const uint32_t t = (uint32_t)(wave & 3) * TOK + ((xy >> 8) & 15u) + (SBT > 1 && e >= ent.mid ? 16u : 0u), ch = xy & (uint32_t)(n - 1);
-        if (e < ent.to && ent.t0 + (int)t < b_end)
-            *(uint2v __attribute__((address_space(3))) *)(uintptr_t)(at + t * ROWB + (pf_part<DH>(t, ch >> 1) << 4) + (ch & 1u) * 8u) = __builtin_bit_cast(uint2v, val);
+        if (e < ent.to && ent.t0 + (int)t < b_end) {
+            if (!dec_v) __hip_atomic_fetch_or((uint32_t __attribute__((address_space(3))) *)(uintptr_t)(kPfFlag + buf * 512u + 4u * t), 1u << ch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            *(uint2v __attribute__((address_space(3))) *)(uintptr_t)(buf * kPfBuf + (dec_v ? kPfV : 0u) + t * ROWB + (pf_part<DH>(t, ch >> 1) << 4) + (ch & 1u) * 8u) = __builtin_bit_cast(uint2v, val);
+        }
     };
     struct Codes { uint32_t w[NW], aux, aux2, sh, scale; };
     auto request = [&](int t0, Codes &c) PF_INLINE {
@@ -185,7 +205,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     // radii unpacked (2, 3), products stored (4 .. 7); in registers between them:
     half4 wg[8];
     half2v wr[4];
-    float w_scale = 0.f;
+    float w_scale = 0.f, w_mul = 1.f;
     uint32_t w_at = (dec_v ? kPfV : 0u) + (uint32_t)d_tok * ROWB + (pf_part<DH>((uint32_t)d_tok, (uint32_t)(d_grp * 4)) << 4);
     uint32_t ws_at = kPfScale + (dec_v ? kPfScaleV : 0u) + 4u * (uint32_t)d_tok;
     const bool w_lane = d_grp == 0;
@@ -218,32 +238,35 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
                     wr[i] = __builtin_bit_cast(half2v, t) - half2v{(_Float16)1024.0f, (_Float16)1024.0f};
                 }
             }
-            // K and V keep their radius codes; the token's scales are applied to the score and to P, in fp32
+            // K and V keep their radius codes; the token's scales are applied to the score and to P, in fp32.  (FL: V rows hold the
+            // values themselves, rounded once, as its verbatim chunks are)
             if (j == 3) {
                 w_scale = DT == HQMQ_F16 ? __half2float(__ushort_as_half((uint16_t)c.scale)) : __uint_as_float(c.scale << 16);
+                if (FL) w_mul = dec_v ? w_scale * p.inv_qmax : 1.f;
             }
         } else {
             const int i = j - 4;
-            if (FL) {                                                     // the value itself, rounded once, as the verbatim chunks are
-                const float f = w_scale * p.inv_qmax;
+            if (FL) {                                                     // rounded once (K: codeword * radius code, as below)
                 half8 v;
 #pragma unroll
                 for (int x = 0; x < 2; x++) {
-                    const float r = (float)wr[i][x] * f;
+                    const float r = (float)wr[i][x] * w_mul;
 #pragma unroll
                     for (int y = 0; y < 4; y++) v[4 * x + y] = (_Float16)__builtin_fmaf((float)wg[2 * i + x][y], r, 0.f);
                 }
                 *(uint4v __attribute__((address_space(3))) *)(uintptr_t)(w_at ^ ((uint32_t)i << 4)) = __builtin_bit_cast(uint4v, v);
             } else *(uint4v __attribute__((address_space(3))) *)(uintptr_t)(w_at ^ ((uint32_t)i << 4)) =
                 __builtin_bit_cast(uint4v, cat8(wg[2 * i] * wr[i][0], wg[2 * i + 1] * wr[i][1]));
-            if (FL && j == 7) {
-                asm volatile("" ::: "memory");                            // the wavefront's LDS writes keep their order
-                const uint32_t at = (w_at & kPfBuf) | (dec_v ? kPfV : 0u);
-                patch(ent.from + lane, ent.val, ent.xy, at);
-                for (int e = ent.from + 64 + lane; e < ent.to; e += 64) patch(e, sb_val[e], sb_xy[e], at);
-            }
             if (j == 7) {
-                if (!FL && w_lane) *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = dec_v ? w_scale : w_scale * p.c_log2;
+                if (w_lane) *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = dec_v ? w_scale : w_scale * p.c_log2;
+                if (FL) {
+                    if (w_lane && !dec_v) *(uint32_t __attribute__((address_space(3))) *)(uintptr_t)(ws_at + (kPfFlag - kPfScale)) = 0u;
+                    asm volatile("" ::: "memory");                        // the wavefront's LDS accesses keep their order
+                    const uint32_t buf = w_at / kPfBuf;
+                    const int first = ent.from + lane_id();
+                    patch(first, ent.val, ent.xy, buf);
+                    for (int e = first + 64; e < ent.to; e += 64) patch(e, sb_val[e], sb_xy[e], buf);
+                }
                 w_at ^= kPfBuf;
                 ws_at ^= 512u;
             }
@@ -290,7 +313,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     __syncthreads();
 
     // ---- LDS addresses of the operands (tile buffer 0) ----
-    uint32_t ka[KS], va[2][DB];
+    uint32_t ka[KS], va[2][DB], ka0;
     const uint32_t wo = (uint32_t)kvg * (32u * NSUB * ROWB);              // this wavefront's share of a tile
 #pragma unroll
     for (int kk = 0; kk < KS; kk++) ka[kk] = wo + (uint32_t)col * ROWB + (pf_part<DH>((uint32_t)col, (uint32_t)(2 * kk + half)) << 4);
@@ -303,7 +326,9 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
             const uint32_t q = (uint32_t)(4 * db + 2 * ((lane >> 4) & 1)) + ((i & 3) >> 1);
             va[hf][db] = wo + kPfV + t * ROWB + (pf_part<DH>(t, q) << 4) + (i & 1) * 8u;
         }
+    ka0 = ka[0];                                                          // the parts of a row differ by an exclusive-or
     const uint32_t sa = kPfScale + 16u * (uint32_t)half + 128u * NSUB * (uint32_t)kvg;
+    const uint32_t fa = kPfFlag + 4u * (uint32_t)col + 128u * NSUB * (uint32_t)kvg;
 
     // exponents are in base 2: s becomes score * scale - (running maximum); seen is -inf until a column has met a token, then 0
     float neg_m = 0.f, seen = -INFINITY, l_run = 0.f;
@@ -314,10 +339,10 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         for (int e = 0; e < 16; e++) acc[db][e] = 0.f;
 
     // sub-unit u of the tile in buffer buf, u == NSUB: the first one of the next tile
-    constexpr int AHEAD = 4;
+    constexpr int AHEAD = FL ? 2 : 4;                                     // (FL: a step takes twice as long, and registers are short)
     auto k_load = [&](uint32_t buf, int u, int kk) PF_INLINE {
         const uint32_t at = ((u == NSUB ? buf ^ 1u : buf) * kPfBuf + (uint32_t)(u % NSUB) * (32u * ROWB)) / 16;
-        return __builtin_bit_cast(half8, ((lds_u4_ptr)(uintptr_t)ka[kk])[at]);
+        return __builtin_bit_cast(half8, ((lds_u4_ptr)(uintptr_t)(LEAN ? ka0 ^ ((uint32_t)kk << 5) : ka[kk]))[at]);
     };
     auto v_load = [&](uint32_t buf, int u, int i) PF_INLINE {             // operand i: tokens 16 (i / DB) .. + 15, d block i % DB
         typedef short4v __attribute__((address_space(3))) *lds_s4;
@@ -334,12 +359,34 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         const uint32_t at = (kPfScaleV + buf * 512u + 128u * (uint32_t)u + 32u * i) / 16;
         return __builtin_bit_cast(float4v, ((lds_u4_ptr)(uintptr_t)sa)[at]);
     };
+    // FL: the flags of the lane's K row, shifted to the chunks the lane holds
+    auto f_load = [&](uint32_t buf, int u) PF_INLINE {
+        const uint32_t at = ((u == NSUB ? buf ^ 1u : buf) * 512u + 128u * (uint32_t)(u % NSUB)) / 4;
+        return ((const uint32_t __attribute__((address_space(3))) *)(uintptr_t)fa)[at] >> (2 * half);
+    };
+    // One step of the scores.  FL: flagged chunks hold their verbatim values, the others codeword * radius code; the operand is
+    // split by chunk, and the two sums meet in maxima, the token's scale on the second.
+    auto score_step = [&](half8 k8, int kk, uint32_t flags, float16v &sn, float16v &svn) PF_INLINE {
+        if (FL) {
+            const uint4v w = __builtin_bit_cast(uint4v, k8);
+            const uint32_t m0 = (uint32_t)__builtin_amdgcn_sbfe((int)flags, 4 * kk, 1), m1 = (uint32_t)__builtin_amdgcn_sbfe((int)flags, 4 * kk + 1, 1);
+            const uint4v verb = uint4v{w[0] & m0, w[1] & m0, w[2] & m1, w[3] & m1};
+            const uint4v code = uint4v{w[0] & ~m0, w[1] & ~m0, w[2] & ~m1, w[3] & ~m1};
+            sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, code), qf[kk], sn, 0, 0, 0);
+            svn = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, verb), qf[kk], svn, 0, 0, 0);
+        } else sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(k8, qf[kk], sn, 0, 0, 0);
+    };
+    // FL: rows 8 x + 4 half .. + 3 of a unit's scores, relative to the running maximum: the codes' part times the token's scale
+    auto join = [&](int x, float16v &sn, const float16v &svn, float4v ks) PF_INLINE {
+#pragma unroll
+        for (int e = 4 * x; e < 4 * x + 4; e++) sn[e] = __builtin_fmaf(sn[e], ks[e & 3], __builtin_fmaf(svn[e], p.c_plain, neg_m));
+    };
     // scores of a unit (first token tw): times their K scale, relative to the running maximum, which moves if it has to
     auto maxima = [&](int tw, const float4v (&ks)[4]) PF_INLINE {
         const bool edge = !(tw + 32 <= wave_min && tw + 32 <= b_end && tw >= col_start);
         float tmax = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < 16; e++) s[e] = __builtin_fmaf(s[e], FL ? p.c_plain : ks[e >> 2][e & 3], neg_m);
+        for (int e = 0; e < 16 && !FL; e++) s[e] = __builtin_fmaf(s[e], ks[e >> 2][e & 3], neg_m);
         if (edge) {
 #pragma unroll
             for (int e = 0; e < 16; e++) {
@@ -371,17 +418,19 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     // One unit of 32 tokens.  In program order, one matrix instruction at a time with vector work behind it:
     //   S^T of the next unit, with the exponentials of this one; O^T += V^T . P^T of this one, with the decoding.
     half8 kf[AHEAD];                                                      // operands of the next unit's first products
+    uint32_t kfl = 0u;                                                    // and its flags
     auto unit = [&](int tw, uint32_t buf, int u) PF_INLINE {
+        if (LEAN) asm volatile("" : "+v"(ka0));                         // (or all eight addresses would be kept)
         constexpr int NV = 2 * DB, PER = 8 / KS;               // pairs of exponentials per matrix instruction
         const bool dec = u == NSUB - 1;
         half8 vf[AHEAD];
         float4v ks[4], vs[4];
-        float16v sn;
+        float16v sn, svn;
         float pe[2 * PER];
         uint32_t pp[8];
         if (FL && u == 0) entries(d_t - 2 * TILE);                        // of the tile decoded next
 #pragma unroll
-        for (int e = 0; e < 16; e++) sn[e] = 0.f;
+        for (int e = 0; e < 16; e++) sn[e] = svn[e] = 0.f;
         if (!FL) vs[0] = vs_load(buf, u, 0);
         auto finish = [&](int k) PF_INLINE {                              // the exponentials of step k: summed, times V's scale, packed
 #pragma unroll
@@ -395,7 +444,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
 #pragma unroll
         for (int k = 0; k < KS; k++) {
             __builtin_amdgcn_sched_barrier(0);
-            sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[k % AHEAD], qf[k], sn, 0, 0, 0);
+            score_step(kf[k % AHEAD], k, kfl, sn, svn);
             if (k + AHEAD < KS) kf[k % AHEAD] = k_load(buf, u + 1, k + AHEAD);
             else vf[k + AHEAD - KS] = v_load(buf, u, k + AHEAD - KS);
             if (k > 0) finish(k - 1);
@@ -405,6 +454,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         }
 #pragma unroll
         for (int i = 0; i < NV; i++) {
+            if (FL && i == 0 && NV / 2 - 2 == 0) ks[0] = s_load(buf, u + 1, 0);
             if (i == 0) finish(KS - 1);
             if (i > 0) __builtin_amdgcn_sched_barrier(0);
             const int st = i / DB, db = i % DB;
@@ -418,7 +468,11 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
                     d_t += TILE;
                 }
             }
-            if (!FL && i == NV / 2) {
+            if (FL) {                                                     // in registers no longer than needed
+                constexpr int J0 = NV / 2 - 2;
+                if (i >= J0 && i < J0 + 4) join(i - J0, sn, svn, ks[i - J0]);
+                if (i + 1 >= J0 && i + 1 < J0 + 4) ks[i + 1 - J0] = s_load(buf, u + 1, i + 1 - J0);
+            } else if (i == NV / 2) {
 #pragma unroll
                 for (int x = 0; x < 4; x++) ks[x] = s_load(buf, u + 1, x);
             }
@@ -428,6 +482,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         const bool over = u + 1 == NSUB;                                  // the next unit is the first one of the next tile
 #pragma unroll
         for (int i = 0; i < AHEAD; i++) kf[i] = k_load(over ? buf ^ 1u : buf, over ? 1 : u + 2, i);
+        if (FL) kfl = f_load(over ? buf ^ 1u : buf, over ? 1 : u + 2);
         maxima(over ? tw + 32 + TILE - 32 * NSUB : tw + 32, ks);
     };
     auto tile = [&](int t0, uint32_t buf) PF_INLINE {
@@ -440,13 +495,18 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     if (work) {
         float4v ks[4];
 #pragma unroll
-        for (int x = 0; x < 4 && !FL; x++) ks[x] = s_load(0u, 0, x);
+        for (int x = 0; x < 4; x++) ks[x] = s_load(0u, 0, x);
+        float16v sv0;
+        const uint32_t fl0 = FL ? f_load(0u, 0) : 0u;
 #pragma unroll
-        for (int e = 0; e < 16; e++) s[e] = 0.f;
+        for (int e = 0; e < 16; e++) s[e] = sv0[e] = 0.f;
 #pragma unroll
-        for (int kk = 0; kk < KS; kk++) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k_load(0u, 0, kk), qf[kk], s, 0, 0, 0);
+        for (int kk = 0; kk < KS; kk++) score_step(k_load(0u, 0, kk), kk, fl0, s, sv0);
+#pragma unroll
+        for (int x = 0; x < 4 && FL; x++) join(x, s, sv0, ks[x]);
 #pragma unroll
         for (int i = 0; i < AHEAD; i++) kf[i] = k_load(0u, 1, i);
+        if (FL) kfl = f_load(0u, 1);
         maxima(b_begin + 32 * NSUB * kvg, ks);
     }
     // (a wavefront whose columns end before the block's goes on with masked scores: it has to decode anyway)
@@ -523,14 +583,14 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
 }
 
 // Launch plan, from measured times in us: a tile takes a block of 128 columns 1.37, one of 256 columns 2.7 (all compute units
-// busy); starting (tables, first tiles) and finishing take a block 12; a compute unit holds one block; partials are written
+// busy), over outlier caches 1.75 and 3.5; starting (tables, first tiles) and finishing take a block 12; a compute unit holds one block; partials are written
 // and merged at 2 TB/s.
 struct PfPlan {
     bool wide;
     int splits;
     double us;
 };
-static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int causal, int64_t off, int fixed_splits) {
+static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int causal, int64_t off, int fixed_splits, bool flags) {
     const double last = causal ? std::max(1.0, std::min((double)Tkv, (double)off + Tq)) : std::max(Tkv, 1);      // tokens the last query sees
     const double mean = causal ? std::min(1.0, std::max(0.5, ((double)off + 0.5 * Tq) / last)) : 1.0;            // all, relative to it
     const int tiles = (int)((last * d_h + 8191) / 8192);
@@ -542,7 +602,7 @@ static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int ca
         for (int wide = 0; wide < 2; wide++) {
             const double rounds = (double)(((cols + (wide ? 255 : 127)) / (wide ? 256 : 128) * nz * s + 255) / 256);
             // the longest block or a compute unit's share of all of them, whichever is more; partials: written and read at 3 TB/s
-            const double us = std::max(1.0, mean * rounds) * ((tiles + s - 1) / s) * (wide ? 2.7 : 1.37) + 12.0 * rounds +
+            const double us = std::max(1.0, mean * rounds) * ((tiles + s - 1) / s) * (flags ? (wide ? 3.5 : 1.75) : wide ? 2.7 : 1.37) + 12.0 * rounds +
                               (s > 1 ? 5.0 + (double)(cols * nz) * s * (d_h + 4) * 8 / 2e6 : 0.0);
             if (us < best.us) best = PfPlan{wide != 0, s, us};
         }
@@ -557,7 +617,7 @@ static bool attn_prefill_takes(const hqmq_attn_args *a) {
     if (a->main_bits != 16 && (a->main_bits != 12 || a->aux_bits < 1)) return false;
     if (a->idx_bits < 6 || a->aux_bits > 4) return false;                          // the 16-bit decode needs radius codes below 1024
     if (a->t_cap % 64 || a->t_cap >= (1 << 25)) return false;                      // rows are addressed by 32-bit offsets
-    if (kPfTab + ((size_t)a->K.K + a->V.K) * 8 + 128 > 160 * 1024) return false;
+    if (pf_tab(a->K.flag_plane || a->V.flag_plane) + ((size_t)a->K.K + a->V.K) * 8 + 128 > 160 * 1024) return false;
     if (a->K.flag_plane || a->V.flag_plane) {
         if (a->dtype != HQMQ_F16) return false;                                   // verbatim bf16 chunks need not fit fp16
         const hqmq_packed *kv[2] = {&a->K, &a->V};
@@ -583,11 +643,10 @@ static double fast_us(int64_t cols, int64_t nz, int Tkv, int d_h, int splits, bo
 int attn_prefill_splits(const hqmq_attn_args *a, int splits) {
     const int64_t cols = (int64_t)a->T_q * (a->H_q / a->H_kv), nz = (int64_t)a->B * a->H_kv;
     if (cols < 64 || !attn_prefill_takes(a)) return 0;
-    const PfPlan plan = pf_plan(cols, nz, a->T_q, a->T_kv, 4 * a->n_chunks, a->causal, a->causal_offset, splits);
+    const PfPlan plan = pf_plan(cols, nz, a->T_q, a->T_kv, 4 * a->n_chunks, a->causal, a->causal_offset, splits, a->K.flag_plane != nullptr);
     const int other = splits > 0 ? splits : hqmq_attn_pick_splits(a->B, a->H_q, a->H_kv, a->T_q, a->T_kv, a->kv_len != nullptr);
-    // Outlier caches of three radius bits: most radius codes are 1, 2 or 4, with which the decode kernels' codeword * radius code is
-    // exact, and a value rounded once is up to 16 % further from 64-bit results (s24_r3, lognormal channels; s96 and s192 are 5 %
-    // nearer on average): they keep those kernels.
+    // Outlier caches of three radius bits keep the decode kernels: most radius codes are 1, 2 or 4, with which those kernels' V is
+    // exact, and V rounded as a value left lognormal channels 0.5 % further from 64-bit results (s24_r3; 6 % nearer on average).
     if (a->K.flag_plane && a->qmax < 15 && a->force_generic != 3) return 0;
     return a->force_generic == 3 || plan.us < 0.85 * fast_us(cols, nz, a->T_kv, 4 * a->n_chunks, other, a->K.flag_plane != nullptr) ? plan.splits : 0;
 }
@@ -595,7 +654,7 @@ int attn_prefill_splits(const hqmq_attn_args *a, int splits) {
 template <int DH, int MB, bool AUX, int DT, bool FL>
 static int launch_pf(const AttnParams &p, hipStream_t st, const LaunchTiming &tm) {
     const int64_t cols = (int64_t)p.Tq * p.G, nz = (int64_t)p.B * p.Hkv * p.n_splits;
-    const bool wide = pf_plan(cols, (int64_t)p.B * p.Hkv, p.Tq, p.Tkv, DH, p.causal, p.causal_offset, p.n_splits).wide;
+    const bool wide = pf_plan(cols, (int64_t)p.B * p.Hkv, p.Tq, p.Tkv, DH, p.causal, p.causal_offset, p.n_splits, FL).wide;
     const int64_t gx = (cols + (wide ? 255 : 127)) / (wide ? 256 : 128);
     // Column blocks per block, one after the other (the tables stay in LDS): as few rounds of 256 blocks as possible.  Ragged
     // batches leave the choice of the next block to the hardware.
@@ -608,7 +667,7 @@ static int launch_pf(const AttnParams &p, hipStream_t st, const LaunchTiming &tm
         }
     }
     if (rows * nz > 0x7fffffff) return HQMQ_ERR_SHAPE;
-    const size_t shmem = kPfTab + (size_t)((p.Kc.K * 8 + 127) & ~127) + (size_t)p.Vc.K * 8;
+    const size_t shmem = pf_tab(FL) + (size_t)((p.Kc.K * 8 + 127) & ~127) + (size_t)p.Vc.K * 8;
     auto kern = wide ? attn_prefill_kernel<DH, MB, AUX, DT, 1, FL> : attn_prefill_kernel<DH, MB, AUX, DT, 2, FL>;
     const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     if (e != hipSuccess) return (int)e;

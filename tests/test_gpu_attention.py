@@ -800,3 +800,54 @@ def test_unpacked_codes_at_odd_sizes(d_h, T, S, b_r, dn, odd):
         assert bit_equal(ops.dequant(*t, qmax), want)
     O = hqmq.fused_attention(Q.to(DEV), *dev[0], *dev[1], r_qmax=qmax, causal=False)
     assert_close(O, CO.attention_dense(Q, dense[0], dense[1], causal=False), dt, 1e-3 if dn == "fp32" else 2e-3)
+
+
+@pytest.mark.parametrize("S,b_r,d_h", [(96, 4, 128), (192, 6, 128), (96, 4, 64)])
+@pytest.mark.parametrize("magnitude", [30.0, 1.0, 1e-3, 1e-4, 3e-5])
+def test_prefill_over_outlier_caches_keeps_small_keys(S, b_r, d_h, magnitude):
+    """fp16 outlier caches in chunked prefill, K of every magnitude (queries the other way, so that scores are of order one), against
+    64-bit results: no further off than the decode kernels.  K is rounded as there.  V is rounded for every radius code, there for
+    the codes that are no power of two, at four bits 15 instead of 11 of 15: sqrt(15 / 11) on V's part, which is half of the
+    variance at most, so sqrt(1 + 2 / 11) = 1.087 in all if nothing else were better."""
+    import hqmq
+    dt = torch.float16
+    B, Hq, Hkv, T, Tq = 2, 8, 2, 700, 96
+    k = (kv_input((B, Hkv, T, d_h), torch.float32, 61, outlier_p=0.01, outlier_gain=(4, 9)) * magnitude).to(dt).to(DEV)
+    v = kv_input((B, Hkv, T, d_h), dt, 62, outlier_p=0.01, outlier_gain=(4, 9)).to(DEV)
+    Q = (torch.randn(B, Hq, Tq, d_h, generator=torch.Generator().manual_seed(63)) / magnitude).clamp(-6e4, 6e4).to(dt).to(DEV)
+    w = hqmq.with_outlier_extraction(hqmq.HQMQ(n_layers=1, n_heads=Hkv, secondary_size=S, radius_bits=b_r, device=DEV), C=3.0)
+    cache = w.new_cache(B, T, d_h, dt, 0)
+    w.append(cache, k, v, 0)
+    dense = []
+    for x, c in ((k, w.encode_K(k, 0)), (v, w.encode_V(v, 0))):
+        J, heads = c["joint"].double(), torch.arange(Hkv, device=DEV).view(1, Hkv, 1, 1)
+        y = J[heads, c["idx"].long()] * (c["rq"].double() * c["r_max"].double().unsqueeze(-1) / (2 ** b_r - 1)).unsqueeze(-1)
+        dense.append(torch.where(c["mask"].unsqueeze(-1), x.double().view(y.shape), y).reshape(B, Hkv, T, d_h).repeat_interleave(Hq // Hkv, 1))
+        assert int(c["mask"].sum()) > 50
+    K, V = dense
+    s = torch.matmul(Q.double(), K.transpose(2, 3).contiguous()) * d_h ** -0.5
+    seen = torch.arange(T, device=DEV).view(1, T) <= torch.arange(Tq, device=DEV).view(Tq, 1) + T - Tq
+    ref = torch.matmul(torch.softmax(s.masked_fill(~seen, float("-inf")), -1), V)
+    err = [float((hqmq.fused_attention_packed(Q, cache, causal=True, causal_offset=T - Tq, force_generic=f).double() - ref).norm() / ref.norm()) for f in (2, 3)]
+    assert err[1] <= 1.087 * err[0], f"prefill {err[1]:.3e}, decode kernels {err[0]:.3e}"
+
+
+def test_prefill_over_outlier_caches_with_unusual_scales():
+    """Tokens whose scale is 0, subnormal or (K, a norm beyond fp16) infinite beside ordinary ones: queries that do not see the last
+    kind get the decode kernels' results, verbatim chunks of their neighbours included."""
+    import hqmq
+    dt = torch.float16
+    B, Hq, Hkv, T, d_h = 1, 8, 2, 400, 128
+    k, v = kv_input((B, Hkv, T, d_h), dt, 71, outlier_p=0.03, outlier_gain=(5, 20)), kv_input((B, Hkv, T, d_h), dt, 72, outlier_p=0.03)
+    k[:, :, 40:44], v[:, :, 41:46] = 0, 0
+    k[:, :, 100], v[:, :, 101] = k[:, :, 100] * 1e-6, v[:, :, 101] * 1e-6
+    k[:, :, 392:394, :4] = 50000.0
+    w = hqmq.with_outlier_extraction(hqmq.HQMQ(n_layers=1, n_heads=Hkv, secondary_size=96, radius_bits=4, device=DEV), C=3.0)
+    cache = w.new_cache(B, T, d_h, dt, 0)
+    w.append(cache, k.to(DEV), v.to(DEV), 0)
+    assert bool(torch.isinf(cache.K.scale).any()) and float(cache.V.scale[:, :, 41].max()) < 1e-7
+    Q = torch.randn(B, Hq, 300, d_h, generator=torch.Generator().manual_seed(73)).to(dt).to(DEV)
+    for offset in (92, 91):                               # the last query sees token 391 / 390
+        a, b = (hqmq.fused_attention_packed(Q, cache, causal=True, causal_offset=offset, force_generic=f).float() for f in (2, 3))
+        assert torch.isfinite(a).all() and torch.isfinite(b).all()
+        assert (a - b).abs().max().item() < 2e-3 * max(1.0, float(a.abs().max()))
