@@ -27,19 +27,22 @@ def test_threshold_at_the_edges(dn, shape):
 
 @pytest.mark.parametrize("dn", ["fp16", "bf16"])
 def test_wide_and_packed_counters_agree(dn):
-    """A head of 5 M chunks (32-bit counters) and the order statistics of torch.sort on its norms."""
+    """6.3 M chunks of one head (512 blocks, packed counters) and the same five times over (31 M: 256 blocks of 122880, beyond what
+    16 bits count).  The two middle norms are equal, which the counts on either side show, so whatever the interpolation the
+    median is that norm in both calls, the threshold is equal and the count five times."""
     from hqmq_amd import ops
     dt = DT[dn]
-    x = torch.randn(5, 1, 32768, 128, generator=torch.Generator(device=DEV).manual_seed(3), device=DEV).to(dt)
-    med, thr, cnt = ops.med3x_threshold(x, 1.5)
-    mask = ops.outlier_mask(x, thr)
-    assert int(mask.sum()) == int(cnt[0])
-    below, above = int((~ops.outlier_mask(x, med.to(dt))).sum()), int(ops.outlier_mask(x, med.to(dt)).sum())
-    n = mask.numel()
-    assert above <= n // 2 and below >= n // 2                   # the median is a norm of the call: at most half lie above it
-    a, b = ops.med3x_threshold(x[:1], 1.5), ops.med3x_threshold(torch.cat([x[:1]] * 5), 1.5)      # the same norms five times over
-    assert float(a[1]) == float(b[1]) or abs(float(a[0]) - float(b[0])) < 1e-2 * float(a[0])
-    assert 5 * int(a[2]) == int(b[2]) or float(a[1]) != float(b[1])
+    x = torch.randn(1, 1, 49152, 512, generator=torch.Generator(device=DEV).manual_seed(3), device=DEV).to(dt)
+    five = x.expand(5, -1, -1, -1).contiguous()
+    n = x.numel() // 4
+    assert n * 5 / 512 > 60000 and n / 512 < 60000               # the launch's rule for the counters
+    (med, thr, cnt), (med5, thr5, cnt5) = ops.med3x_threshold(x, 1.5), ops.med3x_threshold(five, 1.5)
+    m = med.to(dt)
+    assert torch.equal(m.float(), med.float())                   # a norm of the call
+    above, from_it = int(ops.outlier_mask(x, m).sum()), int(ops.outlier_mask(x, (m.view(torch.int16) - 1).view(dt)).sum())
+    assert above < n // 2 < from_it                              # norms > median, norms >= median
+    assert torch.equal(med, med5) and bit_equal(thr, thr5)
+    assert int(ops.outlier_mask(x, thr).sum()) == int(cnt[0]) > 0 and int(cnt5[0]) == 5 * int(cnt[0])
 
 
 @pytest.mark.parametrize("dn,d_h", [("fp16", 128), ("bf16", 64), ("fp32", 48), ("fp16", 16)])
