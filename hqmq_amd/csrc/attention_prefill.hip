@@ -36,8 +36,9 @@
 // values only in tokens with verbatim chunks, in units of a power of two: 0.80 and 0.107, still up to 1.11.)  Error against 64-bit
 // results relative to the decode kernels', 162 calls: K from 3e-5 to 30 at V of order one 0.92 on average, 0.99 at most; V of 1e-4
 // 0.77 and 1.00, V of 3e-5, where outputs are fp16 subnormals, 0.81 and 1.08.
-// What bounds it (plain caches): a compute unit spends 36 % of the time in the matrix pipe, 50 % issuing vector instructions (a
-// quarter of them decode) and 46 % in LDS, at 2.0 to 2.1 GHz.
+// What bounds it: overlap, no pipe is full.  By the counters (profiles/attn_prefill_kernel_instruction_counters.txt) a compute unit
+// spends 37 % of its busy cycles in the matrix pipe, 50 % issuing vector instructions and 63 % in LDS, a third of that bank
+// conflicts (plain, 1024 on 32768), at 2.0 to 2.1 GHz; with verbatim chunks 37, 64 and 40 %; 2048 on 2048 causal 21, 51 and 38 %.
 #include "attention_mfma.h"
 #include <algorithm>
 
@@ -583,8 +584,8 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
 }
 
 // Launch plan, from measured times in us: a tile takes a block of 128 columns 1.37, one of 256 columns 2.7 (all compute units
-// busy), over outlier caches 1.75 and 3.5; starting (tables, first tiles) and finishing take a block 12; a compute unit holds one block; partials are written
-// and merged at 2 TB/s.
+// busy), over outlier caches 1.75 and 3.5; starting (tables, first tiles) and finishing take a block 12; a compute unit holds one
+// block; partials are written and merged at 2 TB/s.
 struct PfPlan {
     bool wide;
     int splits;
@@ -601,7 +602,7 @@ static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int ca
         if (i > 0 && s > tiles / 2) break;
         for (int wide = 0; wide < 2; wide++) {
             const double rounds = (double)(((cols + (wide ? 255 : 127)) / (wide ? 256 : 128) * nz * s + 255) / 256);
-            // the longest block or a compute unit's share of all of them, whichever is more; partials: written and read at 3 TB/s
+            // the longest block or a compute unit's share of all of them, whichever is more; partials: written and read at 2 TB/s
             const double us = std::max(1.0, mean * rounds) * ((tiles + s - 1) / s) * (flags ? (wide ? 3.5 : 1.75) : wide ? 2.7 : 1.37) + 12.0 * rounds +
                               (s > 1 ? 5.0 + (double)(cols * nz) * s * (d_h + 4) * 8 / 2e6 : 0.0);
             if (us < best.us) best = PfPlan{wide != 0, s, us};

@@ -26,9 +26,10 @@
 // fp32) or 371 KB (bf16) at every S.  Behind the lists of all heads lies what only the build reads and a caller may drop
 // afterwards (hqmq_search_grid_kept_bytes): the pools' counters, the centres and radii of the codewords.
 //
-// What it costs: per wavefront of 64 chunks about 330 vector-ALU instructions (180 for norm, division, nearest unit and
-// box, 11 per list entry, 60 - 80 for scale, radius code and packing) where the scan over 96 secondaries takes 1,885.
-// Bound by vector-ALU issue and the LDS gathers of the table rows.  K and V of 8 x 32768 tokens, fp16, s96_r4, packed:
+// What it costs: per 64 chunks 342 vector-ALU instructions at fp16 s96_r4, 450 at bf16 s24_r3 with flags (180 for norm,
+// division, nearest unit and box, 11 per list entry, 60 - 80 for scale, radius code and packing) where the scan over 96
+// secondaries takes 1,885.  Bound by vector-ALU issue: 0.89 and 0.90 of the cycles a compute unit is busy, its LDS pipe 24
+// and 19 % (profiles/quantize_grid_kernel_instruction_counters.txt).  K and V of 8 x 32768 tokens, fp16, s96_r4, packed:
 // 792 -> 189 us; 8 x 4 x 4001 tokens bf16 s24_r3 with flags 371 -> 128 us; one tensor of 8 x 2048 tokens s192_r6,
 // fake-quant output: 51 -> 11 us.  40 boxes per axis instead of 32 shorten the lists by a fifth and bought 3 %.
 //
