@@ -324,7 +324,10 @@ __device__ __forceinline__ void quantize_body(const QParams &a) {
     }
 
     ChunkSink<D, kQThreads, ROWS, kUnpacked | kPlanes | kCompact, 0> sink(a, b, h, tok_local, c, code_sh, aux_sh);
-    sink.put(blockIdx.x * a.tokens_per_block, active && writer, raw, nrm, r, idx, jh + (size_t)idx * 4);
+    auto row = [&](float (&g)[4]) {
+        for (int j = 0; j < 4; j++) g[j] = D::load(jh + (size_t)idx * 4 + j);
+    };
+    sink.put(blockIdx.x * a.tokens_per_block, active && writer, raw, nrm, r, idx, row, std::false_type());
     sink.done();
 }
 

@@ -5,6 +5,8 @@
 #pragma once
 #include "common.h"
 
+#include <type_traits>
+
 namespace hqmq {
 
 constexpr int kQThreads = 256;   // short appends: all new rows of a (b, h) in one block of this many lanes
@@ -73,6 +75,7 @@ struct QParams {
 };
 struct QPair {
     QParams p[2];               // K, V: blockIdx.z picks one
+    int per_head;               // cell-list kernel, long calls: blocks per tensor, b and h
 };
 
 // The four stored elements of a chunk, as they are in memory.
@@ -192,6 +195,7 @@ struct ChunkSink {
     int b, h, tok_local, c;
     uint32_t *code_sh, *aux_sh;     // NT words of LDS each (aux_sh: without ROWS, with compaction, or n = 4)
     int64_t bh, row0;               // row0: the plane row of token 0
+    int t_lo, t_hi;                 // this lane's rows of the planes are those of rounds t_lo <= t0 < t_hi
     float thr, qmaxf, inv_qmax;
     uint32_t seen = 0;              // the largest finite scale this lane has written so far, as bits
 
@@ -199,27 +203,33 @@ struct ChunkSink {
         : a(a_), b(b_), h(h_), tok_local(tok_local_), c(c_), code_sh(code_sh_), aux_sh(aux_sh_) {
         bh = (int64_t)b * a.H + h;
         row0 = (WHAT & kPlanes) ? (int64_t)(a.pos ? a.pos[b] : 0) + a.t_off : 0;
+        if (WHAT & kPlanes) {       // (a bad pos[] must not write outside the plane)
+            const int64_t lo = -(row0 + tok_local), hi = a.t_cap + lo;
+            t_lo = (int)(lo < 0 ? 0 : lo > INT32_MAX ? INT32_MAX : lo);
+            t_hi = (int)(hi < 0 ? 0 : hi > INT32_MAX ? INT32_MAX : hi);
+        }
         thr = a.thr ? D::load((const ST *)a.thr + h) : INFINITY;
         qmaxf = (float)a.qmax;
         inv_qmax = __builtin_amdgcn_rcpf(qmaxf);
     }
 
-    __device__ __forceinline__ void put(int t0, bool active, const RawChunk<D> &raw, float nrm, float r, int idx, const ST *jrow) {
+    // jrow(g): the chunk's row of the joint table.  QUICK (std::true_type): every norm of the wavefront is an ordinary number of
+    // a 16-bit type (quick_divisor), at or above the clamp.
+    template <class ROW, class QUICK>
+    __device__ __forceinline__ void put(int t0, bool active, const RawChunk<D> &raw, float nrm, float r, int idx, ROW jrow, QUICK) {
+        constexpr bool quick = QUICK::value;
         const int tid = threadIdx.x, n = a.n, lane = tid & 63;
         const int lane_base = ROWS ? (lane & ~(n - 1)) : 0;
         const uint64_t tok_lanes = n >= 64 ? ~0ull : ((1ull << n) - 1ull) << lane_base;      // ROWS only
         // ---- per-token scale and radius code ----
         float rm = -INFINITY;
-        bool rm_nan = false;
         if (ROWS) {
-            const uint64_t nans = __builtin_amdgcn_ballot_w64(is_nan(r));
-            rm = r;
-            if (nans) {
-                rm_nan = (nans & tok_lanes) != 0ull;
-                rm = is_nan(r) ? -INFINITY : r;
-            }
-            rm = group_max(rm, n, [](float p, float q) { return q > p ? q : p; });
+            // norms are not negative, so their bits order like the values, with NaN (made the positive one) above all others
+            uint32_t bits = __float_as_uint(r);
+            if (!quick) bits = is_nan(r) ? 0x7fc00000u : bits;
+            rm = __uint_as_float(group_max(bits, n, [](uint32_t p, uint32_t q) { return max(p, q); }));
         } else {
+            bool rm_nan = false;
             float *radius_sh = reinterpret_cast<float *>(aux_sh);
             __syncthreads();
             radius_sh[tid] = r;
@@ -231,13 +241,16 @@ struct ChunkSink {
                 else if (o > rm) rm = o;
             }
             __syncthreads();
+            if (rm_nan) rm = NAN;
         }
-        rm = clamp_min_d<D>(rm_nan ? NAN : rm, 1e-8f);
-        const bool quick = D::code != HQMQ_F32 && __builtin_amdgcn_ballot_w64(!quick_divisor<D>(rm)) == 0ull;       // qmax divides it: at most 255
-        const float scale = quick ? quick_div<D>(rm, qmaxf, inv_qmax) : D::rnd(rm / qmaxf);
-        float qf = rintf(div_d<D>(r, scale));
-        if (!is_nan(qf)) qf = fminf(fmaxf(qf, 0.f), qmaxf);
-        const int rq = is_nan(qf) ? 0 : (int)qf;
+        if (!quick) rm = clamp_min_d<D>(rm, 1e-8f);
+        float scale, qf;
+        if (D::code != HQMQ_F32 && (quick || __builtin_amdgcn_ballot_w64(!quick_divisor<D>(rm)) == 0ull)) scale = quick_div<D>(rm, qmaxf, inv_qmax);      // qmax: at most 255
+        else scale = D::rnd(rm / qmaxf);
+        qf = rintf(div_d<D>(r, scale));
+        if (quick) qf = fminf(qf, qmaxf);
+        else if (!is_nan(qf)) qf = fminf(fmaxf(qf, 0.f), qmaxf);
+        const int rq = !quick && is_nan(qf) ? 0 : (int)qf;
         const bool flagged = nrm > thr;
 
         if ((WHAT & kUnpacked) && active) {
@@ -250,8 +263,10 @@ struct ChunkSink {
                 RawChunk<D> dst = raw;                   // a flagged chunk comes out as it went in
                 if (!flagged) {
                     const float rqs = D::rnd(qf * scale);
+                    float g[4];
+                    jrow(g);
 #pragma unroll
-                    for (int j = 0; j < 4; j++) dst.set(j, D::rnd(rqs * D::load(jrow + j)));
+                    for (int j = 0; j < 4; j++) dst.set(j, D::rnd(rqs * g[j]));
                 }
                 dst.store((ST *)a.dense_out + tok * n * 4 + tid * 4, a.vec_out);
             }
@@ -261,7 +276,7 @@ struct ChunkSink {
 
         // ---- packed rows ----
         const int64_t row = row0 + t0 + tok_local;
-        const bool row_ok = active && row >= 0 && row < a.t_cap;  // a bad pos[] must not write outside the plane
+        const bool row_ok = active && t0 >= t_lo && t0 < t_hi;
         // Sideband compaction in the same launch, for appends whose new rows of a (b, h) all sit in this block
         // (T <= tokens_per_block; n a power of two, so the lanes of a token share a wavefront).  Entries, tile
         // offsets and counters come out as the in-order compaction kernel leaves them: flagged chunks in

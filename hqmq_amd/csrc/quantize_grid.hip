@@ -1,79 +1,71 @@
 // Codeword search through cell lists.
 //
 // The codebook {q_p * q_s} is closed under left multiplication by the 24 Hurwitz units, and so is the score:
-// <u, q_p * q_s> = <conj(q_g) * u, (conj(q_g) * q_p) * q_s> for every unit q_g.  Multiplying a direction u by the
-// conjugate of its nearest unit q_g brings it into the cell of S^3 around 1, where w0 is the largest scalar part:
-// w = conj(q_g) * u has |w1| + |w2| + |w3| <= w0, i.e. y = (w1, w2, w3) / w0 lies in the octahedron |y|_1 <= 1.  Only
-// 1 / 24 of the directions are left to be searched, and every codebook of S secondaries has about S codewords there.
-// A grid of kGrid^3 boxes over [-1, 1]^3 (those that meet the octahedron) carries, per box, the list of all codewords
-// (p', s) that can win the reference's rounded comparison for some direction inside it; the lists are worked out once
-// per codebook (hqmq_build_search_grid).  A search is then: nearest unit, one quaternion product, one list look-up,
-// and the reference's own rounded score (bit for bit) for the few codewords of the list; the largest score wins, the
-// smallest index k = p * S + s among equals.
+// <u, q_p * q_s> = <conj(e) * u, (conj(e) * q_p) * q_s> for every unit e.  Eight of the units are the axes {+-1, +-i, +-j,
+// +-k}: multiplying a direction u by the conjugate of the axis nearest to it (its component of largest magnitude) permutes
+// its components and changes signs, no more, and brings it into the cell of S^3 around 1, |w_i| <= w0.  Only 1 / 8 of the
+// directions are left to be searched.  Seen in stereographic projection, z = (w1, w2, w3) / (w0 + 1), that cell almost
+// fills the cube |z_i| <= sqrt(2) - 1, and equal boxes of the cube are nearly equal pieces of the sphere (the scale goes
+// from 2 to 1.5).  A grid of kGrid^3 boxes over the cube carries, per box, the list of all codewords (p', s) that can win
+// the reference's rounded comparison for some direction inside it; the lists are worked out once per codebook
+// (hqmq_build_search_grid).  A search is then: the largest component, one reciprocal, one list look-up, and the
+// reference's own rounded score (bit for bit) for the few codewords of the list; the largest score wins, the smallest index
+// k = p * S + s among equals.
 //
-// The reference scores with the stored table J, whose rows are rounded products: conj(q_g) * J[k] depends on g.  A
-// codeword (p', s) therefore stands for 24 points, taken as a centre and the radius rho of the ball around it.
+// The box is found without carrying out the multiplication: two packed multiply-adds put the positions t_j of u's four
+// components into 16-bit halves, and since w is u with components exchanged and signs changed, the box number is a sum of
+// +-1, +-kGrid, +-kGrid^2 times three of them - two dot products with constants that belong to the axis.  kGrid is odd, so
+// rounding to the nearest box commutes with a change of sign.
+//
+// The reference scores with the stored table J, whose rows are rounded products: conj(e) * J[k] depends on e.  A
+// codeword (p', s) therefore stands for 8 points, taken as a centre and the radius rho of the ball around it.
 // A codeword g is left out of a box when some codeword g* beats it by more than any rounding can turn, everywhere in
-// the box: <(1, y), g* - g> > (rho_g + rho_g* + m) |(1, y)|.  The left side is linear in y, so its minimum over the box
-// is the value at the centre less half the box's width times |g*_i - g_i| summed over the three coordinates; |(1, y)| is
-// largest in the corner farthest from 0.  m covers the roundings of the two scores to D: half a unit in the last place
-// each, 2^-12 (fp16) and 2^-9 (bf16) for scores in [0.5, 1), twice that where a score can reach 1 (directions are
-// vectors of length 1 within 1.5 %; others are scored against all rows).
+// the box: <(1 - |z|^2, 2 z), g* - g> > (rho_g + rho_g* + m) (1 + |z|^2).  That is one parabola per coordinate, so its
+// least value in the box is three least values on an interval.  g* is the best codeword at the box's centre, then every
+// other one of the box's list.  m covers the roundings of the two scores to D: half a unit in the last place each, 2^-12
+// (fp16) and 2^-9 (bf16) for scores in [0.5, 1), twice that where a score can reach 1 (directions are vectors of length 1
+// within 1.5 %; others are scored against all rows).
 //
-// Lists, per head, in blocks of 16 bytes: seven 16-bit entries p' << 2 | s' << 7 (s' = S - 1 - s; p' = 31: no entry) and
-// the number of the block that goes on (0: none, 0xffff: no list, score all rows).  The first kCells blocks are the
-// boxes', the others a pool that the build hands out; block 0 of the pool holds no entry.  That is 185 KB per head (fp16,
-// fp32) or 371 KB (bf16) at every S.  Behind the lists of all heads lies what only the build reads and a caller may drop
-// afterwards (hqmq_search_grid_kept_bytes): the pools' counters, the centres and radii of the codewords.
+// Lists, per head, in blocks of 16 bytes: seven 16-bit entries and the number of the block that goes on (0: none, 0xffff: no
+// list, score all rows).  An entry holds p' << 2 and bit 8 of s' = S - 1 - s in its lower byte, the other bits of s' in its
+// upper one (p' = 31: no entry): a byte is an operand of the vector unit, and the lower one, exclusive-or'ed with the axis,
+// is the address of the number of row q_e * q_p', 0.  The first kCells blocks are the boxes', the others a pool that the
+// build hands out; block 0 of the pool holds no entry.  That is 384 KB per head for fp16, fp32 and bf16 up to S = 32, for
+// bf16 615 KB up to S = 96, 922 KB up to 192 and 1230 KB above.  Behind the lists of all heads lies what only the build
+// reads and a caller may drop afterwards (hqmq_search_grid_kept_bytes): the pools' counters, the centres and radii of the
+// codewords.
 //
-// What it costs: per 64 chunks 342 vector-ALU instructions at fp16 s96_r4, 450 at bf16 s24_r3 with flags (180 for norm,
-// division, nearest unit and box, 11 per list entry, 60 - 80 for scale, radius code and packing) where the scan over 96
-// secondaries takes 1,885.  Bound by vector-ALU issue: 0.89 and 0.90 of the cycles a compute unit is busy, its LDS pipe 24
-// and 19 % (profiles/quantize_grid_kernel_instruction_counters.txt).  K and V of 8 x 32768 tokens, fp16, s96_r4, packed:
-// 792 -> 189 us; 8 x 4 x 4001 tokens bf16 s24_r3 with flags 371 -> 128 us; one tensor of 8 x 2048 tokens s192_r6,
-// fake-quant output: 51 -> 11 us.  40 boxes per axis instead of 32 shorten the lists by a fifth and bought 3 %.
+// What it costs: per 64 chunks 180 vector-ALU instructions at fp16 s96_r4, 249 at bf16 s24_r3 with flags, where the scan
+// over 96 secondaries takes 1,885.  Bound by vector-ALU issue: 0.82 (fp16) and 0.78 (bf16) of the cycles a compute unit is
+// busy, transcendental instructions counted once; its LDS pipe 33 %.  The form before this one reduced directions to the
+// cell of all 24 units (75 instructions for unit, quaternion product and box, where this takes 25), listed 3.35 codewords
+// per box on average (S = 96, fp16; 8.7 is the longest of 64) where this lists 3.1 (7.5), and rounded every 16-bit number
+// by itself: 342 and 450 instructions.  K and V of 8 x 32768 tokens, fp16, s96_r4, packed: 186 -> 123 us; 8 x 4 x 4001 tokens
+// bf16 s24_r3 with Med3x, whole call: 163 -> 117 us.  33 boxes per axis instead of 27 take 5 % fewer instructions, 1 % less
+// time and 1.8 times the memory; 27 without the comparison of all pairs: lists of 3.35 (9.3).
 //
 // Compiled with -ffp-contract=off; fused multiply-adds are written explicitly.
 #include "quantize_common.h"
 
+#include <type_traits>
+
 namespace hqmq {
 
-constexpr int kCoarse = 8;                      // boxes per axis of the build's first level
-constexpr int kFine = 4;                        // boxes per axis inside one of those
-constexpr int kGrid = kCoarse * kFine;
+constexpr int kCoarse = 9;                      // boxes per axis of the build's first level
+constexpr int kFine = 3;                        // boxes per axis inside one of those
+constexpr int kGrid = kCoarse * kFine;          // odd: a box's mirror image is a box
+constexpr int kMid = kGrid / 2;
+constexpr int kCells = kGrid * kGrid * kGrid;
 constexpr int kGridSMax = 341;                  // 24 * 341 rows of 8 bytes: row offsets fit 16 bits, s' fits 9
 constexpr uint32_t kNone = 31u << 2;            // an empty entry
-
-// Does box (i, j, k) of a grid of `g` boxes per axis meet the octahedron (a hair dilated: w is computed in fp32)?
-constexpr bool box_meets(int i, int j, int k, int g) {
-    auto dist = [g](int x) {                    // smallest |y| of the box, in units of 1 / g
-        const int lo = 2 * x - g, hi = lo + 2;
-        return lo > 0 ? lo : hi < 0 ? -hi : 0;
-    };
-    return 1000 * (dist(i) + dist(j) + dist(k)) <= 1001 * g;
-}
-struct GridMap {
-    int cells;
-    int16_t off[kGrid * kGrid];                 // box (i, j, k) has number off[i * kGrid + j] + k
-};
-constexpr GridMap make_map() {
-    GridMap m{};
-    int n = 0;
-    for (int i = 0; i < kGrid; i++)
-        for (int j = 0; j < kGrid; j++) {
-            int first = -1;
-            for (int k = 0; k < kGrid; k++)
-                if (box_meets(i, j, k, kGrid)) {
-                    if (first < 0) { first = k; m.off[i * kGrid + j] = (int16_t)(n - k); }
-                    n++;
-                }
-        }
-    m.cells = n;
-    return m;
-}
-constexpr GridMap kMap = make_map();
-constexpr int kCells = kMap.cells;
-static_assert(kCells < 32768, "box numbers are 16-bit");
+constexpr float kScale = (0.5f * kGrid - 0.1f) / 0.41422f;       // boxes per unit of z; the cell reaches |z_i| = sqrt(2) - 1
+// How far, in boxes, the position that the search computes may lie from the direction's own: the reciprocal and (fp32) the
+// components are rounded to fp16 (2^-11 of at most 13.4 each), w0 may be the unrounded quotient (fp16: half of 2^-11), and
+// the search takes 1 for the length of a direction whose norm and components were rounded to D (2^-10 and 2^-7, two thirds
+// of which reach z).
+template <class D>
+constexpr float slack_boxes() { return D::code == HQMQ_BF16 ? 0.085f : 0.022f; }
+static_assert(0.5f * kGrid - 0.1f + 0.085f < kMid + 0.5f, "every direction's box is inside the grid");
 
 constexpr float unit_part(int p, int j) {       // component j of Hurwitz unit p, in the order of the joint table
     return p < 8 ? (j == (p >> 1) ? ((p & 1) ? -1.f : 1.f) : 0.f) : (((p - 8) >> (3 - j)) & 1 ? -0.5f : 0.5f);
@@ -96,17 +88,47 @@ constexpr Units make_units() {
         }
     return t;
 }
-__device__ const GridMap d_map = make_map();
 __device__ const Units d_units = make_units();
 
-// Blocks of the pool: random codebooks take 1.05 blocks per box at most (bf16, S = 192; fp16 0.1).  A box that finds
-// the pool empty scores all rows.
-constexpr int64_t pool_blocks(int dtype) { return dtype == HQMQ_BF16 ? 2 * kCells : kCells / 2; }
-static_assert(2 * kCells < 65535, "block numbers are 16-bit");
+// What the search needs to know of a unit e of {+-1, +-i, +-j, +-k}: the box number of w = conj(e) * u from the positions
+// t_0 .. t_3 of u's components, 16 * (sum_j a_j t_j) + first, as two dot products of 16-bit numbers.  The positions come as
+// the bits of fp16 numbers 1536 + t, which is 0x6600 + t.
+struct AxisUnits {
+    uint32_t a01[8], a23[8];
+    int32_t first[8];
+};
+constexpr AxisUnits make_axis_units() {
+    AxisUnits t{};
+    const int stride[4] = {0, kGrid * kGrid, kGrid, 1};
+    for (int e = 0; e < 8; e++) {
+        int a[4] = {};
+        const float q[4] = {unit_part(e, 0), -unit_part(e, 1), -unit_part(e, 2), -unit_part(e, 3)};
+        for (int j = 0; j < 4; j++) {
+            float u[4] = {};
+            u[j] = 1.f;
+            const float w[4] = {q[0] * u[0] - q[1] * u[1] - q[2] * u[2] - q[3] * u[3], q[0] * u[1] + q[1] * u[0] + q[2] * u[3] - q[3] * u[2],
+                                q[0] * u[2] - q[1] * u[3] + q[2] * u[0] + q[3] * u[1], q[0] * u[3] + q[1] * u[2] - q[2] * u[1] + q[3] * u[0]};
+            for (int c = 1; c < 4; c++) a[j] += 16 * stride[c] * (int)w[c];
+        }
+        t.a01[e] = ((uint32_t)a[0] & 0xffffu) | (uint32_t)a[1] << 16;
+        t.a23[e] = ((uint32_t)a[2] & 0xffffu) | (uint32_t)a[3] << 16;
+        t.first[e] = 16 * kMid * (kGrid * kGrid + kGrid + 1) - 0x6600 * (a[0] + a[1] + a[2] + a[3]);
+    }
+    return t;
+}
+__device__ const AxisUnits d_axis = make_axis_units();
+static_assert(16 * kGrid * kGrid < 32768, "strides are 16-bit");
+
+// Blocks of the pool.  Random codebooks (16 heads each) take at most 19 / 214 / 929 / 2903 at S = 24 / 96 / 192 / 341 with
+// fp16, less with fp32, 190 / 7319 / 18733 / 33140 with bf16.  A box that finds the pool empty scores all rows.
+constexpr int64_t pool_blocks(int S, int dtype) {
+    return dtype != HQMQ_BF16 || S <= 32 ? kCells / 4 : S <= 96 ? kCells : S <= 192 ? 2 * kCells : 3 * kCells;
+}
+static_assert(3 * kCells < 65535, "block numbers are 16-bit");
 
 int64_t search_grid_blocks(int S, int dtype) {
     if (S < 1 || S > kGridSMax) return 0;
-    return kCells + pool_blocks(dtype);
+    return kCells + pool_blocks(S, dtype);
 }
 
 // ---------------------------------------------------------------- build
@@ -125,22 +147,22 @@ __device__ __forceinline__ float4 quat_mul(float4 a, float4 b) {
                   a.x * b.z - a.y * b.w + a.z * b.x + a.w * b.y, a.x * b.w + a.y * b.z - a.z * b.y + a.w * b.x};
 }
 
-// Centre and radius of the 24 points conj(q_g) * J[q_g * q_p', s] for every (p', s), 32 lanes per codeword (lane = g; the
-// last eight repeat g = 23); the head's counter and empty block.
+// Centre and radius of the 8 points conj(e) * J[e * q_p', s] for every (p', s), 8 lanes per codeword; the head's counter
+// and empty block.
 template <class D>
 __global__ __launch_bounds__(256) void grid_codewords_kernel(const typename D::storage *joint, int S, uint4 *grid, int64_t stride, int H) {
-    const int h = blockIdx.y, k = blockIdx.x * 8 + (threadIdx.x >> 5), g = min((int)threadIdx.x & 31, 23);
+    const int h = blockIdx.y, k = blockIdx.x * 32 + (threadIdx.x >> 3), g = threadIdx.x & 7;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         grid_counters(grid, stride, H)[h] = 1;
         grid[stride * h + kCells] = uint4{kNone | kNone << 16, kNone | kNone << 16, kNone | kNone << 16, kNone};
     }
-    if (k >= 24 * S) return;            // (24 S is a multiple of 8: whole blocks)
+    if (k >= 24 * S) return;            // (24 S is a multiple of 8: whole wavefronts)
     const int p = k / S, s = k - p * S;
     const typename D::storage *r = joint + ((size_t)h * 24 * S + (size_t)d_units.mul[g][p] * S + s) * 4;
     const float *q = d_units.q[g];
     const float4 v = quat_mul(float4{q[0], -q[1], -q[2], -q[3]}, float4{D::load(r), D::load(r + 1), D::load(r + 2), D::load(r + 3)});
     auto most = [](float x, auto op) {
-        for (int o = 16; o; o >>= 1) x = op(x, __shfl_xor(x, o, 32));
+        for (int o = 4; o; o >>= 1) x = op(x, __shfl_xor(x, o, 8));
         return x;
     };
     auto mid = [&](float x) {
@@ -151,67 +173,105 @@ __global__ __launch_bounds__(256) void grid_codewords_kernel(const typename D::s
     // (a NaN row makes the radius NaN: nothing is left out because of it, and it is left out nowhere)
     const float far = most(sqrtf(d0 * d0 + d1 * d1 + d2 * d2 + d3 * d3), [](float i, float j) { return i > j || is_nan(i) ? i : j; });
     const Codewords cw = grid_codewords(grid, stride, H, S);
-    if ((threadIdx.x & 31) == 0) {
+    if (g == 0) {
         cw.centre[(size_t)h * 24 * S + k] = c;
         cw.rho[(size_t)h * 24 * S + k] = far * 1.00001f + 1e-6f;
     }
 }
 
 // One block per coarse box and head.  First the codewords that matter anywhere in the coarse box are listed in LDS
-// (lanes over codewords), then the kFine^3 boxes inside it are worked out from that list, kLanes lanes per box: 248 x 4608
-// tests per head instead of 7728 x 4608.  kListCap bounds the coarse list (random codebooks: 30 - 250), kBoxCap a box's
-// (random codebooks: 48 at most); beyond either the box scores all rows.
+// (lanes over codewords), then the kFine^3 boxes inside it are worked out from that list, kLanes lanes per box, and every
+// listed codeword is held against every other one.  kListCap bounds the coarse list, kBoxCap a box's (random codebooks stay
+// far below both: no box of S = 24 ... 341 goes without a list); beyond either the box scores all rows.
 constexpr int kListCap = 1024;
 constexpr int kBoxCap = 126;
 constexpr int kBuildThreads = 256;
-constexpr int kLanes = kBuildThreads / (kFine * kFine * kFine);
-static_assert(kLanes == 4, "lanes per box");
+constexpr int kBoxes = kFine * kFine * kFine;
+constexpr int kLanes = 8;                       // per box
+static_assert(kBoxes * kLanes <= kBuildThreads && kLanes == 8, "lanes per box");
 template <class D>
 __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 *grid, int64_t stride, int pool, int H) {
     const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
     const int ci = blockIdx.x / (kCoarse * kCoarse), cj = blockIdx.x / kCoarse % kCoarse, ck = blockIdx.x % kCoarse;
-    if (!box_meets(ci, cj, ck, kCoarse)) return;
     __shared__ float4 geo[kListCap];
     __shared__ float rad[kListCap];
-    __shared__ uint16_t id[kListCap];
-    __shared__ uint16_t entries[kFine * kFine * kFine][kBoxCap + 1];
-    __shared__ int count[kFine * kFine * kFine];
+    __shared__ uint16_t id[kListCap];                          // as an entry
+    __shared__ uint16_t entries[kBoxes][kBoxCap + 1];          // positions in the coarse list
+    __shared__ uint8_t out[kBoxes][kBoxCap + 2];               // beaten by another codeword of the box
+    __shared__ int count[kBoxes];
     __shared__ float best_sh[kBuildThreads / 64];
     __shared__ int arg_sh[kBuildThreads / 64], n_sh;
     const int K = 24 * S;
     const Codewords all = grid_codewords(grid, stride, H, S);
     const float4 *centre = all.centre + (size_t)h * K;
     const float *rho = all.rho + (size_t)h * K;
-    struct Box { float y0, y1, y2, hw, longest, shortest; };             // centre, half width, |(1, y)| over the box
-    auto box_at = [](int i, int j, int k, int g) {
-        const float w = 2.f / (float)g, hw = 1.f / (float)g + 2e-5f;
-        Box b{((float)i + 0.5f) * w - 1.f, ((float)j + 0.5f) * w - 1.f, ((float)k + 0.5f) * w - 1.f, hw, 0.f, 0.f};
-        auto sq = [](float v) { return v * v; };
-        b.longest = sqrtf(1.f + sq(fabsf(b.y0) + hw) + sq(fabsf(b.y1) + hw) + sq(fabsf(b.y2) + hw)) * 1.00001f;
-        b.shortest = sqrtf(1.f + sq(fmaxf(fabsf(b.y0) - hw, 0.f)) + sq(fmaxf(fabsf(b.y1) - hw, 0.f)) + sq(fmaxf(fabsf(b.y2) - hw, 0.f))) * 0.99999f;
+    struct Box { float lo[3], hi[3]; float4 mid; float reach; bool met; };       // mid: the direction at its centre; reach: the farthest one's angle
+    auto box_at = [](int i, int j, int k, int fine) {           // fine: fine boxes per axis of this one
+        Box b;
+        const int at[3] = {i, j, k};
+        const float hw = (0.5f * (float)fine + slack_boxes<D>()) * (1.f / kScale) + 2e-6f;
+        float c[3], near2 = 0.f, mid2 = 0.f, near[3];
+        for (int a = 0; a < 3; a++) {
+            c[a] = ((float)(at[a] * fine - kMid) + 0.5f * (float)(fine - 1)) * (1.f / kScale);
+            b.lo[a] = c[a] - hw;
+            b.hi[a] = c[a] + hw;
+            near[a] = fmaxf(fabsf(c[a]) - hw, 0.f);
+            near2 += near[a] * near[a];
+            mid2 += c[a] * c[a];
+        }
+        // the cell: |w_i| <= w0, that is |z|^2 + 2 |z_i| <= 1
+        b.met = near2 + 2.f * fmaxf(near[0], fmaxf(near[1], near[2])) <= 1.0005f;
+        const float inv = 1.f / (1.f + mid2);
+        b.mid = float4{(1.f - mid2) * inv, 2.f * c[0] * inv, 2.f * c[1] * inv, 2.f * c[2] * inv};
+        b.reach = 2.f * 1.7321f * hw;
         return b;
     };
-    auto dot = [](float4 g, const Box &b) { return g.x + b.y0 * g.y + b.y1 * g.z + b.y2 * g.w; };
-    // what g* has to lead by, less the radii: the roundings of both scores, and of this kernel
-    auto rounding = [&](float4 star, float r, const Box &b) {
-        const float most = (dot(star, b) + b.hw * (fabsf(star.y) + fabsf(star.z) + fabsf(star.w))) / b.shortest + r;
-        return 1.016f * (most * 1.016f < 1.f ? 1.f : 2.f) * D::eps() + 1.2e-5f;
+    auto dot = [](float4 g, float4 m) { return g.x * m.x + g.y * m.y + g.z * m.z + g.w * m.w; };
+    // what g* has to lead by, less the radius of g: its own radius, the roundings of both scores, and of this kernel
+    auto needs = [&](float4 star, float r, const Box &b) {
+        // its largest score in the box: from the angle at the centre, less the box's reach
+        const float len = sqrtf(star.x * star.x + star.y * star.y + star.z * star.z + star.w * star.w);
+        const float c = fminf(dot(star, b.mid) / len, 1.f), s = sqrtf(fmaxf(1.f - c * c, 0.f));
+        const float cr = 1.f - 0.5f * b.reach * b.reach, sr = b.reach;          // cos >= cr, sin <= sr
+        const float most = (c > cr ? 1.f : fminf(c + s * sr, 1.f)) * len + r;
+        return 1.016f * (most * 1.016f < 1.f ? 1.f : 2.f) * D::eps() + 1.2e-5f + r;
     };
-    auto beaten = [&](float4 s, float need, float4 g, float r, const Box &b) {
-        const float d0 = s.x - g.x, d1 = s.y - g.y, d2 = s.z - g.z, d3 = s.w - g.w;
-        const float lead = d0 + b.y0 * d1 + b.y1 * d2 + b.y2 * d3 - b.hw * (fabsf(d1) + fabsf(d2) + fabsf(d3));
-        return lead > (need + r) * b.longest;
+    // Is <g* - g, (1 - |z|^2, 2 z)> > m (1 + |z|^2) all over the box?  A sum of one parabola per coordinate.
+    auto beaten = [](float4 s, float need, float4 g, float r, const Box &b) {
+        const float d[4] = {s.x - g.x, s.y - g.y, s.z - g.z, s.w - g.w}, m = (need + r) * 1.0001f;
+        const float a = -(d[0] + m);
+        float lead = d[0] - m;
+        for (int i = 0; i < 3; i++) {
+            const float e = 2.f * d[i + 1];
+            const float at_lo = (e + a * b.lo[i]) * b.lo[i], at_hi = (e + a * b.hi[i]) * b.hi[i];
+            float least = fminf(at_lo, at_hi);
+            if (a > 0.f) {
+                const float z = fminf(fmaxf(-0.5f * e / a, b.lo[i]), b.hi[i]);
+                least = fminf(least, (e + a * z) * z);
+            }
+            lead += least;
+        }
+        return lead > 2e-6f;
     };
+    uint4 *lists = grid + stride * h;
+    const int f = tid / kLanes, part = tid % kLanes;
+    const int i = ci * kFine + f / (kFine * kFine), j = cj * kFine + f / kFine % kFine, k = ck * kFine + f % kFine;
+    const bool mine = f < kBoxes;
+    const uint4 empty = uint4{kNone | kNone << 16, kNone | kNone << 16, kNone | kNone << 16, kNone};
+    const Box coarse = box_at(ci, cj, ck, kFine);
+    if (!coarse.met) {                      // (no direction looks there; a block all the same, for lanes whose box is not used)
+        if (mine && part == 0) lists[(i * kGrid + j) * kGrid + k] = empty;
+        return;
+    }
     if (tid == 0) n_sh = 0;
-    if (tid < kFine * kFine * kFine) count[tid] = 0;
+    if (tid < kBoxes) count[tid] = 0;
     {
-        const Box b = box_at(ci, cj, ck, kCoarse);
         float best = -INFINITY;
         int arg = 0;
 #pragma unroll 4
-        for (int k = tid; k < K; k += kBuildThreads) {
-            const float v = dot(centre[k], b) - rho[k] * b.longest;
-            if (v > best) { best = v; arg = k; }
+        for (int k2 = tid; k2 < K; k2 += kBuildThreads) {
+            const float v = dot(centre[k2], coarse.mid) - rho[k2];
+            if (v > best) { best = v; arg = k2; }
         }
         for (int o = 32; o; o >>= 1) {
             const float v = __shfl_xor(best, o);
@@ -223,32 +283,34 @@ __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 
         for (int w = 0; w < kBuildThreads / 64; w++)
             if (best_sh[w] > best || (best_sh[w] == best && arg_sh[w] < arg)) { best = best_sh[w]; arg = arg_sh[w]; }
         const float4 star = centre[arg];
-        const float need = rounding(star, rho[arg], b) + rho[arg];
+        const float need = needs(star, rho[arg], coarse), inv_s = 1.f / (float)S;
         for (int k0 = 0; k0 < K; k0 += kBuildThreads) {
-            const int k = k0 + tid;
-            const float4 g = centre[min(k, K - 1)];
-            const float r = rho[min(k, K - 1)];
-            const bool take = k < K && !beaten(star, need, g, r, b);
+            const int k2 = k0 + tid;
+            const float4 g = centre[min(k2, K - 1)];
+            const float r = rho[min(k2, K - 1)];
+            const bool take = k2 < K && !beaten(star, need, g, r, coarse);
             const uint64_t mask = __builtin_amdgcn_ballot_w64(take);
             int at = 0;
             if (lane == 0 && mask) at = atomicAdd(&n_sh, (int)__popcll(mask));
             at = __shfl(at, 0) + __popcll(mask & ((1ull << lane) - 1ull));
-            if (take && at < kListCap) { geo[at] = g; rad[at] = r; id[at] = (uint16_t)k; }
+            if (take && at < kListCap) {
+                const int p = (int)(((float)k2 + 0.5f) * inv_s), s = S - 1 - (k2 - p * S);       // (k2 < 8192: exact)
+                geo[at] = g;
+                rad[at] = r;
+                id[at] = (uint16_t)(p << 2 | (s >> 8) << 7 | (s & 0xff) << 8);
+            }
         }
         __syncthreads();
     }
     const int n_list = n_sh;
-    uint4 *lists = grid + stride * h;
     uint32_t *used = grid_counters(grid, stride, H) + h;
-    const int f = tid / kLanes, part = tid % kLanes;
-    const int i = ci * kFine + f / (kFine * kFine), j = cj * kFine + f / kFine % kFine, k = ck * kFine + f % kFine;
-    const bool wanted = box_meets(i, j, k, kGrid), listed = n_list <= kListCap;
-    if (wanted && listed) {
-        const Box b = box_at(i, j, k, kGrid);
+    const Box b = box_at(i, j, k, 1);
+    const bool listed = n_list <= kListCap, wanted = mine && b.met && listed;
+    if (wanted) {
         float best = -INFINITY;
         int arg = 0;
         for (int e = part; e < n_list; e += kLanes) {
-            const float v = dot(geo[e], b) - rad[e] * b.longest;
+            const float v = dot(geo[e], b.mid) - rad[e];
             if (v > best) { best = v; arg = e; }
         }
         for (int o = 1; o < kLanes; o <<= 1) {
@@ -257,223 +319,411 @@ __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 
             if (v > best || (v == best && g < arg)) { best = v; arg = g; }
         }
         const float4 star = geo[arg];
-        const float need = rounding(star, rad[arg], b) + rad[arg];
+        const float need = needs(star, rad[arg], b);
         for (int e = part; e < n_list; e += kLanes) {
             if (beaten(star, need, geo[e], rad[e], b)) continue;
             const int at = atomicAdd(&count[f], 1);
-            if (at < kBoxCap) entries[f][at] = id[e];
+            if (at < kBoxCap) entries[f][at] = (uint16_t)e;
         }
     }
     __syncthreads();
-    if (tid >= kFine * kFine * kFine) return;
-    {
-        const int f2 = tid, i2 = ci * kFine + f2 / (kFine * kFine), j2 = cj * kFine + f2 / kFine % kFine, k2 = ck * kFine + f2 % kFine;
-        if (!box_meets(i2, j2, k2, kGrid)) return;
-        const int cell = d_map.off[i2 * kGrid + j2] + k2, n = count[f2], more = n > 7 ? (n - 1) / 7 : 0;      // blocks from the pool
-        uint32_t next = 0;
-        bool full = !listed || n > kBoxCap;
-        if (!full && more) {
-            next = atomicAdd(used, (uint32_t)more);
-            full = next + more > (uint32_t)pool;
-        }
-        int at = cell;
-        for (int e0 = 0;; e0 += 7) {
-            uint32_t w[8];
-#pragma unroll
-            for (int e = 0; e < 7; e++) {
-                w[e] = kNone;
-                if (!full && e0 + e < n) {
-                    const int kk = entries[f2][e0 + e], p = kk / S;
-                    w[e] = (uint32_t)p << 2 | (uint32_t)(S - 1 - (kk - p * S)) << 7;
-                }
+    // (a codeword that another one beats all over the box is beaten by one that stays: the leads add up)
+    if (wanted && count[f] <= kBoxCap) {
+        const int n = count[f];
+        for (int x = part; x < n; x += kLanes) {
+            const float4 g = geo[entries[f][x]];
+            const float r = rad[entries[f][x]];
+            bool lost = false;
+            for (int y = 0; y < n && !lost; y++) {
+                const float4 s = geo[entries[f][y]];
+                lost = y != x && beaten(s, needs(s, rad[entries[f][y]], b), g, r, b);
             }
-            const bool last = full || e0 + 7 >= n;
-            w[7] = full ? 0xffffu : last ? 0u : next;
-            lists[at] = uint4{w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16};
-            if (last) break;
-            at = kCells + (int)next++;
+            out[f][x] = lost;
         }
+    }
+    __syncthreads();
+    if (!mine || part) return;
+    const int cell = (i * kGrid + j) * kGrid + k;
+    if (!b.met) { lists[cell] = empty; return; }
+    bool full = !listed || count[f] > kBoxCap;
+    int n = 0;
+    if (!full)
+        for (int x = 0; x < count[f]; x++)
+            if (!out[f][x]) entries[f][n++] = entries[f][x];
+    const int more = n > 7 ? (n - 1) / 7 : 0;                   // blocks from the pool
+    uint32_t next = 0;
+    if (more) {
+        next = atomicAdd(used, (uint32_t)more);
+        full = next + more > (uint32_t)pool;
+    }
+    int at = cell;
+    for (int e0 = 0;; e0 += 7) {
+        uint32_t w[8];
+#pragma unroll
+        for (int e = 0; e < 7; e++) w[e] = !full && e0 + e < n ? id[entries[f][e0 + e]] : kNone;
+        const bool last = full || e0 + 7 >= n;
+        w[7] = full ? 0xffffu : last ? 0u : next;
+        lists[at] = uint4{w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16};
+        if (last) break;
+        at = kCells + (int)next++;
     }
 }
 
 // ---------------------------------------------------------------- search
-// LDS: [K rows of the joint table, last row first (JLDS)] | 24 x 32 row offsets by (unit of the direction, p') | box
-// numbers | two words per lane.  The dynamic block is the kernel's only LDS, so it starts at LDS address 0 and the row
-// offset of a codeword is its address.
-constexpr int lds_rows_at(int table_bytes) { return (table_bytes + 127) & ~127; }
-constexpr int kBoxesAt = 24 * 32 * 4, kLanesAt = (kBoxesAt + kGrid * kGrid * 2 + 15) & ~15;       // behind the row offsets
+// LDS: the axis units | row numbers by (unit of the direction, low byte of the entry) | K rows of the joint table, last row
+// first (JLDS; bf16 widened to fp32) | one or two words per lane.  The dynamic block is the kernel's only LDS, so it starts
+// at LDS address 0.
+template <class D>
+constexpr int lds_row_bytes() { return D::code == HQMQ_F16 ? 8 : 16; }
+constexpr int kUnitsAt = 256, kRowsAt = kUnitsAt + 8 * 64 * 4;
+// ChunkSink's second word per lane
+template <bool ROWS, int WHAT>
+constexpr bool needs_aux(int n) { return !ROWS || (WHAT & kCompact) || n < 8; }
+
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef short s2 __attribute__((ext_vector_type(2)));
+// two fp32 numbers rounded to 16 bits each, in one instruction
+__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
+    return __builtin_bit_cast(uint32_t, h2{(_Float16)a, (_Float16)b});
+}
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) { return __builtin_bit_cast(uint32_t, b2{(__bf16)a, (__bf16)b}); }
+// a ^ one byte of b (the compiler shifts first)
+__device__ __forceinline__ uint32_t xor_byte0(uint32_t a, uint32_t b) { return a ^ (b & 0xffu); }
+__device__ __forceinline__ uint32_t xor_byte2(uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_xor_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// k's upper half = s rounded to fp16 (from fp32: see F16::rnd); the s_nop lets the half written last arrive
+__device__ __forceinline__ void round_over(uint32_t &k0, float s0, uint32_t &k1, float s1) {
+    asm("v_cvt_f16_f32_sdwa %0, %2 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD\n\t"
+        "v_cvt_f16_f32_sdwa %1, %3 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD\n\ts_nop 0" : "+v"(k0), "+v"(k1) : "v"(s0), "v"(s1));
+}
+__device__ __forceinline__ void round_over(uint32_t &k, float s) {
+    asm("v_cvt_f16_f32_sdwa %0, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD\n\ts_nop 0" : "+v"(k) : "v"(s));
+}
+// mixed multiply-adds on half j of w (the compiler converts the halves first): w_j * y, and w_j - r * q in one rounding
+__device__ __forceinline__ float half_times(uint32_t w, int j, float y) {
+    float o;
+    if (j) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(o) : "v"(w), "v"(y));
+    else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(o) : "v"(w), "v"(y));
+    return o;
+}
+__device__ __forceinline__ float half_less(uint32_t w, int j, float r, float q) {
+    float o;
+    if (j) asm("v_fma_mix_f32 %0, -%2, %3, %1 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(o) : "v"(w), "v"(r), "v"(q));
+    else asm("v_fma_mix_f32 %0, -%2, %3, %1 op_sel_hi:[0,0,1]" : "=v"(o) : "v"(w), "v"(r), "v"(q));
+    return o;
+}
+__device__ __forceinline__ float half_at(uint32_t w, int j) { return (float)__builtin_bit_cast(h2, w)[j]; }
+
+// A row of the joint table as the search holds it: as stored, or bf16 widened to fp32 (from LDS)
+template <class D, bool JLDS>
+struct RowWords {
+    RawChunk<D> raw;
+    uint32_t (&w)[sizeof(typename D::storage)] = raw.w;
+    __device__ __forceinline__ float get(int j) const { return raw.get(j); }
+};
+template <>
+struct RowWords<BF16, true> {
+    uint32_t w[4];
+    __device__ __forceinline__ float get(int j) const { return __uint_as_float(w[j]); }
+};
 
 template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB>
-__device__ __forceinline__ void grid_body(const QParams &a) {
+__device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
     using ST = typename D::storage;
     typedef const uint32_t __attribute__((address_space(3))) *lds_u32;
-    typedef const int16_t __attribute__((address_space(3))) *lds_i16;
     typedef uint32_t __attribute__((ext_vector_type(2))) u32x2;
     typedef uint32_t __attribute__((ext_vector_type(4))) u32x4;
     typedef const u32x2 __attribute__((address_space(3))) *lds_u64;
     typedef const u32x4 __attribute__((address_space(3))) *lds_u128;
-    constexpr int RB = 4 * sizeof(ST), RSH = RB == 8 ? 3 : 4;            // bytes of a row
+    constexpr int RB = JLDS ? lds_row_bytes<D>() : 4 * (int)sizeof(ST);            // bytes of a row where it is read
     extern __shared__ __align__(16) unsigned char lds[];
     const int tid = threadIdx.x, n = a.n, S = a.S, K = 24 * S;
-    const int bh = blockIdx.y, b = bh / a.H, h = bh - b * a.H;
+    const int b = bh / a.H, h = bh - b * a.H;
     const ST *jh = (const ST *)a.joint + (size_t)h * K * 4;
-    const uint32_t rows_at = JLDS ? (uint32_t)lds_rows_at(K * RB) : 0u;
-    uint32_t *code_sh = reinterpret_cast<uint32_t *>(lds + rows_at + kLanesAt), *aux_sh = code_sh + NT;
+    uint32_t *code_sh = reinterpret_cast<uint32_t *>(lds + kRowsAt + (JLDS ? K * RB : 0)), *aux_sh = code_sh + NT;
     const int tpb = NT / n, tok_local = tid / n, c = tid - tok_local * n;
-    const int t_first = blockIdx.x * a.iters * tpb;
+    const int t_first = block * a.iters * tpb;
     const ST *xl = (const ST *)a.x + b * a.xsb + h * a.xsh + (int64_t)(t_first + tok_local) * a.xst + c * 4;
     const int64_t x_step = tpb * a.xst;
     const int t_left = tok_local < tpb ? a.T - t_first - tok_local : 0;     // this lane has a token while t0 - t_first < t_left
-    RawChunk<D> raw = {};
+    RawChunk<D> none = {};                                                        // what lanes without a token work on: an ordinary direction
+    for (int j = 0; j < 4; j++) none.set(j, 1.f);
+    RawChunk<D> raw = none;
     if (t_left > 0) raw.load(xl, a.vec_in);
     {
         // every load of the set-up is requested before the first one is used: one round trip
-        constexpr int NP = (24 * 32 + NT - 1) / NT, NB = (kGrid * kGrid / 2 + NT - 1) / NT;
-        uint32_t unit_mul[NP], boxes[NB];
+        constexpr int NP = (8 * 32 + NT - 1) / NT;
+        uint32_t unit_mul[NP];
 #pragma unroll
         for (int i = 0; i < NP; i++) {
-            const int k = min(tid + i * NT, 24 * 32 - 1);
+            const int k = min(tid + i * NT, 8 * 32 - 1);
             unit_mul[i] = d_units.mul[k >> 5][min(k & 31, 23)];
         }
-#pragma unroll
-        for (int i = 0; i < NB; i++) boxes[i] = reinterpret_cast<const uint32_t *>(d_map.off)[min(tid + i * NT, kGrid * kGrid / 2 - 1)];
+        const int e = min(tid, 7);
+        const uint32_t a01 = d_axis.a01[e], a23 = d_axis.a23[e], first = (uint32_t)d_axis.first[e];
         if (JLDS) {
             for (int k = tid; k < K; k += NT) {
                 RawChunk<D> g;
                 g.load(jh + (size_t)k * 4, true);
-                g.store(reinterpret_cast<ST *>(lds) + (size_t)(K - 1 - k) * 4, true);
+                unsigned char *row = lds + kRowsAt + (K - 1 - k) * RB;
+                if constexpr (D::code == HQMQ_BF16)
+                    *reinterpret_cast<float4 *>(row) = float4{g.get(0), g.get(1), g.get(2), g.get(3)};
+                else g.store(reinterpret_cast<ST *>(row), true);
             }
         }
+        uint32_t *rows = reinterpret_cast<uint32_t *>(lds + kUnitsAt);
 #pragma unroll
         for (int i = 0; i < NP; i++) {
-            const int k = tid + i * NT;
-            // Most entries have p' = 0, so the offsets of one p' would share a bank: the units are spread over the banks by an
-            // exclusive-or (14.8 -> 4.5 cycles per LDS access over the kernel).  No entry: a row like any other.
-            if (k < 24 * 32) reinterpret_cast<uint32_t *>(lds + rows_at)[k ^ (k >> 5)] = (k & 31) < 24 ? (23u - unit_mul[i]) * (uint32_t)(S * RB) : 0u;
+            const int k = tid + i * NT, g = k >> 5, p = k & 31;
+            // Most entries have p' = 0, so the words of one p' would share a bank: the units are spread over the banks by an
+            // exclusive-or.  Bit 7 of an entry's low byte is bit 8 of s'.  No entry: a row like any other.
+            if (k < 8 * 32) {
+                const uint32_t row = p < 24 ? (23u - unit_mul[i]) * (uint32_t)S : 0u;
+                rows[g * 64 + (p ^ g)] = row;
+                rows[g * 64 + ((p + 32) ^ g)] = p < 24 ? row + 256u : 0u;
+            }
         }
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-            if (tid + i * NT < kGrid * kGrid / 2) reinterpret_cast<uint32_t *>(lds + rows_at + kBoxesAt)[tid + i * NT] = boxes[i];
+        if (tid < 8) *reinterpret_cast<uint4 *>(lds + tid * 16) = uint4{a01, a23, first, (uint32_t)(kUnitsAt + tid * 260)};
     }
     __syncthreads();
 
-    const uint4 *lists = a.grid + a.grid_stride * h;
+    const unsigned char *lists = reinterpret_cast<const unsigned char *>(a.grid + a.grid_stride * h);
     ChunkSink<D, NT, ROWS, WHAT, MB> sink(a, b, h, tok_local, c, code_sh, aux_sh);
     const int t_end = JLDS ? a.iters * tpb : tpb;
-    for (int t0 = 0; t0 < t_end; t0 += tpb) {
-        const bool active = t0 < t_left;
-        const RawChunk<D> cur = raw;
-        raw = {};
-        xl += x_step;
-        if (t0 + tpb < t_end && t0 + tpb < t_left) raw.load(xl, a.vec_in);      // the next round's chunk
-        const float nrm = chunk_norm_d<D>(cur.get(0), cur.get(1), cur.get(2), cur.get(3));
-        const float r = clamp_min_d<D>(nrm, 1e-8f);
-        float u[4] = {cur.get(0), cur.get(1), cur.get(2), cur.get(3)};
-        div4_d<D>(u, r);
+    // One round, once norm and direction are known: the search and everything after it.  QUICK: every lane of the wavefront has
+    // an ordinary norm of a 16-bit type.  u: the direction; with QUICK fp16, the quotients before their rounding to fp16.
+    auto rest = [&](auto QUICK, int t0, bool active, const RawChunk<D> &cur, float nrm, float r, const float (&u)[4], float len, bool brute, bool zero) {
+        // the direction as fp16 (fp16: exactly; otherwise for its box only)
+        uint32_t ud[2] = {pack_f16(u[0], u[1]), pack_f16(u[2], u[3])};
+        if (D::code == HQMQ_F16) asm("" : "+v"(ud[0]), "+v"(ud[1]));          // (read as they are by mixed multiply-adds)
+        // ---- the axis unit nearest to u: the component of largest magnitude.  Each competes as its bits, sign last, with
+        // the number of its unit in place of the last three ----
+        uint32_t best_axis = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t x = __float_as_uint(u[j]);
+            const uint32_t v = (__builtin_amdgcn_alignbit(x, x, 31) & ~6u) | (uint32_t)(2 * j);
+            best_axis = max(best_axis, v);
+        }
+        const float w0 = __uint_as_float(best_axis >> 1);
+        const u32x4 axis = *(lds_u128)(uintptr_t)(best_axis << 4 & 0x70u);
 
-        // ---- the unit nearest to u, and w = conj(unit) * u (half units doubled: only the ratios are used) ----
-        const float a0 = fabsf(u[0]), a1 = fabsf(u[1]), a2 = fabsf(u[2]), a3 = fabsf(u[3]);
-        const float sum = (a0 + a1) + (a2 + a3), mx = fmaxf(fmaxf(a0, a1), fmaxf(a2, a3));
-        // directions of length 1: the others (NaN, infinite, clamped or subnormal radius) follow the reference row by
-        // row, an all-zero direction scores 0 everywhere and takes row 0
-        const float len2 = fmaf(u[3], u[3], fmaf(u[2], u[2], fmaf(u[1], u[1], u[0] * u[0])));
-        const bool ordinary = len2 > 0.97f && len2 < 1.03f;
-        const bool zero = sum == 0.f;
-        const bool half = sum > mx + mx;
-        const bool i0 = a0 == mx, i1 = !i0 && a1 == mx, i2 = !i0 && !i1 && a2 == mx, i3 = !i0 && !i1 && !i2;
-        const float q0 = (half || i0) ? copysignf(1.f, u[0]) : 0.f, q1 = (half || i1) ? copysignf(1.f, u[1]) : 0.f;
-        const float q2 = (half || i2) ? copysignf(1.f, u[2]) : 0.f, q3 = (half || i3) ? copysignf(1.f, u[3]) : 0.f;
-        const uint32_t n0 = __float_as_uint(u[0]) >> 31, n1 = __float_as_uint(u[1]) >> 31, n2 = __float_as_uint(u[2]) >> 31, n3 = __float_as_uint(u[3]) >> 31;
-        const uint32_t p_axis = i0 ? n0 : i1 ? 2u + n1 : i2 ? 4u + n2 : 6u + n3;
-        const uint32_t p_half = 8u + (((n0 * 2u + n1) * 2u + n2) * 2u + n3);
-        const uint32_t unit = half ? p_half : p_axis;
-        const float w0 = half ? sum : mx;
-        const float w1 = fmaf(q3, u[2], fmaf(-q2, u[3], fmaf(q0, u[1], -q1 * u[0])));
-        const float w2 = fmaf(-q3, u[1], fmaf(q1, u[3], fmaf(q0, u[2], -q2 * u[0])));
-        const float w3 = fmaf(q2, u[1], fmaf(-q1, u[2], fmaf(q0, u[3], -q3 * u[0])));
-        const float inv = __builtin_amdgcn_rcpf(w0) * (0.5f * kGrid);
-        // (a NaN ends up in box 0: such a lane's result is not used)
-        auto box = [&](float w) { return (uint32_t)fminf(fmaxf(fmaf(w, inv, 0.5f * kGrid), 0.f), kGrid - 0.5f); };
-        const uint32_t bx = box(w1), by = box(w2), bz = box(w3);
-        const int box_no = *(lds_i16)(uintptr_t)(rows_at + kBoxesAt + (bx * kGrid + by) * 2u) + (int)bz;
-        uint4 e = lists[min(max(box_no, 0), kCells - 1)];
+        // ---- its box: z = w / (w0 + |u|), positions as fp16 numbers 1536 + t ----
+        const float inv = __builtin_amdgcn_rcpf(fmaf(w0, 1.f / kScale, len * (1.f / kScale)));
+        const h2 inv2 = __builtin_bit_cast(h2, pack_f16(inv, inv)), magic = {(_Float16)1536.f, (_Float16)1536.f};
+        const h2 t01 = __builtin_elementwise_fma(__builtin_bit_cast(h2, ud[0]), inv2, magic), t23 = __builtin_elementwise_fma(__builtin_bit_cast(h2, ud[1]), inv2, magic);
+        const uint32_t a01 = axis[0], a23 = axis[1];
+        int at_box = __builtin_amdgcn_sdot2(__builtin_bit_cast(s2, t01), __builtin_bit_cast(s2, a01), (int)axis[2], false);
+        at_box = __builtin_amdgcn_sdot2(__builtin_bit_cast(s2, t23), __builtin_bit_cast(s2, a23), at_box, false);
+        // (a direction that is not of length 1 may end up anywhere: its list is not used)
+        uint4 e = *reinterpret_cast<const uint4 *>(lists + min((uint32_t)at_box, (uint32_t)(kCells - 1) * 16u));
 
         // ---- the reference's score of every codeword of the list ----
-        int key = 0;                                                    // 16-bit types: rounded score << 16 | row offset
+        int key = 0;                                                    // 16-bit types: rounded score << 16 | row number
         float best = -INFINITY;                                         // fp32
         uint32_t best_at = 0;
-        bool brute = active && !ordinary && !zero;
-        const uint32_t unit_row = rows_at + unit * 132u;
-        auto score = [&](uint32_t entry) {
-            // row offset from the end of the table: the larger of two offsets is the smaller index k
-            const uint32_t at = *(lds_u32)(uintptr_t)(unit_row ^ (entry & 0x7cu)) + ((entry >> 7 & 0x1ffu) << RSH);
-            RawChunk<D> g;
-            if constexpr (!JLDS) g.load(reinterpret_cast<const ST *>((const unsigned char *)(jh + (size_t)(K - 1) * 4) - at), true);
-            else if constexpr (RB == 8) { const u32x2 v = *(lds_u64)(uintptr_t)at; g.w[0] = v[0]; g.w[1] = v[1]; }
-            else { const u32x4 v = *(lds_u128)(uintptr_t)at; g.w[0] = v[0]; g.w[1] = v[1]; g.w[2] = v[2]; g.w[3] = v[3]; }
-            float s = fmaf(u[0], g.get(0), 0.f);                        // the product's own rounding (a sum with 0 keeps it)
-            s = fmaf(u[1], g.get(1), s);
-            s = fmaf(u[2], g.get(2), s);
-            s = fmaf(u[3], g.get(3), s);
-            if constexpr (D::code == HQMQ_F16) {
-                asm("" : "+v"(s));                                      // rounded to fp32 first, then to fp16
-                key = max(key, (int)((uint32_t)__half_as_ushort(__float2half_rn(s)) << 16 | at));
-            } else if constexpr (D::code == HQMQ_BF16) {
-                const uint32_t x = __float_as_uint(s);
-                key = max(key, (int)(((x + 0x7fffu + ((x >> 16) & 1u)) & 0xffff0000u) | at));
-            } else {
-                const bool more = s > best || (s == best && at > best_at);
-                best = more ? s : best;
-                best_at = more ? at : best_at;
+        const uint32_t unit_row = axis[3];
+        // The entries of `words` dwords (the upper half of the last one is none with ODD): row numbers, rows, scores, each
+        // asked for together.  A row number counts from the end of the table: the larger of two is the smaller index k.
+        auto score = [&](const uint32_t *e, auto WORDS, auto ODD) {
+            constexpr int N = 2 * WORDS.value - ODD.value;
+            uint32_t at[N];
+            RowWords<D, JLDS> row[N];
+            float s[N];
+#pragma unroll
+            for (int i = 0; i < N; i++) at[i] = *(lds_u32)(uintptr_t)(i & 1 ? xor_byte2(unit_row, e[i >> 1]) : xor_byte0(unit_row, e[i >> 1]));
+#pragma unroll
+            for (int i = 0; i < N; i++) at[i] += (i & 1 ? e[i >> 1] >> 24 : e[i >> 1] >> 8 & 0xffu);
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                if constexpr (!JLDS) row[i].raw.load(reinterpret_cast<const ST *>(reinterpret_cast<const unsigned char *>(jh + (size_t)(K - 1) * 4) - at[i] * RB), true);
+                else if constexpr (RB == 8) { const u32x2 v = *(lds_u64)(uintptr_t)(kRowsAt + at[i] * RB); row[i].w[0] = v[0]; row[i].w[1] = v[1]; }
+                else { const u32x4 v = *(lds_u128)(uintptr_t)(kRowsAt + at[i] * RB); for (int j = 0; j < 4; j++) row[i].w[j] = v[j]; }
             }
-        };
-        while (true) {
-            score(e.x);
-            score(e.x >> 16);
-            const uint32_t none2 = kNone | kNone << 16;
-            if (__builtin_amdgcn_ballot_w64(e.y != none2)) {
-                score(e.y);
-                score(e.y >> 16);
-                if (__builtin_amdgcn_ballot_w64(e.z != none2)) {
-                    score(e.z);
-                    score(e.z >> 16);
-                    score(e.w);
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                auto dir = [&](int j) { return D::code == HQMQ_F16 ? half_at(ud[j >> 1], j & 1) : u[j]; };
+                s[i] = fmaf(dir(0), row[i].get(0), 0.f);                // the product's own rounding (a sum with 0 keeps it)
+#pragma unroll
+                for (int j = 1; j < 4; j++) s[i] = fmaf(dir(j), row[i].get(j), s[i]);
+            }
+            if constexpr (D::code == HQMQ_F32) {
+#pragma unroll
+                for (int i = 0; i < N; i++) {
+                    const bool more = s[i] > best || (s[i] == best && at[i] > best_at);
+                    best = more ? s[i] : best;
+                    best_at = more ? at[i] : best_at;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < N; i += 2) {
+                    if constexpr (D::code == HQMQ_F16) {
+                        if (i + 1 < N) round_over(at[i], s[i], at[i + 1], s[i + 1]);
+                        else round_over(at[i], s[i]);
+                    } else {
+                        const uint32_t v = pack_bf16(s[i], s[min(i + 1, N - 1)]);
+                        at[i] |= v << 16;
+                        if (i + 1 < N) at[i + 1] |= v & 0xffff0000u;
+                    }
+                    key = i + 1 < N ? max(max((int)at[i], (int)at[i + 1]), key) : max((int)at[i], key);
                 }
             }
+        };
+        using std::integral_constant;
+        typedef integral_constant<int, 0> Even;
+        typedef integral_constant<int, 1> One;
+        // (the first block whole: among 64 lists one has more than four entries nearly always)
+        {
+            const uint32_t w[4] = {e.x, e.y, e.z, e.w};
+            if constexpr (RB == 8) score(w, integral_constant<int, 4>(), One());
+            else {                  // (rows of 16 bytes: seven of them would not fit the registers)
+                score(w, integral_constant<int, 2>(), Even());
+                score(w + 2, integral_constant<int, 2>(), One());
+            }
+        }
+        constexpr uint32_t none2 = kNone | kNone << 16;
+        while (true) {
             const uint32_t next = e.w >> 16;
             if (__builtin_amdgcn_ballot_w64(next != 0u) == 0ull) break;
-            if (next == 0xffffu) brute |= active && ordinary;           // (a direction that is not ordinary keeps its own reason)
-            e = lists[kCells + (next == 0xffffu ? 0u : next)];
+            if (next == 0xffffu) brute |= active && !zero;              // (a direction that is not ordinary keeps its own reason)
+            e = *reinterpret_cast<const uint4 *>(lists + (kCells + (next == 0xffffu ? 0u : next)) * 16u);
+            if (D::code == HQMQ_F16) asm volatile("" : "+v"(ud[0]), "+v"(ud[1]));      // (or the compiler converts them ahead of the loop)
+            score(&e.x, One(), Even());
+            if (__builtin_amdgcn_ballot_w64(e.y != none2)) {
+                score(&e.y, One(), Even());
+                if (__builtin_amdgcn_ballot_w64(e.z != none2)) {
+                    const uint32_t w[2] = {e.z, e.w};
+                    score(w, integral_constant<int, 2>(), One());
+                }
+            }
         }
-        const uint32_t at = D::code == HQMQ_F32 ? best_at : (uint32_t)key & 0xffffu;
-        int idx = zero ? 0 : K - 1 - (int)(at >> RSH);
-        if (brute) idx = brute_argmax<D>(u, jh, K);
+        int idx = zero ? 0 : K - 1 - (int)(D::code == HQMQ_F32 ? best_at : (uint32_t)key & 0xffffu);
+        if (brute) {
+            float ur[4];
+            for (int j = 0; j < 4; j++) ur[j] = D::code == HQMQ_F16 ? half_at(ud[j >> 1], j & 1) : u[j];
+            idx = brute_argmax<D>(ur, jh, K);
+        }
         if ((WHAT & kUnpacked) && a.stats && active) {
             if (brute) atomicAdd(a.stats, 1);
             else if (!zero) atomicAdd(a.stats + 1, 1);
         }
-        const ST *jrow = JLDS ? reinterpret_cast<const ST *>(lds) + (size_t)(K - 1 - idx) * 4 : jh + (size_t)idx * 4;
-        sink.put(t_first + t0, active, cur, nrm, r, idx, jrow);
+        auto row = [&](float (&g)[4]) {
+            if constexpr (JLDS && D::code == HQMQ_BF16) {
+                const float4 v = *reinterpret_cast<const float4 *>(lds + kRowsAt + (K - 1 - idx) * RB);
+                g[0] = v.x; g[1] = v.y; g[2] = v.z; g[3] = v.w;
+            } else {
+                RawChunk<D> v;
+                v.load(JLDS ? reinterpret_cast<const ST *>(lds + kRowsAt) + (K - 1 - idx) * 4 : jh + (size_t)idx * 4, true);
+                for (int j = 0; j < 4; j++) g[j] = v.get(j);
+            }
+        };
+        sink.put(t_first + t0, active, cur, nrm, r, idx, row, QUICK);
+    };
+    for (int t0 = 0; t0 < t_end; t0 += tpb) {
+        const bool active = t0 < t_left;
+        const RawChunk<D> cur = raw;
+        raw = none;
+        xl += x_step;
+        if (t0 + tpb < t_end && t0 + tpb < t_left) raw.load(xl, a.vec_in);      // the next round's chunk
+
+        // ---- norm and direction ----
+        // 16-bit types: products of two numbers are exact in fp32, so fused multiply-adds round as products and sums do.
+        // Norms of the quick range, far from D's ends, take the short forms of chunk_norm_d and div4_d; a wavefront with any
+        // other (NaN, infinite, clamped, subnormal) takes the reference's operations one by one.
+        if constexpr (D::code != HQMQ_F32) {
+            float s = fmaf(cur.get(0), cur.get(0), 0.f);
+#pragma unroll
+            for (int j = 1; j < 4; j++) s = fmaf(cur.get(j), cur.get(j), s);
+            const float ys = __builtin_amdgcn_rsqf(s);
+            float g = s * ys;
+            g = fmaf(fmaf(-g, g, s), 0.5f * ys, g);
+            const float r = D::code == HQMQ_F16 ? D::rnd(g) : __uint_as_float(pack_bf16(0.f, g));
+            const uint32_t lo = D::code == HQMQ_F16 ? 0x387bb000u : 0x32ac0000u, hi = D::code == HQMQ_F16 ? 0x47800000u : 0x71490000u;
+            // (fp16: 6.0e-5 .. 65536, bf16: 2.0e-8 .. 9.9e29)
+            if (__builtin_amdgcn_ballot_w64(__float_as_uint(r) - lo >= hi - lo) == 0ull) {
+                float y = __builtin_amdgcn_rcpf(r);
+                asm("s_nop 0" : "+v"(y));       // (one wait state between v_rcp and its use, which the compiler leaves to inline assembly)
+                float u[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if constexpr (D::code == HQMQ_F16) {
+                        u[j] = half_times(cur.w[j >> 1], j & 1, y);
+                        u[j] = fmaf(half_less(cur.w[j >> 1], j & 1, r, u[j]), y, u[j]);
+                        asm("" : "+v"(u[j]));                       // rounded to fp32 first, see F16::rnd
+                    } else u[j] = cur.get(j) * y;
+                }
+                if constexpr (D::code == HQMQ_BF16) {
+                    const uint32_t d01 = pack_bf16(u[0], u[1]), d23 = pack_bf16(u[2], u[3]);
+                    u[0] = __uint_as_float(d01 << 16);
+                    u[1] = __uint_as_float(d01 & 0xffff0000u);
+                    u[2] = __uint_as_float(d23 << 16);
+                    u[3] = __uint_as_float(d23 & 0xffff0000u);
+                }
+                rest(std::true_type(), t0, active, cur, r, r, u, 1.f, false, false);
+                continue;
+            }
+        }
+        // (a copy the compiler takes for another chunk: the quick path's multiply-adds then read the 16-bit values as they are)
+        RawChunk<D> x = cur;
+#pragma unroll
+        for (uint32_t &w : x.w) asm("" : "+v"(w));
+        float u[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) u[j] = x.get(j);
+        const float nrm = chunk_norm_d<D>(u[0], u[1], u[2], u[3]);
+        float r = clamp_min_d<D>(nrm, 1e-8f);
+        if (is_nan(r)) r = NAN;
+        div4_d<D>(u, r);
+        // directions of length 1: the others follow the reference row by row, an all-zero direction scores 0 everywhere and
+        // takes row 0
+        const float len2 = fmaf(u[3], u[3], fmaf(u[2], u[2], fmaf(u[1], u[1], u[0] * u[0])));
+        const bool ordinary = len2 > 0.97f && len2 < 1.03f, zero = u[0] == 0.f && u[1] == 0.f && u[2] == 0.f && u[3] == 0.f;
+        rest(std::false_type(), t0, active, cur, nrm, r, u, __builtin_amdgcn_sqrtf(len2), active && !ordinary && !zero, zero);
     }
     sink.done();
 }
 
 template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB>
-__global__ __launch_bounds__(NT) void quantize_grid_kernel(QPair kv) {
-    grid_body<D, NT, ROWS, JLDS, WHAT, MB>(kv.p[blockIdx.z]);
+__global__ __launch_bounds__(NT, NT == 1024 ? 8 : 1) void quantize_grid_kernel(QPair kv) {
+    if constexpr (JLDS) {
+        // blockIdx.x counts `per_head` blocks for each (tensor, b, h).  Workgroups go round-robin over the 8 XCDs; with a
+        // multiple of 8 heads the blocks of one head stay on one, whose L2 then holds that head's lists and not everyone's
+        // (8 heads of 32768 tokens, K and V, 512 blocks: 1.4 million cache lines from beyond the L2
+        // instead of 4.3, half of which would be lists; 140 -> 123 us).
+        auto same = [](int v) { return __builtin_amdgcn_readfirstlane(v); };        // (quotients come from the vector unit)
+        const int per_head = kv.per_head, heads = same((int)gridDim.x / per_head), spread = heads % 8 == 0 ? 8 : 1;
+        const int i = blockIdx.x / spread, q = same(i / per_head), which = q * spread + blockIdx.x % spread, bhs = kv.p[0].B * kv.p[0].H;
+        const int z = same(which >= bhs ? 1 : 0);
+        grid_body<D, NT, ROWS, JLDS, WHAT, MB>(kv.p[z], same(which - z * bhs), same(i - q * per_head));
+    } else grid_body<D, NT, ROWS, JLDS, WHAT, MB>(kv.p[blockIdx.z], blockIdx.y, blockIdx.x);
 }
 
 template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB>
 static int launch_kernel(QPair &kv, int count, hipStream_t st) {
     const QParams &p = kv.p[0];
     const int tpb = NT / p.n, rounds = (p.T + tpb - 1) / tpb;
-    // A block copies its head's table to LDS first: as many rounds of tokens per block as leave every CU two blocks or so
-    const int64_t blocks = (int64_t)rounds * p.B * p.H * count;
-    int iters = (int)(blocks / 1024);
-    iters = iters < 1 ? 1 : iters > 8 ? 8 : iters;
-    kv.p[0].iters = kv.p[1].iters = JLDS ? iters : 1;
-    const dim3 grid((rounds + kv.p[0].iters - 1) / kv.p[0].iters, p.B * p.H, count);
-    const size_t shmem = (JLDS ? (size_t)lds_rows_at(24 * p.S * 4 * (int)sizeof(typename D::storage)) : 0) + kLanesAt + (size_t)NT * 8;
+    const size_t shmem = kRowsAt + (JLDS ? (size_t)(24 * p.S * lds_row_bytes<D>()) : 0) + (size_t)NT * (needs_aux<ROWS, WHAT>(p.n) ? 8 : 4);
+    // A block copies its head's table to LDS first, about as much work as one round.  Blocks come in waves of as many as the
+    // CUs hold; the number of waves is chosen for the fewest rounds in a row, set-up included.
+    int iters = 1;
+    if (JLDS) {
+        const int heads = p.B * p.H * count, slots = (160 * 1024 / shmem >= 2 ? 2 : 1) * 256;
+        int least = INT32_MAX;
+        for (int waves = 1; waves <= 8; waves++) {
+            int per_head = waves * slots / heads;
+            per_head = per_head < 1 ? 1 : per_head > rounds ? rounds : per_head;
+            const int it = (rounds + per_head - 1) / per_head;
+            const int blocks = (rounds + it - 1) / it * heads, cost = (blocks + slots - 1) / slots * (it + 1);
+            if (cost < least) { least = cost; iters = it; }
+        }
+    }
+    kv.p[0].iters = kv.p[1].iters = iters;
+    kv.per_head = (rounds + iters - 1) / iters;
+    const dim3 grid = JLDS ? dim3(kv.per_head * p.B * p.H * count) : dim3(rounds, p.B * p.H, count);
     auto kern = quantize_grid_kernel<D, NT, ROWS, JLDS, WHAT, MB>;
     if (shmem > 48 * 1024) {
         const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
@@ -539,8 +789,8 @@ extern "C" int hqmq_build_search_grid(const void *joint, int H, int S, int dtype
     if ((uintptr_t)grid & 15) return HQMQ_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
     const int64_t stride = search_grid_blocks(S, dtype);
-    const int pool = (int)pool_blocks(dtype);
-    const dim3 gc(3 * S, H), gb(kCoarse * kCoarse * kCoarse, H);
+    const int pool = (int)pool_blocks(S, dtype);
+    const dim3 gc((24 * S + 31) / 32, H), gb(kCoarse * kCoarse * kCoarse, H);
 #define LAUNCH(DT, ST)                                                                                                              \
     do {                                                                                                                            \
         hipLaunchKernelGGL(grid_codewords_kernel<DT>, gc, dim3(256), 0, st, (const ST *)joint, S, (uint4 *)grid, stride, H);        \

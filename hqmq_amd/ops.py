@@ -51,7 +51,10 @@ def _book(joint: torch.Tensor, slack: Optional[torch.Tensor], radius_bits: int, 
     a.dtype, a.H, a.n_chunks = _dt(joint), joint.shape[0], n
     a.joint, a.slack = L.addr(joint), L.addr(slack)
     a.secondary_size, a.radius_bits = joint.shape[1] // 24, radius_bits
-    grid = L.addr(getattr(slack, "hqmq_grid", None))
+    grid = getattr(slack, "hqmq_grid", None)
+    if grid is not None and grid.numel() != L.lib().hqmq_search_grid_kept_bytes(C.c_int(a.H), C.c_int(a.secondary_size), C.c_int(a.dtype)):
+        grid = None                 # lists of another library version (loaded from a file): the scan gives the same codes
+    grid = L.addr(grid)
     if slack is not None:
         slack.hqmq_book = L.Kept((joint, joint.data_ptr(), (radius_bits, n), a, grid))
     return a, grid

@@ -104,7 +104,7 @@ typedef struct hqmq_quantize_args {
 } hqmq_quantize_args;
 int hqmq_quantize(const hqmq_quantize_args *a, void *stream);
 
-/* Cell lists of a codebook: for every box of a grid over the directions next to one Hurwitz unit, the codewords that
+/* Cell lists of a codebook: for every box of a grid over the directions next to one axis unit, the codewords that
  * can win the reference's rounded comparison there (see csrc/quantize_grid.hip).  Worked out once per codebook, they
  * replace the quantize kernel's scan over the secondaries; the codes are the same, bit for bit.
  *   hqmq_search_grid_bytes    size for H heads of S secondaries; 0 where the lists do not exist (S > 341)

@@ -81,3 +81,37 @@ def test_unordinary_chunks_in_boxes_without_a_list(S, dn):
             assert torch.equal(scan["idx"].cpu(), ref["idx"]), (t, t0)
             assert torch.equal(got["idx"].cpu(), ref["idx"]) and torch.equal(got["rq"].cpu(), ref["rq"]), (t, t0)
             assert bit_equal(got["out"], ref["out"]) and bit_equal(got["r_max"], ref["r_max"]), (t, t0)
+
+
+def _border_directions(n, g):
+    """Unit quaternions on and next to the borders of the search's boxes (27 per axis of the stereographic cube), turned by every
+    axis unit, some with equal or vanishing components."""
+    scale = (13.5 - 0.1) / 0.41422
+    z = (torch.randint(-14, 14, (n, 3), generator=g) + 0.5) / scale + torch.randn(n, 3, generator=g) * 10.0 ** -torch.randint(2, 7, (n, 1), generator=g)
+    z = torch.where(torch.rand(n, 3, generator=g) < 0.1, torch.zeros(()), z).clamp(-0.4142, 0.4142)
+    z = torch.where(torch.rand(n, 1, generator=g) < 0.1, z[:, :1].expand(n, 3), z)
+    s = (z * z).sum(1, keepdim=True)
+    w = torch.cat([(1 - s) / (1 + s), 2 * z / (1 + s)], 1)
+    turned = torch.stack([w, torch.stack([-w[:, 1], w[:, 0], -w[:, 3], w[:, 2]], 1), torch.stack([-w[:, 2], w[:, 3], w[:, 0], -w[:, 1]], 1),
+                          torch.stack([-w[:, 3], -w[:, 2], w[:, 1], w[:, 0]], 1)])
+    u = turned[torch.randint(0, 4, (n,), generator=g), torch.arange(n)]
+    return u * (1 - 2 * torch.randint(0, 2, (n, 1), generator=g))
+
+
+@pytest.mark.parametrize("dn", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("H,S,T,d_h", [(8, 96, 1100, 128), (3, 24, 2500, 64), (2, 341, 1500, 96)])
+def test_box_borders_and_many_rounds(H, S, T, d_h, dn):
+    """Long calls: blocks of several rounds, with heads that fill the XCDs evenly and heads that do not; norms from ordinary down to
+    where a wavefront leaves the short forms (16-bit subnormals), mixed with whole wavefronts that take them."""
+    from hqmq_amd import ops
+    dt = DT[dn]
+    g = torch.Generator().manual_seed(S + H)
+    J, slack = ops.build_joint(torch.randn(H, S, 4, generator=g).to(DEV), dt)
+    u = _border_directions(H * T * d_h // 4, g)
+    gain = torch.where(torch.rand(H * T, 1, generator=g) < 0.05, 10.0 ** -(3 + 4 * torch.rand(H * T, 1, generator=g)), 0.2 + 4 * torch.rand(H * T, 1, generator=g))
+    x = (u.view(H * T, -1) * gain).view(1, H, T, d_h).to(dt).to(DEV)
+    got = ops.quantize(x, J, slack, 4, want_dense=True)
+    scan = ops.quantize(x, J, slack.clone(), 4, want_dense=True)
+    assert hasattr(slack, "hqmq_grid")
+    assert torch.equal(got["idx"], scan["idx"]) and torch.equal(got["rq"], scan["rq"])
+    assert bit_equal(got["out"], scan["out"]) and bit_equal(got["r_max"], scan["r_max"])
