@@ -197,36 +197,38 @@ __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 
     __shared__ float rad[kListCap];
     __shared__ uint16_t id[kListCap];                          // as an entry
     __shared__ uint16_t entries[kBoxes][kBoxCap + 1];          // positions in the coarse list
-    __shared__ uint8_t out[kBoxes][kBoxCap + 2];               // beaten by another codeword of the box
+    __shared__ uint16_t kept[kBoxes][kBoxCap + 1];             // what stays of them, as entries
+    __shared__ float needs_sh[kBoxes][kBoxCap + 1];
     __shared__ int count[kBoxes];
     __shared__ float best_sh[kBuildThreads / 64];
-    __shared__ int arg_sh[kBuildThreads / 64], n_sh;
+    __shared__ int arg_sh[kBuildThreads / 64], n_sh, more_sh;
+    __shared__ uint32_t first_sh;
     const int K = 24 * S;
     const Codewords all = grid_codewords(grid, stride, H, S);
     const float4 *centre = all.centre + (size_t)h * K;
     const float *rho = all.rho + (size_t)h * K;
-    struct Box { float lo[3], hi[3]; float4 mid; float reach; bool met; };       // mid: the direction at its centre; reach: the farthest one's angle
+    // c: centre, hw: half width, c2: |c|^2; mid: the direction at the centre; reach: the farthest one's angle
+    struct Box { float c[3], hw, c2; float4 mid; float reach; bool met; };
     auto box_at = [](int i, int j, int k, int fine) {           // fine: fine boxes per axis of this one
         Box b;
         const int at[3] = {i, j, k};
-        const float hw = (0.5f * (float)fine + slack_boxes<D>()) * (1.f / kScale) + 2e-6f;
-        float c[3], near2 = 0.f, mid2 = 0.f, near[3];
+        b.hw = (0.5f * (float)fine + slack_boxes<D>()) * (1.f / kScale) + 2e-6f;
+        float near2 = 0.f, near[3];
+        b.c2 = 0.f;
         for (int a = 0; a < 3; a++) {
-            c[a] = ((float)(at[a] * fine - kMid) + 0.5f * (float)(fine - 1)) * (1.f / kScale);
-            b.lo[a] = c[a] - hw;
-            b.hi[a] = c[a] + hw;
-            near[a] = fmaxf(fabsf(c[a]) - hw, 0.f);
+            b.c[a] = ((float)(at[a] * fine - kMid) + 0.5f * (float)(fine - 1)) * (1.f / kScale);
+            near[a] = fmaxf(fabsf(b.c[a]) - b.hw, 0.f);
             near2 += near[a] * near[a];
-            mid2 += c[a] * c[a];
+            b.c2 += b.c[a] * b.c[a];
         }
         // the cell: |w_i| <= w0, that is |z|^2 + 2 |z_i| <= 1
         b.met = near2 + 2.f * fmaxf(near[0], fmaxf(near[1], near[2])) <= 1.0005f;
-        const float inv = 1.f / (1.f + mid2);
-        b.mid = float4{(1.f - mid2) * inv, 2.f * c[0] * inv, 2.f * c[1] * inv, 2.f * c[2] * inv};
-        b.reach = 2.f * 1.7321f * hw;
+        const float inv = 1.f / (1.f + b.c2);
+        b.mid = float4{(1.f - b.c2) * inv, 2.f * b.c[0] * inv, 2.f * b.c[1] * inv, 2.f * b.c[2] * inv};
+        b.reach = 2.f * 1.7321f * b.hw;
         return b;
     };
-    auto dot = [](float4 g, float4 m) { return g.x * m.x + g.y * m.y + g.z * m.z + g.w * m.w; };
+    auto dot = [](float4 g, float4 m) { return fmaf(g.w, m.w, fmaf(g.z, m.z, fmaf(g.y, m.y, g.x * m.x))); };
     // what g* has to lead by, less the radius of g: its own radius, the roundings of both scores, and of this kernel
     auto needs = [&](float4 star, float r, const Box &b) {
         // its largest score in the box: from the angle at the centre, less the box's reach
@@ -236,22 +238,14 @@ __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 
         const float most = (c > cr ? 1.f : fminf(c + s * sr, 1.f)) * len + r;
         return 1.016f * (most * 1.016f < 1.f ? 1.f : 2.f) * D::eps() + 1.2e-5f + r;
     };
-    // Is <g* - g, (1 - |z|^2, 2 z)> > m (1 + |z|^2) all over the box?  A sum of one parabola per coordinate.
+    // Is <d, (1 - |z|^2, 2 z)> > m (1 + |z|^2) with d = g* - g all over the box?  A sum of one parabola 2 d_i z - a z^2 per
+    // coordinate, a = d_0 + m: at least its value at the centre less the slope there times half the width, and less a hw^2
+    // where it bends down.
     auto beaten = [](float4 s, float need, float4 g, float r, const Box &b) {
-        const float d[4] = {s.x - g.x, s.y - g.y, s.z - g.z, s.w - g.w}, m = (need + r) * 1.0001f;
-        const float a = -(d[0] + m);
-        float lead = d[0] - m;
-        for (int i = 0; i < 3; i++) {
-            const float e = 2.f * d[i + 1];
-            const float at_lo = (e + a * b.lo[i]) * b.lo[i], at_hi = (e + a * b.hi[i]) * b.hi[i];
-            float least = fminf(at_lo, at_hi);
-            if (a > 0.f) {
-                const float z = fminf(fmaxf(-0.5f * e / a, b.lo[i]), b.hi[i]);
-                least = fminf(least, (e + a * z) * z);
-            }
-            lead += least;
-        }
-        return lead > 2e-6f;
+        const float d0 = s.x - g.x, d1 = s.y - g.y, d2 = s.z - g.z, d3 = s.w - g.w, m = (need + r) * 1.0001f, a = d0 + m;
+        const float slopes = fabsf(fmaf(-a, b.c[0], d1)) + fabsf(fmaf(-a, b.c[1], d2)) + fabsf(fmaf(-a, b.c[2], d3));
+        const float half = fmaf(d3, b.c[2], fmaf(d2, b.c[1], fmaf(d1, b.c[0], -b.hw * slopes)));
+        return fmaf(2.f, half, d0 - m) - fmaf(a, b.c2, 3.f * b.hw * b.hw * fmaxf(a, 0.f)) > 2e-6f;
     };
     uint4 *lists = grid + stride * h;
     const int f = tid / kLanes, part = tid % kLanes;
@@ -263,12 +257,12 @@ __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 
         if (mine && part == 0) lists[(i * kGrid + j) * kGrid + k] = empty;
         return;
     }
-    if (tid == 0) n_sh = 0;
+    if (tid == 0) n_sh = more_sh = 0;
     if (tid < kBoxes) count[tid] = 0;
     {
         float best = -INFINITY;
         int arg = 0;
-#pragma unroll 4
+#pragma unroll 8
         for (int k2 = tid; k2 < K; k2 += kBuildThreads) {
             const float v = dot(centre[k2], coarse.mid) - rho[k2];
             if (v > best) { best = v; arg = k2; }
@@ -284,10 +278,14 @@ __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 
             if (best_sh[w] > best || (best_sh[w] == best && arg_sh[w] < arg)) { best = best_sh[w]; arg = arg_sh[w]; }
         const float4 star = centre[arg];
         const float need = needs(star, rho[arg], coarse), inv_s = 1.f / (float)S;
+        float4 ahead = centre[min(tid, K - 1)];
+        float ahead_r = rho[min(tid, K - 1)];
         for (int k0 = 0; k0 < K; k0 += kBuildThreads) {
             const int k2 = k0 + tid;
-            const float4 g = centre[min(k2, K - 1)];
-            const float r = rho[min(k2, K - 1)];
+            const float4 g = ahead;
+            const float r = ahead_r;
+            ahead = centre[min(k2 + kBuildThreads, K - 1)];
+            ahead_r = rho[min(k2 + kBuildThreads, K - 1)];
             const bool take = k2 < K && !beaten(star, need, g, r, coarse);
             const uint64_t mask = __builtin_amdgcn_ballot_w64(take);
             int at = 0;
@@ -309,6 +307,7 @@ __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 
     if (wanted) {
         float best = -INFINITY;
         int arg = 0;
+#pragma unroll 4
         for (int e = part; e < n_list; e += kLanes) {
             const float v = dot(geo[e], b.mid) - rad[e];
             if (v > best) { best = v; arg = e; }
@@ -327,45 +326,51 @@ __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 
         }
     }
     __syncthreads();
-    // (a codeword that another one beats all over the box is beaten by one that stays: the leads add up)
-    if (wanted && count[f] <= kBoxCap) {
-        const int n = count[f];
-        for (int x = part; x < n; x += kLanes) {
-            const float4 g = geo[entries[f][x]];
-            const float r = rad[entries[f][x]];
-            bool lost = false;
-            for (int y = 0; y < n && !lost; y++) {
-                const float4 s = geo[entries[f][y]];
-                lost = y != x && beaten(s, needs(s, rad[entries[f][y]], b), g, r, b);
-            }
-            out[f][x] = lost;
-        }
-    }
+    // every codeword of the box against every other one (one that is beaten all over the box is beaten by one that stays: the
+    // leads add up), then the blocks, a lane each
+    if (wanted && count[f] <= kBoxCap)
+        for (int x = part; x < count[f]; x += kLanes) needs_sh[f][x] = needs(geo[entries[f][x]], rad[entries[f][x]], b);
     __syncthreads();
-    if (!mine || part) return;
     const int cell = (i * kGrid + j) * kGrid + k;
-    if (!b.met) { lists[cell] = empty; return; }
-    bool full = !listed || count[f] > kBoxCap;
+    const bool listed_here = wanted && count[f] <= kBoxCap;
+    const int all_n = listed_here ? count[f] : 0;
     int n = 0;
-    if (!full)
-        for (int x = 0; x < count[f]; x++)
-            if (!out[f][x]) entries[f][n++] = entries[f][x];
-    const int more = n > 7 ? (n - 1) / 7 : 0;                   // blocks from the pool
-    uint32_t next = 0;
-    if (more) {
-        next = atomicAdd(used, (uint32_t)more);
-        full = next + more > (uint32_t)pool;
+    for (int x0 = 0; x0 < all_n; x0 += kLanes) {
+        const int x = x0 + part;
+        bool stays = x < all_n;
+        int e = 0;
+        if (stays) {
+            e = entries[f][x];
+            const float4 g = geo[e];
+            const float r = rad[e];
+#pragma unroll 4
+            for (int y = 0; y < all_n; y++) stays &= y == x || !beaten(geo[entries[f][y]], needs_sh[f][y], g, r, b);
+        }
+        const uint32_t votes = (uint32_t)(__builtin_amdgcn_ballot_w64(stays) >> (lane & ~(kLanes - 1))) & ((1u << kLanes) - 1u);
+        if (stays) kept[f][n + __popc(votes & ((1u << part) - 1u))] = id[e];
+        n += __popc(votes);
     }
-    int at = cell;
-    for (int e0 = 0;; e0 += 7) {
+    // blocks from the pool, for all boxes together (every box asking for its own: the additions to the head's one counter took
+    // most of the build at bf16)
+    const int more = n > 7 ? (n - 1) / 7 : 0;
+    uint32_t next = 0;
+    if (more && part == 0) next = (uint32_t)atomicAdd(&more_sh, more);
+    __syncthreads();
+    if (tid == 0) first_sh = more_sh ? atomicAdd(used, (uint32_t)more_sh) : 0u;
+    __syncthreads();
+    if (!mine) return;
+    if (!b.met) {
+        if (part == 0) lists[cell] = empty;
+        return;
+    }
+    next = __shfl(next, 0, kLanes) + first_sh;
+    const bool full = !listed_here || next + more > (uint32_t)pool;
+    for (int q = part; q <= (full ? 0 : more); q += kLanes) {
         uint32_t w[8];
 #pragma unroll
-        for (int e = 0; e < 7; e++) w[e] = !full && e0 + e < n ? id[entries[f][e0 + e]] : kNone;
-        const bool last = full || e0 + 7 >= n;
-        w[7] = full ? 0xffffu : last ? 0u : next;
-        lists[at] = uint4{w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16};
-        if (last) break;
-        at = kCells + (int)next++;
+        for (int e = 0; e < 7; e++) w[e] = !full && 7 * q + e < n ? kept[f][7 * q + e] : kNone;
+        w[7] = full ? 0xffffu : q == more ? 0u : next + q;
+        lists[q == 0 ? cell : kCells + (int)next + q - 1] = uint4{w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16};
     }
 }
 
