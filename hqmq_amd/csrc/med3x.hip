@@ -7,10 +7,11 @@
 // multiplier, rounded to D.  The order statistics are exact: chunk norms are
 // non-negative, so their bit patterns sort like the values.  Calls of at most
 // 8192 chunks per head keep the keys in registers and search the key bit by bit
-// (one launch); larger ones take a 32768-bin histogram per head of the top 16
-// bits, which is the whole key of a 16-bit type, and for fp32 a second pass over
-// the low 16 bits of the bin(s) holding the two ranks.  K and V of one append
-// share the launches.
+// (one launch); larger ones of a 16-bit type take a 32768-bin histogram of its
+// whole key per block, which the selection adds up where it looks (two launches);
+// fp32, and calls too large for 16-bit counters, one histogram per head of the top
+// 16 bits, and fp32 a second pass over the low 16 bits of the bin(s) holding the
+// two ranks.  K and V of one append share the launches.
 //
 // hqmq_outlier_compact has no counterpart in the reference: it copies the
 // flagged chunks into the fp16/bf16/fp32 sideband in (token, chunk) order.
@@ -29,8 +30,16 @@ constexpr int kGroups = 64, kGroupBins = kBins1 / kGroups, kGroupAt = kBins1 - k
 
 // workspace (uint32 units): hist1[H][kBins1] | state[H][kState] | (fp32 only) hist2[H][2][kBins2]
 // state: 0 nan count, 1 key_lo, 2 key_hi, 3 rank_lo within bin, 4 rank_hi within bin
-__host__ __device__ inline int64_t ws_words(int H, bool f32) {
+// or, of a 16-bit type, per block of the histogram: bins[kBins1 / 2] (two 16-bit counters a word; only those of groups whose
+// sum is not zero are written) | sums[kGroups] | NaN count | padding
+constexpr int kPartWords = kBins1 / 2 + kGroups + 64, kPartSums = kBins1 / 2, kPartNan = kPartSums + kGroups;
+constexpr int kPartBlocks = 256;        // at most, and one per head where there are more heads
+__host__ __device__ inline int64_t ws_words_hist(int H, bool f32) {
     return (int64_t)H * (kBins1 + kState) + (f32 ? (int64_t)H * 2 * kBins2 : 0);
+}
+inline int64_t ws_words(int H, bool f32) {
+    const int64_t parts = f32 ? 0 : (int64_t)(H > kPartBlocks ? H : kPartBlocks) * kPartWords, hist = ws_words_hist(H, f32);
+    return parts > hist ? parts : hist;
 }
 
 // One tensor of a call, as the kernels see it; a launch takes one or two of equal shape (blockIdx.z).
@@ -122,23 +131,24 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
     return q[0] + q[1];
 }
 
-// Histogram of the top 16 bits: the 32768 bins live in LDS, and a block adds only its non-zero bins (some 3000 of an
-// ordinary tensor) to the global histogram.  Blocks of at most 65535 chunks pack two 16-bit counters in a word: 64 KB,
-// two blocks per CU and half the bins to clear and to look through (8 heads x 65536 chunks fp16: 44 us with one
-// global atomic per chunk).
+// fp32 and very large calls: a histogram of the top 16 bits per head.  The 32768 bins live in LDS, and a block adds only its
+// non-zero bins (some 3000 of an ordinary tensor) to the global histogram.  Blocks of at most 65535 chunks pack two 16-bit
+// counters in a word: 64 KB, two blocks per CU and half the bins to clear and to look through.  The groups' sums are collected in LDS first: all blocks of a head add to the same dozen words,
+// and with an atomic per 64 bins those additions, one after the other, were most of the kernel (8 heads x 32768 tokens fp16:
+// 54 us instead of 33).
 template <class D, bool WIDE>
 __global__ __launch_bounds__(1024) void med_hist_kernel(MedPair a, int64_t rows_per_block) {
-    extern __shared__ uint32_t lh[];    // [words] + 1 (NaN count)
-    constexpr int words = WIDE ? kBins1 : kBins1 / 2;
+    extern __shared__ uint32_t lh[];    // [words] | sums of the groups | NaN count
+    constexpr int words = WIDE ? kBins1 : kBins1 / 2, sums = words, nans = words + kGroups;
     const MedTensor &m = a.t[blockIdx.z];
     const int h = blockIdx.y;
     for (int i = threadIdx.x; i < words / 4; i += 1024) reinterpret_cast<uint4 *>(lh)[i] = uint4{0, 0, 0, 0};
-    if (threadIdx.x == 0) lh[words] = 0;
+    if (threadIdx.x <= kGroups) lh[sums + threadIdx.x] = 0;
     __syncthreads();
     const int64_t rows = (int64_t)a.B * a.T, r0 = blockIdx.x * rows_per_block;
     for_each_norm<D, 1024, 4>(m, a, h, r0, min(rows, r0 + rows_per_block), [&](float nrm) {
         const uint32_t key = norm_bits<D>(nrm) >> 16;
-        if (is_nan(nrm)) atomicAdd(&lh[words], 1u);
+        if (is_nan(nrm)) atomicAdd(&lh[nans], 1u);
         else if (WIDE) atomicAdd(&lh[key], 1u);
         else atomicAdd(&lh[key >> 1], 1u << (16 * (key & 1)));
     });
@@ -157,9 +167,11 @@ __global__ __launch_bounds__(1024) void med_hist_kernel(MedPair a, int64_t rows_
         }
         if (__builtin_amdgcn_ballot_w64(sum != 0u) == 0ull) continue;
         sum = wave_sum(sum);
-        if ((threadIdx.x & 63) == 0) atomicAdd(&hist1[kGroupAt + (WIDE ? i : 2 * i) / kGroupBins], sum);
+        if ((threadIdx.x & 63) == 0) atomicAdd(&lh[sums + (WIDE ? i : 2 * i) / kGroupBins], sum);
     }
-    if (threadIdx.x == 0 && lh[words]) atomicAdd(&med_state(m, a.H, h)[0], lh[words]);
+    __syncthreads();
+    if (threadIdx.x < kGroups && lh[sums + threadIdx.x]) atomicAdd(&hist1[kGroupAt + threadIdx.x], lh[sums + threadIdx.x]);
+    if (threadIdx.x == 0 && lh[nans]) atomicAdd(&med_state(m, a.H, h)[0], lh[nans]);
 }
 
 // fp32, second pass: low 16 bits of the norms whose top bits are a selected bin
@@ -246,6 +258,173 @@ __device__ __forceinline__ void nan_threshold(const MedTensor &m, int h) {
     m.median[h] = NAN;
     D::store((typename D::storage *)m.thr + h, NAN);
     if (m.n_out) m.n_out[h] = 0;
+}
+
+// 16-bit types, first of two launches: every block counts the keys of its rows (at most 65535 chunks) in 32768 bins in LDS,
+// two 16-bit counters a word, and stores the groups of bins that hold any, and the sums of all groups, in a part of the
+// workspace that is its own: nothing to clear beforehand and no atomics behind.  A wavefront's 16-byte reads take one group
+// at a time, so its sum is there when the words are, in registers, to be stored.  8 heads fp16, this launch and the selection:
+// 2048 tokens 17.7 -> 12.0 us, 32768 tokens 60 -> 23.5 (18.0 for this launch: 3.7 TB/s); with bins added to one histogram per
+// head by atomics, cleared by a launch of its own, the additions of the blocks to the same words took longer than the counting.
+template <class D>
+__global__ __launch_bounds__(1024) void med_hist16_kernel(MedPair a, int64_t rows_per_block) {
+    extern __shared__ uint32_t lh[];    // [kBins1 / 2] | NaN count
+    constexpr int words = kBins1 / 2;
+    const MedTensor &m = a.t[blockIdx.z];
+    const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int i = tid; i < words / 4; i += 1024) reinterpret_cast<uint4 *>(lh)[i] = uint4{0, 0, 0, 0};
+    if (tid == 0) lh[words] = 0;
+    __syncthreads();
+    const int64_t rows = (int64_t)a.B * a.T, r0 = blockIdx.x * rows_per_block;
+    for_each_norm<D, 1024, 4>(m, a, h, r0, min(rows, r0 + rows_per_block), [&](float nrm) {
+        const uint32_t key = norm_bits<D>(nrm) >> 16;
+        if (is_nan(nrm)) atomicAdd(&lh[words], 1u);
+        else atomicAdd(&lh[key >> 1], 1u << (16 * (key & 1)));
+    });
+    __syncthreads();
+    uint32_t *part = m.ws + (size_t)(h * gridDim.x + blockIdx.x) * kPartWords;
+    static_assert(kGroupBins / 2 == 4 * 64, "a group is one 16-byte read of a wavefront");
+#pragma unroll
+    for (int group = wave; group < kGroups; group += 16) {
+        const uint4 v = reinterpret_cast<const uint4 *>(lh)[group * 64 + lane];
+        auto both = [](uint32_t w) { return (w & 0xffffu) + (w >> 16); };
+        const uint32_t sum = wave_sum(both(v.x) + both(v.y) + both(v.z) + both(v.w));
+        if (sum) reinterpret_cast<uint4 *>(part)[group * 64 + lane] = v;
+        if (lane == 0) part[kPartSums + group] = sum;
+    }
+    if (tid == 0) part[kPartNan] = lh[words];
+}
+
+// The bin with rank `rank` among the 512 counters of a group, 8 per lane: its number, in the lane that holds it (-1 elsewhere).
+__device__ __forceinline__ uint32_t lanes_before(uint32_t v) {          // exclusive prefix sum over the wavefront
+    const int lane = threadIdx.x & 63;
+    uint32_t incl = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += u;
+    }
+    return incl - v;
+}
+__device__ __forceinline__ int bin_of_rank(const uint32_t (&v)[8], uint32_t rank) {
+    uint32_t tot = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) tot += v[i];
+    const uint32_t first = lanes_before(tot);
+    if (rank < first || rank >= first + tot) return -1;
+    rank -= first;
+    int i = 0;
+#pragma unroll
+    for (int k = 0; k < 7; k++)
+        if (i == k && rank >= v[k]) { rank -= v[k]; i = k + 1; }
+    return (int)(threadIdx.x & 63) * 8 + i;
+}
+
+// Second launch, one block per head: sums of the groups over the head's parts, the group of each rank, that group's bins over
+// the parts (a wavefront per part, 1 KB a time), the bin inside it.  The count wants the bins of the threshold's group as
+// well; the median's group leaves two for it nearly always, which are asked for along with the median's (a third round
+// trip otherwise: 6.9 -> 5.5 us; with every loop unrolled, 7.5: a launch this short waits for its code).
+template <class D>
+__global__ __launch_bounds__(1024) void med_select16_kernel(MedPair a, int parts) {
+    const MedTensor &m = a.t[blockIdx.z];
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t per_head = (uint32_t)((int64_t)a.B * a.T * a.n);
+    const uint32_t *ws = m.ws + (size_t)h * parts * kPartWords;
+    __shared__ uint32_t sums_sh[16][kGroups], bins_sh[4][kGroupBins], key_sh[2], nan_sh;
+    __shared__ uint64_t some_sh[kPartBlocks];           // the groups a part has any of
+    for (int i = tid; i < 4 * kGroupBins; i += 1024) (&bins_sh[0][0])[i] = 0;
+    if (tid == 0) nan_sh = 0;
+    uint32_t s = 0, nan = 0;
+    if (tid < parts) nan = ws[(size_t)tid * kPartWords + kPartNan];
+    for (int p0 = wave; p0 < parts; p0 += 32) {         // (two requested at a time)
+        const int p1 = p0 + 16;
+        const uint32_t v0 = ws[(size_t)p0 * kPartWords + kPartSums + lane], v1 = ws[(size_t)min(p1, parts - 1) * kPartWords + kPartSums + lane];
+        s += v0 + (p1 < parts ? v1 : 0u);
+        const uint64_t some0 = __builtin_amdgcn_ballot_w64(v0 != 0u), some1 = __builtin_amdgcn_ballot_w64(v1 != 0u);
+        if (lane == 0) {
+            some_sh[p0] = some0;
+            if (p1 < parts) some_sh[p1] = some1;
+        }
+    }
+    sums_sh[wave][lane] = s;
+    __syncthreads();
+    if (nan) nan_sh = 1;
+    uint32_t sum = 0;                                   // of group `lane`, in every wavefront
+#pragma unroll
+    for (int w = 0; w < 16; w++) sum += sums_sh[w][lane];
+    const uint32_t at = lanes_before(sum), rank[2] = {(per_head - 1) / 2, per_head / 2};
+    int group[2];
+    uint32_t rest[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint64_t here = __builtin_amdgcn_ballot_w64(rank[i] >= at && rank[i] < at + sum);
+        group[i] = here ? (int)__builtin_ctzll(here) : kGroups - 1;
+        rest[i] = rank[i] - __shfl(at, group[i]);
+    }
+    // the bins of group g, added up over the parts first, first + step, .. by this wavefront
+    auto gather = [&](int g, uint32_t *to, int first, int step) {
+        uint32_t v[8] = {};
+        for (int p0 = first; p0 < parts; p0 += 4 * step) {
+            uint4 x[4];                                 // (all four requested, also where the group was not written: not used then)
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[i] = reinterpret_cast<const uint4 *>(ws + (size_t)min(p0 + i * step, parts - 1) * kPartWords)[g * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const bool some = p0 + i * step < parts && (some_sh[min(p0 + i * step, parts - 1)] >> g & 1ull);
+                const uint32_t w[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
+#pragma unroll
+                for (int k = 0; k < 4; k++) { v[2 * k] += some ? w[k] & 0xffffu : 0u; v[2 * k + 1] += some ? w[k] >> 16 : 0u; }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (v[i]) atomicAdd(&to[lane * 8 + i], v[i]);
+    };
+    auto bins = [&](const uint32_t *from, uint32_t (&v)[8]) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = from[lane * 8 + i];
+    };
+    // the group of the threshold that a median of this key has (a threshold below every norm or beyond infinity: 0, or the last)
+    auto group_above = [&](float tv) { return (int)min((norm_bits<D>(fmaxf(tv, 0.f)) >> 16) / kGroupBins, (uint32_t)kGroups - 1u); };
+    const int top_lo = group_above(D::rnd(key_value<D>((uint32_t)(group[0] * kGroupBins)) * m.mult));
+    {
+        const int q = wave >> 2, g = q == 0 ? group[0] : q == 1 ? group[1] : min(top_lo + q - 2, kGroups - 1);
+        if (q < 2 || m.n_out) gather(g, bins_sh[q], wave & 3, 4);
+    }
+    __syncthreads();
+    if (nan_sh) {
+        if (tid == 0) nan_threshold<D>(m, h);
+        return;
+    }
+    if (wave < 2) {
+        const int side = wave;
+        uint32_t v[8];
+        bins(bins_sh[side], v);
+        const int bin = bin_of_rank(v, rest[side]);
+        if (bin >= 0) key_sh[side] = (uint32_t)(group[side] * kGroupBins + bin);
+    }
+    __syncthreads();
+    const bool same = rank[0] == rank[1];
+    const float lo = key_value<D>(key_sh[0]), hi = key_value<D>(key_sh[1]);
+    const float tv = D::rnd((same ? lo : hi - (hi - lo) * 0.5f) * m.mult);
+    if (tid == 0) finish_threshold<D>(lo, hi, same, m.mult, h, m.median, (typename D::storage *)m.thr);
+    if (!m.n_out) return;
+    // chunks with norm > thr: whole groups above the one that holds the threshold, and the bins above it in there
+    const int top = group_above(tv);
+    uint32_t *there = bins_sh[top == top_lo ? 2 : 3];
+    if (top != top_lo && top != top_lo + 1) {           // the median's bin is far from its group's first
+        for (int i = tid; i < kGroupBins; i += 1024) there[i] = 0;
+        __syncthreads();
+        gather(top, there, wave, 16);
+        __syncthreads();
+    }
+    if (wave != 0) return;
+    uint32_t v[8], n = lane > top ? sum : 0u;
+    bins(there, v);
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        if (key_value<D>((uint32_t)(top * kGroupBins + lane * 8 + i)) > tv) n += v[i];
+    n = wave_sum(n);
+    if (lane == 0) m.n_out[h] = (int32_t)n;
 }
 
 // One wavefront per rank: the group that holds it (64 sums), then the bin inside the group (8 bins per lane).
@@ -693,27 +872,45 @@ static int run_med3x(const MedPair &a, int count, hipStream_t st) {
         else hipLaunchKernelGGL((med_small_kernel<D, 1024, 8>), grid, dim3(1024), 0, st, a);
         return hip_status(hipGetLastError());
     }
-    const int64_t words = ws_words(a.H, f32);
+    // Blocks of about 4096 chunks while that leaves at most two per CU; larger calls get larger blocks, beyond 65535 chunks
+    // with 32-bit counters, one block per CU and tensor.
+    const int rps = a.n <= 1024 ? 1024 / a.n : 1;        // rows a block takes per step
+    auto blocks_of = [&](int64_t most, int64_t &rpb) {
+        int64_t blocks = (per_head + 4095) / 4096;
+        most = most > 0 ? most : 1;
+        if (blocks > most) blocks = most;
+        rpb = (rows + blocks - 1) / blocks;
+        rpb = (rpb + rps - 1) / rps * rps;
+        return (rows + rpb - 1) / rpb;
+    };
+    int64_t rpb, blocks;
+    if constexpr (D::code != HQMQ_F32) {
+        blocks = blocks_of(kPartBlocks / a.H, rpb);
+        if (rpb * a.n <= 65535) {
+            const size_t lds = ((size_t)kBins1 / 2 + 1) * sizeof(uint32_t);
+            const hipError_t e = hipFuncSetAttribute((const void *)med_hist16_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return (int)e;
+            hipLaunchKernelGGL(med_hist16_kernel<D>, dim3((unsigned)blocks, a.H, count), dim3(1024), lds, st, a, rpb);
+            hipLaunchKernelGGL(med_select16_kernel<D>, dim3(a.H, 1, count), dim3(1024), 0, st, a, (int)blocks);
+            return hip_status(hipGetLastError());
+        }
+    }
+    const int64_t words = ws_words_hist(a.H, f32);
     hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)(words / 1024 < 1024 ? (words + 1023) / 1024 : 1024), count), dim3(256), 0, st, a.t[0].ws,
                        a.t[count - 1].ws, words);
-    // Blocks of about 4096 chunks while that leaves at most two per CU; larger calls get larger blocks (each costs its
-    // 32768 bins and some 3000 atomics), beyond 65535 chunks with 32-bit counters, one block per CU and tensor.
-    const int rps = a.n <= 1024 ? 1024 / a.n : 1;        // rows a block takes per step
-    int64_t blocks = (per_head + 4095) / 4096;
-    const int64_t most = 512 / ((int64_t)a.H * count) > 0 ? 512 / ((int64_t)a.H * count) : 1;
-    if (blocks > most) blocks = most;
-    bool wide = (rows + blocks - 1) / blocks * a.n > 60000;
+    blocks = blocks_of(512 / ((int64_t)a.H * count), rpb);
+    bool wide = rpb * a.n > 60000;
     if (wide) {
         blocks = 256 / ((int64_t)a.H * count) > 0 ? 256 / ((int64_t)a.H * count) : 1;
         if (blocks < 16) blocks = 16;
+        rpb = (rows + blocks - 1) / blocks;
+        rpb = (rpb + rps - 1) / rps * rps;
+        blocks = (rows + rpb - 1) / rpb;
+        wide = rpb * a.n > 65535;
     }
-    int64_t rpb = (rows + blocks - 1) / blocks;
-    rpb = (rpb + rps - 1) / rps * rps;
-    wide = rpb * a.n > 65535;
-    blocks = (rows + rpb - 1) / rpb;
     const dim3 grid((unsigned)blocks, a.H, count);
     auto kern = wide ? med_hist_kernel<D, true> : med_hist_kernel<D, false>;
-    const size_t lds = ((size_t)(wide ? kBins1 : kBins1 / 2) + 1) * sizeof(uint32_t);
+    const size_t lds = ((size_t)(wide ? kBins1 : kBins1 / 2) + kGroups + 1) * sizeof(uint32_t);
     const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
     hipLaunchKernelGGL(kern, grid, dim3(1024), lds, st, a, rpb);

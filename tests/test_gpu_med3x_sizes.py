@@ -98,3 +98,30 @@ def test_crop_of_a_cache_made_for_cuda_without_an_index():
     assert K.sb_count.flatten().tolist() == [2 * 40, 2 * 128] and V.sb_count.flatten().tolist() == [2 * 40, 2 * 128]
     K.crop_(16)
     assert K.sb_count.flatten().tolist() == [2 * 16, 2 * 16] and not bool(K.flags[:, :, 16:].any())
+
+
+@pytest.mark.parametrize("dn", ["fp16", "bf16"])
+@pytest.mark.parametrize("H,rows,mult", [(1, 4100, 3.0), (7, 600, 100.0), (300, 257, 0.01), (2, 4097, 0.0), (3, 5000, 1e5)])
+def test_histograms_of_blocks(dn, H, rows, mult):
+    """16-bit types beyond 8192 chunks per head: one part of the workspace per block, from one part for a head to as many as a
+    launch may have; thresholds in the median's group of bins, next to it and far from it; the two middle norms in different
+    groups; a head of equal norms; infinite norms, NaN and zeros."""
+    from hqmq_amd import ops
+    dt = DT[dn]
+    x = kv_input((1, H, rows, 128), dt, seed=H + rows, outlier_p=0.03)
+    if H >= 3:
+        half = rows * 16                                    # of rows * 32 chunks
+        x[0, 1] = 0.25
+        x[0, 1].view(-1, 4)[half:] *= 4096.0                # the middle two: 0.5 and 2048
+        x[0, 2] = 1.5
+    if H >= 7:
+        x[0, 3].view(-1, 4)[:40] = float("inf")
+        x[0, 4, 5, 7] = float("nan")
+        x[0, 5].view(-1, 4)[: half + 9] = 0
+        x[0, 6].view(-1, 4)[:] = 6e-5 * (1 + torch.arange(rows * 32) % 9).to(dt).view(-1, 1)
+    want = CO.med3x(x, mult)
+    med, thr, cnt = ops.med3x_threshold(x.to(DEV), mult)
+    assert bit_equal(med, want["median"]) and bit_equal(thr, want["threshold"])
+    assert torch.equal(cnt.cpu().long(), want["mask"].sum(dim=(0, 2, 3)))
+    again = ops.med3x_threshold(x.to(DEV), mult)            # over what the first call left in the workspace
+    assert bit_equal(again[0], med) and bit_equal(again[1], thr) and torch.equal(again[2], cnt)
