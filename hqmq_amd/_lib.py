@@ -99,7 +99,7 @@ EXPORTS = [
     "hqmq_pack_codes", "hqmq_dequant_packed", "hqmq_attn_workspace_bytes", "hqmq_attn_pick_splits", "hqmq_attn_splits",
     "hqmq_attn_fwd", "hqmq_attn_combine", "hqmq_append_kv", "hqmq_attn_static_scratch_bytes", "hqmq_attn_fwd_static",
     "hqmq_search_grid_bytes", "hqmq_search_grid_kept_bytes", "hqmq_build_search_grid", "hqmq_quantize_grid", "hqmq_append_kv_grid", "hqmq_crop",
-    "hqmq_pack_kv",
+    "hqmq_pack_kv", "hqmq_med3x_workspace_best_bytes",
 ]
 BENCH_EXPORTS = ["hqmq_bench_read_planes_sink_bytes", "hqmq_bench_read_planes", "hqmq_bench_read_plain", "hqmq_bench_read_lds",
                  "hqmq_bench_empty"]
@@ -118,7 +118,7 @@ def lib():
         L = C.CDLL(str(_SO))
         L.hqmq_status_string.restype = C.c_char_p
         L.hqmq_status_string.argtypes = [C.c_int]
-        for name in ("hqmq_med3x_workspace_bytes", "hqmq_attn_workspace_bytes", "hqmq_attn_static_scratch_bytes",
+        for name in ("hqmq_med3x_workspace_bytes", "hqmq_med3x_workspace_best_bytes", "hqmq_attn_workspace_bytes", "hqmq_attn_static_scratch_bytes",
                      "hqmq_search_grid_bytes", "hqmq_search_grid_kept_bytes"):
             getattr(L, name).restype = i64
         # the calls of a decode loop take addresses as plain integers

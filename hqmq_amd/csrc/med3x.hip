@@ -9,9 +9,9 @@
 // 8192 chunks per head keep the keys in registers and search the key bit by bit
 // (one launch); larger ones of a 16-bit type take a 32768-bin histogram of its
 // whole key per block, which the selection adds up where it looks (two launches);
-// fp32, and calls too large for 16-bit counters, one histogram per head of the top
-// 16 bits, and fp32 a second pass over the low 16 bits of the bin(s) holding the
-// two ranks.  K and V of one append share the launches.
+// fp32, calls too large for 16-bit counters and workspaces too small for that take
+// one histogram per head of the top 16 bits, and fp32 a second pass over the low 16
+// bits of the bin(s) holding the two ranks.  K and V of one append share the launches.
 //
 // hqmq_outlier_compact has no counterpart in the reference: it copies the
 // flagged chunks into the fp16/bf16/fp32 sideband in (token, chunk) order.
@@ -34,13 +34,10 @@ constexpr int kGroups = 64, kGroupBins = kBins1 / kGroups, kGroupAt = kBins1 - k
 // sum is not zero are written) | sums[kGroups] | NaN count | padding
 constexpr int kPartWords = kBins1 / 2 + kGroups + 64, kPartSums = kBins1 / 2, kPartNan = kPartSums + kGroups;
 constexpr int kPartBlocks = 256;        // at most, and one per head where there are more heads
-__host__ __device__ inline int64_t ws_words_hist(int H, bool f32) {
+__host__ __device__ inline int64_t ws_words(int H, bool f32) {
     return (int64_t)H * (kBins1 + kState) + (f32 ? (int64_t)H * 2 * kBins2 : 0);
 }
-inline int64_t ws_words(int H, bool f32) {
-    const int64_t parts = f32 ? 0 : (int64_t)(H > kPartBlocks ? H : kPartBlocks) * kPartWords, hist = ws_words_hist(H, f32);
-    return parts > hist ? parts : hist;
-}
+inline int64_t ws_words_parts(int H) { return (int64_t)(H > kPartBlocks ? H : kPartBlocks) * kPartWords; }
 
 // One tensor of a call, as the kernels see it; a launch takes one or two of equal shape (blockIdx.z).
 struct MedTensor {
@@ -131,7 +128,7 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
     return q[0] + q[1];
 }
 
-// fp32 and very large calls: a histogram of the top 16 bits per head.  The 32768 bins live in LDS, and a block adds only its
+// fp32, very large calls and small workspaces: a histogram of the top 16 bits per head.  The 32768 bins live in LDS, and a block adds only its
 // non-zero bins (some 3000 of an ordinary tensor) to the global histogram.  Blocks of at most 65535 chunks pack two 16-bit
 // counters in a word: 64 KB, two blocks per CU and half the bins to clear and to look through.  The groups' sums are collected in LDS first: all blocks of a head add to the same dozen words,
 // and with an atomic per 64 bins those additions, one after the other, were most of the kernel (8 heads x 32768 tokens fp16:
@@ -857,8 +854,14 @@ extern "C" int64_t hqmq_med3x_workspace_bytes(int H, int dtype) {
     return ws_words(H, dtype == HQMQ_F32) * 4;
 }
 
+extern "C" int64_t hqmq_med3x_workspace_best_bytes(int H, int dtype) {
+    if (H < 1) return 0;
+    const int64_t least = ws_words(H, dtype == HQMQ_F32) * 4, parts = dtype == HQMQ_F32 ? 0 : ws_words_parts(H) * 4;
+    return parts > least ? parts : least;
+}
+
 template <class D>
-static int run_med3x(const MedPair &a, int count, hipStream_t st) {
+static int run_med3x(const MedPair &a, int count, bool parts, hipStream_t st) {
     const bool f32 = D::code == HQMQ_F32;
     const int64_t per_head = (int64_t)a.B * a.T * a.n, rows = (int64_t)a.B * a.T;
     // Few keys per lane before few lanes: such a call lasts about as long as its code takes to arrive (every launch starts
@@ -886,7 +889,7 @@ static int run_med3x(const MedPair &a, int count, hipStream_t st) {
     int64_t rpb, blocks;
     if constexpr (D::code != HQMQ_F32) {
         blocks = blocks_of(kPartBlocks / a.H, rpb);
-        if (rpb * a.n <= 65535) {
+        if (parts && rpb * a.n <= 65535) {
             const size_t lds = ((size_t)kBins1 / 2 + 1) * sizeof(uint32_t);
             const hipError_t e = hipFuncSetAttribute((const void *)med_hist16_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) return (int)e;
@@ -895,7 +898,7 @@ static int run_med3x(const MedPair &a, int count, hipStream_t st) {
             return hip_status(hipGetLastError());
         }
     }
-    const int64_t words = ws_words_hist(a.H, f32);
+    const int64_t words = ws_words(a.H, f32);
     hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)(words / 1024 < 1024 ? (words + 1023) / 1024 : 1024), count), dim3(256), 0, st, a.t[0].ws,
                        a.t[count - 1].ws, words);
     blocks = blocks_of(512 / ((int64_t)a.H * count), rpb);
@@ -933,11 +936,12 @@ static int check_med3x(const Med3xCall &c) {
     return HQMQ_OK;
 }
 
-static int med3x_launch(const MedPair &a, int dtype, int count, hipStream_t st) {
+// parts: the workspaces hold a part per block
+static int med3x_launch(const MedPair &a, int dtype, int count, bool parts, hipStream_t st) {
     switch (dtype) {
-        case HQMQ_F32: return run_med3x<F32>(a, count, st);
-        case HQMQ_F16: return run_med3x<F16>(a, count, st);
-        default: return run_med3x<BF16>(a, count, st);
+        case HQMQ_F32: return run_med3x<F32>(a, count, false, st);
+        case HQMQ_F16: return run_med3x<F16>(a, count, parts, st);
+        default: return run_med3x<BF16>(a, count, parts, st);
     }
 }
 
@@ -952,12 +956,16 @@ int hqmq::med3x_calls(const Med3xCall *c, int count, hipStream_t st) {
     }
     // one set of launches for both tensors where their shapes agree and their workspaces are apart
     if (count == 2 && c[0].dtype == c[1].dtype && c[0].B == c[1].B && c[0].H == c[1].H && c[0].T == c[1].T && c[0].n == c[1].n) {
-        const int64_t need = hqmq_med3x_workspace_bytes(c[0].H, c[0].dtype);
         const uintptr_t w0 = (uintptr_t)c[0].ws, w1 = (uintptr_t)c[1].ws;
-        if (w0 + need <= w1 || w1 + need <= w0) return med3x_launch(MedPair{{t[0], t[1]}, c[0].B, c[0].H, c[0].T, c[0].n}, c[0].dtype, 2, st);
+        auto apart = [&](int64_t need) { return w0 + need <= w1 || w1 + need <= w0; };
+        const int64_t best = hqmq_med3x_workspace_best_bytes(c[0].H, c[0].dtype);
+        const bool parts = c[0].ws_bytes >= best && c[1].ws_bytes >= best && apart(best);
+        if (parts || apart(hqmq_med3x_workspace_bytes(c[0].H, c[0].dtype)))
+            return med3x_launch(MedPair{{t[0], t[1]}, c[0].B, c[0].H, c[0].T, c[0].n}, c[0].dtype, 2, parts, st);
     }
     for (int i = 0; i < count; i++) {
-        const int rc = med3x_launch(MedPair{{t[i], t[i]}, c[i].B, c[i].H, c[i].T, c[i].n}, c[i].dtype, 1, st);
+        const bool parts = c[i].ws_bytes >= hqmq_med3x_workspace_best_bytes(c[i].H, c[i].dtype);
+        const int rc = med3x_launch(MedPair{{t[i], t[i]}, c[i].B, c[i].H, c[i].T, c[i].n}, c[i].dtype, 1, parts, st);
         if (rc) return rc;
     }
     return HQMQ_OK;

@@ -183,7 +183,7 @@ def _med_workspace(x: torch.Tensor, tag: str) -> torch.Tensor:
     key = (H, f32)
     nbytes = _MED_BYTES.get(key)
     if nbytes is None:
-        nbytes = _MED_BYTES[key] = int(L.lib().hqmq_med3x_workspace_bytes(C.c_int(H), C.c_int(_dt(x))))
+        nbytes = _MED_BYTES[key] = int(L.lib().hqmq_med3x_workspace_best_bytes(C.c_int(H), C.c_int(_dt(x))))
     return _workspace(nbytes + 12 * H + 16, x.device, tag)        # behind it: room for a median and a threshold nobody asked for
 
 

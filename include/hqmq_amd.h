@@ -122,10 +122,13 @@ int hqmq_quantize_grid(const hqmq_quantize_args *a, const void *grid, void *stre
 /* Med3x statistics: per-head median of the chunk norms of one call and the
  * threshold RNE_D(median * mult).  Replaces the torch.quantile half of
  * OutlierAwareHQMQQuantizer._qdq (src/quantizers/outlier_aware.py:60-69).
- *   workspace  hqmq_med3x_workspace_bytes(H, dtype) bytes, any content
+ *   workspace  at least hqmq_med3x_workspace_bytes(H, dtype) bytes, any content, 16-byte aligned for best; from
+ *              hqmq_med3x_workspace_best_bytes(H, dtype) on (16.9 MB up to 256 heads of a 16-bit type) calls beyond 8192
+ *              chunks per head take two launches instead of three and a third to two thirds of the time
  *   median     [H] fp32 (out);  thr [H] D (out);  n_out [H] int32 (out, may be NULL):
  *              number of chunks with norm > thr */
 int64_t hqmq_med3x_workspace_bytes(int H, int dtype);
+int64_t hqmq_med3x_workspace_best_bytes(int H, int dtype);
 int hqmq_med3x_threshold(const void *x, int64_t x_stride_b, int64_t x_stride_h, int64_t x_stride_t, int dtype,
                          int B, int H, int T, int n_chunks, float mult, void *workspace, int64_t workspace_bytes,
                          float *median, void *thr, int32_t *n_out, void *stream);
@@ -186,7 +189,7 @@ int hqmq_crop(const hqmq_crop_args *a, void *stream);
 typedef struct hqmq_append_args {
     hqmq_quantize_args q;
     float median_mult;
-    void *med_workspace; int64_t med_workspace_bytes;  /* hqmq_med3x_workspace_bytes(H, dtype) */
+    void *med_workspace; int64_t med_workspace_bytes;  /* hqmq_med3x_workspace_bytes(H, dtype), or .._best_bytes */
     float *median; void *thr; int32_t *n_out;          /* [H] outputs: fp32, D, int32 (n_out may be NULL) */
     void *sideband; int64_t sb_cap;
     int32_t *sb_tile_off, *sb_count, *overflow;

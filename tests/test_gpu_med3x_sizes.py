@@ -106,7 +106,7 @@ def test_histograms_of_blocks(dn, H, rows, mult):
     """16-bit types beyond 8192 chunks per head: one part of the workspace per block, from one part for a head to as many as a
     launch may have; thresholds in the median's group of bins, next to it and far from it; the two middle norms in different
     groups; a head of equal norms; infinite norms, NaN and zeros."""
-    from hqmq_amd import ops
+    from hqmq_amd import _lib, ops
     dt = DT[dn]
     x = kv_input((1, H, rows, 128), dt, seed=H + rows, outlier_p=0.03)
     if H >= 3:
@@ -125,3 +125,9 @@ def test_histograms_of_blocks(dn, H, rows, mult):
     assert torch.equal(cnt.cpu().long(), want["mask"].sum(dim=(0, 2, 3)))
     again = ops.med3x_threshold(x.to(DEV), mult)            # over what the first call left in the workspace
     assert bit_equal(again[0], med) and bit_equal(again[1], thr) and torch.equal(again[2], cnt)
+    # the smaller workspace: one histogram per head
+    xg, med2, thr2, cnt2 = x.to(DEV), torch.empty_like(med), torch.empty_like(thr), torch.empty_like(cnt)
+    ws = torch.full((_lib.lib().hqmq_med3x_workspace_bytes(H, _lib.DT_CODE[dt]),), 255, dtype=torch.uint8, device=DEV)
+    _lib.call(_lib.lib().hqmq_med3x_threshold, "hqmq_med3x_threshold", 0, xg.data_ptr(), *xg.stride()[:3], _lib.DT_CODE[dt], 1, H, rows, 32, mult,
+              ws.data_ptr(), ws.numel(), med2.data_ptr(), thr2.data_ptr(), cnt2.data_ptr())
+    assert bit_equal(med2, med) and bit_equal(thr2, thr) and torch.equal(cnt2, cnt)
