@@ -496,28 +496,52 @@ extern "C" int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, i
     return (int64_t)B * H_q * T_q * n_splits * (d_h + kPartialHead) * 4;
 }
 
-// Blocks per (sequence, KV head, column group): one block per CU, blocks of at least 128 tokens (short contexts are
-// bound by the launch's fixed costs: more, shorter blocks are faster down to that size even though half of such a
-// block's wavefronts have no half-step).
+// How many blocks share the tokens of one (sequence, KV head, 16 columns); `base` of these there are.  A block runs alone on its
+// compute unit, so that blocks come in rounds of 256, and one block more than a round costs a whole one: the estimate is
+// rounds x (start of a block + its tokens) + merge, in tokens of d_h 128 (4.6 us per 1000 over plain fp16 caches).  A start, tables
+// and query, is worth 500 of them; `merge`, the second launch and the blocks' way through memory, 500 over plain caches, 350 where
+// the radii have a plane of their own, 250 over outlier caches and 100 in the generic kernels, whose tokens cost more; a split more 5.
+// Sequences of different lengths, started longest first, even out: a round counts by its share, 0.8 of the blocks (mean over the
+// longest) and 0.3 for the last ones.  Measured against the best of 8 to 14 counts at 120 shapes with equal lengths, 101 with lengths
+// of their own (6 cache layouts, 4 to 400 heads, 600 to 20000 tokens) and 230 of 1 to 7 queries replayed in graphs, the choice takes
+// 0.5, 1.9 and 0.5 % longer; 256 blocks rounded up (512 over such lengths), the rule before, took 25, 32 and 23 %.  us before -> now:
+// s96_r4 fp16, 32 / 8 heads of 128, 1 x 300 tokens 10.7 -> 7.0 (one block, no merge), 3 x 20000 30.2 -> 20.0, 10 x 6000 28.4 -> 20.6,
+// 20 x 600 14.9 -> 8.5; s24_r3 bf16 with verbatim chunks, 10 x 6000 47.4 -> 34.2.
+static int decode_splits(int64_t base, int T_kv, bool ragged, double unit, double merge) {
+    if (base < 1) return 1;
+    int64_t top = ((int64_t)T_kv + 2 * kSuper - 1) / (2 * kSuper);       // blocks of at least 128 tokens (4k tokens: 32 splits, 8.7 against 8.95 us)
+    if (top > 512) top = 512;
+    if (top > 1024 / base) top = 1024 / base;                              // past four rounds the last one weighs little: 832 blocks of 9000 tokens 104 us, halved 128
+    const int64_t tiles = ((int64_t)T_kv + kSuper - 1) / kSuper;
+    double least = 0.0;
+    int best = 1;
+    for (int64_t s = 1; s <= top || s == 1; s++) {
+        const int64_t blocks = base * s;
+        double rounds = ragged ? 0.8 / 256 * (double)blocks + 0.3 : (double)((blocks + 255) / 256);
+        if (rounds < 1.0) rounds = 1.0;
+        const double t = rounds * (500.0 + unit * (double)((tiles + s - 1) / s * kSuper)) + (s > 1 ? merge + 5.0 * (double)s : 0.0);
+        if (s == 1 || t < least) { least = t; best = (int)s; }
+    }
+    return best;
+}
+
+// From the shapes alone, and never more than the 256 blocks rounded up (512 of sequences of different lengths) that callers with
+// a workspace of their own size were told before.
 extern "C" int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv, int ragged) {
     if (B < 1 || H_q < 1 || H_kv < 1 || T_q < 1 || T_kv < 1) return 1;
     const int G = H_q / H_kv;
-    const int64_t base = (int64_t)B * H_kv * ((T_q * G + 15) / 16);
-    // sequences of different lengths: two rounds of blocks, started longest first (batch_order), even out the finishing
-    // times (config 4, 512 (sequence, head) pairs: 248 us with one block per pair, 264 with two, 287 with four)
-    const int64_t target = ragged ? 512 : 256;
-    int64_t s = (target + base - 1) / base;
-    const int64_t cap = (T_kv + 2 * kSuper - 1) / (2 * kSuper);       // blocks of at least 128 tokens (4k tokens: 32 splits, 8.7 against 8.95 us)
-    if (s > cap) s = cap;
-    if (s < 1) s = 1;
-    if (s > 512) s = 512;
-    return (int)s;
+    const int64_t base = (int64_t)B * H_kv * (((int64_t)T_q * G + 15) / 16), target = ragged ? 512 : 256;
+    const int s = decode_splits(base, T_kv, ragged != 0, 1.0, 500.0);
+    return s > 1 && s > (target + base - 1) / base ? (int)((target + base - 1) / base) : s;
 }
 
 extern "C" int hqmq_attn_splits(const hqmq_attn_args *a) {
     if (!a || a->B < 1 || a->H_kv < 1 || a->H_q < 1 || a->T_q < 1 || a->T_kv < 1) return 1;
     const int splits = attn_prefill_splits(a, 0);
-    return splits > 0 ? splits : hqmq_attn_pick_splits(a->B, a->H_q, a->H_kv, a->T_q, a->T_kv, a->kv_len != nullptr);
+    if (splits > 0) return splits;
+    const bool generic = a->dtype == HQMQ_F32 || a->wide_range || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
+    return decode_splits((int64_t)a->B * a->H_kv * (((int64_t)a->T_q * (a->H_q / a->H_kv) + 15) / 16), a->T_kv, a->kv_len != nullptr,
+                         a->n_chunks / 32.0, generic ? 100.0 : a->K.flag_plane ? 250.0 : a->aux_bits ? 350.0 : 500.0);
 }
 
 extern "C" int hqmq_attn_combine(const void *workspace, void *O, int dtype, int B, int H_q, int T_q, int d_h, int n_splits,

@@ -430,7 +430,7 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
     plan = Kc._attn_plans.get((shape, stride))
     if plan is None or plan[0] is not ks or plan[1] is not vs or plan[2] is not Q.dtype:
         plan = _attn_plan(Q, Kc, Vc, ks, vs)
-    _, _, _, tmpl, o_stride, rows, floats = plan
+    _, _, _, tmpl, o_stride, rows, floats, splits = plan
     dev = Q.device
     index = dev.index
     O = torch.empty_like(Q) if out is None else out
@@ -459,10 +459,6 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
         a.batch_order = batch_order.data_ptr()
     if causal:
         a.causal, a.causal_offset = 1, causal_offset
-    many = False
-    if n_splits <= 0:
-        n_splits = pick_splits(shape[0], shape[1], Kc.H, shape[2], max(T_kv, 1), kv_lens is not None)
-        many = shape[2] > 1 and not static_scratch
     if skip_combine:
         a.skip_combine = 1
     if force_generic:
@@ -473,8 +469,18 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
         a.wide_range = 1
     if kernel_events is not None:
         a.start_event, a.stop_event = kernel_events
-    if many:
-        n_splits = L.lib().hqmq_attn_splits(C.addressof(a))
+    if n_splits <= 0:
+        if static_scratch:
+            n_splits = pick_splits(shape[0], shape[1], Kc.H, shape[2], max(T_kv, 1), kv_lens is not None)
+        elif shape[2] > 1 or shape[1] >= 64 * Kc.H:        # the prefill kernels may take it: the choice looks at more than the key below
+            n_splits = L.lib().hqmq_attn_splits(C.addressof(a))
+        else:                                      # of one token, the library's choice changes at multiples of 64 tokens only
+            key = ((T_kv + 63) // 64, kv_lens is None, a.wide_range, a.force_generic)
+            n_splits = splits.get(key)
+            if n_splits is None:
+                if len(splits) >= 4096:
+                    splits.clear()
+                n_splits = splits[key] = L.lib().hqmq_attn_splits(C.addressof(a))
     a.n_splits = n_splits
     if static_scratch:
         L.call(L.lib().hqmq_attn_fwd_static, "hqmq_attn_fwd_static", index, C.addressof(a))
@@ -607,7 +613,7 @@ def _fused_plan(Q: torch.Tensor, idx: torch.Tensor, T_v: int, K: int, K_v: int, 
 
 def _attn_plan(Q: torch.Tensor, Kc, Vc, ks, vs):
     """What a shape of Q and a pair of packed tensors fix of an attention call, kept with the K cache: the argument block,
-    the strides of an output like Q, the partial rows and floats per row and split."""
+    the strides of an output like Q, the partial rows and floats per row and split, the library's split counts by context."""
     B, Hq, Tq, d_h = Q.shape
     if d_h != Kc.d_head or d_h != Vc.d_head:
         raise AssertionError(f"d_h={d_h} != n_chunks*4={Kc.d_head}")
@@ -627,7 +633,7 @@ def _attn_plan(Q: torch.Tensor, Kc, Vc, ks, vs):
     a.softmax_scale = d_h ** -0.5
     per_split = int(L.lib().hqmq_attn_workspace_bytes(C.c_int(B), C.c_int(Hq), C.c_int(Tq), C.c_int(d_h), C.c_int(2))) // 8
     rows = B * Hq * Tq
-    plan = (ks, vs, Q.dtype, a, o_stride, rows, per_split // rows)
+    plan = (ks, vs, Q.dtype, a, o_stride, rows, per_split // rows, {})
     if len(Kc._attn_plans) >= 64:                  # shapes that no longer come
         Kc._attn_plans.clear()
     Kc._attn_plans[(Q.shape, Q.stride())] = plan

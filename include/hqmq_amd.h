@@ -308,10 +308,12 @@ typedef struct hqmq_attn_args {
                                  when it leaves [2^-8, 2^15); data of ordinary magnitude never does. */
 } hqmq_attn_args;
 int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, int n_splits);
-/* The n_splits hqmq_attn_fwd would choose; ragged = 1 when kv_len is passed (more, smaller blocks). */
+/* The n_splits hqmq_attn_fwd would choose, from the shapes alone; ragged = 1 when kv_len is passed (sequences of different
+   lengths). */
 int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv, int ragged);
 /* The n_splits that suits these arguments best (a->n_splits is not looked at), for callers that size the workspace by it:
-   chunked prefill wants other counts than hqmq_attn_pick_splits names from the shapes alone. */
+   chunked prefill, heads of 64 and outlier caches want other counts than hqmq_attn_pick_splits names.  May be larger than
+   that one's.  Of one query per sequence it changes at multiples of 64 tokens only. */
 int hqmq_attn_splits(const hqmq_attn_args *a);
 int hqmq_attn_fwd(const hqmq_attn_args *a, void *stream);
 /* Merge of the split-KV partials (m, l, acc) left in the workspace; hqmq_attn_fwd runs it unless skip_combine. */

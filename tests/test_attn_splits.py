@@ -1,0 +1,70 @@
+"""The number of blocks that share one sequence: what the choice promises to its callers (CPU) and, on the GPU, attention over
+contexts and batches on both sides of where it changes, against dense attention over the dequantized cache."""
+import ctypes as C
+
+import pytest
+import torch
+
+from tests.helpers import assert_attention_close, masked_two_refs
+
+
+def _args(B, Hq, Hkv, Tq, T, n, flags, dtype, kv_len=False, generic=0):
+    from hqmq_amd import _lib as L
+    a = L.AttnArgs()
+    a.B, a.H_q, a.H_kv, a.T_q, a.T_kv, a.t_cap, a.n_chunks, a.dtype, a.qmax, a.idx_bits, a.force_generic = B, Hq, Hkv, Tq, T, T, n, dtype, 15, 12, generic
+    a.K.flag_plane = 16 if flags else None
+    a.kv_len = 16 if kv_len else None
+    return a
+
+
+def test_splits_keep_to_rounds_of_blocks_and_to_earlier_workspaces():
+    from hqmq_amd import _lib as L
+    lib = L.lib()
+    for ragged in (0, 1):
+        for n, flags, dtype, generic in ((32, 0, L.DT_CODE[torch.float16], 0), (32, 1, L.DT_CODE[torch.bfloat16], 0), (16, 1, L.DT_CODE[torch.float16], 0),
+                                         (16, 0, L.DT_CODE[torch.bfloat16], 1), (20, 0, L.DT_CODE[torch.float32], 0)):
+            for B in (1, 2, 3, 5, 31, 32, 33, 64, 127, 128, 129, 130, 1000):
+                for T in (1, 63, 64, 65, 127, 128, 129, 300, 511, 513, 1025, 4096, 6145, 20001, 1 << 20):
+                    base = B * 8
+                    old = max(1, min(((512 if ragged else 256) + base - 1) // base, (T + 127) // 128, 512))
+                    assert 1 <= lib.hqmq_attn_pick_splits(B, 32, 8, 1, T, ragged) <= old
+                    a = _args(B, 32, 8, 1, T, n, flags, dtype, ragged, generic)
+                    s = lib.hqmq_attn_splits(C.addressof(a))
+                    assert 1 <= s <= max(1, (T + 127) // 128) and (s == 1 or base * s <= 1024), (B, T, s)
+                    a.T_kv = a.t_cap = (T + 63) // 64 * 64
+                    assert lib.hqmq_attn_splits(C.addressof(a)) == s                    # the key under which callers keep it
+    assert lib.hqmq_attn_pick_splits(1, 32, 8, 1, 0, 0) == 1 and lib.hqmq_attn_pick_splits(1, 4, 8, 1, 500, 0) == 1
+    for T, s in ((300, 1), (4096, 32), (32768, 32)):       # one block, whole rounds of 256
+        assert lib.hqmq_attn_pick_splits(1, 32, 8, 1, T, 0) == s
+    assert lib.hqmq_attn_pick_splits(12, 32, 8, 1, 4096, 0) == 2                        # 192 blocks, not 288
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("S,b_r,dn,d_h,med,B,contexts", [
+    (96, 4, "fp16", 128, False, 1, (1, 64, 300, 640, 704, 768, 1025)), (192, 4, "fp16", 128, False, 33, (257, 1100)),
+    (24, 3, "bf16", 128, True, 1, (255, 384, 385, 450)), (96, 4, "bf16", 64, True, 5, (300, 640, 1024, 1025)),
+    (96, 4, "fp16", 64, False, 12, (500, 1500, 2100)), (24, 3, "fp32", 128, False, 3, (129, 600))])
+def test_attention_on_both_sides_of_the_choice(S, b_r, dn, d_h, med, B, contexts):
+    import hqmq
+    dt = {"fp16": torch.float16, "bf16": torch.bfloat16, "fp32": torch.float32}[dn]
+    Hq, Hkv, T = 32, 8, max(contexts)
+    g = torch.Generator().manual_seed(S + d_h)
+    k, v = (torch.randn(B, Hkv, T, d_h, generator=g) for _ in range(2))
+    if med:
+        k[..., ::37, 3] = 30.0
+    q = hqmq.HQMQ(n_layers=1, n_heads=Hkv, secondary_size=S, radius_bits=b_r, device="cuda")
+    if med:
+        q = hqmq.with_outlier_extraction(q, C=3.0)
+    cache = q.new_cache(B, T, d_h, dt, 0)
+    q.append(cache, k.to(dt).cuda(), v.to(dt).cuda(), 0)
+    Q = torch.randn(B, Hq, 1, d_h, generator=g).to(dt).cuda()
+    for t in contexts:
+        lens = torch.randint(1, t + 1, (B,), generator=g).int()
+        lens[0] = t
+        for kw in ({}, {"kv_lens": lens.cuda()}):
+            vis = torch.arange(t).view(1, 1, 1, t) < lens.view(B, 1, 1, 1) if kw else None
+            refs = masked_two_refs(cache, Q, t, None if vis is None else vis.cuda())
+            for ns in (0, 1, 5):
+                O = hqmq.fused_attention_packed(Q, cache, T_kv=t, n_splits=ns, **kw)
+                assert_attention_close(O, *refs, base=1e-3 if dn == "fp32" else 2e-3, what=f"T={t} {list(kw)} n_splits={ns}")
