@@ -64,7 +64,7 @@ __device__ __forceinline__ void touch_kernargs() {
     asm volatile("" ::"s"(t));
 }
 
-constexpr int kFastWaves = 8;     // wavefronts per block; 12 (three per SIMD) for plain 16+0 caches with long ranges per block
+constexpr int kFastWaves = 8;     // wavefronts per block; 12 (three per SIMD) with long ranges per block, see launch_layout
 
 // codes, aux bits and raw 16-bit scales of 32 tokens (two 16-token tiles) for one lane
 template <int NW, int AB, bool FLAGS>
@@ -122,7 +122,7 @@ constexpr int kAuxTabOffset = 36864;        // s192_r6: 64 dwords with the high 
 // s24_r3 (13-bit codes, K <= 1024, qmax = 7): the tables are kept multiplied out, entry [rq][idx] = codeword * rq at byte
 // (rq << 10 | idx) * 8, so that the 13-bit code is the table index and a decode is one gather (no radius arithmetic).
 constexpr int kPsTabBytes = 8 * 1024 * 8;   // 64 KB per tensor
-constexpr bool is_prescaled(int CPL, int MB, int AB, int IB) { return CPL == 8 && MB == 12 && AB == 1 && IB == 10; }
+constexpr bool is_prescaled(int MB, int AB, int IB) { return MB == 12 && AB == 1 && IB == 10; }
 constexpr int vtab_offset(bool ps) { return ps ? kPsTabBytes : kVTabOffset; }
 constexpr int q_offset(bool ps) { return ps ? 2 * kPsTabBytes : kQOffset; }
 constexpr int sel_offset(bool ps) { return q_offset(ps) + 4096; }      // nine rows of eight fp16: row r < 8 = qmax times unit vector r, row 8 = 0
@@ -208,17 +208,17 @@ __device__ __forceinline__ void gather_chunks(const uint32_t (&w)[NW], uint32_t 
             const uint32_t t = ((w[i] >> 13) & 0x00070007u) | hi;
             r[i] = __builtin_bit_cast(half2v, t) - k1024;
         }
-    } else if constexpr (MB == 12 && AB == 1 && IB == 10 && CPL == 8) {
+    } else if constexpr (MB == 12 && AB == 1 && IB == 10) {
         static_assert(!F8, "the float8 table variants exist for 16-bit main fields");
-        // s24_r3, tables multiplied out (see kPsTabBytes): eight 12-bit fields (idx in the low 10 bits, the low two
-        // radius bits above) in three dwords and one aux byte with the eight high radius bits; field | aux bit << 12 is
-        // the table index.  No radius arithmetic: r stays unused.
-        const uint32_t w0 = w[0], w1 = w[1], w2 = w[2];
+        // s24_r3, tables multiplied out (see kPsTabBytes): eight (d_h 64: four) 12-bit fields (idx in the low 10 bits, the
+        // low two radius bits above) in three dwords (one and a half) and the high radius bits in the low bits of aux;
+        // field | aux bit << 12 is the table index.  No radius arithmetic: r stays unused.
+        const uint32_t w0 = w[0], w1 = w[1], w2 = w[NW - 1];
         constexpr uint32_t M = 0x7ff8u;
         const uint32_t ad[8] = {(w0 << 3) & M, (w0 >> 9) & M, __builtin_amdgcn_alignbit(w1, w0, 21) & M, (w1 >> 1) & M,
                                 (w1 >> 13) & M, __builtin_amdgcn_alignbit(w2, w1, 25) & M, (w2 >> 5) & M, (w2 >> 17) & M};
 #pragma unroll
-        for (int j = 0; j < 8; j++) g[j] = gather8<TAB_OFF>(((aux << (15 - j)) & 0x8000u) | ad[j]);
+        for (int j = 0; j < CPL; j++) g[j] = gather8<TAB_OFF>(((aux << (15 - j)) & 0x8000u) | ad[j]);
     } else {
         static_assert(!F8, "the float8 table variants exist for the layouts with compile-time index widths");
 #pragma unroll
@@ -269,8 +269,9 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     static_assert(NCG == 1 || !FLAGS, "outlier variants take one column group");
     constexpr int NB = CPL * MB / 8;
     constexpr int NW = (NB + 3) / 4;
-    constexpr int ABYTES = CPL * AB / 8;     // aux bytes per lane (CPL * AB is a multiple of 8 here)
-    static_assert(AB == 0 || (CPL * AB) % 8 == 0, "aux bits of one lane must be whole bytes");
+    constexpr int ABYTES = CPL * AB / 8;     // aux bytes per lane where its bits are whole bytes, see load_aux_word
+    static_assert((CPL * AB) % 8 == 0 || (CPL == 4 && (AB == 1 || AB == 3)), "aux bits of one lane");
+    static_assert(NB % 4 == 0 || NB == 6, "main bytes of one lane");
     static_assert(CPL % 2 == 0, "two chunks per 16x16x32 operand");
     constexpr int NT = WV * 64;
     constexpr int kKPre = CPL >= 8 ? 3 : 1;     // batches of outlier entries requested ahead (d_h 64 has half the chunks)
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const unsigned long long t_in_ = __builtin_amdgcn_s_memrealtime();
     unsigned long long t_loop_ = 0;
 #endif
-    constexpr bool PS = is_prescaled(CPL, MB, AB, IB);
+    constexpr bool PS = is_prescaled(MB, AB, IB);
     constexpr int VTAB = vtab_offset(PS), QOFF = q_offset(PS), SELOFF = sel_offset(PS);
     uint2 *ktab = lds_tab, *vtab = lds_tab + VTAB / 8;
     touch_kernargs();
@@ -314,7 +315,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     // codewords, all unconditional (clamped): straight-line code, exact wait counts.
     // (every pair of the largest table the LDS slots hold, 2560 pairs, in one round of requests: a second round would
     // be a loop of loads, and the wait at its head covers every request in flight, the first tile's included)
-    constexpr int FU = is_prescaled(CPL, MB, AB, IB) ? (512 + NT - 1) / NT : (kVTabOffset / 16 + NT - 1) / NT;
+    constexpr int FU = is_prescaled(MB, AB, IB) ? (512 + NT - 1) / NT : (kVTabOffset / 16 + NT - 1) / NT;
     const uint4v *ksrc = (const uint4v *)((const uint2 *)p.Kc.joint + hkv * (p.Kc.jsh / 4));
     const uint4v *vsrc = (const uint4v *)((const uint2 *)p.Vc.joint + hkv * (p.Vc.jsh / 4));
     const int Kk2 = p.Kc.K >> 1, Kv2 = p.Vc.K >> 1;        // tables of an even number of codewords (checked at launch)
@@ -395,7 +396,22 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const uint8_t *va_rows = AB ? p.Vc.aux_plane + plane_row0 * arb : nullptr;
     const int32_t *k_toff = FLAGS ? p.Kc.sb_tile_off + (size_t)bh * tiles_cap : nullptr;
     const int32_t *v_toff = FLAGS ? p.Vc.sb_tile_off + (size_t)bh * tiles_cap : nullptr;
-    const uint32_t main_off = (uint32_t)(col * mrb + grp * NB), aux_off = (uint32_t)(col * arb + grp * ABYTES);
+    // The lane's CPL * AB aux bits start at bit aux_sh of the word at aux_off.  At d_h 64 they are 4 or 12 bits of a row of 2 or
+    // 6 bytes: the whole row, or the dword (2-byte aligned) at its byte 0 or 2, is loaded and shifted where it is used.
+    constexpr bool kAuxRow2 = CPL == 4 && AB == 1, kAuxRow6 = CPL == 4 && AB == 3;
+    const uint32_t main_off = (uint32_t)(col * mrb + grp * NB), aux_off = (uint32_t)(col * arb + (kAuxRow2 ? 0 : kAuxRow6 ? (grp & 2) : grp * ABYTES));
+    const uint32_t aux_sh = kAuxRow2 ? 4u * (uint32_t)grp : kAuxRow6 ? 12u * (uint32_t)grp - 8u * (uint32_t)(grp & 2) : 0u;
+    auto load_aux_word = [&](const uint8_t *q) -> uint32_t {
+        if constexpr (kAuxRow2) return *reinterpret_cast<const uint16_t *>(q);
+        else if constexpr (kAuxRow6) return *reinterpret_cast<const uint32_a2 *>(q);
+        else return load_small<ABYTES>(q);
+    };
+    auto load_main = [&](const uint8_t *q, uint32_t (&w)[NW]) {
+        if constexpr (NB == 6) {        // 2-byte aligned; as loaded, like everything here: put together at once they would be waited for
+            w[0] = *reinterpret_cast<const uint32_a2 *>(q);
+            w[1] = *reinterpret_cast<const uint16_t *>(q + 4);
+        } else load_bytes<NB>(q, w);
+    };
     const uint32_t scale_off = (uint32_t)(4 * grp);
     const int k_count = FLAGS ? (int)min((int64_t)max(w_kcount, 0), p.Kc.sb_cap) : 0;
     const int v_count = FLAGS ? (int)min((int64_t)max(w_vcount, 0), p.Vc.sb_cap) : 0;
@@ -415,14 +431,14 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
             HalfTile<NW, AB, FLAGS> &h = s.h[hh];
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                load_bytes<NB>(kb + main_off + u * 16 * mrb, h.kw[u]);
-                if (AB) h.kaux[u] = load_small<ABYTES>(ka_rows + (size_t)th * arb + aux_off + u * 16 * arb);
+                load_main(kb + main_off + u * 16 * mrb, h.kw[u]);
+                if constexpr (AB > 0) h.kaux[u] = load_aux_word(ka_rows + (size_t)th * arb + aux_off + u * 16 * arb);
                 h.ks[u] = *reinterpret_cast<const uint2 *>(ks_plane + th + scale_off + 16 * u);
             }
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                load_bytes<NB>(vb + main_off + u * 16 * mrb, h.vw[u]);
-                if (AB) h.vaux[u] = load_small<ABYTES>(va_rows + (size_t)th * arb + aux_off + u * 16 * arb);
+                load_main(vb + main_off + u * 16 * mrb, h.vw[u]);
+                if constexpr (AB > 0) h.vaux[u] = load_aux_word(va_rows + (size_t)th * arb + aux_off + u * 16 * arb);
                 h.vs[u] = *reinterpret_cast<const uint2 *>(vs_plane + th + scale_off + 16 * u);
             }
         }
@@ -769,13 +785,13 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         half2v rk[2][CPL / 2];
         if constexpr (kBatchGathers) {
 #pragma unroll
-            for (int u = 0; u < 2; u++) gather_chunks<CPL, MB, AB, IB, NW, 0, F8>(h.kw[u], AB ? h.kaux[u] : 0u, idx_bits, gk[u], rk[u]);
+            for (int u = 0; u < 2; u++) gather_chunks<CPL, MB, AB, IB, NW, 0, F8>(h.kw[u], AB ? h.kaux[u] >> aux_sh : 0u, idx_bits, gk[u], rk[u]);
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             half4 a[CPL];
-            if constexpr (!kBatchGathers) gather_chunks<CPL, MB, AB, IB, NW, 0, F8>(h.kw[u], AB ? h.kaux[u] : 0u, idx_bits, gk[u], rk[u]);
+            if constexpr (!kBatchGathers) gather_chunks<CPL, MB, AB, IB, NW, 0, F8>(h.kw[u], AB ? h.kaux[u] >> aux_sh : 0u, idx_bits, gk[u], rk[u]);
             scale_chunks<CPL, PS>(gk[u], rk[u], a);
 #pragma unroll
             for (int cgi = 0; cgi < NCG; cgi++) {
@@ -811,7 +827,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         half2v rv[2][CPL / 2];
         if constexpr (kBatchGathers) {
 #pragma unroll
-            for (int u = 0; u < 2; u++) gather_chunks<CPL, MB, AB, IB, NW, VTAB, F8>(h.vw[u], AB ? h.vaux[u] : 0u, idx_bits, gv[u], rv[u]);
+            for (int u = 0; u < 2; u++) gather_chunks<CPL, MB, AB, IB, NW, VTAB, F8>(h.vw[u], AB ? h.vaux[u] >> aux_sh : 0u, idx_bits, gv[u], rv[u]);
             __builtin_amdgcn_sched_barrier(0);
         }
         // ---- mask (boundary half-steps only), online softmax, per column group ----
@@ -868,7 +884,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         half4 av[2][CPL];
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            if constexpr (!kBatchGathers) gather_chunks<CPL, MB, AB, IB, NW, VTAB, F8>(h.vw[u], AB ? h.vaux[u] : 0u, idx_bits, gv[u], rv[u]);
+            if constexpr (!kBatchGathers) gather_chunks<CPL, MB, AB, IB, NW, VTAB, F8>(h.vw[u], AB ? h.vaux[u] >> aux_sh : 0u, idx_bits, gv[u], rv[u]);
             scale_chunks<CPL, PS>(gv[u], rv[u], av[u]);
         }
 #pragma unroll
@@ -1427,7 +1443,7 @@ template <int CPL, int MB, int AB, int IB, int DT, int WV = kFastWaves, int NCG 
 static int launch_one(const AttnParams &p, bool flags, dim3 grid, hipStream_t st, const LaunchTiming &tm) {
     if (NCG > 1) grid.y = (grid.y + NCG - 1) / NCG;
     // LDS: K table at 0, V table at kVTabOffset; reused afterwards for the cross-wave merge [wave][16][d_h + 4] floats
-    constexpr bool PS = is_prescaled(CPL, MB, AB, IB);
+    constexpr bool PS = is_prescaled(MB, AB, IB);
     size_t shmem = flags ? (size_t)sel_offset(PS) + 192 : PS ? (size_t)2 * kPsTabBytes : (size_t)kVTabOffset + (size_t)p.Vc.K * 8;
     shmem += 64;        // the wavefronts' progress slots
     const size_t merge = (size_t)WV * 16 * (16 * CPL + 4) * sizeof(float);     // WV >= the wavefronts actually launched
@@ -1454,9 +1470,13 @@ static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hip
     if ((p.Kc.K & 1) || (p.Vc.K & 1) || (p.Kc.jsh & 7) || (p.Vc.jsh & 7) || (((uintptr_t)p.Kc.joint | (uintptr_t)p.Vc.joint) & 15))
         return HQMQ_OK;
     *handled = true;
-    // long ranges per block (large batches): twelve wavefronts per block, three per SIMD, stream 3-12 % faster; the
-    // variants that need more than 168 registers and short launches stay at eight
-    const bool wide = (CPL == 8 ? !flags : flags) && p.Tkv / p.n_splits >= 6144;
+    // Long ranges per block run with twelve wavefronts, three per SIMD, which hide more of each other's waits than the extra partials
+    // of the block's merge cost; the variants that need more than 168 registers stay at eight.  Lines where both measure alike, with
+    // 224 blocks: d_h 128 plain 3000 tokens (4000 / 5500 tokens of s96_r4 30.1 -> 29.1 / 38.3 -> 36.3 us), d_h 64 over outlier caches
+    // 1200 (3000 / 5500 tokens 26.1 -> 23.3 / 42.3 -> 36.3 us), d_h 64 plain 4000 (8000 tokens 34.4 -> 32.3 us), there only while no
+    // compute unit holds two blocks of eight (480 blocks of 4000 tokens 33.3 against 38.2 us).
+    const int range = p.Tkv / p.n_splits;
+    const bool wide = CPL == 8 ? !flags && range >= 4096 : flags ? range >= 1536 : range >= 4096 && (int64_t)grid.x * grid.y * grid.z <= 256;
     // chunked prefill (more than 16 columns per KV head) of plain caches: two column groups per wavefront
     // (only while a block per CU is left: fewer, larger blocks lose more than the shared decode wins)
     const bool two = !flags && p.n_cg > 1 && (int64_t)p.n_splits * ((p.n_cg + 1) / 2) * p.B * p.Hkv >= 256;
@@ -1479,28 +1499,33 @@ static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hip
         if (two) return launch_one<CPL, 16, 0, 0, DT, kFastWaves, 2>(p, flags, grid, st, tm);
         return wide ? launch_one<CPL, 16, 0, 0, DT, 12>(p, flags, grid, st, tm) : launch_one<CPL, 16, 0, 0, DT>(p, flags, grid, st, tm);
     }
-    if (mb == 12 && p.aux_bits == 1 && CPL == 8 && p.idx_bits == 10 && p.Kc.K <= 1024) {
-        if (two) return launch_one<8, 12, 1, 10, DT, kFastWaves, 2>(p, flags, grid, st, tm);
-        return wide ? launch_one<8, 12, 1, 10, DT, 12>(p, flags, grid, st, tm) : launch_one<8, 12, 1, 10, DT>(p, flags, grid, st, tm);
+    // Heads of 64 take these layouts here as well.  Before, the layout-generic kernel had them: 8 sequences x 3000 tokens, 64 / 8 heads,
+    // 28.8 (s24_r3 fp16) to 47.3 us (s192_r6 bf16), with verbatim chunks 52 to 83, 40 queries each then 940 to 1350; now 14.3 to
+    // 14.8, 16.7 to 17.3 and 133 to 142 us.  Tables multiplied out pay there too (4 x 32000 tokens 32.7 without them, 28.8 with).
+    if (mb == 12 && p.aux_bits == 1 && p.idx_bits == 10 && p.Kc.K <= 1024 && p.Vc.K <= 1024) {
+        if (two) return launch_one<CPL, 12, 1, 10, DT, kFastWaves, 2>(p, flags, grid, st, tm);
+        return wide ? launch_one<CPL, 12, 1, 10, DT, 12>(p, flags, grid, st, tm) : launch_one<CPL, 12, 1, 10, DT>(p, flags, grid, st, tm);
     }
-    if (mb == 12 && p.aux_bits == 1 && CPL == 8) return launch_one<8, 12, 1, 0, DT>(p, flags, grid, st, tm);
-    // (the 16+3 decode needs 182 registers: at three wavefronts per SIMD it spills and runs 40 % slower)
-    if (mb == 16 && p.aux_bits == 3 && CPL == 8 && p.idx_bits == 13 && p.Kc.K <= 4608)
-        return two ? launch_one<8, 16, 3, 13, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<8, 16, 3, 13, DT>(p, flags, grid, st, tm);
-    if (mb == 16 && p.aux_bits == 3 && CPL == 8) return launch_one<8, 16, 3, 0, DT>(p, flags, grid, st, tm);
+    if (mb == 12 && p.aux_bits == 1) return launch_one<CPL, 12, 1, 0, DT>(p, flags, grid, st, tm);
+    // (the 16+3 decode needs 182 registers at d_h 128: at three wavefronts per SIMD it spills and runs 40 % slower)
+    if constexpr (CPL == 4) {
+        if (wide && mb == 16 && p.aux_bits == 3 && p.idx_bits == 13 && p.Kc.K <= 4608) return launch_one<CPL, 16, 3, 13, DT, 12>(p, flags, grid, st, tm);
+        if (wide && mb == 16 && p.aux_bits == 1) return launch_one<CPL, 16, 1, 0, DT, 12>(p, flags, grid, st, tm);
+    }
+    if (mb == 16 && p.aux_bits == 3 && p.idx_bits == 13 && p.Kc.K <= 4608)
+        return two ? launch_one<CPL, 16, 3, 13, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<CPL, 16, 3, 13, DT>(p, flags, grid, st, tm);
+    if (mb == 16 && p.aux_bits == 3) return launch_one<CPL, 16, 3, 0, DT>(p, flags, grid, st, tm);
     // 16 + 1 bits (s192 with four radius bits, the shape of the reference's published prefill figure): generic field decode
-    if (mb == 16 && p.aux_bits == 1 && CPL == 8)
-        return two ? launch_one<8, 16, 1, 0, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<8, 16, 1, 0, DT>(p, flags, grid, st, tm);
-    // the remaining widths the layout rule produces for d_h 128 (16 + 2: s96_r6, s192_r5; 12 + 2: s24_r4; 12 + 3: s96_r3,
-    // s24_r5), generic field decode: five times faster than the layout-generic kernel at batch 8
-    if constexpr (CPL == 8) {
-        if (mb == 16 && p.aux_bits == 2)
-            return two ? launch_one<8, 16, 2, 0, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<8, 16, 2, 0, DT>(p, flags, grid, st, tm);
-        if (mb == 12 && p.aux_bits == 2)
-            return two ? launch_one<8, 12, 2, 0, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<8, 12, 2, 0, DT>(p, flags, grid, st, tm);
-        if (mb == 12 && p.aux_bits == 3)
-            return two ? launch_one<8, 12, 3, 0, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<8, 12, 3, 0, DT>(p, flags, grid, st, tm);
-    }
+    if (mb == 16 && p.aux_bits == 1)
+        return two ? launch_one<CPL, 16, 1, 0, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<CPL, 16, 1, 0, DT>(p, flags, grid, st, tm);
+    // the remaining widths the layout rule produces (16 + 2: s96_r6, s192_r5; 12 + 2: s24_r4; 12 + 3: s96_r3, s24_r5), generic
+    // field decode: five times faster than the layout-generic kernel at batch 8
+    if (mb == 16 && p.aux_bits == 2)
+        return two ? launch_one<CPL, 16, 2, 0, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<CPL, 16, 2, 0, DT>(p, flags, grid, st, tm);
+    if (mb == 12 && p.aux_bits == 2)
+        return two ? launch_one<CPL, 12, 2, 0, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<CPL, 12, 2, 0, DT>(p, flags, grid, st, tm);
+    if (mb == 12 && p.aux_bits == 3)
+        return two ? launch_one<CPL, 12, 3, 0, DT, kFastWaves, 2>(p, flags, grid, st, tm) : launch_one<CPL, 12, 3, 0, DT>(p, flags, grid, st, tm);
     *handled = false;
     return HQMQ_OK;
 }
