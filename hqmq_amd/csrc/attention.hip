@@ -500,14 +500,17 @@ extern "C" int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, i
 // compute unit, so that blocks come in rounds of 256, and one block more than a round costs a whole one: the estimate is
 // rounds x (start of a block + its tokens) + merge, in tokens of d_h 128 (4.6 us per 1000 over plain fp16 caches).  A start, tables
 // and query, is worth 500 of them; `merge`, the second launch and the blocks' way through memory, 500 over plain caches, 350 where
-// the radii have a plane of their own, 250 over outlier caches and 100 in the generic kernels, whose tokens cost more; a split more 5.
+// the radii have a plane of their own, 250 over outlier caches and 100 in the generic kernels, whose tokens cost more; it doubles with
+// 5000 partial rows, and a split more is worth 2.
 // Sequences of different lengths, started longest first, even out: a round counts by its share, 0.8 of the blocks (mean over the
 // longest) and 0.3 for the last ones.  Measured against the best of 8 to 14 counts at 120 shapes with equal lengths, 101 with lengths
-// of their own (6 cache layouts, 4 to 400 heads, 600 to 20000 tokens) and 230 of 1 to 7 queries replayed in graphs, the choice takes
-// 0.5, 1.9 and 0.5 % longer; 256 blocks rounded up (512 over such lengths), the rule before, took 25, 32 and 23 %.  us before -> now:
+// of their own (6 cache layouts, 4 to 400 heads, 600 to 20000 tokens), 230 of 1 to 7 queries replayed in graphs and 65 prefill chunks,
+// the choice takes 0.6, 2.7, 0.9 and 2.1 % longer; 256 blocks rounded up (512 over such lengths), the rule before, took 25, 32 and 23 %
+// at the first three.  us before -> now:
 // s96_r4 fp16, 32 / 8 heads of 128, 1 x 300 tokens 10.7 -> 7.0 (one block, no merge), 3 x 20000 30.2 -> 20.0, 10 x 6000 28.4 -> 20.6,
 // 20 x 600 14.9 -> 8.5; s24_r3 bf16 with verbatim chunks, 10 x 6000 47.4 -> 34.2.
-static int decode_splits(int64_t base, int T_kv, bool ragged, double unit, double merge) {
+// `pairs` (or 0): the blocks where two column groups share one, which the specialised kernels do beyond a round, at 1.28 times the time.
+static int decode_splits(int64_t base, int64_t pairs, int64_t rows, int T_kv, bool ragged, double unit, double merge) {
     if (base < 1) return 1;
     int64_t top = ((int64_t)T_kv + 2 * kSuper - 1) / (2 * kSuper);       // blocks of at least 128 tokens (4k tokens: 32 splits, 8.7 against 8.95 us)
     if (top > 512) top = 512;
@@ -516,10 +519,12 @@ static int decode_splits(int64_t base, int T_kv, bool ragged, double unit, doubl
     double least = 0.0;
     int best = 1;
     for (int64_t s = 1; s <= top || s == 1; s++) {
-        const int64_t blocks = base * s;
+        const bool two = pairs > 0 && base * s > 256;
+        const int64_t blocks = two ? pairs * s : base * s;
         double rounds = ragged ? 0.8 / 256 * (double)blocks + 0.3 : (double)((blocks + 255) / 256);
         if (rounds < 1.0) rounds = 1.0;
-        const double t = rounds * (500.0 + unit * (double)((tiles + s - 1) / s * kSuper)) + (s > 1 ? merge + 5.0 * (double)s : 0.0);
+        const double t = rounds * (500.0 + (two ? 1.28 * unit : unit) * (double)((tiles + s - 1) / s * kSuper)) +
+                         (s > 1 ? merge * (1.0 + 2e-4 * (double)rows * (double)s) + 2.0 * (double)s : 0.0);
         if (s == 1 || t < least) { least = t; best = (int)s; }
     }
     return best;
@@ -531,7 +536,7 @@ extern "C" int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv
     if (B < 1 || H_q < 1 || H_kv < 1 || T_q < 1 || T_kv < 1) return 1;
     const int G = H_q / H_kv;
     const int64_t base = (int64_t)B * H_kv * (((int64_t)T_q * G + 15) / 16), target = ragged ? 512 : 256;
-    const int s = decode_splits(base, T_kv, ragged != 0, 1.0, 500.0);
+    const int s = decode_splits(base, 0, (int64_t)B * H_q * T_q, T_kv, ragged != 0, 1.0, 500.0);
     return s > 1 && s > (target + base - 1) / base ? (int)((target + base - 1) / base) : s;
 }
 
@@ -540,7 +545,9 @@ extern "C" int hqmq_attn_splits(const hqmq_attn_args *a) {
     const int splits = attn_prefill_splits(a, 0);
     if (splits > 0) return splits;
     const bool generic = a->dtype == HQMQ_F32 || a->wide_range || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
-    return decode_splits((int64_t)a->B * a->H_kv * (((int64_t)a->T_q * (a->H_q / a->H_kv) + 15) / 16), a->T_kv, a->kv_len != nullptr,
+    const int64_t nz = (int64_t)a->B * a->H_kv, groups = ((int64_t)a->T_q * (a->H_q / a->H_kv) + 15) / 16;
+    return decode_splits(nz * groups, generic || a->K.flag_plane || groups < 2 ? 0 : nz * ((groups + 1) / 2),
+                         (int64_t)a->B * a->H_q * a->T_q, a->T_kv, a->kv_len != nullptr,
                          a->n_chunks / 32.0, generic ? 100.0 : a->K.flag_plane ? 250.0 : a->aux_bits ? 350.0 : 500.0);
 }
 

@@ -596,7 +596,7 @@ static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int ca
     const double mean = causal ? std::min(1.0, std::max(0.5, ((double)off + 0.5 * Tq) / last)) : 1.0;            // all, relative to it
     const int tiles = (int)((last * d_h + 8191) / 8192);
     PfPlan best{false, 1, 1e30};
-    static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+    static const int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 20, 24, 32};
     for (int i = 0; i < (fixed_splits > 0 ? 1 : (int)(sizeof(kSplits) / sizeof(int))); i++) {
         const int s = fixed_splits > 0 ? fixed_splits : kSplits[i];
         if (i > 0 && s > tiles / 2) break;
@@ -630,11 +630,11 @@ static bool attn_prefill_takes(const hqmq_attn_args *a) {
     if ((((uintptr_t)a->O) | (uintptr_t)(a->o_sb * 2) | (uintptr_t)(a->o_sh * 2) | (uintptr_t)(a->o_st * 2)) & 7) return false;
     return true;
 }
-// The same for the kernels of attention_fast.hip: blocks of 16 columns (0.47 us a tile) or, where that leaves a block per
-// compute unit, of 32 (0.6 us), over outlier caches always of 16 (0.7 us), which start and finish in 6 us.
+// The same for the kernels of attention_fast.hip: blocks of 16 columns (0.47 us a tile) or, where those are more than the
+// compute units, of 32 (0.6 us), over outlier caches always of 16 (0.7 us), which start and finish in 6 us.
 static double fast_us(int64_t cols, int64_t nz, int Tkv, int d_h, int splits, bool flags) {
     const int64_t cg = (cols + 15) / 16, pairs = (cg + 1) / 2 * nz * splits;
-    const bool two = !flags && cg > 1 && pairs >= 256;
+    const bool two = !flags && cg > 1 && cg * nz * splits > 256;
     const double tiles = ((double)Tkv * d_h + 8191) / 8192;
     return 3.0 + (double)(((two ? pairs : cg * nz * splits) + 255) / 256) * (6.0 + tiles / splits * (two ? 0.6 : flags ? 0.7 : 0.47)) +
            (splits > 1 ? 3.0 + (double)(cols * nz) * splits * (d_h + 4) * 8 / 2e6 : 0.0);

@@ -68,3 +68,26 @@ def test_attention_on_both_sides_of_the_choice(S, b_r, dn, d_h, med, B, contexts
             for ns in (0, 1, 5):
                 O = hqmq.fused_attention_packed(Q, cache, T_kv=t, n_splits=ns, **kw)
                 assert_attention_close(O, *refs, base=1e-3 if dn == "fp32" else 2e-3, what=f"T={t} {list(kw)} n_splits={ns}")
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("S,b_r,dn,d_h", [(96, 4, "fp16", 128), (96, 4, "bf16", 64), (192, 4, "bf16", 128), (24, 3, "fp16", 128)])
+def test_column_groups_between_one_and_two_rounds(S, b_r, dn, d_h):
+    """More than 256 blocks of one column group and fewer than 256 of two: 32 (sequence, head) pairs x 9 groups, the last block's second
+    group past the end; 255 and 256 tokens where the choice looks at the length too."""
+    import hqmq
+    dt = {"fp16": torch.float16, "bf16": torch.bfloat16}[dn]
+    B, Hq, Hkv, Tq = 4, 32, 8, 33
+    g = torch.Generator().manual_seed(S + d_h)
+    k, v = (torch.randn(B, Hkv, 300, d_h, generator=g).to(dt).cuda() for _ in range(2))
+    q = hqmq.HQMQ(n_layers=1, n_heads=Hkv, secondary_size=S, radius_bits=b_r, device="cuda")
+    cache = q.new_cache(B, 300, d_h, dt, 0)
+    q.append(cache, k, v, 0)
+    Q = torch.randn(B, Hq, Tq, d_h, generator=g).to(dt).cuda()
+    for t in (40, 255, 256, 300):
+        vis = (torch.arange(t).view(1, 1, 1, t) <= torch.arange(t - Tq, t).view(1, 1, Tq, 1)).cuda()
+        refs = masked_two_refs(cache, Q, t, vis)
+        for ns in (0, 1):
+            O = hqmq.fused_attention_packed(Q, cache, T_kv=t, causal=True, causal_offset=t - Tq, n_splits=ns)
+            assert_attention_close(O, *refs, base=2e-3, what=f"T={t} n_splits={ns}")
