@@ -514,7 +514,10 @@ static int decode_splits(int64_t base, int64_t pairs, int64_t rows, int T_kv, bo
     if (base < 1) return 1;
     int64_t top = ((int64_t)T_kv + 2 * kSuper - 1) / (2 * kSuper);       // blocks of at least 128 tokens (4k tokens: 32 splits, 8.7 against 8.95 us)
     if (top > 512) top = 512;
-    if (top > 1024 / base) top = 1024 / base;                              // past four rounds the last one weighs little: 832 blocks of 9000 tokens 104 us, halved 128
+    // past four rounds the last one weighs little (832 blocks of 9000 tokens 104 us, halved 128), and lengths of their own even out from
+    // two and a half on (512 of up to 16384 tokens 242 us, halved 248)
+    const int64_t most = (ragged ? 640 : 1024) / base;
+    if (top > most) top = most;
     const int64_t tiles = ((int64_t)T_kv + kSuper - 1) / kSuper;
     double least = 0.0;
     int best = 1;

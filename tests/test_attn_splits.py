@@ -30,7 +30,7 @@ def test_splits_keep_to_rounds_of_blocks_and_to_earlier_workspaces():
                     assert 1 <= lib.hqmq_attn_pick_splits(B, 32, 8, 1, T, ragged) <= old
                     a = _args(B, 32, 8, 1, T, n, flags, dtype, ragged, generic)
                     s = lib.hqmq_attn_splits(C.addressof(a))
-                    assert 1 <= s <= max(1, (T + 127) // 128) and (s == 1 or base * s <= 1024), (B, T, s)
+                    assert 1 <= s <= max(1, (T + 127) // 128) and (s == 1 or base * s <= (640 if ragged else 1024)), (B, T, s)
                     a.T_kv = a.t_cap = (T + 63) // 64 * 64
                     assert lib.hqmq_attn_splits(C.addressof(a)) == s                    # the key under which callers keep it
     assert lib.hqmq_attn_pick_splits(1, 32, 8, 1, 0, 0) == 1 and lib.hqmq_attn_pick_splits(1, 4, 8, 1, 500, 0) == 1
