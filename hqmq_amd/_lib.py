@@ -131,6 +131,29 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The compiled host side of the hot calls (csrc_host/native.cpp); raises if it has not been built."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise HqmqError(f"hqmq_amd/_native.so is missing or does not load: build it with `python -m hqmq_amd.build` ({e})") from e
+        _native = module
+    return _native
+
+
+def tensors(result, what: str):
+    """What a function of native() returned: its tensors; raises if it is the library's status."""
+    if type(result) is int:
+        check(result, what)
+    return result
+
+
 _bench_lib = None
 
 

@@ -1,6 +1,7 @@
 """Builds hqmq_amd/libhqmq_amd.so from hqmq_amd/csrc/*.hip with hipcc for gfx950, and beside it
 hqmq_amd/libhqmq_bench.so from hqmq_amd/csrc_bench/*.hip: the read-only measurement kernels that bench.py and
-hqmq_amd/bench_ceiling.py time (nothing in the product path loads that one).
+hqmq_amd/bench_ceiling.py time (nothing in the product path loads that one), and hqmq_amd/_native.so from
+hqmq_amd/csrc_host/native.cpp with g++: the host side of the hot calls.
 
     python -m hqmq_amd.build            # compile (always) and link
     python -m hqmq_amd.build --stamps   # also hqmq_amd/libhqmq_amd_stamps.so: the same library with attention_fast.hip compiled
@@ -29,6 +30,24 @@ BENCH_OUT = HERE / "libhqmq_bench.so"
 COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 EXACT = {"joint.hip", "quantize.hip", "quantize_grid.hip", "med3x.hip", "dequant.hip"}
+
+
+def build_native() -> Path:
+    """hqmq_amd/_native.so: plain C++ against torch's headers, linked to libhqmq_amd.so beside it."""
+    import sysconfig
+
+    import torch
+    t = Path(torch.__file__).resolve().parent
+    out = HERE / "_native.so"
+    cmd = ["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{t / 'include'}", f"-I{t / 'include/torch/csrc/api/include'}", f"-I{sysconfig.get_paths()['include']}", f"-I{Path(hipcc()).resolve().parent.parent / 'include'}",
+           str(HERE / "csrc_host" / "native.cpp"), "-o", str(out), f"-L{t / 'lib'}", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip",
+           f"-L{HERE}", "-l:libhqmq_amd.so", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode:
+        sys.stderr.write(" ".join(cmd) + "\n" + r.stdout + r.stderr)
+        raise RuntimeError("g++ failed on native.cpp")
+    return out
 
 
 def hipcc() -> str:
@@ -69,6 +88,7 @@ def build(verbose: bool = False, stamps: bool = False) -> Path:
     if r.returncode:
         sys.stderr.write(r.stdout + r.stderr)
         raise RuntimeError("link failed")
+    build_native()
     if bench_objs:
         cmd = [cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(BENCH_OUT), *map(str, bench_objs)]
         r = subprocess.run(cmd, capture_output=True, text=True)

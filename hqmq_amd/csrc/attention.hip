@@ -518,7 +518,7 @@ static int decode_splits(int64_t base, int64_t pairs, int64_t rows, int T_kv, bo
     // two and a half on (512 of up to 16384 tokens 242 us, halved 248)
     const int64_t most = (ragged ? 640 : 1024) / base;
     if (top > most) top = most;
-    const int64_t tiles = ((int64_t)T_kv + kSuper - 1) / kSuper;
+    const uint32_t tiles = (uint32_t)(((int64_t)T_kv + kSuper - 1) / kSuper);
     double least = 0.0;
     int best = 1;
     for (int64_t s = 1; s <= top || s == 1; s++) {
@@ -526,7 +526,7 @@ static int decode_splits(int64_t base, int64_t pairs, int64_t rows, int T_kv, bo
         const int64_t blocks = two ? pairs * s : base * s;
         double rounds = ragged ? 0.8 / 256 * (double)blocks + 0.3 : (double)((blocks + 255) / 256);
         if (rounds < 1.0) rounds = 1.0;
-        const double t = rounds * (500.0 + (two ? 1.28 * unit : unit) * (double)((tiles + s - 1) / s * kSuper)) +
+        const double t = rounds * (500.0 + (two ? 1.28 * unit : unit) * (double)((tiles + (uint32_t)s - 1) / (uint32_t)s * kSuper)) +
                          (s > 1 ? merge * (1.0 + 2e-4 * (double)rows * (double)s) + 2.0 * (double)s : 0.0);
         if (s == 1 || t < least) { least = t; best = (int)s; }
     }

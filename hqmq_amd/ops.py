@@ -57,6 +57,7 @@ def _book(joint: torch.Tensor, slack: Optional[torch.Tensor], radius_bits: int, 
     grid = L.addr(grid)
     if slack is not None:
         slack.hqmq_book = L.Kept((joint, joint.data_ptr(), (radius_bits, n), a, grid))
+    a.address = C.addressof(a)
     return a, grid
 
 
@@ -84,14 +85,21 @@ def quantize(x: torch.Tensor, joint: torch.Tensor, slack: Optional[torch.Tensor]
     [t_off, t_off + T) (shifted by pos[b] per sequence) receive the packed codes.
     """
     L.require_gpu(x, "x")
-    x = _strided_x(x)
-    B, H, T, d_h = x.shape
+    d_h = x.shape[-1]
     if d_h % 4 != 0:
         raise ValueError(f"d_head={d_h} not divisible by 4")
     n = d_h // 4
+    tmpl, grid = _book(joint, slack, radius_bits, n)
+    if want_codes and not want_dense and cache is None and stats is None and algo == 0:
+        idx, rq, r_max, mask = L.tensors(L.native().codes(x, joint, tmpl.address, grid, thr, want_mask), "hqmq_quantize_grid")
+        out = {"idx": idx, "rq": rq, "r_max": r_max}
+        if mask is not None:
+            out["mask"] = mask
+        return out
+    x = _strided_x(x)
+    B, H, T, _ = x.shape
     _check_joint(x, joint)
     dev = x.device
-    tmpl, grid = _book(joint, slack, radius_bits, n)
     a = L.QuantizeArgs.from_buffer_copy(tmpl)
     a.x = x.data_ptr()
     a.x_stride_b, a.x_stride_h, a.x_stride_t, _ = x.stride()
@@ -165,17 +173,11 @@ def med3x_threshold(x: torch.Tensor, mult: float = 3.0, want_count: bool = True,
     """Per-head (median fp32, threshold in x.dtype, #chunks above threshold int32) over the whole call.
     strict_quantile_limit: raise as the reference does when a head has more than 2^24 chunks in this call."""
     L.require_gpu(x, "x")
-    x = _strided_x(x)
-    B, H, T, d_h = x.shape
-    n = d_h // 4
-    check_quantile_limit(B * T * n, strict_quantile_limit)
-    dev = x.device
-    ws = _med_workspace(x, "med3x")
-    med = torch.empty(H, dtype=torch.float32, device=dev)
-    thr = torch.empty(H, dtype=x.dtype, device=dev)
-    cnt = torch.empty(H, dtype=torch.int32, device=dev) if want_count else None     # written for every head
-    _median(x, mult, ws, med.data_ptr(), thr.data_ptr(), L.addr(cnt))
-    return med, thr, cnt
+    if x.dim() != 4:
+        raise ValueError(f"expected (B, H, T, d_head), got {tuple(x.shape)}")
+    if strict_quantile_limit:
+        check_quantile_limit(x.shape[0] * x.shape[2] * (x.shape[3] // 4), True)
+    return L.tensors(L.native().med3x(x, mult, _med_workspace(x, "med3x"), want_count), "hqmq_med3x_threshold")
 
 
 def _med_workspace(x: torch.Tensor, tag: str) -> torch.Tensor:
@@ -190,38 +192,16 @@ def _med_workspace(x: torch.Tensor, tag: str) -> torch.Tensor:
 _MED_BYTES = {}
 
 
-def _median(x: torch.Tensor, mult: float, ws: torch.Tensor, med: int, thr: int, cnt: int) -> None:
-    B, H, T, d_h = x.shape
-    sb, sh, st, _ = x.stride()
-    L.call(L.lib().hqmq_med3x_threshold, "hqmq_med3x_threshold", x.device.index, x.data_ptr(), sb, sh, st, _dt(x), B, H, T, d_h // 4, mult,
-           ws.data_ptr(), ws.numel(), med, thr, cnt)
-
-
 def fake_quant(x: torch.Tensor, joint: torch.Tensor, slack: torch.Tensor, radius_bits: int, median_mult: Optional[float] = None):
     """The fake-quant tensor of x (B, H, T, d_h), with Med-C extraction when median_mult is given: what med3x_threshold
     and quantize(want_dense=True) give, without tensors for the statistics in between.  Returns (out, flagged chunks
     per head or None)."""
     L.require_gpu(x, "x")
-    x = _strided_x(x)
-    B, H, T, d_h = x.shape
-    _check_joint(x, joint)
-    tmpl, grid = _book(joint, slack, radius_bits, d_h // 4)
-    a = L.QuantizeArgs.from_buffer_copy(tmpl)
-    a.x = x.data_ptr()
-    a.x_stride_b, a.x_stride_h, a.x_stride_t, _ = x.stride()
-    a.B, a.T = B, T
-    out = x.new_empty((B, H, T, d_h))
-    a.dense_out = out.data_ptr()
-    cnt = None
-    if median_mult is not None:
-        ws = _med_workspace(x, "med3x")
-        cnt = torch.empty(H, dtype=torch.int32, device=x.device)
-        spare = ws.data_ptr() + (ws.numel() - 12 * H & -16)
-        a.thr = spare + 4 * H
-        _median(x, median_mult, ws, spare, spare + 4 * H, cnt.data_ptr())
-    if T > 0:
-        L.call(L.lib().hqmq_quantize_grid, "hqmq_quantize_grid", x.device.index, C.addressof(a), grid)
-    return out, cnt
+    if x.dim() != 4:
+        raise ValueError(f"expected (B, H, T, d_head), got {tuple(x.shape)}")
+    tmpl, grid = _book(joint, slack, radius_bits, x.shape[3] // 4)
+    ws = None if median_mult is None else _med_workspace(x, "med3x")
+    return L.tensors(L.native().fake(x, joint, tmpl.address, grid, median_mult, ws), "hqmq_quantize_grid")
 
 
 def outlier_mask(x: torch.Tensor, thr: torch.Tensor) -> torch.Tensor:
@@ -283,21 +263,17 @@ def append_kv(k: torch.Tensor, v: torch.Tensor, k_cache, v_cache, k_joint, k_sla
     L.require_gpu(v, "v")
     if k.shape[2] == 0 and v.shape[2] == 0:        # an empty tensor has no address to pass
         return None, None
-    dev = k.device
-    if pos is not None:
-        pos = pos.to(device=dev, dtype=torch.int32).contiguous()
-    ak, grid_k, k, cnt_k, ws_k = _append_args(k, k_cache, k_joint, k_slack, radius_bits, t_off, pos, median_mult, "med3x_k")
-    av, grid_v, v, cnt_v, ws_v = _append_args(v, v_cache, v_joint, v_slack, radius_bits, t_off, pos, median_mult, "med3x_v")
-    L.call(L.lib().hqmq_append_kv_grid, "hqmq_append_kv_grid", dev.index, C.addressof(ak), C.addressof(av), grid_k, grid_v)
-    return cnt_k, cnt_v
+    ak, grid_k, ws_k = _append_block(k, k_cache, k_joint, k_slack, radius_bits, median_mult, "med3x_k")
+    av, grid_v, ws_v = _append_block(v, v_cache, v_joint, v_slack, radius_bits, median_mult, "med3x_v")
+    return L.tensors(L.native().append(k, v, ak.address, av.address, grid_k, grid_v, t_off, pos, median_mult, ws_k, ws_v), "hqmq_append_kv_grid")
 
 
-def _append_args(x, cache, joint, slack, radius_bits, t_off, pos, median_mult, tag):
-    """The arguments of one tensor's append, and the tensors whose addresses they hold (the caller keeps them until the launch).
-    What the cache and its codebook fix is filled in once and copied; the copy is this call's own (several threads may append to
-    one cache on streams of their own)."""
-    x = _strided_x(x)
-    B, H, T, d_h = x.shape
+def _append_block(x, cache, joint, slack, radius_bits, median_mult, tag):
+    """What a cache and its codebook fix of one tensor's append, filled in once (the library's caller copies it: several threads may
+    append to one cache on streams of their own), the cell lists, the workspace of the call's median."""
+    if x.dim() != 4:
+        raise ValueError(f"expected (B, H, T, d_head), got {tuple(x.shape)}")
+    _, H, T, d_h = x.shape
     med = median_mult is not None and T > 0
     tmpl = cache._append_template
     if tmpl is None or tmpl[0] is not joint or tmpl[1] is not slack or tmpl[2] != (joint.data_ptr(), cache.main.data_ptr(), radius_bits, d_h, med):
@@ -316,25 +292,11 @@ def _append_args(x, cache, joint, slack, radius_bits, t_off, pos, median_mult, t
             a.sideband, a.sb_cap = L.addr(cache.sideband), cache.sb_cap
             a.sb_tile_off, a.sb_count = L.addr(cache.sb_tile_off), L.addr(cache.sb_count)
             a.overflow, a.sb_coord = L.addr(cache.sb_overflow), L.addr(cache.sb_coord)
+        a.address = C.addressof(a)
         tmpl = cache._append_template = (joint, slack, (joint.data_ptr(), cache.main.data_ptr(), radius_bits, d_h, med), a, grid)
     elif joint.dtype != x.dtype or joint.shape[0] != H:
         _check_joint(x, joint)
-    a = L.AppendArgs.from_buffer_copy(tmpl[3])
-    q = a.q
-    q.x = x.data_ptr()
-    q.x_stride_b, q.x_stride_h, q.x_stride_t, _ = x.stride()
-    q.B, q.T, q.t_off = B, T, t_off
-    if pos is not None:
-        q.pos = pos.data_ptr()
-    cnt = ws = None
-    if med:
-        ws = _med_workspace(x, tag)
-        cnt = torch.empty(H, dtype=torch.int32, device=x.device)           # every path of the library writes all H counts
-        base, n = ws.data_ptr(), ws.numel()
-        spare = base + (n - 12 * H & -16)
-        a.median_mult, a.med_workspace, a.med_workspace_bytes = median_mult, base, n
-        a.median, a.thr, a.n_out = spare, spare + 4 * H, cnt.data_ptr()
-    return a, tmpl[4], x, cnt, ws
+    return tmpl[3], tmpl[4], _med_workspace(x, tag) if med else None
 
 
 def _i32(t: torch.Tensor) -> torch.Tensor:
@@ -345,16 +307,8 @@ def _i32(t: torch.Tensor) -> torch.Tensor:
 def dequant(idx, radius_q, radius_scale, joint, r_qmax: int) -> torch.Tensor:
     """Unpacked codes -> dense (B, H, T, 4n) in joint.dtype (rounding of the reference's torch decode)."""
     L.require_gpu(idx, "idx")
-    idx, rq = _i32(idx), _i32(radius_q)
-    B, H, T, n = idx.shape
-    rs = radius_scale.to(joint.dtype)
-    if joint.stride(-1) != 1 or joint.stride(1) != 4:
-        joint = joint.contiguous()
-    out = torch.empty(B, H, T, 4 * n, dtype=joint.dtype, device=idx.device)
-    si, sr, ss = idx.stride(), rq.stride(), rs.stride()
-    L.call(L.lib().hqmq_dequant, "hqmq_dequant", idx.device.index, idx.data_ptr(), si[0], si[1], si[2], rq.data_ptr(), sr[0], sr[1], sr[2],
-           rs.data_ptr(), ss[0], ss[1], ss[2], joint.data_ptr(), joint.stride(0), joint.shape[1], _dt(joint), B, H, T, n, r_qmax, out.data_ptr())
-    return out
+    _dt(joint)
+    return L.tensors(L.native().dequant(idx, radius_q, radius_scale, joint, r_qmax), "hqmq_dequant")
 
 
 def pack_codes(idx, radius_q, cache, T: Optional[int] = None) -> None:
@@ -432,6 +386,17 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
         plan = _attn_plan(Q, Kc, Vc, ks, vs)
     _, _, _, tmpl, o_stride, rows, floats, splits = plan
     dev = Q.device
+    few = shape[2] == 1 and shape[1] < 64 * Kc.H       # not for the prefill kernels: the choice looks at nothing but the key below
+    if not (skip_combine or static_scratch or kernel_events or workspace is not None) and (few or n_splits > 0):
+        wide = Vc.wide_range                       # V scales outside [2^-8, 2^15): the generic kernel guards the range
+        n = n_splits if n_splits > 0 else splits.get(((T_kv + 63) // 64, kv_lens is None, wide, force_generic))
+        if n is not None:
+            for t, what in ((kv_starts, "kv_starts must hold one entry per sequence"), (batch_order, "batch_order must be a permutation of the sequences")):
+                if t is not None and t.numel() != shape[0]:
+                    raise L.HqmqError(f"{what} ({shape[0]})")
+            return L.tensors(L.native().attn(Q, tmpl.address, out, T_kv, kv_lens, kv_starts, batch_order, causal, causal_offset, softmax_scale, n,
+                                             force_generic, fp8_table_storage, wide, _workspace(rows * floats * n * 4, dev, "attn") if n > 1 else None),
+                             "hqmq_attn_fwd")
     index = dev.index
     O = torch.empty_like(Q) if out is None else out
     a = L.AttnArgs.from_buffer_copy(tmpl)          # this call's own: several threads may attend over one cache
@@ -472,15 +437,13 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
     if n_splits <= 0:
         if static_scratch:
             n_splits = pick_splits(shape[0], shape[1], Kc.H, shape[2], max(T_kv, 1), kv_lens is not None)
-        elif shape[2] > 1 or shape[1] >= 64 * Kc.H:        # the prefill kernels may take it: the choice looks at more than the key below
+        elif not few:
             n_splits = L.lib().hqmq_attn_splits(C.addressof(a))
         else:                                      # of one token, the library's choice changes at multiples of 64 tokens only
-            key = ((T_kv + 63) // 64, kv_lens is None, a.wide_range, a.force_generic)
-            n_splits = splits.get(key)
-            if n_splits is None:
-                if len(splits) >= 4096:
-                    splits.clear()
-                n_splits = splits[key] = L.lib().hqmq_attn_splits(C.addressof(a))
+            if len(splits) >= 4096:
+                splits.clear()
+            key = ((T_kv + 63) // 64, kv_lens is None, Vc.wide_range, force_generic)
+            n_splits = splits[key] = L.lib().hqmq_attn_splits(C.addressof(a))
     a.n_splits = n_splits
     if static_scratch:
         L.call(L.lib().hqmq_attn_fwd_static, "hqmq_attn_fwd_static", index, C.addressof(a))
@@ -511,73 +474,30 @@ def fused_unpacked(Q: torch.Tensor, k: tuple, v: tuple, r_qmax: int, *, kv_lens:
     """Attention of Q over unpacked codes: k and v are (idx, radius_q, radius_scale, joint).  One launch packs both tensors into
     planes of this call, then the packed attention runs over them."""
     dt = Q.dtype
-    sides = []
-    for idx, rq, rs, joint in (k, v):
-        idx, rq = _i32(idx), _i32(rq)
-        if rq.shape != idx.shape:
-            raise L.HqmqError(f"radius codes {tuple(rq.shape)} and indices {tuple(idx.shape)} differ in shape")
-        if rs.dtype is not dt:
-            rs = rs.to(dt)
-        if rs.shape != idx.shape[:3]:
-            rs = rs.expand(idx.shape[:3])
-        if joint.stride(-1) != 1 or joint.stride(1) != 4:
-            joint = joint.contiguous()
-        sides.append((idx, rq, rs, joint))
-    (idx, _, _, joint), (idx_v, _, _, joint_v) = sides
+    idx, rq, _, joint = k
+    idx_v, rq_v, _, joint_v = v
+    for i, r in ((idx, rq), (idx_v, rq_v)):
+        if r.shape != i.shape:
+            raise L.HqmqError(f"radius codes {tuple(r.shape)} and indices {tuple(i.shape)} differ in shape")
     if idx_v.shape[0] != idx.shape[0] or idx_v.shape[1] != idx.shape[1] or idx_v.shape[3] != idx.shape[3] or Q.shape[0] != idx.shape[0]:
         raise L.HqmqError("K and V codes must have equal batch, head and chunk counts, Q the same batch")
     if Q.stride(-1) != 1:
         Q = Q.contiguous()
-    dev = idx.device
     key = (Q.shape, Q.stride(), idx.shape, idx_v.shape[2], joint.shape[1], joint_v.shape[1], r_qmax, dt)
     plan = _FUSED.get(key)
     if plan is None:
         if len(_FUSED) >= 256:                     # shapes that no longer come
             _FUSED.clear()
         plan = _FUSED[key] = _fused_plan(Q, idx, idx_v.shape[2], joint.shape[1], joint_v.shape[1], r_qmax)
-    pack_tmpl, attn_tmpl, offsets, nbytes, o_stride, per_split = plan
-    buf = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    base = buf.data_ptr()
-    most = None if dt is torch.float16 else torch.zeros(2, dtype=torch.int32, device=dev)
-    pack, a = L.PackArgs.from_buffer_copy(pack_tmpl), L.AttnArgs.from_buffer_copy(attn_tmpl)
-    for i, (t, (ix, rq, rs, jt)) in enumerate(zip((a.K, a.V), sides)):
-        p = pack.side[i]
-        p.idx, p.rq, p.scale_in = ix.data_ptr(), rq.data_ptr(), rs.data_ptr()
-        p.idx_sb, p.idx_sh, p.idx_st, _ = ix.stride()
-        p.rq_sb, p.rq_sh, p.rq_st, _ = rq.stride()
-        p.scale_sb, p.scale_sh, p.scale_st = rs.stride()
-        p.main_plane = t.main_plane = base + offsets[i]
-        p.scale_plane = t.scale_plane = base + offsets[2 + i]
-        if pack.aux_bits:
-            p.aux_plane = t.aux_plane = base + offsets[4 + i]
-        t.joint, t.joint_sh = jt.data_ptr(), jt.stride(0)
-        if most is not None:
-            p.scale_max_bits = t.scale_max_bits = most.data_ptr() + 4 * i
-    L.call(L.lib().hqmq_pack_kv, "hqmq_pack_kv", dev.index, C.addressof(pack))
-    if dt is torch.bfloat16 and not torch.cuda.is_current_stream_capturing():
-        # one device read: V scales outside [2^-8, 2^15) take the kernel that guards the fp16 range
-        top = float(most.cpu().view(torch.float32)[1])
-        a.wide_range = 1 if top >= 32768.0 or 0.0 < top < 2.0 ** -8 else 0
-    O = torch.empty_like(Q)
-    a.Q, a.O = Q.data_ptr(), O.data_ptr()
-    if softmax_scale is not None:
-        a.softmax_scale = softmax_scale
-    if kv_lens is not None:
-        kv_lens = kv_lens.to(device=dev, dtype=torch.int32).contiguous()
-        a.kv_len = kv_lens.data_ptr()
-    if causal:
-        a.causal, a.causal_offset = 1, causal_offset
-    a.n_splits = n_splits if n_splits > 0 else L.lib().hqmq_attn_splits(C.addressof(a))
-    if a.n_splits > 1:
-        ws = _workspace(per_split * a.n_splits, dev, "attn")
-        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel() * ws.element_size()
-    L.call(L.lib().hqmq_attn_fwd, "hqmq_attn_fwd", dev.index, C.addressof(a))
-    return O
+    pack, a, nbytes = plan
+    capturing = dt is torch.bfloat16 and torch.cuda.is_current_stream_capturing()
+    return L.tensors(L.native().fused(Q, *k, *v, pack.address, a.address, nbytes, kv_lens, causal, causal_offset, softmax_scale, n_splits, capturing),
+                     "hqmq_attn_fwd")
 
 
 def _fused_plan(Q: torch.Tensor, idx: torch.Tensor, T_v: int, K: int, K_v: int, r_qmax: int):
-    """What the shapes fix of a fused_unpacked call: both argument blocks, where the planes lie in its buffer, the bytes of the
-    buffer, the output's strides, the workspace bytes per split."""
+    """What the shapes fix of a fused_unpacked call: both argument blocks, with the planes' offsets in its buffer, and the bytes of
+    the buffer."""
     B, H, T, n = idx.shape
     Hq, Tq = Q.shape[1], Q.shape[2]
     radius_bits = max(1, int(r_qmax).bit_length())
@@ -594,21 +514,20 @@ def _fused_plan(Q: torch.Tensor, idx: torch.Tensor, T_v: int, K: int, K_v: int, 
         offsets.append(at)
         at += (size + 255) // 256 * 256
     pack, a = L.PackArgs(), L.AttnArgs()
-    for p, t in zip(pack.side, (T, T_v)):
-        p.T = t
+    for i, t in enumerate((T, T_v)):
+        p = pack.side[i]
+        p.T, p.main_plane, p.scale_plane, p.aux_plane = t, offsets[i], offsets[2 + i], offsets[4 + i]
     code = L.DT_CODE[Q.dtype]
     pack.dtype, pack.B, pack.H, pack.n_chunks, pack.t_cap = code, B, H, n, cap
     pack.idx_bits, pack.main_bits, pack.aux_bits = ib, mb, ab
     a.q_sb, a.q_sh, a.q_st = Q.stride(0), Q.stride(1), Q.stride(2)
-    o_stride = torch.empty_like(Q).stride()
-    a.o_sb, a.o_sh, a.o_st = o_stride[0], o_stride[1], o_stride[2]
     for t, rows in ((a.K, K), (a.V, K_v)):
         t.scale_sb, t.scale_sh, t.scale_st, t.K = H * cap, cap, 1, rows
     a.dtype, a.B, a.H_q, a.H_kv, a.T_q, a.T_kv, a.n_chunks, a.t_cap = code, B, Hq, H, Tq, T, n, cap
     a.idx_bits, a.main_bits, a.aux_bits, a.qmax = ib, mb, ab, int(r_qmax)
     a.softmax_scale = Q.shape[3] ** -0.5
-    per_split = int(L.lib().hqmq_attn_workspace_bytes(C.c_int(B), C.c_int(Hq), C.c_int(Tq), C.c_int(Q.shape[3]), C.c_int(2))) // 2
-    return pack, a, offsets, max(at, 256), o_stride, per_split
+    pack.address, a.address = C.addressof(pack), C.addressof(a)
+    return pack, a, max(at, 256)
 
 
 def _attn_plan(Q: torch.Tensor, Kc, Vc, ks, vs):
@@ -636,6 +555,7 @@ def _attn_plan(Q: torch.Tensor, Kc, Vc, ks, vs):
     plan = (ks, vs, Q.dtype, a, o_stride, rows, per_split // rows, {})
     if len(Kc._attn_plans) >= 64:                  # shapes that no longer come
         Kc._attn_plans.clear()
+    a.address = C.addressof(a)
     Kc._attn_plans[(Q.shape, Q.stride())] = plan
     return plan
 

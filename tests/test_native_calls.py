@@ -1,0 +1,127 @@
+"""The compiled host side of the calls: inputs as they come (strides, integer and float types, expanded scales) against the same values
+laid out plainly, errors as exceptions, calls from several threads on streams of their own."""
+import threading
+
+import pytest
+import torch
+
+from tests.helpers import bit_equal
+
+DEV = "cuda:0"
+
+
+def test_refuses_what_is_not_a_call():
+    from hqmq_amd import _lib as L
+    n = L.native()
+    for f in (n.codes, n.fake, n.med3x, n.append, n.dequant, n.attn, n.fused):
+        with pytest.raises(TypeError):
+            f()
+    with pytest.raises(TypeError):
+        n.dequant(1, 2, 3, 4, 5)
+    with pytest.raises(ValueError):
+        n.med3x(torch.zeros(3, 4), 3.0, torch.zeros(4), True)
+    with pytest.raises(L.HqmqError):
+        L.tensors(-2, "a call")
+
+
+def _setup(dt, med, T=70):
+    import hqmq
+    q = hqmq.HQMQ(n_layers=1, n_heads=3, secondary_size=24, radius_bits=4, device=DEV)
+    g = torch.Generator().manual_seed(7)
+    k, v = (torch.randn(2, 3, T, 64, generator=g).to(dt).to(DEV) for _ in range(2))
+    return (hqmq.with_outlier_extraction(q, C=2.0) if med else q), k, v
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dn", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("med", [False, True])
+def test_inputs_as_they_come(dn, med):
+    import hqmq
+    from hqmq.kernels import decode_dequant
+    dt = getattr(torch, dn)
+    w, k, v = _setup(dt, med)
+    plain = w.encode_K(k, 0)
+    views = [k.transpose(1, 2).contiguous().transpose(1, 2), torch.nn.functional.pad(k, (3, 2))[..., 3:67], k.transpose(2, 3).contiguous().transpose(2, 3)]
+    for view in views:
+        assert view.stride() != k.stride()
+        got = w.encode_K(view, 0)
+        assert got.keys() == plain.keys()
+        assert all(bit_equal(got[n], plain[n]) if plain[n].is_floating_point() else torch.equal(got[n], plain[n]) for n in plain)
+        assert bit_equal(w.quantize_K(view, 0), w.quantize_K(k, 0))
+        a, b = w.new_cache(2, 128, 64, dt, 0), w.new_cache(2, 128, 64, dt, 0)
+        w.append(a, view, v, 0)
+        w.append(b, k, v, 0)
+        assert torch.equal(a.K.main, b.K.main) and torch.equal(a.V.main, b.V.main) and bit_equal(a.K.scale, b.K.scale)
+    vc = w.encode_V(v, 0)
+    qmax = 15
+    dense = decode_dequant(plain["idx"], plain["rq"], plain["r_max"], plain["joint"], qmax)
+    odd = (plain["idx"].long(), plain["rq"].to(torch.int16).transpose(0, 1).contiguous().transpose(0, 1), plain["r_max"].float(), plain["joint"])
+    assert bit_equal(decode_dequant(*odd, qmax), dense)
+    Q = torch.randn(2, 6, 1, 64, generator=torch.Generator().manual_seed(1)).to(dt).to(DEV)
+    one = torch.ones_like(plain["r_max"][:, :, :1])
+    V = (vc["idx"], vc["rq"], vc["r_max"], vc["joint"])
+    want = hqmq.fused_attention(Q, plain["idx"], plain["rq"], one.expand(2, 3, 70).contiguous(), plain["joint"], *V, qmax, causal=False)
+    got = hqmq.fused_attention(Q.expand(2, 6, 1, 64), odd[0], odd[1], one, plain["joint"], *V, qmax, causal=False)
+    assert bit_equal(got, want)
+    for lens in (torch.tensor([70, 9]), torch.tensor([70, 9], dtype=torch.int32, device=DEV)):
+        O = hqmq.fused_attention_packed(Q, b, kv_lens=lens, T_kv=70)
+        assert bit_equal(O, hqmq.fused_attention_packed(Q, b, kv_lens=lens.to(DEV).int(), T_kv=70, out=torch.empty_like(Q)))
+        assert bit_equal(hqmq.fused_attention(Q, plain["idx"], plain["rq"], plain["r_max"], plain["joint"], *V, qmax, causal=False, kv_lens=lens),
+                         hqmq.fused_attention(Q, plain["idx"], plain["rq"], plain["r_max"], plain["joint"], *V, qmax, causal=False, kv_lens=lens.to(DEV).int()))
+
+
+@pytest.mark.gpu
+def test_errors_are_exceptions():
+    import hqmq
+    from hqmq.kernels import decode_dequant
+    from hqmq_amd import _lib as L, ops
+    w, k, v = _setup(torch.float16, False)
+    c = w.encode_K(k, 0)
+    joint, slack = w._joint_and_slack(0, 0, k)
+    for call in (lambda: ops.quantize(k.float(), joint, slack, 4), lambda: ops.quantize(k[:, :2], joint, slack, 4), lambda: ops.fake_quant(k[0], joint, slack, 4)):
+        with pytest.raises(ValueError):
+            call()
+    with pytest.raises(L.HqmqError):                        # a status of the library
+        decode_dequant(c["idx"], c["rq"], c["r_max"], c["joint"], 0)
+    with pytest.raises(L.HqmqError):
+        decode_dequant(c["idx"], c["rq"], c["r_max"], c["joint"].double(), 15)
+    with pytest.raises(L.HqmqError):
+        ops.quantize(k.cpu(), joint, slack, 4)
+    cache = w.new_cache(2, 128, 64, torch.float16, 0)
+    w.append(cache, k, v, 0)
+    Q = torch.zeros(2, 6, 1, 64, dtype=torch.float16, device=DEV)
+    for kw in (dict(batch_order=torch.zeros(3, dtype=torch.int32, device=DEV)), dict(kv_starts=torch.zeros(1, dtype=torch.int32, device=DEV))):
+        for _ in range(2):                                  # the first call works out the splits
+            with pytest.raises(L.HqmqError):
+                hqmq.fused_attention_packed(Q, cache, **kw)
+            hqmq.fused_attention_packed(Q, cache)
+
+
+@pytest.mark.gpu
+def test_threads_on_streams_of_their_own():
+    import hqmq
+    w, k, v = _setup(torch.float16, True, T=300)
+    Q = torch.randn(2, 6, 1, 64, generator=torch.Generator().manual_seed(1)).half().to(DEV)
+    want = (w.encode_K(k, 0)["idx"], w.quantize_K(k, 0))
+    cache = w.new_cache(2, 300, 64, torch.float16, 0)
+    w.append(cache, k, v, 0)
+    O = hqmq.fused_attention_packed(Q, cache, n_splits=2)
+    torch.cuda.synchronize()
+    bad = []
+
+    def work():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(20):
+                own = w.new_cache(2, 300, 64, torch.float16, 0)
+                w.append(own, k, v, 0)
+                got = w.encode_K(k, 0)["idx"], w.quantize_K(k, 0), hqmq.fused_attention_packed(Q, cache, n_splits=2), own.K.main
+                torch.cuda.current_stream().synchronize()
+                if not (torch.equal(got[0], want[0]) and bit_equal(got[1], want[1]) and bit_equal(got[2], O) and torch.equal(got[3], cache.K.main)):
+                    bad.append(1)
+
+    threads = [threading.Thread(target=work) for _ in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
