@@ -56,7 +56,7 @@ __device__ __forceinline__ void load_scales4(const void *plane, int dtype, int64
 }
 
 template <int CPL, int MB, bool FLAGS>
-__global__ __launch_bounds__(kAttnWaves * 64) void attn_kernel(AttnParams p) {
+__device__ __forceinline__ void attn_block(const AttnParams &p, const int sp, const int cg, const int bz) {
     constexpr int NB = CPL * MB / 8;
     constexpr int NW = (NB + 3) / 4;
     extern __shared__ uint2 lds_tab[];
@@ -64,10 +64,9 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_kernel(AttnParams p) {
 
     // blocks are dispatched in grid order: batch_order lists the sequences in the order they should start
     // (longest first for ragged batches, so that no long sequence is left for the end)
-    const int slot = blockIdx.z / p.Hkv, hkv = blockIdx.z - slot * p.Hkv;
+    const int slot = bz / p.Hkv, hkv = bz - slot * p.Hkv;
     const int b = p.batch_order ? min(max(p.batch_order[slot], 0), p.B - 1) : slot;
     const int bh = b * p.Hkv + hkv;
-    const int cg = blockIdx.y, sp = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int dtype = p.dtype;
     const int n = p.n, G = p.G;
@@ -308,6 +307,23 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_kernel(AttnParams p) {
         }
     }
 }
+template <int CPL, int MB, bool FLAGS>
+__global__ __launch_bounds__(kAttnWaves * 64) void attn_kernel(AttnParams p) {
+    attn_block<CPL, MB, FLAGS>(p, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+// Behind a specialised kernel whose results stand only if the largest V scale, which the GPU has just worked out, lies in
+// [2^-8, 2^15): does nothing then (256 blocks that read one word, 3 us), else the whole call again.  (Reading the scale back and
+// choosing on the host left the GPU idle for 18 us: bf16 attention over unpacked codes, 64 tokens, 30.9 us instead of 21.5.)
+template <int CPL, int MB>
+__global__ __launch_bounds__(kAttnWaves * 64) void attn_again_kernel(AttnParams p, unsigned gx, unsigned gy, unsigned blocks) {
+    const float top = __uint_as_float(*p.Vc.scale_max);
+    if (!(top >= 32768.f || (top > 0.f && top < 0.00390625f))) return;
+    for (unsigned i = blockIdx.x; i < blocks; i += gridDim.x) {
+        const unsigned y = i / gx, z = y / gy;
+        attn_block<CPL, MB, false>(p, (int)(i - y * gx), (int)(y - z * gy), (int)z);
+        __syncthreads();            // the LDS of one block is the next one's
+    }
+}
 
 // Merge of the split partials: one block of 256 threads per output row.  A thread owns four consecutive output
 // elements (one 16-byte load per split) and every (256 / (d_h / 4))-th split; it loads its splits in batches of four
@@ -475,6 +491,17 @@ static int launch_attn(const AttnParams &p, bool flags, dim3 grid, size_t shmem,
     return hip_status(hipGetLastError());
 }
 
+template <int CPL, int MB>
+static int launch_again(const AttnParams &p, dim3 grid, size_t shmem, hipStream_t st) {
+    auto kern = attn_again_kernel<CPL, MB>;
+    const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+    if (e != hipSuccess) return (int)e;
+    const uint64_t blocks = (uint64_t)grid.x * grid.y * grid.z;
+    if (blocks > 0x7fffffffull) return HQMQ_ERR_SHAPE;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(blocks < 256 ? blocks : 256)), dim3(kAttnWaves * 64), shmem, st, p, grid.x, grid.y, (unsigned)blocks);
+    return hip_status(hipGetLastError());
+}
+
 template <int CPL>
 static int launch_attn_mb(const AttnParams &p, int mb, bool flags, dim3 grid, size_t shmem, hipStream_t st, const LaunchTiming &tm) {
     switch (mb) {
@@ -547,7 +574,7 @@ extern "C" int hqmq_attn_splits(const hqmq_attn_args *a) {
     if (!a || a->B < 1 || a->H_kv < 1 || a->H_q < 1 || a->T_q < 1 || a->T_kv < 1) return 1;
     const int splits = attn_prefill_splits(a, 0);
     if (splits > 0) return splits;
-    const bool generic = a->dtype == HQMQ_F32 || a->wide_range || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
+    const bool generic = a->dtype == HQMQ_F32 || attn_wide(a) || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
     const int64_t nz = (int64_t)a->B * a->H_kv, groups = ((int64_t)a->T_q * (a->H_q / a->H_kv) + 15) / 16;
     return decode_splits(nz * groups, generic || a->K.flag_plane || groups < 2 ? 0 : nz * ((groups + 1) / 2),
                          (int64_t)a->B * a->H_q * a->T_q, a->T_kv, a->kv_len != nullptr,
@@ -632,7 +659,7 @@ static int attn_fwd_impl(const hqmq_attn_args *a, void *stream) {
     // Ragged batches keep the sequence-major order that batch_order relies on.
     p.xcd_remap = (!a->kv_len && !a->batch_order && ((a->B * a->H_kv) % 8) == 0) ? 1 : 0;
     p.tab_fp8 = a->fp8_table_storage ? 1 : 0;
-    p.wide_range = a->wide_range ? 1 : 0;
+    p.wide_range = attn_wide(a) ? 1 : 0;
     p.no_lds_landing = a->force_generic == 2 ? 1 : 0;
     // 4 consecutive scales with one vector load: unit stride, aligned rows, and capacity rows readable
     const int salign = a->dtype == HQMQ_F32 ? 16 : 8;
@@ -678,6 +705,12 @@ static int attn_fwd_impl(const hqmq_attn_args *a, void *stream) {
         default: return HQMQ_ERR_SHAPE;
     }
     if (rc) return rc;
+    if (handled && a->wide_range) {         // the specialised kernels ran on trust: attn_wide saw that the GPU can tell
+        const bool w16 = a->main_bits == 16;
+        rc = n == 32 ? (w16 ? launch_again<8, 16>(p, grid, shmem, st) : launch_again<8, 12>(p, grid, shmem, st))
+                     : (w16 ? launch_again<4, 16>(p, grid, shmem, st) : launch_again<4, 12>(p, grid, shmem, st));
+        if (rc) return rc;
+    }
     if (n_splits > 1 && !a->skip_combine)
         rc = hqmq_attn_combine(a->workspace, a->O, a->dtype, a->B, a->H_q, a->T_q, 4 * n, n_splits, a->o_sb, a->o_sh, a->o_st,
                                stream);

@@ -9,8 +9,6 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
-#include <cstring>
-
 #include "../../include/hqmq_amd.h"
 
 namespace {
@@ -290,10 +288,10 @@ PyObject *attn(PyObject *, PyObject *const *o, Py_ssize_t count) {
 }
 
 // fused(Q, K idx, rq, scale, joint, V idx, rq, scale, joint, pack block, attention block, bytes of the planes, kv_lens or None,
-//       causal, causal_offset, scale or None, n_splits, capturing) -> O.  The blocks hold the planes' offsets in place of addresses.
+//       causal, causal_offset, scale or None, n_splits) -> O.  The blocks hold the planes' offsets in place of addresses.
 PyObject *fused(PyObject *, PyObject *const *o, Py_ssize_t count) {
     HANDLE_TH_ERRORS
-    arguments(count, 18);
+    arguments(count, 17);
     const at::Tensor &Q = tensor(o[0]);
     const auto dt = Q.scalar_type();
     hqmq_pack_args pack = *address<hqmq_pack_args>(o[9]);
@@ -333,16 +331,7 @@ PyObject *fused(PyObject *, PyObject *const *o, Py_ssize_t count) {
     }
     int status = go([&](void *stream) { return hqmq_pack_kv(&pack, stream); });
     if (status) return PyLong_FromLong(status);
-    if (dt == at::kBFloat16 && !PyObject_IsTrue(o[17])) {
-        // one device read: V scales outside [2^-8, 2^15) take the kernel that guards the fp16 range
-        float top;
-        {
-            WithoutGil release;
-            const at::Tensor host = most.cpu();
-            std::memcpy(&top, (const char *)host.data_ptr() + 4, 4);
-        }
-        a.wide_range = top >= 32768.f || (top > 0.f && top < 0.00390625f) ? 1 : 0;
-    }
+    if (dt == at::kBFloat16) a.wide_range = 2;          // V scales outside [2^-8, 2^15) need the kernel that guards the fp16 range
     const at::Tensor O = at::empty_like(Q);
     output(a, Q, O);
     at::Tensor lens, ws;

@@ -490,8 +490,7 @@ def fused_unpacked(Q: torch.Tensor, k: tuple, v: tuple, r_qmax: int, *, kv_lens:
             _FUSED.clear()
         plan = _FUSED[key] = _fused_plan(Q, idx, idx_v.shape[2], joint.shape[1], joint_v.shape[1], r_qmax)
     pack, a, nbytes = plan
-    capturing = dt is torch.bfloat16 and torch.cuda.is_current_stream_capturing()
-    return L.tensors(L.native().fused(Q, *k, *v, pack.address, a.address, nbytes, kv_lens, causal, causal_offset, softmax_scale, n_splits, capturing),
+    return L.tensors(L.native().fused(Q, *k, *v, pack.address, a.address, nbytes, kv_lens, causal, causal_offset, softmax_scale, n_splits),
                      "hqmq_attn_fwd")
 
 

@@ -305,7 +305,9 @@ typedef struct hqmq_attn_args {
                                  subnormals; such a cache takes the layout-generic kernel, which reads
                                  hqmq_packed.scale_max_bits and keeps every product inside the normal fp16 range (fp32 caches
                                  always take it).  Callers that track the bound (hqmq_quantize_args.scale_max_bits) set this
-                                 when it leaves [2^-8, 2^15); data of ordinary magnitude never does. */
+                                 when it leaves [2^-8, 2^15); data of ordinary magnitude never does.
+                                 2: the GPU decides, from V.scale_max_bits as it stands when the call's kernels run (16-bit
+                                 caches without outliers; as 1 where that word is NULL). */
 } hqmq_attn_args;
 int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, int n_splits);
 /* The n_splits hqmq_attn_fwd would choose, from the shapes alone; ragged = 1 when kv_len is passed (sequences of different

@@ -125,3 +125,36 @@ def test_threads_on_streams_of_their_own():
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,b_r,d_h", [(96, 4, 128), (24, 3, 64), (192, 6, 64), (24, 3, 128)])
+@pytest.mark.parametrize("B,T,Tq,n_splits", [(1, 70, 1, 0), (2, 700, 1, 5), (1, 300, 300, 0), (3, 200, 7, 1), (9, 65, 40, 2)])
+def test_unpacked_bf16_scales_of_any_size(S, b_r, d_h, B, T, Tq, n_splits):
+    """V scales times a power of two: the outputs times the same power, whichever kernel the GPU lets run.  Each kernel keeps
+    to 2e-3 plus fp16 noise (8 * 2^-11 of the attention-weighted |V|, about 1 here) of exact arithmetic, and each output is rounded to
+    bf16 once, by half a unit in the last place, which is 2^-8 of the value at most."""
+    import hqmq
+    dt = torch.bfloat16
+    q = hqmq.HQMQ(n_layers=1, n_heads=2, secondary_size=S, radius_bits=b_r, device=DEV)
+    g = torch.Generator().manual_seed(T)
+    k, v = (torch.randn(B, 2, T, d_h, generator=g).to(dt).to(DEV) for _ in range(2))
+    Q = torch.randn(B, 8, Tq, d_h, generator=g).to(dt).to(DEV)
+    ck, cv = q.encode_K(k, 0), q.encode_V(v, 0)
+    qmax = (1 << b_r) - 1
+
+    def attend(power):
+        return hqmq.fused_attention(Q, ck["idx"], ck["rq"], ck["r_max"], ck["joint"], cv["idx"], cv["rq"], cv["r_max"] * 2.0 ** power, cv["joint"], qmax,
+                                    causal=Tq > 1, n_splits=n_splits)
+
+    want = attend(0).float()
+    for power in (20, -30, 13, -7, 60, -60):
+        got = attend(power).float() * 2.0 ** -power
+        assert bool(((got - want).abs() <= 1.2e-2 + 2.0 ** -7 * want.abs()).all()), (power, float((got - want).abs().max()))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = attend(20)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool(((out.float() * 2.0 ** -20 - want).abs() <= 1.2e-2 + 2.0 ** -7 * want.abs()).all())
