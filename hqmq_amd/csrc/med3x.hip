@@ -541,7 +541,7 @@ __global__ __launch_bounds__(1024) void count_gt_kernel(MedPair a, int64_t rows_
     if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(&m.n_out[h], (int)cnt);
 }
 
-// Small calls (a decode step appends B * n chunks per head): norms, exact order statistics and count in one launch, one
+// Small calls (a decode step appends B * n chunks per head), fp32, or of at most 64 chunks: norms, exact order statistics and count in one launch, one
 // block per head, up to eight keys per lane in registers.  The key of rank r is the largest v with fewer than r + 1 keys below
 // it, found bit by bit from the top: a compare and a scalar bit count per key, one barrier per round (none in a block of
 // one wavefront); two bits, three thresholds a round.  The second rank is the next one: the same key again, or the smallest key above it.
@@ -651,6 +651,128 @@ __global__ __launch_bounds__(NT) void med_small_kernel(MedPair a) {
         if (tid == 0) m.n_out[h] = (int32_t)c;
     }
     if (tid == 0) finish_threshold<D>(x, y, r_lo == r_hi, m.mult, h, m.median, (ST *)m.thr);
+}
+
+// 16-bit calls of 65 to 16384 chunks per head: one block per head and a histogram of the 15-bit keys in LDS, 16-bit counters two to a
+// word, instead of a search bit by bit (a barrier, 24 compares and three LDS atomics per wavefront for every two bits).  A wavefront
+// owns 2048 neighbouring keys, a lane four words of each quarter of them (reads of 16 bytes side by side): a sum per quarter, the
+// wavefronts' sums through LDS, then the wavefront that holds a rank finds its quarter, lane and key.  Ranks, NaN rule and count as in
+// med_small_kernel.  Clearing, four barriers and code that arrives cold bound it, so the code is no longer than its keys per lane ask
+// for; us replayed in a graph, 8 heads fp16, against the search: 512 chunks 5.3 -> 4.8, 1024 7.2 -> 4.9, 2048 7.6 -> 5.5, 4096 7.3 -> 6.1, 8192
+// 7.4; against two launches over histograms of blocks: 16384 10.4 -> 10.0, one launch saved.  Up to 64 chunks the search is one wavefront
+// without a barrier: 2.7 against 4.7.
+constexpr int kLdsBins = 32768;
+template <class D, int KEYS>
+__global__ __launch_bounds__(1024) void med_lds_kernel(MedPair a) {
+    constexpr int NT = 1024;
+    extern __shared__ uint4 bins[];                 // kLdsBins / 8 of them, then the wavefronts' sums and the results
+    uint32_t *const words = reinterpret_cast<uint32_t *>(bins), *const sums = words + kLdsBins / 2, *const res = sums + 16;
+    const MedTensor &m = a.t[blockIdx.z];
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int per_head = a.B * a.T * a.n, rows = a.B * a.T;
+    using ST = typename D::storage;
+    const int per = NT / a.n, rl = tid / a.n, c = tid - rl * a.n;
+    RawChunk<D> raw[KEYS] = {};
+    bool have[KEYS];
+    {
+        const int b0 = rl / a.T;
+        int r = rl < per ? rl : rows, t = rl - b0 * a.T;
+        const ST *p = (const ST *)m.x + b0 * m.xsb + h * m.xsh + (int64_t)t * m.xst + c * 4;
+        const int dq = per / a.T, dt = per - dq * a.T;
+        const int64_t step = dq * m.xsb + dt * m.xst, wrap = m.xsb - a.T * m.xst;
+#pragma unroll
+        for (int i = 0; i < KEYS; i++) {
+            have[i] = r < rows;
+            if (have[i]) raw[i].load(p, m.vec);
+            r += per;
+            t += dt;
+            p += step;
+            if (t >= a.T) { t -= a.T; p += wrap; }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kLdsBins / 8 / NT; i++) bins[tid + i * NT] = uint4{0, 0, 0, 0};
+    if (tid < 4) res[tid] = 0;                      // low key, high key, NaN seen, count
+    __syncthreads();
+    uint32_t key[KEYS];
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < KEYS; i++) {
+        const float nrm = chunk_norm_d<D>(raw[i].get(0), raw[i].get(1), raw[i].get(2), raw[i].get(3));
+        nan |= have[i] && is_nan(nrm);
+        key[i] = (norm_bits<D>(nrm) >> 16) & 0x7fffu;
+        if (have[i]) atomicAdd(&words[key[i] >> 1], 1u << (16 * (key[i] & 1)));
+    }
+    if (__builtin_amdgcn_ballot_w64(nan) != 0ull && lane == 0) res[2] = 1;
+    __syncthreads();
+    if (res[2]) {
+        if (tid == 0) nan_threshold<D>(m, h);
+        return;
+    }
+    uint4 own[4];
+    uint32_t quarter[4], mine = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        own[i] = bins[wave * 256 + i * 64 + lane];
+        const uint32_t s = own[i].x + own[i].y, t = own[i].z + own[i].w;      // at most 8192 in each half: no carry between them
+        quarter[i] = (s & 0xffffu) + (s >> 16) + (t & 0xffffu) + (t >> 16);
+        mine += quarter[i];
+    }
+    const uint32_t total = wave_sum(mine);
+    if (lane == 0) sums[wave] = total;
+    __syncthreads();
+    uint32_t before = 0;
+    for (int w = 0; w < 16; w++) {
+        const uint32_t s = sums[w];
+        before += w < wave ? s : 0u;
+    }
+    const uint32_t ranks[2] = {(uint32_t)((per_head - 1) / 2), (uint32_t)(per_head / 2)};
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        if (ranks[k] < before || ranks[k] >= before + total) continue;        // wave-uniform
+        uint32_t left = ranks[k] - before;
+        bool found = false;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t sum = wave_sum(quarter[i]);
+            if (!found && left < sum) {
+                found = true;
+                uint32_t up = quarter[i];                                     // running sum over the lanes
+                for (int d = 1; d < 64; d <<= 1) {
+                    const uint32_t v = __shfl_up(up, d);
+                    if (lane >= d) up += v;
+                }
+                const uint32_t lo = up - quarter[i];
+                if (left >= lo && left < up) {
+                    const uint32_t w4[4] = {own[i].x, own[i].y, own[i].z, own[i].w};
+                    uint32_t at = left - lo, key16 = 0;
+                    bool hit = false;
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        const uint32_t n = (w4[j >> 1] >> (16 * (j & 1))) & 0xffffu;
+                        if (!hit && at < n) { hit = true; key16 = (uint32_t)j; }
+                        if (!hit) at -= n;
+                    }
+                    res[k] = (uint32_t)((wave * 256 + i * 64 + lane) * 8) + key16;
+                }
+            } else if (!found) {
+                left -= sum;
+            }
+        }
+    }
+    __syncthreads();
+    const float x = key_value<D>(res[0]), y = key_value<D>(res[1]);
+    const bool same = ranks[0] == ranks[1];
+    if (m.n_out) {
+        const float med = same ? x : y - (y - x) * 0.5f, tv = D::rnd(med * m.mult);
+        uint32_t above = 0;
+#pragma unroll
+        for (int i = 0; i < KEYS; i++) above += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(have[i] && key_value<D>(key[i]) > tv));
+        if (lane == 0) atomicAdd(&res[3], above);
+        __syncthreads();
+        if (tid == 0) m.n_out[h] = (int32_t)res[3];
+    }
+    if (tid == 0) finish_threshold<D>(x, y, same, m.mult, h, m.median, (ST *)m.thr);
 }
 
 // The flag bits of a row (up to 256 chunks) in registers; dwords where the row's address allows it.
@@ -864,15 +986,27 @@ template <class D>
 static int run_med3x(const MedPair &a, int count, bool parts, hipStream_t st) {
     const bool f32 = D::code == HQMQ_F32;
     const int64_t per_head = (int64_t)a.B * a.T * a.n, rows = (int64_t)a.B * a.T;
-    // Few keys per lane before few lanes: such a call lasts about as long as its code takes to arrive (every launch starts
+    // Few keys per lane: such a call lasts about as long as its code takes to arrive (every launch starts
     // with cold instruction caches), and the code is written out once per key.
     auto fits = [&](int nt, int keys) { return a.n <= nt && rows <= (int64_t)(nt / a.n) * keys; };
-    if (fits(1024, 8)) {
-        const dim3 grid(a.H, 1, count);
-        if (fits(64, 1)) hipLaunchKernelGGL((med_small_kernel<D, 64, 1>), grid, dim3(64), 0, st, a);
-        else if (fits(256, 2)) hipLaunchKernelGGL((med_small_kernel<D, 256, 2>), grid, dim3(256), 0, st, a);
-        else if (fits(1024, 2)) hipLaunchKernelGGL((med_small_kernel<D, 1024, 2>), grid, dim3(1024), 0, st, a);
-        else hipLaunchKernelGGL((med_small_kernel<D, 1024, 8>), grid, dim3(1024), 0, st, a);
+    const dim3 heads(a.H, 1, count);
+    if (fits(64, 1)) {
+        hipLaunchKernelGGL((med_small_kernel<D, 64, 1>), heads, dim3(64), 0, st, a);
+        return hip_status(hipGetLastError());
+    }
+    if constexpr (D::code == HQMQ_F32) {
+        if (fits(1024, 8)) {
+            auto kern = fits(256, 2) ? med_small_kernel<D, 256, 2> : fits(1024, 2) ? med_small_kernel<D, 1024, 2> : med_small_kernel<D, 1024, 8>;
+            hipLaunchKernelGGL(kern, heads, dim3(fits(256, 2) ? 256 : 1024), 0, st, a);
+            return hip_status(hipGetLastError());
+        }
+    } else if (fits(1024, 16)) {        // beyond, a block per head is slower than two launches (19200 chunks 15.3 against 10.5 us)
+        auto kern = fits(1024, 1) ? med_lds_kernel<D, 1> : fits(1024, 2) ? med_lds_kernel<D, 2> : fits(1024, 4) ? med_lds_kernel<D, 4>
+                  : fits(1024, 8) ? med_lds_kernel<D, 8> : med_lds_kernel<D, 16>;
+        const size_t lds = (kLdsBins / 2 + 20) * sizeof(uint32_t);
+        const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+        hipLaunchKernelGGL(kern, heads, dim3(1024), lds, st, a);
         return hip_status(hipGetLastError());
     }
     // Blocks of about 4096 chunks while that leaves at most two per CU; larger calls get larger blocks, beyond 65535 chunks

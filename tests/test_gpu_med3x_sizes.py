@@ -101,6 +101,30 @@ def test_crop_of_a_cache_made_for_cuda_without_an_index():
 
 
 @pytest.mark.parametrize("dn", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", [(1, 3, 2, 128), (1, 3, 3, 128), (2, 2, 16, 128), (1, 2, 33, 124), (5, 1, 13, 64), (1, 2, 65, 128), (2, 2, 64, 128), (1, 1, 129, 128),
+                                   (1, 2, 511, 128), (4, 1, 128, 128), (1, 2, 513, 128), (1, 2, 3, 4000), (1, 1, 16, 4096), (1, 1, 17, 4096), (3, 1, 20, 12)])
+def test_histogram_of_a_block(dn, shape):
+    """65 to 16384 chunks per head, on both sides of 1, 2, 4, 8 and 16 keys per lane and with rows that do not fill the lanes; ordinary
+    norms, all equal, two values of which the middle ranks take one each, zeros, infinities, a NaN."""
+    from hqmq_amd import ops
+    dt = DT[dn]
+    x = kv_input(shape, dt, seed=sum(shape) + 1, outlier_p=0.05)
+    n = shape[0] * shape[2] * shape[3] // 4
+    flat = torch.arange(n).view(1, n, 1).expand(shape[1], n, 4)
+    two = torch.where(flat < n // 2, 0.25, 2.0).reshape(shape[1], shape[0], shape[2], shape[3]).transpose(0, 1)
+    inf = x.clone()
+    inf[:, :, ::2, 0] = float("inf")
+    nan = x.clone()
+    nan[-1, -1, -1, -1] = float("nan")
+    for y in (x, torch.full(shape, 0.5).to(dt), two.to(dt), torch.zeros(shape).to(dt), inf, nan):
+        want = CO.med3x(y, 3.0)
+        med, thr, cnt = ops.med3x_threshold(y.to(DEV), 3.0)
+        same = (med.cpu() == want["median"]) | (med.cpu().isnan() & want["median"].isnan())
+        assert same.all() and (bit_equal(thr, want["threshold"]) or thr.isnan().any())
+        assert torch.equal(cnt.cpu().long(), want["mask"].sum(dim=(0, 2, 3)))
+
+
+@pytest.mark.parametrize("dn", ["fp16", "bf16"])
 @pytest.mark.parametrize("H,rows,mult", [(1, 4100, 3.0), (7, 600, 100.0), (300, 257, 0.01), (2, 4097, 0.0), (3, 5000, 1e5)])
 def test_histograms_of_blocks(dn, H, rows, mult):
     """16-bit types beyond 8192 chunks per head: one part of the workspace per block, from one part for a head to as many as a
