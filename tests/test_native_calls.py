@@ -158,3 +158,25 @@ def test_unpacked_bf16_scales_of_any_size(S, b_r, d_h, B, T, Tq, n_splits):
         graph.replay()
         torch.cuda.synchronize()
         assert bool(((out.float() * 2.0 ** -20 - want).abs() <= 1.2e-2 + 2.0 ** -7 * want.abs()).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [24, 192, 213])
+@pytest.mark.parametrize("dn", ["float16", "bfloat16"])
+def test_prefill_over_tables_of_any_alignment(dn, S):
+    """Tables read two codewords at a time, and tables that cannot be: an odd number of codewords, a base on 8 bytes."""
+    import hqmq
+    dt, T, qmax = getattr(torch, dn), 700, 15                # long enough for the prefill kernels
+    g = torch.Generator().manual_seed(S)
+    Q = torch.randn(4, 16, T, 128, generator=g).to(dt).to(DEV)
+    joint = torch.nn.functional.normalize(torch.randn(2, 24 * S, 4, generator=g), dim=-1).to(dt).to(DEV)
+    codes = [[torch.randint(1, hi, (4, 2, T, 32), generator=g).int().to(DEV) for hi in (24 * S, qmax + 1)] for _ in range(2)]
+    rs = (torch.rand(4, 2, T, generator=g) + 0.5).to(dt).to(DEV)
+    (ki, kr), (vi, vr) = codes
+
+    def attend(table, first):
+        return hqmq.fused_attention(Q, ki - first, kr, rs, table, vi - first, vr, rs, table, qmax)
+
+    want = attend(joint, 0)
+    assert bit_equal(attend(joint[:, 1:], 1), want) and bit_equal(attend(joint[:, 1:].contiguous(), 1), want)
+    assert bit_equal(attend(torch.nn.functional.pad(joint, (0, 0, 1, 0))[:, 1:], 0), want)
