@@ -310,11 +310,16 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     half8 qf[KS];
     {
         const uint16_t *qp = (const uint16_t *)p.Q + b * p.qsb + hq * p.qsh + (int64_t)tq * p.qst + 8 * half;
+        const bool wide_q = ((((uintptr_t)p.Q) | (uintptr_t)(p.qsb * 2) | (uintptr_t)(p.qsh * 2) | (uintptr_t)(p.qst * 2)) & 15) == 0;
 #pragma unroll
         for (int kk = 0; kk < KS; kk++) {
-            const uint2 lo = *reinterpret_cast<const uint2 *>(qp + 16 * kk), hi = *reinterpret_cast<const uint2 *>(qp + 16 * kk + 4);
-            const half4 z = half4{0, 0, 0, 0};
-            qf[kk] = cat8(col_ok ? chunk_to_half<DT>(lo) : z, col_ok ? chunk_to_half<DT>(hi) : z);
+            uint4v w;
+            if (wide_q) w = *reinterpret_cast<const uint4v *>(qp + 16 * kk);
+            else {
+                const uint2 lo = *reinterpret_cast<const uint2 *>(qp + 16 * kk), hi = *reinterpret_cast<const uint2 *>(qp + 16 * kk + 4);
+                w = uint4v{lo.x, lo.y, hi.x, hi.y};
+            }
+            qf[kk] = __builtin_bit_cast(half8, col_ok ? pair_to_half<DT>(w) : uint4v{0, 0, 0, 0});
         }
     }
     if (it == 0) tables();
@@ -573,18 +578,31 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     if (!col_ok || (KVG == 2 && kvg == 1)) {
     } else if (p.n_splits == 1) {
         const float f = l_run > 0.f ? (FL ? 1.f : p.inv_qmax) / l_run : 0.f;
-        uint16_t *o = (uint16_t *)p.O + b * p.osb + hq * p.osh + (int64_t)tq * p.ost + 4 * half;
+        const bool wide_out = ((((uintptr_t)p.O) | (uintptr_t)(p.osb * 2) | (uintptr_t)(p.osh * 2) | (uintptr_t)(p.ost * 2)) & 15) == 0;
+        uint16_t *o = (uint16_t *)p.O + b * p.osb + hq * p.osh + (int64_t)tq * p.ost;
+        // Two quarters at a time: the halves of a column exchange four dims, so that each lane stores eight in a row, in one piece
+        // where the rows are aligned to it (as the queries are loaded).  With 8-byte accesses both ways a block started and ended
+        // slower: unpacked 8 x 118 tokens s192_r6 20.9 -> 18.0 us, 2048 x 2048 87.5 -> 81.6 (kernel and packing, replayed in a
+        // graph), a chunk of 8 x 353 queries on 451 tokens 55.6 -> 49.3.
 #pragma unroll
         for (int db = 0; db < DB; db++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint16_t h[4];
+            for (int i = 0; i < 4; i += 2) {
+                uint32_t w[2][2];
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float v = acc[db][4 * i + j] * f;
-                    h[j] = DT == HQMQ_F16 ? __half_as_ushort(__float2half_rn(v)) : f32_to_bf16_bits(v);
+                for (int k = 0; k < 2; k++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        const float v0 = acc[db][4 * (i + k) + 2 * j] * f, v1 = acc[db][4 * (i + k) + 2 * j + 1] * f;
+                        w[k][j] = DT == HQMQ_F16 ? (uint32_t)__half_as_ushort(__float2half_rn(v0)) | (uint32_t)__half_as_ushort(__float2half_rn(v1)) << 16
+                                                 : (uint32_t)f32_to_bf16_bits(v0) | (uint32_t)f32_to_bf16_bits(v1) << 16;
+                    }
+                const auto x = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false), y = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
+                if (wide_out) *reinterpret_cast<uint4 *>(o + 32 * db + 8 * (i + half)) = uint4{x[0], y[0], x[1], y[1]};
+                else {
+                    *reinterpret_cast<uint2 *>(o + 32 * db + 8 * (i + half)) = uint2{x[0], y[0]};
+                    *reinterpret_cast<uint2 *>(o + 32 * db + 8 * (i + half) + 4) = uint2{x[1], y[1]};
                 }
-                *reinterpret_cast<uint2 *>(o + 32 * db + 8 * i) = uint2{(uint32_t)h[0] | (uint32_t)h[1] << 16, (uint32_t)h[2] | (uint32_t)h[3] << 16};
             }
     } else {
         float *wp = p.ws + ((((size_t)b * p.Hq + hq) * p.Tq + tq) * p.n_splits + sp) * (size_t)(DH + kPartialHead);

@@ -180,3 +180,27 @@ def test_prefill_over_tables_of_any_alignment(dn, S):
     want = attend(joint, 0)
     assert bit_equal(attend(joint[:, 1:], 1), want) and bit_equal(attend(joint[:, 1:].contiguous(), 1), want)
     assert bit_equal(attend(torch.nn.functional.pad(joint, (0, 0, 1, 0))[:, 1:], 0), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d_h", [64, 128])
+@pytest.mark.parametrize("dn", ["float16", "bfloat16"])
+def test_prefill_queries_and_outputs_of_any_alignment(dn, d_h):
+    """Rows of Q and O aligned to 16 bytes and to 8: the same bits."""
+    import hqmq
+    dt = getattr(torch, dn)
+    q = hqmq.HQMQ(n_layers=1, n_heads=2, secondary_size=96, radius_bits=4, device=DEV)
+    g = torch.Generator().manual_seed(d_h)
+    k, v = (torch.randn(2, 2, 150, d_h, generator=g).to(dt).to(DEV) for _ in range(2))
+    cache = q.new_cache(2, 150, d_h, dt, 0)
+    q.append(cache, k, v, 0)
+    Q = torch.randn(2, 6, 90, d_h, generator=g).to(dt).to(DEV)
+    kw = dict(causal=True, causal_offset=60, force_generic=3)
+    for n_splits in (1, 2):
+        want = hqmq.fused_attention_packed(Q, cache, n_splits=n_splits, **kw)
+        odd_q = torch.nn.functional.pad(Q, (4, 0))[..., 4:]
+        out = torch.full((2, 6, 90, d_h + 4), 7.0, dtype=dt, device=DEV)
+        assert odd_q.data_ptr() % 16 == 8 and odd_q.stride(2) * 2 % 16 == 8
+        assert bit_equal(hqmq.fused_attention_packed(odd_q, cache, n_splits=n_splits, **kw), want)
+        hqmq.fused_attention_packed(Q, cache, n_splits=n_splits, out=out[..., :d_h], **kw)
+        assert bit_equal(out[..., :d_h].contiguous(), want) and bool((out[..., d_h:] == 7).all())
