@@ -204,3 +204,31 @@ def test_prefill_queries_and_outputs_of_any_alignment(dn, d_h):
         assert bit_equal(hqmq.fused_attention_packed(odd_q, cache, n_splits=n_splits, **kw), want)
         hqmq.fused_attention_packed(Q, cache, n_splits=n_splits, out=out[..., :d_h], **kw)
         assert bit_equal(out[..., :d_h].contiguous(), want) and bool((out[..., d_h:] == 7).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("generic", [0, 2])
+@pytest.mark.parametrize("dn,d_h,med", [("float16", 64, False), ("bfloat16", 64, True), ("float16", 128, False), ("bfloat16", 128, True)])
+def test_decode_queries_and_outputs_of_any_alignment(dn, d_h, med, generic):
+    """The same of the kernels for few columns: 3 and 15 of them, a part of a second group, one and two splits."""
+    import hqmq
+    dt = getattr(torch, dn)
+    q = hqmq.HQMQ(n_layers=1, n_heads=2, secondary_size=96, radius_bits=4, device=DEV)
+    q = hqmq.with_outlier_extraction(q, C=2.0) if med else q
+    g = torch.Generator().manual_seed(d_h)
+    k, v = (torch.randn(2, 2, 150, d_h, generator=g).to(dt).to(DEV) for _ in range(2))
+    cache = q.new_cache(2, 150, d_h, dt, 0)
+    q.append(cache, k, v, 0)
+    for Tq in (1, 5, 7):
+        Q = torch.randn(2, 6, Tq, d_h, generator=g).to(dt).to(DEV)
+        kw = dict(causal=True, causal_offset=150 - Tq, force_generic=generic)
+        for n_splits in (1, 2):
+            want = hqmq.fused_attention_packed(Q, cache, n_splits=n_splits, **kw)
+            odd_q = torch.nn.functional.pad(Q, (4, 0))[..., 4:]
+            assert odd_q.data_ptr() % 16 == 8
+            assert bit_equal(hqmq.fused_attention_packed(odd_q, cache, n_splits=n_splits, **kw), want)
+            for first in (0, 1, 4):
+                out = torch.full((2, 6, Tq, d_h + 5), 7.0, dtype=dt, device=DEV)
+                hqmq.fused_attention_packed(Q, cache, n_splits=n_splits, out=out[..., first:first + d_h], **kw)
+                assert bit_equal(out[..., first:first + d_h].contiguous(), want)
+                assert bool((out[..., :first] == 7).all()) and bool((out[..., first + d_h:] == 7).all())
