@@ -438,41 +438,49 @@ __device__ __forceinline__ float wave_reduce(float x, Op op) {
     return op(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
-// The same merge for the common decode shape (d_h = 128, at most 32 splits, 16-bit output): one wavefront per row and
-// no LDS.  A lane owns two output elements and loads them from all 32 split records at once (8 bytes each, 512 bytes
+// The same merge for the common decode shapes (d_h 64 or 128, at most 32 splits, 16-bit output): one wavefront per row and
+// no LDS.  A lane owns DH / 64 output elements and loads them from all NS split records at once (256 or 512 bytes
 // per wavefront and record), together with the (m, l) pair of split (lane & 31): one round trip to memory.  The
-// maximum and the denominator are reduced across the lanes, the 32 weights are read back lane by lane into scalar
-// registers and multiply the records in place.
+// maximum and the denominator are reduced across the lanes, the NS weights are read back lane by lane into scalar
+// registers and multiply the records in place.  NS is 4, 8 or 32, the smallest that holds the splits: a batch has many rows of few.
+// us of a whole call before -> now: d_h 64 (which had the kernel above) 1 x 4000 tokens 10.4 -> 8.3, 8 x 3000 bf16 s24_r3 with verbatim
+// chunks 16.7 -> 13.8; d_h 128 with 32 records read whatever the splits, 2 x 71 queries on 3856 tokens 33.6 -> 30.6, 1 x 4096 8.0 -> 7.8.
+template <int DH, int NS>
 __global__ __launch_bounds__(64) void attn_combine_wave_kernel(const float *__restrict__ ws, uint16_t *__restrict__ O, int dtype, int Hq, int Tq,
                                                               int n_splits, int64_t osb, int64_t osh, int64_t ost) {
-    constexpr int d_h = 128, rec = d_h + kPartialHead, NS = 32;
+    constexpr int rec = DH + kPartialHead, E = DH / 64;
+    typedef float floats __attribute__((ext_vector_type(E)));
     const unsigned row = blockIdx.x;
     const int lane = threadIdx.x;
     const float *base = ws + (size_t)row * (size_t)n_splits * rec;
     const int sl = lane & 31;
     float2 ml = *reinterpret_cast<const float2 *>(base + (size_t)min(sl, n_splits - 1) * rec);
-    float2 as[NS];
+    floats as[NS];
 #pragma unroll
-    for (int s = 0; s < NS; s++) as[s] = *reinterpret_cast<const float2 *>(base + (size_t)min(s, n_splits - 1) * rec + kPartialHead + 2 * lane);
+    for (int s = 0; s < NS; s++) as[s] = *reinterpret_cast<const floats *>(base + (size_t)min(s, n_splits - 1) * rec + kPartialHead + E * lane);
     if (sl >= n_splits) ml = float2{-INFINITY, 0.f};
     // reductions over the wavefront inside the vector unit (lane permutations, no LDS round trips): the upper half
     // repeats the lower one, so it takes no part in the sum
     const float M = wave_reduce(ml.x, [](float p, float q) { return fmaxf(p, q); });
     const float w = M > -INFINITY ? __builtin_amdgcn_exp2f(ml.x - M) : 0.f;        // -inf - finite = -inf -> 0
     const float L = wave_reduce(lane < 32 ? ml.y * w : 0.f, [](float p, float q) { return p + q; });
-    float a0 = 0.f, a1 = 0.f;
+    float acc[E] = {};
 #pragma unroll
     for (int s = 0; s < NS; s++) {
         const float wsc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), s));
-        a0 = fmaf(as[s].x, wsc, a0);
-        a1 = fmaf(as[s].y, wsc, a1);
+#pragma unroll
+        for (int e = 0; e < E; e++) acc[e] = fmaf(as[s][e], wsc, acc[e]);
     }
-    const float r0 = L > 0.f ? a0 / L : 0.f, r1 = L > 0.f ? a1 / L : 0.f;
     const unsigned bh = row / (unsigned)Tq, tq = row - bh * (unsigned)Tq, b = bh / (unsigned)Hq, hq = bh - b * (unsigned)Hq;
-    const int64_t o = (int64_t)b * osb + (int64_t)hq * osh + (int64_t)tq * ost + 2 * lane;
-    const uint32_t h0 = dtype == HQMQ_F16 ? __half_as_ushort(__float2half_rn(r0)) : f32_to_bf16_bits(r0);
-    const uint32_t h1 = dtype == HQMQ_F16 ? __half_as_ushort(__float2half_rn(r1)) : f32_to_bf16_bits(r1);
-    *reinterpret_cast<uint32_t *>(O + o) = h0 | h1 << 16;
+    uint16_t *o = O + (int64_t)b * osb + (int64_t)hq * osh + (int64_t)tq * ost + E * lane;
+    uint32_t h[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const float r = L > 0.f ? acc[e] / L : 0.f;
+        h[e] = dtype == HQMQ_F16 ? __half_as_ushort(__float2half_rn(r)) : f32_to_bf16_bits(r);
+    }
+    if constexpr (E == 2) *reinterpret_cast<uint32_t *>(o) = h[0] | h[1] << 16;
+    else *o = (uint16_t)h[0];
 }
 
 static PackedDev to_dev(const hqmq_packed &k) {
@@ -589,9 +597,12 @@ extern "C" int hqmq_attn_combine(const void *workspace, void *O, int dtype, int 
     const int64_t rows = (int64_t)B * H_q * T_q;
     if (rows > 0x7fffffff) return HQMQ_ERR_SHAPE;
     if ((uintptr_t)workspace & 15) return HQMQ_ERR_ALIGN;
-    if (d_h == 128 && n_splits <= 32 && dtype != HQMQ_F32 && ((((uintptr_t)O) | (uintptr_t)(o_sb * 2) | (uintptr_t)(o_sh * 2) | (uintptr_t)(o_st * 2)) & 3) == 0) {
-        hipLaunchKernelGGL(attn_combine_wave_kernel, dim3((unsigned)rows), dim3(64), 0, (hipStream_t)stream, (const float *)workspace,
-                           (uint16_t *)O, dtype, H_q, T_q, n_splits, o_sb, o_sh, o_st);
+    const bool pairs = ((((uintptr_t)O) | (uintptr_t)(o_sb * 2) | (uintptr_t)(o_sh * 2) | (uintptr_t)(o_st * 2)) & 3) == 0;      // of d_h 128, two elements a store
+    if (n_splits <= 32 && dtype != HQMQ_F32 && (d_h == 64 || (d_h == 128 && pairs))) {
+        auto kern = d_h == 64 ? (n_splits <= 4 ? attn_combine_wave_kernel<64, 4> : n_splits <= 8 ? attn_combine_wave_kernel<64, 8> : attn_combine_wave_kernel<64, 32>)
+                              : (n_splits <= 4 ? attn_combine_wave_kernel<128, 4> : n_splits <= 8 ? attn_combine_wave_kernel<128, 8> : attn_combine_wave_kernel<128, 32>);
+        hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(64), 0, (hipStream_t)stream, (const float *)workspace, (uint16_t *)O, dtype, H_q, T_q, n_splits, o_sb,
+                           o_sh, o_st);
         return hip_status(hipGetLastError());
     }
     hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)rows), dim3(kCombineThreads), 0, (hipStream_t)stream,

@@ -91,3 +91,29 @@ def test_column_groups_between_one_and_two_rounds(S, b_r, dn, d_h):
         for ns in (0, 1):
             O = hqmq.fused_attention_packed(Q, cache, T_kv=t, causal=True, causal_offset=t - Tq, n_splits=ns)
             assert_attention_close(O, *refs, base=2e-3, what=f"T={t} n_splits={ns}")
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("dn,d_h", [("fp16", 64), ("bf16", 64), ("fp16", 128), ("bf16", 128), ("fp16", 32), ("fp32", 64)])
+def test_merge_of_any_number_of_splits(dn, d_h):
+    """The merge kernels at the edges of their record counts, with splits that hold no token and outputs of any alignment."""
+    import hqmq
+    dt = {"fp16": torch.float16, "bf16": torch.bfloat16, "fp32": torch.float32}[dn]
+    g = torch.Generator().manual_seed(d_h)
+    k, v = (torch.randn(2, 2, 700, d_h, generator=g).to(dt).cuda() for _ in range(2))
+    q = hqmq.HQMQ(n_layers=1, n_heads=2, secondary_size=96, radius_bits=4, device="cuda")
+    cache = q.new_cache(2, 700, d_h, dt, 0)
+    q.append(cache, k, v, 0)
+    Q = torch.randn(2, 6, 3, d_h, generator=g).to(dt).cuda()
+    lens = torch.tensor([700, 90], dtype=torch.int32)
+    vis = torch.arange(700).view(1, 1, 1, 700) < lens.view(2, 1, 1, 1)
+    refs = masked_two_refs(cache, Q, 700, vis.cuda())
+    for ns in (1, 2, 4, 5, 8, 9, 11, 32, 33, 40):
+        O = hqmq.fused_attention_packed(Q, cache, T_kv=700, kv_lens=lens.cuda(), n_splits=ns)
+        assert_attention_close(O, *refs, base=1e-3 if dn == "fp32" else 2e-3, what=f"n_splits={ns}")
+        for first in (1, 2):
+            out = torch.full((2, 6, 3, d_h + 3), 7.0, dtype=dt, device="cuda")
+            hqmq.fused_attention_packed(Q, cache, T_kv=700, kv_lens=lens.cuda(), n_splits=ns, out=out[..., first:first + d_h])
+            assert_attention_close(out[..., first:first + d_h], *refs, base=1e-3 if dn == "fp32" else 2e-3, what=f"n_splits={ns} at {first}")
+            assert bool((out[..., :first] == 7).all()) and bool((out[..., first + d_h:] == 7).all())
