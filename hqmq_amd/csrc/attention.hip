@@ -18,6 +18,7 @@
 //   * KV is walked in super-tiles of 64 tokens; each lane reads its codes with one aligned
 //     vector load per 16-token tile, a wavefront covering whole 128-byte lines of the plane;
 //   * split-KV partials (m, l, acc) go to a workspace and are merged by a second kernel.
+#include <algorithm>
 #include "attention_common.h"
 #include <mutex>
 
@@ -545,10 +546,10 @@ extern "C" int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, i
 // s96_r4 fp16, 32 / 8 heads of 128, 1 x 300 tokens 10.7 -> 7.0 (one block, no merge), 3 x 20000 30.2 -> 20.0, 10 x 6000 28.4 -> 20.6,
 // 20 x 600 14.9 -> 8.5; s24_r3 bf16 with verbatim chunks, 10 x 6000 47.4 -> 34.2.
 // `pairs` (or 0): the blocks where two column groups share one, which the specialised kernels do beyond a round, at 1.28 times the time.
-static int decode_splits(int64_t base, int64_t pairs, int64_t rows, int T_kv, bool ragged, double unit, double merge) {
+static int decode_splits(int64_t base, int64_t pairs, int64_t rows, int64_t limit, int T_kv, bool ragged, double unit, double merge) {
     if (base < 1) return 1;
     int64_t top = ((int64_t)T_kv + 2 * kSuper - 1) / (2 * kSuper);       // blocks of at least 128 tokens (4k tokens: 32 splits, 8.7 against 8.95 us)
-    if (top > 512) top = 512;
+    if (top > limit) top = limit;
     // past four rounds the last one weighs little (832 blocks of 9000 tokens 104 us, halved 128), and lengths of their own even out from
     // two and a half on (512 of up to 16384 tokens 242 us, halved 248)
     const int64_t most = (ragged ? 640 : 1024) / base;
@@ -574,8 +575,7 @@ extern "C" int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv
     if (B < 1 || H_q < 1 || H_kv < 1 || T_q < 1 || T_kv < 1) return 1;
     const int G = H_q / H_kv;
     const int64_t base = (int64_t)B * H_kv * (((int64_t)T_q * G + 15) / 16), target = ragged ? 512 : 256;
-    const int s = decode_splits(base, 0, (int64_t)B * H_q * T_q, T_kv, ragged != 0, 1.0, 500.0);
-    return s > 1 && s > (target + base - 1) / base ? (int)((target + base - 1) / base) : s;
+    return base < 1 ? 1 : decode_splits(base, 0, (int64_t)B * H_q * T_q, std::min<int64_t>(512, (target + base - 1) / base), T_kv, ragged != 0, 1.0, 500.0);
 }
 
 extern "C" int hqmq_attn_splits(const hqmq_attn_args *a) {
@@ -585,7 +585,7 @@ extern "C" int hqmq_attn_splits(const hqmq_attn_args *a) {
     const bool generic = a->dtype == HQMQ_F32 || attn_wide(a) || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
     const int64_t nz = (int64_t)a->B * a->H_kv, groups = ((int64_t)a->T_q * (a->H_q / a->H_kv) + 15) / 16;
     return decode_splits(nz * groups, generic || a->K.flag_plane || groups < 2 ? 0 : nz * ((groups + 1) / 2),
-                         (int64_t)a->B * a->H_q * a->T_q, a->T_kv, a->kv_len != nullptr,
+                         (int64_t)a->B * a->H_q * a->T_q, 512, a->T_kv, a->kv_len != nullptr,
                          a->n_chunks / 32.0, generic ? 100.0 : a->K.flag_plane ? 250.0 : a->aux_bits ? 350.0 : 500.0);
 }
 
