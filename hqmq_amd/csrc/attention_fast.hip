@@ -936,11 +936,8 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
                     pe[e] = __builtin_amdgcn_exp2f(fmaf(sT[cgi][u][e], c, mc));
                     l_run[cgi] += pe[e];
                 }
-                const half2v u01 = half2v{(_Float16)pe[0], (_Float16)pe[1]}, u23 = half2v{(_Float16)pe[2], (_Float16)pe[3]};
-                const half2v p01 = u01 * scale_h2<DT>(h.vs[u].x);
-                const half2v p23 = u23 * scale_h2<DT>(h.vs[u].y);
-                pT[u] = half4{p01[0], p01[1], p23[0], p23[1]};
-                if (FLAGS) pTo[u] = half4{u01[0], u01[1], u23[0], u23[1]};      // unscaled: the selector rows hold qmax
+                pT[u] = weigh<DT>(pe, h.vs[u]);
+                if (FLAGS) pTo[u] = half4{(_Float16)pe[0], (_Float16)pe[1], (_Float16)pe[2], (_Float16)pe[3]};      // unscaled: the selector rows hold qmax
             }
             pp[cgi] = cat8(pT[0], pT[1]);
         }
@@ -1386,9 +1383,7 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
                 pe[e] = __builtin_amdgcn_exp2f(fmaf(sT[u][e], c, mc));
                 l_run += pe[e];
             }
-            const half2v p01 = half2v{(_Float16)pe[0], (_Float16)pe[1]} * scale_h2<DT>(vs[u].x);
-            const half2v p23 = half2v{(_Float16)pe[2], (_Float16)pe[3]} * scale_h2<DT>(vs[u].y);
-            pT[u] = half4{p01[0], p01[1], p23[0], p23[1]};
+            pT[u] = weigh<DT>(pe, vs[u]);
         }
         const half8 pp = cat8(pT[0], pT[1]);
         if (left == 2) __builtin_amdgcn_s_setprio(2);

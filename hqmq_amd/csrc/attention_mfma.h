@@ -38,20 +38,20 @@ __device__ __forceinline__ int32_t uniform_word(const int32_t *a, int64_t i) {
     return ((const_i32_ptr)(uintptr_t)a)[i];
 }
 
-// two 16-bit scales (raw bits of dtype DT) as a packed fp16 pair
-template <int DT>
-__device__ __forceinline__ half2v scale_h2(uint32_t pair) {
-    if (DT == HQMQ_F16) return __builtin_bit_cast(half2v, pair);
-    half2v r;
-    r[0] = (_Float16)__uint_as_float(pair << 16);
-    r[1] = (_Float16)__uint_as_float(pair & 0xffff0000u);
-    return r;
-}
 // acc * scale[hi] (+ add): for fp16 scales one mixed-precision fma reads the half directly
 template <int DT>
 __device__ __forceinline__ float scaled(float acc, uint32_t pair, int hi, float add) {
     if (DT == HQMQ_F16) return __builtin_fmaf(acc, (float)__builtin_bit_cast(half2v, pair)[hi], add);
     return __builtin_fmaf(acc, __uint_as_float(hi ? (pair & 0xffff0000u) : (pair << 16)), add);
+}
+// Four weights times the scales of their tokens, each product rounded to fp16 once: for fp16 scales one mixed-precision fma a weight,
+// no more than the conversions and packed products that rounded the weight first and the product again.
+template <int DT>
+__device__ __forceinline__ half4 weigh(const float (&w)[4], uint2 scales) {
+    half4 r;
+#pragma unroll
+    for (int e = 0; e < 4; e++) r[e] = (_Float16)scaled<DT>(w[e], e < 2 ? scales.x : scales.y, e & 1, 0.f);
+    return r;
 }
 
 typedef const uint4v __attribute__((address_space(3))) *lds_u4_ptr;
