@@ -125,7 +125,7 @@ constexpr int kPsTabBytes = 8 * 1024 * 8;   // 64 KB per tensor
 constexpr bool is_prescaled(int MB, int AB, int IB) { return MB == 12 && AB == 1 && IB == 10; }
 constexpr int vtab_offset(bool ps) { return ps ? kPsTabBytes : kVTabOffset; }
 constexpr int q_offset(bool ps) { return ps ? 2 * kPsTabBytes : kQOffset; }
-constexpr int sel_offset(bool ps) { return q_offset(ps) + 4096; }      // nine rows of eight fp16: row r < 8 = qmax times unit vector r, row 8 = 0
+constexpr int sel_offset(bool ps) { return q_offset(ps) + 4096; }      // nine rows of eight fp16: row r < 8 = unit vector r, row 8 = 0
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 template <int TAB_OFF>
@@ -671,9 +671,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     }
     if (FLAGS && threadIdx.x >= 64 && threadIdx.x < 100) {
         const uint32_t w = threadIdx.x - 64, row = w >> 2, d = w & 3;
-        // the selector rows carry qmax instead of 1: the gathered probabilities come out scaled for the verbatim
-        // chunks (whose 1 / qmax is applied with everything else in the epilogue) at no cost
-        const uint32_t one = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)p.qmax);
+        const uint32_t one = 0x3c00u;       // 1 in fp16
         reinterpret_cast<uint32_t *>(lds_tab)[SELOFF / 4 + w] = (row < 8 && (row >> 1) == d) ? one << (16 * (row & 1)) : 0u;
     }
     half8 qf[NCG][CPL / 2];
@@ -783,8 +781,9 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     };
     // V side, also from the entry list, sixteen entries of the half-step per batch (lane 16 * grp + col holds
     // entry `col`):
-    //   Pg[e][column] = qmax P[token(e)][column] one 16x16x32 MFMA: A = qmax times the unit vector of the entry's token
-    //                                            slot (LDS rows), B = the unscaled probabilities of the 32 tokens;
+    //   Pg[e][column] = qmax P[token(e)][column] one 16x16x32 MFMA: A = the unit vector of the entry's token slot (LDS
+    //                                            rows), B = qmax P of the 32 tokens (verbatim chunks go through the
+    //                                            epilogue's 1 / qmax like the others), already in fp16: exact;
     //   for every chunk position j in use:       X_j^T by the transposing MFMA (A = the entry's chunk in the row
     //   acc[j] += X_j^T . Pg                     group that owns it, else zero), then one 16x16x16 MFMA over entries.
     // the selector row of the lane's entry (A operand of the MFMA that gathers the probabilities), read ahead of use
@@ -937,7 +936,10 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
                     l_run[cgi] += pe[e];
                 }
                 pT[u] = weigh<DT>(pe, h.vs[u]);
-                if (FLAGS) pTo[u] = half4{(_Float16)pe[0], (_Float16)pe[1], (_Float16)pe[2], (_Float16)pe[3]};      // unscaled: the selector rows hold qmax
+                if constexpr (FLAGS) {          // for the verbatim chunks, see v_batch; qmax P is rounded to fp16 here and nowhere else
+#pragma unroll
+                    for (int e = 0; e < 4; e++) pTo[u][e] = (_Float16)(pe[e] * qmaxf);
+                }
             }
             pp[cgi] = cat8(pT[0], pT[1]);
         }

@@ -17,7 +17,7 @@ def merged(O, partials, n_splits):
     return (r[..., 4:] * w).sum(3) / (r[..., 1:2] * w).sum(3)
 
 
-@pytest.mark.parametrize("med", [False])
+@pytest.mark.parametrize("med", [False, True])
 @pytest.mark.parametrize("dn", ["fp16", "bf16"])
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("S,b_r", [(96, 4), (24, 3), (192, 6), (192, 4)])
