@@ -545,8 +545,8 @@ extern "C" int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, i
 // at the first three.  us before -> now:
 // s96_r4 fp16, 32 / 8 heads of 128, 1 x 300 tokens 10.7 -> 7.0 (one block, no merge), 3 x 20000 30.2 -> 20.0, 10 x 6000 28.4 -> 20.6,
 // 20 x 600 14.9 -> 8.5; s24_r3 bf16 with verbatim chunks, 10 x 6000 47.4 -> 34.2.
-// `pairs` (or 0): the blocks where two column groups share one, which the specialised kernels do beyond a round, at 1.28 times the time.
-static int decode_splits(int64_t base, int64_t pairs, int64_t rows, int64_t limit, int T_kv, bool ragged, double unit, double merge) {
+// `a` (or null): a call of the specialised kernels, whose blocks may hold two column groups each (attn_two_groups), at 1.28 times the time.
+static int decode_splits(int64_t base, const hqmq_attn_args *a, int64_t rows, int64_t limit, int T_kv, bool ragged, double unit, double merge) {
     if (base < 1) return 1;
     int64_t top = ((int64_t)T_kv + 2 * kSuper - 1) / (2 * kSuper);       // blocks of at least 128 tokens (4k tokens: 32 splits, 8.7 against 8.95 us)
     if (top > limit) top = limit;
@@ -555,10 +555,12 @@ static int decode_splits(int64_t base, int64_t pairs, int64_t rows, int64_t limi
     const int64_t most = (ragged ? 640 : 1024) / base;
     if (top > most) top = most;
     const uint32_t tiles = (uint32_t)(((int64_t)T_kv + kSuper - 1) / kSuper);
+    const int n_cg = a ? (int)(base / ((int64_t)a->B * a->H_kv)) : 1;
+    const int64_t pairs = a ? (int64_t)a->B * a->H_kv * ((n_cg + 1) / 2) : 0;
     double least = 0.0;
     int best = 1;
     for (int64_t s = 1; s <= top || s == 1; s++) {
-        const bool two = pairs > 0 && base * s > 256;
+        const bool two = a && attn_two_groups(n_cg, a->K.flag_plane != nullptr, base * s, T_kv / (int)s, a->n_chunks, a->aux_bits);
         const int64_t blocks = two ? pairs * s : base * s;
         double rounds = ragged ? 0.8 / 256 * (double)blocks + 0.3 : (double)((blocks + 255) / 256);
         if (rounds < 1.0) rounds = 1.0;
@@ -575,18 +577,20 @@ extern "C" int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv
     if (B < 1 || H_q < 1 || H_kv < 1 || T_q < 1 || T_kv < 1) return 1;
     const int G = H_q / H_kv;
     const int64_t base = (int64_t)B * H_kv * (((int64_t)T_q * G + 15) / 16), target = ragged ? 512 : 256;
-    return base < 1 ? 1 : decode_splits(base, 0, (int64_t)B * H_q * T_q, std::min<int64_t>(512, (target + base - 1) / base), T_kv, ragged != 0, 1.0, 500.0);
+    return base < 1 ? 1 : decode_splits(base, nullptr, (int64_t)B * H_q * T_q, std::min<int64_t>(512, (target + base - 1) / base), T_kv, ragged != 0, 1.0, 500.0);
+}
+
+int hqmq::attn_decode_splits(const hqmq_attn_args *a) {
+    const bool generic = a->dtype == HQMQ_F32 || attn_wide(a) || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
+    const int64_t groups = ((int64_t)a->T_q * (a->H_q / a->H_kv) + 15) / 16;
+    return decode_splits((int64_t)a->B * a->H_kv * groups, generic ? nullptr : a, (int64_t)a->B * a->H_q * a->T_q, 512, a->T_kv,
+                         a->kv_len != nullptr, a->n_chunks / 32.0, generic ? 100.0 : a->K.flag_plane ? 250.0 : a->aux_bits ? 350.0 : 500.0);
 }
 
 extern "C" int hqmq_attn_splits(const hqmq_attn_args *a) {
     if (!a || a->B < 1 || a->H_kv < 1 || a->H_q < 1 || a->T_q < 1 || a->T_kv < 1) return 1;
     const int splits = attn_prefill_splits(a, 0);
-    if (splits > 0) return splits;
-    const bool generic = a->dtype == HQMQ_F32 || attn_wide(a) || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
-    const int64_t nz = (int64_t)a->B * a->H_kv, groups = ((int64_t)a->T_q * (a->H_q / a->H_kv) + 15) / 16;
-    return decode_splits(nz * groups, generic || a->K.flag_plane || groups < 2 ? 0 : nz * ((groups + 1) / 2),
-                         (int64_t)a->B * a->H_q * a->T_q, 512, a->T_kv, a->kv_len != nullptr,
-                         a->n_chunks / 32.0, generic ? 100.0 : a->K.flag_plane ? 250.0 : a->aux_bits ? 350.0 : 500.0);
+    return splits > 0 ? splits : attn_decode_splits(a);
 }
 
 extern "C" int hqmq_attn_combine(const void *workspace, void *O, int dtype, int B, int H_q, int T_q, int d_h, int n_splits,

@@ -241,6 +241,18 @@ inline void launch_timed(Kern kern, dim3 grid, dim3 block, size_t shmem, hipStre
 
 // Implemented in attention_prefill.hip: many query columns per KV head over plain 16-bit and fp16 outlier caches.
 int attn_prefill_splits(const hqmq_attn_args *a, int splits);
+// Implemented in attention.hip: the number of splits with which the other kernels take a call that leaves it open.
+int attn_decode_splits(const hqmq_attn_args *a);
+
+// Chunked prefill (more than 16 columns per KV head) of plain caches in the specialised decode kernels: two column groups per wavefront
+// wherever one group per block would start a second round of 256 blocks.  A tile then takes 1.28 times as long for twice the columns:
+// 600 / 2500 tokens, 280 blocks of one group, d_h 128 fp16 s96_r4 17.5 -> 16.2 / 40.7 -> 30.5 us, bf16 s192_r4 24.5 -> 18.3 / 50.5 ->
+// 36.0; d_h 64, 320 blocks, 12.5 -> 11.3 / 24.0 -> 21.0.  In a single round one group is faster (5 % to 30 %), and so are two rounds
+// of the kernel whose loads land in LDS (d_h 128, codes of 16 bits) over less than 256 tokens (130 tokens 11.6 against 12.2 us).
+// `blocks`: of one group each; `range`: tokens per block.
+inline bool attn_two_groups(int n_cg, bool flags, int64_t blocks, int range, int n_chunks, int aux_bits) {
+    return !flags && n_cg > 1 && blocks > 256 && (blocks >= 512 || range >= 256 || n_chunks == 16 || aux_bits);
+}
 int launch_attn_prefill(const AttnParams &p, int main_bits, bool flags, hipStream_t st, const LaunchTiming &tm);
 int launch_attn_fast(const AttnParams &p, int main_bits, bool flags, dim3 grid, size_t table_bytes, hipStream_t st,
                      const LaunchTiming &tm, bool *handled);

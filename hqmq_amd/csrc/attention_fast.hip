@@ -1492,13 +1492,7 @@ static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hip
     // compute unit holds two blocks of eight (480 blocks of 4000 tokens 33.3 against 38.2 us).
     const int range = p.Tkv / p.n_splits;
     const bool wide = CPL == 8 ? !flags && range >= 4096 : flags ? range >= 1536 : range >= 4096 && (int64_t)grid.x * grid.y * grid.z <= 256;
-    // Chunked prefill (more than 16 columns per KV head) of plain caches: two column groups per wavefront wherever one group per block
-    // would start a second round of 256 blocks.  A tile then takes 1.28 times as long for twice the columns: 600 / 2500 tokens, 280
-    // blocks of one group, d_h 128 fp16 s96_r4 17.5 -> 16.2 / 40.7 -> 30.5 us, bf16 s192_r4 24.5 -> 18.3 / 50.5 -> 36.0; d_h 64, 320 blocks,
-    // 12.5 -> 11.3 / 24.0 -> 21.0.  In a single round one group is faster (5 % to 30 %), and so are two rounds of the kernel whose loads
-    // land in LDS over less than 256 tokens (130 tokens 11.6 against 12.2 us).
-    const int64_t groups = (int64_t)p.n_splits * p.n_cg * p.B * p.Hkv;
-    const bool two = !flags && p.n_cg > 1 && groups > 256 && (groups >= 512 || range >= 256 || CPL == 4 || p.aux_bits);
+    const bool two = attn_two_groups(p.n_cg, flags, (int64_t)p.n_splits * p.n_cg * p.B * p.Hkv, range, p.n, p.aux_bits);
     // tables of e4m3 numbers kept as float8 in LDS, on request (decode shapes of the 16-bit layouts at d_h 128)
     if (p.tab_fp8 && CPL == 8 && !two) {
         if (mb == 16 && p.aux_bits == 0 && p.idx_bits == 12) return launch_one<8, 16, 0, 12, DT, kFastWaves, 1, true>(p, flags, grid, st, tm);

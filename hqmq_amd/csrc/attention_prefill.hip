@@ -668,26 +668,31 @@ static bool attn_prefill_takes(const hqmq_attn_args *a) {
     if ((((uintptr_t)a->O) | (uintptr_t)(a->o_sb * 2) | (uintptr_t)(a->o_sh * 2) | (uintptr_t)(a->o_st * 2)) & 7) return false;
     return true;
 }
-// The same for the kernels of attention_fast.hip: blocks of 16 columns (0.47 us a tile) or, where those are more than the
-// compute units, of 32 (0.6 us), over outlier caches always of 16 (0.7 us), which start and finish in 6 us.
-static double fast_us(int64_t cols, int64_t nz, int Tkv, int d_h, int splits, bool flags) {
-    const int64_t cg = (cols + 15) / 16, pairs = (cg + 1) / 2 * nz * splits;
-    const bool two = !flags && cg > 1 && cg * nz * splits > 256;
-    const double tiles = ((double)Tkv * d_h + 8191) / 8192;
+// The same for the kernels of attention_fast.hip: blocks of 16 columns (0.47 us a tile) or of 32 (attn_two_groups, 0.6 us), over
+// outlier caches always of 16 (0.7 us), which start and finish in 6 us.
+static double fast_us(const hqmq_attn_args *a, int64_t cols, int splits) {
+    const int64_t nz = (int64_t)a->B * a->H_kv, cg = (cols + 15) / 16, pairs = (cg + 1) / 2 * nz * splits;
+    const int d_h = 4 * a->n_chunks;
+    const bool flags = a->K.flag_plane != nullptr, two = attn_two_groups((int)cg, flags, cg * nz * splits, a->T_kv / splits, a->n_chunks, a->aux_bits);
+    const double tiles = ((double)a->T_kv * d_h + 8191) / 8192;
     return 3.0 + (double)(((two ? pairs : cg * nz * splits) + 255) / 256) * (6.0 + tiles / splits * (two ? 0.6 : flags ? 0.7 : 0.47)) +
            (splits > 1 ? 3.0 + (double)(cols * nz) * splits * (d_h + 4) * 8 / 2e6 : 0.0);
 }
-// The number of splits of a call that leaves it open, 0 if it is better off with the other kernels (by a clear margin: the
-// estimates are good to some 15 %); splits > 0: the same decision for a given number.
+// The number of splits of a call that leaves it open, 0 if it is better off with the other kernels; splits > 0: the same decision for
+// a given number.  Both estimates are of the plan that would run, the other kernels' with the splits of attn_decode_splits; nine of ten
+// calls take 0.77 to 1.17 of them, mostly both kernels alike.  Over 430 prefill chunks of 64 to 900 columns and 200 to 32768 tokens, plain
+// and outlier caches, the choice takes 0.4 % longer than the faster of the two kernels (28 % at worst).  With the other kernels judged by
+// hqmq_attn_pick_splits, which knows no pairs of column groups, and a margin of 15 % for that, it took 1.5 % (35 %).  us, and with the
+// kernel chosen before: 1 x 33 queries on 19403 tokens, 32 / 8 heads of 128, s24_r3, 37.8 (prefill kernel 47.2); 3 x 70 on 5811,
+// 28 / 4, s192_r4, 50.8 (decode kernels 62.9).
 int attn_prefill_splits(const hqmq_attn_args *a, int splits) {
     const int64_t cols = (int64_t)a->T_q * (a->H_q / a->H_kv), nz = (int64_t)a->B * a->H_kv;
     if (cols < 64 || !attn_prefill_takes(a)) return 0;
     const PfPlan plan = pf_plan(cols, nz, a->T_q, a->T_kv, 4 * a->n_chunks, a->causal, a->causal_offset, splits, a->K.flag_plane != nullptr);
-    const int other = splits > 0 ? splits : hqmq_attn_pick_splits(a->B, a->H_q, a->H_kv, a->T_q, a->T_kv, a->kv_len != nullptr);
     // Outlier caches of three radius bits keep the decode kernels: most radius codes are 1, 2 or 4, with which those kernels' V is
     // exact, and V rounded as a value left lognormal channels 0.5 % further from 64-bit results (s24_r3; 6 % nearer on average).
     if (a->K.flag_plane && a->qmax < 15 && a->force_generic != 3) return 0;
-    return a->force_generic == 3 || plan.us < 0.85 * fast_us(cols, nz, a->T_kv, 4 * a->n_chunks, other, a->K.flag_plane != nullptr) ? plan.splits : 0;
+    return a->force_generic == 3 || plan.us < 0.95 * fast_us(a, cols, splits > 0 ? splits : attn_decode_splits(a)) ? plan.splits : 0;
 }
 
 template <int DH, int MB, bool AUX, int DT, bool FL>

@@ -39,6 +39,26 @@ def test_splits_keep_to_rounds_of_blocks_and_to_earlier_workspaces():
     assert lib.hqmq_attn_pick_splits(12, 32, 8, 1, 4096, 0) == 2                        # 192 blocks, not 288
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,d_h,T,Tq,S,b_r,dn,splits", [
+    # us measured with the decode kernels and with the prefill kernel; the two would run with different numbers of splits
+    (1, 32, 8, 128, 19403, 33, 24, 3, "fp16", 6),       # 37.8, 47.2 with 16
+    (1, 32, 8, 128, 21640, 43, 24, 3, "fp16", 5),       # 45.3, 52.1 with 16
+    (1, 32, 8, 128, 9170, 127, 24, 3, "bf16", 2),       # 46.6, 51.2 with 8
+    (10, 64, 8, 64, 2717, 16, 192, 4, "bf16", 3),       # 46.5 with 1, 34.4
+    (2, 64, 8, 64, 2070, 76, 24, 3, "fp16", 3),         # 36.7 with 1, 29.4
+    (3, 28, 4, 128, 5811, 70, 192, 4, "bf16", 5),       # 62.9 with 1, 50.8
+    (7, 28, 4, 128, 2990, 73, 192, 6, "fp16", 2)])      # 70.9 with 1, 60.5
+def test_prefill_chunks_take_the_faster_kernel(B, Hq, Hkv, d_h, T, Tq, S, b_r, dn, splits):
+    from hqmq_amd import _lib as L
+    a = _args(B, Hq, Hkv, Tq, T, d_h // 4, False, L.DT_CODE[{"fp16": torch.float16, "bf16": torch.bfloat16}[dn]])
+    a.idx_bits, a.main_bits, a.aux_bits = L.layout_bits(S, b_r)
+    a.K.K = a.V.K = 24 * S
+    a.t_cap, a.qmax, a.softmax_scale, a.causal, a.causal_offset = (T + 63) // 64 * 64, (1 << b_r) - 1, d_h ** -0.5, 1, T - Tq
+    assert L.lib().hqmq_attn_splits(C.addressof(a)) == splits
+    a.force_generic = 2           # never the prefill kernel
+    assert (L.lib().hqmq_attn_splits(C.addressof(a)) == splits) == (S == 24 and T > 9000)
+
+
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
 @pytest.mark.parametrize("S,b_r,dn,d_h,med,B,contexts", [
