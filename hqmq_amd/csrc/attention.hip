@@ -538,32 +538,39 @@ extern "C" int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, i
 // and query, is worth 500 of them; `merge`, the second launch and the blocks' way through memory, 500 over plain caches, 350 where
 // the radii have a plane of their own, 250 over outlier caches and 100 in the generic kernels, whose tokens cost more; it doubles with
 // 5000 partial rows, and a split more is worth 2.
-// Sequences of different lengths, started longest first, even out: a round counts by its share, 0.8 of the blocks (mean over the
-// longest) and 0.3 for the last ones.  Measured against the best of 8 to 14 counts at 120 shapes with equal lengths, 101 with lengths
-// of their own (6 cache layouts, 4 to 400 heads, 600 to 20000 tokens), 230 of 1 to 7 queries replayed in graphs and 65 prefill chunks,
-// the choice takes 0.6, 2.7, 0.9 and 2.1 % longer; 256 blocks rounded up (512 over such lengths), the rule before, took 25, 32 and 23 %
-// at the first three.  us before -> now:
-// s96_r4 fp16, 32 / 8 heads of 128, 1 x 300 tokens 10.7 -> 7.0 (one block, no merge), 3 x 20000 30.2 -> 20.0, 10 x 6000 28.4 -> 20.6,
-// 20 x 600 14.9 -> 8.5; s24_r3 bf16 with verbatim chunks, 10 x 6000 47.4 -> 34.2.
+// Sequences of different lengths, started longest first, even out: a round counts by its share, 0.75 of the blocks (0.53 of the longest
+// each if lengths are uniform, up to all of it) and 0.3 for the last ones, or 0.6 and 0.5 where two blocks share a compute unit.  The parts
+// of few sequences even out less: a second round they have begun counts 0.4 (3 x 20000 tokens, 240 blocks 21.9 us, 264 30.3, 384 25.6).
+// The choice against the best of 6 to 14 counts: 150 shapes with equal lengths (6 cache layouts, 8 to 400 sequences x heads, 600 to 20000
+// tokens) 0.8 % longer, 159 of 1 to 7 queries 1.2 %, 126 with lengths of their own 2.4 % and 979 of 16 to 900 sequences x heads, lengths equal,
+// uniform, exponential or the upper half of a uniform distribution, 2.1 %.  256 blocks rounded up (512 over such lengths) took 25, 23 and 32 % at
+// shapes like the first three.  us then -> now: s96_r4 fp16, 32 / 8 heads of 128, 1 x 300 tokens 10.7 -> 7.0 (one block, no merge), 3 x 20000
+// 30.2 -> 20.0, 10 x 6000 28.4 -> 20.6, 20 x 600 14.9 -> 8.5; s24_r3 bf16 with verbatim chunks, 10 x 6000 47.4 -> 34.2.
 // `a` (or null): a call of the specialised kernels, whose blocks may hold two column groups each (attn_two_groups), at 1.28 times the time.
 static int decode_splits(int64_t base, const hqmq_attn_args *a, int64_t rows, int64_t limit, int T_kv, bool ragged, double unit, double merge) {
     if (base < 1) return 1;
     int64_t top = ((int64_t)T_kv + 2 * kSuper - 1) / (2 * kSuper);       // blocks of at least 128 tokens (4k tokens: 32 splits, 8.7 against 8.95 us)
     if (top > limit) top = limit;
-    // past four rounds the last one weighs little (832 blocks of 9000 tokens 104 us, halved 128), and lengths of their own even out from
-    // two and a half on (512 of up to 16384 tokens 242 us, halved 248)
-    const int64_t most = (ragged ? 640 : 1024) / base;
-    if (top > most) top = most;
-    const uint32_t tiles = (uint32_t)(((int64_t)T_kv + kSuper - 1) / kSuper);
     const int n_cg = a ? (int)(base / ((int64_t)a->B * a->H_kv)) : 1;
     const int64_t pairs = a ? (int64_t)a->B * a->H_kv * ((n_cg + 1) / 2) : 0;
+    // d_h 64 over plain caches, tables not multiplied out: two blocks share a compute unit
+    const bool shared = a && a->n_chunks == 16 && !a->K.flag_plane && !(a->main_bits == 12 && a->aux_bits == 1 && a->idx_bits == 10);
+    // Past four rounds the last one weighs little (832 blocks of 9000 tokens 104 us, halved 128).  Lengths of their own even out earlier:
+    // up to 640 blocks, or halves of up to 500 sequences x heads.  Halves against whole sequences of up to 16384 tokens, mean over six
+    // layouts: 328 sequences x heads 0.77 of the time with uniform or exponential lengths, 0.88 with equal ones or the upper half of a
+    // uniform distribution; 400 0.97 and 1.06, 512 1.00 and 1.06, 640 1.08 and 0.95, 900 1.10 and 1.01.  Where two blocks share a compute unit the
+    // longest bounds the call for longer, so up to 1024 as with equal lengths: 328 0.69 and 0.83, 512 0.84 and 1.06, 640 0.94 and 0.96.
+    const int64_t most = !ragged || shared ? 1024 / base : std::max<int64_t>(640 / base, base <= 500 ? 2 : 1);
+    if (top > most) top = most;
+    const uint32_t tiles = (uint32_t)(((int64_t)T_kv + kSuper - 1) / kSuper);
     double least = 0.0;
     int best = 1;
     for (int64_t s = 1; s <= top || s == 1; s++) {
         const bool two = a && attn_two_groups(n_cg, a->K.flag_plane != nullptr, base * s, T_kv / (int)s, a->n_chunks, a->aux_bits);
         const int64_t blocks = two ? pairs * s : base * s;
-        double rounds = ragged ? 0.8 / 256 * (double)blocks + 0.3 : (double)((blocks + 255) / 256);
+        double rounds = ragged ? (shared ? 0.6 : 0.75) / 256 * (double)blocks + (shared ? 0.5 : 0.3) : (double)((blocks + 255) / 256);
         if (rounds < 1.0) rounds = 1.0;
+        if (ragged && base < 256 && blocks > 256 && rounds < 1.4) rounds = 1.4;
         const double t = rounds * (500.0 + (two ? 1.28 * unit : unit) * (double)((tiles + (uint32_t)s - 1) / (uint32_t)s * kSuper)) +
                          (s > 1 ? merge * (1.0 + 2e-4 * (double)rows * (double)s) + 2.0 * (double)s : 0.0);
         if (s == 1 || t < least) { least = t; best = (int)s; }

@@ -39,6 +39,18 @@ def test_splits_keep_to_rounds_of_blocks_and_to_earlier_workspaces():
     assert lib.hqmq_attn_pick_splits(12, 32, 8, 1, 4096, 0) == 2                        # 192 blocks, not 288
 
 
+def test_ragged_batches_beyond_one_round():
+    from hqmq_amd import _lib as L
+    f16 = L.DT_CODE[torch.float16]
+    for n, flags, counts in ((32, False, {41: 2, 48: 2, 56: 2, 62: 2, 63: 1, 64: 1, 80: 1}), (32, True, {41: 2, 48: 2, 56: 2, 62: 2, 63: 1, 64: 1}),
+                             (16, True, {41: 2, 62: 2, 64: 1}), (16, False, {41: 3, 48: 2, 64: 2, 65: 1})):
+        for B, splits in counts.items():      # 328 to 1024 pairs of up to 16384 tokens; whole sequences of few tokens
+            a = _args(B, 32, 8, 1, 16384, n, flags, f16, True)
+            assert L.lib().hqmq_attn_splits(C.addressof(a)) == splits, (n, flags, B)
+            a.T_kv = a.t_cap = 1024
+            assert L.lib().hqmq_attn_splits(C.addressof(a)) == 1, (n, flags, B)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,d_h,T,Tq,S,b_r,dn,splits", [
     # us measured with the decode kernels and with the prefill kernel; the two would run with different numbers of splits
     (1, 32, 8, 128, 19403, 33, 24, 3, "fp16", 6),       # 37.8, 47.2 with 16
