@@ -588,7 +588,7 @@ extern "C" int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv
 }
 
 int hqmq::attn_decode_splits(const hqmq_attn_args *a) {
-    const bool generic = a->dtype == HQMQ_F32 || attn_wide(a) || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
+    const bool generic = a->dtype == HQMQ_F32 || a->wide_range || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
     const int64_t groups = ((int64_t)a->T_q * (a->H_q / a->H_kv) + 15) / 16;
     return decode_splits((int64_t)a->B * a->H_kv * groups, generic ? nullptr : a, (int64_t)a->B * a->H_q * a->T_q, 512, a->T_kv,
                          a->kv_len != nullptr, a->n_chunks / 32.0, generic ? 100.0 : a->K.flag_plane ? 250.0 : a->aux_bits ? 350.0 : 500.0);
@@ -621,7 +621,8 @@ extern "C" int hqmq_attn_combine(const void *workspace, void *O, int dtype, int 
     return hip_status(hipGetLastError());
 }
 
-static int attn_fwd_impl(const hqmq_attn_args *a, void *stream) {
+// `guarded`: the specialised kernels run on trust, attn_again_kernel behind them does the call again if the largest V scale asks for it
+static int attn_fwd_impl(const hqmq_attn_args *a, void *stream, bool guarded = false) {
     if (!a || !a->Q || !a->O) return HQMQ_ERR_NULL;
     const hqmq_packed *pk[2] = {&a->K, &a->V};
     for (const hqmq_packed *k : pk) {
@@ -681,7 +682,7 @@ static int attn_fwd_impl(const hqmq_attn_args *a, void *stream) {
     // Ragged batches keep the sequence-major order that batch_order relies on.
     p.xcd_remap = (!a->kv_len && !a->batch_order && ((a->B * a->H_kv) % 8) == 0) ? 1 : 0;
     p.tab_fp8 = a->fp8_table_storage ? 1 : 0;
-    p.wide_range = attn_wide(a) ? 1 : 0;
+    p.wide_range = a->wide_range ? 1 : 0;
     p.no_lds_landing = a->force_generic == 2 ? 1 : 0;
     // 4 consecutive scales with one vector load: unit stride, aligned rows, and capacity rows readable
     const int salign = a->dtype == HQMQ_F32 ? 16 : 8;
@@ -727,7 +728,7 @@ static int attn_fwd_impl(const hqmq_attn_args *a, void *stream) {
         default: return HQMQ_ERR_SHAPE;
     }
     if (rc) return rc;
-    if (handled && a->wide_range) {         // the specialised kernels ran on trust: attn_wide saw that the GPU can tell
+    if (handled && guarded) {
         const bool w16 = a->main_bits == 16;
         rc = n == 32 ? (w16 ? launch_again<8, 16>(p, grid, shmem, st) : launch_again<8, 12>(p, grid, shmem, st))
                      : (w16 ? launch_again<4, 16>(p, grid, shmem, st) : launch_again<4, 12>(p, grid, shmem, st));
@@ -740,6 +741,13 @@ static int attn_fwd_impl(const hqmq_attn_args *a, void *stream) {
 }
 
 extern "C" int hqmq_attn_fwd(const hqmq_attn_args *a, void *stream) { return attn_fwd_impl(a, stream); }
+
+extern "C" int hqmq_attn_fwd_guarded(const hqmq_attn_args *a, void *stream) {
+    if (!a || !a->V.scale_max_bits) return HQMQ_ERR_NULL;
+    if (a->wide_range || a->K.flag_plane || a->V.flag_plane) return HQMQ_ERR_LAYOUT;      // a verbatim chunk may be large where no scale is
+    if (a->dtype != HQMQ_F16 && a->dtype != HQMQ_BF16) return HQMQ_ERR_DTYPE;
+    return attn_fwd_impl(a, stream, true);
+}
 
 // ---- the entry point that allocates nothing: split partials in a static device array ----
 // Every GPU the library runs on holds its own copy of this array at its own address until the process ends.

@@ -55,10 +55,6 @@ struct AttnParams {
     int no_lds_landing; // keep the specialised kernels that hold their tiles in registers (testing, measurements)
 };
 
-// Whether the call is for the layout-generic kernel because of its range.  With wide_range 2 the GPU decides, from the largest V
-// scale, behind a specialised kernel (attn_again_kernel); without that word, or where a verbatim chunk may be large too, the host has to.
-inline bool attn_wide(const hqmq_attn_args *a) { return a->wide_range && !(a->wide_range == 2 && a->V.scale_max_bits && !a->K.flag_plane && !a->V.flag_plane); }
-
 __device__ __forceinline__ float load_any(const void *p, int dtype, int64_t i) {
     if (dtype == HQMQ_F16) return __half2float(__ushort_as_half(((const uint16_t *)p)[i]));
     if (dtype == HQMQ_BF16) return __uint_as_float((uint32_t)((const uint16_t *)p)[i] << 16);

@@ -1552,8 +1552,7 @@ int launch_attn_fast(const AttnParams &p, int main_bits, bool flags, dim3 grid, 
     (void)table_bytes;
     *handled = false;
     if (p.dtype != HQMQ_F16 && p.dtype != HQMQ_BF16) return HQMQ_OK;
-    // The kernels of this file form P * (V scale) and convert verbatim chunks in fp16: a bf16 cache whose scales reach
-    // 2^15 (the caller says so: wide_range) takes the layout-generic kernel, which carries the range guard.
+    // The kernels of this file round P * (V scale) and verbatim chunks to fp16: a bf16 cache whose scales reach 2^15 (the caller says so: wide_range) takes the layout-generic kernel, which carries the range guard.
     if (p.wide_range) return HQMQ_OK;
     if (p.n != 16 && p.n != 32) return HQMQ_OK;
     if (p.t_cap % kSuper) return HQMQ_OK;

@@ -650,7 +650,7 @@ static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int ca
 }
 // Whether these kernels can take the call at all.
 static bool attn_prefill_takes(const hqmq_attn_args *a) {
-    if ((a->dtype != HQMQ_F16 && a->dtype != HQMQ_BF16) || attn_wide(a) || (a->n_chunks != 16 && a->n_chunks != 32) ||
+    if ((a->dtype != HQMQ_F16 && a->dtype != HQMQ_BF16) || a->wide_range || (a->n_chunks != 16 && a->n_chunks != 32) ||
         a->fp8_table_storage || (a->force_generic && a->force_generic != 3) || a->softmax_scale <= 0.f)
         return false;
     if (a->main_bits != 16 && (a->main_bits != 12 || a->aux_bits < 1)) return false;

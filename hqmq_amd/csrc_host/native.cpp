@@ -331,7 +331,6 @@ PyObject *fused(PyObject *, PyObject *const *o, Py_ssize_t count) {
     }
     int status = go([&](void *stream) { return hqmq_pack_kv(&pack, stream); });
     if (status) return PyLong_FromLong(status);
-    if (dt == at::kBFloat16) a.wide_range = 2;          // V scales outside [2^-8, 2^15) need the kernel that guards the fp16 range
     const at::Tensor O = at::empty_like(Q);
     output(a, Q, O);
     at::Tensor lens, ws;
@@ -348,7 +347,8 @@ PyObject *fused(PyObject *, PyObject *const *o, Py_ssize_t count) {
         ws = at::empty({a.workspace_bytes}, planes.options());
         a.workspace = ws.data_ptr();
     }
-    status = go([&](void *stream) { return hqmq_attn_fwd(&a, stream); });
+    // bf16 V scales outside [2^-8, 2^15) need the kernel that guards the fp16 range; only the GPU knows them by now
+    status = go([&](void *stream) { return dt == at::kBFloat16 ? hqmq_attn_fwd_guarded(&a, stream) : hqmq_attn_fwd(&a, stream); });
     if (status) return PyLong_FromLong(status);
     return wrap(O);
     END_HANDLE_TH_ERRORS

@@ -299,15 +299,13 @@ typedef struct hqmq_attn_args {
                                  the kernel may keep them as float8 in LDS (4 bytes per codeword, widened after the
                                  gather as :133-135 there does).  Same results as 0 on such tables; honoured by the
                                  specialised decode kernels of the 16-bit layouts at d_h 128, ignored elsewhere. */
-    int wide_range;           /* 1: a bf16 cache whose per-token scales may reach 2^15 (or whose verbatim outlier values may
-                                 exceed 65504), or whose largest scale is below 2^-8.  The specialised kernels multiply the
-                                 softmax weights with the V scales in fp16 and would overflow, or lose the product to fp16
+    int wide_range;           /* not 0: a bf16 cache whose per-token scales may reach 2^15 (or whose verbatim outlier values may
+                                 exceed 65504), or whose largest scale is below 2^-8.  The specialised kernels round the
+                                 softmax weights times the V scales to fp16 and would overflow, or lose the product to fp16
                                  subnormals; such a cache takes the layout-generic kernel, which reads
                                  hqmq_packed.scale_max_bits and keeps every product inside the normal fp16 range (fp32 caches
                                  always take it).  Callers that track the bound (hqmq_quantize_args.scale_max_bits) set this
-                                 when it leaves [2^-8, 2^15); data of ordinary magnitude never does.
-                                 2: the GPU decides, from V.scale_max_bits as it stands when the call's kernels run (16-bit
-                                 caches without outliers; as 1 where that word is NULL). */
+                                 when it leaves [2^-8, 2^15); data of ordinary magnitude never does. */
 } hqmq_attn_args;
 int64_t hqmq_attn_workspace_bytes(int B, int H_q, int T_q, int d_h, int n_splits);
 /* The n_splits hqmq_attn_fwd would choose, from the shapes alone; ragged = 1 when kv_len is passed (sequences of different
@@ -318,6 +316,9 @@ int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv, int ragge
    that one's.  Of one query per sequence it changes at multiples of 64 tokens only. */
 int hqmq_attn_splits(const hqmq_attn_args *a);
 int hqmq_attn_fwd(const hqmq_attn_args *a, void *stream);
+/* hqmq_attn_fwd for callers that do not know the largest V scale yet: the GPU takes wide_range from V.scale_max_bits as it stands
+   when the call's kernels run (a->wide_range is 0).  16-bit caches without outliers; that word must be given. */
+int hqmq_attn_fwd_guarded(const hqmq_attn_args *a, void *stream);
 /* Merge of the split-KV partials (m, l, acc) left in the workspace; hqmq_attn_fwd runs it unless skip_combine. */
 int hqmq_attn_combine(const void *workspace, void *O, int dtype, int B, int H_q, int T_q, int d_h, int n_splits,
                       int64_t o_sb, int64_t o_sh, int64_t o_st, void *stream);

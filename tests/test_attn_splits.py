@@ -39,6 +39,21 @@ def test_splits_keep_to_rounds_of_blocks_and_to_earlier_workspaces():
     assert lib.hqmq_attn_pick_splits(12, 32, 8, 1, 4096, 0) == 2                        # 192 blocks, not 288
 
 
+def test_any_wide_range_is_the_generic_kernel():
+    from hqmq_amd import _lib as L
+    lib, word = L.lib(), C.c_uint32()
+    a = _args(4, 32, 8, 1, 700, 32, False, L.DT_CODE[torch.bfloat16])
+    a.V.scale_max_bits = C.addressof(word)
+    few = lib.hqmq_attn_splits(C.addressof(a))
+    for w in (1, 2, 3, -1):
+        a.wide_range = w
+        assert lib.hqmq_attn_splits(C.addressof(a)) > few, w
+    assert lib.hqmq_attn_fwd_guarded(C.byref(a), None) != 0             # either the caller knows or the GPU decides
+    a.wide_range, a.V.scale_max_bits = 0, None
+    assert lib.hqmq_attn_fwd_guarded(C.byref(a), None) != 0
+    assert lib.hqmq_attn_fwd_guarded(None, None) != 0
+
+
 def test_ragged_batches_beyond_one_round():
     from hqmq_amd import _lib as L
     f16 = L.DT_CODE[torch.float16]
