@@ -5,6 +5,7 @@
 // block may serve several threads.  A function returns its tensors, or the library's status as an int if that is not 0.
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/utils/object_ptr.h>
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -254,10 +255,12 @@ void output(hqmq_attn_args &a, const at::Tensor &Q, const at::Tensor &O) {
 }
 
 // attn(Q, block, out or None, T_kv, kv_lens, kv_starts, batch_order (each or None), causal, causal_offset, scale or None, n_splits,
-//      force_generic, fp8_table_storage, wide_range, workspace or None) -> O
+//      force_generic, fp8_table_storage, wide_range, kept_workspace, options or None) -> O, or (O, partials or None, n_splits)
+//   kept_workspace(bytes, device, "attn") names the buffer that the calls of a stream share;
+//   options: (skip_combine, static_scratch, workspace or None, begin event, end event)
 PyObject *attn(PyObject *, PyObject *const *o, Py_ssize_t count) {
     HANDLE_TH_ERRORS
-    arguments(count, 15);
+    arguments(count, 16);
     const at::Tensor &Q = tensor(o[0]);
     hqmq_attn_args a = *address<hqmq_attn_args>(o[1]);
     const at::Tensor O = o[2] == Py_None ? at::empty_like(Q) : tensor(o[2]);
@@ -276,14 +279,41 @@ PyObject *attn(PyObject *, PyObject *const *o, Py_ssize_t count) {
     a.force_generic = (int)integer(o[11]);
     a.fp8_table_storage = PyObject_IsTrue(o[12]) ? 1 : 0;
     a.wide_range = PyObject_IsTrue(o[13]) ? 1 : 0;
-    if (o[14] != Py_None) {
-        const at::Tensor &ws = tensor(o[14]);
+    bool own_scratch = false;
+    at::Tensor ws;
+    if (o[15] != Py_None) {
+        TORCH_CHECK_TYPE(PyTuple_Check(o[15]) && PyTuple_GET_SIZE(o[15]) == 5, "expected a tuple of five options");
+        PyObject *const *opt = &PyTuple_GET_ITEM(o[15], 0);
+        a.skip_combine = PyObject_IsTrue(opt[0]) ? 1 : 0;
+        own_scratch = PyObject_IsTrue(opt[1]);
+        if (opt[2] != Py_None) ws = tensor(opt[2]);
+        a.start_event = address<void>(opt[3]);
+        a.stop_event = address<void>(opt[4]);
+    }
+    if (own_scratch) {
+        const int status = Launch(Q)([&](void *stream) { return hqmq_attn_fwd_static(&a, stream); });
+        return status ? PyLong_FromLong(status) : wrap(O);
+    }
+    if (a.n_splits <= 0) a.n_splits = hqmq_attn_splits(&a);
+    if (a.n_splits > 1) {
+        const int64_t bytes = hqmq_attn_workspace_bytes(a.B, a.H_q, a.T_q, 4 * a.n_chunks, a.n_splits);
+        if (ws.defined()) {
+            if (ws.device() != Q.device()) return PyLong_FromLong(HQMQ_ERR_WORKSPACE);
+        } else if (a.skip_combine) {
+            ws = at::empty({bytes}, Q.options().dtype(at::kByte));          // the caller's from here on
+        } else {
+            THPObjectPtr device(PyObject_GetAttrString(o[0], "device")), kept(device ? PyObject_CallFunction(o[14], "LOs", (long long)bytes, device.get(), "attn") : nullptr);
+            if (!kept) throw python_error();
+            ws = tensor(kept.get());
+        }
         a.workspace = ws.data_ptr();
         a.workspace_bytes = (int64_t)ws.nbytes();
-    }
+    } else ws = at::Tensor();
     const int status = Launch(Q)([&](void *stream) { return hqmq_attn_fwd(&a, stream); });
     if (status) return PyLong_FromLong(status);
-    return wrap(O);
+    if (!a.skip_combine) return wrap(O);
+    THPObjectPtr n(PyLong_FromLong(a.n_splits)), o_out(wrap(O)), ws_out(wrap(ws));
+    return PyTuple_Pack(3, o_out.get(), ws_out.get(), n.get());
     END_HANDLE_TH_ERRORS
 }
 

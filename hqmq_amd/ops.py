@@ -384,86 +384,17 @@ def attn_fwd(Q: torch.Tensor, Kc, Vc, T_kv: int, *, kv_lens: Optional[torch.Tens
     plan = Kc._attn_plans.get((shape, stride))
     if plan is None or plan[0] is not ks or plan[1] is not vs or plan[2] is not Q.dtype:
         plan = _attn_plan(Q, Kc, Vc, ks, vs)
-    _, _, _, tmpl, o_stride, rows, floats, splits = plan
-    dev = Q.device
-    few = shape[2] == 1 and shape[1] < 64 * Kc.H       # not for the prefill kernels: the choice looks at nothing but the key below
-    if not (skip_combine or static_scratch or kernel_events or workspace is not None) and (few or n_splits > 0):
-        wide = Vc.wide_range                       # V scales outside [2^-8, 2^15): the generic kernel guards the range
-        n = n_splits if n_splits > 0 else splits.get(((T_kv + 63) // 64, kv_lens is None, wide, force_generic))
-        if n is not None:
-            for t, what in ((kv_starts, "kv_starts must hold one entry per sequence"), (batch_order, "batch_order must be a permutation of the sequences")):
-                if t is not None and t.numel() != shape[0]:
-                    raise L.HqmqError(f"{what} ({shape[0]})")
-            return L.tensors(L.native().attn(Q, tmpl.address, out, T_kv, kv_lens, kv_starts, batch_order, causal, causal_offset, softmax_scale, n,
-                                             force_generic, fp8_table_storage, wide, _workspace(rows * floats * n * 4, dev, "attn") if n > 1 else None),
-                             "hqmq_attn_fwd")
-    index = dev.index
-    O = torch.empty_like(Q) if out is None else out
-    a = L.AttnArgs.from_buffer_copy(tmpl)          # this call's own: several threads may attend over one cache
-    a.Q, a.O = Q.data_ptr(), O.data_ptr()
-    strides = O.stride()
-    if strides != o_stride:
-        a.o_sb, a.o_sh, a.o_st = strides[0], strides[1], strides[2]
-    a.T_kv = T_kv
-    if softmax_scale is not None:
-        a.softmax_scale = softmax_scale
-    if kv_lens is not None:
-        if kv_lens.dtype is not torch.int32 or kv_lens.device != dev or not kv_lens.is_contiguous():
-            kv_lens = kv_lens.to(device=dev, dtype=torch.int32).contiguous()
-        a.kv_len = kv_lens.data_ptr()
-    if kv_starts is not None:
-        kv_starts = kv_starts.to(device=dev, dtype=torch.int32).contiguous()
-        if kv_starts.numel() != shape[0]:
-            raise L.HqmqError(f"kv_starts must hold one entry per sequence ({shape[0]})")
-        a.kv_start = kv_starts.data_ptr()
-    if batch_order is not None:
-        if batch_order.dtype is not torch.int32 or batch_order.device != dev or not batch_order.is_contiguous():
-            batch_order = batch_order.to(device=dev, dtype=torch.int32).contiguous()
-        if batch_order.numel() != shape[0]:
-            raise L.HqmqError(f"batch_order must be a permutation of the {shape[0]} sequences")
-        a.batch_order = batch_order.data_ptr()
-    if causal:
-        a.causal, a.causal_offset = 1, causal_offset
-    if skip_combine:
-        a.skip_combine = 1
-    if force_generic:
-        a.force_generic = int(force_generic)
-    if fp8_table_storage:
-        a.fp8_table_storage = 1
-    if Vc.wide_range:                              # V scales outside [2^-8, 2^15): the generic kernel guards the range
-        a.wide_range = 1
-    if kernel_events is not None:
-        a.start_event, a.stop_event = kernel_events
-    if n_splits <= 0:
-        if static_scratch:
-            n_splits = pick_splits(shape[0], shape[1], Kc.H, shape[2], max(T_kv, 1), kv_lens is not None)
-        elif not few:
-            n_splits = L.lib().hqmq_attn_splits(C.addressof(a))
-        else:                                      # of one token, the library's choice changes at multiples of 64 tokens only
-            if len(splits) >= 4096:
-                splits.clear()
-            key = ((T_kv + 63) // 64, kv_lens is None, Vc.wide_range, force_generic)
-            n_splits = splits[key] = L.lib().hqmq_attn_splits(C.addressof(a))
-    a.n_splits = n_splits
-    if static_scratch:
-        L.call(L.lib().hqmq_attn_fwd_static, "hqmq_attn_fwd_static", index, C.addressof(a))
-        return O
-    ws = None
-    if n_splits > 1:
-        nbytes = rows * floats * n_splits * 4
-        if workspace is not None:
-            if workspace.device != dev or workspace.numel() * workspace.element_size() < nbytes:
-                raise L.HqmqError(f"workspace must hold {nbytes} bytes on {dev}")
-            ws = workspace
-        elif skip_combine:
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-        else:
-            ws = _workspace(nbytes, dev, "attn")
-        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel() * ws.element_size()
-    L.call(L.lib().hqmq_attn_fwd, "hqmq_attn_fwd", index, C.addressof(a))
-    if skip_combine:
-        return O, ws, n_splits
-    return O
+    for t, what in ((kv_starts, "kv_starts must hold one entry per sequence"), (batch_order, "batch_order must be a permutation of the sequences")):
+        if t is not None and t.numel() != shape[0]:
+            raise L.HqmqError(f"{what} ({shape[0]})")
+    options = None
+    if skip_combine or static_scratch or kernel_events or workspace is not None:
+        start, stop = kernel_events or (0, 0)
+        options = (skip_combine, static_scratch, workspace, start or 0, stop or 0)
+    # (wide_range: V scales outside [2^-8, 2^15), the generic kernel guards the range)
+    return L.tensors(L.native().attn(Q, plan[3].address, out, T_kv, kv_lens, kv_starts, batch_order, causal, causal_offset, softmax_scale, n_splits,
+                                     force_generic, fp8_table_storage, Vc.wide_range, _workspace, options),
+                     "hqmq_attn_fwd_static" if static_scratch else "hqmq_attn_fwd")
 
 
 _FUSED = {}
@@ -530,8 +461,7 @@ def _fused_plan(Q: torch.Tensor, idx: torch.Tensor, T_v: int, K: int, K_v: int, 
 
 
 def _attn_plan(Q: torch.Tensor, Kc, Vc, ks, vs):
-    """What a shape of Q and a pair of packed tensors fix of an attention call, kept with the K cache: the argument block,
-    the strides of an output like Q, the partial rows and floats per row and split, the library's split counts by context."""
+    """What a shape of Q and a pair of packed tensors fix of an attention call, kept with the K cache."""
     B, Hq, Tq, d_h = Q.shape
     if d_h != Kc.d_head or d_h != Vc.d_head:
         raise AssertionError(f"d_h={d_h} != n_chunks*4={Kc.d_head}")
@@ -541,17 +471,13 @@ def _attn_plan(Q: torch.Tensor, Kc, Vc, ks, vs):
         raise L.HqmqError(f"Q dtype {Q.dtype} differs from the cache dtype {Kc.dtype}")
     a = L.AttnArgs()
     a.q_sb, a.q_sh, a.q_st = Q.stride(0), Q.stride(1), Q.stride(2)
-    o_stride = torch.empty_like(Q).stride()
-    a.o_sb, a.o_sh, a.o_st = o_stride[0], o_stride[1], o_stride[2]
     a.K, a.V = ks, vs
     a.dtype = L.DT_CODE[Q.dtype]
     a.B, a.H_q, a.H_kv, a.T_q, a.n_chunks = B, Hq, Kc.H, Tq, Kc.n
     a.t_cap = Kc.t_cap
     a.idx_bits, a.main_bits, a.aux_bits, a.qmax = Kc.idx_bits, Kc.main_bits, Kc.aux_bits, Kc.qmax
     a.softmax_scale = d_h ** -0.5
-    per_split = int(L.lib().hqmq_attn_workspace_bytes(C.c_int(B), C.c_int(Hq), C.c_int(Tq), C.c_int(d_h), C.c_int(2))) // 8
-    rows = B * Hq * Tq
-    plan = (ks, vs, Q.dtype, a, o_stride, rows, per_split // rows, {})
+    plan = (ks, vs, Q.dtype, a)
     if len(Kc._attn_plans) >= 64:                  # shapes that no longer come
         Kc._attn_plans.clear()
     a.address = C.addressof(a)
