@@ -1,5 +1,6 @@
 // Attention kernels specialised at compile time for the layouts of the benchmark shapes:
-// d_h = 64 / 128, fp16 or bf16 caches, codes of 16+0 (s96_r4), 12+1 (s24_r3) or 16+3 (s192_r6) bits.
+// d_h = 64 / 128, fp16 or bf16 caches, codes of 16+0 (s96_r4), 12+1 (s24_r3) or 16+3 (s192_r6) bits, and with a generic field decode
+// of 16+1, 16+2, 12+2 or 12+3.
 //
 // Lane mapping (one wavefront, one 16-token tile): lane = 16 * grp + col decodes the CPL = d_h / 16 chunks
 // grp * CPL ... of token `col`, for K and for V alike.
@@ -9,7 +10,8 @@
 //                     identity (exact: every output is one fp16 input times 1.0) and two packed conversions,
 //                     instead of a dozen cross-lane VALU operations per chunk.
 //   O^T += V^T . P^T  v_mfma_f32_16x16x32_f16 over two tiles (32 tokens) at a time.
-// Row j of the V-side product is d = (grp * CPL + j) * 4 + e, the order the epilogue writes back.
+// P times the token's V scale is an fp32 product rounded to fp16 once, as in the other attention kernels; so is qmax P, the weight of
+// verbatim chunks.  Row j of the V-side product is d = (grp * CPL + j) * 4 + e, the order the epilogue writes back.
 // Scores are kept as S^T * rs; 1/qmax is folded into the softmax scale and the epilogue.  Outlier chunks
 // carry radius code 0 in the planes, so they decode to zero; their verbatim values enter through extra MFMAs
 // that walk the sideband entry list (values + coordinates), never the flag plane.

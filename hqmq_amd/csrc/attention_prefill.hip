@@ -34,8 +34,9 @@
 // 32768 tokens 0.93 ms against 2.88, 300 on 8000 (28 / 4 heads, s192_r6) 0.122 against 0.318.  (K held as values like V, without the
 // second product: 0.70 and 0.101, but up to 1.55 times as far from 64-bit results at K of 3e-5 and 1.34 times at K of order one;
 // values only in tokens with verbatim chunks, in units of a power of two: 0.80 and 0.107, still up to 1.11.)  Error against 64-bit
-// results relative to the decode kernels', 162 calls: K from 3e-5 to 30 at V of order one 0.92 on average, 0.99 at most; V of 1e-4
-// 0.77 and 1.00, V of 3e-5, where outputs are fp16 subnormals, 0.81 and 1.08.
+// results relative to the decode kernels', 162 calls: K from 3e-5 to 30 at V of order one 0.96 on average, 1.03 at most; V of 1e-4
+// 0.96 and 1.00, V of 3e-5, where outputs are fp16 subnormals, 1.02 and 1.08; plain fp16 caches 1.00 to 1.01, bf16 1.00 to 1.02
+// (s24_r3, where the codes are exact in fp16 and little but P is rounded, 1.30 to 1.45).
 // What bounds it: overlap, no pipe is full.  By the counters (profiles/attn_prefill_kernel_instruction_counters.txt) a compute unit
 // spends 37 % of its busy cycles in the matrix pipe, 50 % issuing vector instructions and 63 % in LDS, a third of that bank
 // conflicts (plain, 1024 on 32768), at 2.0 to 2.1 GHz; with verbatim chunks 37, 64 and 40 %; 2048 on 2048 causal 21, 51 and 38 %.

@@ -5,11 +5,12 @@
 // reference): per head, the median over every chunk norm of the call (fp32
 // interpolation between the two middle order statistics), times the
 // multiplier, rounded to D.  The order statistics are exact: chunk norms are
-// non-negative, so their bit patterns sort like the values.  Calls of at most
-// 8192 chunks per head keep the keys in registers and search the key bit by bit
-// (one launch); larger ones of a 16-bit type take a 32768-bin histogram of its
-// whole key per block, which the selection adds up where it looks (two launches);
-// fp32, calls too large for 16-bit counters and workspaces too small for that take
+// non-negative, so their bit patterns sort like the values.  Calls of a 16-bit
+// type with 65 to 16384 chunks per head take one block per head and a histogram of
+// its whole key in LDS (one launch); at most 64 chunks, and fp32 up to 8192, keep the
+// keys in registers and search the key bit by bit (one launch); larger 16-bit calls
+// take such a histogram per block, which the selection adds up where it looks (two
+// launches); larger fp32, calls too large for 16-bit counters and workspaces too small for that take
 // one histogram per head of the top 16 bits, and fp32 a second pass over the low 16
 // bits of the bin(s) holding the two ranks.  K and V of one append share the launches.
 //

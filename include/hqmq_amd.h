@@ -123,7 +123,7 @@ int hqmq_quantize_grid(const hqmq_quantize_args *a, const void *grid, void *stre
  * threshold RNE_D(median * mult).  Replaces the torch.quantile half of
  * OutlierAwareHQMQQuantizer._qdq (src/quantizers/outlier_aware.py:60-69).
  *   workspace  at least hqmq_med3x_workspace_bytes(H, dtype) bytes, any content, 16-byte aligned for best; from
- *              hqmq_med3x_workspace_best_bytes(H, dtype) on (16.9 MB up to 256 heads of a 16-bit type) calls beyond 8192
+ *              hqmq_med3x_workspace_best_bytes(H, dtype) on (16.9 MB up to 256 heads of a 16-bit type) calls beyond 16384
  *              chunks per head take two launches instead of three and a third to two thirds of the time
  *   median     [H] fp32 (out);  thr [H] D (out);  n_out [H] int32 (out, may be NULL):
  *              number of chunks with norm > thr */
