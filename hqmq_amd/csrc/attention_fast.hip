@@ -81,20 +81,11 @@ struct FlagTile {
     int koff[3];               // K: sideband entries [koff[u], koff[u + 1]) belong to tile u (wave-uniform)
     int voff[3];               // V: the same
 };
-// K outliers of one half-step, requested ahead: the first NB batches of eight sideband entries.  Lane
-// 16 * grp + col holds entries 2 * grp and 2 * grp + 1 of a batch (the same in all 16 lanes of a row).
-template <int NB>
-struct KPre {
+// verbatim chunks of one half-step and tensor, requested ahead: lane i holds the i-th of its first 64 sideband entries
+struct Entries {
     int off[3];
-    uint4v x[NB];              // two verbatim chunks (raw bits of the cache dtype) as loaded, see k_load
-    uint32_t cc[NB];           // their coordinates as loaded: (token & 15) << 8 | chunk, two 16-bit fields
-};
-// V outliers of one half-step: the first NB batches of sixteen entries; lane 16 * grp + col holds entry `col`.
-template <int NB>
-struct VPre {
-    int off[3];
-    uint2 x[NB];
-    uint32_t cc[NB];
+    uint2 x;                   // the chunk (raw bits of the cache dtype) and its coordinates, (token & 15) << 8 | chunk, as loaded
+    uint32_t cc;
 };
 // the unit of prefetch: NH half-tiles of 32 tokens
 template <int NW, int AB, bool FLAGS, int NH>
@@ -117,19 +108,24 @@ __device__ __forceinline__ uint32_t load_small(const uint8_t *p) {
 // The dynamic LDS block is the kernel's only LDS, so it starts at LDS address 0: the K table sits at byte 0,
 // the V table at kVTabOffset, and a gather addresses them with idx * 8 (+ the instruction's immediate offset).
 constexpr int kVTabOffset = 40960;          // bytes; room for 5120 K codewords in front of it
-constexpr int kQOffset = kVTabOffset + 36864;     // outlier variants: Q as [chunk][column] fp16 chunks, after the V table
-constexpr int kFlagsTabMax = (kQOffset - kVTabOffset) / 8;      // codewords the V slot of the outlier variants holds
-static_assert(kFlagsTabMax * 8 + kVTabOffset == kQOffset && kFlagsTabMax == 4608, "V table slot of the outlier variants");
+constexpr int kStageOffset = kVTabOffset + 36864;       // outlier variants: staging rows of the wavefronts, after the V table
+constexpr int kFlagsTabMax = (kStageOffset - kVTabOffset) / 8;  // codewords the V slot of the outlier variants holds
+static_assert(kFlagsTabMax == 4608, "V table slot of the outlier variants");
 constexpr int kAuxTabOffset = 36864;        // s192_r6: 64 dwords with the high radius bits of a pair of chunks, see gather_chunks
 // s24_r3 (13-bit codes, K <= 1024, qmax = 7): the tables are kept multiplied out, entry [rq][idx] = codeword * rq at byte
 // (rq << 10 | idx) * 8, so that the 13-bit code is the table index and a decode is one gather (no radius arithmetic).
 constexpr int kPsTabBytes = 8 * 1024 * 8;   // 64 KB per tensor
 constexpr bool is_prescaled(int MB, int AB, int IB) { return MB == 12 && AB == 1 && IB == 10; }
 constexpr int vtab_offset(bool ps) { return ps ? kPsTabBytes : kVTabOffset; }
-constexpr int q_offset(bool ps) { return ps ? 2 * kPsTabBytes : kQOffset; }
-constexpr int sel_offset(bool ps) { return q_offset(ps) + 4096; }      // nine rows of eight fp16: row r < 8 = unit vector r, row 8 = 0
+// Outlier variants: a wavefront's staging rows hold this many 16-token tiles (beside the multiplied tables there is room for one)
+constexpr int stage_offset(bool ps) { return ps ? 2 * kPsTabBytes : kStageOffset; }
+constexpr int stage_tiles(bool ps) { return ps ? 1 : 2; }
+constexpr int stage_bytes(bool ps, int CPL) { return stage_tiles(ps) * 16 * 32 * CPL; }
+// The wavefronts' progress slots: behind the staging rows, or in the last eight entries of the multiplied V table (Vc.K <= 1016)
+constexpr int flags_prog_offset(bool ps, int CPL, int WV) { return ps ? 2 * kPsTabBytes - 64 : stage_offset(ps) + WV * stage_bytes(ps, CPL); }
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short short4v __attribute__((ext_vector_type(4)));
+typedef uint32_t uint2v_t __attribute__((ext_vector_type(2)));
 template <int TAB_OFF>
 __device__ __forceinline__ half4 gather8(uint32_t byte_addr) {
     return __builtin_bit_cast(half4, *(lds_u2_ptr)(uintptr_t)(byte_addr + TAB_OFF));
@@ -335,7 +331,6 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     static_assert(NB % 4 == 0 || NB == 6, "main bytes of one lane");
     static_assert(CPL % 2 == 0, "two chunks per 16x16x32 operand");
     constexpr int NT = WV * 64;
-    constexpr int kKPre = CPL >= 8 ? 3 : 1;     // batches of outlier entries requested ahead (d_h 64 has half the chunks)
     constexpr bool kBatchGathers = false;       // see half_step: measured, no gain on any shape (178 against 157 registers)
     constexpr int NH = 1;       // half-steps per prefetched tile: one measures faster than two on every shape
     extern __shared__ uint2 lds_tab[];
@@ -346,7 +341,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     unsigned long long t_loop_ = 0;
 #endif
     constexpr bool PS = is_prescaled(MB, AB, IB);
-    constexpr int VTAB = vtab_offset(PS), QOFF = q_offset(PS), SELOFF = sel_offset(PS);
+    constexpr int VTAB = vtab_offset(PS);
     uint2 *ktab = lds_tab, *vtab = lds_tab + VTAB / 8;
     touch_kernargs();
 
@@ -480,8 +475,6 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const char *v_side = FLAGS ? (const char *)p.Vc.sideband + (size_t)bh * p.Vc.sb_cap * 8 : nullptr;
     const char *k_coord = FLAGS ? (const char *)p.Kc.sb_coord + (size_t)bh * p.Kc.sb_cap * 2 : nullptr;
     const char *v_coord = FLAGS ? (const char *)p.Vc.sb_coord + (size_t)bh * p.Vc.sb_cap * 2 : nullptr;
-    const uint32_t v_cap1 = FLAGS ? (uint32_t)(p.Vc.sb_cap - 1) : 0u;
-    const uint32_t k_cap2 = FLAGS ? (uint32_t)(p.Kc.sb_cap - 2) : 0u;        // sb_cap >= 2 is checked at launch
 
     auto load_super = [&](int t0, FastTile<NW, AB, FLAGS, NH> &s) {
         // in the order the half-steps consume them: K, then V, of tokens 0..31, then the same of tokens 32..63
@@ -543,52 +536,22 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 
     // Every load of the loop is issued unconditionally (clamped addresses): a load inside a branch would make the
     // compiler's wait counts assume it was not issued, and the waits would then cover the next tile's prefetch.
-    // K side.  The sideband entries of a half-step are a contiguous range known from three tile offsets, so no
-    // flag is read: a batch of eight entries is the reduction dimension of one MFMA per tile,
-    //   so[token][column] += sum over entries e of the batch, i < 4:  [token(e) == token] x_e[i] * Q[column][4 chunk(e) + i],
-    // A = the lane's two entries where their token is the lane's row (else zero), B = the Q chunks they meet (LDS).
-    // The lane's two entries are neighbours in the list: one 16-byte load of the chunks (8-byte aligned) and one 4-byte
-    // load of the coordinates (2-byte aligned), at 32-bit byte offsets from wave-uniform bases (sb_cap < 2^28 is checked
-    // at launch).  The pair is clamped to the last pair of the list's storage: an entry that is the very last slot of
-    // a full list then arrives in the upper half.  (A wave-uniform branch to an unclamped variant measures slower.)
-    // (The loaded words are kept as they come and put right by k_fix_x / k_fix_cc where they are used: touching them here would
-    // make the request wait for its own data, and for every request before it.)
-    auto k_load = [&](int bs, uint4v &x, uint32_t &cc) {
-        const uint32_t ec = min((uint32_t)bs + 2u * (uint32_t)grp, k_cap2);
-        x = *reinterpret_cast<const uint4v_a8 *>(k_side + ec * 8u);
-        cc = *reinterpret_cast<const uint32_a2 *>(k_coord + ec * 2u);
-    };
-    auto k_fix_cc = [&](int bs, uint32_t cc) { return (uint32_t)bs + 2u * (uint32_t)grp > k_cap2 ? cc >> 16 : cc; };
-    auto k_fix_x = [&](int bs, uint4v X, uint2 (&x)[2]) {
-        const bool up = (uint32_t)bs + 2u * (uint32_t)grp > k_cap2;
-        x[0] = uint2{up ? X[2] : X[0], up ? X[3] : X[1]};
-        x[1] = uint2{X[2], X[3]};
-    };
-    auto k_issue = [&](const FlagTile &f, KPre<kKPre> &k) {
-#pragma unroll
-        for (int i = 0; i < 3; i++) k.off[i] = f.koff[i];
-#pragma unroll
-        for (int bq = 0; bq < kKPre; bq++) k_load(k.off[0] + 8 * bq, k.x[bq], k.cc[bq]);
-    };
-    constexpr int kVPre = CPL >= 8 ? 2 : 1;
-    auto v_load = [&](int bs, uint2 &x, uint32_t &cc) {
-        const uint32_t e = min((uint32_t)bs + (uint32_t)col, v_cap1);
-        x = *reinterpret_cast<const uint2 *>(v_side + e * 8u);
-        cc = *reinterpret_cast<const uint16_t *>(v_coord + e * 2u);
-    };
-    auto v_issue = [&](const FlagTile &f, VPre<kVPre> &v) {
-#pragma unroll
-        for (int i = 0; i < 3; i++) v.off[i] = f.voff[i];
-#pragma unroll
-        for (int bq = 0; bq < kVPre; bq++) v_load(v.off[0] + 16 * bq, v.x[bq], v.cc[bq]);
+    // The sideband entries of a half-step are a contiguous range known from three tile offsets, so no flag is read.  Lane i takes
+    // entry i of the range (the last one again behind its end), at 32-bit byte offsets from wave-uniform bases (sb_cap < 2^28 is
+    // checked at launch).
+    auto entry_load = [&](const char *side, const char *coord, const int (&off)[3], int e, uint2 &x, uint32_t &cc) {
+        const uint32_t at = min((uint32_t)e, (uint32_t)max(off[2] - 1, 0));       // (inconsistent offsets of a caller may be negative)
+        x = *reinterpret_cast<const uint2 *>(side + at * 8u);
+        cc = *reinterpret_cast<const uint16_t *>(coord + at * 2u);
     };
     // sideband requests of one half-step
-    auto issue_all = [&](const FlagTile &f, KPre<kKPre> &k, VPre<kVPre> &v) {
-        k_issue(f, k);
-        v_issue(f, v);
+    auto issue_all = [&](const FlagTile &f, Entries &k, Entries &v) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) { k.off[i] = f.koff[i]; v.off[i] = f.voff[i]; }
+        entry_load(k_side, k_coord, k.off, k.off[0] + lane, k.x, k.cc);
+        entry_load(v_side, v_coord, v.off, v.off[0] + lane, v.x, v.cc);
     };
-    KPre<kKPre> kc = {};
-    VPre<kVPre> vc = {};
+    Entries kc = {}, vc = {};
     FastTile<NW, AB, FLAGS, NH> cur;
     FlagTile f0 = {}, f1 = {};
     uint2 q_raw[NCG][CPL];      // the query rows as stored
@@ -640,12 +603,8 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     half4 ident;                        // B operand of the transposing MFMA: the 16x16 identity
 #pragma unroll
     for (int e = 0; e < 4; e++) ident[e] = (_Float16)((4 * grp + e) == col ? 1.f : 0.f);
-    // bf16 caches: the verbatim sideband chunks (and the Q copy they meet) go into bf16 MFMAs as they are stored,
-    // which saves their conversion to fp16 (6 VALU per chunk); the products are exact either way
+    // bf16 caches: K's verbatim chunks (and the Q they meet) go into bf16 MFMAs as they are stored; the products are exact
     constexpr bool kBfEntries = FLAGS && DT == HQMQ_BF16;
-    short4v ident_bf;
-#pragma unroll
-    for (int e = 0; e < 4; e++) ident_bf[e] = (short)((4 * grp + e) == col ? 0x3F80 : 0);
 
     {
         if constexpr (PS) {
@@ -671,11 +630,6 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
             }
         }
     }
-    if (FLAGS && threadIdx.x >= 64 && threadIdx.x < 100) {
-        const uint32_t w = threadIdx.x - 64, row = w >> 2, d = w & 3;
-        const uint32_t one = 0x3c00u;       // 1 in fp16
-        reinterpret_cast<uint32_t *>(lds_tab)[SELOFF / 4 + w] = (row < 8 && (row >> 1) == d) ? one << (16 * (row & 1)) : 0u;
-    }
     half8 qf[NCG][CPL / 2];
 #pragma unroll
     for (int cgi = 0; cgi < NCG; cgi++) {
@@ -685,21 +639,24 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
             qf[cgi][j] = cat8(col_ok[cgi] ? chunk_to_half<DT>(q_raw[cgi][2 * j]) : z, col_ok[cgi] ? chunk_to_half<DT>(q_raw[cgi][2 * j + 1]) : z);
         }
     }
-    if (FLAGS && wave == 0) {       // every wavefront of the block has the same 16 columns
+    bf16x8 qb[kBfEntries ? CPL / 2 : 1];            // the stored bf16 values
+    if constexpr (kBfEntries) {
 #pragma unroll
-        for (int jj = 0; jj < CPL / 2; jj++) {
-            uint4v q8 = __builtin_bit_cast(uint4v, qf[0][jj]);
-            if constexpr (kBfEntries) {         // the stored bf16 values
-                const uint2 lo = col_ok[0] ? q_raw[0][2 * jj] : uint2{0, 0}, hi = col_ok[0] ? q_raw[0][2 * jj + 1] : uint2{0, 0};
-                q8 = uint4v{lo.x, lo.y, hi.x, hi.y};
-            }
-            const int c0 = grp * CPL + 2 * jj;
-            lds_tab[QOFF / 8 + c0 * 16 + col] = uint2{q8[0], q8[1]};
-            lds_tab[QOFF / 8 + (c0 + 1) * 16 + col] = uint2{q8[2], q8[3]};
+        for (int j = 0; j < CPL / 2; j++) {
+            const uint2 lo = col_ok[0] ? q_raw[0][2 * j] : uint2{0, 0}, hi = col_ok[0] ? q_raw[0][2 * j + 1] : uint2{0, 0};
+            qb[j] = __builtin_bit_cast(bf16x8, uint4v{lo.x, lo.y, hi.x, hi.y});
         }
     }
+    // staging rows for verbatim chunks, cleared here and after every use
+    constexpr int ST = stage_tiles(PS), ROWB = 32 * CPL, STB = 16 * ROWB;
+    const uint32_t stage = (uint32_t)(stage_offset(PS) + wave * stage_bytes(PS, CPL));
+    auto wipe = [&]() {
+#pragma unroll
+        for (int i = 0; i < ST * STB / 1024; i++) *(uint4v __attribute__((address_space(3))) *)(uintptr_t)(stage + 1024u * i + 16u * (uint32_t)lane) = uint4v{0, 0, 0, 0};
+    };
+    if constexpr (FLAGS) wipe();
     // Progress slots of the wavefronts (see `publish` below), behind everything else the loop keeps in LDS
-    const uint32_t prog_base = FLAGS ? (uint32_t)SELOFF + 192u : PS ? 2u * (uint32_t)kPsTabBytes : (uint32_t)kVTabOffset + (uint32_t)p.Vc.K * 8u;
+    const uint32_t prog_base = FLAGS ? (uint32_t)flags_prog_offset(PS, CPL, WV) : PS ? 2u * (uint32_t)kPsTabBytes : (uint32_t)kVTabOffset + (uint32_t)p.Vc.K * 8u;
     typedef int __attribute__((address_space(3))) *lds_i32_ptr;
     if (threadIdx.x < 16) *(lds_i32_ptr)(uintptr_t)(prog_base + 4u * threadIdx.x) = 0;
     if constexpr (MB == 16 && AB == 3 && IB == 13) {
@@ -728,125 +685,80 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         for (int j = 0; j < CPL; j++) acc[cgi][j] = float4v{0.f, 0.f, 0.f, 0.f};
     }
     const float4v zero4 = float4v{0.f, 0.f, 0.f, 0.f};
-    const half4 zero_h4 = half4{0, 0, 0, 0};
-    // the Q chunks the lane's two entries meet (B operand rows), read from LDS well before the batch's MFMAs
-    auto k_qrows = [&](uint32_t cc, uint2 (&q)[2]) {
-        const uint32_t c0 = cc & (uint32_t)(n - 1), c1 = (cc >> 16) & (uint32_t)(n - 1);
-        q[0] = __builtin_bit_cast(uint2, *(lds_u2_ptr)(uintptr_t)(QOFF + c0 * 128u + (uint32_t)col * 8u));
-        q[1] = __builtin_bit_cast(uint2, *(lds_u2_ptr)(uintptr_t)(QOFF + c1 * 128u + (uint32_t)col * 8u));
+    // Verbatim chunks.  The wavefront writes a half-step's entries (K's, then V's) over zeros into rows of its own in LDS,
+    // [token][chunk], reads them as whole matrix operands and clears what it wrote: its LDS accesses keep their order, so nothing
+    // has to be waited for but the data itself.  The chunks of a row are permuted by the token (16-byte parts, exclusive-or), so
+    // that K's reads (16 tokens at the same part) and V's transposing ones (4 tokens at 4 parts) meet 64 different banks.
+    typedef uint2v_t __attribute__((address_space(3))) *lds_w2_ptr;
+    auto swizzled = [&](uint32_t row, uint32_t byte) {          // byte: 8 * chunk
+        return CPL == 8 ? byte ^ row * 0x110u : byte ^ (row * 0x88u & ~8u);
     };
-    auto k_batch = [&](const int (&off)[3], int bs, uint4v x_loaded, uint32_t cc_loaded, const uint2 (&q)[2], float4v (&so)[2]) {
-        const int e0 = bs + 2 * grp;
-        uint2 x[2];
-        k_fix_x(bs, x_loaded, x);
-        const uint32_t cc = k_fix_cc(bs, cc_loaded);
-        // the row of the half-step (0..31) an entry belongs to; 64 for a slot behind the half-step's entries
-        const uint32_t k0 = e0 < off[2] ? ((cc >> 8) & 15u) + (e0 >= off[1] ? 16u : 0u) : 64u;
-        const uint32_t k1 = e0 + 1 < off[2] ? ((cc >> 24) & 15u) + (e0 + 1 >= off[1] ? 16u : 0u) : 64u;
-        const uint2 zero_u2 = uint2{0u, 0u};
-        half4 h0 = zero_h4, h1 = zero_h4;
-        if constexpr (!kBfEntries) { h0 = chunk_to_half<DT>(x[0]); h1 = chunk_to_half<DT>(x[1]); }
-        const half8 qq = cat8(__builtin_bit_cast(half4, q[0]), __builtin_bit_cast(half4, q[1]));
-        // both tiles, no branch: the matrix unit is idle here and a skipped MFMA saves less than its test costs
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const bool v0 = k0 == (uint32_t)(col + 16 * u), v1 = k1 == (uint32_t)(col + 16 * u);
-            if constexpr (kBfEntries) {
-                const uint2 a0 = v0 ? x[0] : zero_u2, a1 = v1 ? x[1] : zero_u2;
-                so[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, uint4v{a0.x, a0.y, a1.x, a1.y}),
-                                                                __builtin_bit_cast(bf16x8, uint4v{q[0].x, q[0].y, q[1].x, q[1].y}),
-                                                                so[u], 0, 0, 0);
-            } else {
-                so[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cat8(v0 ? h0 : zero_h4, v1 ? h1 : zero_h4), qq, so[u], 0, 0, 0);
-            }
-        }
+    auto entry_at = [&](const int (&off)[3], int e, uint32_t cc) {
+        const uint32_t at = swizzled((cc >> 8) & 15u, (cc & (uint32_t)(n - 1)) << 3) + stage;
+        return ST == 2 && e >= off[1] ? at + (uint32_t)STB : at;
     };
-    struct KRows {
-        uint2 q[kKPre][2];
+    auto mine = [&](const int (&off)[3], int u0, int e) { return (ST == 2 || e >= off[u0]) && e < off[u0 + ST]; };
+    auto verbatim = [&](uint2 x, bool v) {                      // V meets fp16 weights
+        if (!kBfEntries || !v) return x;
+        return __builtin_bit_cast(uint2, pack4(float4v{__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u), __uint_as_float(x.y << 16), __uint_as_float(x.y & 0xffff0000u)}));
     };
-    auto k_prepare = [&](const KPre<kKPre> &k, KRows &r) {
-#pragma unroll
-        for (int bq = 0; bq < kKPre; bq++) k_qrows(k_fix_cc(k.off[0] + 8 * bq, k.cc[bq]), r.q[bq]);
-    };
-    auto k_apply = [&](const KPre<kKPre> &k, const KRows &r, float4v (&so)[2]) {
-#pragma unroll
-        for (int bq = 0; bq < kKPre; bq++)
-            if (k.off[0] + 8 * bq < k.off[2]) k_batch(k.off, k.off[0] + 8 * bq, k.x[bq], k.cc[bq], r.q[bq], so);
-        for (int bs = k.off[0] + 8 * kKPre; bs < k.off[2]; bs += 8) {      // more than the prefetched batches: rare
-            uint4v x;
-            uint2 q[2];
-            uint32_t cc;
-            k_load(bs, x, cc);
-            k_qrows(k_fix_cc(bs, cc), q);
-            k_batch(k.off, bs, x, cc, q, so);
-        }
-    };
-    // V side, also from the entry list, sixteen entries of the half-step per batch (lane 16 * grp + col holds
-    // entry `col`):
-    //   Pg[e][column] = qmax P[token(e)][column] one 16x16x32 MFMA: A = the unit vector of the entry's token slot (LDS
-    //                                            rows), B = qmax P of the 32 tokens (verbatim chunks go through the
-    //                                            epilogue's 1 / qmax like the others), already in fp16: exact;
-    //   for every chunk position j in use:       X_j^T by the transposing MFMA (A = the entry's chunk in the row
-    //   acc[j] += X_j^T . Pg                     group that owns it, else zero), then one 16x16x16 MFMA over entries.
-    // the selector row of the lane's entry (A operand of the MFMA that gathers the probabilities), read ahead of use
-    auto v_sel = [&](const int (&off)[3], int bs, uint32_t cc) {
-        const int e = bs + col;
-        const uint32_t t = (cc >> 8) & 15u;
-        const uint32_t slot = (e >= off[1] ? 4u : 0u) + (t & 3u);             // position among the row group's 8 tokens
-        const bool mine = e < off[2] && (int)(t >> 2) == grp;
-        return *(lds_u4_ptr)(uintptr_t)(SELOFF + (mine ? slot : 8u) * 16u);
-    };
-    auto v_batch = [&](const int (&off)[3], int bs, uint2 x, uint32_t cc, uint4v sel, half8 ppo) {
-        const int e = bs + col;
-        const uint32_t ch = cc & (uint32_t)(n - 1);
-        const half4 pg = pack4(__builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sel), ppo, zero4, 0, 0, 0));
-        half4 h = zero_h4;
-        if constexpr (!kBfEntries) h = chunk_to_half<DT>(x);
-        const bool owner = e < off[2] && (int)(ch / CPL) == grp;
-        const int jq = (int)(ch % CPL);
-        // every chunk position, no test whether the batch meets it: straight-line code measures faster than skipping
-        // the positions without an entry (the matrix unit is idle here, and a wave-uniform branch costs more than two MFMAs)
-#pragma unroll
-        for (int j = 0; j < CPL; j++) {
-            const bool mj = owner && jq == j;
-            float4v tr;
-            if constexpr (kBfEntries)
-                tr = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4v, mj ? x : uint2{0u, 0u}), ident_bf, zero4, 0, 0, 0);
-            else
-                tr = __builtin_amdgcn_mfma_f32_16x16x16f16(mj ? h : zero_h4, ident, zero4, 0, 0, 0);
-            acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x16f16(pack4(tr), pg, acc[0][j], 0, 0, 0);
-        }
-    };
-    struct VSel {
-        uint4v s[kVPre];
-    };
-    auto v_prepare = [&](const VPre<kVPre> &v, VSel &r) {
-#pragma unroll
-        for (int bq = 0; bq < kVPre; bq++) r.s[bq] = v_sel(v.off, v.off[0] + 16 * bq, v.cc[bq]);
-    };
-    auto v_apply = [&](const VPre<kVPre> &v, const VSel &r, half8 ppo) {
-#pragma unroll
-        for (int bq = 0; bq < kVPre; bq++)
-            if (v.off[0] + 16 * bq < v.off[2]) v_batch(v.off, v.off[0] + 16 * bq, v.x[bq], v.cc[bq], r.s[bq], ppo);
-        for (int bs = v.off[0] + 16 * kVPre; bs < v.off[2]; bs += 16) {     // more than the prefetched batches: rare
+    auto stage_entries = [&](const Entries &q, int u0, bool v) {
+        const int e = q.off[0] + lane;
+        const uint32_t at = entry_at(q.off, e, q.cc);
+        if (mine(q.off, u0, e)) *(lds_w2_ptr)(uintptr_t)at = __builtin_bit_cast(uint2v_t, verbatim(q.x, v));
+        for (int bs = q.off[0] + 64; bs < q.off[2]; bs += 64) {             // more than 64: rare
             uint2 x;
             uint32_t cc;
-            v_load(bs, x, cc);
-            v_batch(v.off, bs, x, cc, v_sel(v.off, bs, cc), ppo);
+            entry_load(v ? v_side : k_side, v ? v_coord : k_coord, q.off, bs + lane, x, cc);
+            if (mine(q.off, u0, bs + lane)) *(lds_w2_ptr)(uintptr_t)entry_at(q.off, bs + lane, cc) = __builtin_bit_cast(uint2v_t, verbatim(x, v));
         }
+        asm volatile("" ::: "memory");
+        return at;
+    };
+    auto unstage = [&](const Entries &q, int u0, uint32_t at) {
+        asm volatile("" ::: "memory");
+        if (mine(q.off, u0, q.off[0] + lane)) *(lds_w2_ptr)(uintptr_t)at = uint2v_t{0u, 0u};
+        if (q.off[2] - q.off[0] > 64) wipe();
+        asm volatile("" ::: "memory");
+    };
+    // K: A operands of S^T, as the main product has them
+    const uint32_t k_at = stage + swizzled((uint32_t)col, (uint32_t)(grp * CPL * 8));
+    auto k_operands = [&](int u, uint4v (&a)[CPL / 2]) {
+#pragma unroll
+        for (int jj = 0; jj < CPL / 2; jj++) a[jj] = *(lds_u4_ptr)(uintptr_t)((k_at ^ (uint32_t)(16 * jj)) + (uint32_t)(u % ST * STB));
+    };
+    auto k_products = [&](const uint4v (&a)[CPL / 2], float4v &so) {
+#pragma unroll
+        for (int jj = 0; jj < CPL / 2; jj++) {
+            if constexpr (kBfEntries) so = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[jj]), qb[jj], so, 0, 0, 0);
+            else so = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[jj]), qf[0][jj], so, 0, 0, 0);
+        }
+    };
+    // V: lane i of a group of 16 reads chunk (i % 4) CPL + j of token 4 grp + i / 4; the transposing read leaves it element i % 4 of
+    // chunk (i / 4) CPL + j of the four tokens: the rows of the main V product, tokens as P has them
+    const uint32_t v_at = stage + swizzled((uint32_t)(4 * grp + (col >> 2)), (uint32_t)((col & 3) * CPL * 8));
+    auto v_operands = [&](int u, half4 (&a)[CPL]) {
+        typedef short4v __attribute__((address_space(3))) *lds_s4;
+#pragma unroll
+        for (int j = 0; j < CPL; j++)
+            a[j] = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(uintptr_t)((v_at ^ (uint32_t)(16 * (j >> 1))) + (uint32_t)(8 * (j & 1) + u % ST * STB))));
     };
 
     // One half-step: 32 tokens (two tiles) through scores, online softmax and the V product.  A flagged chunk
     // carries radius code 0 in the main plane, so its decoded value is exactly zero and only the verbatim
     // value from the sideband contributes.
-    auto half_step = [&](const HalfTile<NW, AB, FLAGS> &h, int th, const KPre<kKPre> &kc, const VPre<kVPre> &vc) {
+    auto half_step = [&](const HalfTile<NW, AB, FLAGS> &h, int th, const Entries &kc, const Entries &vc) {
         float4v sT[NCG][2], so[2] = {zero4, zero4};
-        // the LDS operands of the outlier batches are requested first and used after the main products
-        KRows kr;
-        VSel vr;
+        // the operands of the verbatim chunks are requested first and used after the main product
+        uint4v kv[2][CPL / 2];
         if constexpr (FLAGS) {
-            k_prepare(kc, kr);
-            v_prepare(vc, vr);
+#pragma unroll
+            for (int u0 = 0; u0 < 2; u0 += ST) {
+                const uint32_t at = stage_entries(kc, u0, false);
+#pragma unroll
+                for (int u = u0; u < u0 + ST; u++) k_operands(u, kv[u]);
+                unstage(kc, u0, at);
+            }
         }
         // every gather of the 32 K tokens is requested before the first one is used: the wavefront waits for LDS
         // once per half-step and tensor, not once per pair of chunks
@@ -881,7 +793,8 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         PHASE(1);
 #endif
         if constexpr (FLAGS) {
-            k_apply(kc, kr, so);
+#pragma unroll
+            for (int u = 0; u < 2; u++) k_products(kv[u], so[u]);
 #pragma unroll
             for (int u = 0; u < 2; u++)
 #pragma unroll
@@ -938,7 +851,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
                     l_run[cgi] += pe[e];
                 }
                 pT[u] = weigh<DT>(pe, h.vs[u]);
-                if constexpr (FLAGS) {          // for the verbatim chunks, see v_batch; qmax P is rounded to fp16 here and nowhere else
+                if constexpr (FLAGS) {          // for the verbatim chunks; qmax P is rounded to fp16 here and nowhere else
 #pragma unroll
                     for (int e = 0; e < 4; e++) pTo[u][e] = (_Float16)(pe[e] * qmaxf);
                 }
@@ -969,7 +882,18 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         asm volatile("" ::"v"(acc[0][0]), "v"(acc[0][CPL - 1]));
         PHASE(4);
 #endif
-        if constexpr (FLAGS) v_apply(vc, vr, cat8(pTo[0], pTo[1]));
+        if constexpr (FLAGS) {
+            half4 vv[2][CPL];
+#pragma unroll
+            for (int u0 = 0; u0 < 2; u0 += ST) {
+                const uint32_t at = stage_entries(vc, u0, true);
+#pragma unroll
+                for (int u = u0; u < u0 + ST; u++) v_operands(u, vv[u]);
+                unstage(vc, u0, at);
+            }
+#pragma unroll
+            for (int j = 0; j < CPL; j++) acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cat8(vv[0][j], vv[1][j]), cat8(pTo[0], pTo[1]), acc[0][j], 0, 0, 0);
+        }
 #ifdef HQMQ_STAMPS
         asm volatile("" ::"v"(acc[0][0]), "v"(acc[0][CPL - 1]));
         PHASE(5);
@@ -1029,12 +953,10 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         // Tile offsets travel two half-steps ahead, sideband entries one (their offsets were requested a step ago); past
         // the end the current tile is requested again.
         FastTile<NW, AB, FLAGS, NH> tile_b;
-        KPre<kKPre> k_b = {};
-        VPre<kVPre> v_b = {};
+        Entries k_b = {}, v_b = {};
         FlagTile f2 = {};
-        auto one = [&](int t0, const FastTile<NW, AB, FLAGS, NH> &tile_use, const KPre<kKPre> &k_use, const VPre<kVPre> &v_use,
-                       FastTile<NW, AB, FLAGS, NH> &tile_load, KPre<kKPre> &k_load_to, VPre<kVPre> &v_load_to, const FlagTile &f_use,
-                       FlagTile &f_load) {
+        auto one = [&](int t0, const FastTile<NW, AB, FLAGS, NH> &tile_use, const Entries &k_use, const Entries &v_use,
+                       FastTile<NW, AB, FLAGS, NH> &tile_load, Entries &k_load_to, Entries &v_load_to, const FlagTile &f_use, FlagTile &f_load) {
             const bool more = t0 + TS < t_end, more2 = t0 + 2 * TS < t_end;
 #ifdef HQMQ_STAMPS
             if (tl_ == 0) tl_ = t_loop_ = __builtin_amdgcn_s_memrealtime();
@@ -1461,8 +1383,8 @@ static int launch_one(const AttnParams &p, bool flags, dim3 grid, hipStream_t st
     if (NCG > 1) grid.y = (grid.y + NCG - 1) / NCG;
     // LDS: K table at 0, V table at kVTabOffset; reused afterwards for the cross-wave merge [wave][16][d_h + 4] floats
     constexpr bool PS = is_prescaled(MB, AB, IB);
-    size_t shmem = flags ? (size_t)sel_offset(PS) + 192 : PS ? (size_t)2 * kPsTabBytes : (size_t)kVTabOffset + (size_t)p.Vc.K * 8;
-    shmem += 64;        // the wavefronts' progress slots
+    size_t shmem = flags ? (size_t)stage_offset(PS) + (size_t)(CPL == 4 ? WV : kFastWaves) * stage_bytes(PS, CPL) : PS ? (size_t)2 * kPsTabBytes : (size_t)kVTabOffset + (size_t)p.Vc.K * 8;
+    if (!flags || !PS) shmem += 64;        // the wavefronts' progress slots
     const size_t merge = (size_t)WV * 16 * (16 * CPL + 4) * sizeof(float);     // WV >= the wavefronts actually launched
     if (shmem < merge) shmem = merge;
     constexpr int WF = CPL == 4 ? WV : kFastWaves;      // outlier variants fit three wavefronts per SIMD only at d_h 64
@@ -1517,7 +1439,7 @@ static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hip
     // Heads of 64 take these layouts here as well.  Before, the layout-generic kernel had them: 8 sequences x 3000 tokens, 64 / 8 heads,
     // 28.8 (s24_r3 fp16) to 47.3 us (s192_r6 bf16), with verbatim chunks 52 to 83, 40 queries each then 940 to 1350; now 14.3 to
     // 14.8, 16.7 to 17.3 and 133 to 142 us.  Tables multiplied out pay there too (4 x 32000 tokens 32.7 without them, 28.8 with).
-    if (mb == 12 && p.aux_bits == 1 && p.idx_bits == 10 && p.Kc.K <= 1024 && p.Vc.K <= 1024) {
+    if (mb == 12 && p.aux_bits == 1 && p.idx_bits == 10 && p.Kc.K <= 1024 && p.Vc.K <= (flags ? 1016 : 1024)) {
         if (two) return launch_one<CPL, 12, 1, 10, DT, kFastWaves, 2>(p, flags, grid, st, tm);
         return wide ? launch_one<CPL, 12, 1, 10, DT, 12>(p, flags, grid, st, tm) : launch_one<CPL, 12, 1, 10, DT>(p, flags, grid, st, tm);
     }
