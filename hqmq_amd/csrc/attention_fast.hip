@@ -13,8 +13,8 @@
 // P times the token's V scale is an fp32 product rounded to fp16 once, as in the other attention kernels; so is qmax P, the weight of
 // verbatim chunks.  Row j of the V-side product is d = (grp * CPL + j) * 4 + e, the order the epilogue writes back.
 // Scores are kept as S^T * rs; 1/qmax is folded into the softmax scale and the epilogue.  Outlier chunks
-// carry radius code 0 in the planes, so they decode to zero; their verbatim values enter through extra MFMAs
-// that walk the sideband entry list (values + coordinates), never the flag plane.
+// carry radius code 0 in the planes, so they decode to zero; their verbatim values, found through the sideband entry list (values +
+// coordinates, never the flag plane), enter through products of their own.
 #include "attention_mfma.h"
 #include <cstdlib>
 
@@ -687,7 +687,12 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const float4v zero4 = float4v{0.f, 0.f, 0.f, 0.f};
     // Verbatim chunks.  The wavefront writes a half-step's entries (K's, then V's) over zeros into rows of its own in LDS,
     // [token][chunk], reads them as whole matrix operands and clears what it wrote: its LDS accesses keep their order, so nothing
-    // has to be waited for but the data itself.  The chunks of a row are permuted by the token (16-byte parts, exclusive-or), so
+    // has to be waited for but the data itself.  The walk over the list in batches that this replaced (eight entries of K, sixteen of
+    // V the reduction dimension of a product, with masks, look-ups and a transposition per chunk position) was 173 of 567 vector
+    // instructions per half-step at d_h 128 and a chain of 40 matrix instructions; this is 60 and 16.  64 sequences of 1k to 16k, bf16
+    // s24_r3, 1.7 % of the chunks verbatim, one step 229 -> 188 us; 8 x 32768, 28 / 4 heads, s192_r6, 2 % of K's 53.0 -> 45.5; 4 x 131072,
+    // heads of 64, bf16, 1 % 94.2 -> 89.9; 8 x 16000, heads of 64, bf16 s24_r3 37.4 -> 32.4.  Without the test in front of V's part calls
+    // whose values have no outliers take 8 % longer (45.5 -> 48.8) and calls with both 1 to 2 % less (188 -> 185).  The chunks of a row are permuted by the token (16-byte parts, exclusive-or), so
     // that K's reads (16 tokens at the same part) and V's transposing ones (4 tokens at 4 parts) meet 64 different banks.
     typedef uint2v_t __attribute__((address_space(3))) *lds_w2_ptr;
     auto swizzled = [&](uint32_t row, uint32_t byte) {          // byte: 8 * chunk
@@ -882,7 +887,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         asm volatile("" ::"v"(acc[0][0]), "v"(acc[0][CPL - 1]));
         PHASE(4);
 #endif
-        if constexpr (FLAGS) {
+        if (FLAGS && vc.off[0] < vc.off[2]) {   // (tested for V only: keys have outliers far more often than values)
             half4 vv[2][CPL];
 #pragma unroll
             for (int u0 = 0; u0 < 2; u0 += ST) {
