@@ -3,12 +3,13 @@
 // of 16+1, 16+2, 12+2 or 12+3.
 //
 // Lane mapping (one wavefront, one 16-token tile): lane = 16 * grp + col decodes the CPL = d_h / 16 chunks
-// grp * CPL ... of token `col`, for K and for V alike.
+// grp * CPL ... of token `col` of K.
 //   S^T = K . Q^T     v_mfma_f32_16x16x32_f16: A = two decoded K chunks of the lane, B = the matching Q chunks.
-//   V^T               the A operand of O^T = V^T . P^T needs 4 tokens of one d per lane, a decoded chunk is
-//                     4 d of one token.  The 16x16 transposition is one v_mfma_f32_16x16x16_f16 against the
-//                     identity (exact: every output is one fp16 input times 1.0) and two packed conversions,
-//                     instead of a dozen cross-lane VALU operations per chunk.
+//   V^T               the A operand of O^T = V^T . P^T needs 4 tokens of one d per lane, a codeword is 4 d of one token: the
+//                     codewords and radius codes are gathered from LDS by transposing reads (gather_tokens), for which lane
+//                     4 * token + part holds the codes of a quarter of its token's chunks.  Float8 tables: lanes as for K,
+//                     transposed by one v_mfma_f32_16x16x16_f16 against the identity (exact: every output is one fp16 input
+//                     times 1.0) and two packed conversions per chunk.
 //   O^T += V^T . P^T  v_mfma_f32_16x16x32_f16 over two tiles (32 tokens) at a time.
 // P times the token's V scale is an fp32 product rounded to fp16 once, as in the other attention kernels; so is qmax P, the weight of
 // verbatim chunks.  Row j of the V-side product is d = (grp * CPL + j) * 4 + e, the order the epilogue writes back.
@@ -107,7 +108,9 @@ __device__ __forceinline__ uint32_t load_small(const uint8_t *p) {
 
 // The dynamic LDS block is the kernel's only LDS, so it starts at LDS address 0: the K table sits at byte 0,
 // the V table at kVTabOffset, and a gather addresses them with idx * 8 (+ the instruction's immediate offset).
-constexpr int kVTabOffset = 40960;          // bytes; room for 5120 K codewords in front of it
+constexpr int kTabMax = 5120;               // codewords the K slot has room for
+constexpr int kRadiusTabOffset = kTabMax * 8;           // 64 entries of 8 bytes: radius code rq as four fp16, see gather_tokens
+constexpr int kVTabOffset = kRadiusTabOffset + 512;
 constexpr int kStageOffset = kVTabOffset + 36864;       // outlier variants: staging rows of the wavefronts, after the V table
 constexpr int kFlagsTabMax = (kStageOffset - kVTabOffset) / 8;  // codewords the V slot of the outlier variants holds
 static_assert(kFlagsTabMax == 4608, "V table slot of the outlier variants");
@@ -173,7 +176,9 @@ __device__ __forceinline__ half4 gather_pair_half(uint32_t ix) {
 // 16+0 layout: the two radius codes of a dword become an fp16 pair with one shift, one and-or
 // (0x6400 | rq is the fp16 number 1024 + rq) and one packed subtract.  IB = idx_bits when known at compile
 // time (12 for s96), else 0.
-template <int CPL, int MB, int AB, int IB, int NW, int TAB_OFF, bool F8 = false>
+template <int OFF>
+__device__ __forceinline__ half4 gather8_tr(uint32_t byte_addr);
+template <int CPL, int MB, int AB, int IB, int NW, int TAB_OFF, bool F8 = false, bool TR = false>
 __device__ __forceinline__ void gather_chunks(const uint32_t (&w)[NW], uint32_t aux, int idx_bits_rt, half4 (&g)[CPL], half2v (&r)[CPL / 2]) {
     const int idx_bits = IB ? IB : idx_bits_rt;
     const uint32_t idx_mask = (1u << idx_bits) - 1u;
@@ -216,7 +221,11 @@ __device__ __forceinline__ void gather_chunks(const uint32_t (&w)[NW], uint32_t 
         const uint32_t ad[8] = {(w0 << 3) & M, (w0 >> 9) & M, __builtin_amdgcn_alignbit(w1, w0, 21) & M, (w1 >> 1) & M,
                                 (w1 >> 13) & M, __builtin_amdgcn_alignbit(w2, w1, 25) & M, (w2 >> 5) & M, (w2 >> 17) & M};
 #pragma unroll
-        for (int j = 0; j < CPL; j++) g[j] = gather8<TAB_OFF>(((aux << (15 - j)) & 0x8000u) | ad[j]);
+        for (int j = 0; j < CPL; j++) {
+            const uint32_t at = ((aux << (15 - j)) & 0x8000u) | ad[j];
+            if constexpr (TR) g[j] = gather8_tr<TAB_OFF>(at);
+            else g[j] = gather8<TAB_OFF>(at);
+        }
     } else {
         static_assert(!F8, "the float8 table variants exist for the layouts with compile-time index widths");
 #pragma unroll
@@ -232,6 +241,65 @@ template <int CPL, bool PS = false>
 __device__ __forceinline__ void scale_chunks(const half4 (&g)[CPL], const half2v (&r)[CPL / 2], half4 (&a)[CPL]) {
 #pragma unroll
     for (int j = 0; j < CPL; j++) a[j] = PS ? g[j] : g[j] * r[j >> 1][j & 1];
+}
+
+// V: the codewords arrive transposed.  ds_read_b64_tr_b16 takes an address per lane like any gather and then transposes 4 x 4 blocks of
+// 16-bit elements among 16 lanes: with lane i of a group of 16 asking for a codeword of token i / 4 it holds element i % 4 of that
+// lane group's chunk (of lane 4 t + i / 4) for the tokens t = 0..3 afterwards, which is the A operand of O^T = V^T . P^T.  The
+// radius codes have to be transposed too: a second gather, of a table whose entry rq is four times fp16(rq), hands them over in the
+// same places.  The products are the ones scale_chunks forms, rounded alike, and so are the outputs.  This replaced a product with the
+// identity (one matrix instruction and two packs of its fp32 results per chunk position and tile, 16 and 32 per half-step at d_h 128)
+// by as many LDS reads; what it took from the vector and matrix units is worth more than what it adds to LDS, which was busy 60 %.
+// One call before -> now: 64 sequences of 1k to 16k, bf16 s24_r3 with outliers (multiplied tables: no second gather), whole step
+// 193 -> 175 us; 4 x 131072, heads of 64, bf16 s96_r4 with outliers 94 -> 84.5; 8 x 32768, s192_r6 with outliers 49.4 -> 47.6;
+// 32768, s96_r4 13.4 -> 12.9.
+template <int OFF>
+__device__ __forceinline__ half4 gather8_tr(uint32_t byte_addr) {
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    typedef short4v __attribute__((address_space(3))) *lds_s4;
+    return __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(uintptr_t)(byte_addr + OFF)));
+}
+// (x's low / high 16 bits) >> SH in one instruction
+template <int HI>
+__device__ __forceinline__ uint32_t half_shr(uint32_t pair, int sh) {
+    uint32_t r;
+    if constexpr (HI)
+        asm("v_lshrrev_b32_sdwa %0, %2, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1" : "=v"(r) : "v"(pair), "s"(sh));
+    else
+        asm("v_lshrrev_b32_sdwa %0, %2, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0" : "=v"(r) : "v"(pair), "s"(sh));
+    return r;
+}
+template <int CPL, int MB, int AB, int IB, int NW, int TAB_OFF, int RAD_OFF>
+__device__ __forceinline__ void gather_tokens(const uint32_t (&w)[NW], uint32_t aux, int idx_bits_rt, half4 (&a)[CPL]) {
+    const int idx_bits = IB ? IB : idx_bits_rt;
+    const uint32_t idx_mask = (1u << idx_bits) - 1u;
+    if constexpr (is_prescaled(MB, AB, IB)) {
+        half2v unused[CPL / 2];
+        gather_chunks<CPL, MB, AB, IB, NW, TAB_OFF, false, true>(w, aux, idx_bits, a, unused);
+    } else if constexpr (MB == 16 && AB == 0) {
+        const uint32_t im2 = idx_mask * 0x00010001u, rm2 = ~im2;
+        const int sh = idx_bits - 3;                    // (a code has at least three index bits)
+#pragma unroll
+        for (int i = 0; i < CPL / 2; i++) {
+            const uint32_t ix = w[i] & im2, rx = w[i] & rm2;
+            a[2 * i] = gather8_tr<TAB_OFF>(half_addr8<0>(ix)) * gather8_tr<RAD_OFF>(half_shr<0>(rx, sh));
+            a[2 * i + 1] = gather8_tr<TAB_OFF>(half_addr8<1>(ix)) * gather8_tr<RAD_OFF>(half_shr<1>(rx, sh));
+        }
+    } else if constexpr (MB == 16 && AB == 3 && IB == 13) {
+        constexpr uint32_t im2 = 0x1fff1fffu;
+#pragma unroll
+        for (int j = 0; j < CPL; j++) {
+            const uint32_t ix = w[j / 2] & im2, lo = j & 1 ? w[j / 2] >> 26 : w[j / 2] >> 10, hi = 3 * j < 6 ? aux << (6 - 3 * j) : aux >> (3 * j - 6);
+            a[j] = gather8_tr<TAB_OFF>(j & 1 ? half_addr8<1>(ix) : half_addr8<0>(ix)) * gather8_tr<RAD_OFF>(((lo & 0x38u) | (hi & ~0x38u)) & 0x1f8u);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < CPL; j++) {
+            uint32_t code = code_at<MB, NW>(w, j);
+            if (AB) code |= ((aux >> (j * AB)) & ((1u << AB) - 1u)) << MB;
+            a[j] = gather8_tr<TAB_OFF>((code & idx_mask) << 3) * gather8_tr<RAD_OFF>((code >> idx_bits) << 3);
+        }
+    }
 }
 
 // max over the four 16-lane rows (lanes l, l^16, l^32, l^48) without going through LDS
@@ -371,7 +439,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     // codewords, all unconditional (clamped): straight-line code, exact wait counts.
     // (every pair of the largest table the LDS slots hold, 2560 pairs, in one round of requests: a second round would
     // be a loop of loads, and the wait at its head covers every request in flight, the first tile's included)
-    constexpr int FU = is_prescaled(MB, AB, IB) ? (512 + NT - 1) / NT : (kVTabOffset / 16 + NT - 1) / NT;
+    constexpr int FU = is_prescaled(MB, AB, IB) ? (512 + NT - 1) / NT : (kTabMax / 2 + NT - 1) / NT;
     const uint4v *ksrc = (const uint4v *)((const uint2 *)p.Kc.joint + hkv * (p.Kc.jsh / 4));
     const uint4v *vsrc = (const uint4v *)((const uint2 *)p.Vc.joint + hkv * (p.Vc.jsh / 4));
     const int Kk2 = p.Kc.K >> 1, Kv2 = p.Vc.K >> 1;        // tables of an even number of codewords (checked at launch)
@@ -457,6 +525,10 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     constexpr bool kAuxRow2 = CPL == 4 && AB == 1, kAuxRow6 = CPL == 4 && AB == 3;
     const uint32_t main_off = (uint32_t)(col * mrb + grp * NB), aux_off = (uint32_t)(col * arb + (kAuxRow2 ? 0 : kAuxRow6 ? (grp & 2) : grp * ABYTES));
     const uint32_t aux_sh = kAuxRow2 ? 4u * (uint32_t)grp : kAuxRow6 ? 12u * (uint32_t)grp - 8u * (uint32_t)(grp & 2) : 0u;
+    // V: lane 4 * token + chunk group, as gather_tokens has it (the float8 variants decode V like K and transpose it by matrix products)
+    const int vcol = F8 ? col : lane >> 2, vgrp = F8 ? grp : lane & 3;
+    const uint32_t vmain_off = (uint32_t)(vcol * mrb + vgrp * NB), vaux_off = (uint32_t)(vcol * arb + (kAuxRow2 ? 0 : kAuxRow6 ? (vgrp & 2) : vgrp * ABYTES));
+    const uint32_t vaux_sh = kAuxRow2 ? 4u * (uint32_t)vgrp : kAuxRow6 ? 12u * (uint32_t)vgrp - 8u * (uint32_t)(vgrp & 2) : 0u;
     auto load_aux_word = [&](const uint8_t *q) -> uint32_t {
         if constexpr (kAuxRow2) return *reinterpret_cast<const uint16_t *>(q);
         else if constexpr (kAuxRow6) return *reinterpret_cast<const uint32_a2 *>(q);
@@ -491,8 +563,8 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
             }
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                load_main(vb + main_off + u * 16 * mrb, h.vw[u]);
-                if constexpr (AB > 0) h.vaux[u] = load_aux_word(va_rows + (size_t)th * arb + aux_off + u * 16 * arb);
+                load_main(vb + vmain_off + u * 16 * mrb, h.vw[u]);
+                if constexpr (AB > 0) h.vaux[u] = load_aux_word(va_rows + (size_t)th * arb + vaux_off + u * 16 * arb);
                 h.vs[u] = *reinterpret_cast<const uint2 *>(vs_plane + th + scale_off + 16 * u);
             }
         }
@@ -600,7 +672,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     auto readable = [&](int t) { return min(t, (int)p.t_cap - 32); };
     FastTile<NW, AB, FLAGS, NH> tb;
     if constexpr (!FLAGS) load_super(readable(t_begin + TS < t_end ? t_begin + TS : t_begin), tb);
-    half4 ident;                        // B operand of the transposing MFMA: the 16x16 identity
+    half4 ident;                        // float8 variants, B operand of the transposing MFMA: the 16x16 identity
 #pragma unroll
     for (int e = 0; e < 4; e++) ident[e] = (_Float16)((4 * grp + e) == col ? 1.f : 0.f);
     // bf16 caches: K's verbatim chunks (and the Q they meet) go into bf16 MFMAs as they are stored; the products are exact
@@ -659,6 +731,12 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const uint32_t prog_base = FLAGS ? (uint32_t)flags_prog_offset(PS, CPL, WV) : PS ? 2u * (uint32_t)kPsTabBytes : (uint32_t)kVTabOffset + (uint32_t)p.Vc.K * 8u;
     typedef int __attribute__((address_space(3))) *lds_i32_ptr;
     if (threadIdx.x < 16) *(lds_i32_ptr)(uintptr_t)(prog_base + 4u * threadIdx.x) = 0;
+    if constexpr (!PS && !F8) {
+        if (threadIdx.x < 64) {
+            const half4 r = half4{1, 1, 1, 1} * (_Float16)(uint16_t)threadIdx.x;
+            lds_tab[kRadiusTabOffset / 8 + threadIdx.x] = __builtin_bit_cast(uint2, r);
+        }
+    }
     if constexpr (MB == 16 && AB == 3 && IB == 13) {
         if (threadIdx.x < 64) {
             const uint32_t b6 = threadIdx.x;
@@ -810,14 +888,6 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         asm volatile("" ::"v"(sT[0][0]), "v"(sT[0][1]));
         PHASE(2);
 #endif
-        // the V gathers fly while the softmax below keeps the vector unit busy
-        half4 gv[2][CPL];
-        half2v rv[2][CPL / 2];
-        if constexpr (kBatchGathers) {
-#pragma unroll
-            for (int u = 0; u < 2; u++) gather_chunks<CPL, MB, AB, IB, NW, VTAB, F8>(h.vw[u], AB ? h.vaux[u] >> aux_sh : 0u, idx_bits, gv[u], rv[u]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
         // ---- mask (boundary half-steps only), online softmax, per column group ----
         const bool edge = !(th + 32 <= lim_min && th + 32 <= t_end && th >= col_start);
         half8 pp[NCG];
@@ -868,21 +938,29 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         PHASE(3);
 #endif
         // ---- O^T += V^T . P^T, both tiles in one MFMA (the 1/qmax of the radius is applied once, in the epilogue) ----
-        if constexpr (kBatchGathers) __builtin_amdgcn_sched_barrier(0);
-        half4 av[2][CPL];
+        half8 vt[CPL];
+        if constexpr (F8) {
+            half4 g[CPL], av[2][CPL];
+            half2v r[CPL / 2];
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            if constexpr (!kBatchGathers) gather_chunks<CPL, MB, AB, IB, NW, VTAB, F8>(h.vw[u], AB ? h.vaux[u] >> aux_sh : 0u, idx_bits, gv[u], rv[u]);
-            scale_chunks<CPL, PS>(gv[u], rv[u], av[u]);
+            for (int u = 0; u < 2; u++) {
+                gather_chunks<CPL, MB, AB, IB, NW, VTAB, F8>(h.vw[u], AB ? h.vaux[u] >> vaux_sh : 0u, idx_bits, g, r);
+                scale_chunks<CPL, PS>(g, r, av[u]);
+            }
+#pragma unroll
+            for (int j = 0; j < CPL; j++)
+                vt[j] = cat8(pack4(__builtin_amdgcn_mfma_f32_16x16x16f16(av[0][j], ident, zero4, 0, 0, 0)), pack4(__builtin_amdgcn_mfma_f32_16x16x16f16(av[1][j], ident, zero4, 0, 0, 0)));
+        } else {
+            half4 av[2][CPL];
+#pragma unroll
+            for (int u = 0; u < 2; u++) gather_tokens<CPL, MB, AB, IB, NW, VTAB, kRadiusTabOffset>(h.vw[u], AB ? h.vaux[u] >> vaux_sh : 0u, idx_bits, av[u]);
+#pragma unroll
+            for (int j = 0; j < CPL; j++) vt[j] = cat8(av[0][j], av[1][j]);
         }
 #pragma unroll
-        for (int j = 0; j < CPL; j++) {
-            const float4v t0v = __builtin_amdgcn_mfma_f32_16x16x16f16(av[0][j], ident, zero4, 0, 0, 0);
-            const float4v t1v = __builtin_amdgcn_mfma_f32_16x16x16f16(av[1][j], ident, zero4, 0, 0, 0);
-            const half8 vt = cat8(pack4(t0v), pack4(t1v));
+        for (int j = 0; j < CPL; j++)
 #pragma unroll
-            for (int cgi = 0; cgi < NCG; cgi++) acc[cgi][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt, pp[cgi], acc[cgi][j], 0, 0, 0);
-        }
+            for (int cgi = 0; cgi < NCG; cgi++) acc[cgi][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt[j], pp[cgi], acc[cgi][j], 0, 0, 0);
 #ifdef HQMQ_STAMPS
         asm volatile("" ::"v"(acc[0][0]), "v"(acc[0][CPL - 1]));
         PHASE(4);
@@ -1047,11 +1125,12 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 // No tile lives in registers while in flight (111 registers against 145 - 256).  The compiler neither sees these
 // loads nor counts them: every wait is written by hand (s_waitcnt vmcnt(n) lets the n youngest requests stay
 // outstanding; requests complete in order), and the kernel has no other vector loads before its epilogue.
-// LDS: K table at 0, V table at 18432, 4 KB of query rows, then per wavefront two slots of
+// LDS: K table at 0, V table at 18432, 4 KB of query rows, 512 bytes of radius codes, then per wavefront two slots of
 // [256 B scales: K tokens 0..31, V tokens 0..31, the same again][K rows of 32 tokens, 2 KB][V rows, 2 KB].
 constexpr int kLdVTab = 2304 * 8;
 constexpr int kLdQ = 2 * kLdVTab;
-constexpr int kLdSlot0 = kLdQ + 4096;
+constexpr int kLdRad = kLdQ + 4096;        // the radius codes, see gather_tokens
+constexpr int kLdSlot0 = kLdRad + 512;
 constexpr int kLdSlotBytes = 256 + 4096;
 
 template <int N>
@@ -1175,7 +1254,7 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
     // instruction offsets count for the memory and the LDS side alike: the bases are moved back by the slot offsets
     const uint8_t *k_rows = p.Kc.main_plane + plane_row0 * mrb - 256;
     const uint8_t *v_rows = p.Vc.main_plane + plane_row0 * mrb - 2304;
-    const uint32_t main_off = (uint32_t)(col * mrb + grp * 16);
+    const uint32_t main_off = (uint32_t)(col * mrb + grp * 16), vmain_off = 16u * (uint32_t)lane;    // V: see gather_tokens
     // scales: lanes 0..15 fetch the K scales of tokens 2 lane, 2 lane + 1, lanes 16..31 the V scales; the upper half repeats
     const uint8_t *sc_lane = (lane & 16) ? (const uint8_t *)((const uint16_t *)p.Vc.scale_plane + b * p.Vc.ssb + hkv * p.Vc.ssh)
                                          : (const uint8_t *)((const uint16_t *)p.Kc.scale_plane + b * p.Kc.ssb + hkv * p.Kc.ssh);
@@ -1188,9 +1267,9 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
                      "global_load_lds_dwordx4 %2, %3 offset:256\n\t"
                      "global_load_lds_dwordx4 %2, %3 offset:1280\n\t"
                      "global_load_lds_dword %1, off\n\t"
-                     "global_load_lds_dwordx4 %2, %4 offset:2304\n\t"
-                     "global_load_lds_dwordx4 %2, %4 offset:3328"
-                     ::"s"(slot_lds), "v"(sa), "v"(main_off), "s"(kb), "s"(vb) : "memory");
+                     "global_load_lds_dwordx4 %5, %4 offset:2304\n\t"
+                     "global_load_lds_dwordx4 %5, %4 offset:3328"
+                     ::"s"(slot_lds), "v"(sa), "v"(main_off), "s"(kb), "s"(vb), "v"(vmain_off) : "memory");
     };
     // ---- query rows (first wavefront): column c of the block at kLdQ + 256 c, raw 16-bit values ----
     if (wave == 0) {
@@ -1205,9 +1284,11 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
     // the first half-step; the later ones are requested from inside the loop, one ahead
     if (n_hs > 0) request(t_begin, slot_base);
     STAMP(2);
-    half4 ident;
-#pragma unroll
-    for (int e = 0; e < 4; e++) ident[e] = (_Float16)((4 * grp + e) == col ? 1.f : 0.f);
+    if (threadIdx.x < 64) {
+        const half4 r = half4{1, 1, 1, 1} * (_Float16)(uint16_t)threadIdx.x;
+        lds_tab[kLdRad / 8 + threadIdx.x] = __builtin_bit_cast(uint2, r);
+        __builtin_amdgcn_s_waitcnt(0xc07f);         // lgkmcnt(0): the store is in LDS
+    }
     wait_groups(n_hs > 0 ? 1 : 0);            // tables (and query rows) in: only the tile request may still be outstanding
     STAMP(3);
     asm volatile("s_barrier" ::: "memory");
@@ -1322,18 +1403,11 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
         half4 av[2][CPL];
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            half4 g[CPL];
-            half2v r[CPL / 2];
             const uint32_t w[NW] = {vw[u][0], vw[u][1], vw[u][2], vw[u][3]};
-            gather_chunks<CPL, 16, 0, IB, NW, kLdVTab, false>(w, 0u, idx_bits, g, r);
-            scale_chunks<CPL, false>(g, r, av[u]);
+            gather_tokens<CPL, 16, 0, IB, NW, kLdVTab, kLdRad>(w, 0u, idx_bits, av[u]);
         }
 #pragma unroll
-        for (int j = 0; j < CPL; j++) {
-            const float4v t0v = __builtin_amdgcn_mfma_f32_16x16x16f16(av[0][j], ident, zero4, 0, 0, 0);
-            const float4v t1v = __builtin_amdgcn_mfma_f32_16x16x16f16(av[1][j], ident, zero4, 0, 0, 0);
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cat8(pack4(t0v), pack4(t1v)), pp, acc[j], 0, 0, 0);
-        }
+        for (int j = 0; j < CPL; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cat8(av[0][j], av[1][j]), pp, acc[j], 0, 0, 0);
 #ifdef HQMQ_STAMPS
         asm volatile("" ::"v"(acc[0]), "v"(acc[7]));
         { const unsigned long long t_ = __builtin_amdgcn_s_memrealtime();
@@ -1404,7 +1478,7 @@ static int launch_one(const AttnParams &p, bool flags, dim3 grid, hipStream_t st
 
 template <int CPL, int DT>
 static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hipStream_t st, const LaunchTiming &tm, bool *handled) {
-    if (p.Kc.K > kVTabOffset / 8 || p.Vc.K > kVTabOffset / 8) return HQMQ_OK;     // tables beyond the fixed LDS slots
+    if (p.Kc.K > kTabMax || p.Vc.K > kTabMax) return HQMQ_OK;     // tables beyond the fixed LDS slots
     // the kernels divide by multiplication only (fast_div): sizes for which a multiplier cannot be promised (index times
     // divisor beyond 2^32: millions of tokens times thousands of splits) stay with the layout-generic kernel
     if ((p.Hkv > 1 && !p.m_hkv) || (p.G > 1 && !p.m_G) || (p.n_splits > 1 && !p.m_splits)) return HQMQ_OK;
