@@ -115,11 +115,15 @@ constexpr int kStageOffset = kVTabOffset + 36864;       // outlier variants: sta
 constexpr int kFlagsTabMax = (kStageOffset - kVTabOffset) / 8;  // codewords the V slot of the outlier variants holds
 static_assert(kFlagsTabMax == 4608, "V table slot of the outlier variants");
 constexpr int kAuxTabOffset = 36864;        // s192_r6: 64 dwords with the high radius bits of a pair of chunks, see gather_chunks
-// s24_r3 (13-bit codes, K <= 1024, qmax = 7): the tables are kept multiplied out, entry [rq][idx] = codeword * rq at byte
+// s24_r3 (13-bit codes, K <= 1022, qmax = 7): the tables are kept multiplied out, entry [rq][idx] = codeword * rq at byte
 // (rq << 10 | idx) * 8, so that the 13-bit code is the table index and a decode is one gather (no radius arithmetic).
 constexpr int kPsTabBytes = 8 * 1024 * 8;   // 64 KB per tensor
+// The V table starts two entries before the K table's end (K <= 1022: they are free): an LDS instruction's immediate offset ends at 65535,
+// beyond which every address takes an addition of its own (16 + 16 of some 330 vector instructions per half-step at d_h 128).
+constexpr int kPsVTabOffset = kPsTabBytes - 16;
+constexpr int kPsKMax = 1022;
 constexpr bool is_prescaled(int MB, int AB, int IB) { return MB == 12 && AB == 1 && IB == 10; }
-constexpr int vtab_offset(bool ps) { return ps ? kPsTabBytes : kVTabOffset; }
+constexpr int vtab_offset(bool ps) { return ps ? kPsVTabOffset : kVTabOffset; }
 // Outlier variants: a wavefront's staging rows hold this many 16-token tiles (beside the multiplied tables there is room for one)
 constexpr int stage_offset(bool ps) { return ps ? 2 * kPsTabBytes : kStageOffset; }
 constexpr int stage_tiles(bool ps) { return ps ? 1 : 2; }
@@ -680,7 +684,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 
     {
         if constexpr (PS) {
-            // tables multiplied out: codeword * rq for rq = 0..7 at (rq << 10 | idx) * 8 (K <= 1024: FU * NT pairs cover it)
+            // tables multiplied out: codeword * rq for rq = 0..7 at (rq << 10 | idx) * 8 (K <= 1022: FU * NT pairs cover it)
 #pragma unroll
             for (int u = 0; u < FU; u++) {
                 const int k = threadIdx.x + u * NT;
@@ -1287,9 +1291,9 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
     if (threadIdx.x < 64) {
         const half4 r = half4{1, 1, 1, 1} * (_Float16)(uint16_t)threadIdx.x;
         lds_tab[kLdRad / 8 + threadIdx.x] = __builtin_bit_cast(uint2, r);
-        __builtin_amdgcn_s_waitcnt(0xc07f);         // lgkmcnt(0): the store is in LDS
     }
     wait_groups(n_hs > 0 ? 1 : 0);            // tables (and query rows) in: only the tile request may still be outstanding
+    __builtin_amdgcn_s_waitcnt(0xc07f);         // lgkmcnt(0): the radius codes are in LDS
     STAMP(3);
     asm volatile("s_barrier" ::: "memory");
     if constexpr (DT != HQMQ_F16) {
@@ -1518,7 +1522,7 @@ static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hip
     // Heads of 64 take these layouts here as well.  Before, the layout-generic kernel had them: 8 sequences x 3000 tokens, 64 / 8 heads,
     // 28.8 (s24_r3 fp16) to 47.3 us (s192_r6 bf16), with verbatim chunks 52 to 83, 40 queries each then 940 to 1350; now 14.3 to
     // 14.8, 16.7 to 17.3 and 133 to 142 us.  Tables multiplied out pay there too (4 x 32000 tokens 32.7 without them, 28.8 with).
-    if (mb == 12 && p.aux_bits == 1 && p.idx_bits == 10 && p.Kc.K <= 1024 && p.Vc.K <= (flags ? 1016 : 1024)) {
+    if (mb == 12 && p.aux_bits == 1 && p.idx_bits == 10 && p.Kc.K <= kPsKMax && p.Vc.K <= (flags ? 1016 : kPsKMax)) {
         if (two) return launch_one<CPL, 12, 1, 10, DT, kFastWaves, 2>(p, flags, grid, st, tm);
         return wide ? launch_one<CPL, 12, 1, 10, DT, 12>(p, flags, grid, st, tm) : launch_one<CPL, 12, 1, 10, DT>(p, flags, grid, st, tm);
     }
