@@ -109,8 +109,9 @@ __device__ __forceinline__ uint32_t load_small(const uint8_t *p) {
 // The dynamic LDS block is the kernel's only LDS, so it starts at LDS address 0: the K table sits at byte 0,
 // the V table at kVTabOffset, and a gather addresses them with idx * 8 (+ the instruction's immediate offset).
 constexpr int kTabMax = 5120;               // codewords the K slot has room for
-constexpr int kRadiusTabOffset = kTabMax * 8;           // 64 entries of 8 bytes: radius code rq as four fp16, see gather_tokens
-constexpr int kVTabOffset = kRadiusTabOffset + 512;
+constexpr int kRadiusCodes = 256;           // radius codes have at most 8 bits
+constexpr int kRadiusTabOffset = kTabMax * 8;           // 8 bytes a code: rq as four fp16, see gather_tokens
+constexpr int kVTabOffset = kRadiusTabOffset + 8 * kRadiusCodes;
 constexpr int kStageOffset = kVTabOffset + 36864;       // outlier variants: staging rows of the wavefronts, after the V table
 constexpr int kFlagsTabMax = (kStageOffset - kVTabOffset) / 8;  // codewords the V slot of the outlier variants holds
 static_assert(kFlagsTabMax == 4608, "V table slot of the outlier variants");
@@ -736,7 +737,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     typedef int __attribute__((address_space(3))) *lds_i32_ptr;
     if (threadIdx.x < 16) *(lds_i32_ptr)(uintptr_t)(prog_base + 4u * threadIdx.x) = 0;
     if constexpr (!PS && !F8) {
-        if (threadIdx.x < 64) {
+        if (threadIdx.x < kRadiusCodes) {
             const half4 r = half4{1, 1, 1, 1} * (_Float16)(uint16_t)threadIdx.x;
             lds_tab[kRadiusTabOffset / 8 + threadIdx.x] = __builtin_bit_cast(uint2, r);
         }
@@ -1129,12 +1130,12 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 // No tile lives in registers while in flight (111 registers against 145 - 256).  The compiler neither sees these
 // loads nor counts them: every wait is written by hand (s_waitcnt vmcnt(n) lets the n youngest requests stay
 // outstanding; requests complete in order), and the kernel has no other vector loads before its epilogue.
-// LDS: K table at 0, V table at 18432, 4 KB of query rows, 512 bytes of radius codes, then per wavefront two slots of
+// LDS: K table at 0, V table at 18432, 4 KB of query rows, 2 KB of radius codes, then per wavefront two slots of
 // [256 B scales: K tokens 0..31, V tokens 0..31, the same again][K rows of 32 tokens, 2 KB][V rows, 2 KB].
 constexpr int kLdVTab = 2304 * 8;
 constexpr int kLdQ = 2 * kLdVTab;
 constexpr int kLdRad = kLdQ + 4096;        // the radius codes, see gather_tokens
-constexpr int kLdSlot0 = kLdRad + 512;
+constexpr int kLdSlot0 = kLdRad + 8 * kRadiusCodes;
 constexpr int kLdSlotBytes = 256 + 4096;
 
 template <int N>
@@ -1288,7 +1289,7 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
     // the first half-step; the later ones are requested from inside the loop, one ahead
     if (n_hs > 0) request(t_begin, slot_base);
     STAMP(2);
-    if (threadIdx.x < 64) {
+    if (threadIdx.x < kRadiusCodes) {
         const half4 r = half4{1, 1, 1, 1} * (_Float16)(uint16_t)threadIdx.x;
         lds_tab[kLdRad / 8 + threadIdx.x] = __builtin_bit_cast(uint2, r);
     }
