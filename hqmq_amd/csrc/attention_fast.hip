@@ -404,6 +404,9 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     static_assert(NB % 4 == 0 || NB == 6, "main bytes of one lane");
     static_assert(CPL % 2 == 0, "two chunks per 16x16x32 operand");
     constexpr int NT = WV * 64;
+    // Outlier variants gather V before the softmax, whose exponentials then cover the LDS reads (64 sequences of 1k to 16k, bf16 s24_r3, one
+    // call 157.2 -> 153.9 us, 8 x 32768, s192_r6 46.4 -> 45.0); the plain ones, at three wavefronts per SIMD, would spill (111 -> 195 us).
+    constexpr bool kEarlyV = FLAGS && !F8;
     constexpr bool kBatchGathers = false;       // see half_step: measured, no gain on any shape (178 against 157 registers)
     constexpr int NH = 1;       // half-steps per prefetched tile: one measures faster than two on every shape
     extern __shared__ uint2 lds_tab[];
@@ -553,34 +556,35 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const char *k_coord = FLAGS ? (const char *)p.Kc.sb_coord + (size_t)bh * p.Kc.sb_cap * 2 : nullptr;
     const char *v_coord = FLAGS ? (const char *)p.Vc.sb_coord + (size_t)bh * p.Vc.sb_cap * 2 : nullptr;
 
+    auto load_k = [&](int th, HalfTile<NW, AB, FLAGS> &h) {
+        const uint8_t *kb = k_rows + (size_t)th * mrb;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            load_main(kb + main_off + u * 16 * mrb, h.kw[u]);
+            if constexpr (AB > 0) h.kaux[u] = load_aux_word(ka_rows + (size_t)th * arb + aux_off + u * 16 * arb);
+            h.ks[u] = *reinterpret_cast<const uint2 *>(ks_plane + th + scale_off + 16 * u);
+        }
+    };
+    auto load_v = [&](int th, HalfTile<NW, AB, FLAGS> &h) {
+        const uint8_t *vb = v_rows + (size_t)th * mrb;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            load_main(vb + vmain_off + u * 16 * mrb, h.vw[u]);
+            if constexpr (AB > 0) h.vaux[u] = load_aux_word(va_rows + (size_t)th * arb + vaux_off + u * 16 * arb);
+            h.vs[u] = *reinterpret_cast<const uint2 *>(vs_plane + th + scale_off + 16 * u);
+        }
+    };
     auto load_super = [&](int t0, FastTile<NW, AB, FLAGS, NH> &s) {
         // in the order the half-steps consume them: K, then V, of tokens 0..31, then the same of tokens 32..63
 #pragma unroll
         for (int hh = 0; hh < NH; hh++) {
-            const int th = t0 + 32 * hh;
-            const uint8_t *kb = k_rows + (size_t)th * mrb, *vb = v_rows + (size_t)th * mrb;
-            HalfTile<NW, AB, FLAGS> &h = s.h[hh];
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                load_main(kb + main_off + u * 16 * mrb, h.kw[u]);
-                if constexpr (AB > 0) h.kaux[u] = load_aux_word(ka_rows + (size_t)th * arb + aux_off + u * 16 * arb);
-                h.ks[u] = *reinterpret_cast<const uint2 *>(ks_plane + th + scale_off + 16 * u);
-            }
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                load_main(vb + vmain_off + u * 16 * mrb, h.vw[u]);
-                if constexpr (AB > 0) h.vaux[u] = load_aux_word(va_rows + (size_t)th * arb + vaux_off + u * 16 * arb);
-                h.vs[u] = *reinterpret_cast<const uint2 *>(vs_plane + th + scale_off + 16 * u);
-            }
+            load_k(t0 + 32 * hh, s.h[hh]);
+            load_v(t0 + 32 * hh, s.h[hh]);
         }
     };
 
-    // Tile offsets of one half-step, in two parts.  The loads (of wave-uniform addresses) are requested two half-steps
-    // ahead; their clamping happens only when flags_ready has let them through at the end of a half-step: placed right
-    // behind the loads it would wait for them with every later load in flight.
-    // The offsets are read through the constant address space (nothing writes them while this kernel runs), which
-    // makes them scalar loads: as vector loads of one address for all lanes, the six of a half-step took a memory
-    // pipeline slot each and came back through v_readfirstlane (config 4: 10 % of the launch).
+    // Tile offsets of the first two half-steps, in two parts: the loads (scalar ones, through the constant address space: nothing writes the
+    // offsets while this kernel runs), and their clamping once flags_ready has let them through.
     typedef const int32_t __attribute__((address_space(4))) *const_i32_ptr;
     const const_i32_ptr k_toff_c = (const_i32_ptr)(uintptr_t)k_toff, v_toff_c = (const_i32_ptr)(uintptr_t)v_toff;
     auto load_flags = [&](int th, FlagTile &f) {
@@ -611,6 +615,24 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         }
     };
 
+    // The same in the loop, as one vector load: lane i holds K's offset i (V's: lane 32 + i), read lane by lane when it has arrived.  Scalar
+    // loads share their counter with LDS and return out of order: with one outstanding every wait for LDS is a wait for everything.
+    const int lane_tile = min(lane & 31, 2), lane_count = lane & 32 ? v_count : k_count;
+    const int32_t *const lane_toff = lane & 32 ? v_toff : k_toff;
+    auto load_offsets = [&](int th) { return lane_toff[min((th >> 4) + lane_tile, tiles_cap1)]; };
+    auto offsets_ready = [&](int th, int w, FlagTile &f) {
+        w = min((th >> 4) + lane_tile <= tiles_cap1 ? w : 0x7fffffff, lane_count);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            f.koff[i] = __builtin_amdgcn_readlane(w, i);
+            f.voff[i] = __builtin_amdgcn_readlane(w, 32 + i);
+        }
+#pragma unroll
+        for (int i = 1; i < 3; i++) {
+            f.koff[i] = min(f.koff[i], f.koff[i - 1] + 16 * n);
+            f.voff[i] = min(f.voff[i], f.voff[i - 1] + 16 * n);
+        }
+    };
     // Every load of the loop is issued unconditionally (clamped addresses): a load inside a branch would make the
     // compiler's wait counts assume it was not issued, and the waits would then cover the next tile's prefetch.
     // The sideband entries of a half-step are a contiguous range known from three tile offsets, so no flag is read.  Lane i takes
@@ -620,6 +642,11 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         const uint32_t at = min((uint32_t)e, (uint32_t)max(off[2] - 1, 0));       // (inconsistent offsets of a caller may be negative)
         x = *reinterpret_cast<const uint2 *>(side + at * 8u);
         cc = *reinterpret_cast<const uint16_t *>(coord + at * 2u);
+    };
+    auto issue_one = [&](const char *side, const char *coord, const int (&off)[3], Entries &q) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) q.off[i] = off[i];
+        entry_load(side, coord, q.off, q.off[0] + lane, q.x, q.cc);
     };
     // sideband requests of one half-step
     auto issue_all = [&](const FlagTile &f, Entries &k, Entries &v) {
@@ -835,7 +862,8 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     // One half-step: 32 tokens (two tiles) through scores, online softmax and the V product.  A flagged chunk
     // carries radius code 0 in the main plane, so its decoded value is exactly zero and only the verbatim
     // value from the sideband contributes.
-    auto half_step = [&](const HalfTile<NW, AB, FLAGS> &h, int th, const Entries &kc, const Entries &vc) {
+    // next_*: the requests for the next half-step that take the place of what has just been used (outlier variants at d_h 64)
+    auto half_step = [&](const HalfTile<NW, AB, FLAGS> &h, int th, const Entries &kc, const Entries &vc, auto next_k_entries, auto next_k, auto next_v, auto next_v_entries) {
         float4v sT[NCG][2], so[2] = {zero4, zero4};
         // the operands of the verbatim chunks are requested first and used after the main product
         uint4v kv[2][CPL / 2];
@@ -847,6 +875,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
                 for (int u = u0; u < u0 + ST; u++) k_operands(u, kv[u]);
                 unstage(kc, u0, at);
             }
+            next_k_entries();
         }
         // every gather of the 32 K tokens is requested before the first one is used: the wavefront waits for LDS
         // once per half-step and tensor, not once per pair of chunks
@@ -888,11 +917,18 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 #pragma unroll
                 for (int e = 0; e < 4; e++)
                     sT[0][u][e] = scaled<DT>(sT[0][u][e], e < 2 ? h.ks[u].x : h.ks[u].y, e & 1, so[u][e] * qmaxf);
+            next_k();
         }
 #ifdef HQMQ_STAMPS
         asm volatile("" ::"v"(sT[0][0]), "v"(sT[0][1]));
         PHASE(2);
 #endif
+        half4 early[kEarlyV ? 2 : 1][CPL];
+        if constexpr (kEarlyV) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) gather_tokens<CPL, MB, AB, IB, NW, VTAB, kRadiusTabOffset>(h.vw[u], AB ? h.vaux[u] >> vaux_sh : 0u, idx_bits, early[u]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         // ---- mask (boundary half-steps only), online softmax, per column group ----
         const bool edge = !(th + 32 <= lim_min && th + 32 <= t_end && th >= col_start);
         half8 pp[NCG];
@@ -938,6 +974,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
             }
             pp[cgi] = cat8(pT[0], pT[1]);
         }
+        if constexpr (kEarlyV) next_v();
 #ifdef HQMQ_STAMPS
         asm volatile("" ::"v"(pp[0]));
         PHASE(3);
@@ -955,6 +992,9 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 #pragma unroll
             for (int j = 0; j < CPL; j++)
                 vt[j] = cat8(pack4(__builtin_amdgcn_mfma_f32_16x16x16f16(av[0][j], ident, zero4, 0, 0, 0)), pack4(__builtin_amdgcn_mfma_f32_16x16x16f16(av[1][j], ident, zero4, 0, 0, 0)));
+        } else if constexpr (kEarlyV) {
+#pragma unroll
+            for (int j = 0; j < CPL; j++) vt[j] = cat8(early[0][j], early[1][j]);
         } else {
             half4 av[2][CPL];
 #pragma unroll
@@ -962,6 +1002,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 #pragma unroll
             for (int j = 0; j < CPL; j++) vt[j] = cat8(av[0][j], av[1][j]);
         }
+        if constexpr (!kEarlyV) next_v();
 #pragma unroll
         for (int j = 0; j < CPL; j++)
 #pragma unroll
@@ -982,6 +1023,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 #pragma unroll
             for (int j = 0; j < CPL; j++) acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cat8(vv[0][j], vv[1][j]), cat8(pTo[0], pTo[1]), acc[0][j], 0, 0, 0);
         }
+        next_v_entries();
 #ifdef HQMQ_STAMPS
         asm volatile("" ::"v"(acc[0][0]), "v"(acc[0][CPL - 1]));
         PHASE(5);
@@ -1009,25 +1051,26 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 
     if constexpr (!FLAGS) {
         // ring of three tile buffers, every load unconditional (past the end the current tile is requested again)
+        auto nothing = [] {};
         FastTile<NW, AB, FLAGS, NH> tc;
         int t0 = t_begin;
         if (t0 < t_end) {
             while (true) {
                 load_super(readable(t0 + 2 * TS < t_end ? t0 + 2 * TS : t0), tc);
                 publish(t0);
-                half_step(cur.h[0], t0, kc, vc);
+                half_step(cur.h[0], t0, kc, vc, nothing, nothing, nothing, nothing);
                 rebalance(t0);
                 t0 += TS;
                 if (t0 >= t_end) break;
                 load_super(readable(t0 + 2 * TS < t_end ? t0 + 2 * TS : t0), cur);
                 publish(t0);
-                half_step(tb.h[0], t0, kc, vc);
+                half_step(tb.h[0], t0, kc, vc, nothing, nothing, nothing, nothing);
                 rebalance(t0);
                 t0 += TS;
                 if (t0 >= t_end) break;
                 load_super(readable(t0 + 2 * TS < t_end ? t0 + 2 * TS : t0), tb);
                 publish(t0);
-                half_step(tc.h[0], t0, kc, vc);
+                half_step(tc.h[0], t0, kc, vc, nothing, nothing, nothing, nothing);
                 rebalance(t0);
                 t0 += TS;
                 if (t0 >= t_end) break;
@@ -1035,38 +1078,50 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         }
     }
     if constexpr (FLAGS) {
-        // Outlier variants: one half-step in flight.  Two sets of buffers (tile, sideband entries, tile offsets) take
-        // turns, written out as two half-steps per round of the loop: with one set handed on at the end of every
-        // half-step (cur = nxt) the compiler copied some fifty registers per half-step.
-        // Tile offsets travel two half-steps ahead, sideband entries one (their offsets were requested a step ago); past
-        // the end the current tile is requested again.
+        // Outlier variants, tile offsets two half-steps ahead; past the end the current tile is requested again.  d_h 128: two sets of buffers
+        // (tile, entries) take turns, requested one half-step ahead and written out as two half-steps per round of the loop: with one set
+        // handed on (cur = nxt) the compiler copied some fifty registers per half-step.  d_h 64: one set, refilled piece by piece as a
+        // half-step uses it up (K's entries, K, V, V's entries: the order of their use).  Each form where it is the better one, caches read
+        // from HBM: 16 x 5000 tokens, heads of 64, bf16 s24_r3 24.5 us with two sets, 22.4 with one; 8 x 32768 tokens, 28 / 4 heads of 128,
+        // s96_r4 41.6 and 43.1; 64 sequences of 1k to 16k, 4 x 131072 tokens, heads of 64, alike.  (Twelve wavefronts of 168 registers
+        // at d_h 128, staging rows in the gaps of the multiplied tables, nothing spilled in the loop, s24_r3: 154.4 where eight take 152.3, and
+        // 175 against 163 with bf16 s96_r4: LDS is busy 60 % of the time, the vector units 64 %.)
         FastTile<NW, AB, FLAGS, NH> tile_b;
         Entries k_b = {}, v_b = {};
-        FlagTile f2 = {};
+        auto nothing = [] {};
+        constexpr bool kRefill = CPL == 4;
         auto one = [&](int t0, const FastTile<NW, AB, FLAGS, NH> &tile_use, const Entries &k_use, const Entries &v_use,
-                       FastTile<NW, AB, FLAGS, NH> &tile_load, Entries &k_load_to, Entries &v_load_to, const FlagTile &f_use, FlagTile &f_load) {
+                       FastTile<NW, AB, FLAGS, NH> &tile_load, Entries &k_load_to, Entries &v_load_to) {
             const bool more = t0 + TS < t_end, more2 = t0 + 2 * TS < t_end;
+            const int t1 = more ? t0 + TS : t0, t2 = more2 ? t0 + 2 * TS : t0;
 #ifdef HQMQ_STAMPS
             if (tl_ == 0) tl_ = t_loop_ = __builtin_amdgcn_s_memrealtime();
             n_steps_++;
 #endif
-            load_super(more ? t0 + TS : t0, tile_load);
-            load_flags(more2 ? t0 + 2 * TS : t0, f_load);           // made ready at the end of this half-step
-            issue_all(f_use, k_load_to, v_load_to);
+            auto next_ke = [&] { issue_one(k_side, k_coord, f1.koff, k_load_to); };
+            auto next_ve = [&] { issue_one(v_side, v_coord, f1.voff, v_load_to); };
+            if constexpr (!kRefill) load_super(t1, tile_load);
+            const int w = load_offsets(t2);
+            if constexpr (!kRefill) { next_ke(); next_ve(); }
             publish(t0);
             PHASE(0);
-            half_step(tile_use.h[0], t0, k_use, v_use);
+            if constexpr (kRefill) half_step(tile_use.h[0], t0, k_use, v_use, next_ke, [&] { load_k(t1, tile_load.h[0]); }, [&] { load_v(t1, tile_load.h[0]); }, next_ve);
+            else half_step(tile_use.h[0], t0, k_use, v_use, nothing, nothing, nothing, nothing);
             rebalance(t0);
-            if (more) flags_ready(more2 ? t0 + 2 * TS : t0, f_load);
+            offsets_ready(t2, w, f1);
             PHASE(6);
             return more;
         };
         if (t_begin < t_end) {
             int t0 = t_begin;
             while (true) {
-                if (!one(t0, cur, kc, vc, tile_b, k_b, v_b, f1, f2)) break;
-                t0 += TS;
-                if (!one(t0, tile_b, k_b, v_b, cur, kc, vc, f2, f1)) break;
+                if constexpr (kRefill) {
+                    if (!one(t0, cur, kc, vc, cur, kc, vc)) break;
+                } else {
+                    if (!one(t0, cur, kc, vc, tile_b, k_b, v_b)) break;
+                    t0 += TS;
+                    if (!one(t0, tile_b, k_b, v_b, cur, kc, vc)) break;
+                }
                 t0 += TS;
             }
         }
