@@ -1554,7 +1554,11 @@ static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hip
     // 1200 (3000 / 5500 tokens 26.1 -> 23.3 / 42.3 -> 36.3 us), d_h 64 plain 4000 (8000 tokens 34.4 -> 32.3 us), there only while no
     // compute unit holds two blocks of eight (480 blocks of 4000 tokens 33.3 against 38.2 us).
     const int range = p.Tkv / p.n_splits;
-    const bool wide = CPL == 8 ? !flags && range >= 4096 : flags ? range >= 1536 : range >= 4096 && (int64_t)grid.x * grid.y * grid.z <= 256;
+    // Where the kernel whose loads land in LDS can take the call it keeps it up to 5000 tokens (256 blocks of 4100 / 5000 / 6000 tokens of bf16
+    // s96_r4 32.9 / 41.5 / 48.1 us, twelve wavefronts 35.1 / 40.7 / 46.9).
+    const bool lands = CPL == 8 && mb == 16 && p.aux_bits == 0 && !flags && !p.no_lds_landing && p.Kc.K <= 2304 && p.Vc.K <= 2304 && p.Kc.K >= 2 && p.Vc.K >= 2 &&
+                       ((((uintptr_t)p.Q) | (uintptr_t)(p.qsb * 2) | (uintptr_t)(p.qsh * 2) | (uintptr_t)(p.qst * 2)) & 15) == 0;
+    const bool wide = CPL == 8 ? !flags && range >= (lands ? 5000 : 4096) : flags ? range >= 1536 : range >= 4096 && (int64_t)grid.x * grid.y * grid.z <= 256;
     const bool two = attn_two_groups(p.n_cg, flags, (int64_t)p.n_splits * p.n_cg * p.B * p.Hkv, range, p.n, p.aux_bits);
     // tables of e4m3 numbers kept as float8 in LDS, on request (decode shapes of the 16-bit layouts at d_h 128)
     if (p.tab_fp8 && CPL == 8 && !two) {
@@ -1563,8 +1567,7 @@ static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hip
     }
     // plain 16+0 caches with small tables at d_h 128, one column group, eight wavefronts: every load lands in LDS
     if constexpr (CPL == 8) {
-        if (mb == 16 && p.aux_bits == 0 && !flags && !two && !wide && !p.no_lds_landing && p.Kc.K <= 2304 && p.Vc.K <= 2304 && p.Kc.K >= 2 &&
-            p.Vc.K >= 2 && ((((uintptr_t)p.Q) | (uintptr_t)(p.qsb * 2) | (uintptr_t)(p.qsh * 2) | (uintptr_t)(p.qst * 2)) & 15) == 0)
+        if (lands && !two && !wide)
             return p.idx_bits == 12 ? launch_lds<DT, 12>(p, grid, st, tm) : launch_lds<DT, 0>(p, grid, st, tm);
     }
     if (mb == 16 && p.aux_bits == 0 && p.idx_bits == 12) {

@@ -16,7 +16,7 @@ def test_every_token_chunk_and_radius(S, b_r, d):
     from hqmq_amd import ops
     B, Hkv, G, n = 3, 2, 4, d // 4
     q = hqmq.HQMQ(n_layers=1, n_heads=Hkv, secondary_size=S, radius_bits=b_r, device="cuda")
-    for T, Tq, ns, med, dt in ((1, 1, 1, False, torch.float16), (77, 1, 1, False, torch.bfloat16), (333, 5, 2, True, torch.float16), (1100, 1, 1, True, torch.bfloat16)):
+    for T, Tq, ns, med, dt in ((1, 1, 1, False, torch.float16), (77, 1, 1, False, torch.bfloat16), (333, 5, 2, True, torch.float16), (1100, 1, 1, True, torch.bfloat16), (4600, 1, 1, False, torch.float16), (5003, 1, 1, False, torch.bfloat16)):
         g = torch.Generator().manual_seed(S + d + T)
         # norms spread over the whole range of a token's radius codes
         x = torch.nn.functional.normalize(torch.randn(2, B, Hkv, T, n, 4, generator=g), dim=-1) * torch.rand(2, B, Hkv, T, n, 1, generator=g)
