@@ -50,16 +50,7 @@ typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kPfV = 16384, kPfBuf = 32768, kPfScale = 2 * kPfBuf, kPfScaleV = 1024, kPfFlag = kPfScale + 2048;   // LDS: K | V, twice; scales; flags (FL); tables
-// (without FL, the word at kPfFlag is not zero once the block has met a V scale too large for weights above 1)
-constexpr uint32_t pf_tab(bool fl) { return kPfFlag + (fl ? 1024u : 128u); }
-
-// d_h 128 without FL: how far, in powers of two, a weight may pass 1 before sums and accumulators are scaled down to a new reference (117
-// vector instructions), while V's scales stay below kHeadroomScale, so that the products fit fp16; elsewhere weights stay at or below
-// 1.  (A weight above 1 is rounded as finely as one below, and sums are fp32.)  With the reference at the running maximum, which moves in
-// one of five units over 32768 tokens and more often over fewer: 2048 x 2048 causal, unpacked codes, 73.7 us, now 69.0; 2 x 512
-// queries on 6000 tokens, 28 / 4 heads, bf16 s192_r4 139 -> 132; 1024 on 32768 672 -> 664.  d_h 64, which has half the accumulators: 2 x 300
-// queries on 6000 tokens, s24_r3, 177 with the maximum, 181 without; FL, which multiplies twice: alike.  The decode kernels: alike.
-constexpr float kHeadroom = 4.f, kHeadroomScale = 2048.f;
+constexpr uint32_t pf_tab(bool fl) { return kPfFlag + (fl ? 1024u : 0u); }
 
 // permutation of a row's 16-byte parts
 template <int DH>
@@ -76,7 +67,6 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     constexpr int TILE = 8192 / DH, NSUB = TILE / 32 / KVG;              // tokens per tile; units of 32 of them per wavefront
     constexpr int TOK = DH == 128 ? 16 : 32;                             // tokens a wavefront decodes: 8 chunks per lane
     constexpr uint32_t kPfTab = pf_tab(FL);
-    constexpr bool ROOM = DH == 128 && !FL;
     extern __shared__ uint2 lds_tab[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5, col = lane & 31;
@@ -290,11 +280,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
             } else *(uint4v __attribute__((address_space(3))) *)(uintptr_t)(w_at ^ ((uint32_t)i << 4)) =
                 __builtin_bit_cast(uint4v, cat8(wg[2 * i] * wr[i][0], wg[2 * i + 1] * wr[i][1]));
             if (j == 7) {
-                if (w_lane) {
-                    *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = dec_v ? w_scale : w_scale * p.c_log2;
-                    // (to the word behind it if there is nothing to say: no branch in the unit's block)
-                    if (ROOM) *(uint32_t __attribute__((address_space(3))) *)(uintptr_t)(dec_v && !(w_scale < kHeadroomScale) ? kPfFlag : kPfFlag + 4u) = 1u;
-                }
+                if (w_lane) *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = dec_v ? w_scale : w_scale * p.c_log2;
                 if (FL) {
                     if (w_lane && !dec_v) *(uint32_t __attribute__((address_space(3))) *)(uintptr_t)(ws_at + (kPfFlag - kPfScale)) = 0u;
                     asm volatile("" ::: "memory");                        // the wavefront's LDS accesses keep their order
@@ -338,7 +324,6 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         }
     }
     if (it == 0) tables();
-    if (ROOM && tid == 0) *(uint32_t __attribute__((address_space(3))) *)(uintptr_t)kPfFlag = 0u;
     __syncthreads();
     if (work) {
 #pragma unroll
@@ -424,9 +409,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         for (int e = 4 * x; e < 4 * x + 4; e++) sn[e] = __builtin_fmaf(sn[e], ks[e & 3], __builtin_fmaf(svn[e], p.c_plain, neg_m));
     };
     // scores of a unit (first token tw): times their K scale, relative to the running maximum, which moves if it has to
-    // (by more than kHeadroom, where that is allowed)
-    auto large_scales = [&]() PF_INLINE { return ROOM ? *(lds_u1_ptr)(uintptr_t)kPfFlag : 0u; };
-    auto maxima = [&](int tw, const float4v (&ks)[4], uint32_t large) PF_INLINE {
+    auto maxima = [&](int tw, const float4v (&ks)[4]) PF_INLINE {
         const bool edge = !(tw + 32 <= wave_min && tw + 32 <= b_end && tw >= col_start);
         float tmax = -INFINITY;
 #pragma unroll
@@ -445,8 +428,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
             const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
             tmax = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
         }
-        const float room = ROOM && large == 0u ? kHeadroom : 0.f;
-        if (__builtin_amdgcn_ballot_w64(tmax > seen + room) != 0) {
+        if (__builtin_amdgcn_ballot_w64(tmax > seen) != 0) {
             const float d = tmax > seen ? tmax : 0.f;
             const float alpha = seen == 0.f ? __builtin_amdgcn_exp2f(-d) : 0.f;
             l_run *= alpha;
@@ -525,11 +507,10 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         s = sn;
         if (dec) __syncthreads();
         const bool over = u + 1 == NSUB;                                  // the next unit is the first one of the next tile
-        const uint32_t large = large_scales();                            // (first: LDS answers in order)
 #pragma unroll
         for (int i = 0; i < AHEAD; i++) kf[i] = k_load(over ? buf ^ 1u : buf, over ? 1 : u + 2, i);
         if (FL) kfl = f_load(over ? buf ^ 1u : buf, over ? 1 : u + 2);
-        maxima(over ? tw + 32 + TILE - 32 * NSUB : tw + 32, ks, large);
+        maxima(over ? tw + 32 + TILE - 32 * NSUB : tw + 32, ks);
     };
     auto tile = [&](int t0, uint32_t buf) PF_INLINE {
 #pragma unroll
@@ -553,7 +534,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
 #pragma unroll
         for (int i = 0; i < AHEAD; i++) kf[i] = k_load(0u, 1, i);
         if (FL) kfl = f_load(0u, 1);
-        maxima(b_begin + 32 * NSUB * kvg, ks, large_scales());
+        maxima(b_begin + 32 * NSUB * kvg, ks);
     }
     // (a wavefront whose columns end before the block's goes on with masked scores: it has to decode anyway)
     for (int t0 = b_begin; t0 < b_end;) {
