@@ -67,6 +67,32 @@ __device__ __forceinline__ void touch_kernargs() {
     asm volatile("" ::"s"(t));
 }
 
+// Loads that land in LDS.  The compiler neither sees nor counts them; loads come back in the order they were requested, so vmcnt(n) with n
+// no more than the loads requested after them waits for them.
+template <int N>
+__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+__device__ __forceinline__ const uint8_t *uniform_ptr(const uint8_t *p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (const uint8_t *)(((uint64_t)hi << 32) | lo);
+}
+// 64 lanes x 16 bytes from base + voff (+ the instruction's offset, which counts for both sides) to LDS at m0 + 16 * lane
+__device__ __forceinline__ void lds_load16(uint32_t lds_base, const uint8_t *base, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(base) : "memory");
+}
+// The K and V codeword tables in 1 KB units dealt to the wavefronts round-robin, straight to their places in LDS (whole units: the last
+// pair of codewords again past a table's end).
+template <int WV>
+__device__ __forceinline__ void land_tables(const uint8_t *k, uint32_t kbytes, const uint8_t *v, uint32_t vbytes, uint32_t v_at, int wave, int lane) {
+    const int ku = (int)((kbytes + 1023u) >> 10), nu = ku + (int)((vbytes + 1023u) >> 10);
+    for (int u = wave; u < nu; u += WV) {
+        const bool isv = u >= ku;
+        const uint32_t uu = (uint32_t)(isv ? u - ku : u);
+        const uint32_t off = min(uu * 1024u + (uint32_t)lane * 16u, (isv ? vbytes : kbytes) - 16u);
+        lds_load16((isv ? v_at : 0u) + uu * 1024u, isv ? v : k, off);
+    }
+}
+
 constexpr int kFastWaves = 8;     // wavefronts per block; 12 (three per SIMD) with long ranges per block, see launch_layout
 
 // codes, aux bits and raw 16-bit scales of 32 tokens (two 16-token tiles) for one lane
@@ -405,8 +431,9 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     static_assert(CPL % 2 == 0, "two chunks per 16x16x32 operand");
     constexpr int NT = WV * 64;
     // Outlier variants gather V before the softmax, whose exponentials then cover the LDS reads (64 sequences of 1k to 16k, bf16 s24_r3, one
-    // call 157.2 -> 153.9 us, 8 x 32768, s192_r6 46.4 -> 45.0); the plain ones, at three wavefronts per SIMD, would spill (111 -> 195 us).
-    constexpr bool kEarlyV = FLAGS && !F8;
+    // call 157.2 -> 153.9 us, 8 x 32768, s192_r6 46.4 -> 45.0); the plain ones, at three wavefronts per SIMD, would spill (111 -> 195 us),
+    // and bf16 ones of 16 + 2 and 16 + 3 bits with the generic field decode.
+    constexpr bool kEarlyV = FLAGS && !F8 && !(CPL == 8 && DT == HQMQ_BF16 && MB == 16 && AB >= 2 && IB == 0);
     constexpr bool kBatchGathers = false;       // see half_step: measured, no gain on any shape (178 against 157 registers)
     constexpr int NH = 1;       // half-steps per prefetched tile: one measures faster than two on every shape
     extern __shared__ uint2 lds_tab[];
@@ -418,6 +445,11 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
 #endif
     constexpr bool PS = is_prescaled(MB, AB, IB);
     constexpr int VTAB = vtab_offset(PS);
+    // fp16 tables that stay as they are land in LDS where that is the better form, kernel in us through registers -> landing: outlier caches
+    // at d_h 128, s96_r4, 27 sequences of 222 tokens 9.1 -> 8.5, 8 of 2000 10.7 -> 9.8, s192_r6, 8 x 32768 48.4 -> 47.4 (4 x 1000 10.1 -> 10.3).
+    // Not so plain s192_r6 (1 x 2000 8.4 -> 8.7), heads of 64 (6 x 900, s192_r4 8.6 -> 9.2), bf16, which is converted in place behind a
+    // barrier of its own (64 / 8 heads of 64, 300 tokens, whole call 7.8 -> 9.1).
+    constexpr bool kLand = FLAGS && CPL == 8 && MB == 16 && IB != 0 && !F8 && DT == HQMQ_F16;
     uint2 *ktab = lds_tab, *vtab = lds_tab + VTAB / 8;
     touch_kernargs();
 
@@ -451,12 +483,16 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const uint4v *ksrc = (const uint4v *)((const uint2 *)p.Kc.joint + hkv * (p.Kc.jsh / 4));
     const uint4v *vsrc = (const uint4v *)((const uint2 *)p.Vc.joint + hkv * (p.Vc.jsh / 4));
     const int Kk2 = p.Kc.K >> 1, Kv2 = p.Vc.K >> 1;        // tables of an even number of codewords (checked at launch)
-    uint4v tk[FU], tv[FU];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint4v tk[kLand ? 1 : FU], tv[kLand ? 1 : FU];
+    if constexpr (kLand) land_tables<WV>(uniform_ptr((const uint8_t *)ksrc), 16u * (uint32_t)Kk2, uniform_ptr((const uint8_t *)vsrc), 16u * (uint32_t)Kv2, VTAB, wave, lane);
+    else {
 #pragma unroll
-    for (int u = 0; u < FU; u++) {
-        const int k = threadIdx.x + u * NT;
-        tk[u] = ksrc[min(k, Kk2 - 1)];
-        tv[u] = vsrc[min(k, Kv2 - 1)];
+        for (int u = 0; u < FU; u++) {
+            const int k = threadIdx.x + u * NT;
+            tk[u] = ksrc[min(k, Kk2 - 1)];
+            tv[u] = vsrc[min(k, Kv2 - 1)];
+        }
     }
 #ifdef HQMQ_STAMPS
     ph_[0] = __builtin_amdgcn_s_memrealtime();      // table loads requested
@@ -464,7 +500,6 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const int b = p.batch_order ? min(max(uniform_word(p.batch_order, slot), 0), p.B - 1) : slot;
     const int bh = b * p.Hkv + hkv;
     const int cg0 = by * NCG, sp = bx;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int G = p.G;
     constexpr int n = 4 * CPL, d_h = 16 * CPL;
     const int col = lane & 15, grp = lane >> 4;
@@ -725,7 +760,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
                     if (k < Kv2) reinterpret_cast<uint4v *>(vtab)[rq * 512 + k] = uint4v{mul(hv[0]), mul(hv[1]), mul(hv[2]), mul(hv[3])};
                 }
             }
-        } else {
+        } else if constexpr (!kLand) {
 #pragma unroll
             for (int u = 0; u < FU; u++) {
                 const int k = threadIdx.x + u * NT;
@@ -775,6 +810,8 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
             reinterpret_cast<uint32_t *>(lds_tab)[kAuxTabOffset / 4 + b6] = ((b6 & 7u) << 3) | ((b6 >> 3) << 19) | 0x64006400u;
         }
     }
+    // tables in: behind them were requested the queries, the first tile and its entries, at least this many loads
+    if constexpr (kLand) wait_vm<CPL / 2 + 8 + 4>();
 #ifdef HQMQ_STAMPS
     const unsigned long long t_fill_ = __builtin_amdgcn_s_memrealtime();
 #endif
@@ -1193,23 +1230,12 @@ constexpr int kLdRad = kLdQ + 4096;        // the radius codes, see gather_token
 constexpr int kLdSlot0 = kLdRad + 8 * kRadiusCodes;
 constexpr int kLdSlotBytes = 256 + 4096;
 
-template <int N>
-__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 // wait until at most `groups` (0..3) groups of five requests are outstanding
 __device__ __forceinline__ void wait_groups(int groups) {
     if (groups >= 3) wait_vm<15>();
     else if (groups == 2) wait_vm<10>();
     else if (groups == 1) wait_vm<5>();
     else wait_vm<0>();
-}
-__device__ __forceinline__ const uint8_t *uniform_ptr(const uint8_t *p) {
-    const uint64_t v = (uint64_t)p;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (const uint8_t *)(((uint64_t)hi << 32) | lo);
-}
-// 64 lanes x 16 bytes from base + voff (+ the instruction's offset, which counts for both sides) to LDS at m0 + 16 * lane
-__device__ __forceinline__ void lds_load16(uint32_t lds_base, const uint8_t *base, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(base) : "memory");
 }
 __device__ __forceinline__ void lds_load16_addr(uint32_t lds_base, const uint8_t *addr) {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(addr) : "memory");
@@ -1260,18 +1286,11 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
     int kv_end = len_p ? uniform_word(len_p, b) : Tkv;
     kv_end = min(max(kv_end, 0), Tkv);
     const int kv_first = start_p ? max(uniform_word(start_p, b), 0) : 0;
-    // ---- tables: 1 KB units dealt to the wavefronts round-robin, straight to their place in LDS ----
+    // ---- tables ----
     {
-        const uint32_t kbytes = (uint32_t)KK * 8u, vbytes = (uint32_t)KV * 8u;
         const uint8_t *ksrc = uniform_ptr(kj + (size_t)hkv * kjsh * 2);
         const uint8_t *vsrc = uniform_ptr(vj + (size_t)hkv * vjsh * 2);
-        const int ku = (int)((kbytes + 1023u) >> 10), nu = ku + (int)((vbytes + 1023u) >> 10);
-        for (int u = wave; u < nu; u += WV) {
-            const bool isv = u >= ku;
-            const uint32_t uu = (uint32_t)(isv ? u - ku : u);
-            const uint32_t off = min(uu * 1024u + (uint32_t)lane * 16u, (isv ? vbytes : kbytes) - 16u);      // past the end: the last pair again
-            lds_load16((isv ? (uint32_t)kLdVTab : 0u) + uu * 1024u, isv ? vsrc : ksrc, off);
-        }
+        land_tables<WV>(ksrc, (uint32_t)KK * 8u, vsrc, (uint32_t)KV * 8u, kLdVTab, wave, lane);
     }
     STAMP(1);
     const int bh = b * p.Hkv + hkv;

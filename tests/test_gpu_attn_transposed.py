@@ -8,8 +8,8 @@ from tests.test_gpu_attn_rounding import merged
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")]
 
 
-# 16+0 (index widths 12, 11 and 8), 12+1 (10: tables multiplied out, 9, 6), 16+3 (13, 12, 11), 16+1, 16+2, 12+2, 12+3; up to 8 radius bits
-@pytest.mark.parametrize("S,b_r", [(96, 4), (64, 5), (24, 3), (21, 4), (192, 6), (192, 4), (96, 6), (24, 4), (24, 5), (96, 7), (10, 8), (48, 8), (2, 8)])
+# 16+0 (index widths 12, 11 and 8), 12+1 (10: tables multiplied out, 9, 6), 16+3 (13, 12, 11), 16+1, 16+2, 12+2, 12+3; up to 8 radius bits; tables of odd sizes
+@pytest.mark.parametrize("S,b_r", [(96, 4), (64, 5), (24, 3), (21, 4), (192, 6), (192, 4), (96, 6), (24, 4), (24, 5), (96, 7), (10, 8), (48, 8), (2, 8), (90, 4), (171, 6)])
 @pytest.mark.parametrize("d", [64, 128])
 def test_every_token_chunk_and_radius(S, b_r, d):
     import hqmq
