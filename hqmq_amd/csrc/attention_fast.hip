@@ -1561,7 +1561,7 @@ static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hip
     // the kernels divide by multiplication only (fast_div): sizes for which a multiplier cannot be promised (index times
     // divisor beyond 2^32: millions of tokens times thousands of splits) stay with the layout-generic kernel
     if ((p.Hkv > 1 && !p.m_hkv) || (p.G > 1 && !p.m_G) || (p.n_splits > 1 && !p.m_splits)) return HQMQ_OK;
-    // the outlier variants keep Q and the selector rows behind a smaller V slot
+    // the outlier variants keep their staging rows behind a smaller V slot
     if (flags && (p.Kc.K > kFlagsTabMax || p.Vc.K > kFlagsTabMax)) return HQMQ_OK;
     // tables are read two codewords (16 bytes) at a time
     if ((p.Kc.K & 1) || (p.Vc.K & 1) || (p.Kc.jsh & 7) || (p.Vc.jsh & 7) || (((uintptr_t)p.Kc.joint | (uintptr_t)p.Vc.joint) & 15))
