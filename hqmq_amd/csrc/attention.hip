@@ -591,7 +591,8 @@ extern "C" int hqmq_attn_pick_splits(int B, int H_q, int H_kv, int T_q, int T_kv
 }
 
 int hqmq::attn_decode_splits(const hqmq_attn_args *a) {
-    const bool generic = a->dtype == HQMQ_F32 || a->wide_range || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32);
+    const bool generic = a->dtype == HQMQ_F32 || a->wide_range || a->force_generic == 1 || (a->n_chunks != 16 && a->n_chunks != 32) ||
+                         !attn_radius_in_table(a->main_bits, a->aux_bits, a->idx_bits);
     const int64_t groups = ((int64_t)a->T_q * (a->H_q / a->H_kv) + 15) / 16;
     return decode_splits((int64_t)a->B * a->H_kv * groups, generic ? nullptr : a, (int64_t)a->B * a->H_q * a->T_q, 512, a->T_kv,
                          a->kv_len != nullptr, a->n_chunks / 32.0, generic ? 100.0 : a->K.flag_plane ? 250.0 : a->aux_bits ? 350.0 : 500.0);

@@ -249,6 +249,13 @@ int attn_decode_splits(const hqmq_attn_args *a);
 inline bool attn_two_groups(int n_cg, bool flags, int64_t blocks, int range, int n_chunks, int aux_bits) {
     return !flags && n_cg > 1 && blocks > 256 && (blocks >= 512 || range >= 256 || n_chunks == 16 || aux_bits);
 }
+
+// The specialised decode kernels look V's radius codes up in a table of this many (8 bits are the most the quantizer writes).  Layouts whose
+// radius field is wider stay with the layout-generic kernel, which converts a code of any width: tested on the field, not on qmax, so that
+// no code a plane can hold is looked up behind the table's end.  (Main rows have at least 12 bits: with 8 for the radius, 4 and more are left
+// for the index, of which the look-ups' shifts need 3.)
+constexpr int kRadiusCodes = 256;
+inline bool attn_radius_in_table(int main_bits, int aux_bits, int idx_bits) { return main_bits + aux_bits - idx_bits <= 8; }
 int launch_attn_prefill(const AttnParams &p, int main_bits, bool flags, hipStream_t st, const LaunchTiming &tm);
 int launch_attn_fast(const AttnParams &p, int main_bits, bool flags, dim3 grid, size_t table_bytes, hipStream_t st,
                      const LaunchTiming &tm, bool *handled);

@@ -135,7 +135,6 @@ __device__ __forceinline__ uint32_t load_small(const uint8_t *p) {
 // The dynamic LDS block is the kernel's only LDS, so it starts at LDS address 0: the K table sits at byte 0,
 // the V table at kVTabOffset, and a gather addresses them with idx * 8 (+ the instruction's immediate offset).
 constexpr int kTabMax = 5120;               // codewords the K slot has room for
-constexpr int kRadiusCodes = 256;           // radius codes have at most 8 bits
 constexpr int kRadiusTabOffset = kTabMax * 8;           // 8 bytes a code: rq as four fp16, see gather_tokens
 constexpr int kVTabOffset = kRadiusTabOffset + 8 * kRadiusCodes;
 constexpr int kStageOffset = kVTabOffset + 36864;       // outlier variants: staging rows of the wavefronts, after the V table
@@ -309,7 +308,7 @@ __device__ __forceinline__ void gather_tokens(const uint32_t (&w)[NW], uint32_t 
         gather_chunks<CPL, MB, AB, IB, NW, TAB_OFF, false, true>(w, aux, idx_bits, a, unused);
     } else if constexpr (MB == 16 && AB == 0) {
         const uint32_t im2 = idx_mask * 0x00010001u, rm2 = ~im2;
-        const int sh = idx_bits - 3;                    // (a code has at least three index bits)
+        const int sh = idx_bits - 3;                    // (at least 5, see attn_radius_in_table)
 #pragma unroll
         for (int i = 0; i < CPL / 2; i++) {
             const uint32_t ix = w[i] & im2, rx = w[i] & rm2;
@@ -1558,6 +1557,7 @@ static int launch_one(const AttnParams &p, bool flags, dim3 grid, hipStream_t st
 template <int CPL, int DT>
 static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hipStream_t st, const LaunchTiming &tm, bool *handled) {
     if (p.Kc.K > kTabMax || p.Vc.K > kTabMax) return HQMQ_OK;     // tables beyond the fixed LDS slots
+    if (!attn_radius_in_table(mb, p.aux_bits, p.idx_bits)) return HQMQ_OK;
     // the kernels divide by multiplication only (fast_div): sizes for which a multiplier cannot be promised (index times
     // divisor beyond 2^32: millions of tokens times thousands of splits) stay with the layout-generic kernel
     if ((p.Hkv > 1 && !p.m_hkv) || (p.G > 1 && !p.m_G) || (p.n_splits > 1 && !p.m_splits)) return HQMQ_OK;

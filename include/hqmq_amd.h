@@ -16,7 +16,9 @@
  *
  * Packed cache layout (one "plane set" per tensor K or V of one layer), all
  * planes contiguous [B][H][t_cap][row]:
- *   code      = idx | rq << idx_bits,  idx_bits = ceil(log2(24*S)), rq < 2^radius_bits
+ *   code      = idx | rq << idx_bits,  idx_bits = ceil(log2(24*S)), rq < 2^radius_bits, radius_bits <= 8
+ *               (attention also takes wider radius fields, main_bits + aux_bits - idx_bits > 8: the
+ *               specialised decode kernels leave them to the layout-generic one)
  *   main row  = little-endian bit stream of the low main_bits of each of the n codes
  *   aux row   = bit stream of the remaining aux_bits (absent when aux_bits == 0)
  *   scale     = per-token r_max in D

@@ -54,3 +54,38 @@ def test_every_token_chunk_and_radius(S, b_r, d):
                 O = ops.attn_fwd(Q, cache.K, cache.V, T, n_splits=1, force_generic=form)
                 eps = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
                 assert bool(((O.double() - ref).abs() <= bound + eps * ref.abs() + 2.0 ** -24).all()), (T, form)
+
+
+# (index bits, main bits, aux bits) of radius fields with more than 8 bits, and of an index field with less than 3: the table of radius codes
+# ends at 256, so the layout-generic kernel has these calls
+@pytest.mark.parametrize("layout,b_r", [((7, 16, 0), 9), ((6, 16, 0), 10), ((2, 16, 0), 9), ((1, 16, 0), 4), ((6, 12, 3), 9), ((5, 12, 2), 8), ((8, 16, 1), 9)])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_radius_fields_wider_than_the_table(layout, b_r, d, dt):
+    from hqmq_amd import ops
+    from hqmq_amd.packed import PackedTensor
+    B, H, G, T, n, K = 2, 2, 4, 333, d // 4, min(120, 1 << layout[0])
+    g = torch.Generator().manual_seed(d + b_r + layout[0])
+    most = min((1 << b_r) - 1, 1023)
+    sides, dense = [], []
+    for _ in range(2):
+        idx = torch.randint(0, K, (B, H, T, n), generator=g, dtype=torch.int32)
+        rq = torch.randint(0, most + 1, (B, H, T, n), generator=g, dtype=torch.int32)
+        rq[:, :, 0, :2] = torch.tensor([0, most], dtype=torch.int32)
+        joint = torch.nn.functional.normalize(torch.randn(H, K, 4, generator=g), dim=-1).to(dt)
+        t = PackedTensor(B, H, T, d, 1, b_r, dt, "cuda", joint=joint.cuda(), layout=layout)
+        t.scale[:, :, :T] = (0.5 + torch.rand(B, H, T, generator=g)).to(dt).cuda()
+        ops.pack_codes(idx.cuda(), rq.cuda(), t)
+        sides.append(t)
+        cw = torch.stack([joint[h].half()[idx[:, h].long()] for h in range(H)], 1)
+        y = (cw * rq.unsqueeze(-1).half()).double() * (t.scale[:, :, :T].cpu().double() / t.qmax).view(B, H, T, 1, 1)
+        dense.append(y.view(B, H, T, d))
+    Q = torch.randn(B, H * G, 1, d, generator=g).to(dt).cuda()
+    P = torch.softmax(Q.cpu().double().view(B, H, G, d) @ dense[0].transpose(2, 3).contiguous() * d ** -0.5, -1)
+    ref, size = (P @ dense[1]).view(B, H * G, 1, d), (P @ dense[1].abs()).view(B, H * G, 1, d)
+    eps = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    for ns in (1, 2):
+        for form in (0, 1, 2):
+            O = ops.attn_fwd(Q, sides[0], sides[1], T, n_splits=ns, force_generic=form).cpu().double()
+            # two roundings of the weight, 2^-11 each, fp32 scores and exponential as above, and the output's own rounding
+            assert bool(((O - ref).abs() <= (2.0 ** -10 + 1e-4) * size + eps * ref.abs() + 1e-6).all()), (ns, form)
