@@ -76,9 +76,11 @@ __device__ __forceinline__ const uint8_t *uniform_ptr(const uint8_t *p) {
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
     return (const uint8_t *)(((uint64_t)hi << 32) | lo);
 }
-// 64 lanes x 16 bytes from base + voff (+ the instruction's offset, which counts for both sides) to LDS at m0 + 16 * lane
+// 64 lanes x 16 bytes from base + voff (+ the instruction's offset, which counts for both sides) to LDS at m0 + 16 * lane.  Between a
+// write of m0 and the load that reads it the hardware asks for one wait state; the compiler, which inserts it elsewhere, does not look
+// inside an asm block.
 __device__ __forceinline__ void lds_load16(uint32_t lds_base, const uint8_t *base, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(base) : "memory");
 }
 // The K and V codeword tables in 1 KB units dealt to the wavefronts round-robin, straight to their places in LDS (whole units: the last
 // pair of codewords again past a table's end).
@@ -1237,7 +1239,7 @@ __device__ __forceinline__ void wait_groups(int groups) {
     else wait_vm<0>();
 }
 __device__ __forceinline__ void lds_load16_addr(uint32_t lds_base, const uint8_t *addr) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(addr) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(addr) : "memory");
 }
 __device__ __forceinline__ uint4v lds_read16(uint32_t a) { return *(lds_u4_ptr)(uintptr_t)a; }
 __device__ __forceinline__ uint2 lds_read8(uint32_t a) { return __builtin_bit_cast(uint2, *(lds_u2_ptr)(uintptr_t)a); }
@@ -1342,6 +1344,7 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
         const uint8_t *kb = uniform_ptr(k_rows + (size_t)th * mrb), *vb = uniform_ptr(v_rows + (size_t)th * mrb);
         const uint8_t *sa = sc_lane + 2 * (size_t)th;
         asm volatile("s_mov_b32 m0, %0\n\t"
+                     "s_nop 0\n\t"
                      "global_load_lds_dwordx4 %2, %3 offset:256\n\t"
                      "global_load_lds_dwordx4 %2, %3 offset:1280\n\t"
                      "global_load_lds_dword %1, off\n\t"

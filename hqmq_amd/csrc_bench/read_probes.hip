@@ -116,6 +116,7 @@ __global__ __launch_bounds__(512) void read_lds_kernel(const uint8_t *__restrict
         const uint8_t *src = (const uint8_t *)(((uint64_t)hi << 32) | lo);
         const uint32_t dst = __builtin_amdgcn_readfirstlane((wave * 4 + (uint32_t)(i & 3)) * 4096u);
         asm volatile("s_mov_b32 m0, %0\n\t"
+                     "s_nop 0\n\t"         // one wait state before a load reads m0
                      "global_load_lds_dwordx4 %1, %2 offset:0\n\t"
                      "global_load_lds_dwordx4 %1, %2 offset:1024\n\t"
                      "global_load_lds_dwordx4 %1, %2 offset:2048\n\t"

@@ -1,0 +1,23 @@
+"""Hand-written loads that land in LDS: what the compiler would see to, were it not for the asm block."""
+import re
+from pathlib import Path
+
+SOURCES = sorted((Path(__file__).resolve().parent.parent / "hqmq_amd").glob("csrc*/*.h*"))
+
+
+def _asm_blocks(text):
+    for m in re.finditer(r"\basm\b[^;]*?\(\s*((?:\"(?:[^\"\\]|\\.)*\"|//[^\n]*|\s)+)", text):
+        code = "".join(re.findall(r"\"((?:[^\"\\]|\\.)*)\"", re.sub(r"//[^\n]*", "", m.group(1))))
+        yield [line.strip() for line in re.split(r"\\n|\\t", code) if line.strip()]
+
+
+def test_a_wait_state_between_m0_and_the_load_that_reads_it():
+    """A scalar write of m0 needs one wait state before a load to LDS reads it."""
+    seen = 0
+    for path in SOURCES:
+        for block in _asm_blocks(path.read_text()):
+            for line, behind in zip(block, block[1:] + [""]):
+                if re.match(r"s_\w+ m0\b", line):
+                    seen += 1
+                    assert behind.startswith("s_nop"), (path.name, block)
+    assert seen >= 4        # attention_fast.hip and read_probes.hip have them
