@@ -68,7 +68,7 @@ __device__ __forceinline__ void touch_kernargs() {
 }
 
 // Loads that land in LDS.  The compiler neither sees nor counts them; loads come back in the order they were requested, so vmcnt(n) with n
-// no more than the loads requested after them waits for them.
+// no more than the loads requested after them waits for them, and so does the use of a register loaded after them.
 template <int N>
 __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ const uint8_t *uniform_ptr(const uint8_t *p) {
@@ -811,8 +811,9 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
             reinterpret_cast<uint32_t *>(lds_tab)[kAuxTabOffset / 4 + b6] = ((b6 & 7u) << 3) | ((b6 >> 3) << 19) | 0x64006400u;
         }
     }
-    // tables in: behind them were requested the queries, the first tile and its entries, at least this many loads
-    if constexpr (kLand) wait_vm<CPL / 2 + 8 + 4>();
+    // Tables in: a query chunk, requested behind them, is used here, so the compiler waits for it and with it for them.  (Not by a count of the
+    // loads behind the tables: how many those are is the compiler's choice.)
+    if constexpr (kLand) asm volatile("" ::"v"(q_raw[0][CPL - 1].y) : "memory");
 #ifdef HQMQ_STAMPS
     const unsigned long long t_fill_ = __builtin_amdgcn_s_memrealtime();
 #endif

@@ -21,3 +21,14 @@ def test_a_wait_state_between_m0_and_the_load_that_reads_it():
                     seen += 1
                     assert behind.startswith("s_nop"), (path.name, block)
     assert seen >= 4        # attention_fast.hip and read_probes.hip have them
+
+
+def test_waits_by_count_only_where_the_loads_are_written_by_hand():
+    """attn_lds_kernel writes every load it counts; in attn_fast_kernel their number is the compiler's choice, so it may not wait by count."""
+    text = next(p for p in SOURCES if p.name == "attention_fast.hip").read_text()
+    fast, lds = text.index("void attn_fast_kernel("), text.index("void attn_lds_kernel(")
+    bodies = [text[fast:lds], text[lds:text.index("template <", text.index("\n}\n", lds))]]
+    bodies[0] = bodies[0][:bodies[0].index("\n}\n")]
+    assert "land_tables" in bodies[0] and "land_tables" in bodies[1]
+    assert not re.search(r"wait_(vm|groups)\b|s_waitcnt\b", bodies[0])
+    assert re.search(r"wait_groups\(", bodies[1])
