@@ -95,6 +95,17 @@ __device__ __forceinline__ void land_tables(const uint8_t *k, uint32_t kbytes, c
     }
 }
 
+// The same wave-uniform address, known to be one: added to a lane's offset the compiler would otherwise keep row + offset of every plane, six
+// 64-bit addresses per lane.  As scalar base + 32-bit offset the plain variants take fewer registers: at twelve wavefronts s24_r3 in fp16
+// reloaded V's address from scratch once a round, behind a wait for every load in flight (32 x 8000 tokens, 32 / 8 heads of 128, whole call
+// 53.8 -> 49.9 us; 4500 tokens 34.1 -> 32.0).
+template <bool ON, class T>
+__device__ __forceinline__ const T *scalar_base(const T *p) {
+    auto g = (const __attribute__((address_space(1))) T *)p;       // (a generic address out of an asm block would be read by flat loads)
+    if constexpr (ON) asm("" : "+s"(g));
+    return (const T *)g;
+}
+
 constexpr int kFastWaves = 8;     // wavefronts per block; 12 (three per SIMD) with long ranges per block, see launch_layout
 
 // codes, aux bits and raw 16-bit scales of 32 tokens (two 16-token tiles) for one lane
@@ -592,22 +603,25 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const char *k_coord = FLAGS ? (const char *)p.Kc.sb_coord + (size_t)bh * p.Kc.sb_cap * 2 : nullptr;
     const char *v_coord = FLAGS ? (const char *)p.Vc.sb_coord + (size_t)bh * p.Vc.sb_cap * 2 : nullptr;
 
+    constexpr bool kScalarRows = !FLAGS && NCG == 1 && !F8;        // (with two column groups 12 + 2 bits took 39.5 us where it takes 38.6)
     auto load_k = [&](int th, HalfTile<NW, AB, FLAGS> &h) {
-        const uint8_t *kb = k_rows + (size_t)th * mrb;
+        const uint8_t *kb = scalar_base<kScalarRows>(k_rows + (size_t)th * mrb), *ka = scalar_base<kScalarRows>(AB ? ka_rows + (size_t)th * arb : nullptr);
+        const uint16_t *kp = scalar_base<kScalarRows>(ks_plane + th);
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             load_main(kb + main_off + u * 16 * mrb, h.kw[u]);
-            if constexpr (AB > 0) h.kaux[u] = load_aux_word(ka_rows + (size_t)th * arb + aux_off + u * 16 * arb);
-            h.ks[u] = *reinterpret_cast<const uint2 *>(ks_plane + th + scale_off + 16 * u);
+            if constexpr (AB > 0) h.kaux[u] = load_aux_word(ka + aux_off + u * 16 * arb);
+            h.ks[u] = *reinterpret_cast<const uint2 *>(kp + scale_off + 16 * u);
         }
     };
     auto load_v = [&](int th, HalfTile<NW, AB, FLAGS> &h) {
-        const uint8_t *vb = v_rows + (size_t)th * mrb;
+        const uint8_t *vb = scalar_base<kScalarRows>(v_rows + (size_t)th * mrb), *va = scalar_base<kScalarRows>(AB ? va_rows + (size_t)th * arb : nullptr);
+        const uint16_t *vp = scalar_base<kScalarRows>(vs_plane + th);
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             load_main(vb + vmain_off + u * 16 * mrb, h.vw[u]);
-            if constexpr (AB > 0) h.vaux[u] = load_aux_word(va_rows + (size_t)th * arb + vaux_off + u * 16 * arb);
-            h.vs[u] = *reinterpret_cast<const uint2 *>(vs_plane + th + scale_off + 16 * u);
+            if constexpr (AB > 0) h.vaux[u] = load_aux_word(va + vaux_off + u * 16 * arb);
+            h.vs[u] = *reinterpret_cast<const uint2 *>(vp + scale_off + 16 * u);
         }
     };
     auto load_super = [&](int t0, FastTile<NW, AB, FLAGS, NH> &s) {
