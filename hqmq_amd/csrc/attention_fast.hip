@@ -432,8 +432,14 @@ __device__ __forceinline__ void merge_waves(const AttnParams &p, const float *re
 // NCG: column groups (of 16 columns) per wavefront.  Two for chunked prefill with more than 16 columns per KV head:
 // a decoded tile and its V transposition then serve 32 columns.
 // F8: the codeword tables are kept as float8 e4m3 in LDS (callers that rounded their tables to e4m3)
+// Plain caches at d_h 64, tables not multiplied out: two blocks of eight wavefronts share a compute unit (LDS has room for both), which the host
+// plans with; four wavefronts per SIMD leave a form 128 registers.  With 130 to 136 (whole calls of 64 / 8 heads, 512 blocks, one block ->
+// two): bf16 s192_r4 2000 / 4000 tokens 31.2 -> 27.6 / 47.5 -> 43.5 us, s192_r6 32.7 -> 30.1 / 50.5 -> 48.4, 48 x 1500 s96_r6 23.5 -> 19.5.
+constexpr bool two_blocks(int CPL, int MB, int AB, int IB, bool flags, int WV, int NCG) {
+    return CPL == 4 && !flags && WV == 8 && NCG == 1 && !is_prescaled(MB, AB, IB);
+}
 template <int CPL, int MB, int AB, int IB, int DT, bool FLAGS, int WV = kFastWaves, int NCG = 1, bool F8 = false>
-__global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(AttnParams p) {
+__global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : two_blocks(CPL, MB, AB, IB, FLAGS, WV, NCG) ? 4 : 2) void attn_fast_kernel(AttnParams p) {
     static_assert(NCG == 1 || !FLAGS, "outlier variants take one column group");
     constexpr int NB = CPL * MB / 8;
     constexpr int NW = (NB + 3) / 4;
@@ -604,9 +610,12 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
     const char *v_coord = FLAGS ? (const char *)p.Vc.sb_coord + (size_t)bh * p.Vc.sb_cap * 2 : nullptr;
 
     constexpr bool kScalarRows = !FLAGS && NCG == 1 && !F8;        // (with two column groups 12 + 2 bits took 39.5 us where it takes 38.6)
+    // At d_h 64 two planes stay with lane addresses, or the 128 registers that a second block leaves (see the launch bounds) do not hold
+    // the form: 64 x 3000 tokens, bf16, 12 + 2 bits 42.9 us with all scalar, 40.9 so; 12 + 3 bits 44.9, 43.8 so.
+    constexpr bool kScalarAux = kScalarRows && !(CPL == 4 && MB == 12 && AB == 2), kScalarScales = kScalarRows && !(CPL == 4 && MB == 12 && AB == 3);
     auto load_k = [&](int th, HalfTile<NW, AB, FLAGS> &h) {
-        const uint8_t *kb = scalar_base<kScalarRows>(k_rows + (size_t)th * mrb), *ka = scalar_base<kScalarRows>(AB ? ka_rows + (size_t)th * arb : nullptr);
-        const uint16_t *kp = scalar_base<kScalarRows>(ks_plane + th);
+        const uint8_t *kb = scalar_base<kScalarRows>(k_rows + (size_t)th * mrb), *ka = scalar_base<kScalarAux>(AB ? ka_rows + (size_t)th * arb : nullptr);
+        const uint16_t *kp = scalar_base<kScalarScales>(ks_plane + th);
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             load_main(kb + main_off + u * 16 * mrb, h.kw[u]);
@@ -615,8 +624,8 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : 2) void attn_fast_kernel(At
         }
     };
     auto load_v = [&](int th, HalfTile<NW, AB, FLAGS> &h) {
-        const uint8_t *vb = scalar_base<kScalarRows>(v_rows + (size_t)th * mrb), *va = scalar_base<kScalarRows>(AB ? va_rows + (size_t)th * arb : nullptr);
-        const uint16_t *vp = scalar_base<kScalarRows>(vs_plane + th);
+        const uint8_t *vb = scalar_base<kScalarRows>(v_rows + (size_t)th * mrb), *va = scalar_base<kScalarAux>(AB ? va_rows + (size_t)th * arb : nullptr);
+        const uint16_t *vp = scalar_base<kScalarScales>(vs_plane + th);
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             load_main(vb + vmain_off + u * 16 * mrb, h.vw[u]);
@@ -1562,6 +1571,16 @@ static int launch_one(const AttnParams &p, bool flags, dim3 grid, hipStream_t st
     if (!flags || !PS) shmem += 64;        // the wavefronts' progress slots
     const size_t merge = (size_t)WV * 16 * (16 * CPL + 4) * sizeof(float);     // WV >= the wavefronts actually launched
     if (shmem < merge) shmem = merge;
+    // Long sequences of different lengths, whole and started longest first, one or two for every compute unit: the longest bounds the call and is
+    // slowed by a block beside it, so each gets a unit of its own, by asking for more than half the LDS.  Two blocks -> one, 44 / 52 /
+    // 64 sequences of up to 8000 tokens, 64 / 8 heads of 64, bf16, uniform lengths: s192_r6 50.6 -> 41.5 / 56.0 -> 45.5 / 61.9 -> 55.1 us,
+    // s192_r4 44.6 -> 40.6 / 47.7 -> 43.3 / 53.8 -> 53.2; exponential ones 41.2 -> 38.3 and 41.4 -> 40.1 (44 sequences), the upper half of a
+    // uniform distribution 66.4 -> 60.2 and 58.5 -> 58.9.  At 4000 tokens both measure alike (64 sequences, uniform: 32.6 -> 31.2, 30.8 -> 31.2),
+    // at 3000 two are faster (24.4 against 27.0), as with 576 blocks (72 of 5000 44.8 against 49.6) and over equal lengths (3 to 16 %).
+    if (two_blocks(CPL, MB, AB, IB, flags, WV, NCG) && AB && p.kv_len && p.batch_order && p.n_splits == 1 && p.Tkv >= 4000) {
+        const int64_t blocks = (int64_t)grid.x * grid.y * grid.z;
+        if (blocks > 256 && blocks <= 512 && shmem < 84 * 1024) shmem = 84 * 1024;
+    }
     constexpr int WF = CPL == 4 ? WV : kFastWaves;      // outlier variants fit three wavefronts per SIMD only at d_h 64
     auto kern = flags ? attn_fast_kernel<CPL, MB, AB, IB, DT, true, WF, 1, F8> : attn_fast_kernel<CPL, MB, AB, IB, DT, false, WV, NCG, F8>;
     if (shmem > 48 * 1024) {

@@ -89,3 +89,23 @@ def test_radius_fields_wider_than_the_table(layout, b_r, d, dt):
             O = ops.attn_fwd(Q, sides[0], sides[1], T, n_splits=ns, force_generic=form).cpu().double()
             # two roundings of the weight, 2^-11 each, fp32 scores and exponential as above, and the output's own rounding
             assert bool(((O - ref).abs() <= (2.0 ** -10 + 1e-4) * size + eps * ref.abs() + 1e-6).all()), (ns, form)
+
+
+# 264 blocks of heads of 64, whole sequences: started longest first each has a compute unit of its own, else two share one
+@pytest.mark.parametrize("S,b_r,dt", [(192, 4, torch.bfloat16), (192, 6, torch.float16), (24, 5, torch.bfloat16)])
+@pytest.mark.parametrize("T", [3900, 4000, 4200])
+def test_the_order_of_the_sequences_changes_nothing(S, b_r, dt, T):
+    import hqmq
+    from hqmq_amd import ops
+    B, H = 33, 8
+    q = hqmq.HQMQ(n_layers=1, n_heads=H, secondary_size=S, radius_bits=b_r, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(T)
+    k, v = (torch.randn(B, H, T, 64, generator=g, device="cuda", dtype=dt) for _ in range(2))
+    cache = q.new_cache(B, T, 64, dt, 0)
+    q.append(cache, k, v, 0)
+    lens = torch.randint(1, T + 1, (B,), generator=g, device="cuda", dtype=torch.int32)
+    lens[3] = T
+    Q = torch.randn(B, 2 * H, 1, 64, generator=g, device="cuda", dtype=dt)
+    plain, ordered = (ops.attn_fwd(Q, cache.K, cache.V, T, kv_lens=lens, batch_order=o, n_splits=1) for o in (None, ops.longest_first(lens)))
+    assert torch.equal(plain, ordered)
+    assert bool(((plain - ops.attn_fwd(Q, cache.K, cache.V, T, kv_lens=lens, force_generic=1)).abs() <= (2e-3 if dt == torch.float16 else 1e-2)).all())

@@ -55,3 +55,13 @@ def fast():
 
 def test_decode_kernels_use_no_scratch(fast):
     assert {k: m[".private_segment_fixed_size"] for k, m in fast.items() if m[".private_segment_fixed_size"]} == {}
+
+
+def test_two_blocks_of_plain_heads_of_64_fit_a_compute_unit(fast):
+    """Eight wavefronts a block, four per SIMD: 512 / 4 registers each.  (Tables multiplied out fill the LDS with one block.)"""
+    seen = 0
+    for (cpl, mb, ab, ib, _, flags, waves, groups, _), m in fast.items():
+        if cpl == 4 and not flags and waves == 8 and groups == 1 and (mb, ab, ib) != (12, 1, 10):
+            seen += 1
+            assert m[".vgpr_count"] <= 128, (mb, ab, ib, m[".vgpr_count"])
+    assert seen == 18           # 16+0 (index width known or not), 16+1, 16+2, 16+3 (twice), 12+1, 12+2, 12+3, in both types
