@@ -1605,16 +1605,21 @@ static int launch_layout(const AttnParams &p, int mb, bool flags, dim3 grid, hip
         return HQMQ_OK;
     *handled = true;
     // Long ranges per block run with twelve wavefronts, three per SIMD, which hide more of each other's waits than the extra partials
-    // of the block's merge cost; the variants that need more than 168 registers stay at eight.  Lines where both measure alike, with
-    // 224 blocks: d_h 128 plain 3000 tokens (4000 / 5500 tokens of s96_r4 30.1 -> 29.1 / 38.3 -> 36.3 us), d_h 64 over outlier caches
-    // 1200 (3000 / 5500 tokens 26.1 -> 23.3 / 42.3 -> 36.3 us), d_h 64 plain 4000 (8000 tokens 34.4 -> 32.3 us), there only while no
-    // compute unit holds two blocks of eight (480 blocks of 4000 tokens 33.3 against 38.2 us).
+    // of the block's merge cost; the variants that need more than 168 registers stay at eight: from 4096 tokens on over plain caches, from 1536 on
+    // over outlier caches at d_h 64.  (The lines lie a little above where both measured alike in the kernels' first twelve-wavefront form, with 224
+    // blocks: d_h 128 plain 3000 tokens, 4000 / 5500 tokens of s96_r4 30.1 -> 29.1 / 38.3 -> 36.3 us; d_h 64 over outlier caches 1200, 3000 / 5500 tokens
+    // 26.1 -> 23.3 / 42.3 -> 36.3 us; d_h 64 plain 4000, 8000 tokens 34.4 -> 32.3 us.)  d_h 64 plain only while no compute unit holds two blocks of
+    // eight (480 blocks of 4000 tokens 33.3 against 38.2 us).
     const int range = p.Tkv / p.n_splits;
-    // Where the kernel whose loads land in LDS can take the call it keeps it up to 5000 tokens (256 blocks of 4100 / 5000 / 6000 tokens of bf16
-    // s96_r4 32.9 / 41.5 / 48.1 us, twelve wavefronts 35.1 / 40.7 / 46.9).
+    const int64_t blocks = (int64_t)grid.x * grid.y * grid.z;
+    // Where the kernel whose loads land in LDS can take the call it keeps it up to 5000 tokens a block if there is a block for every compute unit;
+    // with fewer, loads come back sooner and twelve wavefronts are ahead.  us landing / twelve wavefronts, 4100, 4600 and 4900 tokens, codebooks of 288
+    // (bf16), 576 (fp16) and 2304 codewords (fp16, bf16): 256 blocks 31.5..33.0 / 32.8..33.1, 34.2..35.2 / 35.6..35.7, 38.1..38.3 / 37.6..39.0; 384 blocks 54.9..56.6 /
+    // 57.1..57.6, 60.3..62.8 / 61.4..62.1, 63.8..66.1 / 64.9..65.6; 224 blocks, alike, 29.5..29.9 / 29.7..30.5, 32.2..32.6 / 31.7..32.2, 33.3..35.0 / 33.6..34.0; 160 blocks
+    // 27.7..28.9 / 26.9..27.9, 30.4..31.9 / 29.1..30.3, 32.2..33.6 / 30.7..31.9.
     const bool lands = CPL == 8 && mb == 16 && p.aux_bits == 0 && !flags && !p.no_lds_landing && p.Kc.K <= 2304 && p.Vc.K <= 2304 && p.Kc.K >= 2 && p.Vc.K >= 2 &&
                        ((((uintptr_t)p.Q) | (uintptr_t)(p.qsb * 2) | (uintptr_t)(p.qsh * 2) | (uintptr_t)(p.qst * 2)) & 15) == 0;
-    const bool wide = CPL == 8 ? !flags && range >= (lands ? 5000 : 4096) : flags ? range >= 1536 : range >= 4096 && (int64_t)grid.x * grid.y * grid.z <= 256;
+    const bool wide = CPL == 8 ? !flags && range >= (lands && blocks >= 256 ? 5000 : 4096) : flags ? range >= 1536 : range >= 4096 && blocks <= 256;
     const bool two = attn_two_groups(p.n_cg, flags, (int64_t)p.n_splits * p.n_cg * p.B * p.Hkv, range, p.n, p.aux_bits);
     // tables of e4m3 numbers kept as float8 in LDS, on request (decode shapes of the 16-bit layouts at d_h 128)
     if (p.tab_fp8 && CPL == 8 && !two) {

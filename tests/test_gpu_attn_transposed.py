@@ -109,3 +109,22 @@ def test_the_order_of_the_sequences_changes_nothing(S, b_r, dt, T):
     plain, ordered = (ops.attn_fwd(Q, cache.K, cache.V, T, kv_lens=lens, batch_order=o, n_splits=1) for o in (None, ops.longest_first(lens)))
     assert torch.equal(plain, ordered)
     assert bool(((plain - ops.attn_fwd(Q, cache.K, cache.V, T, kv_lens=lens, force_generic=1)).abs() <= (2e-3 if dt == torch.float16 else 1e-2)).all())
+
+
+# 248 and 256 blocks of whole sequences around the lines between the kernel whose loads land in LDS and twelve wavefronts
+@pytest.mark.parametrize("S,b_r,dt", [(96, 4, torch.float16), (12, 7, torch.bfloat16)])
+@pytest.mark.parametrize("B", [31, 32])
+def test_lines_of_the_twelve_wavefront_form(S, b_r, dt, B):
+    import hqmq
+    from hqmq_amd import ops
+    H, T = 8, 5010
+    q = hqmq.HQMQ(n_layers=1, n_heads=H, secondary_size=S, radius_bits=b_r, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(B)
+    k, v = (torch.randn(B, H, T, 128, generator=g, device="cuda", dtype=dt) for _ in range(2))
+    cache = q.new_cache(B, T, 128, dt, 0)
+    q.append(cache, k, v, 0)
+    Q = torch.randn(B, 2 * H, 1, 128, generator=g, device="cuda", dtype=dt)
+    for t in (4095, 4096, 4999, 5000):
+        O, plain = (ops.attn_fwd(Q, cache.K, cache.V, t, n_splits=1, force_generic=form) for form in (0, 1))
+        # each weight rounded to fp16 twice at most, outputs (means of 4000 values and more: below 0.5) once: 2^-10 and the type's epsilon, on both sides
+        assert float((O.float() - plain.float()).abs().max()) <= 2 * (2.0 ** -10 + 0.5 * (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8)), t
