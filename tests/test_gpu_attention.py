@@ -418,6 +418,37 @@ def test_clustered_outlier_channels(d_h, Tq, hot, dn):
             assert_attention_close(O, *refs, base=2e-3, what=f"generic={generic} n_splits={ns}")
 
 
+# More than 64 entries in a half-step of 32 tokens: a second round over the list, and rows that are wiped whole instead of entry by entry.
+# s24_r3 stages one tile of 16 tokens at a time, the others two.  1100 tokens in one split: four or five half-steps for each wavefront.
+@pytest.mark.parametrize("S,b_r", [(24, 3), (96, 4), (192, 6)])
+@pytest.mark.parametrize("d_h,dn", [(64, "fp16"), (64, "bf16"), (128, "fp16"), (128, "bf16")])
+def test_many_verbatim_chunks_in_a_half_step(S, b_r, d_h, dn):
+    import hqmq
+    dt = DT[dn]
+    B, Hq, Hkv, T = 2, 8, 2, 1100
+    g = torch.Generator().manual_seed(S + d_h)
+    w = hqmq.with_outlier_extraction(hqmq.HQMQ(n_layers=1, n_heads=Hkv, secondary_size=S, radius_bits=b_r, device=DEV), C=3.0)
+    cache = w.new_cache(B, T, d_h, dt, 0, sideband_frac=0.5)
+    x = []
+    for _ in range(2):
+        y = torch.randn(B, Hkv, T, d_h // 4, 4, generator=g)
+        # a quarter, then two fifths, then hardly any of the chunks (a half-step has 512 of them at d_h 64, 1024 at 128)
+        share = torch.where(torch.arange(T) < 400, 0.25, torch.where(torch.arange(T) < 800, 0.4, 0.01)).view(T, 1, 1)
+        y = torch.where(torch.rand(B, Hkv, T, d_h // 4, 1, generator=g) < share, y * 12.0, y)
+        x.append(y.reshape(B, Hkv, T, d_h).to(dt).to(DEV))
+    w.append(cache, *x, 0)
+    for t in (cache.K, cache.V):
+        t.check_overflow()
+        off = t.sb_tile_off[:, :, :48:2]
+        assert int((off[..., 1:] - off[..., :-1]).max()) > d_h
+    Q = torch.randn(B, Hq, 1, d_h, generator=g).to(dt).to(DEV)
+    refs = masked_two_refs(cache, Q, T)
+    for generic in (False, True):
+        for ns in (1, 3):
+            O = hqmq.fused_attention_packed(Q, cache, force_generic=generic, n_splits=ns)
+            assert_attention_close(O, *refs, base=2e-3, what=f"generic={generic} n_splits={ns}")
+
+
 def _planted(B, H, T, d, seed, dt):
     g = torch.Generator().manual_seed(seed)
     x = torch.randn(B, H, T, d, generator=g)
