@@ -452,7 +452,6 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : two_blocks(CPL, MB, AB, IB,
     // call 157.2 -> 153.9 us, 8 x 32768, s192_r6 46.4 -> 45.0); the plain ones, at three wavefronts per SIMD, would spill (111 -> 195 us),
     // and bf16 ones of 16 + 2 and 16 + 3 bits with the generic field decode.
     constexpr bool kEarlyV = FLAGS && !F8 && !(CPL == 8 && DT == HQMQ_BF16 && MB == 16 && AB >= 2 && IB == 0);
-    constexpr bool kBatchGathers = false;       // see half_step: measured, no gain on any shape (178 against 157 registers)
     constexpr int NH = 1;       // half-steps per prefetched tile: one measures faster than two on every shape
     extern __shared__ uint2 lds_tab[];
 #ifdef HQMQ_STAMPS
@@ -709,10 +708,8 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : two_blocks(CPL, MB, AB, IB,
     };
     // sideband requests of one half-step
     auto issue_all = [&](const FlagTile &f, Entries &k, Entries &v) {
-#pragma unroll
-        for (int i = 0; i < 3; i++) { k.off[i] = f.koff[i]; v.off[i] = f.voff[i]; }
-        entry_load(k_side, k_coord, k.off, k.off[0] + lane, k.x, k.cc);
-        entry_load(v_side, v_coord, v.off, v.off[0] + lane, v.x, v.cc);
+        issue_one(k_side, k_coord, f.koff, k);
+        issue_one(v_side, v_coord, f.voff, v);
     };
     Entries kc = {}, vc = {};
     FastTile<NW, AB, FLAGS, NH> cur;
@@ -939,20 +936,14 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : two_blocks(CPL, MB, AB, IB,
             }
             next_k_entries();
         }
-        // every gather of the 32 K tokens is requested before the first one is used: the wavefront waits for LDS
-        // once per half-step and tensor, not once per pair of chunks
-        // (the variants that have no registers to spare keep the compiler's own interleaving of gathers and multiplies)
+        // (gathers and multiplies interleaved by the compiler: every gather of the 32 K tokens requested before the first one is used was no faster
+        // on any shape, at 178 registers against 157)
         half4 gk[2][CPL];
         half2v rk[2][CPL / 2];
-        if constexpr (kBatchGathers) {
-#pragma unroll
-            for (int u = 0; u < 2; u++) gather_chunks<CPL, MB, AB, IB, NW, 0, F8>(h.kw[u], AB ? h.kaux[u] >> aux_sh : 0u, idx_bits, gk[u], rk[u]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             half4 a[CPL];
-            if constexpr (!kBatchGathers) gather_chunks<CPL, MB, AB, IB, NW, 0, F8>(h.kw[u], AB ? h.kaux[u] >> aux_sh : 0u, idx_bits, gk[u], rk[u]);
+            gather_chunks<CPL, MB, AB, IB, NW, 0, F8>(h.kw[u], AB ? h.kaux[u] >> aux_sh : 0u, idx_bits, gk[u], rk[u]);
             scale_chunks<CPL, PS>(gk[u], rk[u], a);
 #pragma unroll
             for (int cgi = 0; cgi < NCG; cgi++) {
