@@ -103,7 +103,8 @@ def build(verbose: bool = False, stamps: bool = False) -> Path:
             sys.stderr.write(r.stdout + r.stderr)
             raise RuntimeError("hipcc failed on attention_fast.hip (stamps)")
         others = [o for o in objs if o.name != "attention_fast.o"]
-        cmd = [cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(HERE / "libhqmq_amd_stamps.so"), *map(str, others), str(obj)]
+        # (under the library's own name, so that _native.so, loaded after it, calls this one and not the library beside it)
+        cmd = [cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-soname,libhqmq_amd.so", "-o", str(HERE / "libhqmq_amd_stamps.so"), *map(str, others), str(obj)]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode:
             sys.stderr.write(r.stdout + r.stderr)
