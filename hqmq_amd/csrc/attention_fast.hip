@@ -293,9 +293,9 @@ __device__ __forceinline__ void scale_chunks(const half4 (&g)[CPL], const half2v
 // same places.  The products are the ones scale_chunks forms, rounded alike, and so are the outputs.  This replaced a product with the
 // identity (one matrix instruction and two packs of its fp32 results per chunk position and tile, 16 and 32 per half-step at d_h 128)
 // by as many LDS reads; what it took from the vector and matrix units is worth more than what it adds to LDS, which was busy 60 %.
-// One call before -> now: 64 sequences of 1k to 16k, bf16 s24_r3 with outliers (multiplied tables: no second gather), whole step
-// 193 -> 175 us; 4 x 131072, heads of 64, bf16 s96_r4 with outliers 94 -> 84.5; 8 x 32768, s192_r6 with outliers 49.4 -> 47.6;
-// 32768, s96_r4 13.4 -> 12.9.
+// Whole calls over one cache, without -> with: 64 sequences of 1k to 16k, bf16 s24_r3 with outliers (multiplied tables: no second gather),
+// decode step 191 -> 175 us; 4 x 131072, heads of 64, bf16 s96_r4 with outliers 89.7 -> 84.8; 8 x 32768, s192_r6 with outliers
+// 48.8 -> 47.6; 32768, s96_r4 13.3 -> 13.0.
 template <int OFF>
 __device__ __forceinline__ half4 gather8_tr(uint32_t byte_addr) {
     typedef short short4v __attribute__((ext_vector_type(4)));
@@ -448,9 +448,10 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : two_blocks(CPL, MB, AB, IB,
     static_assert(NB % 4 == 0 || NB == 6, "main bytes of one lane");
     static_assert(CPL % 2 == 0, "two chunks per 16x16x32 operand");
     constexpr int NT = WV * 64;
-    // Outlier variants gather V before the softmax, whose exponentials then cover the LDS reads (64 sequences of 1k to 16k, bf16 s24_r3, one
-    // call 157.2 -> 153.9 us, 8 x 32768, s192_r6 46.4 -> 45.0); the plain ones, at three wavefronts per SIMD, would spill (111 -> 195 us),
-    // and bf16 ones of 16 + 2 and 16 + 3 bits with the generic field decode.
+    // Outlier variants gather V before the softmax, whose exponentials then cover the LDS reads (caches read from HBM: 64 sequences of 1k to 16k,
+    // bf16 s24_r3, 157.2 -> 153.9 us, 8 x 32768, s192_r6 46.4 -> 45.0; calls over one cache, with the tile offsets by vector loads that came
+    // with it, decode step 174 -> 165, s192_r6 47.6 -> 48.3); the plain ones, at three wavefronts per SIMD, would spill (111 -> 195 us), and
+    // bf16 ones of 16 + 2 and 16 + 3 bits with the generic field decode.
     constexpr bool kEarlyV = FLAGS && !F8 && !(CPL == 8 && DT == HQMQ_BF16 && MB == 16 && AB >= 2 && IB == 0);
     constexpr int NH = 1;       // half-steps per prefetched tile: one measures faster than two on every shape
     extern __shared__ uint2 lds_tab[];
@@ -858,11 +859,12 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : two_blocks(CPL, MB, AB, IB,
     // [token][chunk], reads them as whole matrix operands and clears what it wrote: its LDS accesses keep their order, so nothing
     // has to be waited for but the data itself.  The walk over the list in batches that this replaced (eight entries of K, sixteen of
     // V the reduction dimension of a product, with masks, look-ups and a transposition per chunk position) was 173 of 567 vector
-    // instructions per half-step at d_h 128 and a chain of 40 matrix instructions; this is 60 and 16.  64 sequences of 1k to 16k, bf16
-    // s24_r3, 1.7 % of the chunks verbatim, one step 229 -> 188 us; 8 x 32768, 28 / 4 heads, s192_r6, 2 % of K's 53.0 -> 45.5; 4 x 131072,
-    // heads of 64, bf16, 1 % 94.2 -> 89.9; 8 x 16000, heads of 64, bf16 s24_r3 37.4 -> 32.4.  Without the test in front of V's part calls
-    // whose values have no outliers take 8 % longer (45.5 -> 48.8) and calls with both 1 to 2 % less (188 -> 185).  The chunks of a row are permuted by the token (16-byte parts, exclusive-or), so
-    // that K's reads (16 tokens at the same part) and V's transposing ones (4 tokens at 4 parts) meet 64 different banks.
+    // instructions per half-step at d_h 128 and a chain of 40 matrix instructions; this is 60 and 16.  Whole calls over
+    // one cache, before -> now: 64 sequences of 1k to 16k, bf16 s24_r3, 1.7 % of the chunks verbatim, decode step 249 -> 197 us; 8 x 32768,
+    // 28 / 4 heads, s192_r6, 2 % of K's 59.3 -> 48.8; 4 x 131072, heads of 64, bf16, 1 % 95.1 -> 89.7.  Without the test in front of V's part
+    // calls whose values have no outliers take 5 % longer (48.8 -> 51.4) and calls with both 1 to 2 % less (196 -> 193).  The chunks of a
+    // row are permuted by the token (16-byte parts, exclusive-or), so that K's reads (16 tokens at the same part) and V's transposing ones
+    // (4 tokens at 4 parts) meet 64 different banks.
     typedef uint2v_t __attribute__((address_space(3))) *lds_w2_ptr;
     auto swizzled = [&](uint32_t row, uint32_t byte) {          // byte: 8 * chunk
         return CPL == 8 ? byte ^ row * 0x110u : byte ^ (row * 0x88u & ~8u);
@@ -1138,7 +1140,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : two_blocks(CPL, MB, AB, IB,
         // from HBM: 16 x 5000 tokens, heads of 64, bf16 s24_r3 24.5 us with two sets, 22.4 with one; 8 x 32768 tokens, 28 / 4 heads of 128,
         // s96_r4 41.6 and 43.1; 64 sequences of 1k to 16k, 4 x 131072 tokens, heads of 64, alike.  (Twelve wavefronts of 168 registers
         // at d_h 128, staging rows in the gaps of the multiplied tables, nothing spilled in the loop, s24_r3: 154.4 where eight take 152.3, and
-        // 175 against 163 with bf16 s96_r4: LDS is busy 60 % of the time, the vector units 64 %.)
+        // 175 against 163 with bf16 s96_r4: with eight LDS is busy 57 to 70 % of a CU's cycles already, and the vector units issue in 58 to 61 %.)
         FastTile<NW, AB, FLAGS, NH> tile_b;
         Entries k_b = {}, v_b = {};
         auto nothing = [] {};
