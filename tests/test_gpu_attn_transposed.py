@@ -128,3 +128,52 @@ def test_lines_of_the_twelve_wavefront_form(S, b_r, dt, B):
         O, plain = (ops.attn_fwd(Q, cache.K, cache.V, t, n_splits=1, force_generic=form) for form in (0, 1))
         # each weight rounded to fp16 twice at most, outputs (means of 4000 values and more: below 0.5) once: 2^-10 and the type's epsilon, on both sides
         assert float((O.float() - plain.float()).abs().max()) <= 2 * (2.0 ** -10 + 0.5 * (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8)), t
+
+
+# 12 + 1 bits, around the most codewords that tables multiplied out have room for: 1022, and 1016 over an outlier cache's values
+@pytest.mark.parametrize("K", [1014, 1016, 1018, 1022, 1024])
+@pytest.mark.parametrize("med", [False, True])
+@pytest.mark.parametrize("d,dt", [(64, torch.bfloat16), (128, torch.float16)])
+def test_largest_tables_of_ten_index_bits(K, med, d, dt):
+    import hqmq
+    from hqmq_amd import ops
+    B, H, G, T, n = 2, 2, 4, 700, d // 4
+    q = hqmq.HQMQ(n_layers=1, n_heads=H, secondary_size=42, radius_bits=3, device="cuda")
+    w = hqmq.with_outlier_extraction(q, C=3.0) if med else q
+    g = torch.Generator().manual_seed(K + d)
+    x = torch.randn(2, B, H, T, n, 4, generator=g)
+    if med:
+        x = torch.where(torch.rand(2, B, H, T, n, 1, generator=g) < 0.03, 20 * x, x)
+    k, v = (y.reshape(B, H, T, d).to(dt).cuda() for y in x)
+    cache = w.new_cache(B, T, d, dt, 0)
+    w.append(cache, k, v, 0)
+    assert (cache.K.idx_bits, cache.K.main_bits, cache.K.aux_bits) == (10, 12, 1)
+    dense = []
+    for t, raw in ((cache.K, k), (cache.V, v)):     # the codebook's 1008 codewords counted from the end of a table of K
+        codes = [unpack_planes(t, b, T) for b in range(B)]
+        idx, rq = (torch.stack([c[i].cpu() for c in codes]).int() for i in (0, 1))
+        table = torch.nn.functional.normalize(torch.randn(H, K, 4, generator=g), dim=-1).to(dt)
+        table[:, K - 1008:] = t.joint.cpu().flip(1)
+        third = (torch.arange(T) % 3 == 0).view(T, 1)
+        idx = torch.where(third, torch.randint(0, K, idx.shape, generator=g, dtype=torch.int32), K - 1 - idx)    # and every codeword of the table
+        t.joint = table.cuda()
+        ops.pack_codes(idx.cuda(), rq.cuda(), t)
+        cw = torch.stack([table[h].half()[idx[:, h].long()] for h in range(H)], 1)
+        y = (cw * rq.unsqueeze(-1).half()).double() * (t.scale[:, :, :T].cpu().double() / t.qmax).view(B, H, T, 1, 1)
+        if med:
+            flags = torch.stack([c[2].cpu() for c in codes])
+            assert int(flags.sum()) > 0 and int(rq[flags].max()) == 0
+            y = torch.where(flags.unsqueeze(-1), raw.cpu().double().view(B, H, T, n, 4), y)
+        dense.append(y.view(B, H, T, d))
+    Q = torch.randn(B, H * G, 1, d, generator=g).to(dt).cuda()
+    P = torch.softmax(Q.cpu().double().view(B, H, G, d) @ dense[0].transpose(2, 3).contiguous() * d ** -0.5, -1)
+    ref, size = (P @ dense[1]).view(B, H * G, 1, d), (P @ dense[1].abs()).view(B, H * G, 1, d)
+    # what weights below fp16's normal numbers lose: 2^-25 of weight * scale and weight * qmax, layout-generic of weight * scale / qmax and weight
+    small = 2.0 ** -25 / min(float(cache.V.scale[:, :, :T].min()), cache.V.qmax) * dense[1].abs().sum(2, keepdim=True).expand(B, H, G, d).reshape(B, H * G, 1, d)
+    eps = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    for ns in (1, 3):
+        for form in (0, 1):
+            O = ops.attn_fwd(Q, cache.K, cache.V, T, n_splits=ns, force_generic=form).cpu().double()
+            # two roundings of the weight, 2^-11 each, fp32 scores and exponential (6e-5 of a weight), and the output's own rounding
+            bound = (2.0 ** -10 + 1e-4) * size + eps * ref.abs() + (small * cache.V.qmax if form else small) + 2.0 ** -24
+            assert bool(((O - ref).abs() <= bound).all()), (ns, form)
