@@ -186,9 +186,18 @@ __device__ int brute_argmax(const float u[4], const typename D::storage *jh, int
 //   WHAT     what the call can ask for: kUnpacked (codes, scales, masks, dense tensor), kPlanes (packed rows), kCompact
 //            (sideband entries in the same launch); a launch that is known to ask for less carries less
 //   MB       main_bits where known at compile time, else 0
+//   FAST     packed rows of the usual forms (fast_rows): neighbouring lanes put the rows together among themselves (DPP) and
+//            everything that does not change from round to round is worked out once.  Through LDS, with its addresses and the
+//            parameters fetched again in every round, packing took a fifth of the cell-list kernel's time at 16-bit codes and a third at
+//            12 + 1 bits
 // Addresses are a wave-uniform base (scalar arithmetic, once per round) plus a 32-bit lane offset that does not change.
 constexpr int kUnpacked = 1, kPlanes = 2, kCompact = 4;
-template <class D, int NT, bool ROWS, int WHAT, int MB>
+// Rows of 16 or 32 codes of MB + at most three bits, whole chunks of x as vectors, planes at dword addresses.
+inline bool fast_rows(const QParams &p, int mb) {
+    return (p.n == 16 || p.n == 32) && p.vec_in && p.vec_rows && p.main_plane && p.scale_plane && p.main_bits == mb && p.aux_bits <= 3 &&
+           (!p.aux_bits || p.aux_plane) && !p.compact;
+}
+template <class D, int NT, bool ROWS, int WHAT, int MB, bool FAST = false>
 struct ChunkSink {
     using ST = typename D::storage;
     const QParams &a;
@@ -198,6 +207,10 @@ struct ChunkSink {
     int t_lo, t_hi;                 // this lane's rows of the planes are those of rounds t_lo <= t0 < t_hi
     float thr, qmaxf, inv_qmax;
     uint32_t seen = 0;              // the largest finite scale this lane has written so far, as bits
+    // FAST: row 0 of the call in every plane
+    uint8_t *main0, *aux0, *flag0;
+    ST *scale0;
+    int idx_bits, aux_bits;
 
     __device__ __forceinline__ ChunkSink(const QParams &a_, int b_, int h_, int tok_local_, int c_, uint32_t *code_sh_, uint32_t *aux_sh_)
         : a(a_), b(b_), h(h_), tok_local(tok_local_), c(c_), code_sh(code_sh_), aux_sh(aux_sh_) {
@@ -211,6 +224,60 @@ struct ChunkSink {
         thr = a.thr ? D::load((const ST *)a.thr + h) : INFINITY;
         qmaxf = (float)a.qmax;
         inv_qmax = __builtin_amdgcn_rcpf(qmaxf);
+        if constexpr (FAST) {
+            const int n = a.n;
+            const int64_t first = bh * a.t_cap + row0;
+            idx_bits = a.idx_bits;
+            aux_bits = a.aux_bits;
+            main0 = a.main_plane + first * (n * MB >> 3);
+            aux0 = aux_bits ? a.aux_plane + first * (n * aux_bits >> 3) : nullptr;
+            flag0 = a.flag_plane ? a.flag_plane + first * (n >> 3) : nullptr;
+            scale0 = (ST *)a.scale_plane + first;
+            t_hi = t_hi < a.T - tok_local ? t_hi : a.T - tok_local;
+        }
+    }
+
+    // The packed rows of one round (FAST).  keep: stays an outlier.
+    __device__ __forceinline__ void put_rows(int t0, float rm, uint32_t idx, uint32_t rq, bool keep) {
+        const int n = a.n;
+        const bool row_ok = t0 >= t_lo && t0 < t_hi;
+        // the lane's place in a round's rows, worked out anew each time: the search has no registers to spare
+        uint32_t tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const uint32_t lg = n == 32 ? 5 : 4, c = tid & (uint32_t)(n - 1), tok = tid >> lg, eighth = tid >> 3;
+        const uint32_t code = (keep ? 0u : rq) << idx_bits | idx;
+        const uint32_t lane_base = tid & 63u & ~(uint32_t)(n - 1);
+        auto store_ballot = [&](uint8_t *row, uint64_t votes) {                // n bits per token, in its first lane
+            const uint64_t mine = votes >> lane_base;
+            if (row_ok && c == 0) {
+                if (n == 32) *reinterpret_cast<uint32_t *>(row + 4u * tok) = (uint32_t)mine;
+                else *reinterpret_cast<uint16_t *>(row + 2u * tok) = (uint16_t)mine;
+            }
+        };
+        uint8_t *main = main0 + (int64_t)t0 * (n * MB >> 3);
+        if constexpr (MB == 16) {
+            if (row_ok) *reinterpret_cast<uint16_t *>(main + 2u * tid) = (uint16_t)code;
+        } else {
+            // pairs of codes (24 bits) in even lanes; dword k of eight lanes is the pairs k and k + 1 from bit 8 k on
+            const uint32_t low = code & 0xfffu, pair = dpp_u32<0xB1>(low) << 12 | low;             // quad_perm [1,0,3,2]
+            const uint32_t next = dpp_u32<0x102>(pair);                                            // row_shl:2
+            const uint32_t v = __builtin_amdgcn_alignbit(next >> 8, next << 24 | pair, 4u * tid & 24u);
+            if (row_ok && !(tid & 1u) && (tid & 7u) < 6u) *reinterpret_cast<uint32_t *>(main + 4u * (3u * eighth + (tid >> 1 & 3u))) = v;
+        }
+        if (aux_bits == 1) store_ballot(aux0 + (int64_t)t0 * (n >> 3), __builtin_amdgcn_ballot_w64((code & (1u << MB)) != 0u));
+        else if (aux_bits) {
+            // the fields of eight lanes, 16 or 24 bits, or'ed together in all of them, then a byte from each of the first
+            uint32_t v = (code >> MB) << ((uint32_t)aux_bits * (tid & 7u));
+            v |= dpp_u32<0xB1>(v);
+            v |= dpp_u32<0x4E>(v);
+            v |= dpp_u32<0x141>(v);
+            if (row_ok && (tid & 7u) < (uint32_t)aux_bits) (aux0 + (int64_t)t0 * (n * aux_bits >> 3))[(uint32_t)aux_bits * eighth + (tid & 7u)] = (uint8_t)(v >> 8u * (tid & 7u));
+        }
+        if (flag0) store_ballot(flag0 + (int64_t)t0 * (n >> 3), __builtin_amdgcn_ballot_w64(keep));
+        if (row_ok && c == 0) {
+            D::store(scale0 + t0 + tok, rm);
+            if (rm < INFINITY) seen = max(seen, __float_as_uint(rm));       // scales are positive: bits order like values
+        }
     }
 
     // jrow(g): the chunk's row of the joint table.  QUICK (std::true_type): every norm of the wavefront is an ordinary number of
@@ -247,11 +314,21 @@ struct ChunkSink {
         float scale, qf;
         if (D::code != HQMQ_F32 && (quick || __builtin_amdgcn_ballot_w64(!quick_divisor<D>(rm)) == 0ull)) scale = quick_div<D>(rm, qmaxf, inv_qmax);      // qmax: at most 255
         else scale = D::rnd(rm / qmaxf);
+        if constexpr (FAST && quick) {
+            // rounded to a whole number by adding 2^23, whose low bits the sum then holds
+            const float sum = div_d<D>(r, scale) + 8388608.f;
+            put_rows(t0, rm, (uint32_t)idx, min(__float_as_uint(sum) & 0xffffu, (uint32_t)a.qmax), nrm > thr);
+            return;
+        }
         qf = rintf(div_d<D>(r, scale));
         if (quick) qf = fminf(qf, qmaxf);
         else if (!is_nan(qf)) qf = fminf(fmaxf(qf, 0.f), qmaxf);
         const int rq = !quick && is_nan(qf) ? 0 : (int)qf;
         const bool flagged = nrm > thr;
+        if constexpr (FAST) {
+            put_rows(t0, rm, (uint32_t)idx, (uint32_t)rq, flagged);
+            return;
+        }
 
         if ((WHAT & kUnpacked) && active) {
             const int64_t tok = bh * a.T + t0;                           // wave-uniform; the lanes of a round are neighbours

@@ -476,7 +476,7 @@ __device__ __forceinline__ int wave_argmax(const float (&u)[4], const typename D
     return K - (int)(W ? last : key & 0xffffu);
 }
 
-template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB>
+template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB, bool FAST>
 __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
     using ST = typename D::storage;
     typedef const uint32_t __attribute__((address_space(3))) *lds_u32;
@@ -498,7 +498,7 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
     RawChunk<D> none = {};                                                        // what lanes without a token work on: an ordinary direction
     for (int j = 0; j < 4; j++) none.set(j, 1.f);
     RawChunk<D> raw = none;
-    if (t_left > 0) raw.load(xl, a.vec_in);
+    if (t_left > 0) raw.load(xl, FAST || a.vec_in);
     {
         // every load of the set-up is requested before the first one is used: one round trip
         constexpr int NP = (8 * 32 + NT - 1) / NT;
@@ -537,7 +537,7 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
     __syncthreads();
 
     const unsigned char *lists = reinterpret_cast<const unsigned char *>(a.grid + a.grid_stride * h);
-    ChunkSink<D, NT, ROWS, WHAT, MB> sink(a, b, h, tok_local, c, code_sh, aux_sh);
+    ChunkSink<D, NT, ROWS, WHAT, MB, FAST> sink(a, b, h, tok_local, c, code_sh, aux_sh);
     const int t_end = JLDS ? a.iters * tpb : tpb;
     // One round, once norm and direction are known: the search and everything after it.  QUICK: every lane of the wavefront has
     // an ordinary norm of a 16-bit type.  u: the direction; with QUICK fp16, the quotients before their rounding to fp16.
@@ -678,7 +678,7 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
         const RawChunk<D> cur = raw;
         raw = none;
         xl += x_step;
-        if (t0 + tpb < t_end && t0 + tpb < t_left) raw.load(xl, a.vec_in);      // the next round's chunk
+        if (t0 + tpb < t_end && t0 + tpb < t_left) raw.load(xl, FAST || a.vec_in);      // the next round's chunk
 
         // ---- norm and direction ----
         // 16-bit types: products of two numbers are exact in fp32, so fused multiply-adds round as products and sums do.
@@ -737,7 +737,7 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
     sink.done();
 }
 
-template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB>
+template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB, bool FAST>
 __global__ __launch_bounds__(NT, NT == 1024 ? 8 : 1) void quantize_grid_kernel(QPair kv) {
     if constexpr (JLDS) {
         // blockIdx.x counts `per_head` blocks for each (tensor, b, h).  Workgroups go round-robin over the 8 XCDs; with a
@@ -748,11 +748,11 @@ __global__ __launch_bounds__(NT, NT == 1024 ? 8 : 1) void quantize_grid_kernel(Q
         const int per_head = kv.per_head, heads = same((int)gridDim.x / per_head), spread = heads % 8 == 0 ? 8 : 1;
         const int i = blockIdx.x / spread, q = same(i / per_head), which = q * spread + blockIdx.x % spread, bhs = kv.p[0].B * kv.p[0].H;
         const int z = same(which >= bhs ? 1 : 0);
-        grid_body<D, NT, ROWS, JLDS, WHAT, MB>(kv.p[z], same(which - z * bhs), same(i - q * per_head));
-    } else grid_body<D, NT, ROWS, JLDS, WHAT, MB>(kv.p[blockIdx.z], blockIdx.y, blockIdx.x);
+        grid_body<D, NT, ROWS, JLDS, WHAT, MB, FAST>(kv.p[z], same(which - z * bhs), same(i - q * per_head));
+    } else grid_body<D, NT, ROWS, JLDS, WHAT, MB, FAST>(kv.p[blockIdx.z], blockIdx.y, blockIdx.x);
 }
 
-template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB>
+template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB, bool FAST = false>
 static int launch_kernel(QPair &kv, int count, hipStream_t st) {
     const QParams &p = kv.p[0];
     const int tpb = NT / p.n, rounds = (p.T + tpb - 1) / tpb;
@@ -774,7 +774,7 @@ static int launch_kernel(QPair &kv, int count, hipStream_t st) {
     kv.p[0].iters = kv.p[1].iters = iters;
     kv.per_head = (rounds + iters - 1) / iters;
     const dim3 grid = JLDS ? dim3(kv.per_head * p.B * p.H * count) : dim3(rounds, p.B * p.H, count);
-    auto kern = quantize_grid_kernel<D, NT, ROWS, JLDS, WHAT, MB>;
+    auto kern = quantize_grid_kernel<D, NT, ROWS, JLDS, WHAT, MB, FAST>;
     if (shmem > 48 * 1024) {
         const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
         if (e != hipSuccess) return (int)e;
@@ -803,6 +803,10 @@ static int launch_d(QPair &kv, int count, hipStream_t st) {
         planes |= q.main_plane || q.aux_plane || q.flag_plane || q.scale_plane;
     }
     if (!planes) return launch_kernel<D, 1024, true, true, kUnpacked, 0>(kv, count, st);
+    if constexpr (D::code != HQMQ_F32) {
+        if (!unpacked && fast_rows(p, 16) && fast_rows(kv.p[1], 16)) return launch_kernel<D, 1024, true, true, kPlanes, 16, true>(kv, count, st);
+        if (!unpacked && fast_rows(p, 12) && fast_rows(kv.p[1], 12)) return launch_kernel<D, 1024, true, true, kPlanes, 12, true>(kv, count, st);
+    }
     if (!unpacked && p.main_bits == 16 && kv.p[1].main_bits == 16) return launch_kernel<D, 1024, true, true, kPlanes, 16>(kv, count, st);
     if (!unpacked && p.main_bits == 12 && kv.p[1].main_bits == 12) return launch_kernel<D, 1024, true, true, kPlanes, 12>(kv, count, st);
     return launch_kernel<D, 1024, true, true, kUnpacked | kPlanes, 0>(kv, count, st);
