@@ -125,6 +125,14 @@ constexpr int64_t pool_blocks(int S, int dtype) {
     return dtype != HQMQ_BF16 || S <= 32 ? kCells / 4 : S <= 96 ? kCells : S <= 192 ? 2 * kCells : 3 * kCells;
 }
 static_assert(3 * kCells < 65535, "block numbers are 16-bit");
+// The first blocks of the pool, which long calls hold in LDS: as many as random codebooks take where that is few.  One list in 80
+// (fp16, S = 96) goes on in the pool, so half the wavefronts' searches do, and from the L2 the block came last of all a round waits for.
+// us, from the L2 and from LDS: K and V of 8 x 32768 tokens, fp16 s96_r4, 122.4 / 119.1; 8 x 4096 tokens encoded 24.2 / 23.3; 4 x 8 x 4001
+// bf16 s24_r3 with Med3x 106.9 / 104.7.  bf16 codebooks above S = 32 take 7000 blocks and more, fp32 ones hardly any.
+constexpr int pool_blocks_lds(int S, int dtype) {
+    return dtype == HQMQ_F32 ? 0 : dtype == HQMQ_BF16 ? (S <= 32 ? 256 : 0) : S <= 96 ? 256 : S <= 192 ? 1024 : 0;
+}
+constexpr int kPoolRounds = 2;                  // and where a block takes that many rounds: one round of S = 192 lost 0.2 us to the copy
 
 int64_t search_grid_blocks(int S, int dtype) {
     if (S < 1 || S > kGridSMax) return 0;
@@ -376,7 +384,7 @@ __global__ __launch_bounds__(kBuildThreads) void grid_build_kernel(int S, uint4 
 
 // ---------------------------------------------------------------- search
 // LDS: the axis units | row numbers by (unit of the direction, low byte of the entry) | K rows of the joint table, last row
-// first (JLDS; bf16 widened to fp32) | one or two words per lane.  The dynamic block is the kernel's only LDS, so it starts
+// first (JLDS; bf16 widened to fp32) | the first blocks of the pool (JLDS) | one or two words per lane.  The dynamic block is the kernel's only LDS, so it starts
 // at LDS address 0.
 template <class D>
 constexpr int lds_row_bytes() { return D::code == HQMQ_F16 ? 8 : 16; }
@@ -489,7 +497,9 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
     const int tid = threadIdx.x, n = a.n, S = a.S, K = 24 * S;
     const int b = bh / a.H, h = bh - b * a.H;
     const ST *jh = (const ST *)a.joint + (size_t)h * K * 4;
-    uint32_t *code_sh = reinterpret_cast<uint32_t *>(lds + kRowsAt + (JLDS ? K * RB : 0)), *aux_sh = code_sh + NT;
+    const int pool_lds = JLDS && a.iters >= kPoolRounds ? pool_blocks_lds(S, D::code) : 0;
+    const uint32_t pool_at = kRowsAt + (JLDS ? (uint32_t)(K * RB) : 0u);
+    uint32_t *code_sh = reinterpret_cast<uint32_t *>(lds + pool_at + 16 * pool_lds), *aux_sh = code_sh + NT;
     const int tpb = NT / n, tok_local = tid / n, c = tid - tok_local * n;
     const int t_first = block * a.iters * tpb;
     const ST *xl = (const ST *)a.x + b * a.xsb + h * a.xsh + (int64_t)(t_first + tok_local) * a.xst + c * 4;
@@ -520,6 +530,8 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
                 else g.store(reinterpret_cast<ST *>(row), true);
             }
         }
+        for (int k = tid; k < pool_lds; k += NT)
+            *reinterpret_cast<uint4 *>(lds + pool_at + k * 16) = a.grid[a.grid_stride * h + kCells + k];
         uint32_t *rows = reinterpret_cast<uint32_t *>(lds + kUnitsAt);
 #pragma unroll
         for (int i = 0; i < NP; i++) {
@@ -635,7 +647,11 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
             const uint32_t next = e.w >> 16;
             if (__builtin_amdgcn_ballot_w64(next != 0u) == 0ull) break;
             if (next == 0xffffu) brute |= active && !zero;              // (a direction that is not ordinary keeps its own reason)
-            e = *reinterpret_cast<const uint4 *>(lists + (kCells + (next == 0xffffu ? 0u : next)) * 16u);
+            const uint32_t block = next == 0xffffu ? 0u : next;
+            if (JLDS && __builtin_amdgcn_ballot_w64((int)block >= pool_lds) == 0ull) {
+                const u32x4 v = *(lds_u128)(uintptr_t)(pool_at + block * 16u);
+                e = uint4{v[0], v[1], v[2], v[3]};
+            } else e = *reinterpret_cast<const uint4 *>(lists + (kCells + block) * 16u);
             if (D::code == HQMQ_F16) asm volatile("" : "+v"(ud[0]), "+v"(ud[1]));      // (or the compiler converts them ahead of the loop)
             score(&e.x, One(), Even());
             if (__builtin_amdgcn_ballot_w64(e.y != none2)) {
@@ -756,7 +772,7 @@ template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB, bool FAST = f
 static int launch_kernel(QPair &kv, int count, hipStream_t st) {
     const QParams &p = kv.p[0];
     const int tpb = NT / p.n, rounds = (p.T + tpb - 1) / tpb;
-    const size_t shmem = kRowsAt + (JLDS ? (size_t)(24 * p.S * lds_row_bytes<D>()) : 0) + (size_t)NT * (needs_aux<ROWS, WHAT>(p.n) ? 8 : 4);
+    const size_t shmem = kRowsAt + (JLDS ? (size_t)(24 * p.S * lds_row_bytes<D>() + 16 * pool_blocks_lds(p.S, D::code)) : 0) + (size_t)NT * (needs_aux<ROWS, WHAT>(p.n) ? 8 : 4);
     // A block copies its head's table to LDS first, about as much work as one round.  Blocks come in waves of as many as the
     // CUs hold; the number of waves is chosen for the fewest rounds in a row, set-up included.
     int iters = 1;
