@@ -622,9 +622,19 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     }
 }
 
-// Launch plan, from measured times in us: a tile takes a block of 128 columns 1.37, one of 256 columns 2.7 (all compute units
-// busy), over outlier caches 1.75 and 3.5; starting (tables, first tiles) and finishing take a block 12; a compute unit holds one
-// block; partials are written and merged at 2 TB/s.
+// Launch plan, from times in us fitted to 100 chunks of 64 and more columns, every number of splits and both widths of block: a tile takes
+// a block of 128 columns / of 256 columns, starting (tables, first tiles) and finishing take a block; a compute unit holds one block;
+// partials are written and merged at 3.2 TB/s.  The plan takes 0.8 % longer than the best one (14 % at worst).  With one set for both
+// head sizes (1.37 / 2.7, over outlier caches 1.75 / 3.5, 12 and 2 TB/s) blocks of 256 columns were taken too seldom and splits too: 3.4 %
+// (37 %); 1024 queries on 16384 tokens, 32 / 8 heads of 128, fp16 s96_r4 369 us in blocks of 128 columns, 342 in two splits of 256;
+// heads of 64 448 / 390; with 2 % of the K chunks verbatim 483 / 415.
+struct PfTimes {
+    double narrow, wide, start;
+};
+static PfTimes pf_times(int d_h, bool flags) {
+    if (flags) return d_h == 64 ? PfTimes{2.75, 4.7, 11.0} : PfTimes{2.4, 3.1, 13.0};
+    return d_h == 64 ? PfTimes{2.25, 3.5, 9.0} : PfTimes{1.5, 2.65, 11.0};
+}
 struct PfPlan {
     bool wide;
     int splits;
@@ -634,6 +644,7 @@ static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int ca
     const double last = causal ? std::max(1.0, std::min((double)Tkv, (double)off + Tq)) : std::max(Tkv, 1);      // tokens the last query sees
     const double mean = causal ? std::min(1.0, std::max(0.5, ((double)off + 0.5 * Tq) / last)) : 1.0;            // all, relative to it
     const int tiles = (int)((last * d_h + 8191) / 8192);
+    const PfTimes times = pf_times(d_h, flags);
     PfPlan best{false, 1, 1e30};
     static const int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 20, 24, 32};
     for (int i = 0; i < (fixed_splits > 0 ? 1 : (int)(sizeof(kSplits) / sizeof(int))); i++) {
@@ -641,9 +652,9 @@ static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int ca
         if (i > 0 && s > tiles / 2) break;
         for (int wide = 0; wide < 2; wide++) {
             const double rounds = (double)(((cols + (wide ? 255 : 127)) / (wide ? 256 : 128) * nz * s + 255) / 256);
-            // the longest block or a compute unit's share of all of them, whichever is more; partials: written and read at 2 TB/s
-            const double us = std::max(1.0, mean * rounds) * ((tiles + s - 1) / s) * (flags ? (wide ? 3.5 : 1.75) : wide ? 2.7 : 1.37) + 12.0 * rounds +
-                              (s > 1 ? 5.0 + (double)(cols * nz) * s * (d_h + 4) * 8 / 2e6 : 0.0);
+            // the longest block or a compute unit's share of all of them, whichever is more
+            const double us = std::max(1.0, mean * rounds) * ((tiles + s - 1) / s) * (wide ? times.wide : times.narrow) + times.start * rounds +
+                              (s > 1 ? 2.0 + (double)(cols * nz) * s * (d_h + 4) * 8 / 3.2e6 : 0.0);
             if (us < best.us) best = PfPlan{wide != 0, s, us};
         }
     }
@@ -669,23 +680,23 @@ static bool attn_prefill_takes(const hqmq_attn_args *a) {
     if ((((uintptr_t)a->O) | (uintptr_t)(a->o_sb * 2) | (uintptr_t)(a->o_sh * 2) | (uintptr_t)(a->o_st * 2)) & 7) return false;
     return true;
 }
-// The same for the kernels of attention_fast.hip: blocks of 16 columns (0.47 us a tile) or of 32 (attn_two_groups, 0.6 us), over
-// outlier caches always of 16 (0.7 us), which start and finish in 6 us.
+// The same for the kernels of attention_fast.hip: blocks of 16 columns or of 32 (attn_two_groups; over outlier caches always of 16), fitted
+// to the same and 100 more chunks: 4 to 11 % off on average.
 static double fast_us(const hqmq_attn_args *a, int64_t cols, int splits) {
     const int64_t nz = (int64_t)a->B * a->H_kv, cg = (cols + 15) / 16, pairs = (cg + 1) / 2 * nz * splits;
     const int d_h = 4 * a->n_chunks;
     const bool flags = a->K.flag_plane != nullptr, two = attn_two_groups((int)cg, flags, cg * nz * splits, a->T_kv / splits, a->n_chunks, a->aux_bits);
-    const double tiles = ((double)a->T_kv * d_h + 8191) / 8192;
-    return 3.0 + (double)(((two ? pairs : cg * nz * splits) + 255) / 256) * (6.0 + tiles / splits * (two ? 0.6 : flags ? 0.7 : 0.47)) +
-           (splits > 1 ? 3.0 + (double)(cols * nz) * splits * (d_h + 4) * 8 / 2e6 : 0.0);
+    const double tiles = ((double)a->T_kv * d_h + 8191) / 8192, start = d_h == 64 ? (flags ? 4.3 : 4.7) : flags ? 5.3 : 6.4;
+    const double tile = d_h == 64 ? (two ? 0.68 : flags ? 0.6 : 0.41) : two ? 0.5 : flags ? 0.5 : 0.27;
+    return 2.1 + (double)(((two ? pairs : cg * nz * splits) + 255) / 256) * (start + tiles / splits * tile) +
+           (splits > 1 ? 1.5 + (double)(cols * nz) * splits * (d_h + 4) * 8 / 1.95e6 : 0.0);
 }
 // The number of splits of a call that leaves it open, 0 if it is better off with the other kernels; splits > 0: the same decision for
-// a given number.  Both estimates are of the plan that would run, the other kernels' with the splits of attn_decode_splits; nine of ten
-// calls take 0.77 to 1.17 of them, mostly both kernels alike.  Over 430 prefill chunks of 64 to 900 columns and 200 to 32768 tokens, plain
-// and outlier caches, the choice takes 0.4 % longer than the faster of the two kernels (28 % at worst).  With the other kernels judged by
-// hqmq_attn_pick_splits, which knows no pairs of column groups, and a margin of 15 % for that, it took 1.5 % (35 %).  us, and with the
-// kernel chosen before: 1 x 33 queries on 19403 tokens, 32 / 8 heads of 128, s24_r3, 37.8 (prefill kernel 47.2); 3 x 70 on 5811,
-// 28 / 4, s192_r4, 50.8 (decode kernels 62.9).
+// a given number.  Both estimates are of the plan that would run, the other kernels' with the splits of attn_decode_splits.  Over 200
+// prefill chunks of 64 and more columns and 64 to 32768 tokens, plain and outlier caches, the choice takes 0.7 % longer than the fastest
+// plan of either kernel (16 % at worst), 1.8 % less than with one set of times for both head sizes and a margin of 5 %.  us, and with the
+// kernel chosen by numbers of splits that would not run: 1 x 33 queries on 19403 tokens, 32 / 8 heads of 128, s24_r3, 37.8 (prefill
+// kernel 47.2); 3 x 70 on 5811, 28 / 4, s192_r4, 50.8 (decode kernels 62.9).
 int attn_prefill_splits(const hqmq_attn_args *a, int splits) {
     const int64_t cols = (int64_t)a->T_q * (a->H_q / a->H_kv), nz = (int64_t)a->B * a->H_kv;
     if (cols < 64 || !attn_prefill_takes(a)) return 0;
@@ -693,7 +704,7 @@ int attn_prefill_splits(const hqmq_attn_args *a, int splits) {
     // Outlier caches of three radius bits keep the decode kernels: most radius codes are 1, 2 or 4, with which those kernels' V is
     // exact, and V rounded as a value left lognormal channels 0.5 % further from 64-bit results (s24_r3; 6 % nearer on average).
     if (a->K.flag_plane && a->qmax < 15 && a->force_generic != 3) return 0;
-    return a->force_generic == 3 || plan.us < 0.95 * fast_us(a, cols, splits > 0 ? splits : attn_decode_splits(a)) ? plan.splits : 0;
+    return a->force_generic == 3 || plan.us < fast_us(a, cols, splits > 0 ? splits : attn_decode_splits(a)) ? plan.splits : 0;
 }
 
 template <int DH, int MB, bool AUX, int DT, bool FL>
