@@ -54,47 +54,6 @@ __device__ __forceinline__ void store_pair(void *tab, int k, uint4v w) {
     else reinterpret_cast<uint4v *>(tab)[k] = pair_to_half<DT>(w);
 }
 
-// The parameter block spans several 64-byte lines of the kernel-argument segment, and the prologue reads them one
-// after the other as its address arithmetic proceeds: every first touch of a line is a miss of the scalar cache
-// that the next scalar load waits behind.  One dword of every line, requested together at the very start, turns
-// the chain of misses into one.
-__device__ __forceinline__ void touch_kernargs() {
-    typedef const uint32_t __attribute__((address_space(4))) *karg_ptr;
-    karg_ptr ka = (karg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
-    uint32_t t = 0;
-#pragma unroll
-    for (int i = 0; i < (int)((sizeof(AttnParams) + 63) / 64); i++) t |= ka[16 * i];
-    asm volatile("" ::"s"(t));
-}
-
-// Loads that land in LDS.  The compiler neither sees nor counts them; loads come back in the order they were requested, so vmcnt(n) with n
-// no more than the loads requested after them waits for them, and so does the use of a register loaded after them.
-template <int N>
-__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-__device__ __forceinline__ const uint8_t *uniform_ptr(const uint8_t *p) {
-    const uint64_t v = (uint64_t)p;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (const uint8_t *)(((uint64_t)hi << 32) | lo);
-}
-// 64 lanes x 16 bytes from base + voff (+ the instruction's offset, which counts for both sides) to LDS at m0 + 16 * lane.  Between a
-// write of m0 and the load that reads it the hardware asks for one wait state; the compiler, which inserts it elsewhere, does not look
-// inside an asm block.
-__device__ __forceinline__ void lds_load16(uint32_t lds_base, const uint8_t *base, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(base) : "memory");
-}
-// The K and V codeword tables in 1 KB units dealt to the wavefronts round-robin, straight to their places in LDS (whole units: the last
-// pair of codewords again past a table's end).
-template <int WV>
-__device__ __forceinline__ void land_tables(const uint8_t *k, uint32_t kbytes, const uint8_t *v, uint32_t vbytes, uint32_t v_at, int wave, int lane) {
-    const int ku = (int)((kbytes + 1023u) >> 10), nu = ku + (int)((vbytes + 1023u) >> 10);
-    for (int u = wave; u < nu; u += WV) {
-        const bool isv = u >= ku;
-        const uint32_t uu = (uint32_t)(isv ? u - ku : u);
-        const uint32_t off = min(uu * 1024u + (uint32_t)lane * 16u, (isv ? vbytes : kbytes) - 16u);
-        lds_load16((isv ? v_at : 0u) + uu * 1024u, isv ? v : k, off);
-    }
-}
-
 // The same wave-uniform address, known to be one: added to a lane's offset the compiler would otherwise keep row + offset of every plane, six
 // 64-bit addresses per lane.  As scalar base + 32-bit offset the plain variants take fewer registers: at twelve wavefronts s24_r3 in fp16
 // reloaded V's address from scratch once a round, behind a wait for every load in flight (32 x 8000 tokens, 32 / 8 heads of 128, whole call
@@ -503,7 +462,7 @@ __global__ __launch_bounds__(WV * 64, WV == 12 ? 3 : two_blocks(CPL, MB, AB, IB,
     const int Kk2 = p.Kc.K >> 1, Kv2 = p.Vc.K >> 1;        // tables of an even number of codewords (checked at launch)
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint4v tk[kLand ? 1 : FU], tv[kLand ? 1 : FU];
-    if constexpr (kLand) land_tables<WV>(uniform_ptr((const uint8_t *)ksrc), 16u * (uint32_t)Kk2, uniform_ptr((const uint8_t *)vsrc), 16u * (uint32_t)Kv2, VTAB, wave, lane);
+    if constexpr (kLand) land_tables<WV>(uniform_ptr((const uint8_t *)ksrc), 16u * (uint32_t)Kk2, uniform_ptr((const uint8_t *)vsrc), 16u * (uint32_t)Kv2, 0u, VTAB, wave, lane);
     else {
 #pragma unroll
         for (int u = 0; u < FU; u++) {
@@ -1308,7 +1267,7 @@ __global__ __launch_bounds__(WV * 64) void attn_lds_kernel(AttnParams p) {
     {
         const uint8_t *ksrc = uniform_ptr(kj + (size_t)hkv * kjsh * 2);
         const uint8_t *vsrc = uniform_ptr(vj + (size_t)hkv * vjsh * 2);
-        land_tables<WV>(ksrc, (uint32_t)KK * 8u, vsrc, (uint32_t)KV * 8u, kLdVTab, wave, lane);
+        land_tables<WV>(ksrc, (uint32_t)KK * 8u, vsrc, (uint32_t)KV * 8u, 0u, kLdVTab, wave, lane);
     }
     STAMP(1);
     const int bh = b * p.Hkv + hkv;

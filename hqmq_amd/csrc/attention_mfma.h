@@ -65,4 +65,45 @@ __device__ __forceinline__ unsigned fast_div(unsigned x, unsigned d, unsigned m)
 
 __device__ __forceinline__ half8 cat8(half4 x, half4 y) { return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7); }
 
+// The parameter block spans several 64-byte lines of the kernel-argument segment, and the prologue reads them one
+// after the other as its address arithmetic proceeds: every first touch of a line is a miss of the scalar cache
+// that the next scalar load waits behind.  One dword of every line, requested together at the very start, turns
+// the chain of misses into one.
+__device__ __forceinline__ void touch_kernargs() {
+    typedef const uint32_t __attribute__((address_space(4))) *karg_ptr;
+    karg_ptr ka = (karg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+    uint32_t t = 0;
+#pragma unroll
+    for (int i = 0; i < (int)((sizeof(AttnParams) + 63) / 64); i++) t |= ka[16 * i];
+    asm volatile("" ::"s"(t));
+}
+
+// Loads that land in LDS.  The compiler neither sees nor counts them; loads come back in the order they were requested, so vmcnt(n) with n
+// no more than the loads requested after them waits for them, and so does the use of a register loaded after them.
+template <int N>
+__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+__device__ __forceinline__ const uint8_t *uniform_ptr(const uint8_t *p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (const uint8_t *)(((uint64_t)hi << 32) | lo);
+}
+// 64 lanes x 16 bytes from base + voff (+ the instruction's offset, which counts for both sides) to LDS at m0 + 16 * lane.  Between a
+// write of m0 and the load that reads it the hardware asks for one wait state; the compiler, which inserts it elsewhere, does not look
+// inside an asm block.
+__device__ __forceinline__ void lds_load16(uint32_t lds_base, const uint8_t *base, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(base) : "memory");
+}
+// The K and V codeword tables in 1 KB units dealt to the wavefronts round-robin, straight to their places in LDS (whole units: the last
+// pair of codewords again past a table's end).
+template <int WV>
+__device__ __forceinline__ void land_tables(const uint8_t *k, uint32_t kbytes, const uint8_t *v, uint32_t vbytes, uint32_t k_at, uint32_t v_at, int wave, int lane) {
+    const int ku = (int)((kbytes + 1023u) >> 10), nu = ku + (int)((vbytes + 1023u) >> 10);
+    for (int u = wave; u < nu; u += WV) {
+        const bool isv = u >= ku;
+        const uint32_t uu = (uint32_t)(isv ? u - ku : u);
+        const uint32_t off = min(uu * 1024u + (uint32_t)lane * 16u, (isv ? vbytes : kbytes) - 16u);
+        lds_load16((isv ? v_at : k_at) + uu * 1024u, isv ? v : k, off);
+    }
+}
+
 }  // namespace hqmq

@@ -51,6 +51,18 @@ typedef short short4v __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kPfV = 16384, kPfBuf = 32768, kPfScale = 2 * kPfBuf, kPfScaleV = 1024, kPfFlag = kPfScale + 2048;   // LDS: K | V, twice; scales; flags (FL); tables
 constexpr uint32_t pf_tab(bool fl) { return kPfFlag + (fl ? 1024u : 0u); }
+// The codeword tables' places, and whether fp16 tables land in LDS, in whole KB, without passing through registers (not where a KB more each
+// would not fit).  us, through registers and landing: unpacked 8 x 141 tokens, 28 / 4 heads, s192_r4, 20.1 / 19.0, 2 x 1024 heads of 64 s96_r4
+// 46.8 / 45.8, 4 x 300 queries on 300 tokens s192_r4 24.6 / 23.3.
+struct PfTables {
+    uint32_t v, end;            // V's table, the end of LDS
+    bool land;
+};
+__host__ __device__ __forceinline__ PfTables pf_tables(int kk, int vk, bool fl, bool fp16) {
+    const uint32_t tab = pf_tab(fl), k = 8u * (uint32_t)kk, v = 8u * (uint32_t)vk, k1 = (k + 1023u) & ~1023u, v1 = (v + 1023u) & ~1023u;
+    if (fp16 && tab + k1 + v1 <= 160u * 1024u) return PfTables{tab + k1, tab + k1 + v1, true};
+    return PfTables{tab + ((k + 127u) & ~127u), tab + ((k + 127u) & ~127u) + v, false};
+}
 
 // permutation of a row's 16-byte parts
 template <int DH>
@@ -68,6 +80,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     constexpr int TOK = DH == 128 ? 16 : 32;                             // tokens a wavefront decodes: 8 chunks per lane
     constexpr uint32_t kPfTab = pf_tab(FL);
     extern __shared__ uint2 lds_tab[];
+    touch_kernargs();
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5, col = lane & 31;
     const int G = p.G, nz = p.B * p.Hkv;
@@ -81,11 +94,19 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     const int cw = wave % CW, kvg = wave / CW;
 
     // ---- codeword tables as fp16: K, then V; every load is on its way before the first one is stored ----
+    const uint2 *kj = (const uint2 *)p.Kc.joint + hkv * (p.Kc.jsh / 4), *vj = (const uint2 *)p.Vc.joint + hkv * (p.Vc.jsh / 4);
+    const PfTables place = pf_tables(p.Kc.K, p.Vc.K, FL, DT == HQMQ_F16);
+    const bool pairs = ((((uintptr_t)kj) | ((uintptr_t)vj)) & 15) == 0 && ((p.Kc.K | p.Vc.K) & 1) == 0, land = DT == HQMQ_F16 && place.land && pairs;
+    // (requested first of all; the wait for them is behind the first tiles' requests)
+    if (land) land_tables<8>(uniform_ptr((const uint8_t *)kj), 8u * (uint32_t)p.Kc.K, uniform_ptr((const uint8_t *)vj), 8u * (uint32_t)p.Vc.K, kPfTab, place.v, wave, lane);
     auto tables = [&]() PF_INLINE {
-        const uint2 *kj = (const uint2 *)p.Kc.joint + hkv * (p.Kc.jsh / 4), *vj = (const uint2 *)p.Vc.joint + hkv * (p.Vc.jsh / 4);
         const int kk = p.Kc.K, vk = p.Vc.K;
-        const uint32_t vt = kPfTab + ((kk * 8 + 127) & ~127);
-        if (((((uintptr_t)kj) | ((uintptr_t)vj)) & 15) == 0 && ((kk | vk) & 1) == 0) {
+        const uint32_t vt = place.v;
+        if (land) {
+            wait_vm<0>();
+            return;
+        }
+        if (pairs) {
             // two codewords a load, all of 2 x 5120 of them in one round: in rounds of 5 x 512 codewords the tables of s192 took four trips
             // to memory (8 x 141 tokens, unpacked, s192_r4 25.4 -> 24.1 us; a chunk of 8 x 353 on 451 tokens, bf16, 55.5 -> 54.2)
             constexpr int U = 10;
@@ -156,7 +177,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     const uint16_t *d_scale = (const uint16_t *)dc.scale_plane + b * dc.ssb + hkv * dc.ssh;
     const uint32_t idx_mask = (1u << p.idx_bits) - 1u;
     const int idx_bits = p.idx_bits;
-    const uint32_t tab = kPfTab + (dec_v ? (uint32_t)((p.Kc.K * 8 + 127) & ~127) : 0u);
+    const uint32_t tab = dec_v ? place.v : kPfTab;
     // Outlier caches (FL): a wavefront decodes whole 16-token tiles of the sideband (one at d_h 128, two at 64), so it also writes
     // their verbatim chunks, over the zeros that flagged chunks decode to.  Lane e takes entry e of the contiguous range that the tile
     // offsets name; the offsets (scalar loads) travel
@@ -723,7 +744,7 @@ static int launch_pf(const AttnParams &p, hipStream_t st, const LaunchTiming &tm
         }
     }
     if (rows * nz > 0x7fffffff) return HQMQ_ERR_SHAPE;
-    const size_t shmem = pf_tab(FL) + (size_t)((p.Kc.K * 8 + 127) & ~127) + (size_t)p.Vc.K * 8;
+    const size_t shmem = pf_tables(p.Kc.K, p.Vc.K, FL, DT == HQMQ_F16).end;
     auto kern = wide ? attn_prefill_kernel<DH, MB, AUX, DT, 1, FL> : attn_prefill_kernel<DH, MB, AUX, DT, 2, FL>;
     const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     if (e != hipSuccess) return (int)e;
