@@ -99,7 +99,7 @@ EXPORTS = [
     "hqmq_pack_codes", "hqmq_dequant_packed", "hqmq_attn_workspace_bytes", "hqmq_attn_pick_splits", "hqmq_attn_splits",
     "hqmq_attn_fwd", "hqmq_attn_fwd_guarded", "hqmq_attn_combine", "hqmq_append_kv", "hqmq_attn_static_scratch_bytes", "hqmq_attn_fwd_static",
     "hqmq_search_grid_bytes", "hqmq_search_grid_kept_bytes", "hqmq_build_search_grid", "hqmq_quantize_grid", "hqmq_append_kv_grid", "hqmq_crop",
-    "hqmq_pack_kv", "hqmq_med3x_workspace_best_bytes",
+    "hqmq_pack_kv", "hqmq_med3x_workspace_best_bytes", "hqmq_quantize_med3x_grid",
 ]
 BENCH_EXPORTS = ["hqmq_bench_read_planes_sink_bytes", "hqmq_bench_read_planes", "hqmq_bench_read_plain", "hqmq_bench_read_lds",
                  "hqmq_bench_empty"]

@@ -12,6 +12,9 @@ extern "C" int hqmq_append_kv_grid(const hqmq_append_args *k, const hqmq_append_
     Med3xCall med[2];
     CompactCall cmp[2];
     const CompactCall *with_q[2] = {nullptr, nullptr};
+    const void *const grids[2] = {k_grid, v_grid};
+    bool selects = true;        // the quantize launches can work out all thresholds themselves
+    int which[2] = {0, 0};
     int n_med = 0;
     for (int i = 0; i < 2; i++) {
         if (!(a[i]->median_mult > 0.f)) continue;
@@ -30,14 +33,17 @@ extern "C" int hqmq_append_kv_grid(const hqmq_append_args *k, const hqmq_append_
         const int rc = check_compact(cmp[n_med]);
         if (rc) return rc;
         with_q[i] = &cmp[n_med];
+        selects &= quantize_selects(&q[i], grids[i]);
+        which[n_med] = i;
         n_med++;
     }
-    int rc = n_med ? med3x_calls(med, n_med, st) : HQMQ_OK;
+    MedSelect left[2] = {}, of[2] = {};
+    int rc = n_med ? med3x_calls(med, n_med, selects ? left : nullptr, st) : HQMQ_OK;
     if (rc) return rc;
+    for (int i = 0; i < n_med; i++) of[which[i]] = left[i];
     // short appends: the quantize launch compacts as well; longer ones get the compaction kernels
     bool compacted[2];
-    const void *const grids[2] = {k_grid, v_grid};
-    rc = quantize_two(&q[0], &q[1], grids, with_q[0], with_q[1], compacted, st);
+    rc = quantize_two(&q[0], &q[1], grids, of, with_q[0], with_q[1], compacted, st);
     if (rc) return rc;
     CompactCall rest[2];
     int n_rest = 0;

@@ -189,13 +189,24 @@ __device__ __forceinline__ void degrade_to_plain(const CompactCall &a, size_t pr
     const uintptr_t fa = (uintptr_t)(const_cast<uint8_t *>(a.flag_plane) + prow * (size_t)((a.n + 7) >> 3) + (c >> 3));
     atomicAnd(reinterpret_cast<uint32_t *>(fa & ~(uintptr_t)3), ~((1u << (c & 7)) << (8 * (fa & 3))));
 }
-int med3x_calls(const Med3xCall *c, int count, hipStream_t st);                                            // med3x.hip
+// What is left of such a call once the histograms are made (med_select.h): the quantize launch that needs the threshold selects for itself.
+struct MedSelect {
+    const uint32_t *ws;
+    float *median; void *thr; int32_t *n_out;
+    float mult;
+    int parts;                  // blocks per head that counted; 0: nothing is left
+    uint32_t per_head;          // chunks
+};
+// later (may be NULL): where the call can end with its histograms it does, and fills this in
+int med3x_calls(const Med3xCall *c, int count, MedSelect *later, hipStream_t st);                          // med3x.hip
 int compact_calls(const CompactCall *c, int count, hipStream_t st);                                        // med3x.hip
 int check_compact(const CompactCall &c);                                                                   // med3x.hip
 // grids: the cell lists of the two codebooks or NULL; ck / cv (may be NULL): the compaction that follows; compacted[i] tells
 // whether the quantize launch did it
-int quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v, const void *const grids[2], const CompactCall *ck,
+// med: what the tensors' Med3x calls left over (parts = 0: nothing); only of calls that quantize_selects names
+int quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v, const void *const grids[2], const MedSelect med[2], const CompactCall *ck,
                  const CompactCall *cv, bool compacted[2], hipStream_t st);                                    // quantize.hip
+bool quantize_selects(const hqmq_quantize_args *a, const void *grid);                                          // quantize.hip
 int64_t search_grid_blocks(int S, int dtype);      // uint4 per head of the cell lists, 0: none for this size                  quantize_grid.hip
 
 }  // namespace hqmq

@@ -18,23 +18,15 @@
 // flagged chunks into the fp16/bf16/fp32 sideband in (token, chunk) order.
 //
 // Compiled with -ffp-contract=off.
-#include "quantize_common.h"
+#include "med_select.h"
 
 namespace hqmq {
 
-constexpr int kBins1 = 32768;
 constexpr int kBins2 = 65536;
 constexpr int kState = 16;  // ints per head
-// The last 64 bins would count NaN patterns, which are counted apart: they hold the sums of 64 groups of 512 bins instead,
-// which spare the selection all but the two groups it needs.
-constexpr int kGroups = 64, kGroupBins = kBins1 / kGroups, kGroupAt = kBins1 - kGroups;
-
-// workspace (uint32 units): hist1[H][kBins1] | state[H][kState] | (fp32 only) hist2[H][2][kBins2]
+// workspace (uint32 units): hist1[H][kBins1] | state[H][kState] | (fp32 only) hist2[H][2][kBins2], or, of a 16-bit type, a part per
+// block (med_select.h)
 // state: 0 nan count, 1 key_lo, 2 key_hi, 3 rank_lo within bin, 4 rank_hi within bin
-// or, of a 16-bit type, per block of the histogram: bins[kBins1 / 2] (two 16-bit counters a word; only those of groups whose
-// sum is not zero are written) | sums[kGroups] | NaN count | padding
-constexpr int kPartWords = kBins1 / 2 + kGroups + 64, kPartSums = kBins1 / 2, kPartNan = kPartSums + kGroups;
-constexpr int kPartBlocks = 256;        // at most, and one per head where there are more heads
 __host__ __device__ inline int64_t ws_words(int H, bool f32) {
     return (int64_t)H * (kBins1 + kState) + (f32 ? (int64_t)H * 2 * kBins2 : 0);
 }
@@ -67,19 +59,6 @@ __global__ void fill_zero_kernel(uint32_t *p, uint32_t *q, int64_t n) {
 template <class D>
 __device__ __forceinline__ float chunk_norm(const typename D::storage *xp) {
     return chunk_norm_d<D>(D::load(xp), D::load(xp + 1), D::load(xp + 2), D::load(xp + 3));
-}
-
-// fp32 bit pattern whose order is the norm's; of a 16-bit type only the upper 16 bits can be set
-template <class D>
-__device__ __forceinline__ uint32_t norm_bits(float nrm) {
-    if (D::code == HQMQ_F32) return __float_as_uint(nrm);
-    if (D::code == HQMQ_F16) return (uint32_t)__half_as_ushort(__float2half_rn(nrm)) << 16;
-    return __float_as_uint(nrm);  // bf16 value: low 16 bits are zero
-}
-// the norm whose 16-bit key this is (16-bit types)
-template <class D>
-__device__ __forceinline__ float key_value(uint32_t key16) {
-    return D::code == HQMQ_F16 ? __half2float(__ushort_as_half((uint16_t)key16)) : __uint_as_float(key16 << 16);
 }
 
 // f(norm) for the chunks of rows [r0, r1) of head h (row = b * T + t), one chunk per lane of a block of NT threads and
@@ -115,18 +94,6 @@ __device__ __forceinline__ void for_each_norm(const MedTensor &m, const MedPair 
                 if (i < k) f(chunk_norm_d<D>(raw[i].get(0), raw[i].get(1), raw[i].get(2), raw[i].get(3)));
         }
     }
-}
-
-// Sum over the wavefront, in every lane (lane permutations inside the vector unit).
-__device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
-    x += dpp_u32<0xB1>(x);
-    x += dpp_u32<0x4E>(x);
-    x += dpp_u32<0x141>(x);
-    x += dpp_u32<0x140>(x);
-    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-    x = r[0] + r[1];
-    const auto q = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-    return q[0] + q[1];
 }
 
 // fp32, very large calls and small workspaces: a histogram of the top 16 bits per head.  The 32768 bins live in LDS, and a block adds only its
@@ -236,28 +203,6 @@ __device__ __forceinline__ void select_two(const uint32_t *hist, const int64_t (
     for (int which = 0; which < 2; which++) { key[which] = res[which]; inner[which] = resr[which]; }
 }
 
-template <class D>
-__device__ __forceinline__ void finish_threshold(float a, float b, bool same, float mult, int h, float *median,
-                                                 typename D::storage *thr) {
-    float med;
-    if (same) med = a;
-    else {
-        const float d = b - a;
-        const float e = d * 0.5f;
-        med = b - e;
-    }
-    median[h] = med;
-    const float t32 = med * mult;
-    D::store(thr + h, D::rnd(t32));
-}
-// a NaN norm makes the quantile NaN, the mask empty
-template <class D>
-__device__ __forceinline__ void nan_threshold(const MedTensor &m, int h) {
-    m.median[h] = NAN;
-    D::store((typename D::storage *)m.thr + h, NAN);
-    if (m.n_out) m.n_out[h] = 0;
-}
-
 // 16-bit types, first of two launches: every block counts the keys of its rows (at most 65535 chunks) in 32768 bins in LDS,
 // two 16-bit counters a word, and stores the groups of bins that hold any, and the sums of all groups, in a part of the
 // workspace that is its own: nothing to clear beforehand and no atomics behind.  A wavefront's 16-byte reads take one group
@@ -293,136 +238,12 @@ __global__ __launch_bounds__(1024) void med_hist16_kernel(MedPair a, int64_t row
     if (tid == 0) part[kPartNan] = lh[words];
 }
 
-// The bin with rank `rank` among the 512 counters of a group, 8 per lane: its number, in the lane that holds it (-1 elsewhere).
-__device__ __forceinline__ uint32_t lanes_before(uint32_t v) {          // exclusive prefix sum over the wavefront
-    const int lane = threadIdx.x & 63;
-    uint32_t incl = v;
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += u;
-    }
-    return incl - v;
-}
-__device__ __forceinline__ int bin_of_rank(const uint32_t (&v)[8], uint32_t rank) {
-    uint32_t tot = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) tot += v[i];
-    const uint32_t first = lanes_before(tot);
-    if (rank < first || rank >= first + tot) return -1;
-    rank -= first;
-    int i = 0;
-#pragma unroll
-    for (int k = 0; k < 7; k++)
-        if (i == k && rank >= v[k]) { rank -= v[k]; i = k + 1; }
-    return (int)(threadIdx.x & 63) * 8 + i;
-}
-
-// Second launch, one block per head: sums of the groups over the head's parts, the group of each rank, that group's bins over
-// the parts (a wavefront per part, 1 KB a time), the bin inside it.  The count wants the bins of the threshold's group as
-// well; the median's group leaves two for it nearly always, which are asked for along with the median's (a third round
-// trip otherwise: 6.9 -> 5.5 us; with every loop unrolled, 7.5: a launch this short waits for its code).
+// Second launch, one block per head
 template <class D>
 __global__ __launch_bounds__(1024) void med_select16_kernel(MedPair a, int parts) {
     const MedTensor &m = a.t[blockIdx.z];
-    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t per_head = (uint32_t)((int64_t)a.B * a.T * a.n);
-    const uint32_t *ws = m.ws + (size_t)h * parts * kPartWords;
-    __shared__ uint32_t sums_sh[16][kGroups], bins_sh[4][kGroupBins], key_sh[2], nan_sh;
-    __shared__ uint64_t some_sh[kPartBlocks];           // the groups a part has any of
-    for (int i = tid; i < 4 * kGroupBins; i += 1024) (&bins_sh[0][0])[i] = 0;
-    if (tid == 0) nan_sh = 0;
-    uint32_t s = 0, nan = 0;
-    if (tid < parts) nan = ws[(size_t)tid * kPartWords + kPartNan];
-    for (int p0 = wave; p0 < parts; p0 += 32) {         // (two requested at a time)
-        const int p1 = p0 + 16;
-        const uint32_t v0 = ws[(size_t)p0 * kPartWords + kPartSums + lane], v1 = ws[(size_t)min(p1, parts - 1) * kPartWords + kPartSums + lane];
-        s += v0 + (p1 < parts ? v1 : 0u);
-        const uint64_t some0 = __builtin_amdgcn_ballot_w64(v0 != 0u), some1 = __builtin_amdgcn_ballot_w64(v1 != 0u);
-        if (lane == 0) {
-            some_sh[p0] = some0;
-            if (p1 < parts) some_sh[p1] = some1;
-        }
-    }
-    sums_sh[wave][lane] = s;
-    __syncthreads();
-    if (nan) nan_sh = 1;
-    uint32_t sum = 0;                                   // of group `lane`, in every wavefront
-#pragma unroll
-    for (int w = 0; w < 16; w++) sum += sums_sh[w][lane];
-    const uint32_t at = lanes_before(sum), rank[2] = {(per_head - 1) / 2, per_head / 2};
-    int group[2];
-    uint32_t rest[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const uint64_t here = __builtin_amdgcn_ballot_w64(rank[i] >= at && rank[i] < at + sum);
-        group[i] = here ? (int)__builtin_ctzll(here) : kGroups - 1;
-        rest[i] = rank[i] - __shfl(at, group[i]);
-    }
-    // the bins of group g, added up over the parts first, first + step, .. by this wavefront
-    auto gather = [&](int g, uint32_t *to, int first, int step) {
-        uint32_t v[8] = {};
-        for (int p0 = first; p0 < parts; p0 += 4 * step) {
-            uint4 x[4];                                 // (all four requested, also where the group was not written: not used then)
-#pragma unroll
-            for (int i = 0; i < 4; i++) x[i] = reinterpret_cast<const uint4 *>(ws + (size_t)min(p0 + i * step, parts - 1) * kPartWords)[g * 64 + lane];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const bool some = p0 + i * step < parts && (some_sh[min(p0 + i * step, parts - 1)] >> g & 1ull);
-                const uint32_t w[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
-#pragma unroll
-                for (int k = 0; k < 4; k++) { v[2 * k] += some ? w[k] & 0xffffu : 0u; v[2 * k + 1] += some ? w[k] >> 16 : 0u; }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (v[i]) atomicAdd(&to[lane * 8 + i], v[i]);
-    };
-    auto bins = [&](const uint32_t *from, uint32_t (&v)[8]) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = from[lane * 8 + i];
-    };
-    // the group of the threshold that a median of this key has (a threshold below every norm or beyond infinity: 0, or the last)
-    auto group_above = [&](float tv) { return (int)min((norm_bits<D>(fmaxf(tv, 0.f)) >> 16) / kGroupBins, (uint32_t)kGroups - 1u); };
-    const int top_lo = group_above(D::rnd(key_value<D>((uint32_t)(group[0] * kGroupBins)) * m.mult));
-    {
-        const int q = wave >> 2, g = q == 0 ? group[0] : q == 1 ? group[1] : min(top_lo + q - 2, kGroups - 1);
-        if (q < 2 || m.n_out) gather(g, bins_sh[q], wave & 3, 4);
-    }
-    __syncthreads();
-    if (nan_sh) {
-        if (tid == 0) nan_threshold<D>(m, h);
-        return;
-    }
-    if (wave < 2) {
-        const int side = wave;
-        uint32_t v[8];
-        bins(bins_sh[side], v);
-        const int bin = bin_of_rank(v, rest[side]);
-        if (bin >= 0) key_sh[side] = (uint32_t)(group[side] * kGroupBins + bin);
-    }
-    __syncthreads();
-    const bool same = rank[0] == rank[1];
-    const float lo = key_value<D>(key_sh[0]), hi = key_value<D>(key_sh[1]);
-    const float tv = D::rnd((same ? lo : hi - (hi - lo) * 0.5f) * m.mult);
-    if (tid == 0) finish_threshold<D>(lo, hi, same, m.mult, h, m.median, (typename D::storage *)m.thr);
-    if (!m.n_out) return;
-    // chunks with norm > thr: whole groups above the one that holds the threshold, and the bins above it in there
-    const int top = group_above(tv);
-    uint32_t *there = bins_sh[top == top_lo ? 2 : 3];
-    if (top != top_lo && top != top_lo + 1) {           // the median's bin is far from its group's first
-        for (int i = tid; i < kGroupBins; i += 1024) there[i] = 0;
-        __syncthreads();
-        gather(top, there, wave, 16);
-        __syncthreads();
-    }
-    if (wave != 0) return;
-    uint32_t v[8], n = lane > top ? sum : 0u;
-    bins(there, v);
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-        if (key_value<D>((uint32_t)(top * kGroupBins + lane * 8 + i)) > tv) n += v[i];
-    n = wave_sum(n);
-    if (lane == 0) m.n_out[h] = (int32_t)n;
+    __shared__ __align__(8) uint32_t sh[kSelectWords];
+    select16<D>(MedSelect{m.ws, m.median, m.thr, m.n_out, m.mult, parts, (uint32_t)((int64_t)a.B * a.T * a.n)}, blockIdx.x, true, sh, [] {});
 }
 
 // One wavefront per rank: the group that holds it (64 sums), then the bin inside the group (8 bins per lane).
@@ -436,7 +257,7 @@ __global__ __launch_bounds__(128) void med_select_kernel(MedPair a) {
     const uint32_t sum = hist[kGroupAt + lane];
     if (state[0] > 0) {
         if (threadIdx.x == 0) {
-            nan_threshold<D>(m, h);
+            nan_threshold<D>(m.median, m.thr, m.n_out, h);
             state[1] = 0xffffffffu; state[2] = 0xffffffffu;
         }
         return;
@@ -634,7 +455,7 @@ __global__ __launch_bounds__(NT) void med_small_kernel(MedPair a) {
         round++;
     }
     if (any_nan) {
-        if (tid == 0) nan_threshold<D>(m, h);
+        if (tid == 0) nan_threshold<D>(m.median, m.thr, m.n_out, h);
         return;
     }
     const uint32_t k_hi = upto > r_hi ? k_lo : ~above;
@@ -707,7 +528,7 @@ __global__ __launch_bounds__(1024) void med_lds_kernel(MedPair a) {
     if (__builtin_amdgcn_ballot_w64(nan) != 0ull && lane == 0) res[2] = 1;
     __syncthreads();
     if (res[2]) {
-        if (tid == 0) nan_threshold<D>(m, h);
+        if (tid == 0) nan_threshold<D>(m.median, m.thr, m.n_out, h);
         return;
     }
     uint4 own[4];
@@ -738,12 +559,7 @@ __global__ __launch_bounds__(1024) void med_lds_kernel(MedPair a) {
             const uint32_t sum = wave_sum(quarter[i]);
             if (!found && left < sum) {
                 found = true;
-                uint32_t up = quarter[i];                                     // running sum over the lanes
-                for (int d = 1; d < 64; d <<= 1) {
-                    const uint32_t v = __shfl_up(up, d);
-                    if (lane >= d) up += v;
-                }
-                const uint32_t lo = up - quarter[i];
+                const uint32_t lo = lanes_before(quarter[i]), up = lo + quarter[i];
                 if (left >= lo && left < up) {
                     const uint32_t w4[4] = {own[i].x, own[i].y, own[i].z, own[i].w};
                     uint32_t at = left - lo, key16 = 0;
@@ -825,11 +641,7 @@ struct CompactPair {
 template <int NT>
 __device__ __forceinline__ int block_scan(int v, int *part, int &total) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int incl = v;
-    for (int o = 1; o < 64; o <<= 1) {
-        const int u = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += u;
-    }
+    const int incl = (int)lanes_before((uint32_t)v) + v;
     if (NT == 64) {
         total = __shfl(incl, 63);
         return incl - v;
@@ -984,7 +796,7 @@ extern "C" int64_t hqmq_med3x_workspace_best_bytes(int H, int dtype) {
 }
 
 template <class D>
-static int run_med3x(const MedPair &a, int count, bool parts, hipStream_t st) {
+static int run_med3x(const MedPair &a, int count, bool parts, MedSelect *later, hipStream_t st) {
     const bool f32 = D::code == HQMQ_F32;
     const int64_t per_head = (int64_t)a.B * a.T * a.n, rows = (int64_t)a.B * a.T;
     // Few keys per lane: such a call lasts about as long as its code takes to arrive (every launch starts
@@ -1029,7 +841,10 @@ static int run_med3x(const MedPair &a, int count, bool parts, hipStream_t st) {
             const hipError_t e = hipFuncSetAttribute((const void *)med_hist16_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) return (int)e;
             hipLaunchKernelGGL(med_hist16_kernel<D>, dim3((unsigned)blocks, a.H, count), dim3(1024), lds, st, a, rpb);
-            hipLaunchKernelGGL(med_select16_kernel<D>, dim3(a.H, 1, count), dim3(1024), 0, st, a, (int)blocks);
+            if (later)
+                for (int i = 0; i < count; i++)
+                    later[i] = MedSelect{a.t[i].ws, a.t[i].median, a.t[i].thr, a.t[i].n_out, a.t[i].mult, (int)blocks, (uint32_t)per_head};
+            else hipLaunchKernelGGL(med_select16_kernel<D>, dim3(a.H, 1, count), dim3(1024), 0, st, a, (int)blocks);
             return hip_status(hipGetLastError());
         }
     }
@@ -1072,15 +887,15 @@ static int check_med3x(const Med3xCall &c) {
 }
 
 // parts: the workspaces hold a part per block
-static int med3x_launch(const MedPair &a, int dtype, int count, bool parts, hipStream_t st) {
+static int med3x_launch(const MedPair &a, int dtype, int count, bool parts, MedSelect *later, hipStream_t st) {
     switch (dtype) {
-        case HQMQ_F32: return run_med3x<F32>(a, count, false, st);
-        case HQMQ_F16: return run_med3x<F16>(a, count, parts, st);
-        default: return run_med3x<BF16>(a, count, parts, st);
+        case HQMQ_F32: return run_med3x<F32>(a, count, false, later, st);
+        case HQMQ_F16: return run_med3x<F16>(a, count, parts, later, st);
+        default: return run_med3x<BF16>(a, count, parts, later, st);
     }
 }
 
-int hqmq::med3x_calls(const Med3xCall *c, int count, hipStream_t st) {
+int hqmq::med3x_calls(const Med3xCall *c, int count, MedSelect *later, hipStream_t st) {
     MedTensor t[2];
     for (int i = 0; i < count; i++) {
         const int rc = check_med3x(c[i]);
@@ -1096,11 +911,11 @@ int hqmq::med3x_calls(const Med3xCall *c, int count, hipStream_t st) {
         const int64_t best = hqmq_med3x_workspace_best_bytes(c[0].H, c[0].dtype);
         const bool parts = c[0].ws_bytes >= best && c[1].ws_bytes >= best && apart(best);
         if (parts || apart(hqmq_med3x_workspace_bytes(c[0].H, c[0].dtype)))
-            return med3x_launch(MedPair{{t[0], t[1]}, c[0].B, c[0].H, c[0].T, c[0].n}, c[0].dtype, 2, parts, st);
+            return med3x_launch(MedPair{{t[0], t[1]}, c[0].B, c[0].H, c[0].T, c[0].n}, c[0].dtype, 2, parts, later, st);
     }
     for (int i = 0; i < count; i++) {
         const bool parts = c[i].ws_bytes >= hqmq_med3x_workspace_best_bytes(c[i].H, c[i].dtype);
-        const int rc = med3x_launch(MedPair{{t[i], t[i]}, c[i].B, c[i].H, c[i].T, c[i].n}, c[i].dtype, 1, parts, st);
+        const int rc = med3x_launch(MedPair{{t[i], t[i]}, c[i].B, c[i].H, c[i].T, c[i].n}, c[i].dtype, 1, parts, later ? later + i : nullptr, st);
         if (rc) return rc;
     }
     return HQMQ_OK;
@@ -1111,7 +926,7 @@ extern "C" int hqmq_med3x_threshold(const void *x, int64_t x_stride_b, int64_t x
                                     float *median, void *thr, int32_t *n_out, void *stream) {
     const Med3xCall c{x, x_stride_b, x_stride_h, x_stride_t, dtype, B, H, T, n_chunks, mult, workspace, workspace_bytes,
                       median, thr, n_out};
-    return med3x_calls(&c, 1, (hipStream_t)stream);
+    return med3x_calls(&c, 1, nullptr, (hipStream_t)stream);
 }
 
 int hqmq::check_compact(const CompactCall &c) {

@@ -418,7 +418,14 @@ static int fill_qparams(const hqmq_quantize_args *a, const void *grid, QParams *
     p.grid = cells && !((uintptr_t)a->joint & (4 * elt - 1)) ? (const uint4 *)grid : nullptr;      // (rows of the table are read as vectors)
     p.grid_stride = cells;
     p.iters = 1;
+    p.med = MedSelect{};
     return HQMQ_OK;
+}
+
+// Calls of the cell-list kernel whose blocks hold a table in LDS: they can select a Med3x threshold as they start.
+bool hqmq::quantize_selects(const hqmq_quantize_args *a, const void *grid) {
+    return grid && a->joint && !((uintptr_t)a->joint & 7) && (a->dtype == HQMQ_F16 || a->dtype == HQMQ_BF16) && a->algo == 0 &&
+           search_grid_blocks(a->secondary_size, a->dtype) > 0 && (int64_t)a->T * a->n_chunks > kQThreads;
 }
 
 // The compaction of a short append can ride in the quantize launch: all new rows of a (b, h) in one block, the
@@ -451,7 +458,24 @@ extern "C" int hqmq_quantize_grid(const hqmq_quantize_args *a, const void *grid,
 
 extern "C" int hqmq_quantize(const hqmq_quantize_args *a, void *stream) { return hqmq_quantize_grid(a, nullptr, stream); }
 
-int hqmq::quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v, const void *const grids[2], const CompactCall *ck,
+extern "C" int hqmq_quantize_med3x_grid(const hqmq_quantize_args *a, float mult, void *workspace, int64_t workspace_bytes, float *median, void *thr,
+                                        int32_t *n_out, const void *grid, void *stream) {
+    if (!a) return HQMQ_ERR_NULL;
+    const Med3xCall c{a->x, a->x_stride_b, a->x_stride_h, a->x_stride_t, a->dtype, a->B, a->H, a->T, a->n_chunks, mult, workspace, workspace_bytes, median, thr, n_out};
+    MedSelect left{};
+    hqmq_quantize_args q = *a;
+    q.thr = thr;
+    QParams p;
+    bool empty;
+    int rc = fill_qparams(&q, grid, &p, &empty);
+    if (!rc) rc = med3x_calls(&c, 1, quantize_selects(&q, grid) ? &left : nullptr, (hipStream_t)stream);
+    if (rc || empty) return rc;
+    p.med = left;
+    if (p.grid && q.algo == 0) return launch_quantize_grid(QPair{{p, p}}, 1, q.dtype, (hipStream_t)stream);
+    return launch_scan(QPair{{p, p}}, 1, q.dtype, q.algo, (hipStream_t)stream);
+}
+
+int hqmq::quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v, const void *const grids[2], const MedSelect med[2], const CompactCall *ck,
                        const CompactCall *cv, bool compacted[2], hipStream_t st) {
     QParams p[2];
     bool empty[2];
@@ -460,6 +484,7 @@ int hqmq::quantize_two(const hqmq_quantize_args *k, const hqmq_quantize_args *v,
     for (int i = 0; i < 2; i++) {
         const int rc = fill_qparams(a[i], grids[i], &p[i], &empty[i]);
         if (rc) return rc;
+        p[i].med = med[i];
         compacted[i] = !empty[i] && take_compaction(p[i], cc[i]);
     }
     const bool by_cells[2] = {p[0].grid && k->algo == 0, p[1].grid && v->algo == 0};

@@ -72,10 +72,12 @@ struct QParams {
     const uint4 *grid;
     int64_t grid_stride;        // uint4 per head
     int iters;                  // rounds of tokens a block of the cell-list kernel takes
+    MedSelect med;              // parts != 0: blocks of the long-call kernel work the threshold out first (med_select.h)
 };
 struct QPair {
     QParams p[2];               // K, V: blockIdx.z picks one
     int per_head;               // cell-list kernel, long calls: blocks per tensor, b and h
+    int med_at;                 // and where in LDS a threshold is selected (-1: where the table comes afterwards)
 };
 
 // The four stored elements of a chunk, as they are in memory.

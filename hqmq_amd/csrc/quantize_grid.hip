@@ -45,7 +45,7 @@
 // time and 1.8 times the memory; 27 without the comparison of all pairs: lists of 3.35 (9.3).
 //
 // Compiled with -ffp-contract=off; fused multiply-adds are written explicitly.
-#include "quantize_common.h"
+#include "med_select.h"
 
 #include <type_traits>
 
@@ -484,8 +484,8 @@ __device__ __forceinline__ int wave_argmax(const float (&u)[4], const typename D
     return K - (int)(W ? last : key & 0xffffu);
 }
 
-template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB, bool FAST>
-__device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
+template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB, bool FAST, bool SEL>
+__device__ __forceinline__ void grid_body(const QParams &a, int bh, int block, int med_at) {
     using ST = typename D::storage;
     typedef const uint32_t __attribute__((address_space(3))) *lds_u32;
     typedef uint32_t __attribute__((ext_vector_type(2))) u32x2;
@@ -509,7 +509,7 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
     for (int j = 0; j < 4; j++) none.set(j, 1.f);
     RawChunk<D> raw = none;
     if (t_left > 0) raw.load(xl, FAST || a.vec_in);
-    {
+    auto set_up = [&]() {
         // every load of the set-up is requested before the first one is used: one round trip
         constexpr int NP = (8 * 32 + NT - 1) / NT;
         uint32_t unit_mul[NP];
@@ -545,11 +545,27 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
             }
         }
         if (tid < 8) *reinterpret_cast<uint4 *>(lds + tid * 16) = uint4{a01, a23, first, (uint32_t)(kUnitsAt + tid * 260)};
-    }
+    };
+    // Med3x: the histograms are there, and every block works the threshold out for itself while its table travels, the head's first one with
+    // the outputs.  As a launch of its own, whole calls, us: K and V of 2048 tokens fake-quantized, fp16 s192_r6, 45.4 (here 43.0), 700 tokens bf16
+    // s24_r3 38.3 (31.8), 4 x 4001 tokens appended 101.5 (98.1), 32768 fp16 s96_r4 171 (165).
+    float thr = 0.f;
+    const bool selected = SEL && a.med.parts;
+    if constexpr (SEL) {
+        uint32_t *sh = reinterpret_cast<uint32_t *>(lds + (med_at < 0 ? 0 : med_at));
+        if (!selected) set_up();
+        else if (med_at >= 0) thr = select16<D>(a.med, h, b == 0 && block == 0, sh, set_up);
+        else {                          // (no room for both)
+            thr = select16<D>(a.med, h, b == 0 && block == 0, sh, [] {});
+            __syncthreads();
+            set_up();
+        }
+    } else set_up();
     __syncthreads();
 
     const unsigned char *lists = reinterpret_cast<const unsigned char *>(a.grid + a.grid_stride * h);
     ChunkSink<D, NT, ROWS, WHAT, MB, FAST> sink(a, b, h, tok_local, c, code_sh, aux_sh);
+    if (selected) sink.thr = thr;
     const int t_end = JLDS ? a.iters * tpb : tpb;
     // One round, once norm and direction are known: the search and everything after it.  QUICK: every lane of the wavefront has
     // an ordinary norm of a 16-bit type.  u: the direction; with QUICK fp16, the quotients before their rounding to fp16.
@@ -753,7 +769,7 @@ __device__ __forceinline__ void grid_body(const QParams &a, int bh, int block) {
     sink.done();
 }
 
-template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB, bool FAST>
+template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB, bool FAST, bool SEL>
 __global__ __launch_bounds__(NT, NT == 1024 ? 8 : 1) void quantize_grid_kernel(QPair kv) {
     if constexpr (JLDS) {
         // blockIdx.x counts `per_head` blocks for each (tensor, b, h).  Workgroups go round-robin over the 8 XCDs; with a
@@ -764,15 +780,23 @@ __global__ __launch_bounds__(NT, NT == 1024 ? 8 : 1) void quantize_grid_kernel(Q
         const int per_head = kv.per_head, heads = same((int)gridDim.x / per_head), spread = heads % 8 == 0 ? 8 : 1;
         const int i = blockIdx.x / spread, q = same(i / per_head), which = q * spread + blockIdx.x % spread, bhs = kv.p[0].B * kv.p[0].H;
         const int z = same(which >= bhs ? 1 : 0);
-        grid_body<D, NT, ROWS, JLDS, WHAT, MB, FAST>(kv.p[z], same(which - z * bhs), same(i - q * per_head));
-    } else grid_body<D, NT, ROWS, JLDS, WHAT, MB, FAST>(kv.p[blockIdx.z], blockIdx.y, blockIdx.x);
+        grid_body<D, NT, ROWS, JLDS, WHAT, MB, FAST, SEL>(kv.p[z], same(which - z * bhs), same(i - q * per_head), kv.med_at);
+    } else grid_body<D, NT, ROWS, JLDS, WHAT, MB, FAST, SEL>(kv.p[blockIdx.z], blockIdx.y, blockIdx.x, -1);
 }
 
 template <class D, int NT, bool ROWS, bool JLDS, int WHAT, int MB, bool FAST = false>
 static int launch_kernel(QPair &kv, int count, hipStream_t st) {
     const QParams &p = kv.p[0];
     const int tpb = NT / p.n, rounds = (p.T + tpb - 1) / tpb;
-    const size_t shmem = kRowsAt + (JLDS ? (size_t)(24 * p.S * lds_row_bytes<D>() + 16 * pool_blocks_lds(p.S, D::code)) : 0) + (size_t)NT * (needs_aux<ROWS, WHAT>(p.n) ? 8 : 4);
+    size_t shmem = kRowsAt + (JLDS ? (size_t)(24 * p.S * lds_row_bytes<D>() + 16 * pool_blocks_lds(p.S, D::code)) : 0) + (size_t)NT * (needs_aux<ROWS, WHAT>(p.n) ? 8 : 4);
+    kv.med_at = -1;
+    if (JLDS && (p.med.parts || kv.p[1].med.parts)) {           // beside the table, if as many blocks share a compute unit as before
+        const size_t both = (shmem + 15) / 16 * 16 + kSelectWords * 4;
+        if (160 * 1024 / both == 160 * 1024 / shmem || both <= 80 * 1024) {
+            kv.med_at = (int)(both - kSelectWords * 4);
+            shmem = both;
+        } else if (shmem < kSelectWords * 4) shmem = kSelectWords * 4;
+    }
     // A block copies its head's table to LDS first, about as much work as one round.  Blocks come in waves of as many as the
     // CUs hold; the number of waves is chosen for the fewest rounds in a row, set-up included.
     int iters = 1;
@@ -790,7 +814,10 @@ static int launch_kernel(QPair &kv, int count, hipStream_t st) {
     kv.p[0].iters = kv.p[1].iters = iters;
     kv.per_head = (rounds + iters - 1) / iters;
     const dim3 grid = JLDS ? dim3(kv.per_head * p.B * p.H * count) : dim3(rounds, p.B * p.H, count);
-    auto kern = quantize_grid_kernel<D, NT, ROWS, JLDS, WHAT, MB, FAST>;
+    auto kern = quantize_grid_kernel<D, NT, ROWS, JLDS, WHAT, MB, FAST, false>;
+    if constexpr (JLDS && D::code != HQMQ_F32) {
+        if (p.med.parts || kv.p[1].med.parts) kern = quantize_grid_kernel<D, NT, ROWS, JLDS, WHAT, MB, FAST, true>;
+    }
     if (shmem > 48 * 1024) {
         const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
         if (e != hipSuccess) return (int)e;

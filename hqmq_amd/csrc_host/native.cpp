@@ -150,11 +150,13 @@ PyObject *fake(PyObject *, PyObject *const *o, Py_ssize_t count) {
         const at::Tensor &ws = tensor(o[5]);
         flagged = at::empty({H}, x.options().dtype(at::kInt));
         uint8_t *room = spare(ws, H);
-        a.thr = room + 4 * H;
-        const int status = median(go, x, number(o[4]), ws, room, room + 4 * H, flagged.data_ptr());
+        const float mult = (float)number(o[4]);
+        void *w = ws.data_ptr(), *thr = room + 4 * H;
+        const int64_t bytes = (int64_t)ws.nbytes();
+        int32_t *counts = (int32_t *)flagged.data_ptr();
+        const int status = go([&](void *stream) { return hqmq_quantize_med3x_grid(&a, mult, w, bytes, (float *)room, thr, counts, lists, stream); });
         if (status) return PyLong_FromLong(status);
-    }
-    if (x.size(2) > 0) {
+    } else if (x.size(2) > 0) {
         const int status = go([&](void *stream) { return hqmq_quantize_grid(&a, lists, stream); });
         if (status) return PyLong_FromLong(status);
     }
