@@ -54,14 +54,6 @@ __device__ __forceinline__ half4 weigh(const float (&w)[4], uint2 scales) {
     return r;
 }
 
-// When the reference of a column's softmax moves.  Scores may exceed it by kSlack, in base 2, before it does: a weight is at most 2^kSlack
-// then, and its product with a V scale of up to kSlackScale stays an fp16 number; with larger scales the reference is the maximum.  Weights
-// and sums have the precision they had, relative to each other.  A maximum over a few columns moves in most of a wavefront's first dozens of
-// steps, and every move multiplies all accumulators of O and waits for the matrix instructions before it.  The prefill kernels, us, reference
-// = maximum and now: 2048 x 2048 unpacked s192_r4 71.5 / 66.4, 4 x 300 on 300 26.5 / 24.9, 1024 on 32768 s96_r4 632 / 614, on 16384 with heads of
-// 64 387 / 372.  (The decode kernels, where a move is a smaller part of a step, gained 0 to 1 % and keep the maximum.)
-constexpr float kSlack = 6.f, kSlackScale = 512.f;
-
 typedef const uint4v __attribute__((address_space(3))) *lds_u4_ptr;
 typedef const uint32_t __attribute__((address_space(3))) *lds_u1_ptr;
 

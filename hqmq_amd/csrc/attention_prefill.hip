@@ -50,8 +50,7 @@ typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kPfV = 16384, kPfBuf = 32768, kPfScale = 2 * kPfBuf, kPfScaleV = 1024, kPfFlag = kPfScale + 2048;   // LDS: K | V, twice; scales; flags (FL); tables
-constexpr uint32_t kPfLimit = kPfFlag;      // (plain caches) by how much scores may exceed their column's reference, one float
-constexpr uint32_t pf_tab(bool fl) { return kPfFlag + (fl ? 1024u : 128u); }
+constexpr uint32_t pf_tab(bool fl) { return kPfFlag + (fl ? 1024u : 0u); }
 // The codeword tables' places, and whether fp16 tables land in LDS, in whole KB, without passing through registers (not where a KB more each
 // would not fit).  us, through registers and landing: unpacked 8 x 141 tokens, 28 / 4 heads, s192_r4, 20.1 / 19.0, 2 x 1024 heads of 64 s96_r4
 // 46.8 / 45.8, 4 x 300 queries on 300 tokens s192_r4 24.6 / 23.3.
@@ -303,7 +302,6 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
                 __builtin_bit_cast(uint4v, cat8(wg[2 * i] * wr[i][0], wg[2 * i + 1] * wr[i][1]));
             if (j == 7) {
                 if (w_lane) *(float __attribute__((address_space(3))) *)(uintptr_t)ws_at = dec_v ? w_scale : w_scale * p.c_log2;
-                if (!FL && dec_v && __builtin_amdgcn_ballot_w64(!(w_scale <= kSlackScale)) != 0) *(float __attribute__((address_space(3))) *)(uintptr_t)kPfLimit = 0.f;
                 if (FL) {
                     if (w_lane && !dec_v) *(uint32_t __attribute__((address_space(3))) *)(uintptr_t)(ws_at + (kPfFlag - kPfScale)) = 0u;
                     asm volatile("" ::: "memory");                        // the wavefront's LDS accesses keep their order
@@ -347,7 +345,6 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         }
     }
     if (it == 0) tables();
-    if (!FL && tid == 0) *(float __attribute__((address_space(3))) *)(uintptr_t)kPfLimit = kSlack;
     __syncthreads();
     if (work) {
 #pragma unroll
@@ -381,7 +378,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     const uint32_t sa = kPfScale + 16u * (uint32_t)half + 128u * NSUB * (uint32_t)kvg;
     const uint32_t fa = kPfFlag + 4u * (uint32_t)col + 128u * NSUB * (uint32_t)kvg;
 
-    // exponents are in base 2: s becomes score * scale - reference (a maximum, see kSlack); seen is -inf until a column has met a token, then 0
+    // exponents are in base 2: s becomes score * scale - (running maximum); seen is -inf until a column has met a token, then 0
     float neg_m = 0.f, seen = -INFINITY, l_run = 0.f;
     float16v acc[DB], s;
 #pragma unroll
@@ -427,12 +424,12 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
             svn = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, verb), qf[kk], svn, 0, 0, 0);
         } else sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(k8, qf[kk], sn, 0, 0, 0);
     };
-    // FL: rows 8 x + 4 half .. + 3 of a unit's scores, relative to the reference: the codes' part times the token's scale
+    // FL: rows 8 x + 4 half .. + 3 of a unit's scores, relative to the running maximum: the codes' part times the token's scale
     auto join = [&](int x, float16v &sn, const float16v &svn, float4v ks) PF_INLINE {
 #pragma unroll
         for (int e = 4 * x; e < 4 * x + 4; e++) sn[e] = __builtin_fmaf(sn[e], ks[e & 3], __builtin_fmaf(svn[e], p.c_plain, neg_m));
     };
-    // scores of a unit (first token tw): times their K scale, relative to the column's reference, which moves if it has to
+    // scores of a unit (first token tw): times their K scale, relative to the running maximum, which moves if it has to
     auto maxima = [&](int tw, const float4v (&ks)[4]) PF_INLINE {
         const bool edge = !(tw + 32 <= wave_min && tw + 32 <= b_end && tw >= col_start);
         float tmax = -INFINITY;
@@ -447,12 +444,12 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         }
 #pragma unroll
         for (int e = 0; e < 16; e++) tmax = fmaxf(tmax, s[e]);
-        // (FL: P is not multiplied with scales, and a weight of 2^kSlack is an fp16 number)
-        const float limit = FL ? kSlack : *(const float __attribute__((address_space(3))) *)(uintptr_t)kPfLimit;
-        if (__builtin_amdgcn_ballot_w64(tmax > (seen == 0.f ? limit : -INFINITY)) != 0) {
+        {
             const uint32_t x = __float_as_uint(tmax);
             const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
             tmax = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+        }
+        if (__builtin_amdgcn_ballot_w64(tmax > seen) != 0) {
             const float d = tmax > seen ? tmax : 0.f;
             const float alpha = seen == 0.f ? __builtin_amdgcn_exp2f(-d) : 0.f;
             l_run *= alpha;
