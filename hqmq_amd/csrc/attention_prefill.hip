@@ -444,12 +444,11 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         }
 #pragma unroll
         for (int e = 0; e < 16; e++) tmax = fmaxf(tmax, s[e]);
-        {
+        // (the halves of a column meet only where one of them exceeds it: they hold the same `seen`)
+        if (__builtin_amdgcn_ballot_w64(tmax > seen) != 0) {
             const uint32_t x = __float_as_uint(tmax);
             const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
             tmax = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-        }
-        if (__builtin_amdgcn_ballot_w64(tmax > seen) != 0) {
             const float d = tmax > seen ? tmax : 0.f;
             const float alpha = seen == 0.f ? __builtin_amdgcn_exp2f(-d) : 0.f;
             l_run *= alpha;
