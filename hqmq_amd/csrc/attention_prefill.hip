@@ -29,11 +29,11 @@
 //   * two tile buffers, one barrier per tile (two with KVG = 1).  The codes of a tile are requested two tiles ahead into
 //     registers that nothing copies (a copy would wait for them).
 // Measured, B = 1, 32 / 8 heads of 128, s96_r4, 1024 queries on 32768 tokens (541 GFLOP, 0.43 ms at the rate of a large matrix
-// product): 0.68 ms against 0.96 with the decode kernels' two-column-group variants; 4096 on 4096 tokens causal, s24_r3:
-// 0.19 against 0.41; four sequences of 300 on 300: 0.022 against 0.048.  With 2 % of the K and V chunks verbatim: 1024 queries on
-// 32768 tokens 0.93 ms against 2.88, 300 on 8000 (28 / 4 heads, s192_r6) 0.122 against 0.318.  (K held as values like V, without the
-// second product: 0.70 and 0.101, but up to 1.55 times as far from 64-bit results at K of 3e-5 and 1.34 times at K of order one;
-// values only in tokens with verbatim chunks, in units of a power of two: 0.80 and 0.107, still up to 1.11.)  Error against 64-bit
+// product): 0.61 ms against 0.96 with the decode kernels' two-column-group variants; 4096 on 4096 tokens causal, s24_r3:
+// 0.185 against 0.41; four sequences of 300 on 300: 0.023 against 0.048.  With 2 % of the K and V chunks verbatim: 1024 queries on
+// 32768 tokens 0.77 ms against 2.88, 300 on 8000 (28 / 4 heads, s192_r6) 0.088 against 0.318.  (K held as values like V, without the
+// second product, with the launch plans of a time when this took 0.93 and 0.122: 0.70 and 0.101, but up to 1.55 times as far from
+// 64-bit results at K of 3e-5 and 1.34 times at K of order one; values only in tokens with verbatim chunks, in units of a power of two: 0.80 and 0.107, still up to 1.11.)  Error against 64-bit
 // results relative to the decode kernels', 162 calls: K from 3e-5 to 30 at V of order one 0.96 on average, 1.03 at most; V of 1e-4
 // 0.96 and 1.00, V of 3e-5, where outputs are fp16 subnormals, 1.02 and 1.08; plain fp16 caches 1.00 to 1.01, bf16 1.00 to 1.02
 // (s24_r3, where the codes are exact in fp16 and little but P is rounded, 1.30 to 1.45).
@@ -444,7 +444,8 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
         }
 #pragma unroll
         for (int e = 0; e < 16; e++) tmax = fmaxf(tmax, s[e]);
-        // (the halves of a column meet only where one of them exceeds it: they hold the same `seen`)
+        // The halves of a column meet only where one of them exceeds it (they hold the same `seen`): most units move no maximum.  Met in every
+        // unit, us: 1024 on 32768 615 (611), on 16384 with heads of 64 383.7 (379.5), 512 on 16384 with verbatim chunks 266.6 (263.9).
         if (__builtin_amdgcn_ballot_w64(tmax > seen) != 0) {
             const uint32_t x = __float_as_uint(tmax);
             const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
