@@ -63,36 +63,48 @@ __device__ __forceinline__ float chunk_norm(const typename D::storage *xp) {
 
 // f(norm) for the chunks of rows [r0, r1) of head h (row = b * T + t), one chunk per lane of a block of NT threads and
 // step, U loads in flight per lane.  The rows of a lane lie NT / n apart: no division per chunk.
-template <class D, int NT, int U, class F>
-__device__ __forceinline__ void for_each_norm(const MedTensor &m, const MedPair &a, int h, int64_t r0, int64_t r1, F f) {
+// meanwhile(): what every thread does, once, while the first chunks travel (it may wait for the block).
+template <class D, int NT, int U, class F, class M>
+__device__ __forceinline__ void for_each_norm(const MedTensor &m, const MedPair &a, int h, int64_t r0, int64_t r1, F f, M meanwhile) {
     using ST = typename D::storage;
     const int n = a.n, per = n <= NT ? NT / n : 1, rl = n <= NT ? (int)threadIdx.x / n : 0;
-    if (rl >= per || r0 + rl >= r1) return;
-    for (int c = (int)threadIdx.x - rl * n; c < n; c += NT) {           // one round, unless a row has more chunks than the block lanes
-        int64_t r = r0 + rl;
-        const int64_t b = r / a.T;
-        int t = (int)(r - b * a.T);
-        const ST *p = (const ST *)m.x + b * m.xsb + h * m.xsh + (int64_t)t * m.xst + c * 4;
-        const int dq = per / a.T, dt = per - dq * a.T;               // `per` rows on: dq sequences and dt tokens
-        const int64_t step = dq * m.xsb + dt * m.xst, wrap = m.xsb - a.T * m.xst;
-        while (r < r1) {
-            RawChunk<D> raw[U];
-            int k = 0;
+    const int dq = per / a.T, dt = per - dq * a.T;                   // `per` rows on: dq sequences and dt tokens
+    const int64_t step = dq * m.xsb + dt * m.xst, wrap = m.xsb - a.T * m.xst, b0 = (r0 + rl) / a.T;
+    const int t0 = (int)(r0 + rl - b0 * a.T);
+    const ST *p0 = (const ST *)m.x + b0 * m.xsb + h * m.xsh + (int64_t)t0 * m.xst, *p;
+    int c = (int)threadIdx.x - rl * n, t = t0, k;
+    int64_t r = r0 + rl;
+    bool more = rl < per && r < r1;
+    RawChunk<D> raw[U];
+    auto request = [&]() {
+        k = 0;
 #pragma unroll
-            for (int i = 0; i < U; i++) {
-                if (r < r1) {
-                    raw[i].load(p, m.vec);
-                    k = i + 1;
-                }
-                r += per;
-                t += dt;
-                p += step;
-                if (t >= a.T) { t -= a.T; p += wrap; }
+        for (int i = 0; i < U; i++) {
+            if (r < r1) {
+                raw[i].load(p, m.vec);
+                k = i + 1;
             }
-#pragma unroll
-            for (int i = 0; i < U; i++)
-                if (i < k) f(chunk_norm_d<D>(raw[i].get(0), raw[i].get(1), raw[i].get(2), raw[i].get(3)));
+            r += per;
+            t += dt;
+            p += step;
+            if (t >= a.T) { t -= a.T; p += wrap; }
         }
+    };
+    p = p0 + c * 4;
+    if (more) request();
+    meanwhile();
+    while (more) {
+#pragma unroll
+        for (int i = 0; i < U; i++)
+            if (i < k) f(chunk_norm_d<D>(raw[i].get(0), raw[i].get(1), raw[i].get(2), raw[i].get(3)));
+        if (r >= r1) {
+            c += NT;                                                 // one round, unless a row has more chunks than the block lanes
+            if (c >= n) break;
+            r = r0;                                                  // (rl is 0 then)
+            t = t0;
+            p = p0 + c * 4;
+        }
+        request();
     }
 }
 
@@ -116,7 +128,7 @@ __global__ __launch_bounds__(1024) void med_hist_kernel(MedPair a, int64_t rows_
         if (is_nan(nrm)) atomicAdd(&lh[nans], 1u);
         else if (WIDE) atomicAdd(&lh[key], 1u);
         else atomicAdd(&lh[key >> 1], 1u << (16 * (key & 1)));
-    });
+    }, [] {});
     __syncthreads();
     uint32_t *hist1 = med_hist(m, h);
     for (int i = threadIdx.x; i < words; i += 1024) {                    // the 64 words of a wavefront lie in one group
@@ -151,7 +163,7 @@ __global__ __launch_bounds__(1024) void med_hist_low_kernel(MedPair a, int64_t r
         const uint32_t bits = __float_as_uint(nrm);
         if ((bits >> 16) == key_lo) atomicAdd(&hist2[bits & 0xffffu], 1u);
         else if ((bits >> 16) == key_hi) atomicAdd(&hist2[kBins2 + (bits & 0xffffu)], 1u);
-    });
+    }, [] {});
 }
 
 // Finds the bins holding 0-based ranks r[0] <= r[1] in a histogram of PER * 1024 counters (a block of 1024 threads).
@@ -209,20 +221,23 @@ __device__ __forceinline__ void select_two(const uint32_t *hist, const int64_t (
 // at a time, so its sum is there when the words are, in registers, to be stored.  8 heads fp16, this launch and the selection:
 // 2048 tokens 17.7 -> 12.0 us, 32768 tokens 60 -> 23.5 (18.0 for this launch: 3.7 TB/s); with bins added to one histogram per
 // head by atomics, cleared by a launch of its own, the additions of the blocks to the same words took longer than the counting.
+// The bins are cleared while the first chunks travel: cleared before they were requested, 4 x 4001 tokens bf16 s24_r3 appended took 99.1 us
+// (98.0), K and V of 2048 tokens fake-quantized 40.2 (39.7), of 4 x 4000 with heads of 64 62.0 (61.1), of 3 x 2500 bf16 63.4 (62.1).
 template <class D>
 __global__ __launch_bounds__(1024) void med_hist16_kernel(MedPair a, int64_t rows_per_block) {
     extern __shared__ uint32_t lh[];    // [kBins1 / 2] | NaN count
     constexpr int words = kBins1 / 2;
     const MedTensor &m = a.t[blockIdx.z];
     const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < words / 4; i += 1024) reinterpret_cast<uint4 *>(lh)[i] = uint4{0, 0, 0, 0};
-    if (tid == 0) lh[words] = 0;
-    __syncthreads();
     const int64_t rows = (int64_t)a.B * a.T, r0 = blockIdx.x * rows_per_block;
     for_each_norm<D, 1024, 4>(m, a, h, r0, min(rows, r0 + rows_per_block), [&](float nrm) {
         const uint32_t key = norm_bits<D>(nrm) >> 16;
         if (is_nan(nrm)) atomicAdd(&lh[words], 1u);
         else atomicAdd(&lh[key >> 1], 1u << (16 * (key & 1)));
+    }, [&] {
+        for (int i = tid; i < words / 4; i += 1024) reinterpret_cast<uint4 *>(lh)[i] = uint4{0, 0, 0, 0};
+        if (tid == 0) lh[words] = 0;
+        __syncthreads();
     });
     __syncthreads();
     uint32_t *part = m.ws + (size_t)(h * gridDim.x + blockIdx.x) * kPartWords;
@@ -358,7 +373,7 @@ __global__ __launch_bounds__(1024) void count_gt_kernel(MedPair a, int64_t rows_
     const float tv = ((const float *)m.thr)[h];
     uint32_t cnt = 0;
     const int64_t rows = (int64_t)a.B * a.T, r0 = blockIdx.x * rows_per_block;
-    for_each_norm<F32, 1024, 4>(m, a, h, r0, min(rows, r0 + rows_per_block), [&](float nrm) { cnt += nrm > tv ? 1u : 0u; });
+    for_each_norm<F32, 1024, 4>(m, a, h, r0, min(rows, r0 + rows_per_block), [&](float nrm) { cnt += nrm > tv ? 1u : 0u; }, [] {});
     cnt = wave_sum(cnt);
     if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(&m.n_out[h], (int)cnt);
 }

@@ -54,6 +54,26 @@ def test_quantize_launch_selects_the_threshold(dn, S, b_r, shape, what):
         assert torch.equal(w.quantize_K(view, 0).view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("dn", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", [
+    (4400, 2, 1, 16), (300, 2, 3, 76),          # a block's step goes over many sequences, not a whole number of them
+    (1, 3, 4097, 20), (2, 1, 601, 120),         # rows that do not divide a block's lanes
+    (3, 2, 11, 4400),                           # rows of more chunks than a block has lanes
+    (1, 1, 129, 512), (1, 5, 513, 128)])        # last blocks of a single step
+def test_histograms_count_every_chunk_once(dn, shape):
+    """Calls that count in one histogram per block (16-bit types, more than 16384 chunks per head), contiguous and with strides."""
+    from hqmq_amd import ops
+    from oracle import c_oracle as CO
+    B, H, T, d_h = shape
+    assert B * T * (d_h // 4) > 16384
+    x = kv_input(shape, DT[dn], seed=T + d_h, outlier_p=0.03)
+    want = CO.med3x(x, 3.0)
+    for view in (x.to(DEV), x.transpose(1, 2).contiguous().to(DEV).transpose(1, 2)):
+        med, thr, count = ops.med3x_threshold(view, 3.0)
+        assert torch.equal(med.cpu(), want["median"]) and torch.equal(thr.cpu().view(torch.int16), want["threshold"].view(torch.int16))
+        assert torch.equal(count.cpu().long(), want["mask"].sum(dim=(0, 2, 3)))
+
+
 @pytest.mark.parametrize("dn,S,b_r,d_h,med", [
     ("fp16", 96, 4, 128, True), ("bf16", 24, 3, 128, True), ("bf16", 24, 3, 64, True), ("fp16", 192, 6, 128, True), ("fp16", 192, 6, 64, False),
     ("bf16", 192, 5, 128, True), ("fp16", 192, 4, 64, True), ("bf16", 24, 5, 128, False), ("fp16", 24, 4, 64, True)])
