@@ -38,8 +38,8 @@
 // 0.96 and 1.00, V of 3e-5, where outputs are fp16 subnormals, 1.02 and 1.08; plain fp16 caches 1.00 to 1.01, bf16 1.00 to 1.02
 // (s24_r3, where the codes are exact in fp16 and little but P is rounded, 1.30 to 1.45).
 // What bounds it: overlap, no pipe is full.  By the counters (profiles/attn_prefill_kernel_instruction_counters.txt) a compute unit
-// spends 37 % of its busy cycles in the matrix pipe, 50 % issuing vector instructions and 63 % in LDS, a third of that bank
-// conflicts (plain, 1024 on 32768), at 2.0 to 2.1 GHz; with verbatim chunks 37, 64 and 40 %; 2048 on 2048 causal 21, 51 and 38 %.
+// spends 44 % of its busy cycles in the matrix pipe, 49 % issuing vector instructions and 54 % in LDS, a quarter of that bank
+// conflicts (plain, 1024 on 32768), at 2.0 to 2.1 GHz; with verbatim chunks 45, 63 and 34 %; 2048 on 2048 causal 23, 55 and 42 %.
 #include "attention_mfma.h"
 #include <algorithm>
 
