@@ -197,7 +197,8 @@ struct MedSelect {
     int parts;                  // blocks per head that counted; 0: nothing is left
     uint32_t per_head;          // chunks
 };
-// later (may be NULL): where the call can end with its histograms it does, and fills this in
+// later (may be NULL, else one per call): where a call can end with its histograms it does, and fills this in; not where another call's
+// histograms come into the same workspace
 int med3x_calls(const Med3xCall *c, int count, MedSelect *later, hipStream_t st);                          // med3x.hip
 int compact_calls(const CompactCall *c, int count, hipStream_t st);                                        // med3x.hip
 int check_compact(const CompactCall &c);                                                                   // med3x.hip

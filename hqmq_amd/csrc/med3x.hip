@@ -920,18 +920,23 @@ int hqmq::med3x_calls(const Med3xCall *c, int count, MedSelect *later, hipStream
         const int vec = !(((uintptr_t)c[i].x | (uintptr_t)(c[i].xsb * elt) | (uintptr_t)(c[i].xsh * elt) | (uintptr_t)(c[i].xst * elt)) & (4 * elt - 1));
         t[i] = MedTensor{c[i].x, c[i].xsb, c[i].xsh, c[i].xst, vec, c[i].mult, (uint32_t *)c[i].ws, c[i].median, c[i].thr, c[i].n_out};
     }
+    // What a call's launches touch of its workspace.  Two calls may share one, or a part: then they go one after the other, each with its
+    // selection, which cannot wait for the quantize launch: the second call's histograms come over the first one's.
+    auto used = [&](int i, bool best) { return best ? hqmq_med3x_workspace_best_bytes(c[i].H, c[i].dtype) : hqmq_med3x_workspace_bytes(c[i].H, c[i].dtype); };
+    auto has_best = [&](int i) { return c[i].ws_bytes >= used(i, true); };
+    auto apart = [&](bool best0, bool best1) {
+        const uintptr_t w0 = (uintptr_t)c[0].ws, w1 = (uintptr_t)c[1].ws;
+        return w0 + used(0, best0) <= w1 || w1 + used(1, best1) <= w0;
+    };
     // one set of launches for both tensors where their shapes agree and their workspaces are apart
     if (count == 2 && c[0].dtype == c[1].dtype && c[0].B == c[1].B && c[0].H == c[1].H && c[0].T == c[1].T && c[0].n == c[1].n) {
-        const uintptr_t w0 = (uintptr_t)c[0].ws, w1 = (uintptr_t)c[1].ws;
-        auto apart = [&](int64_t need) { return w0 + need <= w1 || w1 + need <= w0; };
-        const int64_t best = hqmq_med3x_workspace_best_bytes(c[0].H, c[0].dtype);
-        const bool parts = c[0].ws_bytes >= best && c[1].ws_bytes >= best && apart(best);
-        if (parts || apart(hqmq_med3x_workspace_bytes(c[0].H, c[0].dtype)))
+        const bool parts = has_best(0) && has_best(1) && apart(true, true);
+        if (parts || apart(false, false))
             return med3x_launch(MedPair{{t[0], t[1]}, c[0].B, c[0].H, c[0].T, c[0].n}, c[0].dtype, 2, parts, later, st);
     }
+    if (count == 2 && later && !apart(has_best(0), has_best(1))) later = nullptr;
     for (int i = 0; i < count; i++) {
-        const bool parts = c[i].ws_bytes >= hqmq_med3x_workspace_best_bytes(c[i].H, c[i].dtype);
-        const int rc = med3x_launch(MedPair{{t[i], t[i]}, c[i].B, c[i].H, c[i].T, c[i].n}, c[i].dtype, 1, parts, later ? later + i : nullptr, st);
+        const int rc = med3x_launch(MedPair{{t[i], t[i]}, c[i].B, c[i].H, c[i].T, c[i].n}, c[i].dtype, 1, has_best(i), later ? later + i : nullptr, st);
         if (rc) return rc;
     }
     return HQMQ_OK;

@@ -106,3 +106,69 @@ def test_long_appends_write_the_rows_of_short_ones(dn, S, b_r, d_h, med, T, t_of
         assert torch.equal(t.scale[:, :, t_off:t_off + T].view(torch.int16), c["r_max"].reshape(B, H, T).view(torch.int16))
     for key, p in planes.items():
         assert torch.equal(p[:, :, :t_off], before[key][:, :, :t_off]) and torch.equal(p[:, :, t_off + T:], before[key][:, :, t_off + T:]), key
+
+
+def _appended_through_the_c_abi(case, ks, vs, med, layout, dt, S, b_r, d_h, H):
+    """hqmq_append_kv_grid with the workspaces laid out as `layout` says; [(x, quantizer, PackedTensor, median, thr, count or None)]."""
+    import ctypes as C
+
+    import hqmq
+    from hqmq_amd import _lib as L, ops
+    q = hqmq.with_outlier_extraction(hqmq.HQMQ(n_layers=1, n_heads=H, secondary_size=S, radius_bits=b_r, device=DEV), C=3.0)
+    lib, code = L.lib(), ops._dt(ks)
+    best = int(lib.hqmq_med3x_workspace_best_bytes(C.c_int(H), C.c_int(code)))
+    least = int(lib.hqmq_med3x_workspace_bytes(C.c_int(H), C.c_int(code)))
+    # (offset, bytes) of K's and V's workspace in one buffer
+    spans = {"apart": ((0, best), (best, best)), "same": ((0, best), (0, best)), "overlap": ((0, best), (65536, best)),
+             "overlap below": ((65536, best), (0, best)), "V's is small": ((0, best), (4096, least)), "K's is small": ((4096, least), (0, best)),
+             "both small": ((0, least), (0, least))}[layout]
+    room = torch.full((2 * best,), 0x5A, dtype=torch.uint8, device=DEV)
+    cache = q.new_cache(ks.shape[0], max(ks.shape[2], vs.shape[2]), d_h, dt, 0)
+    args, keep = [], []
+    for i, (x, t) in enumerate(((ks, cache.K), (vs, cache.V))):
+        joint, slack = q.inner._joint_and_slack(0, i, x)
+        tmpl, grid, _ = ops._append_block(x, t, joint, slack, b_r, 3.0 if i in med else None, "c abi %d" % i)
+        assert grid
+        a = L.AppendArgs.from_buffer_copy(tmpl)
+        a.q.x, a.q.B, a.q.T = x.data_ptr(), x.shape[0], x.shape[2]
+        a.q.x_stride_b, a.q.x_stride_h, a.q.x_stride_t, _ = x.stride()
+        median, thr, count = (torch.full((H,), -1, dtype=d, device=DEV) for d in (torch.float32, dt, torch.int32))
+        if i in med:
+            a.median_mult, a.med_workspace, a.med_workspace_bytes = 3.0, room.data_ptr() + spans[i][0], spans[i][1]
+            a.median, a.thr, a.n_out = median.data_ptr(), thr.data_ptr(), count.data_ptr()
+        args.append((a, grid))
+        keep.append((x, joint, slack, t, median, thr, count))
+    (ak, gk), (av, gv) = args
+    L.call(lib.hqmq_append_kv_grid, case, torch.cuda.current_device(), C.addressof(ak), C.addressof(av), gk, gv)
+    torch.cuda.synchronize()
+    return q, keep
+
+
+@pytest.mark.parametrize("layout", ["apart", "same", "overlap", "overlap below", "V's is small", "K's is small", "both small"])
+@pytest.mark.parametrize("dn,S,b_r,d_h,T_k,T_v,med", [
+    ("fp16", 96, 4, 128, 700, 700, (0, 1)), ("bf16", 24, 3, 128, 650, 650, (0, 1)), ("fp16", 192, 6, 64, 1100, 2300, (0, 1)),
+    ("bf16", 96, 4, 128, 2200, 600, (0, 1)), ("fp16", 24, 3, 128, 600, 300, (0, 1)), ("fp16", 96, 4, 128, 620, 620, (0,)), ("bf16", 24, 3, 128, 620, 700, (1,))])
+def test_appends_whatever_the_workspaces(layout, dn, S, b_r, d_h, T_k, T_v, med):
+    """K and V of one append are the threshold's, the quantizer's and the compaction's calls for K and then for V, also where the two share
+    a workspace or a part of one, differ in length, or only one of them extracts outliers.  V's norms are a hundred times K's."""
+    from hqmq_amd import ops
+    from hqmq_amd.packed import PackedTensor
+    dt, B, H = DT[dn], 1, 3
+    ks = kv_input((B, H, T_k, d_h), dt, seed=T_k, outlier_p=0.02).to(DEV)
+    vs = (kv_input((B, H, T_v, d_h), torch.float32, seed=T_v + 1, outlier_p=0.03, outlier_gain=(5.0, 9.0)) * 100).to(dt).to(DEV)
+    q, got = _appended_through_the_c_abi("append", ks, vs, med, layout, dt, S, b_r, d_h, H)
+    for i, (x, joint, slack, t, median, thr, count) in enumerate(got):
+        want = PackedTensor(B, H, t.t_cap, d_h, S, b_r, dt, DEV, joint, outliers=True, layout=(t.idx_bits, t.main_bits, t.aux_bits))
+        if i in med:
+            m, th, n = ops.med3x_threshold(x, 3.0)
+            assert torch.equal(median, m) and torch.equal(thr.view(torch.int16), th.view(torch.int16)) and torch.equal(count, n) and int(n.min()) > 0
+        ops.quantize(x, joint, slack, b_r, want_codes=False, thr=th if i in med else None, cache=want)
+        if i in med:
+            ops.outlier_compact(x, want)
+        for name in ("main", "aux", "scale", "flags", "sb_tile_off", "sb_count", "sb_overflow"):
+            a, b = getattr(t, name), getattr(want, name)
+            assert (a is None) == (b is None) and (a is None or torch.equal(a.view(torch.uint8), b.view(torch.uint8))), (name, "KV"[i])
+        for b in range(B):
+            for h in range(H):
+                n = int(want.sb_count[b, h])
+                assert torch.equal(t.sideband[b, h, :n].view(torch.int16), want.sideband[b, h, :n].view(torch.int16)) and torch.equal(t.sb_coord[b, h, :n], want.sb_coord[b, h, :n])
