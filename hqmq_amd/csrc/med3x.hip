@@ -857,7 +857,7 @@ static int run_med3x(const MedPair &a, int count, bool parts, MedSelect *later, 
             const hipError_t e = hipFuncSetAttribute((const void *)med_hist16_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) return (int)e;
             hipLaunchKernelGGL(med_hist16_kernel<D>, dim3((unsigned)blocks, a.H, count), dim3(1024), lds, st, a, rpb);
-            if (later)
+            if (later && blocks <= kSelectParts)
                 for (int i = 0; i < count; i++)
                     later[i] = MedSelect{a.t[i].ws, a.t[i].median, a.t[i].thr, a.t[i].n_out, a.t[i].mult, (int)blocks, (uint32_t)per_head};
             else hipLaunchKernelGGL(med_select16_kernel<D>, dim3(a.H, 1, count), dim3(1024), 0, st, a, (int)blocks);

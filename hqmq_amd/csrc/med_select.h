@@ -90,10 +90,18 @@ __device__ __forceinline__ int bin_of_rank(const uint32_t (&v)[8], uint32_t rank
 
 // By a block of 1024 threads: sums of the groups over the head's parts, the group of each rank, that group's bins over
 // the parts (a wavefront per part, 1 KB a time), the bin inside it.  The count wants the bins of the threshold's group as
-// well; the median's group leaves two for it nearly always, which are asked for along with the median's (a third round
-// trip otherwise: 6.9 -> 5.5 us; with every loop unrolled, 7.5: a launch this short waits for its code).
+// well; the median's group leaves two for it nearly always.  Up to kAheadParts parts these are asked for along with the median's (a third
+// round trip otherwise: 8 heads, 32 parts, 6.9 -> 5.5 us; with every loop unrolled, 7.5: a launch this short waits for its code).  Of more
+// parts four wavefronts a group take more trips one after the other than all sixteen do for the median's group and then for the threshold's,
+// and the block with the outputs came last of the whole quantize launch: 32768 tokens of one head, fp16 s96_r4 (256 parts), appended 64.8 -> 54.5 us,
+// with a launch of its own 56.4 -> 51.4; 16384 tokens of two heads fake-quantized (128 parts) 32.4 -> 28.3.
 // outputs: median, threshold and count are wanted; otherwise just the threshold, which is returned to every thread, and the wavefronts
 // share the one or two groups of the median.  sh: kSelectWords words of LDS, which the last wavefront reads until the block's next barrier.
+constexpr int kAheadParts = 32;
+// The quantize launch selects for itself up to this many parts.  Every one of its blocks reads all of them, so what it saves shrinks with their
+// number: over 480 appended and fake-quantized calls of one to six heads 5 % on average up to 64 parts, 2 % at 128 (6 % lost at worst), and
+// beyond, single heads of more than 16384 tokens, 1.4 % with 6 % lost where the blocks fill the chip (54.5 us above, 51.4 with the launch).
+constexpr int kSelectParts = 128;
 constexpr int kSelectWords = 16 * kGroups + 4 * kGroupBins + 2 * kPartBlocks + 4;
 // meanwhile(): what the block does while the first words travel.
 template <class D, class F>
@@ -160,10 +168,11 @@ __device__ __forceinline__ float select16(const MedSelect &m, int h, bool output
     };
     // the group of the threshold that a median of this key has (a threshold below every norm or beyond infinity: 0, or the last)
     auto group_above = [&](float tv) { return (int)min((norm_bits<D>(fmaxf(tv, 0.f)) >> 16) / kGroupBins, (uint32_t)kGroups - 1u); };
+    const bool ahead = outputs && parts <= kAheadParts;
     const int top_lo = group_above(D::rnd(key_value<D>((uint32_t)(group[0] * kGroupBins)) * m.mult));
     {
         const int q = wave >> 2, g = q == 0 ? group[0] : q == 1 ? group[1] : min(top_lo + q - 2, kGroups - 1);
-        if (outputs) {
+        if (ahead) {
             if (q < 2 || m.n_out) gather(g, bins_sh + q * kGroupBins, wave & 3, 4);
         } else if (group[0] == group[1]) gather(group[0], bins_sh, wave, 16);
         else gather(group[wave >> 3], bins_sh + (wave >> 3) * kGroupBins, wave & 7, 8);
@@ -176,7 +185,7 @@ __device__ __forceinline__ float select16(const MedSelect &m, int h, bool output
     if (wave < 2) {
         const int side = wave;
         uint32_t v[8];
-        bins(bins_sh + (!outputs && group[0] == group[1] ? 0 : side) * kGroupBins, v);
+        bins(bins_sh + (!ahead && group[0] == group[1] ? 0 : side) * kGroupBins, v);
         const int bin = bin_of_rank(v, rest[side]);
         if (bin >= 0) key_sh[side] = (uint32_t)(group[side] * kGroupBins + bin);
     }
@@ -189,10 +198,12 @@ __device__ __forceinline__ float select16(const MedSelect &m, int h, bool output
     if (!m.n_out) return tv;
     // chunks with norm > thr: whole groups above the one that holds the threshold, and the bins above it in there
     const int top = group_above(tv);
-    uint32_t *there = bins_sh + (top == top_lo ? 2 : 3) * kGroupBins;
-    if (top != top_lo && top != top_lo + 1) {           // the median's bin is far from its group's first
-        for (int i = tid; i < kGroupBins; i += 1024) there[i] = 0;
-        __syncthreads();
+    uint32_t *there = bins_sh + (!ahead || top == top_lo ? 2 : 3) * kGroupBins;
+    if (!ahead || (top != top_lo && top != top_lo + 1)) {
+        if (ahead) {                                    // the median's bin is far from its group's first
+            for (int i = tid; i < kGroupBins; i += 1024) there[i] = 0;
+            __syncthreads();
+        }
         gather(top, there, wave, 16);
         __syncthreads();
     }

@@ -1,4 +1,4 @@
-"""Calls whose quantize launch works the Med3x threshold out for itself (16-bit types, more than 16384 chunks per head), against the
+"""Calls whose quantize launch works the Med3x threshold out for itself (16-bit types, more than 16384 chunks and up to 128 parts per head), against the
 threshold's own calls, which take a launch for it: the same flags, counts and rows.  Packed rows in the same launch, at the edges of their
 forms."""
 import pytest
@@ -21,7 +21,10 @@ def _two_groups(x):
     ("fp16", 96, 4, (1, 2, 513, 128), "plain"), ("bf16", 24, 3, (3, 2, 700, 128), "plain"), ("fp16", 192, 6, (2, 1, 2100, 64), "two groups"),
     ("bf16", 192, 4, (1, 3, 1200, 64), "two groups"), ("bf16", 341, 4, (1, 1, 600, 128), "plain"), ("fp16", 341, 4, (1, 1, 600, 128), "two groups"),
     ("fp16", 24, 3, (1, 2, 520, 128), "nan"), ("bf16", 96, 4, (1, 2, 4100, 20), "plain"), ("fp16", 96, 4, (1, 1, 9000, 128), "equal"),
-    ("bf16", 24, 3, (1, 9, 530, 128), "zero")])
+    ("bf16", 24, 3, (1, 9, 530, 128), "zero"),
+    # parts per head around the lines of the selection: 32 and 33, 128 and 129
+    ("fp16", 24, 3, (1, 3, 4096, 128), "plain"), ("bf16", 96, 4, (1, 3, 4100, 128), "two groups"),
+    ("bf16", 24, 3, (1, 1, 16384, 128), "two groups"), ("fp16", 96, 4, (1, 1, 16400, 128), "two groups"), ("fp16", 24, 3, (1, 2, 16384, 128), "nan")])
 def test_quantize_launch_selects_the_threshold(dn, S, b_r, shape, what):
     import hqmq
     from hqmq_amd import ops
@@ -59,7 +62,8 @@ def test_quantize_launch_selects_the_threshold(dn, S, b_r, shape, what):
     (4400, 2, 1, 16), (300, 2, 3, 76),          # a block's step goes over many sequences, not a whole number of them
     (1, 3, 4097, 20), (2, 1, 601, 120),         # rows that do not divide a block's lanes
     (3, 2, 11, 4400),                           # rows of more chunks than a block has lanes
-    (1, 1, 129, 512), (1, 5, 513, 128)])        # last blocks of a single step
+    (1, 1, 129, 512), (1, 5, 513, 128),         # last blocks of a single step
+    (1, 2, 4096, 128), (1, 2, 4100, 128), (1, 1, 16400, 128)])      # 32, 33 and 129 parts per head
 def test_histograms_count_every_chunk_once(dn, shape):
     """Calls that count in one histogram per block (16-bit types, more than 16384 chunks per head), contiguous and with strides."""
     from hqmq_amd import ops
