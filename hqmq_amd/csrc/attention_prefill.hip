@@ -650,22 +650,21 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
 // (37 %); 1024 queries on 16384 tokens, 32 / 8 heads of 128, fp16 s96_r4 369 us in blocks of 128 columns, 342 in two splits of 256;
 // heads of 64 448 / 390; with 2 % of the K chunks verbatim 483 / 415.
 struct PfTimes {
-    double narrow, wide, start;
+    double narrow, wide, start, merge, rate;
 };
 static PfTimes pf_times(int d_h, bool flags) {
-    if (flags) return d_h == 64 ? PfTimes{2.75, 4.7, 11.0} : PfTimes{2.4, 3.1, 13.0};
-    return d_h == 64 ? PfTimes{2.25, 3.5, 9.0} : PfTimes{1.5, 2.65, 11.0};
+    if (flags) return d_h == 64 ? PfTimes{2.75, 4.7, 11.0, 2.0, 3.2e6} : PfTimes{2.4, 3.1, 13.0, 2.0, 3.2e6};
+    return d_h == 64 ? PfTimes{2.25, 3.5, 9.0, 2.0, 3.2e6} : PfTimes{1.5, 2.65, 11.0, 2.0, 3.2e6};
 }
 struct PfPlan {
     bool wide;
     int splits;
     double us;
 };
-static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int causal, int64_t off, int fixed_splits, bool flags) {
+static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int causal, int64_t off, int fixed_splits, const PfTimes &times) {
     const double last = causal ? std::max(1.0, std::min((double)Tkv, (double)off + Tq)) : std::max(Tkv, 1);      // tokens the last query sees
     const double mean = causal ? std::min(1.0, std::max(0.5, ((double)off + 0.5 * Tq) / last)) : 1.0;            // all, relative to it
     const int tiles = (int)((last * d_h + 8191) / 8192);
-    const PfTimes times = pf_times(d_h, flags);
     PfPlan best{false, 1, 1e30};
     static const int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 20, 24, 32};
     for (int i = 0; i < (fixed_splits > 0 ? 1 : (int)(sizeof(kSplits) / sizeof(int))); i++) {
@@ -675,7 +674,7 @@ static PfPlan pf_plan(int64_t cols, int64_t nz, int Tq, int Tkv, int d_h, int ca
             const double rounds = (double)(((cols + (wide ? 255 : 127)) / (wide ? 256 : 128) * nz * s + 255) / 256);
             // the longest block or a compute unit's share of all of them, whichever is more
             const double us = std::max(1.0, mean * rounds) * ((tiles + s - 1) / s) * (wide ? times.wide : times.narrow) + times.start * rounds +
-                              (s > 1 ? 2.0 + (double)(cols * nz) * s * (d_h + 4) * 8 / 3.2e6 : 0.0);
+                              (s > 1 ? times.merge + (double)(cols * nz) * s * (d_h + 4) * 8 / times.rate : 0.0);
             if (us < best.us) best = PfPlan{wide != 0, s, us};
         }
     }
@@ -703,35 +702,58 @@ static bool attn_prefill_takes(const hqmq_attn_args *a) {
 }
 // The same for the kernels of attention_fast.hip: blocks of 16 columns or of 32 (attn_two_groups; over outlier caches always of 16), fitted
 // to the same and 100 more chunks: 4 to 11 % off on average.
-static double fast_us(const hqmq_attn_args *a, int64_t cols, int splits) {
+struct FastTimes {
+    double base, start, two, one, merge, rate;
+};
+static FastTimes fast_times(int d_h, bool flags) {
+    if (d_h == 64) return FastTimes{2.1, flags ? 4.3 : 4.7, 0.68, flags ? 0.6 : 0.41, 1.5, 1.95e6};
+    return FastTimes{2.1, flags ? 5.3 : 6.4, 0.5, flags ? 0.5 : 0.27, 1.5, 1.95e6};
+}
+static double fast_us(const hqmq_attn_args *a, int64_t cols, int splits, const FastTimes &times) {
     const int64_t nz = (int64_t)a->B * a->H_kv, cg = (cols + 15) / 16, pairs = (cg + 1) / 2 * nz * splits;
     const int d_h = 4 * a->n_chunks;
     const bool flags = a->K.flag_plane != nullptr, two = attn_two_groups((int)cg, flags, cg * nz * splits, a->T_kv / splits, a->n_chunks, a->aux_bits);
-    const double tiles = ((double)a->T_kv * d_h + 8191) / 8192, start = d_h == 64 ? (flags ? 4.3 : 4.7) : flags ? 5.3 : 6.4;
-    const double tile = d_h == 64 ? (two ? 0.68 : flags ? 0.6 : 0.41) : two ? 0.5 : flags ? 0.5 : 0.27;
-    return 2.1 + (double)(((two ? pairs : cg * nz * splits) + 255) / 256) * (start + tiles / splits * tile) +
-           (splits > 1 ? 1.5 + (double)(cols * nz) * splits * (d_h + 4) * 8 / 1.95e6 : 0.0);
+    const double tiles = ((double)a->T_kv * d_h + 8191) / 8192;
+    return times.base + (double)(((two ? pairs : cg * nz * splits) + 255) / 256) * (times.start + tiles / splits * (two ? times.two : times.one)) +
+           (splits > 1 ? times.merge + (double)(cols * nz) * splits * (d_h + 4) * 8 / times.rate : 0.0);
 }
 // The number of splits of a call that leaves it open, 0 if it is better off with the other kernels; splits > 0: the same decision for
-// a given number.  Both estimates are of the plan that would run, the other kernels' with the splits of attn_decode_splits.  Over 200
-// prefill chunks of 64 and more columns and 64 to 32768 tokens, plain and outlier caches, the choice takes 0.7 % longer than the fastest
-// plan of either kernel (16 % at worst), 1.8 % less than with one set of times for both head sizes and a margin of 5 %.  us, and with the
+// a given number.  Both estimates are of the plan that would run, the other kernels' with the splits of attn_decode_splits.  us, and with the
 // kernel chosen by numbers of splits that would not run: 1 x 33 queries on 19403 tokens, 32 / 8 heads of 128, s24_r3, 37.8 (prefill
 // kernel 47.2); 3 x 70 on 5811, 28 / 4, s192_r4, 50.8 (decode kernels 62.9).
+// fp16 caches have a line of their own, from times of an earlier state of both kernels: the kernels differ in their error, and a line that
+// follows the times moves calls to the less precise one.  Prefill kernel against decode kernels, error against 64 bits, 420 chunks near the line:
+// over outlier caches 0.82 to 0.84 where K's verbatim chunks are large (heads of 128, 2 % of them 50 to 200 times the others), 1.01 to 1.03 on
+// normal and lognormal channels, so a call changes kernel in neither direction; over plain fp16 caches 1.00 to 1.02, so it comes here
+// only where both lines say so; bf16 at most 1.002.  What that costs against the present times for all of them: 10 % of the fp16 chunks over outlier
+// caches take 1.09 of the time (0.86 to 1.52; 8 x 33 queries on 437 tokens, 28 / 4 heads, s192_r4, 30.6 us for 22.4), 2 % of those over
+// plain caches 1.06.
 int attn_prefill_splits(const hqmq_attn_args *a, int splits) {
     const int64_t cols = (int64_t)a->T_q * (a->H_q / a->H_kv), nz = (int64_t)a->B * a->H_kv;
     if (cols < 64 || !attn_prefill_takes(a)) return 0;
-    const PfPlan plan = pf_plan(cols, nz, a->T_q, a->T_kv, 4 * a->n_chunks, a->causal, a->causal_offset, splits, a->K.flag_plane != nullptr);
+    const int d_h = 4 * a->n_chunks;
+    const bool flags = a->K.flag_plane != nullptr;
+    auto plan_of = [&](const PfTimes &times) { return pf_plan(cols, nz, a->T_q, a->T_kv, d_h, a->causal, a->causal_offset, splits, times); };
+    const PfPlan plan = plan_of(pf_times(d_h, flags));
+    if (a->force_generic == 3) return plan.splits;
     // Outlier caches of three radius bits keep the decode kernels: most radius codes are 1, 2 or 4, with which those kernels' V is
-    // exact, and V rounded as a value left lognormal channels 0.5 % further from 64-bit results (s24_r3; 6 % nearer on average).
-    if (a->K.flag_plane && a->qmax < 15 && a->force_generic != 3) return 0;
-    return a->force_generic == 3 || plan.us < fast_us(a, cols, splits > 0 ? splits : attn_decode_splits(a)) ? plan.splits : 0;
+    // exact, and V rounded as a value left lognormal channels 0.5 % further from 64-bit results (s24_r3; 6 % nearer on average).  Plain
+    // bf16 caches of three radius bits may come here: rounding the output to bf16 leaves 0.05 % of that on average, 0.16 % at most (72 chunks).
+    if (flags && a->qmax < 15) return 0;
+    const int other = splits > 0 ? splits : attn_decode_splits(a);
+    if (a->dtype == HQMQ_F16) {
+        const PfTimes then{flags ? 1.75 : 1.37, flags ? 3.5 : 2.7, 12.0, 5.0, 2e6};
+        const FastTimes fast_then{3.0, 6.0, 0.6, flags ? 0.7 : 0.47, 3.0, 2e6};
+        if (plan_of(then).us >= 0.95 * fast_us(a, cols, other, fast_then)) return 0;
+        if (flags) return plan.splits;
+    }
+    return plan.us < fast_us(a, cols, other, fast_times(d_h, flags)) ? plan.splits : 0;
 }
 
 template <int DH, int MB, bool AUX, int DT, bool FL>
 static int launch_pf(const AttnParams &p, hipStream_t st, const LaunchTiming &tm) {
     const int64_t cols = (int64_t)p.Tq * p.G, nz = (int64_t)p.B * p.Hkv * p.n_splits;
-    const bool wide = pf_plan(cols, (int64_t)p.B * p.Hkv, p.Tq, p.Tkv, DH, p.causal, p.causal_offset, p.n_splits, FL).wide;
+    const bool wide = pf_plan(cols, (int64_t)p.B * p.Hkv, p.Tq, p.Tkv, DH, p.causal, p.causal_offset, p.n_splits, pf_times(DH, FL)).wide;
     const int64_t gx = (cols + (wide ? 255 : 127)) / (wide ? 256 : 128);
     // Column blocks per block, one after the other (the tables stay in LDS): as few rounds of 256 blocks as possible.  Ragged
     // batches leave the choice of the next block to the hardware.

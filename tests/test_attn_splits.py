@@ -86,6 +86,58 @@ def test_prefill_chunks_take_the_faster_kernel(B, Hq, Hkv, d_h, T, Tq, S, b_r, d
     assert (L.lib().hqmq_attn_splits(C.addressof(a)) == splits) == (S == 24 and T > 9000)
 
 
+@pytest.mark.parametrize("med,B,Hq,Hkv,d_h,T,Tq,S,b_r", [
+    # over outlier caches: with the prefill kernel, whose error is 0.82 of the decode kernels' where K's verbatim chunks are large
+    (True, 8, 32, 8, 128, 341, 17, 96, 4), (True, 7, 28, 4, 128, 909, 21, 192, 6), (True, 1, 28, 4, 128, 8299, 43, 96, 4),
+    (True, 1, 32, 8, 128, 4393, 101, 192, 6), (True, 5, 28, 4, 128, 215, 29, 192, 4),
+    # over plain fp16 caches: with the decode kernels, up to 2 % nearer to 64-bit results
+    (False, 8, 64, 8, 64, 3109, 31, 192, 4), (False, 6, 32, 8, 128, 1024, 45, 96, 4), (False, 8, 32, 8, 128, 1382, 46, 24, 3),
+    (False, 1, 64, 8, 64, 5289, 79, 192, 4), (False, 3, 32, 8, 128, 1121, 87, 192, 6)])
+def test_fp16_chunks_keep_to_the_kernel_of_smaller_error(med, B, Hq, Hkv, d_h, T, Tq, S, b_r):
+    """Calls near the line between the two kernels, for which the times alone would name the other one (with its own number of splits)."""
+    from hqmq_amd import _lib as L
+    a = _args(B, Hq, Hkv, Tq, T, d_h // 4, False, L.DT_CODE[torch.float16])
+    a.idx_bits, a.main_bits, a.aux_bits = L.layout_bits(S, b_r)
+    a.t_cap, a.qmax, a.softmax_scale, a.causal, a.causal_offset = (T + 63) // 64 * 64, (1 << b_r) - 1, d_h ** -0.5, 1, T - Tq
+    for t in (a.K, a.V):
+        t.K = 24 * S
+        if med:
+            t.flag_plane = t.sideband = t.sb_coord = t.sb_count = t.sb_tile_off = 16
+            t.sb_cap = 64
+    splits = {}
+    for a.force_generic in (0, 2, 3):           # the call's own choice, the decode kernels, the prefill kernel
+        splits[a.force_generic] = L.lib().hqmq_attn_splits(C.addressof(a))
+    assert splits[2] != splits[3] and splits[0] == splits[3 if med else 2]
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("B,Hq,Hkv,T,Tq,S,b_r", [(8, 32, 8, 341, 17, 96, 4), (5, 28, 4, 215, 29, 192, 4), (7, 28, 4, 909, 21, 192, 6)])
+def test_chunks_over_large_verbatim_keys(B, Hq, Hkv, T, Tq, S, b_r):
+    """fp16 outlier caches with 2 % of K's chunks 50 to 200 times the others: a chunk of few queries takes the prefill kernel, with an error of
+    0.82 to 0.84 of the decode kernels' (38 calls measured)."""
+    import hqmq
+    from tests.helpers import exact_dense, kv_input
+    dt, d_h = torch.float16, 128
+    k = kv_input((B, Hkv, T, d_h), dt, 71, lognormal=False, outlier_p=0.02).cuda()
+    v = kv_input((B, Hkv, T, d_h), dt, 72, lognormal=False).cuda()
+    Q = torch.randn(B, Hq, Tq, d_h, generator=torch.Generator().manual_seed(73)).to(dt).cuda()
+    w = hqmq.with_outlier_extraction(hqmq.HQMQ(n_layers=1, n_heads=Hkv, secondary_size=S, radius_bits=b_r, device="cuda"), C=3.0)
+    cache = w.new_cache(B, T, d_h, dt, 0)
+    w.append(cache, k, v, 0)
+    out = {f: hqmq.fused_attention_packed(Q, cache, causal=True, causal_offset=T - Tq, force_generic=f) for f in (0, 2, 3)}
+    seen = torch.arange(T, device="cuda").view(1, T) <= torch.arange(Tq, device="cuda").view(Tq, 1) + T - Tq
+    err = {f: 0.0 for f in out}
+    for b in range(B):
+        K, V = (exact_dense(t, b, T, x[b]).double().repeat_interleave(Hq // Hkv, 0) for t, x in ((cache.K, k), (cache.V, v)))
+        s = torch.matmul(Q[b].double(), K.transpose(1, 2).contiguous()) * d_h ** -0.5
+        ref = torch.matmul(torch.softmax(s.masked_fill(~seen, float("-inf")), -1), V)
+        for f in out:
+            err[f] += float((out[f][b].double() - ref).square().sum())
+    assert torch.equal(out[0].view(torch.int16), out[3].view(torch.int16))
+    assert err[0] < 0.9 ** 2 * err[2], err
+
+
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
 @pytest.mark.parametrize("S,b_r,dn,d_h,med,B,contexts", [
