@@ -55,13 +55,16 @@ constexpr uint32_t pf_tab(bool fl) { return kPfFlag + (fl ? 1024u : 0u); }
 // would not fit).  us, through registers and landing: unpacked 8 x 141 tokens, 28 / 4 heads, s192_r4, 20.1 / 19.0, 2 x 1024 heads of 64 s96_r4
 // 46.8 / 45.8, 4 x 300 queries on 300 tokens s192_r4 24.6 / 23.3.
 struct PfTables {
-    uint32_t v, end;            // V's table, the end of LDS
+    uint32_t unit, end;         // V's table begins a whole number of units behind K's; the end of LDS
     bool land;
 };
+// (Worked out from K's size wherever it is needed, not kept: held as one number chosen between both units, the outlier variants of d_h 128 put nine
+// registers more into scratch: 8 x 335 queries on 793 tokens s192_r6 107.2 us, worked out again 103.5; 8 x 214 on 298 s192_r4 36.7, 33.6.)
+__host__ __device__ __forceinline__ uint32_t pf_behind(int kk, uint32_t unit) { return (8u * (uint32_t)kk + unit - 1u) & ~(unit - 1u); }
 __host__ __device__ __forceinline__ PfTables pf_tables(int kk, int vk, bool fl, bool fp16) {
-    const uint32_t tab = pf_tab(fl), k = 8u * (uint32_t)kk, v = 8u * (uint32_t)vk, k1 = (k + 1023u) & ~1023u, v1 = (v + 1023u) & ~1023u;
-    if (fp16 && tab + k1 + v1 <= 160u * 1024u) return PfTables{tab + k1, tab + k1 + v1, true};
-    return PfTables{tab + ((k + 127u) & ~127u), tab + ((k + 127u) & ~127u) + v, false};
+    const uint32_t tab = pf_tab(fl), whole = tab + pf_behind(kk, 1024u) + pf_behind(vk, 1024u);
+    if (fp16 && whole <= 160u * 1024u) return PfTables{1024u, whole, true};
+    return PfTables{128u, tab + pf_behind(kk, 128u) + 8u * (uint32_t)vk, false};
 }
 
 // permutation of a row's 16-byte parts
@@ -98,10 +101,10 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     const PfTables place = pf_tables(p.Kc.K, p.Vc.K, FL, DT == HQMQ_F16);
     const bool pairs = ((((uintptr_t)kj) | ((uintptr_t)vj)) & 15) == 0 && ((p.Kc.K | p.Vc.K) & 1) == 0, land = DT == HQMQ_F16 && place.land && pairs;
     // (requested first of all; the wait for them is behind the first tiles' requests)
-    if (land) land_tables<8>(uniform_ptr((const uint8_t *)kj), 8u * (uint32_t)p.Kc.K, uniform_ptr((const uint8_t *)vj), 8u * (uint32_t)p.Vc.K, kPfTab, place.v, wave, lane);
+    if (land) land_tables<8>(uniform_ptr((const uint8_t *)kj), 8u * (uint32_t)p.Kc.K, uniform_ptr((const uint8_t *)vj), 8u * (uint32_t)p.Vc.K, kPfTab, kPfTab + pf_behind(p.Kc.K, 1024u), wave, lane);
     auto tables = [&]() PF_INLINE {
         const int kk = p.Kc.K, vk = p.Vc.K;
-        const uint32_t vt = place.v;
+        const uint32_t vt = kPfTab + pf_behind(kk, place.unit);
         if (land) {
             wait_vm<0>();
             return;
@@ -177,7 +180,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(AttnParams p, int 
     const uint16_t *d_scale = (const uint16_t *)dc.scale_plane + b * dc.ssb + hkv * dc.ssh;
     const uint32_t idx_mask = (1u << p.idx_bits) - 1u;
     const int idx_bits = p.idx_bits;
-    const uint32_t tab = dec_v ? place.v : kPfTab;
+    const uint32_t tab = kPfTab + (dec_v ? pf_behind(p.Kc.K, place.unit) : 0u);
     // Outlier caches (FL): a wavefront decodes whole 16-token tiles of the sideband (one at d_h 128, two at 64), so it also writes
     // their verbatim chunks, over the zeros that flagged chunks decode to.  Lane e takes entry e of the contiguous range that the tile
     // offsets name; the offsets (scalar loads) travel

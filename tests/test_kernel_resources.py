@@ -65,3 +65,16 @@ def test_two_blocks_of_plain_heads_of_64_fit_a_compute_unit(fast):
             seen += 1
             assert m[".vgpr_count"] <= 128, (mb, ab, ib, m[".vgpr_count"])
     assert seen == 18           # 16+0 (index width known or not), 16+1, 16+2, 16+3 (twice), 12+1, 12+2, 12+3, in both types
+
+
+def test_prefill_kernels_spill_no_more_registers():
+    """Vector registers that attn_prefill_kernel puts into scratch, by head size and outliers: few enough for the time they were measured with."""
+    spilled, seen = {}, 0
+    for name, k in _kernels().items():
+        m = re.search(r"attn_prefill_kernelILi(\d+)ELi(\d+)ELb(\d)ELi(\d)ELi(\d)ELb(\d)E", name)
+        if m:
+            d_h, _, aux, _, _, flags = (int(g) for g in m.groups())
+            seen += 1
+            if k[".vgpr_spill_count"] > (0 if d_h == 64 else 3 if not flags else 21 if aux else 14):
+                spilled[name] = k[".vgpr_spill_count"]
+    assert seen == 36 and spilled == {}
