@@ -201,7 +201,8 @@ def fake_quant(x: torch.Tensor, joint: torch.Tensor, slack: torch.Tensor, radius
         raise ValueError(f"expected (B, H, T, d_head), got {tuple(x.shape)}")
     tmpl, grid = _book(joint, slack, radius_bits, x.shape[3] // 4)
     ws = None if median_mult is None else _med_workspace(x, "med3x")
-    return L.tensors(L.native().fake(x, joint, tmpl.address, grid, median_mult, ws), "hqmq_quantize_grid")
+    return L.tensors(L.native().fake(x, joint, tmpl.address, grid, median_mult, ws),
+                     "hqmq_quantize_grid" if median_mult is None else "hqmq_quantize_med3x_grid")
 
 
 def outlier_mask(x: torch.Tensor, thr: torch.Tensor) -> torch.Tensor:

@@ -122,7 +122,9 @@ int hqmq_build_search_grid(const void *joint, int H, int S, int dtype, void *gri
 int hqmq_quantize_grid(const hqmq_quantize_args *a, const void *grid, void *stream);
 
 /* hqmq_med3x_threshold over the chunks of `a`, then hqmq_quantize_grid with that threshold (a->thr is not read): the same results,
- * in two launches instead of three for 16-bit calls of more than 16384 chunks per head. */
+ * in two launches instead of three for 16-bit calls of more than 16384 chunks per head, with cell lists, algo = 0, T * n_chunks > 256 and
+ * a workspace of hqmq_med3x_workspace_best_bytes, up to 65535 * max(256 / H, 1) chunks per head (524288 where H is 1).  The quantize launch
+ * reads the workspace then and writes median, thr and n_out: none of them may overlap what `a` names. */
 int hqmq_quantize_med3x_grid(const hqmq_quantize_args *a, float mult, void *workspace, int64_t workspace_bytes, float *median, void *thr,
                              int32_t *n_out, const void *grid, void *stream);
 
@@ -196,7 +198,9 @@ int hqmq_crop(const hqmq_crop_args *a, void *stream);
 typedef struct hqmq_append_args {
     hqmq_quantize_args q;
     float median_mult;
-    void *med_workspace; int64_t med_workspace_bytes;  /* hqmq_med3x_workspace_bytes(H, dtype), or .._best_bytes */
+    void *med_workspace; int64_t med_workspace_bytes;  /* hqmq_med3x_workspace_bytes(H, dtype), or .._best_bytes; in use until the
+                                                          call's launches have run.  K and V may share one, or a part of one: they
+                                                          then take the launches of the statistics one after the other */
     float *median; void *thr; int32_t *n_out;          /* [H] outputs: fp32, D, int32 (n_out may be NULL) */
     void *sideband; int64_t sb_cap;
     int32_t *sb_tile_off, *sb_count, *overflow;

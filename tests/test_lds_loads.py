@@ -32,3 +32,15 @@ def test_waits_by_count_only_where_the_loads_are_written_by_hand():
     assert "land_tables" in bodies[0] and "land_tables" in bodies[1]
     assert not re.search(r"wait_(vm|groups)\b|s_waitcnt\b", bodies[0])
     assert re.search(r"wait_groups\(", bodies[1])
+
+
+def test_prefill_waits_for_every_load_before_the_tables_are_read():
+    """attn_prefill_kernel's loads are the compiler's beside the landing ones, so it waits for all of them, in every wavefront and before the first
+    barrier that the tables are read behind."""
+    text = next(p for p in SOURCES if p.name == "attention_prefill.hip").read_text()
+    body = text[text.index("void attn_prefill_kernel("):text.index("// Launch plan")]
+    assert re.findall(r"wait_vm<\s*(\w+)\s*>|wait_groups|vmcnt", body) == ["0"] and body.count("land_tables<") == 1
+    landed, waited = body.index("if (land) land_tables<8>("), body.index("if (land) {\n            wait_vm<0>();")
+    met = body.index("if (it == 0) tables();\n    __syncthreads();")
+    assert landed < waited < met and "__syncthreads" not in body[landed:met] and body.index("for (int it = 0;") < met
+    assert "int64_t rows = gx;" in text and "per <= gx" in text        # at most as many rows as column blocks: the first round is every block's

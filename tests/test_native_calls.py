@@ -81,6 +81,9 @@ def test_errors_are_exceptions():
     for call in (lambda: ops.quantize(k.float(), joint, slack, 4), lambda: ops.quantize(k[:, :2], joint, slack, 4), lambda: ops.fake_quant(k[0], joint, slack, 4)):
         with pytest.raises(ValueError):
             call()
+    for mult, name in ((None, "hqmq_quantize_grid"), (3.0, "hqmq_quantize_med3x_grid")):        # under the name of the call that was made
+        with pytest.raises(L.HqmqError, match=name):
+            ops.fake_quant(k, joint, slack, 99, mult)
     with pytest.raises(L.HqmqError):                        # a status of the library
         decode_dequant(c["idx"], c["rq"], c["r_max"], c["joint"], 0)
     with pytest.raises(L.HqmqError):
