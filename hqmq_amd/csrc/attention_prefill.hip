@@ -31,7 +31,7 @@
 // Measured, B = 1, 32 / 8 heads of 128, s96_r4, 1024 queries on 32768 tokens (541 GFLOP, 0.43 ms at the rate of a large matrix
 // product): 0.61 ms against 0.96 with the decode kernels' two-column-group variants; 4096 on 4096 tokens causal, s24_r3:
 // 0.185 against 0.41; four sequences of 300 on 300: 0.023 against 0.048.  With 2 % of the K and V chunks verbatim: 1024 queries on
-// 32768 tokens 0.77 ms against 2.88, 300 on 8000 (28 / 4 heads, s192_r6) 0.088 against 0.318.  (K held as values like V, without the
+// 32768 tokens 0.76 ms against 2.88, 300 on 8000 (28 / 4 heads, s192_r6) 0.087 against 0.318.  (K held as values like V, without the
 // second product, with the launch plans of a time when this took 0.93 and 0.122: 0.70 and 0.101, but up to 1.55 times as far from
 // 64-bit results at K of 3e-5 and 1.34 times at K of order one; values only in tokens with verbatim chunks, in units of a power of two: 0.80 and 0.107, still up to 1.11.)  Error against 64-bit
 // results relative to the decode kernels', 162 calls: K from 3e-5 to 30 at V of order one 0.96 on average, 1.03 at most; V of 1e-4

@@ -35,13 +35,14 @@
 // reads and a caller may drop afterwards (hqmq_search_grid_kept_bytes): the pools' counters, the centres and radii of the
 // codewords.
 //
-// What it costs: per 64 chunks 180 vector-ALU instructions at fp16 s96_r4, 249 at bf16 s24_r3 with flags, where the scan
-// over 96 secondaries takes 1,885.  Bound by vector-ALU issue: 0.82 (fp16) and 0.78 (bf16) of the cycles a compute unit is
-// busy, transcendental instructions counted once; its LDS pipe 33 %.  The form before this one reduced directions to the
+// What it costs: per 64 chunks 182 vector-ALU instructions at fp16 s96_r4, 254 at bf16 s24_r3 with flags (the selection of the
+// threshold included), where the scan over 96 secondaries takes 1,885.  Bound by vector-ALU issue: 0.86 (fp16) and 0.90 (bf16) of the
+// cycles a compute unit is busy, transcendental instructions counted once; its LDS pipe 36 and 39 %, half of it bank conflicts.  K and V of
+// 8 x 32768 tokens, fp16, s96_r4, packed: 119.5 us; 8 x 4 x 4001 tokens bf16 s24_r3 with Med3x, whole call: 97 us.  With rows packed through LDS
+// (180 and 249 vector instructions, but 99 and 192 scalar ones instead of 59 and 119): 123 and 117 us.  The form before that reduced directions to the
 // cell of all 24 units (75 instructions for unit, quaternion product and box, where this takes 25), listed 3.35 codewords
 // per box on average (S = 96, fp16; 8.7 is the longest of 64) where this lists 3.1 (7.5), and rounded every 16-bit number
-// by itself: 342 and 450 instructions.  K and V of 8 x 32768 tokens, fp16, s96_r4, packed: 186 -> 123 us; 8 x 4 x 4001 tokens
-// bf16 s24_r3 with Med3x, whole call: 163 -> 117 us.  33 boxes per axis instead of 27 take 5 % fewer instructions, 1 % less
+// by itself: 342 and 450 instructions, 186 and 163 us.  33 boxes per axis instead of 27 take 5 % fewer instructions, 1 % less
 // time and 1.8 times the memory; 27 without the comparison of all pairs: lists of 3.35 (9.3).
 //
 // Compiled with -ffp-contract=off; fused multiply-adds are written explicitly.
