@@ -415,17 +415,17 @@ def main():
         us_quant = event_time_us(quant_only, 10, stream)
         # algorithmic bytes of the call: K and V, 8 heads: the input row (d_h x 2 B) read, the packed row (66 B) written
         q_bytes = 2 * Hkv * T * (D_H * 2 + cache_bytes // (2 * Hkv * T))
-        valu_per_wave, waves = 180.1, 2 * Hkv * T * (D_H // 4) // 64     # instructions per 64 chunks (SQ_INSTS_VALU)
+        valu_per_wave, waves = 181.7, 2 * Hkv * T * (D_H // 4) // 64     # instructions per 64 chunks (SQ_INSTS_VALU)
         result["quantize"] = {"GTok_per_s": round(T / (us_quant * 1e-6) / 1e9, 5), "us_per_call": round(us_quant, 1), "tokens": T,
                               "what": "K and V of one layer, 8 kv heads x d_h 128, s96_r4 fp16, quantize + pack (no Med3x); "
                                       "the config-1 workload (s24_r3 + Med3x) is in the config1 block, GPU and CPU on the same input",
                               "algorithmic_bytes_per_call": q_bytes, "GBps": round(q_bytes / us_quant / 1e3, 1),
                               "bytes_roofline_frac": round(q_bytes / us_quant / 1e3 / HBM_PEAK_GBPS, 4),
                               "valu_issue_frac": round(valu_per_wave * 4 * waves / (1024 * 2.4e3 * us_quant), 3),
-                              "valu_issue_frac_is": "180.1 vector-ALU instructions per 64 chunks (SQ_INSTS_VALU of this shape, "
+                              "valu_issue_frac_is": "181.7 vector-ALU instructions per 64 chunks (SQ_INSTS_VALU of this shape, "
                                                     "profiles/quantize_grid_kernel_instruction_counters.txt, not measured by this run) x 4 cycles "
                                                     "x groups of 64 chunks / (1024 SIMDs x 2.4 GHz x this run's time): the kernel is bound by "
-                                                    "vector-ALU issue, not by bytes; of the cycles a CU is busy, at the clock it has then, it is 0.82"}
+                                                    "vector-ALU issue, not by bytes; of the cycles a CU is busy, at the clock it has then, it is 0.86"}
         k1, v1 = k[:, :, :1].contiguous(), v[:, :, :1].contiguous()
 
         def append_one(i):
